@@ -142,6 +142,17 @@ int mhip_gemm_residual(void* stream, const void* a, const void* b, const void* b
                        int64_t batch, int64_t stride_a, int64_t stride_b, int64_t stride_c,
                        int trans_a, int trans_b, int activation, int dtype);
 
+/* The same (residual may be NULL) with device memory the call may use for partial sums: a problem with few
+ * tiles and a long K is then split along K over the whole device.  mhip_gemm_workspace returns the bytes the
+ * choice for a problem can use (0: none); with less, or none, the result is computed without splitting.  The
+ * workspace is 16-byte aligned, its content is overwritten and meaningless afterwards, and it may be reused as
+ * soon as work enqueued behind this call on the same stream may run. */
+int64_t mhip_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b, int dtype);
+int mhip_gemm_ws(void* stream, const void* a, const void* b, const void* bias, const void* residual, void* c,
+                 int64_t M, int64_t N, int64_t K, int64_t batch, int64_t stride_a, int64_t stride_b,
+                 int64_t stride_c, int trans_a, int trans_b, int activation, int dtype, void* workspace,
+                 int64_t workspace_bytes);
+
 /* Attention -------------------------------------------------------------- */
 
 /* O = softmax(scale * Q K^T + mask, causal) V.

@@ -29,6 +29,9 @@ SIGNATURES = {
                          _i32, _i32, _i32, _i32]),
     "mhip_gemm_residual": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                                   _i32, _i32, _i32, _i32]),
+    "mhip_gemm_workspace": (_i64, [_i64, _i64, _i64, _i64, _i32, _i32, _i32]),
+    "mhip_gemm_ws": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
+                            _i32, _i32, _i32, _i32, _vp, _i64]),
     "mhip_flash_attention": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
                                     _f32, _i32, _i64, _i64, _i32]),
     "mhip_flash_attention_strided": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,

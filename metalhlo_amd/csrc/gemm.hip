@@ -12,21 +12,9 @@
 // plain LDS-tiled kernel.
 #include <mutex>
 
-#include "gemm_common.h"
+#include "gemm_lds.h"
 
 namespace mhip {
-
-// Swizzle of the 16-byte chunk index inside a 128-byte LDS row.  Rows r..r+15
-// (r % 16 == 0) map one chunk column onto 16 distinct bank groups.
-__device__ inline int swz(int row) { return ((row >> 1) ^ (row >> 4)) & 7; }
-
-__device__ inline uint32_t lds_off(int row, int chunk) {
-    return (uint32_t)(row * kRowBytes + ((chunk ^ swz(row)) << 4));
-}
-
-__device__ inline __amdgpu_buffer_rsrc_t make_rsrc(const void* p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
-}
 
 // ---- operand with k contiguous in memory: [rows_total][ld] ----------------
 template <int ROWS, int NT>
@@ -97,13 +85,6 @@ struct MnMajorLoader {
     }
 };
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-
-// MFMA operand (32 mn x 16 k) for k-step `s` out of a k-major tile.
-__device__ inline u32x4 frag_kmajor(const char* tile, int row0, int s, int lane) {
-    return *reinterpret_cast<const u32x4*>(tile + lds_off(row0 + (lane & 31), 2 * s + (lane >> 5)));
-}
 // Same operand out of an mn-major tile via two transposing reads.
 template <int ROWS>
 __device__ inline u32x4 frag_mnmajor(const char* tile, int mn0, int s, int lane) {
@@ -139,8 +120,6 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(GemmArgs g) {
     const int64_t batch = blockIdx.y;
     const T* a = static_cast<const T*>(g.a) + batch * g.sa;
     const T* b = static_cast<const T*>(g.b) + batch * g.sb;
-    T* c = static_cast<T*>(g.c) + batch * g.sc;
-    const T* res = g.residual ? static_cast<const T*>(g.residual) + batch * g.sc : nullptr;
 
     // A is stored [M][K] (k contiguous) unless TA ([K][M]); B is stored [K][N]
     // (k slow) unless TB ([N][K]).
@@ -153,7 +132,6 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(GemmArgs g) {
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = wave / WGN, wn = wave % WGN;
-    const int lrow = lane & 31, lhalf = lane >> 5;
 
     f32x16 acc[TM][TN];
 #pragma unroll
@@ -207,91 +185,7 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(GemmArgs g) {
         __syncthreads();
     }
 
-    // Epilogue.  The MFMAs were issued as (B-fragment, A-fragment), so each
-    // 32x32 accumulator tile is held transposed: a lane owns row m = lrow and,
-    // in register group q = r/4, the four consecutive columns 8q + 4*lhalf + r%4.
-    const T* bias = static_cast<const T*>(g.bias);
-    const bool vec_store = (g.N % 8 == 0) && ((reinterpret_cast<uintptr_t>(c) & 15) == 0);
-    // Stage the wave's sub-tile in LDS as rounded 16-bit rows (padded by 16 bytes
-    // against bank conflicts); the rows then go out with lanes running along n, so
-    // every store instruction writes whole contiguous row segments.
-    constexpr int kRowPad = WTN * 2 + 16;
-    char* stage = smem + wave * (WTM * kRowPad);
-    dispatch_act(g.act, [&](auto act_tag) {
-    constexpr int ACT = decltype(act_tag)::value;
-#pragma unroll
-    for (int j = 0; j < TN; j++) {
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int nl = j * 32 + 8 * q + 4 * lhalf;          // column inside the wave tile
-            const int n = n0 + wn * WTN + nl;
-            float bv[4] = {0.f, 0.f, 0.f, 0.f};
-            if (bias) {
-                if (vec_store && n < g.N) {
-                    const Pack4<T> t = __builtin_bit_cast(Pack4<T>, *reinterpret_cast<const u32x2*>(bias + n));
-#pragma unroll
-                    for (int e = 0; e < 4; e++) bv[e] = Elem<T>::to_f32(t.v[e]);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        if (n + e < g.N) bv[e] = Elem<T>::to_f32(bias[n + e]);
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < TM; i++) {
-                Pack4<T> o;
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    float v = acc[i][j][4 * q + e] + bv[e];
-                    v = apply_act_c<ACT>(v);
-                    o.v[e] = Elem<T>::from_f32(v);
-                }
-                *reinterpret_cast<u32x2*>(stage + (i * 32 + lrow) * kRowPad + nl * 2) =
-                    __builtin_bit_cast(u32x2, o);
-            }
-        }
-    }
-    });
-    // each wave only re-reads what it wrote itself
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (vec_store) {
-        constexpr int kCpr = WTN / 8;                // 16-byte chunks per row
-        constexpr int kRowsPerPass = 64 / kCpr;
-        const int cc = lane % kCpr, rr = lane / kCpr;
-#pragma unroll
-        for (int p = 0; p < WTM / kRowsPerPass; p++) {
-            const int ml = p * kRowsPerPass + rr;
-            const int m = m0 + wm * WTM + ml;
-            const int n = n0 + wn * WTN + cc * 8;
-            if (m < g.M && n < g.N) {
-                u32x4 w = *reinterpret_cast<const u32x4*>(stage + ml * kRowPad + cc * 16);
-                if (res) w = add_chunk<T>(w, *reinterpret_cast<const u32x4*>(res + (int64_t)m * g.N + n));
-                *reinterpret_cast<u32x4*>(c + (int64_t)m * g.N + n) = w;
-            }
-        }
-    } else {
-        // rows of C are not 16-byte aligned (odd N): one element per lane, 64
-        // consecutive columns per store instruction
-        const uint16_t* st16 = reinterpret_cast<const uint16_t*>(stage);
-        uint16_t* c16 = reinterpret_cast<uint16_t*>(c);
-#pragma unroll 4
-        for (int ml = 0; ml < WTM; ml++) {
-            const int m = m0 + wm * WTM + ml;
-            if (m >= g.M) break;
-#pragma unroll
-            for (int cb = 0; cb < WTN / 64; cb++) {
-                const int nl = cb * 64 + lane;
-                const int n = n0 + wn * WTN + nl;
-                if (n < g.N) {
-                    T val = __builtin_bit_cast(T, st16[ml * (kRowPad / 2) + nl]);
-                    if (res) val = Elem<T>::from_f32(Elem<T>::to_f32(val) + Elem<T>::to_f32(res[(int64_t)m * g.N + n]));
-                    c16[(int64_t)m * g.N + n] = __builtin_bit_cast(uint16_t, val);
-                }
-            }
-        }
-    }
+    store_tile<T, TM, TN>(g, acc, smem + wave * (WTM * (WTN * 2 + 16)), m0 + wm * WTM, n0 + wn * WTN, batch, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -403,6 +297,13 @@ int launch_gemm256(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_a,
 bool gemm384_activation_ok(int act);
 bool gemm_stream_eligible(const GemmArgs& g, int64_t batch, int trans_a, int trans_b, int dtype);
 int launch_gemm_stream(hipStream_t s, const GemmArgs& g, int trans_b, int dtype);
+// gemm_skinny.hip: at most 64 rows, the waves of a workgroup split K.
+bool gemm_skinny_eligible(const GemmArgs& g, int trans_a, int elem_bytes);
+int64_t gemm_skinny_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b);
+int launch_gemm_skinny(hipStream_t s, GemmArgs g, int64_t batch, int trans_b, int dtype, int64_t workspace_bytes);
+// gemm_mid.hip: 64- and 128-row tiles through a ring of LDS stages, K split where that leaves units idle.
+int64_t gemm_mid_workspace(int64_t M, int64_t N, int64_t K, int64_t batch);
+int launch_gemm_mid(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_a, int trans_b, int dtype, int64_t workspace_bytes);
 // gemm_f32.hip: fp32 operands on the fp32 matrix instruction, 128x128 tiles.
 bool gemm_f32_mfma_wanted(const GemmArgs& g);
 int launch_gemm_f32_mfma(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_a, int trans_b);
@@ -491,7 +392,7 @@ static thread_local int g_last_variant = 0;
 static inline int chose(int variant, int status) { g_last_variant = variant; return status; }
 
 template <typename T, bool TA, bool TB>
-static int pick_tile(hipStream_t s, const GemmArgs& g, int64_t batch) {
+static int pick_tile(hipStream_t s, const GemmArgs& g, int64_t batch, int64_t workspace_bytes) {
     const int64_t tiles_m = (g.M + 255) / 256;
     const int64_t big = tiles_m * ((g.N + 255) / 256) * batch;
     constexpr int dt = std::is_same<T, bf16_t>::value ? MHIP_BF16 : MHIP_F16;
@@ -530,6 +431,8 @@ static int pick_tile(hipStream_t s, const GemmArgs& g, int64_t batch) {
     if (force == 2567) {
         if (gemm256_eligible(g, batch, TA, TB, dt, 384) && gemm384_activation_ok(g.act)) return chose(2567, launch_gemm256(s, g, batch, TA, TB, dt, 384, 4));
     }
+    // (up to 192 rows: half of a 256-row tile would be padding)
+    if (force == 0 && g.M <= 192) return chose(128, launch_gemm_mid(s, g, batch, TA, TB, dt, workspace_bytes));
     constexpr int cus = 256;                           // compute units of the device this is written for
     const int64_t narrow = tiles_m * ((g.N + 127) / 128) * batch, stages = g.K / 32;
     const int64_t wide_cost = ((big + cus - 1) / cus) * (stages * 32 + 700);
@@ -582,17 +485,20 @@ static int pick_tile(hipStream_t s, const GemmArgs& g, int64_t batch) {
         if (narrow_ok && (!wide_ok || narrow_cost < wide_cost)) return chose(2561, launch_gemm256(s, g, batch, TA, TB, dt, 128));
         if (wide_ok) return chose(2560, launch_gemm256(s, g, batch, TA, TB, dt));
     }
+    // (fewer than 192 tiles of any ring kernel, a ragged K, or so few rows that 256-row tiles are mostly padding)
+    const bool large = big >= 192 && (g.K >= 1024 || g.N % 8 != 0);
+    if (force == 0 && !large) return chose(128, launch_gemm_mid(s, g, batch, TA, TB, dt, workspace_bytes));
     const bool want256 = force == 256 || (force != 128 && big >= 192 && (g.K >= 1024 || g.N % 8 != 0));
     if (want256) return chose(256, launch_mfma<T, 256, 256, 2, 4, TA, TB>(s, g, batch));
     return chose(128, launch_mfma<T, 128, 128, 2, 2, TA, TB>(s, g, batch));
 }
 
 template <typename T>
-static int pick_layout(hipStream_t s, const GemmArgs& g, int64_t batch, int ta, int tb) {
-    if (!ta && !tb) return pick_tile<T, false, false>(s, g, batch);
-    if (!ta && tb) return pick_tile<T, false, true>(s, g, batch);
-    if (ta && !tb) return pick_tile<T, true, false>(s, g, batch);
-    return pick_tile<T, true, true>(s, g, batch);
+static int pick_layout(hipStream_t s, const GemmArgs& g, int64_t batch, int ta, int tb, int64_t workspace_bytes) {
+    if (!ta && !tb) return pick_tile<T, false, false>(s, g, batch, workspace_bytes);
+    if (!ta && tb) return pick_tile<T, false, true>(s, g, batch, workspace_bytes);
+    if (ta && !tb) return pick_tile<T, true, false>(s, g, batch, workspace_bytes);
+    return pick_tile<T, true, true>(s, g, batch, workspace_bytes);
 }
 
 template <typename T>
@@ -618,10 +524,17 @@ static int launch_exact(hipStream_t s, const GemmArgs& g, int64_t batch, int ta,
 
 using namespace mhip;
 
+// Where the few-row kernel is ahead of 64-row tiles (16-bit operands with aligned rows): up to 16 rows always,
+// up to 32 for weights of up to 32 M elements -- beyond that A, re-read for every strip of columns, costs as much
+// L2 traffic as B ([28,6384] x [6384,688] 9.2 us against 12.1; [37,768] x [768,50304] 37 against 16.6).
+static bool skinny_rows(int64_t M, int64_t N, int64_t K, bool is16) {
+    return M <= 16 || !is16 || (M <= 32 && N * K <= (32 << 20));
+}
+
 static int gemm_entry(void* stream, const void* a, const void* b, const void* bias, const void* residual, void* c,
                       int64_t M, int64_t N, int64_t K, int64_t batch, int64_t stride_a,
                       int64_t stride_b, int64_t stride_c, int trans_a, int trans_b,
-                      int activation, int dtype) {
+                      int activation, int dtype, void* workspace = nullptr, int64_t workspace_bytes = 0) {
     if (M < 0 || N < 0 || K < 0 || batch < 0)
         return fail(MHIP_ERR_INVALID_ARGUMENT, "mhip_gemm: negative size");
     if (activation < MHIP_ACT_NONE || activation > MHIP_ACT_GELU_ERF)
@@ -649,9 +562,16 @@ static int gemm_entry(void* stream, const void* a, const void* b, const void* bi
                         (reinterpret_cast<uintptr_t>(b) & 15) == 0 && stride_a % 8 == 0 &&
                         stride_b % 8 == 0 && (int64_t)M * K * 2 < 0x7FFFFFFFLL &&
                         (int64_t)N * K * 2 < 0x7FFFFFFFLL;
+    g.partial = static_cast<float*>(workspace);
+    // Few rows: the kernel that reads B once with all of its loads in flight, unless a tile kernel is asked for by
+    // name or by the tuning table.
+    if ((is16 || dtype == MHIP_F32) && gemm_skinny_eligible(g, trans_a, is16 ? 2 : 4) && (!vec_ok || skinny_rows(M, N, K, is16)) &&
+        tune_int("MHIP_GEMM_TILE", 0) == 0 && tune_int("MHIP_GEMM_F32_MFMA", 1) == 1 &&
+        (!is16 || tuned_gemm_variant(g, batch, trans_a, trans_b, dtype) == 0))
+        return launch_gemm_skinny(s, g, batch, trans_b, dtype, workspace_bytes);
     if (vec_ok) {
-        if (dtype == MHIP_BF16) return pick_layout<bf16_t>(s, g, batch, trans_a, trans_b);
-        return pick_layout<f16_t>(s, g, batch, trans_a, trans_b);
+        if (dtype == MHIP_BF16) return pick_layout<bf16_t>(s, g, batch, trans_a, trans_b, workspace_bytes);
+        return pick_layout<f16_t>(s, g, batch, trans_a, trans_b, workspace_bytes);
     }
     switch (dtype) {
         case MHIP_F32:
@@ -682,4 +602,25 @@ extern "C" int mhip_gemm_residual(void* stream, const void* a, const void* b, co
                                   int trans_a, int trans_b, int activation, int dtype) {
     return gemm_entry(stream, a, b, bias, residual, c, M, N, K, batch, stride_a, stride_b, stride_c, trans_a, trans_b,
                       activation, dtype);
+}
+
+extern "C" int mhip_gemm_ws(void* stream, const void* a, const void* b, const void* bias, const void* residual, void* c,
+                            int64_t M, int64_t N, int64_t K, int64_t batch, int64_t stride_a, int64_t stride_b,
+                            int64_t stride_c, int trans_a, int trans_b, int activation, int dtype, void* workspace,
+                            int64_t workspace_bytes) {
+    if (workspace_bytes < 0 || (reinterpret_cast<uintptr_t>(workspace) & 15) != 0)
+        return fail(MHIP_ERR_INVALID_ARGUMENT, "mhip_gemm_ws: the workspace must be 16-byte aligned");
+    return gemm_entry(stream, a, b, bias, residual, c, M, N, K, batch, stride_a, stride_b, stride_c, trans_a, trans_b,
+                      activation, dtype, workspace_bytes > 0 ? workspace : nullptr, workspace ? workspace_bytes : 0);
+}
+
+extern "C" int64_t mhip_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b, int dtype) {
+    if (M <= 0 || N <= 0 || K <= 0 || batch != 1 || M > 0x7FFFFFFF || N > 0x7FFFFFFF || K > 0x7FFFFFFF) return 0;
+    const bool is16 = dtype == MHIP_BF16 || dtype == MHIP_F16;
+    if (!is16 && dtype != MHIP_F32) return 0;
+    const bool vec = is16 && (trans_a ? M : K) % 8 == 0 && (trans_b ? K : N) % 8 == 0;
+    if (!trans_a && M <= 64 && (!vec || skinny_rows(M, N, K, is16))) return gemm_skinny_workspace(M, N, K, batch, trans_b);
+    // (a large problem goes to the ring kernels, whose tiles fill the device)
+    if (!vec || (M > 192 && (double)M * N * batch >= 192.0 * 256 * 256)) return 0;
+    return gemm_mid_workspace(M, N, K, batch);
 }

@@ -24,6 +24,8 @@ struct GemmArgs {
     int tiles_m, tiles_n;
     const void* residual = nullptr;   // C's layout and batch stride; added after the activation (may alias c)
     int ldc = 0;                      // row stride of C and the residual in elements; 0 = N (gemm256.hip only: a column slice of a wider C)
+    float* partial = nullptr;         // split K: fp32 sums [split][M][N] go here (batch 1) and finish_split() makes C of them
+    int splits = 1;
     int stream_c = 0;                 // gemm256.hip: C is far larger than the L2s, store it with the streaming hint
 };
 

@@ -1,0 +1,135 @@
+// LDS tiles of 16-bit operands and the tile store, shared by the register-staged and the ring-staged
+// MFMA kernels.
+#pragma once
+#include "gemm_common.h"
+
+namespace mhip {
+
+// Swizzle of the 16-byte chunk index inside a 128-byte LDS row.  Rows r..r+15
+// (r % 16 == 0) map one chunk column onto 16 distinct bank groups.
+__device__ inline int swz(int row) { return ((row >> 1) ^ (row >> 4)) & 7; }
+
+__device__ inline uint32_t lds_off(int row, int chunk) {
+    return (uint32_t)(row * kRowBytes + ((chunk ^ swz(row)) << 4));
+}
+
+__device__ inline __amdgpu_buffer_rsrc_t make_rsrc(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+}
+
+// Buffer load of 16 bytes per lane straight into LDS: lane l lands at byte lds + 16 l (lds uniform, a
+// multiple of 16).  As inline assembly because the compiler puts a wait for ALL outstanding loads in
+// front of any LDS read that it cannot tell apart from the builtin's target, which is every read of
+// another stage of a ring; the kernels count their loads and wait themselves.  (M0 is a reserved register
+// that cannot be named as clobbered; nothing else in these kernels uses it.)
+__device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t rsrc, uint32_t lds, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(rsrc) : "memory");
+}
+// LDS address of a shared-memory pointer, as those loads take it.
+__device__ __forceinline__ uint32_t lds_address(const char* p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p;
+}
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
+// MFMA operand (32 mn x 16 k) for k-step `s` out of a k-major tile.
+__device__ inline u32x4 frag_kmajor(const char* tile, int row0, int s, int lane) {
+    return *reinterpret_cast<const u32x4*>(tile + lds_off(row0 + (lane & 31), 2 * s + (lane >> 5)));
+}
+// The wave's (32 TM) x (32 TN) sub-tile at (row0, col0) of C: bias, activation, rounding, residual, store.
+// `stage` is this wave's LDS area of 32 TM rows of 64 TN + 16 bytes.
+template <typename T, int TM, int TN>
+__device__ __forceinline__ void store_tile(const GemmArgs& g, const f32x16 (&acc)[TM][TN], char* stage, int row0, int col0, int64_t batch, int lane) {
+    constexpr int WTM = 32 * TM, WTN = 32 * TN;
+    const int lrow = lane & 31, lhalf = lane >> 5;
+    T* c = static_cast<T*>(g.c) + batch * g.sc;
+    const T* res = g.residual ? static_cast<const T*>(g.residual) + batch * g.sc : nullptr;
+    // Epilogue.  The MFMAs were issued as (B-fragment, A-fragment), so each
+    // 32x32 accumulator tile is held transposed: a lane owns row m = lrow and,
+    // in register group q = r/4, the four consecutive columns 8q + 4*lhalf + r%4.
+    const T* bias = static_cast<const T*>(g.bias);
+    const bool vec_store = (g.N % 8 == 0) && ((reinterpret_cast<uintptr_t>(c) & 15) == 0);
+    // Stage the wave's sub-tile in LDS as rounded 16-bit rows (padded by 16 bytes
+    // against bank conflicts); the rows then go out with lanes running along n, so
+    // every store instruction writes whole contiguous row segments.
+    constexpr int kRowPad = WTN * 2 + 16;
+    dispatch_act(g.act, [&](auto act_tag) {
+    constexpr int ACT = decltype(act_tag)::value;
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int nl = j * 32 + 8 * q + 4 * lhalf;          // column inside the wave tile
+            const int n = col0 + nl;
+            float bv[4] = {0.f, 0.f, 0.f, 0.f};
+            if (bias) {
+                if (vec_store && n < g.N) {
+                    const Pack4<T> t = __builtin_bit_cast(Pack4<T>, *reinterpret_cast<const u32x2*>(bias + n));
+#pragma unroll
+                    for (int e = 0; e < 4; e++) bv[e] = Elem<T>::to_f32(t.v[e]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (n + e < g.N) bv[e] = Elem<T>::to_f32(bias[n + e]);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < TM; i++) {
+                Pack4<T> o;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    float v = acc[i][j][4 * q + e] + bv[e];
+                    v = apply_act_c<ACT>(v);
+                    o.v[e] = Elem<T>::from_f32(v);
+                }
+                *reinterpret_cast<u32x2*>(stage + (i * 32 + lrow) * kRowPad + nl * 2) =
+                    __builtin_bit_cast(u32x2, o);
+            }
+        }
+    }
+    });
+    // each wave only re-reads what it wrote itself
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (vec_store) {
+        constexpr int kCpr = WTN / 8;                // 16-byte chunks per row
+        constexpr int kRowsPerPass = 64 / kCpr;
+        const int cc = lane % kCpr, rr = lane / kCpr;
+#pragma unroll
+        for (int p = 0; p < WTM / kRowsPerPass; p++) {
+            const int ml = p * kRowsPerPass + rr;
+            const int m = row0 + ml;
+            const int n = col0 + cc * 8;
+            if (m < g.M && n < g.N) {
+                u32x4 w = *reinterpret_cast<const u32x4*>(stage + ml * kRowPad + cc * 16);
+                if (res) w = add_chunk<T>(w, *reinterpret_cast<const u32x4*>(res + (int64_t)m * g.N + n));
+                *reinterpret_cast<u32x4*>(c + (int64_t)m * g.N + n) = w;
+            }
+        }
+    } else {
+        // rows of C are not 16-byte aligned (odd N): one element per lane, 64
+        // consecutive columns per store instruction
+        const uint16_t* st16 = reinterpret_cast<const uint16_t*>(stage);
+        uint16_t* c16 = reinterpret_cast<uint16_t*>(c);
+constexpr int kLanes = WTN < 64 ? WTN : 64, kRowsAtOnce = 64 / kLanes;
+#pragma unroll 4
+        for (int mb = 0; mb < WTM; mb += kRowsAtOnce) {
+            const int ml = mb + lane / kLanes, m = row0 + ml;
+            if (m >= g.M) break;
+#pragma unroll
+            for (int cb = 0; cb < WTN / kLanes; cb++) {
+                const int nl = cb * kLanes + lane % kLanes;
+                const int n = col0 + nl;
+                if (n < g.N) {
+                    T val = __builtin_bit_cast(T, st16[ml * (kRowPad / 2) + nl]);
+                    if (res) val = Elem<T>::from_f32(Elem<T>::to_f32(val) + Elem<T>::to_f32(res[(int64_t)m * g.N + n]));
+                    c16[(int64_t)m * g.N + n] = __builtin_bit_cast(uint16_t, val);
+                }
+            }
+        }
+    }
+}
+
+}  // namespace mhip

@@ -1,0 +1,321 @@
+// dot_general with few rows: C = act(A . op(B) + bias) (+ residual) for M <= 64 (a decode step, a short
+// prompt, a small batch), where the product costs nothing and the time is that of reading B once.
+//
+// A tile kernel leaves such a problem on a handful of workgroups ([4,4096] x [4096,4096]: 32 tiles of
+// 128 columns on 256 compute units, each walking K through LDS one load latency at a time).  Here
+//   * a workgroup owns a strip of 16 to 64 columns and ALL of K, its waves split K between them: every wave
+//     has a block of loads in flight from its first instruction on, and the partial sums meet in LDS;
+//   * B goes from memory straight to the operand registers, no LDS, no barrier in the loop.  The matrix
+//     instruction wants eight consecutive k of one column per lane.  Stored [N, K] that is one 16-byte
+//     load.  Stored [K, N] a lane loads VE neighbouring columns of its eight k rows, and one byte
+//     permute per register pairs two k of one column: lane i then owns columns VE*i .. VE*i + VE-1 of the
+//     strip, one per operand f, which only changes where the results go;
+//   * the product is formed transposed (B as first operand), rows of A beyond M are duplicates of the last
+//     row whose results are dropped, k beyond K reads zero through the buffer bounds.
+// fp32 operands take the same path on v_mfma_f32_16x16x4_f32; operands whose rows are not aligned for
+// vector loads (odd K or N) load element by element (VEC = false), still with every load in flight.
+#include <mutex>
+
+#include "gemm_common.h"
+
+namespace mhip {
+
+int launch_gemm_finish(hipStream_t s, const GemmArgs& g, int dtype);     // gemm_mid.hip
+
+namespace {
+
+template <typename T> struct Mfma16;
+template <> struct Mfma16<bf16_t> {
+    static constexpr int kKpl = 8;                   // consecutive k per lane and operand
+    typedef u32x4 frag;
+    __device__ static f32x4 run(frag b, frag a, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b), __builtin_bit_cast(bf16x8, a), c, 0, 0, 0);
+    }
+};
+template <> struct Mfma16<f16_t> {
+    static constexpr int kKpl = 8;
+    typedef u32x4 frag;
+    __device__ static f32x4 run(frag b, frag a, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, b), __builtin_bit_cast(f16x8, a), c, 0, 0, 0);
+    }
+};
+template <> struct Mfma16<float> {
+    static constexpr int kKpl = 4;                   // four issues of k = 4: lane group g supplies k = 4 g + p to issue p
+    typedef u32x4 frag;
+    __device__ static f32x4 run(frag b, frag a, f32x4 c) {
+#pragma unroll
+        for (int p = 0; p < 4; p++)
+            c = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(f32x4, b)[p], __builtin_bit_cast(f32x4, a)[p], c, 0, 0, 0);
+        return c;
+    }
+};
+
+__device__ inline __amdgpu_buffer_rsrc_t skinny_rsrc(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+}
+
+// 16 bytes of consecutive elements at element offset `off` of which `n` exist (n <= 0: none).
+template <typename T, bool VEC>
+__device__ inline u32x4 load_run(__amdgpu_buffer_rsrc_t r, int64_t off, int n) {
+    if (VEC) return __builtin_amdgcn_raw_buffer_load_b128(r, n > 0 ? (uint32_t)(off * (int)sizeof(T)) : kOob, 0, 0);
+    u32x4 v;
+    if (sizeof(T) == 4) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = __builtin_amdgcn_raw_buffer_load_b32(r, e < n ? (uint32_t)((off + e) * 4) : kOob, 0, 0);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const uint32_t lo = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, 2 * e < n ? (uint32_t)((off + 2 * e) * 2) : kOob, 0, 0);
+            const uint32_t hi = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, 2 * e + 1 < n ? (uint32_t)((off + 2 * e + 1) * 2) : kOob, 0, 0);
+            v[e] = lo | (hi << 16);
+        }
+    }
+    return v;
+}
+
+// VE consecutive elements (as dwords; one 16-bit pair per dword) of one row of B stored [K, N].
+template <typename T, int VE, bool VEC> struct RowPiece {
+    static constexpr int kDw = (int)(VE * sizeof(T) / 4);
+    uint32_t w[kDw];
+    __device__ void load(__amdgpu_buffer_rsrc_t r, int64_t off, int n) {
+        if (VEC) {
+            const uint32_t o = n > 0 ? (uint32_t)(off * (int)sizeof(T)) : kOob;
+            if (kDw == 1) w[0] = __builtin_amdgcn_raw_buffer_load_b32(r, o, 0, 0);
+            else {
+                const u32x2 t = __builtin_amdgcn_raw_buffer_load_b64(r, o, 0, 0);
+                w[0] = t.x; w[kDw - 1] = t.y;
+            }
+        } else if (sizeof(T) == 4) {
+#pragma unroll
+            for (int e = 0; e < kDw; e++) w[e] = __builtin_amdgcn_raw_buffer_load_b32(r, e < n ? (uint32_t)((off + e) * 4) : kOob, 0, 0);
+        } else {
+#pragma unroll
+            for (int e = 0; e < kDw; e++) {
+                const uint32_t lo = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, 2 * e < n ? (uint32_t)((off + 2 * e) * 2) : kOob, 0, 0);
+                const uint32_t hi = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, 2 * e + 1 < n ? (uint32_t)((off + 2 * e + 1) * 2) : kOob, 0, 0);
+                w[e] = lo | (hi << 16);
+            }
+        }
+    }
+};
+
+// NF = operands (groups of 16 columns) per strip, MT = groups of 16 rows, U = k steps loaded as one block.
+template <typename T, bool TB, bool VEC, int NF, int MT, int U, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(GemmArgs g) {
+    constexpr int KPL = Mfma16<T>::kKpl, KS = 4 * KPL;      // k per step
+    constexpr int VE = NF, NS = 16 * NF;                     // (stored [K, N]: NF consecutive columns per lane)
+    constexpr int kDw = (int)(VE * sizeof(T) / 4);
+    extern __shared__ __attribute__((aligned(16))) float part[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const int li = lane & 15, lg = lane >> 4;
+    const int n0 = blockIdx.x * NS;
+    const int64_t batch = blockIdx.y;
+    const T* a = static_cast<const T*>(g.a) + batch * g.sa;
+    const T* b = static_cast<const T*>(g.b) + batch * g.sb;
+    const __amdgpu_buffer_rsrc_t ra = skinny_rsrc(a, (uint32_t)((int64_t)g.M * g.lda * sizeof(T)));
+    const __amdgpu_buffer_rsrc_t rb = skinny_rsrc(b, (uint32_t)((int64_t)(TB ? g.N : g.K) * g.ldb * sizeof(T)));
+
+    // this workgroup's k steps (all of them, or one split's), and this wave's share of them
+    const int all_steps = (g.K + KS - 1) / KS, per_split = (all_steps + (int)gridDim.z - 1) / (int)gridDim.z;
+    const int first = (int)blockIdx.z * per_split, steps = min(all_steps - first, per_split), per = (steps + waves - 1) / waves;
+    const int s0 = first + wave * per, s1 = min(first + steps, s0 + per);
+    const int kend = min(g.K, s1 * KS);
+
+    uint32_t arow[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) arow[mt] = (uint32_t)(min(mt * 16 + li, g.M - 1) * g.lda);
+
+    f32x4 acc[NF][MT];
+#pragma unroll
+    for (int f = 0; f < NF; f++)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) acc[f][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    struct Block {
+        u32x4 a[U][MT];
+        u32x4 bt[TB ? U : 1][NF];                            // B stored [N, K]
+        RowPiece<T, VE, VEC> bn[TB ? 1 : U][KPL];            // B stored [K, N]
+    };
+    auto load = [&](Block& blk, int s) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int k = (s + u) * KS + lg * KPL;
+            if (TB) {
+#pragma unroll
+                for (int f = 0; f < NF; f++) {
+                    const int n = n0 + 16 * f + li;
+                    blk.bt[TB ? u : 0][f] = load_run<T, VEC>(rb, (int64_t)n * g.ldb + k, n < g.N ? kend - k : 0);
+                }
+            } else {
+                const int n = n0 + VE * li;
+#pragma unroll
+                for (int j = 0; j < KPL; j++)
+                    blk.bn[TB ? 0 : u][j].load(rb, (int64_t)(k + j) * g.ldb + n, k + j < kend ? g.N - n : 0);
+            }
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) blk.a[u][mt] = load_run<T, VEC>(ra, (int64_t)arow[mt] + k, kend - k);
+        }
+    };
+    auto multiply = [&](const Block& blk) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+#pragma unroll
+            for (int f = 0; f < NF; f++) {
+                u32x4 bf;
+                if (TB) bf = blk.bt[TB ? u : 0][f];
+                else if (sizeof(T) == 4) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) bf[j] = blk.bn[TB ? 0 : u][j].w[f < kDw ? f : 0];
+                } else {
+                    // column f of rows 2j and 2j + 1 as one register: bytes of the second operand are 0..3
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        bf[j] = __builtin_amdgcn_perm(blk.bn[TB ? 0 : u][(2 * j + 1) % KPL].w[(f / 2) % kDw], blk.bn[TB ? 0 : u][(2 * j) % KPL].w[(f / 2) % kDw],
+                                                      (f & 1) ? 0x07060302u : 0x05040100u);
+                }
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++) acc[f][mt] = Mfma16<T>::run(bf, blk.a[u][mt], acc[f][mt]);
+            }
+        }
+    };
+    if (s0 < s1) {
+        Block cur;
+        load(cur, s0);
+        for (int s = s0; s < s1; s += U) {
+            Block nxt;
+            if (s + U < s1) load(nxt, s + U);
+            multiply(cur);
+            if (s + U < s1) cur = nxt;
+        }
+    }
+
+    // ---- the waves' partial sums, in the accumulators' own layout: lane (li, lg) holds row 16 mt + li and,
+    // in its four registers, operand rows 4 lg .. 4 lg + 3
+#pragma unroll
+    for (int f = 0; f < NF; f++)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+            *reinterpret_cast<f32x4*>(part + (((wave * NF + f) * MT + mt) * 64 + lane) * 4) = acc[f][mt];
+    __syncthreads();
+    const T* bias = static_cast<const T*>(g.bias);
+    const T* res = g.residual ? static_cast<const T*>(g.residual) + batch * g.sc : nullptr;
+    T* c = static_cast<T*>(g.c) + batch * g.sc;
+    auto finish = [&](auto act_tag) {
+        constexpr int ACT = decltype(act_tag)::value;
+        const int total = min(g.M, 16 * MT) * NS;
+        for (int idx = threadIdx.x; idx < total; idx += blockDim.x) {
+            const int m = idx / NS, nl = idx % NS, n = n0 + nl;
+            if (n >= g.N) continue;
+            const int f = TB ? nl / 16 : nl % VE, i = TB ? nl % 16 : nl / VE;
+            const float* p = part + ((f * MT + m / 16) * 64 + (i >> 2) * 16 + (m & 15)) * 4 + (i & 3);
+            float v = 0.f;
+            for (int w = 0; w < waves; w++) v += p[w * (NF * MT * 256)];
+            if (g.partial) {
+                g.partial[((int64_t)blockIdx.z * g.M + m) * g.N + n] = v;
+                continue;
+            }
+            if (bias) v += Elem<T>::to_f32(bias[n]);
+            v = sizeof(T) == 4 ? apply_act(v, ACT) : apply_act_c<ACT>(v);
+            T o = Elem<T>::from_f32(v);
+            const int64_t at = (int64_t)m * g.N + n;
+            // (second rounding on purpose: the same result as a separate add over the stored C)
+            if (res) o = Elem<T>::from_f32(Elem<T>::to_f32(o) + Elem<T>::to_f32(res[at]));
+            c[at] = o;
+        }
+    };
+    dispatch_act(g.act, finish);
+}
+
+template <typename T, bool TB, bool VEC, int NF, int MT, int U, int WAVES = 8>
+int launch_one(hipStream_t s, const GemmArgs& g, int64_t batch) {
+    constexpr int KS = 4 * Mfma16<T>::kKpl;
+    auto kern = gemm_skinny_kernel<T, TB, VEC, NF, MT, U, WAVES>;
+    constexpr int kLds = WAVES * NF * MT * 1024;
+    if (kLds > 64 * 1024) {
+        static std::once_flag once;
+        static hipError_t err = hipSuccess;
+        std::call_once(once, [&] { err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kLds); });
+        if (err != hipSuccess) return fail(MHIP_ERR_LAUNCH, "gemm: cannot reserve %d bytes of LDS: %s", kLds, hipGetErrorString(err));
+    }
+    // a wave takes at least one block of loads
+    const int steps = ((g.K + KS - 1) / KS + g.splits - 1) / g.splits, want = (steps + U - 1) / U;
+    const int waves = want < 1 ? 1 : want > WAVES ? WAVES : want;
+    const int64_t strips = (g.N + 16 * NF - 1) / (16 * NF);
+    if (strips > 0x7FFFFFFFLL || batch > 65535) return fail(MHIP_ERR_UNSUPPORTED, "gemm: grid too large");
+    hipLaunchKernelGGL(kern, dim3((unsigned)strips, (unsigned)batch, (unsigned)g.splits), dim3(64 * waves), waves * NF * MT * 1024, s, g);
+    return check_launch("gemm_skinny");
+}
+
+// Strip width: narrow strips put a small weight matrix on as many compute units as it has columns for, wide
+// ones read whole 128-byte lines per row.  Stored [K, N], us narrow / wide: [4,4096] x [4096,4096] 14.4 / 13.0,
+// [4,3072] x [3072,768] 5.8 / 9.4.  Stored [N, K] every strip reads whole lines and the wide one only saves reads
+// of A: [16,8192] x [8192,16384] 67.7 / 62.9, [4,768] x [768,50304] 16.1 / 17.4.
+bool wide_strips(int64_t N, int64_t K, int64_t batch, bool tb) {
+    const int64_t strips = (N + 63) / 64 * batch;
+    return tb ? strips >= 128 && K >= 2048 : strips >= 128 || (strips >= 64 && K >= 2048);
+}
+
+// K split over the grid as well (fp32 sums in a workspace, one more launch) while that leaves every workgroup
+// 2048 k and at most one of them per compute unit: [4,4096] x [4096,4096] 13.0 -> 10.3 us,
+// [28,6384] x [6384,688] 17.4 -> 9.2.
+int skinny_splits(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b) {
+    if (batch != 1 || M * N > (1 << 20)) return 1;
+    const int64_t width = wide_strips(N, K, 1, trans_b != 0) ? (trans_b ? 32 : 64) : (trans_b ? 16 : 32);
+    const int64_t room = 256 / ((N + width - 1) / width), want = K / 2048 + (K % 2048 > 1024);
+    const int64_t n = room < want ? room : want;
+    return n < 2 ? 1 : n > 8 ? 8 : (int)n;
+}
+
+template <typename T, bool TB, bool VEC>
+int launch_shape(hipStream_t s, const GemmArgs& g, int64_t batch) {
+    constexpr bool k16 = sizeof(T) == 2;
+    const bool wide = wide_strips(g.N, g.K, batch, TB);
+    if (g.M <= 16) {
+        if (wide) return k16 || TB ? launch_one<T, TB, VEC, TB ? 2 : 4, 1, 2>(s, g, batch) : launch_one<T, TB, VEC, 2, 1, 2>(s, g, batch);
+        return launch_one<T, TB, VEC, TB ? 1 : k16 ? 2 : 1, 1, 4>(s, g, batch);
+    }
+    if (g.M <= 32) {
+        if (wide) return k16 || TB ? launch_one<T, TB, VEC, TB ? 2 : 4, 2, 2>(s, g, batch) : launch_one<T, TB, VEC, 2, 2, 2>(s, g, batch);
+        return launch_one<T, TB, VEC, TB ? 1 : k16 ? 2 : 1, 2, 2>(s, g, batch);
+    }
+    if (wide) return k16 || TB ? launch_one<T, TB, VEC, TB ? 2 : 4, 4, 1>(s, g, batch) : launch_one<T, TB, VEC, 2, 4, 1>(s, g, batch);
+    return launch_one<T, TB, VEC, TB ? 1 : k16 ? 2 : 1, 4, 2>(s, g, batch);
+}
+
+int dtype_launch(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_b, int dtype) {
+    const int per16 = dtype == MHIP_F32 ? 4 : 8;
+    const bool vec = g.lda % per16 == 0 && g.ldb % per16 == 0 && g.sa % per16 == 0 && g.sb % per16 == 0 &&
+                     ((reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.b)) & 15) == 0;
+#define MHIP_SKINNY(T)                                                                                              \
+    (vec ? (trans_b ? launch_shape<T, true, true>(s, g, batch) : launch_shape<T, false, true>(s, g, batch))         \
+         : (trans_b ? launch_shape<T, true, false>(s, g, batch) : launch_shape<T, false, false>(s, g, batch)))
+    switch (dtype) {
+        case MHIP_F32: return MHIP_SKINNY(float);
+        case MHIP_BF16: return MHIP_SKINNY(bf16_t);
+        default: return MHIP_SKINNY(f16_t);
+    }
+#undef MHIP_SKINNY
+}
+
+}  // namespace
+
+// What this kernel takes: A stored [M, K], at most 64 rows, operands that one buffer descriptor spans.
+bool gemm_skinny_eligible(const GemmArgs& g, int trans_a, int elem_bytes) {
+    return !trans_a && g.M <= 64 && g.K > 0 && g.ldc == 0 && (int64_t)g.M * g.lda * elem_bytes < 0x7FFFFFFFLL &&
+           ((int64_t)g.N + 64) * g.K * elem_bytes < 0x7FFFFFFFLL && ((int64_t)g.K + 64) * g.N * elem_bytes < 0x7FFFFFFFLL;
+}
+
+int64_t gemm_skinny_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b) {
+    const int n = skinny_splits(M, N, K, batch, trans_b);
+    return n == 1 ? 0 : M * N * 4 * n;
+}
+
+int launch_gemm_skinny(hipStream_t s, GemmArgs g, int64_t batch, int trans_b, int dtype, int64_t workspace_bytes) {
+    g.splits = g.partial ? skinny_splits(g.M, g.N, g.K, batch, trans_b) : 1;
+    if ((int64_t)g.M * g.N * 4 * g.splits > workspace_bytes) g.splits = 1;
+    if (g.splits == 1) g.partial = nullptr;
+    const int st = dtype_launch(s, g, batch, trans_b, dtype);
+    return st != MHIP_OK || g.splits == 1 ? st : launch_gemm_finish(s, g, dtype);
+}
+
+}  // namespace mhip

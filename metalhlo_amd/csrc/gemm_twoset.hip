@@ -464,7 +464,22 @@ __device__ __forceinline__ void store_tile192(f32x16 (&acc)[6], char* smem, cons
     });
 }
 
-template <typename T, bool TA, bool TB>
+// Split K: the sub-tile's fp32 sums in the accumulators' own layout (what gemm_finish_tiles_kernel reads:
+// block (i, j) of wave w of tile t, register group q, 1 KB per store).
+__device__ __forceinline__ void store_partial192(f32x16 (&acc)[6], float* p, int tile) {
+    f32x4* d = reinterpret_cast<f32x4*>(p) + ((int64_t)tile * 4 + (threadIdx.x >> 6)) * 6 * 256 + (threadIdx.x & 63);
+    static_for<24>([&](auto x_tag) __attribute__((always_inline)) {
+        constexpr int blk = decltype(x_tag)::value / 4, q = decltype(x_tag)::value % 4;
+        f32x4 v;
+        static_for<4>([&](auto e_tag) { v[decltype(e_tag)::value] = acc_value(acc[blk][4 * q + decltype(e_tag)::value]); });
+        d[decltype(x_tag)::value * 64] = v;
+        __builtin_amdgcn_sched_barrier(0);
+    });
+}
+
+// SPLIT: the grid's second axis is the part of K (g.splits of them, whole stages) instead of the batch, and
+// the tile's sums go to g.partial.
+template <typename T, bool TA, bool TB, bool SPLIT>
 __global__ __launch_bounds__(256) void gemm192_kernel(GemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     using LA = typename std::conditional<TA, MnMajor<128>, KMajor>::type;
@@ -473,13 +488,17 @@ __global__ __launch_bounds__(256) void gemm192_kernel(GemmArgs g) {
     int tm, tn;
     tile_of(blockIdx.x, gridDim.x, g.tiles_m, g.tiles_n, tm, tn);
     const int m0 = tm * 128, n0 = tn * 192;
-    const int64_t batch = blockIdx.y;
-    const char* a = reinterpret_cast<const char*>(static_cast<const T*>(g.a) + batch * g.sa);
-    const char* b = reinterpret_cast<const char*>(static_cast<const T*>(g.b) + batch * g.sb);
+    const int64_t batch = SPLIT ? 0 : blockIdx.y;
+    const int stages = g.K / 32, per = SPLIT ? (stages + g.splits - 1) / g.splits : stages;
+    const int first = SPLIT ? (int)blockIdx.y * per : 0, kt = min(per, stages - first);
+    // (elements of a k-contiguous / a k-slow operand in front of this part)
+    const int64_t skip_a = (int64_t)first * 32 * (TA ? g.lda : 1), skip_b = (int64_t)first * 32 * (TB ? 1 : g.ldb);
+    const char* a = reinterpret_cast<const char*>(static_cast<const T*>(g.a) + batch * g.sa + skip_a);
+    const char* b = reinterpret_cast<const char*>(static_cast<const T*>(g.b) + batch * g.sb + skip_b);
     T* c = static_cast<T*>(g.c) + batch * g.sc;
     const T* res = g.residual ? static_cast<const T*>(g.residual) + batch * g.sc : nullptr;
-    const uint32_t a_bytes = (uint32_t)(((int64_t)((TA ? g.K : g.M) - 1) * g.lda + (TA ? g.M : g.K)) * 2);
-    const uint32_t b_bytes = (uint32_t)(((int64_t)((TB ? g.N : g.K) - 1) * g.ldb + (TB ? g.K : g.N)) * 2);
+    const uint32_t a_bytes = (uint32_t)(((int64_t)((TA ? g.K : g.M) - 1) * g.lda + (TA ? g.M : g.K) - skip_a) * 2);
+    const uint32_t b_bytes = (uint32_t)(((int64_t)((TB ? g.N : g.K) - 1) * g.ldb + (TB ? g.K : g.N) - skip_b) * 2);
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
@@ -500,13 +519,14 @@ __global__ __launch_bounds__(256) void gemm192_kernel(GemmArgs g) {
 
     f32x16 acc[6];
     main_loop192<T, TA, TB>(acc, ra, rb, goff, rsa, rsb, LA::pass_stride(g.lda), LB::pass_stride(g.ldb),
-                            LA::stage_stride(g.lda), LB::stage_stride(g.ldb), m0b, (uint32_t)(g.K / 32));
-    store_tile192<T>(acc, smem, g, c, res, m0, n0);
+                            LA::stage_stride(g.lda), LB::stage_stride(g.ldb), m0b, (uint32_t)kt);
+    if constexpr (SPLIT) store_partial192(acc, g.partial, ((int)blockIdx.y * g.tiles_m + tm) * g.tiles_n + tn);
+    else store_tile192<T>(acc, smem, g, c, res, m0, n0);
 }
 
-template <typename T, bool TA, bool TB>
+template <typename T, bool TA, bool TB, bool SPLIT>
 int launch192(hipStream_t s, GemmArgs g, int64_t batch) {
-    auto kern = gemm192_kernel<T, TA, TB>;
+    auto kern = gemm192_kernel<T, TA, TB, SPLIT>;
     static std::once_flag once;
     static hipError_t attr_err = hipSuccess;
     std::call_once(once, [&] {
@@ -518,17 +538,17 @@ int launch192(hipStream_t s, GemmArgs g, int64_t batch) {
                     hipGetErrorString(attr_err));
     g.tiles_m = (g.M + 127) / 128;
     g.tiles_n = (g.N + 191) / 192;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(g.tiles_m * g.tiles_n), (unsigned)batch), dim3(256),
+    hipLaunchKernelGGL(kern, dim3((unsigned)(g.tiles_m * g.tiles_n), (unsigned)(SPLIT ? g.splits : batch)), dim3(256),
                        k192Smem, s, g);
     return check_launch("gemm192");
 }
 
 template <typename T>
 int layout192(hipStream_t s, const GemmArgs& g, int64_t batch, int ta, int tb) {
-    if (!ta && !tb) return launch192<T, false, false>(s, g, batch);
-    if (!ta && tb) return launch192<T, false, true>(s, g, batch);
-    if (ta && !tb) return launch192<T, true, false>(s, g, batch);
-    return launch192<T, true, true>(s, g, batch);
+    if (!ta && !tb) return g.partial ? launch192<T, false, false, true>(s, g, batch) : launch192<T, false, false, false>(s, g, batch);
+    if (!ta && tb) return g.partial ? launch192<T, false, true, true>(s, g, batch) : launch192<T, false, true, false>(s, g, batch);
+    if (ta && !tb) return g.partial ? launch192<T, true, false, true>(s, g, batch) : launch192<T, true, false, false>(s, g, batch);
+    return g.partial ? launch192<T, true, true, true>(s, g, batch) : launch192<T, true, true, false>(s, g, batch);
 }
 
 // ---- the 256x288 tile --------------------------------------------------------------------------------

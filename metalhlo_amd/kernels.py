@@ -142,16 +142,14 @@ def matmul(a, b, bias=None, activation: str = "none", trans_a: bool = False,
         raise ValueError("bias must be [N] of the operand dtype")
     if out is None:
         out = torch.empty(out_lead + (N,), dtype=a.dtype, device=a.device)
-    if residual is None:
-        _lib.check(lib.mhip_gemm(_stream(), a2.data_ptr(), b.data_ptr(), _ptr(bias), out.data_ptr(),
-                                 M, N, K, batch, sa, sb, M * N, int(trans_a), int(trans_b),
-                                 ACTIVATION_CODE[activation], _code(a)))
-    else:
-        if residual.numel() != out.numel() or residual.dtype != out.dtype:
-            raise ValueError("residual must have the result's size and dtype")
-        _lib.check(lib.mhip_gemm_residual(_stream(), a2.data_ptr(), b.data_ptr(), _ptr(bias), residual.data_ptr(),
-                                          out.data_ptr(), M, N, K, batch, sa, sb, M * N, int(trans_a), int(trans_b),
-                                          ACTIVATION_CODE[activation], _code(a)))
+    if residual is not None and (residual.numel() != out.numel() or residual.dtype != out.dtype):
+        raise ValueError("residual must have the result's size and dtype")
+    # (partial sums of a split K: memory of the current stream's, or a capturing graph's own)
+    nbytes = lib.mhip_gemm_workspace(M, N, K, batch, int(trans_a), int(trans_b), _code(a))
+    work = torch.empty(nbytes, dtype=torch.uint8, device=a.device) if nbytes else None
+    _lib.check(lib.mhip_gemm_ws(_stream(), a2.data_ptr(), b.data_ptr(), _ptr(bias), _ptr(residual), out.data_ptr(),
+                                M, N, K, batch, sa, sb, M * N, int(trans_a), int(trans_b),
+                                ACTIVATION_CODE[activation], _code(a), _ptr(work), nbytes))
     return out
 
 

@@ -1,0 +1,75 @@
+"""GPU parity of the GEMM kernels for problems with few rows or few tiles (gemm_skinny.hip,
+gemm_mid.hip): edges of their tiles, remainders, operands without vector alignment, split K.
+
+Bound: a product of K terms summed in fp32 is off by at most K 2^-24 of sum |a||b|; the result is then
+rounded once to its type (unit roundoff 2^-8 for bf16's 8-bit significand, 2^-11 for f16's 11), twice with a
+residual."""
+import numpy as np
+import pytest
+import torch
+
+from tests.util import NAME, as_f64, to_dev
+
+pytestmark = pytest.mark.gpu
+ROUNDOFF = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}
+
+
+def _check(M, N, K, dtype, ta, tb, residual, seed=7, batch=()):
+    from metalhlo_amd import kernels
+    rng = np.random.default_rng(seed)
+    a = to_dev(rng.standard_normal(batch + ((K, M) if ta else (M, K))), dtype)
+    b = to_dev(rng.standard_normal(batch + ((N, K) if tb else (K, N))), dtype)
+    bias = None if batch else to_dev(rng.standard_normal(N), dtype)
+    r = to_dev(rng.standard_normal(batch + (M, N)), dtype) if residual else None
+    guard = torch.full((int(np.prod(batch + (M,))) * N + 64,), float("nan"), dtype=dtype, device="cuda")
+    out = guard[:-64].view(batch + (M, N))
+    kernels.matmul(a, b, bias=bias, activation="relu", trans_a=ta, trans_b=tb, residual=r, out=out)
+    A, B = as_f64(a), as_f64(b)
+    A, B = (np.swapaxes(A, -1, -2) if ta else A), (np.swapaxes(B, -1, -2) if tb else B)
+    e = A @ B + (0 if bias is None else as_f64(bias))
+    fp32 = (K + 2) * 2.0 ** -24 * (np.abs(A) @ np.abs(B) + (0 if bias is None else np.abs(as_f64(bias))))
+    e = np.maximum(e, 0)
+    bound = fp32 + ROUNDOFF[dtype] * (np.abs(e) + fp32)
+    if residual:
+        e = e + as_f64(r)
+        bound = bound + ROUNDOFF[dtype] * (np.abs(e) + bound)
+    assert np.all(np.abs(as_f64(out) - e) <= bound + 1e-30), (M, N, K, dtype, ta, tb)
+    assert torch.isnan(guard[-64:]).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=lambda d: NAME[d])
+@pytest.mark.parametrize("tb", [False, True], ids=["nn", "nt"])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (1, 64, 8), (15, 31, 33), (16, 40, 264), (17, 4104, 2056), (32, 520, 6400), (33, 50, 100), (64, 129, 1027),
+                                   (4, 4096, 4096), (16, 8200, 72)], ids=lambda v: str(v))
+def test_few_rows(M, N, K, tb, dtype):
+    _check(M, N, K, dtype, False, tb, residual=M % 2 == 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=lambda d: NAME[d])
+@pytest.mark.parametrize("layout", [(False, False), (False, True), (True, False), (True, True)], ids=["nn", "nt", "tn", "tt"])
+@pytest.mark.parametrize("M,N,K", [(40, 8, 8), (72, 64, 136), (136, 136, 1000), (192, 264, 3000), (200, 392, 264), (264, 520, 4104), (768, 1536, 4096), (1000, 1000, 72)],
+                         ids=lambda v: str(v))
+def test_few_tiles(M, N, K, layout, dtype):
+    _check(M, N, K, dtype, *layout, residual=N % 16 == 8)
+
+
+def test_few_tiles_batched():
+    _check(72, 200, 136, torch.bfloat16, False, False, True, batch=(5,))
+    _check(20, 77, 45, torch.float32, False, True, True, batch=(3,))
+
+
+def test_splitting_needs_its_workspace(lib):
+    """Without the workspace the same problem runs unsplit; a misaligned one is refused."""
+    M, N, K = 768, 1536, 8192
+    need = lib.mhip_gemm_workspace(M, N, K, 1, 1, 0, 3)
+    assert need > 0 and lib.mhip_gemm_workspace(4096, 4096, 4096, 1, 0, 0, 3) == 0
+    a, b = (torch.randn(K, n, device="cuda").bfloat16() for n in (M, N))
+    c = [torch.empty(M, N, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    args = lambda out: (torch.cuda.current_stream().cuda_stream, a.data_ptr(), b.data_ptr(), None, None, out.data_ptr(), M, N, K, 1, 0, 0, M * N, 1, 0, 0, 3)
+    assert lib.mhip_gemm_ws(*args(c[0]), ws.data_ptr(), need) == 0
+    assert lib.mhip_gemm_ws(*args(c[1]), None, 0) == 0
+    assert lib.mhip_gemm_ws(*args(c[1]), ws.data_ptr() + 8, need - 8) == 1
+    e = a.double().t().cpu() @ b.double().cpu()
+    for out in c:        # K 2^-24 sum |a||b| is below 2^-8 sqrt(K) here; one rounding to bf16
+        assert ((out.double().cpu() - e).abs() <= 2.0 ** -8 * (e.abs() + K ** 0.5)).all()
