@@ -99,6 +99,19 @@ def load() -> C.CDLL:
     return lib
 
 
+def load_native():
+    """The CPython extension lib/_native.so (csrc/python/native.cpp)."""
+    import importlib.util
+    path = os.path.join(HERE, "lib", "_native.so")
+    if not os.path.exists(path):
+        raise ImportError(f"{path} is not built; run `python -m metalhlo_amd.build`")
+    spec = importlib.util.spec_from_file_location("metalhlo_amd._native", path)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    module.bind(MhipError)
+    return module
+
+
 class MhipError(RuntimeError):
     def __init__(self, code: int, msg: str):
         super().__init__(f"mhip status {code}: {msg}")

@@ -128,9 +128,28 @@ def build_host(verbose: bool = True) -> list:
     return outs
 
 
+def build_native(verbose: bool = True) -> str:
+    """The CPython extension behind metalhlo_amd.kernels (csrc/python/native.cpp), against the installed torch."""
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension
+    out = os.path.join(LIBDIR, "_native.so")
+    inc = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include"]
+    libs = cpp_extension.library_paths()
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+          "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), *[a for i in inc for a in ("-isystem", i)],
+          os.path.join(CSRC, "python", "native.cpp"), "-o", out, "-L", LIBDIR, "-lmetalhlo_hip",
+          *[a for d in libs for a in ("-L", d, "-Wl,-rpath," + d)], "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
+          "-Wl,-rpath,$ORIGIN"])
+    if verbose:
+        print("  link ", os.path.relpath(out, ROOT), flush=True)
+    return out
+
+
 def build_all(verbose: bool = True):
-    """The product: the HIP kernel library and the host libraries over it."""
+    """The product: the HIP kernel library, the host libraries and the Python binding over it."""
     build_kernels(verbose)
+    build_native(verbose)
     build_host(verbose)
 
 

@@ -21,6 +21,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <string>
@@ -40,6 +41,7 @@ struct Entry { std::string choice; float us; };
 std::mutex g_mu;
 std::map<std::string, Entry> g_table;     // "<op> <device> <problem...>" -> choice
 bool g_env_loaded = false;
+std::atomic<uint64_t> g_generation{1};    // raised whenever the table changes
 thread_local int g_forced_gemm = 0;
 thread_local int g_forced_attention = 0;
 
@@ -85,11 +87,13 @@ std::string attention_key(int dt, int64_t bh, int64_t Sq, int64_t Skv, int64_t D
                (long long)D, causal ? 1 : 0);
 }
 
+bool gemm_variant_exists(int v) { return v == 64 || v == 128 || v == 256 || (v >= 2560 && v <= 2570); }
+
 bool valid_choice(const char* line, const std::string& choice) {
     int a = 0, b = 0, c = 0, d = 0;
     if (!strncmp(line, "gemm ", 5)) {
         const int v = atoi(choice.c_str());
-        return v == 128 || v == 256 || (v >= 2560 && v <= 2570);
+        return gemm_variant_exists(v);
     }
     if (!strncmp(line, "row ", 4))
         return sscanf(choice.c_str(), "%d %d %d %d", &a, &b, &c, &d) == 4 && (a == 1 || a == 2) && (b == 1 || b == 2) &&
@@ -116,6 +120,7 @@ int load_file(const char* path, bool quiet) {
             st = quiet ? MHIP_OK : fail(MHIP_ERR_INVALID_ARGUMENT, "tuning: malformed line in %s: %s", path, line);
             break;
         }
+        g_generation++;
         g_table[std::string(line, eq - line)] = Entry{std::string(eq + 3, at - eq - 3), us};
     }
     fclose(f);
@@ -162,7 +167,33 @@ bool lookup(const std::string& key, std::string* choice) {
 
 void record(const std::string& key, const std::string& choice, float us) {
     std::lock_guard<std::mutex> lk(g_mu);
+    g_generation++;
     g_table[key] = Entry{choice, us};
+}
+
+// What the table said about a problem, so that a launch does not build and look up its text key again (0.6 us
+// of the host time of a small operator): 64 slots per thread, dropped when the table or the device changes.
+template <typename V>
+struct Remembered {
+    struct Slot { uint64_t generation = 0; int64_t key[8]; V value; };
+    Slot slots[64];
+    Slot& find(const int64_t (&key)[8]) {
+        uint64_t h = 0;
+        for (int64_t k : key) h = (h ^ (uint64_t)k) * 0x9E3779B97F4A7C15ull;
+        return slots[h >> 58];
+    }
+    static bool same(const Slot& s, const int64_t (&key)[8]) {
+        return s.generation == g_generation.load(std::memory_order_relaxed) && memcmp(s.key, key, sizeof key) == 0;
+    }
+    static void keep(Slot& s, const int64_t (&key)[8], uint64_t generation, const V& v) {
+        s.generation = generation;
+        memcpy(s.key, key, sizeof key);
+        s.value = v;
+    }
+};
+int current_device() {
+    int dev = 0;
+    return hipGetDevice(&dev) == hipSuccess ? dev : -1;
 }
 
 struct Timer {
@@ -194,28 +225,52 @@ struct Timer {
 // Variant a tuned entry (or a running tuning pass) prescribes for this problem; 0 = none.
 int tuned_gemm_variant(const GemmArgs& g, int64_t batch, int ta, int tb, int dtype) {
     if (g_forced_gemm) return g_forced_gemm;
+    static thread_local Remembered<int> memory;
+    const int64_t key[8] = {g.M, g.N, g.K, batch, ta, tb, dtype, current_device()};
+    auto& slot = memory.find(key);
+    if (memory.same(slot, key)) return slot.value;
     std::string c;
-    if (!have_entries() || !lookup(gemm_key(g.M, g.N, g.K, batch, ta, tb, dtype), &c)) return 0;
-    const int v = atoi(c.c_str());
-    return (v == 128 || v == 256 || (v >= 2560 && v <= 2570)) ? v : 0;
+    const bool any = have_entries();
+    const uint64_t generation = g_generation;
+    int v = any && lookup(gemm_key(g.M, g.N, g.K, batch, ta, tb, dtype), &c) ? atoi(c.c_str()) : 0;
+    if (!gemm_variant_exists(v)) v = 0;
+    memory.keep(slot, key, generation, v);
+    return v;
 }
 
 bool tuned_row_launch(int op, int dtype, int64_t rows, int64_t cols, bool has_gamma, bool has_beta, RowLaunch* out) {
-    std::string c;
-    if (!have_entries() || !lookup(row_key(op, dtype, rows, cols, has_gamma, has_beta), &c)) return false;
-    RowLaunch r;
-    if (sscanf(c.c_str(), "%d %d %d %d", &r.kind, &r.r, &r.ordered, &r.per_cu) != 4) return false;
-    if ((r.kind != 1 && r.kind != 2) || r.r < 1 || r.r > 2 || r.ordered < 0 || r.ordered > 1 || r.per_cu < 0 || r.per_cu > 64) return false;
-    *out = r;
+    static thread_local Remembered<RowLaunch> memory;             // (kind 0: no entry)
+    const int64_t key[8] = {op, dtype, rows, cols, has_gamma, has_beta, 0, current_device()};
+    auto& slot = memory.find(key);
+    if (!memory.same(slot, key)) {
+        std::string c;
+        RowLaunch r;
+        const bool any = have_entries();
+        const uint64_t generation = g_generation;
+        if (!any || !lookup(row_key(op, dtype, rows, cols, has_gamma, has_beta), &c) ||
+            sscanf(c.c_str(), "%d %d %d %d", &r.kind, &r.r, &r.ordered, &r.per_cu) != 4 || (r.kind != 1 && r.kind != 2) || r.r < 1 ||
+            r.r > 2 || r.ordered < 0 || r.ordered > 1 || r.per_cu < 0 || r.per_cu > 64)
+            r = RowLaunch();
+        memory.keep(slot, key, generation, r);
+    }
+    if (!slot.value.kind) return false;
+    *out = slot.value;
     return true;
 }
 
 int tuned_attention_variant(int dtype, int64_t batch_heads, int64_t Sq, int64_t Skv, int64_t D, bool causal) {
     if (g_forced_attention) return g_forced_attention;
+    static thread_local Remembered<int> memory;
+    const int64_t key[8] = {dtype, batch_heads, Sq, Skv, D, causal, 0, current_device()};
+    auto& slot = memory.find(key);
+    if (memory.same(slot, key)) return slot.value;
     std::string c;
-    if (!have_entries() || !lookup(attention_key(dtype, batch_heads, Sq, Skv, D, causal), &c)) return 0;
-    const int v = atoi(c.c_str());
-    return v >= 1 && v <= 3 ? v : 0;
+    const bool any = have_entries();
+    const uint64_t generation = g_generation;
+    int v = any && lookup(attention_key(dtype, batch_heads, Sq, Skv, D, causal), &c) ? atoi(c.c_str()) : 0;
+    if (v < 1 || v > 3) v = 0;
+    memory.keep(slot, key, generation, v);
+    return v;
 }
 
 }  // namespace mhip
@@ -225,10 +280,14 @@ using namespace mhip;
 // GEMM candidates a problem can run (the validity filter: shape, alignment, LDS and tile count rules of each kernel).
 static std::vector<int> gemm_candidates(const GemmArgs& g, int64_t batch, int trans_a, int trans_b, int dtype) {
     std::vector<int> out;
-    for (int v : {128, 256, 2560, 2561, 2562, 2563, 2564, 2565, 2566, 2567, 2568, 2569, 2570}) {
+    // (64: the kernels for few rows and few tiles, where they are the default)
+    const bool tiles_fill = g.M > 192 && (gemm256_eligible(g, batch, trans_a, trans_b, dtype) || gemm256_eligible(g, batch, trans_a, trans_b, dtype, 128) ||
+                                          gemm256_eligible(g, batch, trans_a, trans_b, dtype, 192));
+    for (int v : {64, 128, 256, 2560, 2561, 2562, 2563, 2564, 2565, 2566, 2567, 2568, 2569, 2570}) {
         if ((v == 2560 || v == 2566) && !gemm256_eligible(g, batch, trans_a, trans_b, dtype)) continue;
         if ((v == 2561 || v == 2564 || v == 2565 || v == 2568) && !gemm256_eligible(g, batch, trans_a, trans_b, dtype, 128)) continue;
         if (v == 2570 && !(gemm256_eligible(g, batch, trans_a, trans_b, dtype, 288) && gemm384_activation_ok(g.act))) continue;
+        if (v == 64 && tiles_fill) continue;
         if (v == 2569 && !gemm256_eligible(g, batch, trans_a, trans_b, dtype, 192)) continue;
         if (v == 2567 && !(gemm256_eligible(g, batch, trans_a, trans_b, dtype, 384) && gemm384_activation_ok(g.act))) continue;
         if (v == 2562 && !gemm_stream_eligible(g, batch, trans_a, trans_b, dtype)) continue;
@@ -338,6 +397,7 @@ extern "C" int mhip_tuning_set_gemm(int64_t M, int64_t N, int64_t K, int64_t bat
     const std::string key = gemm_key(M, N, K, batch, trans_a, trans_b, dtype);
     if (variant == 0) {
         std::lock_guard<std::mutex> lk(g_mu);
+        g_generation++;
         g_table.erase(key);
         g_env_loaded = true;
         return MHIP_OK;
@@ -454,6 +514,7 @@ extern "C" int mhip_tuning_load(const char* path) {
 
 extern "C" void mhip_tuning_clear(void) {
     std::lock_guard<std::mutex> lk(g_mu);
+    g_generation++;
     g_table.clear();
     g_env_loaded = true;        // an explicit clear also cancels the automatic load at first use
 }

@@ -26,6 +26,18 @@ DTYPE_CODE = {
 ACTIVATION_CODE = {"none": 0, "relu": 1, "gelu": 2, "silu": 3, "tanh": 4, "sigmoid": 5, "gelu_exact": 6}
 
 
+_native = None
+
+
+def _host():
+    """The compiled host path (csrc/python/native.cpp): checks, result tensor, stream and launch."""
+    global _native
+    if _native is None:
+        _lib.load()                                   # (names the build command when the library is missing)
+        _native = _lib.load_native()
+    return _native
+
+
 def _code(t: torch.Tensor) -> int:
     try:
         return DTYPE_CODE[t.dtype]
@@ -52,60 +64,20 @@ def _ptr(t: Optional[torch.Tensor]):
 
 
 def softmax(x: torch.Tensor, axis: int = -1) -> torch.Tensor:
-    _dev(x)
-    lib = _lib.load()
-    if axis < 0:
-        axis += x.dim()
-    if not 0 <= axis < x.dim():
-        raise ValueError("softmax axis out of range")
-    y = torch.empty_like(x)
-    outer = math.prod(x.shape[:axis])
-    inner = math.prod(x.shape[axis + 1:])
-    n = x.shape[axis]
-    if inner == 1:
-        _lib.check(lib.mhip_softmax(_stream(), x.data_ptr(), y.data_ptr(), outer, n, _code(x)))
-    else:
-        _lib.check(lib.mhip_softmax_strided(_stream(), x.data_ptr(), y.data_ptr(), outer, n, inner,
-                                            _code(x)))
-    return y
+    return (_native or _host()).softmax(x, axis)
 
 
 def layer_norm(x, gamma=None, beta=None, eps: float = 1e-5):
-    _dev(x, gamma, beta)
-    lib = _lib.load()
-    cols = x.shape[-1]
-    for p in (gamma, beta):
-        if p is not None and (p.numel() != cols or p.dtype != x.dtype):
-            raise ValueError("gamma/beta must have the row length and dtype of x")
-    y = torch.empty_like(x)
-    _lib.check(lib.mhip_layer_norm(_stream(), x.data_ptr(), _ptr(gamma), _ptr(beta), y.data_ptr(),
-                                   x.numel() // max(cols, 1), cols, eps, _code(x)))
-    return y
+    return (_native or _host()).layer_norm(x, gamma, beta, eps)
 
 
 def rms_norm(x, gamma=None, eps: float = 1e-5):
-    _dev(x, gamma)
-    lib = _lib.load()
-    cols = x.shape[-1]
-    if gamma is not None and (gamma.numel() != cols or gamma.dtype != x.dtype):
-        raise ValueError("gamma must have the row length and dtype of x")
-    y = torch.empty_like(x)
-    _lib.check(lib.mhip_rms_norm(_stream(), x.data_ptr(), _ptr(gamma), y.data_ptr(),
-                                 x.numel() // max(cols, 1), cols, eps, _code(x)))
-    return y
+    return (_native or _host()).rms_norm(x, gamma, eps)
 
 
 def bias_gelu(x, bias=None, exact: bool = False):
     """gelu(x + bias): the tanh approximation, or with `exact` 0.5 v (1 + erf(v / sqrt 2))."""
-    _dev(x, bias)
-    lib = _lib.load()
-    cols = x.shape[-1] if x.dim() else 1
-    if bias is not None and (bias.numel() != cols or bias.dtype != x.dtype):
-        raise ValueError("bias must have the row length and dtype of x")
-    y = torch.empty_like(x)
-    fn = lib.mhip_bias_gelu_erf if exact else lib.mhip_bias_gelu
-    _lib.check(fn(_stream(), x.data_ptr(), _ptr(bias), y.data_ptr(), x.numel() // max(cols, 1), cols, _code(x)))
-    return y
+    return (_native or _host()).bias_gelu(x, bias, exact)
 
 
 def gelu(x, exact: bool = False):
@@ -117,40 +89,7 @@ def matmul(a, b, bias=None, activation: str = "none", trans_a: bool = False,
            residual: Optional[torch.Tensor] = None):
     """act(op(a) @ op(b) + bias) (+ residual, which has the result's shape and may be `out`);
     leading dims of `a` are batch dims when `b` is batched too, otherwise they fold into M."""
-    _dev(a, b, bias, out, residual)
-    lib = _lib.load()
-    if a.dtype != b.dtype:
-        raise TypeError("operand dtypes differ")
-    if b.dim() == 2:
-        if trans_a and a.dim() != 2:
-            raise ValueError("trans_a needs a 2-D lhs when rhs is 2-D")
-        a2 = a if a.dim() == 2 else a.reshape(-1, a.shape[-1])
-        batch, sa, sb = 1, 0, 0
-        out_lead = tuple(a.shape[:-1]) if not trans_a else (a.shape[-1],)
-    else:
-        if a.dim() != b.dim() or a.shape[:-2] != b.shape[:-2]:
-            raise ValueError("batched matmul needs equal batch dims")
-        batch = math.prod(a.shape[:-2])
-        a2 = a
-        sa, sb = a.shape[-1] * a.shape[-2], b.shape[-1] * b.shape[-2]
-        out_lead = tuple(a.shape[:-2]) + ((a.shape[-1],) if trans_a else (a.shape[-2],))
-    M, K = (a2.shape[-1], a2.shape[-2]) if trans_a else (a2.shape[-2], a2.shape[-1])
-    Kb, N = (b.shape[-1], b.shape[-2]) if trans_b else (b.shape[-2], b.shape[-1])
-    if K != Kb:
-        raise ValueError(f"contracting sizes differ: {K} vs {Kb}")
-    if bias is not None and (bias.numel() != N or bias.dtype != a.dtype):
-        raise ValueError("bias must be [N] of the operand dtype")
-    if out is None:
-        out = torch.empty(out_lead + (N,), dtype=a.dtype, device=a.device)
-    if residual is not None and (residual.numel() != out.numel() or residual.dtype != out.dtype):
-        raise ValueError("residual must have the result's size and dtype")
-    # (partial sums of a split K: memory of the current stream's, or a capturing graph's own)
-    nbytes = lib.mhip_gemm_workspace(M, N, K, batch, int(trans_a), int(trans_b), _code(a))
-    work = torch.empty(nbytes, dtype=torch.uint8, device=a.device) if nbytes else None
-    _lib.check(lib.mhip_gemm_ws(_stream(), a2.data_ptr(), b.data_ptr(), _ptr(bias), _ptr(residual), out.data_ptr(),
-                                M, N, K, batch, sa, sb, M * N, int(trans_a), int(trans_b),
-                                ACTIVATION_CODE[activation], _code(a), _ptr(work), nbytes))
-    return out
+    return (_native or _host()).matmul(a, b, bias, ACTIVATION_CODE[activation], trans_a, trans_b, out, residual)
 
 
 def flash_attention(q, k, v, scale: Optional[float] = None, is_causal: bool = False,
@@ -159,43 +98,7 @@ def flash_attention(q, k, v, scale: Optional[float] = None, is_causal: bool = Fa
     Default scale 1/sqrt(D) (FlashAttentionKernel.swift:55).  q, k, v (and `out`, when given)
     may be views with arbitrary batch / head / row strides as long as the last axis is
     contiguous, e.g. slices of a fused QKV projection; packed tensors take the plain entry."""
-    for t in (q, k, v, out):
-        if t is not None and (not t.is_cuda or t.dim() != 4 or t.stride(3) != 1):
-            raise ValueError("attention operands must be 4-D device tensors with a contiguous last axis")
-    _dev(mask)
-    lib = _lib.load()
-    if k.shape != v.shape or q.shape[:2] != k.shape[:2] or q.shape[3] != k.shape[3]:
-        raise ValueError("expected q [B,H,Sq,D] and k,v [B,H,Skv,D]")
-    if not (q.dtype == k.dtype == v.dtype):
-        raise TypeError("q, k, v dtypes differ")
-    B, H, Sq, D = q.shape
-    Skv = k.shape[2]
-    if scale is None:
-        scale = 1.0 / math.sqrt(D)
-    msb = msh = 0
-    if mask is not None:
-        if mask.dtype != q.dtype:
-            raise TypeError("mask dtype must match q")
-        while mask.dim() < 4:
-            mask = mask.unsqueeze(0)
-        if mask.shape[-2:] != (Sq, Skv) or mask.shape[0] not in (1, B) or mask.shape[1] not in (1, H):
-            raise ValueError("mask must broadcast to [B,H,Sq,Skv] with full last two dims")
-        msh = Sq * Skv if mask.shape[1] == H else 0
-        msb = mask.shape[1] * Sq * Skv if mask.shape[0] == B else 0
-    if out is None:
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    elif out.shape != q.shape or out.dtype != q.dtype:
-        raise ValueError("out must have q's shape and dtype")
-    if all(t.is_contiguous() for t in (q, k, v, out)):
-        _lib.check(lib.mhip_flash_attention(_stream(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                                            _ptr(mask), out.data_ptr(), B, H, Sq, Skv, D, float(scale),
-                                            int(is_causal), msb, msh, _code(q)))
-    else:
-        strides = (C.c_int64 * 12)(*[t.stride(i) for t in (q, k, v, out) for i in range(3)])
-        _lib.check(lib.mhip_flash_attention_strided(_stream(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                                                    _ptr(mask), out.data_ptr(), B, H, Sq, Skv, D, float(scale),
-                                                    int(is_causal), msb, msh, _code(q), C.addressof(strides)))
-    return out
+    return (_native or _host()).flash_attention(q, k, v, scale, is_causal, mask, out)
 
 
 # ---- glue -------------------------------------------------------------------
@@ -358,14 +261,9 @@ def iota(shape, dim: int, dtype, device="cuda"):
 
 
 def argmax(x, index_dtype=torch.int32, return_values: bool = False):
-    _dev(x)
-    lib = _lib.load()
-    cols = x.shape[-1]
-    idx = torch.empty(x.shape[:-1], dtype=index_dtype, device=x.device)
-    val = torch.empty(x.shape[:-1], dtype=x.dtype, device=x.device) if return_values else None
-    _lib.check(lib.mhip_argmax(_stream(), x.data_ptr(), idx.data_ptr(), _ptr(val),
-                               x.numel() // cols, cols, _code(x), DTYPE_CODE[index_dtype]))
-    return (idx, val) if return_values else idx
+    if index_dtype not in (torch.int32, torch.int64):
+        raise _lib.MhipError(2, f"mhip_argmax: index dtype {index_dtype} (need i32 or i64)")
+    return (_native or _host()).argmax(x, index_dtype == torch.int64, return_values)
 
 
 def autotune_matmul(a, b, bias=None, activation: str = "none", trans_a: bool = False,
