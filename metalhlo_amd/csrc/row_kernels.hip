@@ -413,8 +413,143 @@ void row_split_kernel(const T* __restrict__ x, const T* __restrict__ gamma, cons
 }
 
 // ---------------------------------------------------------------------------
-// General path: one workgroup per row, scalar accesses, statistics reduced
-// through LDS.  Any `cols`, any alignment.
+// Rows of any length and alignment (an odd vocabulary, a row longer than the kernels above hold): NT threads
+// per row, the row kept in registers (NV raw 16-byte vectors per thread) so that memory sees one read and one
+// write.  A row that starts at an odd address begins with up to 16 / sizeof(T) - 1 single elements, then whole
+// aligned vectors, then the rest; thread t < 16 owns head element t, thread 16 + t tail element t.  The
+// parameters are read at the row's phase, unaligned (cached, and global loads need no alignment here).
+// What bounds a launch with few rows is what one compute unit moves: [128,50257] bf16 107 us with the
+// scalar three-pass kernel below -> 8.5 us.
+// ---------------------------------------------------------------------------
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+
+template <typename T>
+struct RowPhase {
+    int head, nvec, tail;
+    __device__ RowPhase(const T* p, int cols) {
+        constexpr int E = Elem<T>::kPerVec;
+        head = min(cols, (int)(((16 - (reinterpret_cast<uintptr_t>(p) & 15)) & 15) / sizeof(T)));
+        nvec = (cols - head) / E;
+        tail = cols - head - nvec * E;
+    }
+    // the single element of thread t of the row, -1 = none
+    __device__ int edge(int t) const {
+        constexpr int E = Elem<T>::kPerVec;
+        return t < head ? t : t >= 16 && t - 16 < tail ? head + nvec * E + t - 16 : -1;
+    }
+};
+
+// sum or maximum over the NT threads of a row; `slots` = NT / 64 floats of this reduction's own
+template <int NT, bool MAX>
+__device__ inline float row_reduce(float v, float* slots) {
+    v = MAX ? wave_max(v) : wave_sum(v);
+    if (NT == 64) return v;
+    if ((threadIdx.x & 63) == 0) slots[threadIdx.x >> 6] = v;
+    __syncthreads();
+    float r = slots[0];
+#pragma unroll
+    for (int i = 1; i < NT / 64; i++) r = MAX ? fmaxf(r, slots[i]) : r + slots[i];
+    return r;
+}
+
+template <typename T, int OP, int NT, int NV>
+__global__ __launch_bounds__(NT < 256 ? 256 : NT) void row_any_kernel(const T* __restrict__ x, const T* __restrict__ gamma,
+                                                                      const T* __restrict__ beta, T* __restrict__ y, int64_t rows,
+                                                                      int cols, float eps) {
+    constexpr int E = Elem<T>::kPerVec;
+    constexpr float kLog2e = 1.4426950408889634f;
+    constexpr bool k16 = sizeof(T) == 2;
+    __shared__ float red[2][NT / 64];
+    const int64_t row = NT < 256 ? (int64_t)blockIdx.x * (256 / NT) + threadIdx.x / NT : (int64_t)blockIdx.x;
+    const int t = threadIdx.x % NT;
+    if (row >= rows) return;                       // (whole waves: NT >= 64, and only the form without barriers)
+    const T* xr = x + row * cols;
+    T* yr = y + row * cols;
+    const RowPhase<T> ph(xr, cols);
+    const int ei = ph.edge(t);
+    Vec16<T> raw[NV];
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+        const int i = v * NT + t;
+        raw[v] = __builtin_bit_cast(Vec16<T>, u32x4{0, 0, 0, 0});
+        if (i < ph.nvec) raw[v] = load16_stream(xr + ph.head + i * E);
+    }
+    float ev = ei >= 0 ? Elem<T>::to_f32(xr[ei]) : 0.f;
+    const float inv_cols = 1.f / (float)cols;
+    float scale, shift = 0.f;                      // y = f(x) * scale (+ shift)
+    if (OP == kSoftmax) {
+        float m = ei >= 0 ? ev : -INFINITY;
+#pragma unroll
+        for (int v = 0; v < NV; v++)
+            if (v * NT + t < ph.nvec) {
+#pragma unroll
+                for (int e = 0; e < E; e++) m = fmaxf(m, Elem<T>::to_f32(raw[v].v[e]));
+            }
+        m = row_reduce<NT, true>(m, red[0]);
+        shift = k16 ? m * kLog2e : m;
+        float s = ei >= 0 ? (k16 ? __builtin_amdgcn_exp2f(fmaf(ev, kLog2e, -shift)) : expf(ev - m)) : 0.f;
+#pragma unroll
+        for (int v = 0; v < NV; v++)
+            if (v * NT + t < ph.nvec) {
+#pragma unroll
+                for (int e = 0; e < E; e++) {
+                    const float f = Elem<T>::to_f32(raw[v].v[e]);
+                    const float p = k16 ? __builtin_amdgcn_exp2f(fmaf(f, kLog2e, -shift)) : expf(f - m);
+                    if (!k16) raw[v].v[e] = Elem<T>::from_f32(p);       // (kept: exact in fp32)
+                    s += p;
+                }
+            }
+        scale = 1.f / row_reduce<NT, false>(s, red[1]);
+    } else if (OP == kLayerNorm) {
+        float s = ev;
+#pragma unroll
+        for (int v = 0; v < NV; v++) s = VecSum<T>::sum(raw[v], s);
+        const float mean = row_reduce<NT, false>(s, red[0]) * inv_cols;
+        float q = ei >= 0 ? (ev - mean) * (ev - mean) : 0.f;
+#pragma unroll
+        for (int v = 0; v < NV; v++)
+            if (v * NT + t < ph.nvec) {
+#pragma unroll
+                for (int e = 0; e < E; e++) {
+                    const float d = Elem<T>::to_f32(raw[v].v[e]) - mean;
+                    q = fmaf(d, d, q);
+                }
+            }
+        scale = 1.f / sqrtf(row_reduce<NT, false>(q, red[1]) * inv_cols + eps);
+        shift = mean;
+    } else {
+        float q = ev * ev;
+#pragma unroll
+        for (int v = 0; v < NV; v++) q = VecSum<T>::sumsq(raw[v], q);
+        scale = 1.f / sqrtf(row_reduce<NT, false>(q, red[0]) * inv_cols + eps);
+    }
+    auto value = [&](float f, float g, float b) {
+        if (OP == kSoftmax) return (k16 ? __builtin_amdgcn_exp2f(fmaf(f, kLog2e, -shift)) : f) * scale;
+        return fmaf((f - shift) * scale, g, b);
+    };
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+        const int i = v * NT + t;
+        if (i >= ph.nvec) continue;
+        Vec16<T> gv, bv, o;
+        if (OP != kSoftmax && gamma) gv = __builtin_bit_cast(Vec16<T>, *reinterpret_cast<const u32x4_any*>(gamma + ph.head + i * E));
+        if (OP == kLayerNorm && beta) bv = __builtin_bit_cast(Vec16<T>, *reinterpret_cast<const u32x4_any*>(beta + ph.head + i * E));
+#pragma unroll
+        for (int e = 0; e < E; e++)
+            o.v[e] = Elem<T>::from_f32(value(Elem<T>::to_f32(raw[v].v[e]), OP != kSoftmax && gamma ? Elem<T>::to_f32(gv.v[e]) : 1.f,
+                                             OP == kLayerNorm && beta ? Elem<T>::to_f32(bv.v[e]) : 0.f));
+        store16_stream(yr + ph.head + i * E, o);
+    }
+    if (ei >= 0) {
+        if (OP == kSoftmax && !k16) ev = expf(ev - shift);
+        yr[ei] = Elem<T>::from_f32(value(ev, OP != kSoftmax && gamma ? Elem<T>::to_f32(gamma[ei]) : 1.f,
+                                         OP == kLayerNorm && beta ? Elem<T>::to_f32(beta[ei]) : 0.f));
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Rows longer than registers hold, or x and y at different addresses modulo 16: one workgroup per row,
+// scalar accesses, statistics reduced through LDS.
 // ---------------------------------------------------------------------------
 __device__ inline float block_reduce(float v, bool is_max, float* lds) {
     v = is_max ? wave_max(v) : wave_sum(v);
@@ -594,28 +729,68 @@ __global__ __launch_bounds__(256) void bias_gelu_tile_kernel(const T* __restrict
     }
 }
 
+// Rows that are no whole number of vectors: the tensor as one flat run of vectors (x and y aligned, `nvec` of
+// them, the last `n - nvec E` elements one per thread behind them), a vector's first column computed once and
+// its bias read unaligned where the vector does not cross a row's end.
 template <typename T, bool EXACT>
-__global__ __launch_bounds__(256) void bias_gelu_scalar_kernel(const T* __restrict__ x,
-                                                               const T* __restrict__ bias,
-                                                               T* __restrict__ y, int64_t n,
-                                                               int64_t cols) {
+__global__ __launch_bounds__(256) void bias_gelu_flat_kernel(const T* __restrict__ x, const T* __restrict__ bias, T* __restrict__ y,
+                                                             int64_t n, int64_t nvec, int64_t cols) {
+    constexpr int E = Elem<T>::kPerVec;
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    float v = Elem<T>::to_f32(x[i]);
-    if (bias) v += Elem<T>::to_f32(bias[i % cols]);
-    y[i] = Elem<T>::from_f32(gelu_tanh_f<T, EXACT>(v));
+    if (i < nvec) {
+        const int64_t first = i * E;
+        const Vec16<T> in = load16_stream(x + first);
+        float bv[E];
+#pragma unroll
+        for (int e = 0; e < E; e++) bv[e] = 0.f;
+        if (bias) {
+            int64_t c = n < 0x7FFFFFFF ? (int64_t)((uint32_t)first % (uint32_t)cols) : first % cols;
+            if (c + E <= cols) {
+                const Vec16<T> t = __builtin_bit_cast(Vec16<T>, *reinterpret_cast<const u32x4_any*>(bias + c));
+#pragma unroll
+                for (int e = 0; e < E; e++) bv[e] = Elem<T>::to_f32(t.v[e]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < E; e++) {
+                    bv[e] = Elem<T>::to_f32(bias[c]);
+                    if (++c == cols) c = 0;
+                }
+            }
+        }
+        Vec16<T> o;
+#pragma unroll
+        for (int e = 0; e < E; e++) o.v[e] = Elem<T>::from_f32(gelu_tanh_f<T, EXACT>(Elem<T>::to_f32(in.v[e]) + bv[e]));
+        store16_stream(y + first, o);
+    } else {
+        const int64_t j = nvec * E + (i - nvec);
+        if (j >= n) return;
+        float v = Elem<T>::to_f32(x[j]);
+        if (bias) v += Elem<T>::to_f32(bias[j % cols]);
+        y[j] = Elem<T>::from_f32(gelu_tanh_f<T, EXACT>(v));
+    }
 }
 
 // ---------------------------------------------------------------------------
 // Host-side dispatch
 // ---------------------------------------------------------------------------
+// Rows of a workgroup in kernels that give a row `threads` threads (256 threads at least).
+constexpr int rows_per_group(int threads) { return threads < 256 ? 256 / threads : 1; }
+
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 template <typename K, typename... Args>
 static void launch_persistent(K kern, size_t lds, int per_cu, int64_t want, hipStream_t s, Args... args) {
-    if (per_cu <= 0 &&
-        (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 256, lds) != hipSuccess || per_cu <= 0))
-        per_cu = 4;
+    if (per_cu <= 0) {
+        // (the query costs more host time than the launch: one answer per thread, kernel and LDS size)
+        struct Answer { const void* kern; size_t lds; int per_cu; };
+        static thread_local Answer last = {nullptr, 0, 0};
+        if (last.kern != reinterpret_cast<const void*>(kern) || last.lds != lds) {
+            int n = 0;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, 256, lds) != hipSuccess || n <= 0) n = 4;
+            last = {reinterpret_cast<const void*>(kern), lds, n};
+        }
+        per_cu = last.per_cu;
+    }
     // the occupancy query counts LDS to the last byte; keep a margin so that every workgroup of
     // the grid really is resident at once
     if (lds && per_cu > (int)((160 * 1024 - 4096) / (lds + 512))) per_cu = (int)((160 * 1024 - 4096) / (lds + 512));
@@ -689,6 +864,22 @@ static int launch_row(hipStream_t s, const void* x, const void* g, const void* b
             else MHIP_ROW_CASE(16);
 #undef MHIP_ROW_CASE
         }
+    } else if (!forced && ((reinterpret_cast<uintptr_t>(x) ^ reinterpret_cast<uintptr_t>(y)) & 15) == 0 && cols <= 1024 * 16 * E) {
+        // threads per row by its length: a wave up to 128 vectors, 256 threads up to 1024, 1024 beyond
+        const int64_t nvec = cols / E;
+#define MHIP_ROW_ANY(NT, NV)                                                                                            \
+    hipLaunchKernelGGL((row_any_kernel<T, OP, NT, NV>), dim3((unsigned)((rows + rows_per_group(NT) - 1) / rows_per_group(NT))), \
+                       dim3(NT < 256 ? 256 : NT), 0, s, xp, gp, bp, yp, rows, (int)cols, eps)
+        if (nvec <= 64) MHIP_ROW_ANY(64, 1);
+        else if (nvec <= 128) MHIP_ROW_ANY(64, 2);
+        else if (nvec <= 256) MHIP_ROW_ANY(256, 1);
+        else if (nvec <= 512) MHIP_ROW_ANY(256, 2);
+        else if (nvec <= 1024) MHIP_ROW_ANY(256, 4);
+        else if (nvec <= 2048) MHIP_ROW_ANY(1024, 2);
+        else if (nvec <= 4096) MHIP_ROW_ANY(1024, 4);
+        else if (nvec <= 8192) MHIP_ROW_ANY(1024, 8);
+        else MHIP_ROW_ANY(1024, 16);
+#undef MHIP_ROW_ANY
     } else {
         hipLaunchKernelGGL((row_block_kernel<T, OP>), dim3((unsigned)rows), dim3(256), 0, s, xp,
                            gp, bp, yp, cols, eps);
@@ -743,11 +934,12 @@ static int launch_gelu(hipStream_t s, const void* x, const void* bias, void* y, 
                                in_lds ? 1 : 0);
         }
     } else {
-        const int64_t grid = (n + 255) / 256;
+        const int64_t nvec = aligned16(x) && aligned16(y) ? n / E : 0;
+        const int64_t grid = (nvec + (n - nvec * E) + 255) / 256;
         if (grid > 0x7FFFFFFFLL) return fail(MHIP_ERR_UNSUPPORTED, "bias_gelu: tensor too large");
-        hipLaunchKernelGGL((bias_gelu_scalar_kernel<T, EXACT>), dim3((unsigned)grid), dim3(256), 0, s,
+        hipLaunchKernelGGL((bias_gelu_flat_kernel<T, EXACT>), dim3((unsigned)grid), dim3(256), 0, s,
                            static_cast<const T*>(x), static_cast<const T*>(bias),
-                           static_cast<T*>(y), n, cols);
+                           static_cast<T*>(y), n, nvec, cols);
     }
     return check_launch("bias_gelu");
 }
