@@ -183,6 +183,16 @@ int mhip_flash_attention_strided(void* stream, const void* q, const void* k, con
                                  int64_t mask_stride_b, int64_t mask_stride_h, int dtype,
                                  const int64_t* strides);
 
+/* The same (strides may be NULL) with device memory the call may use: a few query rows (a decode step) over a long
+ * cache are then split along the keys over the whole device.  mhip_flash_attention_workspace returns the bytes
+ * that can be used (0: none); with less, or none, the keys are not split.  16-byte aligned; the content is
+ * overwritten and meaningless afterwards. */
+int64_t mhip_flash_attention_workspace(int64_t B, int64_t H, int64_t Sq, int64_t Skv, int64_t D, int is_causal, int dtype);
+int mhip_flash_attention_ws(void* stream, const void* q, const void* k, const void* v, const void* mask, void* o,
+                            int64_t B, int64_t H, int64_t Sq, int64_t Skv, int64_t D, float scale, int is_causal,
+                            int64_t mask_stride_b, int64_t mask_stride_h, int dtype, const int64_t* strides,
+                            void* workspace, int64_t workspace_bytes);
+
 /* Glue operators (index / data movement; integer results are bit-exact) ---- */
 
 /* out[i, :] = table[clamp(idx[i], 0, n_rows-1), :], rows of `row_elems` elements.

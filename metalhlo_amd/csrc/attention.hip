@@ -361,6 +361,10 @@ namespace mhip {
 // attention_pipe.hip: head size 128, four waves x 64 query rows, matrix / softmax overlap in one wave.
 bool fa_pipe_eligible(const FaArgs& a, int64_t D, int dtype, bool has_mask, int variant);
 int launch_fa_pipe(hipStream_t s, const FaArgs& a, int dtype, bool causal, int pair);
+// attention_decode.hip: up to sixteen query rows over a long cache.
+bool fa_decode_eligible(const FaArgs& a);
+int64_t fa_decode_workspace(int64_t bh, int64_t Sq, int64_t Skv, int64_t D);
+int launch_fa_decode(hipStream_t s, const FaArgs& a, int64_t D, int dtype, void* workspace, int64_t workspace_bytes);
 // attention_f32.hip: fp32 tensors on the fp32 matrix instruction.
 bool fa_f32_mfma_eligible(const FaArgs& a, int64_t D);
 int launch_fa_f32_mfma(hipStream_t s, const FaArgs& a, int64_t D, float scale);
@@ -371,7 +375,8 @@ using namespace mhip;
 // `strides`: NULL (packed [B,H,S,D]) or twelve element strides {batch, head, row} x {q, k, v, o}.
 static int fa_entry(const char* name, void* stream, const void* q, const void* k, const void* v, const void* mask, void* o,
                     int64_t B, int64_t H, int64_t Sq, int64_t Skv, int64_t D, float scale, int is_causal,
-                    int64_t mask_stride_b, int64_t mask_stride_h, int dtype, const int64_t* strides) {
+                    int64_t mask_stride_b, int64_t mask_stride_h, int dtype, const int64_t* strides, void* workspace = nullptr,
+                    int64_t workspace_bytes = 0) {
     if (B < 0 || H < 0 || Sq < 0 || Skv < 0 || D <= 0)
         return fail(MHIP_ERR_INVALID_ARGUMENT, "%s: bad size", name);
     if (D > 256) return fail(MHIP_ERR_UNSUPPORTED, "%s: head_dim %lld > 256", name, (long long)D);
@@ -416,6 +421,7 @@ static int fa_entry(const char* name, void* stream, const void* q, const void* k
         const bool hm = mask != nullptr;
         // 0 = no tuned choice; 1 = 128-row kernel; 2 / 3 = 256-row pipelined kernel, causal tiles unpaired / paired
         const int variant = is_packed ? tuned_attention_variant(dtype, B * H, Sq, Skv, D, is_causal != 0) : 0;
+        if (variant == 0 && fa_decode_eligible(a) && B * H <= 0x7FFFFFFF) return launch_fa_decode(s, a, D, dtype, workspace, workspace_bytes);
         if (is_packed && fa_pipe_eligible(a, D, dtype, hm, variant))
             return launch_fa_pipe(s, a, dtype, is_causal != 0, variant == 2 ? 0 : variant == 3 ? 1 : -1);
         if (dtype == MHIP_BF16)
@@ -452,4 +458,19 @@ extern "C" int mhip_flash_attention_strided(void* stream, const void* q, const v
                                             const int64_t* strides) {
     return fa_entry("mhip_flash_attention_strided", stream, q, k, v, mask, o, B, H, Sq, Skv, D, scale, is_causal,
                     mask_stride_b, mask_stride_h, dtype, strides);
+}
+
+extern "C" int mhip_flash_attention_ws(void* stream, const void* q, const void* k, const void* v, const void* mask, void* o,
+                                       int64_t B, int64_t H, int64_t Sq, int64_t Skv, int64_t D, float scale, int is_causal,
+                                       int64_t mask_stride_b, int64_t mask_stride_h, int dtype, const int64_t* strides,
+                                       void* workspace, int64_t workspace_bytes) {
+    if (workspace_bytes < 0 || (reinterpret_cast<uintptr_t>(workspace) & 15) != 0)
+        return fail(MHIP_ERR_INVALID_ARGUMENT, "mhip_flash_attention_ws: the workspace must be 16-byte aligned");
+    return fa_entry("mhip_flash_attention_ws", stream, q, k, v, mask, o, B, H, Sq, Skv, D, scale, is_causal, mask_stride_b,
+                    mask_stride_h, dtype, strides, workspace, workspace_bytes);
+}
+
+extern "C" int64_t mhip_flash_attention_workspace(int64_t B, int64_t H, int64_t Sq, int64_t Skv, int64_t D, int is_causal, int dtype) {
+    if (B <= 0 || H <= 0 || Skv <= 0 || is_causal || (dtype != MHIP_BF16 && dtype != MHIP_F16)) return 0;
+    return fa_decode_workspace(B * H, Sq, Skv, D);
 }

@@ -1,0 +1,249 @@
+// Attention of a few query rows (a decode step, Sq <= 16) over a long key / value cache, 16-bit types, head
+// sizes 64 and 128: the time is that of reading K and V once.
+//
+// A query tile of 128 rows would be almost all padding, and its one workgroup per head walks the keys through
+// LDS stages with little in flight.  Here every wave of a workgroup takes blocks of 32 keys of its own, loads
+// them straight into matrix operands (no LDS, no barrier in the loop) one block ahead, and keeps its own
+// softmax state; the waves meet at the end in LDS, and the parts of a split key range in a workspace.
+//
+//   S^T = K Q^T     v_mfma_f32_16x16x32: operand row = key, so a lane loads 16 bytes of one key's row; a lane
+//                   of the result holds four keys of one query.
+//   O^T += V^T P^T  operand row = d: lane i loads VE = D / 16 neighbouring d of each of its eight keys, and one
+//                   byte permute per register pairs two keys of one d; tile f then holds d = VE i + f.  The
+//                   eight keys of a lane are the ones whose probabilities it just computed.
+#include "attention_common.h"
+
+namespace mhip {
+namespace {
+
+template <typename T> struct Mfma16A;
+template <> struct Mfma16A<bf16_t> {
+    __device__ static f32x4 run(u32x4 a, u32x4 b, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+    }
+};
+template <> struct Mfma16A<f16_t> {
+    __device__ static f32x4 run(u32x4 a, u32x4 b, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+    }
+};
+
+constexpr int kKeys = 32;        // keys per block
+constexpr int kMaxSq = 16;
+constexpr int kPartKeys = 256;   // a part of a split key range is a multiple of this
+
+template <typename T, int D, bool HAS_MASK, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* part, int per_part) {
+    constexpr int NS = D / 32, NF = D / 16, VDw = NF / 2;      // k steps of Q K^T, tiles of O^T, dwords of a lane's V piece
+    __shared__ __attribute__((aligned(16))) float sums[WAVES][NF][64][4];
+    __shared__ float ml[2][WAVES][kMaxSq];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 15, lg = lane >> 4;
+    const int bh = blockIdx.x, b_i = bh / a.H, h_i = bh % a.H;
+    const T* qp = static_cast<const T*>(a.q) + b_i * a.qs[0] + h_i * a.qs[1];
+    const T* kp = static_cast<const T*>(a.k) + b_i * a.ks[0] + h_i * a.ks[1];
+    const T* vp = static_cast<const T*>(a.v) + b_i * a.vs[0] + h_i * a.vs[1];
+    const int q_rs = (int)a.qs[2], k_rs = (int)a.ks[2], v_rs = (int)a.vs[2];
+    const __amdgpu_buffer_rsrc_t rq = fa_rsrc(qp, (uint32_t)((((int64_t)a.Sq - 1) * q_rs + D) * 2));
+    const __amdgpu_buffer_rsrc_t rk = fa_rsrc(kp, (uint32_t)((((int64_t)a.Skv - 1) * k_rs + D) * 2));
+    const __amdgpu_buffer_rsrc_t rv = fa_rsrc(vp, (uint32_t)((((int64_t)a.Skv - 1) * v_rs + D) * 2));
+    const T* mp = HAS_MASK ? static_cast<const T*>(a.mask) + (int64_t)b_i * a.mask_sb + (int64_t)h_i * a.mask_sh : nullptr;
+
+    u32x4 qf[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+        qf[s] = __builtin_amdgcn_raw_buffer_load_b128(rq, li < a.Sq ? (uint32_t)((li * q_rs + 32 * s + 8 * lg) * 2) : kOobA, 0, 0);
+        if (a.negate_q) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) qf[s][e] ^= 0x80008000u;
+        }
+    }
+
+    // this workgroup's keys [k0, k1); block n of wave w is keys k0 + 32 (WAVES n + w) ...  (keys past the end of
+    // the cache lie beyond the buffers' extents and read zero)
+    const int k0 = (int)blockIdx.y * per_part, k1 = min(a.Skv, k0 + per_part);
+    struct Block { u32x4 k[2][NS]; uint32_t v[8][VDw]; };
+    const uint32_t koff = (uint32_t)((li * k_rs + 8 * lg) * 2), voff = (uint32_t)((4 * lg * v_rs + NF * li) * 2);
+    auto load = [&](Block& blk, int key) {
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int s = 0; s < NS; s++)
+                blk.k[j][s] = __builtin_amdgcn_raw_buffer_load_b128(rk, koff + (uint32_t)(((key + 16 * j) * k_rs + 32 * s) * 2), 0, 0);
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            const uint32_t off = voff + (uint32_t)((key + 16 * (t >> 2) + (t & 3)) * v_rs * 2);
+            if constexpr (VDw == 4) {
+                const u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(rv, off, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; e++) blk.v[t][e] = w[e];
+            } else {
+                const u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(rv, off, 0, 0);
+                blk.v[t][0] = w.x; blk.v[t][1] = w.y;
+            }
+        }
+    };
+
+    f32x4 oacc[NF];
+#pragma unroll
+    for (int f = 0; f < NF; f++) oacc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_run = -INFINITY, l_run = 0.f;          // of query li; the sum is this lane's keys only
+    auto attend = [&](const Block& blk, int key) {
+        float sv[8];
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            f32x4 s4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < NS; s++) s4 = Mfma16A<T>::run(blk.k[j][s], qf[s], s4);
+#pragma unroll
+            for (int r = 0; r < 4; r++) sv[4 * j + r] = s4[r] * a.c;
+        }
+        if (HAS_MASK) {
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                const int kk = key + 16 * (t >> 2) + 4 * lg + (t & 3);
+                if (li < a.Sq && kk < a.Skv) sv[t] += Elem<T>::to_f32(mp[(int64_t)li * a.Skv + kk]) * kLog2e;
+            }
+        }
+        if (key + kKeys > k1) {
+#pragma unroll
+            for (int t = 0; t < 8; t++)
+                if (key + 16 * (t >> 2) + 4 * lg + (t & 3) >= k1) sv[t] = -INFINITY;
+        }
+        float mloc = sv[0];
+#pragma unroll
+        for (int t = 1; t < 8; t++) mloc = fmaxf(mloc, sv[t]);
+        mloc = fmaxf(mloc, __shfl_xor(mloc, 16, 64));
+        mloc = half_max(mloc);
+        const float m_new = moved_reference(m_run, mloc), m_use = m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+        m_run = m_new;
+        float lsum = 0.f;
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            sv[t] = __builtin_amdgcn_exp2f(sv[t] - m_use);
+            lsum += sv[t];
+        }
+        l_run = l_run * alpha + lsum;
+        if (__any(alpha != 1.f)) {
+#pragma unroll
+            for (int f = 0; f < NF; f++) oacc[f] *= alpha;
+        }
+        u32x4 pb;
+#pragma unroll
+        for (int e = 0; e < 4; e++) pb[e] = Mfma32A<T>::pack2(sv[2 * e], sv[2 * e + 1]);
+#pragma unroll
+        for (int f = 0; f < NF; f++) {
+            u32x4 vf;
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                vf[e] = __builtin_amdgcn_perm(blk.v[2 * e + 1][f / 2], blk.v[2 * e][f / 2], (f & 1) ? 0x07060302u : 0x05040100u);
+            oacc[f] = Mfma16A<T>::run(vf, pb, oacc[f]);
+        }
+    };
+    int key = k0 + wave * kKeys;
+    if (key < k1) {
+        Block cur;
+        load(cur, key);
+        for (; key < k1; key += WAVES * kKeys) {
+            Block nxt;
+            const bool more = key + WAVES * kKeys < k1;
+            if (more) load(nxt, key + WAVES * kKeys);
+            attend(cur, key);
+            if (more) cur = nxt;
+        }
+    }
+
+    // ---- the waves' states
+    l_run += __shfl_xor(l_run, 16, 64);
+    l_run = half_sum(l_run);
+    if (lg == 0) { ml[0][wave][li] = m_run; ml[1][wave][li] = l_run; }
+#pragma unroll
+    for (int f = 0; f < NF; f++) *reinterpret_cast<f32x4*>(sums[wave][f][lane]) = oacc[f];
+    __syncthreads();
+    T* op = static_cast<T*>(a.o) + b_i * a.os[0] + h_i * a.os[1];
+    for (int idx = threadIdx.x; idx < a.Sq * D; idx += 64 * WAVES) {
+        const int q = idx / D, d = idx % D, f = d % NF, i = d / NF;
+        float m = -INFINITY, l = 0.f, o = 0.f;
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) m = fmaxf(m, ml[0][w][q]);
+        const float m_use = m == -INFINITY ? 0.f : m;
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) {
+            const float al = __builtin_amdgcn_exp2f(ml[0][w][q] - m_use);
+            l = fmaf(ml[1][w][q], al, l);
+            o = fmaf(sums[w][f][(i >> 2) * 16 + q][i & 3], al, o);
+        }
+        if (part) {
+            // [part][bh][Sq][D] sums, then [part][bh][Sq][2] reference maximum and sum
+            const int64_t at = ((int64_t)blockIdx.y * gridDim.x + bh) * a.Sq + q;
+            part[at * D + d] = o;
+            if (d < 2) part[(int64_t)gridDim.y * gridDim.x * a.Sq * D + at * 2 + d] = d ? l : m;
+        } else {
+            op[(int64_t)q * a.os[2] + d] = Elem<T>::from_f32(o * (l > 1e-10f ? 1.f / l : 0.f));
+        }
+    }
+}
+
+// The parts of a split key range: one thread per element of O.
+template <typename T, int D>
+__global__ __launch_bounds__(256) void fa_decode_combine_kernel(FaArgs a, const float* part, int parts) {
+    const int64_t rows = (int64_t)a.B * a.H * a.Sq, idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= rows * D) return;
+    const int64_t row = idx / D;
+    const int d = (int)(idx % D);
+    const float* mls = part + (int64_t)parts * rows * D;
+    float m = -INFINITY, l = 0.f, o = 0.f;
+    for (int p = 0; p < parts; p++) m = fmaxf(m, mls[(p * rows + row) * 2]);
+    const float m_use = m == -INFINITY ? 0.f : m;
+    for (int p = 0; p < parts; p++) {
+        const float al = __builtin_amdgcn_exp2f(mls[(p * rows + row) * 2] - m_use);
+        l = fmaf(mls[(p * rows + row) * 2 + 1], al, l);
+        o = fmaf(part[(p * rows + row) * D + d], al, o);
+    }
+    const int64_t bh = row / a.Sq;
+    static_cast<T*>(a.o)[bh / a.H * a.os[0] + bh % a.H * a.os[1] + row % a.Sq * a.os[2] + d] = Elem<T>::from_f32(o * (l > 1e-10f ? 1.f / l : 0.f));
+}
+
+// Parts of the key range: enough workgroups for two per compute unit, each with at least 256 keys.
+int decode_parts(int64_t bh, int64_t Skv) {
+    const int64_t want = (512 + bh - 1) / bh, most = Skv / kPartKeys;
+    const int64_t n = want < most ? want : most;
+    return n < 2 ? 1 : n > 64 ? 64 : (int)n;
+}
+
+template <typename T, int D>
+int launch(hipStream_t s, const FaArgs& a, float* part, int parts) {
+    const int64_t bh = (int64_t)a.B * a.H;
+    const int per = parts == 1 ? a.Skv : (int)(((a.Skv + parts - 1) / parts + kPartKeys - 1) / kPartKeys * kPartKeys);
+    const dim3 grid((unsigned)bh, (unsigned)((a.Skv + per - 1) / per));
+    constexpr int WAVES = 4;
+    if (a.mask) hipLaunchKernelGGL((fa_decode_kernel<T, D, true, WAVES>), grid, dim3(64 * WAVES), 0, s, a, parts > 1 ? part : nullptr, per);
+    else hipLaunchKernelGGL((fa_decode_kernel<T, D, false, WAVES>), grid, dim3(64 * WAVES), 0, s, a, parts > 1 ? part : nullptr, per);
+    if (parts > 1) {
+        const int64_t n = bh * a.Sq * D;
+        hipLaunchKernelGGL((fa_decode_combine_kernel<T, D>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, part, (int)grid.y);
+    }
+    return check_launch("flash_attention_decode");
+}
+
+}  // namespace
+
+// (checked by the caller: 16-bit, aligned, extents below 2 GB, Skv > 0, D 64 or 128)
+bool fa_decode_eligible(const FaArgs& a) { return a.Sq <= kMaxSq && !a.is_causal; }
+
+int64_t fa_decode_workspace(int64_t bh, int64_t Sq, int64_t Skv, int64_t D) {
+    if (Sq < 1 || Sq > kMaxSq || (D != 64 && D != 128)) return 0;
+    const int parts = decode_parts(bh, Skv);
+    return parts == 1 ? 0 : parts * bh * Sq * (D + 2) * 4;
+}
+
+int launch_fa_decode(hipStream_t s, const FaArgs& a, int64_t D, int dtype, void* workspace, int64_t workspace_bytes) {
+    const int64_t bh = (int64_t)a.B * a.H, need = fa_decode_workspace(bh, a.Sq, a.Skv, D);
+    const int parts = need > 0 && workspace && need <= workspace_bytes ? decode_parts(bh, a.Skv) : 1;
+    float* part = static_cast<float*>(workspace);
+    if (dtype == MHIP_BF16) return D == 128 ? launch<bf16_t, 128>(s, a, part, parts) : launch<bf16_t, 64>(s, a, part, parts);
+    return D == 128 ? launch<f16_t, 128>(s, a, part, parts) : launch<f16_t, 64>(s, a, part, parts);
+}
+
+}  // namespace mhip

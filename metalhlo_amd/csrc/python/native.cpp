@@ -268,17 +268,16 @@ FUNCTION(flash_attention) {
         at::Tensor o = given ? *given : empty(q.sizes(), q.scalar_type(), q);
         const bool causal = truth(arg[4]);
         const int dt = dtype_code(q.scalar_type());
-        if (q.is_contiguous() && k.is_contiguous() && v.is_contiguous() && o.is_contiguous()) {
-            check([&] { return mhip_flash_attention(stream_of(q), q.data_ptr(), k.data_ptr(), v.data_ptr(), ptr(mask), o.data_ptr(), B, H, Sq, Skv, D, (float)scale,
-                                       causal, msb, msh, dt); });
-        } else {
-            int64_t strides[12];
-            views[3] = &o;
-            for (int t = 0; t < 4; t++)
-                for (int d = 0; d < 3; d++) strides[3 * t + d] = views[t]->stride(d);
-            check([&] { return mhip_flash_attention_strided(stream_of(q), q.data_ptr(), k.data_ptr(), v.data_ptr(), ptr(mask), o.data_ptr(), B, H, Sq, Skv, D,
-                                               (float)scale, causal, msb, msh, dt, strides); });
-        }
+        const bool packed = q.is_contiguous() && k.is_contiguous() && v.is_contiguous() && o.is_contiguous();
+        int64_t strides[12];
+        views[3] = &o;
+        for (int t = 0; !packed && t < 4; t++)
+            for (int d = 0; d < 3; d++) strides[3 * t + d] = views[t]->stride(d);
+        const int64_t bytes = mhip_flash_attention_workspace(B, H, Sq, Skv, D, causal, dt);
+        at::Tensor work;
+        if (bytes) work = empty({bytes}, at::kByte, q);
+        check([&] { return mhip_flash_attention_ws(stream_of(q), q.data_ptr(), k.data_ptr(), v.data_ptr(), ptr(mask), o.data_ptr(), B, H, Sq, Skv, D,
+                                                   (float)scale, causal, msb, msh, dt, packed ? nullptr : strides, bytes ? work.data_ptr() : nullptr, bytes); });
         return THPVariable_Wrap(std::move(o));
     });
 }
