@@ -8,8 +8,6 @@
 // ([row][64 k]) because the MFMA wants eight consecutive k per lane; an operand
 // whose memory layout has k as the slow axis is transposed in registers on the
 // way in (16-byte global loads either way).
-// Everything else (fp32, shapes that are not 16-byte friendly) goes through a
-// plain LDS-tiled kernel.
 #include <mutex>
 
 #include "gemm_lds.h"
@@ -189,7 +187,7 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(GemmArgs g) {
 }
 
 // ---------------------------------------------------------------------------
-// Plain tiled kernel: any type, any shape.  16x16 threads, one output each.
+// Plain tiled kernel for products too small or too short for a matrix tile.  16x16 threads, one output each.
 // ---------------------------------------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(256) void gemm_simple_kernel(GemmArgs g, int trans_a, int trans_b) {
@@ -300,6 +298,9 @@ int launch_gemm_stream(hipStream_t s, const GemmArgs& g, int trans_b, int dtype)
 // gemm_skinny.hip: at most 64 rows, the waves of a workgroup split K.
 bool gemm_skinny_eligible(const GemmArgs& g, int trans_a, int elem_bytes);
 int64_t gemm_skinny_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b);
+// gemm_any.hip: any alignment and size.
+int launch_gemm_any(hipStream_t s, GemmArgs g, int64_t batch, int trans_a, int trans_b, int dtype, int64_t workspace_bytes);
+int64_t gemm_any_workspace(int64_t M, int64_t N, int64_t K, int64_t batch);
 int launch_gemm_skinny(hipStream_t s, GemmArgs g, int64_t batch, int trans_b, int dtype, int64_t workspace_bytes);
 // gemm_mid.hip: 64- and 128-row tiles through a ring of LDS stages, K split where that leaves units idle.
 int64_t gemm_mid_workspace(int64_t M, int64_t N, int64_t K, int64_t batch);
@@ -532,6 +533,14 @@ static bool skinny_rows(int64_t M, int64_t N, int64_t K, bool is16) {
     return M <= 16 || !is16 || (M <= 32 && N * K <= (32 << 20));
 }
 
+// 16-bit operands without vector alignment.  The few-row kernel loads those element by element: it is ahead of
+// gemm_any.hip's 64-row tiles for up to 16 rows of a weight matrix that keeps few workgroups busy ([4,767] x
+// [767,769] 7.3 us against 10.1; [4,4097] x [4097,4097] 48 against 19, [16,1001] x K 8191 30 against 21).
+static bool skinny_unaligned(int64_t M, int64_t N, int64_t K) { return M <= 16 && N * K <= (1 << 20); }
+// The plain kernel is ahead of a matrix tile that is mostly edges: [65,33] x [33,77] 3.4 us against 4.7, [300,77] x
+// [77,333] 4.7 against 5.3; behind from there on: [128,130] x [130,129] 6.2 against 5.8, [1000,67] x [67,1001] 14.9 against 5.7.
+static bool short_product(int64_t M, int64_t N, int64_t K) { return K < 96 && M * N <= (1 << 17); }
+
 static bool few_row_choice(int tuned) { return tuned == 0 || tuned == 64; }
 
 static int gemm_entry(void* stream, const void* a, const void* b, const void* bias, const void* residual, void* c,
@@ -568,7 +577,7 @@ static int gemm_entry(void* stream, const void* a, const void* b, const void* bi
     g.partial = static_cast<float*>(workspace);
     // Few rows: the kernel that reads B once with all of its loads in flight, unless a tile kernel is asked for by
     // name or by the tuning table.
-    if ((is16 || dtype == MHIP_F32) && gemm_skinny_eligible(g, trans_a, is16 ? 2 : 4) && (!vec_ok || skinny_rows(M, N, K, is16)) &&
+    if ((is16 || dtype == MHIP_F32) && gemm_skinny_eligible(g, trans_a, is16 ? 2 : 4) && (is16 && !vec_ok ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, is16)) &&
         tune_int("MHIP_GEMM_TILE", 0) == 0 && tune_int("MHIP_GEMM_F32_MFMA", 1) == 1 &&
         (!is16 || few_row_choice(tuned_gemm_variant(g, batch, trans_a, trans_b, dtype)) || !vec_ok))
         return chose(vec_ok ? 64 : 0, launch_gemm_skinny(s, g, batch, trans_b, dtype, workspace_bytes));
@@ -580,8 +589,10 @@ static int gemm_entry(void* stream, const void* a, const void* b, const void* bi
         case MHIP_F32:
             if (gemm_f32_mfma_wanted(g)) return launch_gemm_f32_mfma(s, g, batch, trans_a, trans_b);
             return launch_simple<float>(s, g, batch, trans_a, trans_b);
-        case MHIP_BF16: return launch_simple<bf16_t>(s, g, batch, trans_a, trans_b);
-        case MHIP_F16: return launch_simple<f16_t>(s, g, batch, trans_a, trans_b);
+        case MHIP_BF16:
+        case MHIP_F16:
+            if (!short_product(M, N, K)) return launch_gemm_any(s, g, batch, trans_a, trans_b, dtype, workspace_bytes);
+            return dtype == MHIP_BF16 ? launch_simple<bf16_t>(s, g, batch, trans_a, trans_b) : launch_simple<f16_t>(s, g, batch, trans_a, trans_b);
         case MHIP_I32: return launch_exact<int32_t>(s, g, batch, trans_a, trans_b);
         case MHIP_I64: return launch_exact<int64_t>(s, g, batch, trans_a, trans_b);
         case MHIP_F64: return launch_exact<double>(s, g, batch, trans_a, trans_b);
@@ -622,8 +633,9 @@ extern "C" int64_t mhip_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t 
     const bool is16 = dtype == MHIP_BF16 || dtype == MHIP_F16;
     if (!is16 && dtype != MHIP_F32) return 0;
     const bool vec = is16 && (trans_a ? M : K) % 8 == 0 && (trans_b ? K : N) % 8 == 0;
-    if (!trans_a && M <= 64 && (!vec || skinny_rows(M, N, K, is16))) return gemm_skinny_workspace(M, N, K, batch, trans_b);
+    if (!trans_a && M <= 64 && (is16 && !vec ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, is16))) return gemm_skinny_workspace(M, N, K, batch, trans_b);
     // (a large problem goes to the ring kernels, whose tiles fill the device)
+    if (is16 && !vec) return short_product(M, N, K) ? 0 : gemm_any_workspace(M, N, K, batch);
     if (!vec || (M > 192 && (double)M * N * batch >= 192.0 * 256 * 256)) return 0;
     return gemm_mid_workspace(M, N, K, batch);
 }

@@ -37,6 +37,24 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 __device__ inline u32x4 frag_kmajor(const char* tile, int row0, int s, int lane) {
     return *reinterpret_cast<const u32x4*>(tile + lds_off(row0 + (lane & 31), 2 * s + (lane >> 5)));
 }
+// chunk swizzle of an operand tile that lies [64 k][ROWS] in LDS: the four k rows that a transposing read
+// touches must fall on different banks (rows of 64, 128, 256 bytes)
+template <int ROWS>
+__device__ __forceinline__ int mn_swz(int k) { return ROWS >= 128 ? ((k & 3) << 2) : ROWS == 64 ? (((k >> 1) & 1) << 2) : 0; }
+
+template <int ROWS>
+__device__ inline u32x4 frag_mn(const char* tile, int mn0, int s, int lane) {
+    const int i = lane & 15, g = lane >> 4;
+    const int mn = mn0 + 16 * (g & 1) + 4 * (i & 3);
+    const int k = 16 * s + 8 * (g >> 1) + (i >> 2);
+    const char* p0 = tile + k * (ROWS * 2) + (((mn >> 3) ^ mn_swz<ROWS>(k)) << 4) + (mn & 7) * 2;
+    // (four k further: the same swizzle, four rows down)
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p0);
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p0 + 4 * ROWS * 2));
+    const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+    return u32x4{l2.x, l2.y, h2.x, h2.y};
+}
+
 // The wave's (32 TM) x (32 TN) sub-tile at (row0, col0) of C: bias, activation, rounding, residual, store.
 // `stage` is this wave's LDS area of 32 TM rows of 64 TN + 16 bytes.
 template <typename T, int TM, int TN>
@@ -49,7 +67,7 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, const f32x16 (&acc
     // 32x32 accumulator tile is held transposed: a lane owns row m = lrow and,
     // in register group q = r/4, the four consecutive columns 8q + 4*lhalf + r%4.
     const T* bias = static_cast<const T*>(g.bias);
-    const bool vec_store = (g.N % 8 == 0) && ((reinterpret_cast<uintptr_t>(c) & 15) == 0);
+    const bool vec_store = (g.N % 8 == 0) && (((reinterpret_cast<uintptr_t>(c) | reinterpret_cast<uintptr_t>(res)) & 15) == 0);
     // Stage the wave's sub-tile in LDS as rounded 16-bit rows (padded by 16 bytes
     // against bank conflicts); the rows then go out with lanes running along n, so
     // every store instruction writes whole contiguous row segments.

@@ -24,24 +24,6 @@ int launch_gemm192(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_a,
 
 namespace {
 
-// chunk swizzle of an operand tile that lies [64 k][ROWS] in LDS: the four k rows that a transposing read
-// touches must fall on different banks (rows of 64, 128, 256 bytes)
-template <int ROWS>
-__device__ __forceinline__ int mn_swz(int k) { return ROWS >= 128 ? ((k & 3) << 2) : ROWS == 64 ? (((k >> 1) & 1) << 2) : 0; }
-
-template <int ROWS>
-__device__ inline u32x4 frag_mn(const char* tile, int mn0, int s, int lane) {
-    const int i = lane & 15, g = lane >> 4;
-    const int mn = mn0 + 16 * (g & 1) + 4 * (i & 3);
-    const int k = 16 * s + 8 * (g >> 1) + (i >> 2);
-    const char* p0 = tile + k * (ROWS * 2) + (((mn >> 3) ^ mn_swz<ROWS>(k)) << 4) + (mn & 7) * 2;
-    // (four k further: the same swizzle, four rows down)
-    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p0);
-    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p0 + 4 * ROWS * 2));
-    const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
-    return u32x4{l2.x, l2.y, h2.x, h2.y};
-}
-
 // One operand's loads: the wave-wide load i of wave w fills the KB number i * 4 + w of the stage's tile.
 template <int ROWS, bool KMAJOR>
 struct StageLoader {

@@ -274,12 +274,16 @@ int launch_shape(hipStream_t s, const GemmArgs& g, int64_t batch) {
         if (wide) return k16 || TB ? launch_one<T, TB, VEC, TB ? 2 : 4, 1, 2>(s, g, batch) : launch_one<T, TB, VEC, 2, 1, 2>(s, g, batch);
         return launch_one<T, TB, VEC, TB ? 1 : k16 ? 2 : 1, 1, 4>(s, g, batch);
     }
-    if (g.M <= 32) {
-        if (wide) return k16 || TB ? launch_one<T, TB, VEC, TB ? 2 : 4, 2, 2>(s, g, batch) : launch_one<T, TB, VEC, 2, 2, 2>(s, g, batch);
-        return launch_one<T, TB, VEC, TB ? 1 : k16 ? 2 : 1, 2, 2>(s, g, batch);
+    // (16-bit rows without vector alignment: gemm_any.hip takes them from 17 rows on)
+    if constexpr (k16 && !VEC) return fail(MHIP_ERR_UNSUPPORTED, "gemm: more than 16 unaligned rows");
+    else {
+        if (g.M <= 32) {
+            if (wide) return k16 || TB ? launch_one<T, TB, VEC, TB ? 2 : 4, 2, 2>(s, g, batch) : launch_one<T, TB, VEC, 2, 2, 2>(s, g, batch);
+            return launch_one<T, TB, VEC, TB ? 1 : k16 ? 2 : 1, 2, 2>(s, g, batch);
+        }
+        if (wide) return k16 || TB ? launch_one<T, TB, VEC, TB ? 2 : 4, 4, 1>(s, g, batch) : launch_one<T, TB, VEC, 2, 4, 1>(s, g, batch);
+        return launch_one<T, TB, VEC, TB ? 1 : k16 ? 2 : 1, 4, 2>(s, g, batch);
     }
-    if (wide) return k16 || TB ? launch_one<T, TB, VEC, TB ? 2 : 4, 4, 1>(s, g, batch) : launch_one<T, TB, VEC, 2, 4, 1>(s, g, batch);
-    return launch_one<T, TB, VEC, TB ? 1 : k16 ? 2 : 1, 4, 2>(s, g, batch);
 }
 
 int dtype_launch(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_b, int dtype) {
