@@ -29,6 +29,7 @@ struct FaArgs {
     // Element strides {batch, head, row} of q, k, v, o (the last axis is contiguous).  Only
     // fa_fwd_kernel reads them; every other kernel is given the packed [B,H,S,D] layout.
     int64_t qs[3], ks[3], vs[3], os[3];
+    int D;            // head size (read by fa_fwd_kernel where its rows are padded in LDS)
 };
 
 // Which (batch * head, query tile) a workgroup of the one-tile-per-workgroup kernels takes.

@@ -1,0 +1,51 @@
+"""GPU parity of 16-bit attention for head sizes other than 64 and 128: multiples of 8 on the matrix cores
+(rows padded to 64 or 128 in LDS), the rest on the scalar kernel; block edges, masks, negative scale.
+
+Bound, with P the exact probabilities: a score is off by at most (D + 2) 2^-24 of scale sum |q||k|, a probability
+by twice the largest of those in relative terms, 2^-16 for its two 16-bit parts and Skv 2^-24 for its sums; the
+result is that times sum P |v|, rounded once to its type."""
+import numpy as np
+import pytest
+import torch
+
+from tests.util import NAME, as_f64, to_dev
+
+pytestmark = pytest.mark.gpu
+ROUNDOFF = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+
+
+def _reference(q, k, v, scale, causal, mask):
+    s = (q @ np.swapaxes(k, -1, -2)) * scale
+    err = (q.shape[-1] + 2) * 2.0 ** -24 * np.max((np.abs(q) @ np.swapaxes(np.abs(k), -1, -2)) * abs(scale))
+    if mask is not None:
+        s = s + mask
+    if causal:
+        s = np.where(np.arange(s.shape[-1]) > np.arange(s.shape[-2])[:, None], -np.inf, s)
+    m = s.max(-1, keepdims=True)
+    p = np.exp(s - np.where(np.isfinite(m), m, 0))
+    p = p / np.maximum(p.sum(-1, keepdims=True), 1e-300)
+    return p @ v, (2 * err + 2.0 ** -16 + (s.shape[-1] + 8) * 2.0 ** -24) * (p @ np.abs(v))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=lambda d: NAME[d])
+@pytest.mark.parametrize("D", [4, 8, 24, 32, 40, 56, 72, 80, 96, 104, 120, 136])
+@pytest.mark.parametrize("B,H,Sq,Skv,causal,mask", [(1, 1, 1, 1, False, False), (2, 3, 33, 65, False, True), (1, 8, 127, 127, True, False), (2, 4, 130, 200, True, True),
+                                                    (1, 2, 257, 63, True, False), (3, 1, 5, 321, False, False)], ids=lambda v: str(v))
+def test_head_sizes(B, H, Sq, Skv, causal, mask, D, dtype):
+    from metalhlo_amd import kernels
+    rng = np.random.default_rng(D)
+    q, k, v = (to_dev(rng.standard_normal((B, H, n, D)), dtype) for n in (Sq, Skv, Skv))
+    md = None
+    if mask:
+        m = rng.standard_normal((B, 1, Sq, Skv))
+        m[..., Skv // 2:] = -np.inf
+        m[0, 0, Sq // 2] = -np.inf           # one row hides every key: zeros
+        md = to_dev(m, dtype)
+    scale = -0.3 if Skv == 65 else D ** -0.5
+    guard = torch.full((B * H * Sq * D + 64,), float("nan"), dtype=dtype, device="cuda")
+    got = kernels.flash_attention(q, k, v, scale=scale, is_causal=causal, mask=md, out=guard[:-64].view(B, H, Sq, D))
+    e, bound = _reference(as_f64(q), as_f64(k), as_f64(v), scale, causal, None if md is None else as_f64(md))
+    diff = np.abs(as_f64(got) - e)
+    tiny = 2.0 ** -24 if dtype == torch.float16 else 0.0       # f16's smallest numbers are evenly spaced
+    assert np.all(diff <= bound + ROUNDOFF[dtype] * (np.abs(e) + bound) + tiny), (diff.max(), np.abs(e).max())
+    assert torch.isnan(guard[-64:]).all()
