@@ -307,7 +307,8 @@ int64_t gemm_mid_workspace(int64_t M, int64_t N, int64_t K, int64_t batch);
 int launch_gemm_mid(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_a, int trans_b, int dtype, int64_t workspace_bytes);
 // gemm_f32.hip: fp32 operands on the fp32 matrix instruction, 128x128 tiles.
 bool gemm_f32_mfma_wanted(const GemmArgs& g);
-int launch_gemm_f32_mfma(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_a, int trans_b);
+int launch_gemm_f32_mfma(hipStream_t s, GemmArgs g, int64_t batch, int trans_a, int trans_b, int64_t workspace_bytes);
+int64_t gemm_f32_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b);
 // tuning.hip: variant prescribed by the tuning table for this problem, 0 = none.
 int tuned_gemm_variant(const GemmArgs& g, int64_t batch, int ta, int tb, int dtype);
 
@@ -529,8 +530,11 @@ using namespace mhip;
 // Where the few-row kernel is ahead of 64-row tiles (16-bit operands with aligned rows): up to 16 rows always,
 // up to 32 for weights of up to 32 M elements -- beyond that A, re-read for every strip of columns, costs as much
 // L2 traffic as B ([28,6384] x [6384,688] 9.2 us against 12.1; [37,768] x [768,50304] 37 against 16.6).
-static bool skinny_rows(int64_t M, int64_t N, int64_t K, bool is16) {
-    return M <= 16 || !is16 || (M <= 32 && N * K <= (32 << 20));
+// fp32 up to 64 rows always, and up to 192 while 64x64 tiles would leave compute units idle: [128,4096] x K 1024 (128 tiles)
+// 18.9 us against 25.5, [192,4096] x K 1024 (192) 25.7 against 26.1, [192,16384] x K 8192 (768) 606 against 430.
+static bool skinny_rows(int64_t M, int64_t N, int64_t K, int64_t batch, bool is16) {
+    if (!is16) return M <= 64 || (M <= 192 && (M + 63) / 64 * ((N + 63) / 64) * batch <= 160);
+    return M <= 16 || (M <= 32 && N * K <= (32 << 20));
 }
 
 // 16-bit operands without vector alignment.  The few-row kernel loads those element by element: it is ahead of
@@ -577,7 +581,7 @@ static int gemm_entry(void* stream, const void* a, const void* b, const void* bi
     g.partial = static_cast<float*>(workspace);
     // Few rows: the kernel that reads B once with all of its loads in flight, unless a tile kernel is asked for by
     // name or by the tuning table.
-    if ((is16 || dtype == MHIP_F32) && gemm_skinny_eligible(g, trans_a, is16 ? 2 : 4) && (is16 && !vec_ok ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, is16)) &&
+    if ((is16 || dtype == MHIP_F32) && gemm_skinny_eligible(g, trans_a, is16 ? 2 : 4) && (is16 && !vec_ok ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, batch, is16)) &&
         tune_int("MHIP_GEMM_TILE", 0) == 0 && tune_int("MHIP_GEMM_F32_MFMA", 1) == 1 &&
         (!is16 || few_row_choice(tuned_gemm_variant(g, batch, trans_a, trans_b, dtype)) || !vec_ok))
         return chose(vec_ok ? 64 : 0, launch_gemm_skinny(s, g, batch, trans_b, dtype, workspace_bytes));
@@ -587,7 +591,7 @@ static int gemm_entry(void* stream, const void* a, const void* b, const void* bi
     }
     switch (dtype) {
         case MHIP_F32:
-            if (gemm_f32_mfma_wanted(g)) return launch_gemm_f32_mfma(s, g, batch, trans_a, trans_b);
+            if (gemm_f32_mfma_wanted(g)) return launch_gemm_f32_mfma(s, g, batch, trans_a, trans_b, workspace_bytes);
             return launch_simple<float>(s, g, batch, trans_a, trans_b);
         case MHIP_BF16:
         case MHIP_F16:
@@ -633,9 +637,10 @@ extern "C" int64_t mhip_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t 
     const bool is16 = dtype == MHIP_BF16 || dtype == MHIP_F16;
     if (!is16 && dtype != MHIP_F32) return 0;
     const bool vec = is16 && (trans_a ? M : K) % 8 == 0 && (trans_b ? K : N) % 8 == 0;
-    if (!trans_a && M <= 64 && (is16 && !vec ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, is16))) return gemm_skinny_workspace(M, N, K, batch, trans_b);
+    if (!trans_a && M <= (is16 ? 64 : 192) && (is16 && !vec ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, batch, is16))) return gemm_skinny_workspace(M, N, K, batch, trans_b);
     // (a large problem goes to the ring kernels, whose tiles fill the device)
-    if (is16 && !vec) return short_product(M, N, K) ? 0 : gemm_any_workspace(M, N, K, batch);
-    if (!vec || (M > 192 && (double)M * N * batch >= 192.0 * 256 * 256)) return 0;
+    if (!is16) return gemm_f32_workspace(M, N, K, batch, trans_a, trans_b);
+    if (!vec) return short_product(M, N, K) ? 0 : gemm_any_workspace(M, N, K, batch);
+    if (M > 192 && (double)M * N * batch >= 192.0 * 256 * 256) return 0;
     return gemm_mid_workspace(M, N, K, batch);
 }

@@ -1,6 +1,8 @@
 // fp32 GEMM on the matrix cores of gfx950: v_mfma_f32_32x32x2_f32 (fp32 operands, fp32
 // accumulate -- the products are exact fp32 products, so the 1e-5 bar of fp32 programs holds).
 //
+// Operands whose rows are 16-byte aligned go through the ring further down; this kernel takes the others.
+//
 // One workgroup = a 64x64 tile of C, four waves (2 x 2), one 32x32 accumulator each (or a
 // 128x128 tile, 2 x 2 accumulators per wave).  K advances in steps of 16 through two LDS stage buffers: while a
 // step is multiplied, the next step's operands travel global -> registers, and are written to
@@ -17,11 +19,15 @@
 // The product is issued as (B, A), so an accumulator comes out transposed: a lane holds one
 // row m of the block and, per register group of four, four consecutive columns -- rows of C
 // are written with 16-byte stores.
+#include <mutex>
 #include <type_traits>
 
-#include "gemm_common.h"
+#include "gemm_lds.h"
 
 namespace mhip {
+
+int launch_gemm_finish(hipStream_t s, const GemmArgs& g, int dtype);     // gemm_mid.hip
+
 namespace {
 
 constexpr int kStep = 16;       // k per stage
@@ -35,9 +41,9 @@ constexpr int lds_floats(int rows) { return rows * kPad + 4 * (rows / 16); }
 
 // Copies this thread's share (NF = TILE / 16 floats) of one operand's [TILE x 16] stage into
 // registers.  K_CONTIG: element (row, k) at p[row * ld + k]; otherwise at p[k * ld + row].
-// Out-of-range rows / k read as zero.  `vec` = rows and k offsets are 16-byte aligned.
+// Out-of-range rows / k read as zero.  (A global load of 16 bytes needs no alignment.)
 template <bool K_CONTIG, int NF>
-__device__ inline void stage_load(const float* __restrict__ p, int ld, int row0, int rows, int k0, int K, bool vec, float (&r)[NF]) {
+__device__ inline void stage_load(const float* __restrict__ p, int ld, int row0, int rows, int k0, int K, float (&r)[NF]) {
     const int t = threadIdx.x;
     constexpr int TPR = 16 / NF;           // threads per row of a k-contiguous stage
     if (K_CONTIG) {
@@ -45,8 +51,9 @@ __device__ inline void stage_load(const float* __restrict__ p, int ld, int row0,
 #pragma unroll
         for (int h = 0; h < NF / 4; h++) {
             const int kk = k + 4 * h;
-            if (vec && row < rows && kk + 4 <= K) {
-                const f32x4 v = *reinterpret_cast<const f32x4*>(p + (int64_t)row * ld + kk);
+            if (row < rows && kk + 4 <= K) {
+                f32x4 v;
+                __builtin_memcpy(&v, p + (int64_t)row * ld + kk, 16);
                 r[4 * h + 0] = v[0]; r[4 * h + 1] = v[1]; r[4 * h + 2] = v[2]; r[4 * h + 3] = v[3];
             } else {
 #pragma unroll
@@ -58,8 +65,9 @@ __device__ inline void stage_load(const float* __restrict__ p, int ld, int row0,
 #pragma unroll
         for (int h = 0; h < NF / 4; h++) {
             const int rr = row + 4 * h;
-            if (vec && k < K && rr + 4 <= rows) {
-                const f32x4 v = *reinterpret_cast<const f32x4*>(p + (int64_t)k * ld + rr);
+            if (k < K && rr + 4 <= rows) {
+                f32x4 v;
+                __builtin_memcpy(&v, p + (int64_t)k * ld + rr, 16);
                 r[4 * h + 0] = v[0]; r[4 * h + 1] = v[1]; r[4 * h + 2] = v[2]; r[4 * h + 3] = v[3];
             } else {
 #pragma unroll
@@ -84,9 +92,54 @@ __device__ inline void stage_store(float* lds, const float (&r)[NF]) {
     }
 }
 
+// The wave's (32 WB) x (32 WB) block at (row0, col0) of C, or of this split's sums.
+template <int WB>
+__device__ __forceinline__ void store_f32(const GemmArgs& g, const f32x16 (&acc)[WB][WB], int row0, int col0, int64_t batch, int lane) {
+    const int lrow = lane & 31, lhalf = lane >> 5;
+    float* c = g.partial ? g.partial + (int64_t)blockIdx.z * g.M * g.N : static_cast<float*>(g.c) + batch * g.sc;
+    const float* res = g.residual && !g.partial ? static_cast<const float*>(g.residual) + batch * g.sc : nullptr;
+    // lane = row m of the block; register 4q + e = column 8q + 4 * lhalf + e
+    const float* bias = g.partial ? nullptr : static_cast<const float*>(g.bias);
+    const int act = g.partial ? MHIP_ACT_NONE : g.act;
+    const bool rows_vec = g.N % 4 == 0 && (reinterpret_cast<uintptr_t>(c) & 15) == 0 &&
+                          (!res || (reinterpret_cast<uintptr_t>(res) & 15) == 0);
+#pragma unroll
+    for (int i = 0; i < WB; i++) {
+        const int m = row0 + i * 32 + lrow;
+#pragma unroll
+        for (int j = 0; j < WB; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int n = col0 + j * 32 + 8 * q + 4 * lhalf;
+                if (m >= g.M || n >= g.N) continue;
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    float x = acc[i][j][4 * q + e];
+                    if (bias && n + e < g.N) x += bias[n + e];
+                    if (act != MHIP_ACT_NONE) x = apply_act(x, act);
+                    v[e] = x;
+                }
+                float* dst = c + (int64_t)m * g.N + n;
+                if (rows_vec && n + 4 <= g.N) {
+                    f32x4 o = {v[0], v[1], v[2], v[3]};
+                    if (res) {
+                        const f32x4 r = *reinterpret_cast<const f32x4*>(res + (int64_t)m * g.N + n);
+                        o += r;
+                    }
+                    *reinterpret_cast<f32x4*>(dst) = o;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (n + e < g.N) dst[e] = res ? v[e] + res[(int64_t)m * g.N + n + e] : v[e];
+                }
+            }
+    }
+}
+
 // WB = 32x32 accumulator blocks per wave and side: tile = (64 WB) x (64 WB)
 template <bool TA, bool TB, int WB>
-__global__ __launch_bounds__(256, 2) void gemm_f32_mfma_kernel(GemmArgs g, int vec_a, int vec_b) {
+__global__ __launch_bounds__(256, 2) void gemm_f32_mfma_kernel(GemmArgs g) {
     constexpr int kTile = 64 * WB, NF = kTile / 16;
     __shared__ __attribute__((aligned(16))) float lds[2][2][lds_floats(kTile)];   // [stage][A | B]
     int tm, tn;
@@ -95,8 +148,6 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_mfma_kernel(GemmArgs g, int v
     const int64_t batch = blockIdx.y;
     const float* a = static_cast<const float*>(g.a) + batch * g.sa;
     const float* b = static_cast<const float*>(g.b) + batch * g.sb;
-    float* c = static_cast<float*>(g.c) + batch * g.sc;
-    const float* res = g.residual ? static_cast<const float*>(g.residual) + batch * g.sc : nullptr;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int lrow = lane & 31, lhalf = lane >> 5;
@@ -111,8 +162,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_mfma_kernel(GemmArgs g, int v
 
     float ra[NF], rb[NF];
     // A in memory: [M, K] (k contiguous) unless TA; B in memory: [K, N] (n contiguous) unless TB
-    stage_load<!TA, NF>(a, g.lda, m0, g.M, 0, g.K, vec_a, ra);
-    stage_load<TB, NF>(b, g.ldb, n0, g.N, 0, g.K, vec_b, rb);
+    stage_load<!TA, NF>(a, g.lda, m0, g.M, 0, g.K, ra);
+    stage_load<TB, NF>(b, g.ldb, n0, g.N, 0, g.K, rb);
     stage_store<!TA, NF>(lds[0][0], ra);
     stage_store<TB, NF>(lds[0][1], rb);
     __syncthreads();
@@ -120,8 +171,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_mfma_kernel(GemmArgs g, int v
     for (int t = 0; t < steps; t++) {
         const int cur = t & 1;
         if (t + 1 < steps) {
-            stage_load<!TA, NF>(a, g.lda, m0, g.M, (t + 1) * kStep, g.K, vec_a, ra);
-            stage_load<TB, NF>(b, g.ldb, n0, g.N, (t + 1) * kStep, g.K, vec_b, rb);
+            stage_load<!TA, NF>(a, g.lda, m0, g.M, (t + 1) * kStep, g.K, ra);
+            stage_load<TB, NF>(b, g.ldb, n0, g.N, (t + 1) * kStep, g.K, rb);
         }
         f32x4 fa[WB][2], fb[WB][2];
 #pragma unroll
@@ -147,42 +198,132 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_mfma_kernel(GemmArgs g, int v
         __syncthreads();
     }
 
-    // lane = row m of the block; register 4q + e = column 8q + 4 * lhalf + e
-    const float* bias = static_cast<const float*>(g.bias);
-    const bool rows_vec = g.N % 4 == 0 && (reinterpret_cast<uintptr_t>(c) & 15) == 0 &&
-                          (!res || (reinterpret_cast<uintptr_t>(res) & 15) == 0);
+    store_f32<WB>(g, acc, m0 + wm * 32 * WB, n0 + wn * 32 * WB, batch, lane);
+}
+
+// ---- operands whose rows are 16-byte aligned: a ring of LDS stages filled by the loads themselves ----
+//
+// With one stage of 16 k in flight a problem that does not fill the device waits out a load latency per stage
+// (0.55 us; the stage's matrix instructions take 0.21).  [2048,2048] x K 2048 173 -> 143 us (120 TFLOP/s),
+// [512,768] x K 768 26.7 -> 19.7, 4096^3 1183 -> 1038 (132).  Here S stages of 32 k come straight into LDS (no
+// register stop), S - 1 of them in flight, one barrier per stage.  A k-contiguous operand lies there as rows of
+// 128 bytes (lane = row, 16 bytes = four consecutive k), the other one as it lies in memory, [32 k][rows], read
+// one float per lane with the rows k and k + 4 that one issue takes on different halves of the banks.
+// An issue sums k = 8 s + e (lower half of the wave) and 8 s + 4 + e (upper half).
+template <int ROWS, bool KMAJOR>
+struct RingLoader {
+    static constexpr int kLoads = ROWS * kRowBytes / 1024 / 4;      // wave-wide loads of 1 KB per stage and wave
+    uint32_t off[kLoads];      // byte offset in stage 0, kOob where the row / column does not exist
+    int k[kLoads];             // first k of the piece inside the stage
+    uint32_t step;
+    __device__ void init(int row0, int rows_total, int ld, int wave, int lane) {
+        step = (uint32_t)(KMAJOR ? 128 : (int64_t)32 * ld * 4);
 #pragma unroll
-    for (int i = 0; i < WB; i++) {
-        const int m = m0 + wm * 32 * WB + i * 32 + lrow;
+        for (int i = 0; i < kLoads; i++) {
+            const int p = (i * 4 + wave) * 64 + lane;               // 16-byte slot of the tile
+            if (KMAJOR) {
+                const int r = p >> 3, c = (p & 7) ^ swz(r);
+                k[i] = c * 4;
+                off[i] = row0 + r < rows_total ? (uint32_t)(((int64_t)(row0 + r) * ld + c * 4) * 4) : kOob;
+            } else {
+                constexpr int kCpr = ROWS / 4;
+                const int kk = p / kCpr, c = (p % kCpr) ^ (kk >> 2 & 1) << 3;
+                k[i] = kk;
+                off[i] = row0 + c * 4 < rows_total ? (uint32_t)(((int64_t)kk * ld + row0 + c * 4) * 4) : kOob;
+            }
+        }
+    }
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rsrc, uint32_t tile, int wave, int kt, int K) const {
+        const uint32_t at = (uint32_t)kt * step;
+#pragma unroll
+        for (int i = 0; i < kLoads; i++) {
+            const bool ok = off[i] != kOob && kt * 32 + k[i] < K;
+            load_to_lds(rsrc, tile + (uint32_t)(i * 4 + wave) * 1024u, ok ? off[i] + at : kOob);
+        }
+    }
+};
+
+// The four k of this lane's half in step s (of eight k) of one 32-row block.
+template <int ROWS, bool KMAJOR>
+__device__ __forceinline__ f32x4 ring_frag(const char* tile, int row0, int s, int lane) {
+    const int r = row0 + (lane & 31), h = lane >> 5;
+    if (KMAJOR) return *reinterpret_cast<const f32x4*>(tile + lds_off(r, 2 * s + h));
+    const char* p = tile + (8 * s + 4 * h) * (ROWS * 4) + ((r ^ h << 5) << 2);
+    f32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = *reinterpret_cast<const float*>(p + e * (ROWS * 4));
+    return v;
+}
+
+template <bool TA, bool TB, int WB, int S>
+__global__ __launch_bounds__(256) void gemm_f32_ring_kernel(GemmArgs g) {
+    constexpr int kTile = 64 * WB, kBytes = kTile * kRowBytes, kStage = 2 * kBytes;
+    extern __shared__ __attribute__((aligned(1024))) char smem[];
+    int tm, tn;
+    tile_of(blockIdx.x, gridDim.x, g.tiles_m, g.tiles_n, tm, tn);
+    const int m0 = tm * kTile, n0 = tn * kTile;
+    const int64_t batch = blockIdx.y;
+    const float* a = static_cast<const float*>(g.a) + batch * g.sa;
+    const float* b = static_cast<const float*>(g.b) + batch * g.sb;
+    const __amdgpu_buffer_rsrc_t ra = make_rsrc(a, (uint32_t)((int64_t)g.M * g.K * 4)), rb = make_rsrc(b, (uint32_t)((int64_t)g.N * g.K * 4));
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    // this workgroup's stages: all of K, or one split's
+    const int all = (g.K + 31) / 32, per = (all + g.splits - 1) / g.splits;
+    const int kt0 = (int)blockIdx.z * per, kt1 = min(all, kt0 + per), kend = min(g.K, kt1 * 32);
+    RingLoader<kTile, !TA> la;
+    RingLoader<kTile, TB> lb;
+    la.init(m0, g.M, g.lda, wave, lane);
+    lb.init(n0, g.N, g.ldb, wave, lane);
+    constexpr int kLoads = 2 * RingLoader<kTile, !TA>::kLoads;
+    // (a stage behind the last one is loaded all the same, out of bounds: the waits count loads)
+    const uint32_t ring = lds_address(smem);
+    auto load = [&](int kt) {
+        const uint32_t st = ring + (uint32_t)((kt - kt0) % S) * kStage;
+        la.load(ra, st, wave, kt, kend);
+        lb.load(rb, st + kBytes, wave, kt, kend);
+    };
+
+    f32x16 acc[WB][WB];
+#pragma unroll
+    for (int i = 0; i < WB; i++)
 #pragma unroll
         for (int j = 0; j < WB; j++)
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int n = n0 + wn * 32 * WB + j * 32 + 8 * q + 4 * lhalf;
-                if (m >= g.M || n >= g.N) continue;
-                float v[4];
+            for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    float x = acc[i][j][4 * q + e];
-                    if (bias && n + e < g.N) x += bias[n + e];
-                    if (g.act != MHIP_ACT_NONE) x = apply_act(x, g.act);
-                    v[e] = x;
-                }
-                float* dst = c + (int64_t)m * g.N + n;
-                if (rows_vec && n + 4 <= g.N) {
-                    f32x4 o = {v[0], v[1], v[2], v[3]};
-                    if (res) {
-                        const f32x4 r = *reinterpret_cast<const f32x4*>(res + (int64_t)m * g.N + n);
-                        o += r;
-                    }
-                    *reinterpret_cast<f32x4*>(dst) = o;
-                } else {
+    for (int p = 0; p < S - 1; p++) load(kt0 + p);
+    for (int kt = kt0; kt < kt1; kt++) {
+        // stage kt has landed when only the S - 2 stages behind it are in flight; past the barrier that holds for
+        // every wave's share, and every wave has read stage kt - 1, whose place is reused
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * kLoads) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        load(kt + S - 1);
+        const char* at = smem + ((kt - kt0) % S) * kStage;
+        f32x4 af[2][WB], bf[2][WB];
+        auto read = [&](int s, f32x4(&fa)[WB], f32x4(&fb)[WB]) {
 #pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        if (n + e < g.N) dst[e] = res ? v[e] + res[(int64_t)m * g.N + n + e] : v[e];
-                }
+            for (int i = 0; i < WB; i++) {
+                fa[i] = ring_frag<kTile, !TA>(at, (wm * WB + i) * 32, s, lane);
+                fb[i] = ring_frag<kTile, TB>(at + kBytes, (wn * WB + i) * 32, s, lane);
             }
+        };
+        read(0, af[0], bf[0]);
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            if (s < 3) read(s + 1, af[(s + 1) & 1], bf[(s + 1) & 1]);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int i = 0; i < WB; i++)
+#pragma unroll
+                    for (int j = 0; j < WB; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(bf[s & 1][j][e], af[s & 1][i][e], acc[i][j], 0, 0, 0);
+        }
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // nothing may land in LDS after the workgroup ends
+    store_f32<WB>(g, acc, m0 + wm * 32 * WB, n0 + wn * 32 * WB, batch, lane);
 }
 
 template <bool TA, bool TB, int WB>
@@ -192,23 +333,54 @@ int launch_tile(hipStream_t s, GemmArgs g, int64_t batch) {
     g.tiles_n = (g.N + kTile - 1) / kTile;
     const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n;
     if (tiles > 0x7FFFFFFFLL || batch > 65535) return fail(MHIP_ERR_UNSUPPORTED, "gemm: grid too large");
-    auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    const int vec_a = al(g.a) && g.lda % 4 == 0 && g.sa % 4 == 0;
-    const int vec_b = al(g.b) && g.ldb % 4 == 0 && g.sb % 4 == 0;
-    hipLaunchKernelGGL((gemm_f32_mfma_kernel<TA, TB, WB>), dim3((unsigned)tiles, (unsigned)batch), dim3(256), 0, s, g, vec_a, vec_b);
+    hipLaunchKernelGGL((gemm_f32_mfma_kernel<TA, TB, WB>), dim3((unsigned)tiles, (unsigned)batch), dim3(256), 0, s, g);
     return check_launch("gemm_f32_mfma");
 }
 
-// 128x128 tiles (three workgroups resident per CU: 768 on the device) once there are enough of
-// them for a round and a quarter, 64x64 tiles (eight per CU) below that.  Measured (TFLOP/s,
-// 64 | 128): 4096^3 101 | 116, [8192,3072] x K 768 (1536 large tiles) 100 | 113; [3000,3000] x K 1000
-// (576) 89 | 73, [2048,2048] x K 2048 (256) 99 | 91, [8192,768] x K 3072 (384) 100 | 87, 1024^3 (64)
-// 62 | 23.
+template <bool TA, bool TB, int WB, int S>
+int launch_ring(hipStream_t s, GemmArgs g, int64_t batch) {
+    constexpr int kTile = 64 * WB, kSmem = S * 2 * kTile * kRowBytes;
+    auto kern = gemm_f32_ring_kernel<TA, TB, WB, S>;
+    if (kSmem > 64 * 1024) {
+        static std::once_flag once;
+        static hipError_t err = hipSuccess;
+        std::call_once(once, [&] { err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kSmem); });
+        if (err != hipSuccess) return fail(MHIP_ERR_LAUNCH, "gemm: cannot reserve %d bytes of LDS: %s", kSmem, hipGetErrorString(err));
+    }
+    g.tiles_m = (g.M + kTile - 1) / kTile;
+    g.tiles_n = (g.N + kTile - 1) / kTile;
+    const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n;
+    if (tiles > 0x7FFFFFFFLL || batch > 65535) return fail(MHIP_ERR_UNSUPPORTED, "gemm: grid too large");
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)batch, (unsigned)g.splits), dim3(256), kSmem, s, g);
+    return check_launch("gemm_f32_ring");
+}
+
+int64_t large_tiles(int64_t M, int64_t N, int64_t batch) { return ((M + 127) / 128) * ((N + 127) / 128) * batch; }
+
+// 128x128 tiles once there are enough of them for a round and a quarter of three per compute unit, 64x64 tiles (five
+// per compute unit) below that.  Measured with the ring (us, 64 | 128): 4096^3 1060 | 1038, 2048^3 143 | 157,
+// [8192,768] x K 3072 308 | 405; register-staged 1183 at 4096^3 (128), 173 at 2048^3 and 382 (64).  Rings of
+// three and four stages are 2 to 8 % behind two: the workgroups of a unit hide each other's latency.
 template <bool TA, bool TB>
-int launch(hipStream_t s, const GemmArgs& g, int64_t batch) {
-    const int64_t large_tiles = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * batch;
-    if (large_tiles >= 960) return launch_tile<TA, TB, 2>(s, g, batch);
-    return launch_tile<TA, TB, 1>(s, g, batch);
+int launch(hipStream_t s, const GemmArgs& g, int64_t batch, bool ring) {
+    const bool large = large_tiles(g.M, g.N, batch) >= 960 && g.splits == 1;
+    if (ring) return large ? launch_ring<TA, TB, 2, 2>(s, g, batch) : launch_ring<TA, TB, 1, 2>(s, g, batch);
+    return large ? launch_tile<TA, TB, 2>(s, g, batch) : launch_tile<TA, TB, 1>(s, g, batch);
+}
+
+// Parts of K where a workspace takes them and half of the compute units have no tile: up to two workgroups per compute
+// unit, each with at least 512 k ([512,512] x K 16384 488 -> 89 us; 192 tiles in two parts, [192,4096] x K 1024, take
+// 30.8 us against 26.1 whole).  As with 16-bit operands a sum is left in one piece from 193 rows on unless K is 4096 or more.
+int ring_splits(int64_t M, int64_t N, int64_t K, int64_t batch) {
+    const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
+    if (batch != 1 || tiles > 128 || (M > 192 && K < 4096)) return 1;
+    const int64_t room = 512 / tiles, most = K / 512;
+    const int64_t n = room < most ? room : most;
+    return n < 2 ? 1 : n > 8 ? 8 : (int)n;
+}
+
+bool ring_sizes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb) {
+    return lda % 4 == 0 && ldb % 4 == 0 && M * K < 0x1FFFFFFF && N * K < 0x1FFFFFFF;
 }
 
 }  // namespace
@@ -222,11 +394,22 @@ bool gemm_f32_mfma_wanted(const GemmArgs& g) {
     return mode == 3 || ((int64_t)g.M * g.N >= 48 * 48 && g.K >= 16);
 }
 
-int launch_gemm_f32_mfma(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_a, int trans_b) {
-    if (!trans_a && !trans_b) return launch<false, false>(s, g, batch);
-    if (!trans_a && trans_b) return launch<false, true>(s, g, batch);
-    if (trans_a && !trans_b) return launch<true, false>(s, g, batch);
-    return launch<true, true>(s, g, batch);
+int64_t gemm_f32_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b) {
+    if (!ring_sizes(M, N, K, trans_a ? M : K, trans_b ? K : N)) return 0;
+    const int n = ring_splits(M, N, K, batch);
+    return n == 1 ? 0 : M * N * 4 * n;
+}
+
+// Without the workspace (g.partial), or with a smaller one, K is not split.
+int launch_gemm_f32_mfma(hipStream_t s, GemmArgs g, int64_t batch, int trans_a, int trans_b, int64_t workspace_bytes) {
+    const bool ring = ring_sizes(g.M, g.N, g.K, g.lda, g.ldb) && g.sa % 4 == 0 && g.sb % 4 == 0 &&
+                      ((reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.b)) & 15) == 0;
+    g.splits = ring && g.partial ? ring_splits(g.M, g.N, g.K, batch) : 1;
+    if ((int64_t)g.M * g.N * 4 * g.splits > workspace_bytes) g.splits = 1;
+    if (g.splits == 1) g.partial = nullptr;
+    const int st = !trans_a ? (!trans_b ? launch<false, false>(s, g, batch, ring) : launch<false, true>(s, g, batch, ring))
+                            : (!trans_b ? launch<true, false>(s, g, batch, ring) : launch<true, true>(s, g, batch, ring));
+    return st != MHIP_OK || g.splits == 1 ? st : launch_gemm_finish(s, g, MHIP_F32);
 }
 
 }  // namespace mhip

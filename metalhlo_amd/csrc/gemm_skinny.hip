@@ -1,5 +1,5 @@
-// dot_general with few rows: C = act(A . op(B) + bias) (+ residual) for M <= 64 (a decode step, a short
-// prompt, a small batch), where the product costs nothing and the time is that of reading B once.
+// dot_general with few rows: C = act(A . op(B) + bias) (+ residual) for M <= 64, fp32 also in blocks of rows up
+// to 192 (a decode step, a short prompt, a small batch), where the product costs nothing and the time is that of reading B once.
 //
 // A tile kernel leaves such a problem on a handful of workgroups ([4,4096] x [4096,4096]: 32 tiles of
 // 128 columns on 256 compute units, each walking K through LDS one load latency at a time).  Here
@@ -109,7 +109,9 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(GemmArgs g) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     const int li = lane & 15, lg = lane >> 4;
     const int n0 = blockIdx.x * NS;
-    const int64_t batch = blockIdx.y;
+    int batch_i = blockIdx.y, m0 = 0;
+    if (g.tiles_m > 1) { m0 = batch_i % g.tiles_m * (16 * MT); batch_i /= g.tiles_m; }
+    const int64_t batch = batch_i;
     const T* a = static_cast<const T*>(g.a) + batch * g.sa;
     const T* b = static_cast<const T*>(g.b) + batch * g.sb;
     const __amdgpu_buffer_rsrc_t ra = skinny_rsrc(a, (uint32_t)((int64_t)g.M * g.lda * sizeof(T)));
@@ -123,7 +125,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(GemmArgs g) {
 
     uint32_t arow[MT];
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) arow[mt] = (uint32_t)(min(mt * 16 + li, g.M - 1) * g.lda);
+    for (int mt = 0; mt < MT; mt++) arow[mt] = (uint32_t)(min(m0 + mt * 16 + li, g.M - 1) * g.lda);
 
     f32x4 acc[NF][MT];
 #pragma unroll
@@ -202,7 +204,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(GemmArgs g) {
     T* c = static_cast<T*>(g.c) + batch * g.sc;
     auto finish = [&](auto act_tag) {
         constexpr int ACT = decltype(act_tag)::value;
-        const int total = min(g.M, 16 * MT) * NS;
+        const int total = min(g.M - m0, 16 * MT) * NS;
         for (int idx = threadIdx.x; idx < total; idx += blockDim.x) {
             const int m = idx / NS, nl = idx % NS, n = n0 + nl;
             if (n >= g.N) continue;
@@ -211,13 +213,13 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(GemmArgs g) {
             float v = 0.f;
             for (int w = 0; w < waves; w++) v += p[w * (NF * MT * 256)];
             if (g.partial) {
-                g.partial[((int64_t)blockIdx.z * g.M + m) * g.N + n] = v;
+                g.partial[((int64_t)blockIdx.z * g.M + m0 + m) * g.N + n] = v;
                 continue;
             }
             if (bias) v += Elem<T>::to_f32(bias[n]);
             v = sizeof(T) == 4 ? apply_act(v, ACT) : apply_act_c<ACT>(v);
             T o = Elem<T>::from_f32(v);
-            const int64_t at = (int64_t)m * g.N + n;
+            const int64_t at = (int64_t)(m0 + m) * g.N + n;
             // (second rounding on purpose: the same result as a separate add over the stored C)
             if (res) o = Elem<T>::from_f32(Elem<T>::to_f32(o) + Elem<T>::to_f32(res[at]));
             c[at] = o;
@@ -227,7 +229,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(GemmArgs g) {
 }
 
 template <typename T, bool TB, bool VEC, int NF, int MT, int U, int WAVES = 8>
-int launch_one(hipStream_t s, const GemmArgs& g, int64_t batch) {
+int launch_one(hipStream_t s, GemmArgs g, int64_t batch) {
     constexpr int KS = 4 * Mfma16<T>::kKpl;
     auto kern = gemm_skinny_kernel<T, TB, VEC, NF, MT, U, WAVES>;
     constexpr int kLds = WAVES * NF * MT * 1024;
@@ -241,8 +243,9 @@ int launch_one(hipStream_t s, const GemmArgs& g, int64_t batch) {
     const int steps = ((g.K + KS - 1) / KS + g.splits - 1) / g.splits, want = (steps + U - 1) / U;
     const int waves = want < 1 ? 1 : want > WAVES ? WAVES : want;
     const int64_t strips = (g.N + 16 * NF - 1) / (16 * NF);
-    if (strips > 0x7FFFFFFFLL || batch > 65535) return fail(MHIP_ERR_UNSUPPORTED, "gemm: grid too large");
-    hipLaunchKernelGGL(kern, dim3((unsigned)strips, (unsigned)batch, (unsigned)g.splits), dim3(64 * waves), waves * NF * MT * 1024, s, g);
+    g.tiles_m = (g.M + 16 * MT - 1) / (16 * MT);
+    if (strips > 0x7FFFFFFFLL || batch * g.tiles_m > 65535) return fail(MHIP_ERR_UNSUPPORTED, "gemm: grid too large");
+    hipLaunchKernelGGL(kern, dim3((unsigned)strips, (unsigned)(batch * g.tiles_m), (unsigned)g.splits), dim3(64 * waves), waves * NF * MT * 1024, s, g);
     return check_launch("gemm_skinny");
 }
 
@@ -270,6 +273,17 @@ template <typename T, bool TB, bool VEC>
 int launch_shape(hipStream_t s, const GemmArgs& g, int64_t batch) {
     constexpr bool k16 = sizeof(T) == 2;
     const bool wide = wide_strips(g.N, g.K, batch, TB);
+    if constexpr (!k16) {
+        // fp32 from 33 rows on: blocks of 32 rows by 16 columns until every compute unit has one, beyond that by 32 columns
+        // unless the strips are wide, whose blocks of 64 rows read B half as often.  us, 32 x 16 / 32 x 32 / 64 rows:
+        // [128,768] x K 768 (192 of the first) 6.7 / 9.1 / 10.0 and K 3072 15.9 / 21.2 / 27.1, [64,2304] x K 768 (288)
+        // 10.0 / 9.2 / 10.1, [128,4096] x K 1024 (1024) 23.0 / 18.9 / 23.1, [64,8192] x K 4096 (wide) - / 59.1 / 52.3.  Up to
+        // 64 rows a split K fills the device as it is: [36,768] x K 8192 24.4 / - / 20.8.
+        if (g.M > 32 && (g.M > 64 || g.splits == 1)) {
+            if ((g.N + 15) / 16 * ((g.M + 31) / 32) * batch <= 256) return launch_one<T, TB, VEC, 1, 2, 2>(s, g, batch);
+            if (!wide) return launch_one<T, TB, VEC, 2, 2, 2>(s, g, batch);
+        }
+    }
     if (g.M <= 16) {
         if (wide) return k16 || TB ? launch_one<T, TB, VEC, TB ? 2 : 4, 1, 2>(s, g, batch) : launch_one<T, TB, VEC, 2, 1, 2>(s, g, batch);
         return launch_one<T, TB, VEC, TB ? 1 : k16 ? 2 : 1, 1, 4>(s, g, batch);
@@ -303,9 +317,9 @@ int dtype_launch(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_b, i
 
 }  // namespace
 
-// What this kernel takes: A stored [M, K], at most 64 rows, operands that one buffer descriptor spans.
+// What this kernel takes: A stored [M, K], at most 64 rows (fp32: 192, in blocks), operands that one buffer descriptor spans.
 bool gemm_skinny_eligible(const GemmArgs& g, int trans_a, int elem_bytes) {
-    return !trans_a && g.M <= 64 && g.K > 0 && g.ldc == 0 && (int64_t)g.M * g.lda * elem_bytes < 0x7FFFFFFFLL &&
+    return !trans_a && g.M <= (elem_bytes == 4 ? 192 : 64) && g.K > 0 && g.ldc == 0 && (int64_t)g.M * g.lda * elem_bytes < 0x7FFFFFFFLL &&
            ((int64_t)g.N + 64) * g.K * elem_bytes < 0x7FFFFFFFLL && ((int64_t)g.K + 64) * g.N * elem_bytes < 0x7FFFFFFFLL;
 }
 
