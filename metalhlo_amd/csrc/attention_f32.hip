@@ -172,14 +172,157 @@ __global__ __launch_bounds__(256, 2) void fa_f32_mfma_kernel(FaArgs a, float sca
     }
 }
 
+// The same products with the KEYS dealt over the waves: a workgroup owns 32 query rows, wave w takes blocks w, w + 4, ...
+// of 32 keys and its own softmax state, and the four meet in LDS at the end.  Four times as many workgroups, each
+// with a quarter of the chain; K and V go from memory straight to the operand registers (a lane's 16 bytes of
+// its key's row serve four issues: k = 8 j + 4 h + e on both operands), so there is no barrier in the loop, and
+// each set of registers is loaded again as soon as its product has read it, half a block ahead of its use.
+template <int D, bool CAUSAL, bool HAS_MASK>
+__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaArgs a, float scale) {
+    constexpr int NS = D / 8, ND = D / 32;
+    __shared__ float part[4][32][33];
+    __shared__ float ml[2][4][32];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ln = lane & 31, h = lane >> 5;
+    int bh, qb;
+    tile_of_workgroup<CAUSAL>(a, blockIdx.x, bh, qb);
+    const int q0 = qb * 32, qpos = q0 + ln;
+    const bool q_live = qpos < a.Sq;
+    const float* qp = static_cast<const float*>(a.q) + (int64_t)bh * a.Sq * D;
+    const uint32_t bytes = (uint32_t)((int64_t)a.Skv * D * 4);
+    const __amdgpu_buffer_rsrc_t rk = fa_rsrc(static_cast<const float*>(a.k) + (int64_t)bh * a.Skv * D, bytes);
+    const __amdgpu_buffer_rsrc_t rv = fa_rsrc(static_cast<const float*>(a.v) + (int64_t)bh * a.Skv * D, bytes);
+    const float* mp = HAS_MASK ? static_cast<const float*>(a.mask) + (int64_t)(bh / a.H) * a.mask_sb +
+                                     (int64_t)(bh % a.H) * a.mask_sh + (int64_t)qpos * a.Skv
+                               : nullptr;
+    f32x4 qf[NS];
+#pragma unroll
+    for (int j = 0; j < NS; j++)
+        qf[j] = q_live ? *reinterpret_cast<const f32x4*>(qp + (int64_t)qpos * D + 8 * j + 4 * h) : f32x4{0.f, 0.f, 0.f, 0.f};
+
+    int nkv = (a.Skv + kFBK - 1) / kFBK;
+    if (CAUSAL) nkv = min(nkv, qb + 1);
+
+    // (keys past the end lie beyond the buffers' extents and read zero)
+    f32x4 kr[NS];
+    float vr[ND][16];
+    auto load_k = [&](int blk) __attribute__((always_inline)) {
+        const uint32_t off = (uint32_t)((blk * kFBK + ln) * (D * 4) + 16 * h);
+#pragma unroll
+        for (int j = 0; j < NS; j++) kr[j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, off + 32 * j, 0, 0));
+    };
+    auto load_v = [&](int blk) __attribute__((always_inline)) {
+        const uint32_t off = (uint32_t)((blk * kFBK + 4 * h) * (D * 4) + 4 * ln);
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+#pragma unroll
+            for (int d = 0; d < ND; d++)
+                vr[d][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, off + (uint32_t)((8 * (i >> 2) + (i & 3)) * (D * 4) + 128 * d), 0, 0));
+    };
+
+    f32x16 o[ND];
+#pragma unroll
+    for (int d = 0; d < ND; d++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) o[d][i] = 0.f;
+    float m_run = -INFINITY, l_run = 0.f;
+    if (wave < nkv) { load_k(wave); load_v(wave); }
+    for (int blk = wave; blk < nkv; blk += 4) {
+        const int kb = blk * kFBK;
+        f32x16 sacc;
+#pragma unroll
+        for (int i = 0; i < 16; i++) sacc[i] = 0.f;
+#pragma unroll
+        for (int j = 0; j < NS; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[j][e], qf[j][e], sacc, 0, 0, 0);
+        if (blk + 4 < nkv) load_k(blk + 4);
+        float t[16];
+        float m_blk = -INFINITY;
+        const bool edge = (CAUSAL && kb + kFBK - 1 > q0) || kb + kFBK > a.Skv;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int key = kb + f32_key(i, h);
+            float sv = sacc[i] * scale;
+            const bool keep = !edge || (key < a.Skv && (!CAUSAL || key <= qpos));
+            if (HAS_MASK) { if (q_live && key < a.Skv) sv += mp[key]; }
+            t[i] = keep ? sv * kLog2e : -INFINITY;
+            m_blk = fmaxf(m_blk, t[i]);
+        }
+        m_blk = half_max(m_blk);
+        const float m_new = moved_reference(m_run, m_blk);
+        const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+        m_run = m_new;
+        float psum = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            t[i] = __builtin_amdgcn_exp2f(t[i] - m_use);
+            psum += t[i];
+        }
+        l_run = l_run * alpha + psum;
+        if (__any(alpha != 1.f)) {
+#pragma unroll
+            for (int d = 0; d < ND; d++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) o[d][i] *= alpha;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+#pragma unroll
+            for (int d = 0; d < ND; d++) o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[d][i], t[i], o[d], 0, 0, 0);
+        if (blk + 4 < nkv) load_v(blk + 4);
+    }
+
+    // ---- the waves' states, 32 columns of the output at a time
+    l_run = half_sum(l_run);
+    if (h == 0) { ml[0][wave][ln] = m_run; ml[1][wave][ln] = l_run; }
+    float* op = static_cast<float*>(a.o) + (int64_t)bh * a.Sq * D;
+    const int col = threadIdx.x & 31, row0 = threadIdx.x >> 5;
+#pragma unroll
+    for (int d = 0; d < ND; d++) {
+        if (d) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 16; i++) part[wave][ln][f32_key(i, h)] = o[d][i];
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            const int q = row0 + 8 * p;
+            float m = -INFINITY, l = 0.f, sum = 0.f;
+#pragma unroll
+            for (int w = 0; w < 4; w++) m = fmaxf(m, ml[0][w][q]);
+            const float m_use = m == -INFINITY ? 0.f : m;
+#pragma unroll
+            for (int w = 0; w < 4; w++) {
+                const float al = __builtin_amdgcn_exp2f(ml[0][w][q] - m_use);
+                l = fmaf(ml[1][w][q], al, l);
+                sum = fmaf(part[w][q][col], al, sum);
+            }
+            if (q0 + q < a.Sq) op[(int64_t)(q0 + q) * D + 32 * d + col] = sum * (l > 1e-10f ? 1.f / l : 0.f);
+        }
+    }
+}
+
 template <int D>
 int launch_f32(hipStream_t s, FaArgs a, float scale, bool causal, bool has_mask) {
-    a.nqb = (a.Sq + kFBQ - 1) / kFBQ;
+    // Keys over the waves while tiles of 128 rows leave compute units idle or nearly so (us, 128 rows | split, causal):
+    // 12 tiles [1,12,128,64] 16.2 | 7.6; 64 [2,8,512,64] 48 | 16, D 128 83 | 29; 128 [1,8,2048,64] 175 | 50, D 128 302 | 114.
+    // From 256 on every wave re-reading K and V costs more than the shorter chain gives (256 tiles of D 96 40 | 48, 1024 of
+    // D 128 621 | 738), except where rows are short or keys many: 1024 tiles of D 32 174 | 165, 384 of [4,12,1000,64] 100 | 78
+    // (768 of [16,12,512,64] 81 | 95).
+    const int64_t tiles = (int64_t)a.B * a.H * ((a.Sq + kFBQ - 1) / kFBQ);
+    const bool split = ((int64_t)a.Skv + kFBQ) * D * 4 < 0x7FFFFFFFLL &&
+                       (tiles < 256 || (D == 32 && tiles <= 1024) || (D == 64 && tiles <= 512 && a.Skv >= 768));
+    const int rows = split ? 32 : kFBQ;
+    a.nqb = (a.Sq + rows - 1) / rows;
     set_tile_order(a);
     const int64_t grid = (int64_t)a.B * a.H * a.nqb;
     if (grid > 0x7FFFFFFFLL) return fail(MHIP_ERR_UNSUPPORTED, "flash_attention: grid too large");
-#define MHIP_FA32(C, M) \
-    hipLaunchKernelGGL((fa_f32_mfma_kernel<D, C, M>), dim3((unsigned)grid), dim3(256), 0, s, a, scale)
+#define MHIP_FA32(C, M)                                                                                                     \
+    do {                                                                                                                    \
+        if (split) hipLaunchKernelGGL((fa_f32_split_kernel<D, C, M>), dim3((unsigned)grid), dim3(256), 0, s, a, scale);     \
+        else hipLaunchKernelGGL((fa_f32_mfma_kernel<D, C, M>), dim3((unsigned)grid), dim3(256), 0, s, a, scale);            \
+    } while (0)
     if (causal && has_mask) MHIP_FA32(true, true);
     else if (causal) MHIP_FA32(true, false);
     else if (has_mask) MHIP_FA32(false, true);
