@@ -297,7 +297,7 @@ bool gemm_stream_eligible(const GemmArgs& g, int64_t batch, int trans_a, int tra
 int launch_gemm_stream(hipStream_t s, const GemmArgs& g, int trans_b, int dtype);
 // gemm_skinny.hip: at most 64 rows, the waves of a workgroup split K.
 bool gemm_skinny_eligible(const GemmArgs& g, int trans_a, int elem_bytes);
-int64_t gemm_skinny_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b);
+int64_t gemm_skinny_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b, bool is16);
 // gemm_any.hip: any alignment and size.
 int launch_gemm_any(hipStream_t s, GemmArgs g, int64_t batch, int trans_a, int trans_b, int dtype, int64_t workspace_bytes);
 int64_t gemm_any_workspace(int64_t M, int64_t N, int64_t K, int64_t batch);
@@ -532,9 +532,12 @@ using namespace mhip;
 // L2 traffic as B ([28,6384] x [6384,688] 9.2 us against 12.1; [37,768] x [768,50304] 37 against 16.6).
 // fp32 up to 64 rows always, and up to 192 while 64x64 tiles would leave compute units idle: [128,4096] x K 1024 (128 tiles)
 // 18.9 us against 25.5, [192,4096] x K 1024 (192) 25.7 against 26.1, [192,16384] x K 8192 (768) 606 against 430.
-static bool skinny_rows(int64_t M, int64_t N, int64_t K, int64_t batch, bool is16) {
+// 16-bit rows 33 to 64, in two blocks, with weights that were not just used: [37,768] x K 768 7.5 -> 6.7 us, [64,4096] x K 1024
+// 10.0 -> 8.9, but [64,8192] x K 768 9.0 against 11.6; stored [N, K]: [64,2000] x [1000,2000]^T 8.6 -> 6.5, [64,768] x [3072,768]^T
+// 5.9 against 7.3.
+static bool skinny_rows(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b, bool is16) {
     if (!is16) return M <= 64 || (M <= 192 && (M + 63) / 64 * ((N + 63) / 64) * batch <= 160);
-    return M <= 16 || (M <= 32 && N * K <= (32 << 20));
+    return M <= 16 || (M <= 32 && N * K <= (32 << 20)) || (M <= 64 && (trans_b ? N * batch <= 1536 && K <= 2048 : N * batch <= 4096 && K <= 1536));
 }
 
 // 16-bit operands without vector alignment.  The few-row kernel loads those element by element: it is ahead of
@@ -581,7 +584,7 @@ static int gemm_entry(void* stream, const void* a, const void* b, const void* bi
     g.partial = static_cast<float*>(workspace);
     // Few rows: the kernel that reads B once with all of its loads in flight, unless a tile kernel is asked for by
     // name or by the tuning table.
-    if ((is16 || dtype == MHIP_F32) && gemm_skinny_eligible(g, trans_a, is16 ? 2 : 4) && (is16 && !vec_ok ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, batch, is16)) &&
+    if ((is16 || dtype == MHIP_F32) && gemm_skinny_eligible(g, trans_a, is16 ? 2 : 4) && (is16 && !vec_ok ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, batch, trans_b, is16)) &&
         tune_int("MHIP_GEMM_TILE", 0) == 0 && tune_int("MHIP_GEMM_F32_MFMA", 1) == 1 &&
         (!is16 || few_row_choice(tuned_gemm_variant(g, batch, trans_a, trans_b, dtype)) || !vec_ok))
         return chose(vec_ok ? 64 : 0, launch_gemm_skinny(s, g, batch, trans_b, dtype, workspace_bytes));
@@ -637,7 +640,7 @@ extern "C" int64_t mhip_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t 
     const bool is16 = dtype == MHIP_BF16 || dtype == MHIP_F16;
     if (!is16 && dtype != MHIP_F32) return 0;
     const bool vec = is16 && (trans_a ? M : K) % 8 == 0 && (trans_b ? K : N) % 8 == 0;
-    if (!trans_a && M <= (is16 ? 64 : 192) && (is16 && !vec ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, batch, is16))) return gemm_skinny_workspace(M, N, K, batch, trans_b);
+    if (!trans_a && M <= (is16 ? 64 : 192) && (is16 && !vec ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, batch, trans_b, is16))) return gemm_skinny_workspace(M, N, K, batch, trans_b, is16);
     // (a large problem goes to the ring kernels, whose tiles fill the device)
     if (!is16) return gemm_f32_workspace(M, N, K, batch, trans_a, trans_b);
     if (!vec) return short_product(M, N, K) ? 0 : gemm_any_workspace(M, N, K, batch);

@@ -258,13 +258,16 @@ bool wide_strips(int64_t N, int64_t K, int64_t batch, bool tb) {
     return tb ? strips >= 128 && K >= 2048 : strips >= 128 || (strips >= 64 && K >= 2048);
 }
 
-// K split over the grid as well (fp32 sums in a workspace, one more launch) while that leaves every workgroup
-// 2048 k and at most one of them per compute unit: [4,4096] x [4096,4096] 13.0 -> 10.3 us,
-// [28,6384] x [6384,688] 17.4 -> 9.2.
-int skinny_splits(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b) {
+// K split over the grid as well (fp32 sums in a workspace, one more launch) while that leaves every workgroup 1024 k and
+// at most one of them per compute unit, from a K on where the shorter chain pays for the launch.  us, whole / split:
+// [4,4096] x [4096,4096] 13.0 / 9.5, [28,6384] x [6384,688] 17.4 / 8.4, [32,3072] x [3072,768] 10.4 / 8.8 but
+// [4,3072] x [3072,768] 6.4 / 6.7 and [16,2048] x [2048,2048] 6.2 / 7.3.  fp32 [40,3072] x [3072,768] 15.5 / 13.2; blocks of
+// more than 64 rows fill the device earlier ([128,3072] x [3072,768] 16.4 / 20.5) and keep 2048 k.
+int skinny_splits(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b, bool is16) {
     if (batch != 1 || M * N > (1 << 20)) return 1;
     const int64_t width = wide_strips(N, K, 1, trans_b != 0) ? (trans_b ? 32 : 64) : (trans_b ? 16 : 32);
-    const int64_t room = 256 / ((N + width - 1) / width), want = K / 2048 + (K % 2048 > 1024);
+    const bool fine = K >= 4096 || (K >= 3072 && (M >= 16 || !is16));
+    const int64_t room = 256 / ((N + width - 1) / width), want = M <= 64 && fine ? K / 1024 : K / 2048 + (K % 2048 > 1024);
     const int64_t n = room < want ? room : want;
     return n < 2 ? 1 : n > 8 ? 8 : (int)n;
 }
@@ -295,8 +298,12 @@ int launch_shape(hipStream_t s, const GemmArgs& g, int64_t batch) {
             if (wide) return k16 || TB ? launch_one<T, TB, VEC, TB ? 2 : 4, 2, 2>(s, g, batch) : launch_one<T, TB, VEC, 2, 2, 2>(s, g, batch);
             return launch_one<T, TB, VEC, TB ? 1 : k16 ? 2 : 1, 2, 2>(s, g, batch);
         }
-        if (wide) return k16 || TB ? launch_one<T, TB, VEC, TB ? 2 : 4, 4, 1>(s, g, batch) : launch_one<T, TB, VEC, 2, 4, 1>(s, g, batch);
-        return launch_one<T, TB, VEC, TB ? 1 : k16 ? 2 : 1, 4, 2>(s, g, batch);
+        // 33 to 64 rows of a small 16-bit weight matrix: two blocks of 32 rows (one of 64 takes 8.2 us where they take 6.7)
+        if constexpr (k16) return launch_one<T, TB, VEC, TB ? 1 : 2, 2, 2>(s, g, batch);
+        else {
+            if (wide) return launch_one<T, TB, VEC, 2, 4, 1>(s, g, batch);
+            return launch_one<T, TB, VEC, 1, 4, 2>(s, g, batch);
+        }
     }
 }
 
@@ -323,13 +330,13 @@ bool gemm_skinny_eligible(const GemmArgs& g, int trans_a, int elem_bytes) {
            ((int64_t)g.N + 64) * g.K * elem_bytes < 0x7FFFFFFFLL && ((int64_t)g.K + 64) * g.N * elem_bytes < 0x7FFFFFFFLL;
 }
 
-int64_t gemm_skinny_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b) {
-    const int n = skinny_splits(M, N, K, batch, trans_b);
+int64_t gemm_skinny_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b, bool is16) {
+    const int n = skinny_splits(M, N, K, batch, trans_b, is16);
     return n == 1 ? 0 : M * N * 4 * n;
 }
 
 int launch_gemm_skinny(hipStream_t s, GemmArgs g, int64_t batch, int trans_b, int dtype, int64_t workspace_bytes) {
-    g.splits = g.partial ? skinny_splits(g.M, g.N, g.K, batch, trans_b) : 1;
+    g.splits = g.partial ? skinny_splits(g.M, g.N, g.K, batch, trans_b, dtype != MHIP_F32) : 1;
     if ((int64_t)g.M * g.N * 4 * g.splits > workspace_bytes) g.splits = 1;
     if (g.splits == 1) g.partial = nullptr;
     const int st = dtype_launch(s, g, batch, trans_b, dtype);
