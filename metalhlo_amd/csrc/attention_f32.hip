@@ -193,8 +193,11 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaAr
     const __amdgpu_buffer_rsrc_t rk = fa_rsrc(static_cast<const float*>(a.k) + (int64_t)bh * a.Skv * D, bytes);
     const __amdgpu_buffer_rsrc_t rv = fa_rsrc(static_cast<const float*>(a.v) + (int64_t)bh * a.Skv * D, bytes);
     const float* mp = HAS_MASK ? static_cast<const float*>(a.mask) + (int64_t)(bh / a.H) * a.mask_sb +
-                                     (int64_t)(bh % a.H) * a.mask_sh + (int64_t)qpos * a.Skv
+                                     (int64_t)(bh % a.H) * a.mask_sh + (int64_t)min(qpos, a.Sq - 1) * a.Skv
                                : nullptr;
+    // (a lane's keys of a block are four runs of four, loaded whole; in the last block of a row that is no multiple of four a
+    // run may leave the mask: element by element)
+    const bool whole_runs = a.Skv % 4 == 0;
     f32x4 qf[NS];
 #pragma unroll
     for (int j = 0; j < NS; j++)
@@ -229,6 +232,12 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaAr
     if (wave < nkv) { load_k(wave); load_v(wave); }
     for (int blk = wave; blk < nkv; blk += 4) {
         const int kb = blk * kFBK;
+        f32x4 mrun[HAS_MASK ? 4 : 1];
+        const bool mask_runs = HAS_MASK && (whole_runs || kb + kFBK <= a.Skv);
+        if (mask_runs) {
+#pragma unroll
+            for (int g = 0; g < 4; g++) __builtin_memcpy(&mrun[HAS_MASK ? g : 0], mp + min(kb + 8 * g + 4 * h, a.Skv - 4), 16);
+        }
         f32x16 sacc;
 #pragma unroll
         for (int i = 0; i < 16; i++) sacc[i] = 0.f;
@@ -245,7 +254,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaAr
             const int key = kb + f32_key(i, h);
             float sv = sacc[i] * scale;
             const bool keep = !edge || (key < a.Skv && (!CAUSAL || key <= qpos));
-            if (HAS_MASK) { if (q_live && key < a.Skv) sv += mp[key]; }
+            if (HAS_MASK) sv += mask_runs ? mrun[HAS_MASK ? i >> 2 : 0][i & 3] : key < a.Skv ? mp[key] : 0.f;
             t[i] = keep ? sv * kLog2e : -INFINITY;
             m_blk = fmaxf(m_blk, t[i]);
         }
