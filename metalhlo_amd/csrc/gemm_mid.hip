@@ -60,7 +60,7 @@ struct StageLoader {
 
 // KG groups of four waves: a stage is KG x 64 k, group q multiplies its 64, the groups' sums meet in LDS at the
 // end.  S stages in the ring.
-template <typename T, int BM, int BN, int WGM, bool TA, bool TB, int KG, int S>
+template <typename T, int BM, int BN, int WGM, bool TA, bool TB, int KG, int S, bool AHEAD>
 __global__ __launch_bounds__(256 * KG) void gemm_mid_kernel(GemmArgs g) {
     constexpr int WGN = 4 / WGM, WTM = BM / WGM, WTN = BN / WGN, TM = WTM / 32, TN = WTN / 32;
     constexpr int kATile = BM * kRowBytes, kPart = (BM + BN) * kRowBytes, kStage = KG * kPart;
@@ -102,30 +102,41 @@ __global__ __launch_bounds__(256 * KG) void gemm_mid_kernel(GemmArgs g) {
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
 
+    auto stage_at = [&](int kt) { return smem + ((kt - kt0) % S) * kStage + group * kPart; };
+    auto read = [&](const char* at, int s, u32x4(&fa)[TM], u32x4(&fb)[TN]) {
+        const char* bt = at + kATile;
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+            fa[i] = TA ? frag_mn<BM>(at, wm * WTM + i * 32, s, lane) : frag_kmajor(at, wm * WTM + i * 32, s, lane);
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+            fb[j] = TB ? frag_kmajor(bt, wn * WTN + j * 32, s, lane) : frag_mn<BN>(bt, wn * WTN + j * 32, s, lane);
+    };
+    // AHEAD: the first operands of a stage are read while the one before it is multiplied; a lone wave per SIMD otherwise
+    // waits out an LDS latency behind every barrier.
+    static_assert(!AHEAD || S >= 4, "two stages have to have landed");
+    u32x4 af[2][TM], bf[2][TN];
 #pragma unroll
     for (int p = 0; p < S - 1; p++) load(kt0 + p);
+    if (AHEAD) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * kLoads) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        read(stage_at(kt0), 0, af[0], bf[0]);
+    }
     for (int kt = kt0; kt < kt1; kt++) {
-        // stage kt has landed when only the S - 2 stages behind it are in flight; past the barrier that
+        // stage kt (AHEAD: and kt + 1) has landed when only the stages behind it are in flight; past the barrier that
         // holds for every wave's share, and every wave has read stage kt - 1, whose place is reused
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * kLoads) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((AHEAD ? S - 3 : S - 2) * kLoads) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         load(kt + S - 1);
-        const char* at = smem + ((kt - kt0) % S) * kStage + group * kPart;
-        const char* bt = at + kATile;
-        u32x4 af[2][TM], bf[2][TN];
-        auto read = [&](int s, u32x4(&fa)[TM], u32x4(&fb)[TN]) {
-#pragma unroll
-            for (int i = 0; i < TM; i++)
-                fa[i] = TA ? frag_mn<BM>(at, wm * WTM + i * 32, s, lane) : frag_kmajor(at, wm * WTM + i * 32, s, lane);
-#pragma unroll
-            for (int j = 0; j < TN; j++)
-                fb[j] = TB ? frag_kmajor(bt, wn * WTN + j * 32, s, lane) : frag_mn<BN>(bt, wn * WTN + j * 32, s, lane);
-        };
-        read(0, af[0], bf[0]);
+        const char* at = stage_at(kt);
+        if (!AHEAD) read(at, 0, af[0], bf[0]);
 #pragma unroll
         for (int s = 0; s < kBK / 16; s++) {
-            if (s + 1 < kBK / 16) read(s + 1, af[(s + 1) & 1], bf[(s + 1) & 1]);
+            if (s + 1 < kBK / 16) read(at, s + 1, af[(s + 1) & 1], bf[(s + 1) & 1]);
+            else if (AHEAD) read(stage_at(kt + 1), 0, af[0], bf[0]);
 #pragma unroll
             for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -292,12 +303,12 @@ __global__ __launch_bounds__(256) void gemm_finish_kernel(GemmArgs g) {
     });
 }
 
-template <typename T, int BM, int BN, int WGM, bool TA, bool TB, int KG, int S>
+template <typename T, int BM, int BN, int WGM, bool TA, bool TB, int KG, int S, bool AHEAD = false>
 int launch_tile(hipStream_t s, GemmArgs g, int64_t batch) {
     constexpr int kStage = KG * (BM + BN) * kRowBytes, kRing = S * kStage, kSums = KG / 2 * BM * BN * 4, kOut = 4 * (BM / WGM) * ((BN / (4 / WGM)) * 2 + 16);
     constexpr int kUse = kRing > kOut ? kRing : kOut, kSmem = kUse > kSums ? kUse : kSums;
     static_assert(kSmem <= 160 * 1024, "ring larger than LDS");
-    auto kern = gemm_mid_kernel<T, BM, BN, WGM, TA, TB, KG, S>;
+    auto kern = gemm_mid_kernel<T, BM, BN, WGM, TA, TB, KG, S, AHEAD>;
     static std::once_flag once;
     static hipError_t err = hipSuccess;
     std::call_once(once, [&] { err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kSmem); });
@@ -317,7 +328,7 @@ int launch_tile(hipStream_t s, GemmArgs g, int64_t batch) {
 // shapes from [37,768] x K 768 to [2048,2048] x K 2048 and [512,512] x K 16384, each within about 15 %.
 struct Form { int bm, bn; float lone, ends; bool in_order; };
 constexpr Form kForms[] = {{64, 64, 0.40f, 0.7f, false}, {64, 128, 0.60f, 1.0f, false}, {128, 128, 0.92f, 1.4f, false},   // two groups of waves
-                           {64, 64, 0.53f, 0.7f, true}, {64, 128, 0.80f, 1.0f, true}, {128, 128, 1.20f, 1.4f, true},     // one group
+                           {64, 64, 0.53f, 0.7f, true}, {64, 128, 0.77f, 1.0f, true}, {128, 128, 1.20f, 1.4f, true},     // one group
                            {128, 192, 0.88f, 2.0f, true}};
 constexpr int kRing192 = 6, kMaxSplits = 8;
 
@@ -328,7 +339,10 @@ float form_cost(const Form& f, int64_t M, int64_t N, int64_t K, int64_t batch, i
     const int64_t rounds = (wgs + 255) / 256, at_once = wgs < 256 ? wgs : 256;
     const float bytes = (float)(f.bm + f.bn) * 256.f, l2 = (float)at_once * bytes / 15e6f;
     const float iters = (float)((K / splits + 127) / 128);
-    float t = 3.3f + (float)rounds * (iters * (f.lone > l2 ? f.lone : l2) + f.ends);
+    // (two workgroups of the one-group 64x64 form share a compute unit: up to two rounds of it take 1.25 to 1.45 times one,
+    // [1500,1024] x K 2048 15.8 us where 64x128 tiles take 16.7, [512,2304] x K 768 8.2 and 8.6)
+    const float turns = f.in_order && f.bn == 64 && rounds == 2 ? 1.4f : (float)rounds;
+    float t = 3.3f + turns * (iters * (f.lone > l2 ? f.lone : l2) + f.ends);
     // the sums go out and come back (5 TB/s), one more launch
     if (splits > 1) t += 3.f + (float)(M * N) * 8e-6f * (float)splits / 5.f;
     return t;
@@ -360,13 +374,18 @@ int64_t plan_bytes(const MidPlan& p, int64_t M, int64_t N) {
 
 template <typename T, bool TA, bool TB>
 int launch_form(hipStream_t s, const GemmArgs& g, int64_t batch, int form) {
+    // one workgroup per compute unit or fewer: all of LDS for a ring of four that reads ahead; otherwise the ring that two
+    // workgroups of a unit share ([2000,2000] x K 2000, 256 of 128x128, 29.7 -> 26.6 us; [1000,3000] x K 1000, 384 of 64x128,
+    // 16.4 against 20.2; tiles of 64x64 lose by it, [1000,1000] x K 1000 7.9 against 8.6)
+    const Form& f = kForms[form];
+    const bool one_each = ((g.M + f.bm - 1) / f.bm) * (int64_t)((g.N + f.bn - 1) / f.bn) * batch * g.splits <= 256;
     switch (form) {
         case 0: return launch_tile<T, 64, 64, 2, TA, TB, 2, 3>(s, g, batch);
         case 1: return launch_tile<T, 64, 128, 2, TA, TB, 2, 3>(s, g, batch);
         case 2: return launch_tile<T, 128, 128, 2, TA, TB, 2, 2>(s, g, batch);
         case 3: return launch_tile<T, 64, 64, 2, TA, TB, 1, 4>(s, g, batch);
-        case 4: return launch_tile<T, 64, 128, 2, TA, TB, 1, 3>(s, g, batch);
-        default: return launch_tile<T, 128, 128, 2, TA, TB, 1, 2>(s, g, batch);
+        case 4: return one_each ? launch_tile<T, 64, 128, 2, TA, TB, 1, 4, true>(s, g, batch) : launch_tile<T, 64, 128, 2, TA, TB, 1, 3>(s, g, batch);
+        default: return one_each ? launch_tile<T, 128, 128, 2, TA, TB, 1, 4, true>(s, g, batch) : launch_tile<T, 128, 128, 2, TA, TB, 1, 2>(s, g, batch);
     }
 }
 
