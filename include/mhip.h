@@ -364,11 +364,11 @@ int mhip_fill(void* stream, void* y, int64_t n, uint64_t pattern, int elem_size)
  * point consults before its heuristic, and reports it.  Passes overwrite their output tensor
  * and synchronise with the stream. */
 
-/* GEMM kernel variants (128x128 tiles / 4 waves, 256x256 / 8 waves, the four-wave LDS-ring kernel
+/* GEMM kernel variants (tiles of up to 128 rows and the few-row kernel, 256x256 / 8 waves, the four-wave LDS-ring kernel
  * on 256x256 and on 256x128 tiles, the latter also as persistent workgroups, and wide tiles plus a
- * band of narrow ones): variant code 64 | 128 | 256 | 2560 | 2561 | 2562 | 2563, and the other members of the
+ * band of narrow ones): variant code 128 | 256 | 2560 | 2561 | 2562 | 2563, and the other members of the
  * generated ring-kernel family (tile width 384 / 256 / 128 x ring depth 4 / 5 / 6, those that fit 160 KB of
- * LDS and the register file): 64 = the kernels for few rows and few tiles, 2564 = 256x128 with six stages, 2565 = 256x128 with four, 2566 = 256x256
+ * LDS and the register file): 2564 = 256x128 with six stages, 2565 = 256x128 with four, 2566 = 256x256
  * with four, 2567 = 256x384 with four (a third of its accumulators in ordinary registers; no
  * activation, relu or tanh-GELU), 2568 = 256x128 with three, in 256 registers a wave, two workgroups
  * per compute unit, 2569 = 128x192 with six (for problems with so few columns that 256-row tiles

@@ -365,7 +365,7 @@ static int launch_column_split(hipStream_t s, const GemmArgs& g, int64_t batch, 
     return launch_gemm256(s, w, 1, TA, TB, dt);
 }
 
-// Which kernel serves a 16-bit problem (MHIP_GEMM_TILE = 64 | 128 | 256 | 2560 ... 2570 forces one; 2570 = the 256x288 tile; 2564 / 2565 = the
+// Which kernel serves a 16-bit problem (MHIP_GEMM_TILE = 128 | 256 | 2560 ... 2570 forces one; 2570 = the 256x288 tile; 2564 / 2565 = the
 // 256x128 tile with a ring of six / four stages, 2566 = the 256x256 tile with four, 2568 = the 256x128
 // tile as two workgroups per compute unit: members of the generated family that only a forced choice
 // or the tuning table selects; 2567 = the 256x384 tile):
@@ -387,8 +387,7 @@ static int launch_column_split(hipStream_t s, const GemmArgs& g, int64_t batch, 
 //   * 128x192 tiles (2569) where 256-row tiles would leave compute units idle (few columns);
 //   * the eight-wave 256x256 kernel for large problems the ring kernel cannot take whose
 //     rows of C are not 16-byte aligned (odd N): its eight waves hide the narrow stores;
-//   * otherwise (short K, few tiles, few rows) the ring-staged 64- and 128-row tiles of gemm_mid.hip (64); the
-//     register-staged 128x128 tile (128) runs where it is forced or recorded.
+//   * otherwise (short K, few tiles, few rows) the tiles of up to 128 rows of gemm_mid.hip, or the few-row kernel (128).
 // An entry of the tuning table (mhip_gemm_autotune) for the problem overrides the heuristic.
 // The kernel the last mhip_gemm / mhip_gemm_residual call of this thread chose (mhip_gemm_last_variant).
 static thread_local int g_last_variant = 0;
@@ -435,7 +434,7 @@ static int pick_tile(hipStream_t s, const GemmArgs& g, int64_t batch, int64_t wo
         if (gemm256_eligible(g, batch, TA, TB, dt, 384) && gemm384_activation_ok(g.act)) return chose(2567, launch_gemm256(s, g, batch, TA, TB, dt, 384, 4));
     }
     // (up to 192 rows: half of a 256-row tile would be padding)
-    if (force == 64 || (force == 0 && g.M <= 192)) return chose(64, launch_gemm_mid(s, g, batch, TA, TB, dt, workspace_bytes));
+    if (force == 128 || (force == 0 && g.M <= 192)) return chose(128, launch_gemm_mid(s, g, batch, TA, TB, dt, workspace_bytes));
     constexpr int cus = 256;                           // compute units of the device this is written for
     const int64_t narrow = tiles_m * ((g.N + 127) / 128) * batch, stages = g.K / 32;
     const int64_t wide_cost = ((big + cus - 1) / cus) * (stages * 32 + 700);
@@ -490,10 +489,8 @@ static int pick_tile(hipStream_t s, const GemmArgs& g, int64_t batch, int64_t wo
     }
     // (fewer than 192 tiles of any ring kernel, a ragged K, or so few rows that 256-row tiles are mostly padding)
     const bool large = big >= 192 && (g.K >= 1024 || g.N % 8 != 0);
-    if (force == 0 && !large) return chose(64, launch_gemm_mid(s, g, batch, TA, TB, dt, workspace_bytes));
-    const bool want256 = force == 256 || (force != 128 && big >= 192 && (g.K >= 1024 || g.N % 8 != 0));
-    if (want256) return chose(256, launch_mfma<T, 256, 256, 2, 4, TA, TB>(s, g, batch));
-    return chose(128, launch_mfma<T, 128, 128, 2, 2, TA, TB>(s, g, batch));
+    if (!large && force != 256) return chose(128, launch_gemm_mid(s, g, batch, TA, TB, dt, workspace_bytes));
+    return chose(256, launch_mfma<T, 256, 256, 2, 4, TA, TB>(s, g, batch));
 }
 
 template <typename T>
@@ -548,7 +545,7 @@ static bool skinny_unaligned(int64_t M, int64_t N, int64_t K) { return M <= 16 &
 // [77,333] 4.7 against 5.3; behind from there on: [128,130] x [130,129] 6.2 against 5.8, [1000,67] x [67,1001] 14.9 against 5.7.
 static bool short_product(int64_t M, int64_t N, int64_t K) { return K < 96 && M * N <= (1 << 17); }
 
-static bool few_row_choice(int tuned) { return tuned == 0 || tuned == 64; }
+static bool few_row_choice(int tuned) { return tuned == 0 || tuned == 128; }
 
 static int gemm_entry(void* stream, const void* a, const void* b, const void* bias, const void* residual, void* c,
                       int64_t M, int64_t N, int64_t K, int64_t batch, int64_t stride_a,
@@ -587,7 +584,7 @@ static int gemm_entry(void* stream, const void* a, const void* b, const void* bi
     if ((is16 || dtype == MHIP_F32) && gemm_skinny_eligible(g, trans_a, is16 ? 2 : 4) && (is16 && !vec_ok ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, batch, trans_b, is16)) &&
         tune_int("MHIP_GEMM_TILE", 0) == 0 && tune_int("MHIP_GEMM_F32_MFMA", 1) == 1 &&
         (!is16 || few_row_choice(tuned_gemm_variant(g, batch, trans_a, trans_b, dtype)) || !vec_ok))
-        return chose(vec_ok ? 64 : 0, launch_gemm_skinny(s, g, batch, trans_b, dtype, workspace_bytes));
+        return chose(vec_ok ? 128 : 0, launch_gemm_skinny(s, g, batch, trans_b, dtype, workspace_bytes));
     if (vec_ok) {
         if (dtype == MHIP_BF16) return pick_layout<bf16_t>(s, g, batch, trans_a, trans_b, workspace_bytes);
         return pick_layout<f16_t>(s, g, batch, trans_a, trans_b, workspace_bytes);

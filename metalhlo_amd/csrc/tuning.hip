@@ -87,7 +87,7 @@ std::string attention_key(int dt, int64_t bh, int64_t Sq, int64_t Skv, int64_t D
                (long long)D, causal ? 1 : 0);
 }
 
-bool gemm_variant_exists(int v) { return v == 64 || v == 128 || v == 256 || (v >= 2560 && v <= 2570); }
+bool gemm_variant_exists(int v) { return v == 128 || v == 256 || (v >= 2560 && v <= 2570); }
 
 bool valid_choice(const char* line, const std::string& choice) {
     int a = 0, b = 0, c = 0, d = 0;
@@ -280,14 +280,10 @@ using namespace mhip;
 // GEMM candidates a problem can run (the validity filter: shape, alignment, LDS and tile count rules of each kernel).
 static std::vector<int> gemm_candidates(const GemmArgs& g, int64_t batch, int trans_a, int trans_b, int dtype) {
     std::vector<int> out;
-    // (64: the kernels for few rows and few tiles, where they are the default)
-    const bool tiles_fill = g.M > 192 && (gemm256_eligible(g, batch, trans_a, trans_b, dtype) || gemm256_eligible(g, batch, trans_a, trans_b, dtype, 128) ||
-                                          gemm256_eligible(g, batch, trans_a, trans_b, dtype, 192));
-    for (int v : {64, 128, 256, 2560, 2561, 2562, 2563, 2564, 2565, 2566, 2567, 2568, 2569, 2570}) {
+    for (int v : {128, 256, 2560, 2561, 2562, 2563, 2564, 2565, 2566, 2567, 2568, 2569, 2570}) {
         if ((v == 2560 || v == 2566) && !gemm256_eligible(g, batch, trans_a, trans_b, dtype)) continue;
         if ((v == 2561 || v == 2564 || v == 2565 || v == 2568) && !gemm256_eligible(g, batch, trans_a, trans_b, dtype, 128)) continue;
         if (v == 2570 && !(gemm256_eligible(g, batch, trans_a, trans_b, dtype, 288) && gemm384_activation_ok(g.act))) continue;
-        if (v == 64 && tiles_fill) continue;
         if (v == 2569 && !gemm256_eligible(g, batch, trans_a, trans_b, dtype, 192)) continue;
         if (v == 2567 && !(gemm256_eligible(g, batch, trans_a, trans_b, dtype, 384) && gemm384_activation_ok(g.act))) continue;
         if (v == 2562 && !gemm_stream_eligible(g, batch, trans_a, trans_b, dtype)) continue;
