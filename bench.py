@@ -40,11 +40,12 @@ PEAK_CLOCK_MHZ = 2400.0     # the shader clock the matrix peak is quoted at
 
 # HBM bytes per launch from rocprofv3 FETCH_SIZE + WRITE_SIZE, each scaled by what the same
 # counter reads for the 'copy' workload (256 MiB in, 256 MiB out); see profiles/<workload>.txt.
-# TRAFFIC_COMMIT: the commit of this repository the counter runs were taken at (the profiles say so too).
-TRAFFIC_COMMIT = "78f698b"
+# TRAFFIC_COMMIT: the commits of this repository the counter runs were taken at (the profiles say so too).
+TRAFFIC_COMMIT = dict.fromkeys(("gemm", "attention", "attention_full", "attention_f32", "softmax", "layer_norm", "rms_norm", "bias_gelu", "copy"), "78f698b")
+TRAFFIC_COMMIT["gemm_f32"] = "0b36930"
 MEASURED_TRAFFIC = {
     "gemm": 237458425,
-    "gemm_f32": 812880561,
+    "gemm_f32": 867650167,
     "attention": 753138116,
     "attention_full": 268936609,
     "attention_f32": 1879189489,
@@ -197,7 +198,7 @@ def wl_gemm_f32(torch, kernels, M=4096, N=4096, K=4096):
     c = torch.empty(M, N, dtype=torch.float32, device="cuda")
     return dict(name=f"fp32 GEMM {M}x{N}x{K} (row-major A[M,K], B[K,N]; fp32 operands and accumulate on the fp32 matrix instruction)",
                 fn=lambda i: kernels.matmul(a, b, out=c), flops=2.0 * M * N * K, bytes=4.0 * (M * K + K * N + M * N),
-                bound="mfma", peak=PEAK_F32_TFLOPS, kernel="gemm_f32_mfma_kernel")
+                bound="mfma", peak=PEAK_F32_TFLOPS, kernel="gemm_f32_ring_kernel")
 
 
 def wl_attention(torch, kernels, B=4, H=32, S=4096, D=128, causal=True, fp32=False):
@@ -350,7 +351,7 @@ def measure(wl, steps, warmup, torch, key=None):
         roof = dict(bound="hbm", achieved=round(ach, 1), peak=PEAK_HBM_GBS, unit="GB/s",
                     frac=round(ach / PEAK_HBM_GBS, 4), traffic=MEASURED_TRAFFIC.get(key))
         value, unit = ach, "GB/s"
-    roof["traffic_commit"] = TRAFFIC_COMMIT if MEASURED_TRAFFIC.get(key) else None
+    roof["traffic_commit"] = TRAFFIC_COMMIT.get(key) if MEASURED_TRAFFIC.get(key) else None
     r = dict(workload=wl["name"], kernel=wl["kernel"], value=round(value, 2), unit=unit,
              us_per_launch=round(sec * 1e6, 2), wall_us_per_launch=round(wall * 1e6, 2), roofline=roof)
     if not wl.get("host_timed"):
