@@ -279,16 +279,18 @@ __global__ __launch_bounds__(256) void gemm_finish_kernel(GemmArgs g) {
     const T* bias = static_cast<const T*>(g.bias);
     const T* res = static_cast<const T*>(g.residual);
     T* c = static_cast<T*>(g.c);
-    const int col = (int)(i0 % g.N);
+    int next = (int)(i0 % g.N);           // (four elements cover up to four rows: N may be 1)
     dispatch_act(g.act, [&](auto act_tag) {
         constexpr int ACT = decltype(act_tag)::value;
         T o[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
+            const int col = next;
+            next = col + 1 == g.N ? 0 : col + 1;
             o[e] = Elem<T>::from_f32(0.f);
             if (e >= n_here) continue;
             float x = v[e];
-            if (bias) x += Elem<T>::to_f32(bias[col + e < g.N ? col + e : col + e - g.N]);
+            if (bias) x += Elem<T>::to_f32(bias[col]);
             x = sizeof(T) == 4 ? apply_act(x, ACT) : apply_act_c<ACT>(x);
             o[e] = Elem<T>::from_f32(x);
             // (second rounding on purpose: the same result as a separate add over the stored C)

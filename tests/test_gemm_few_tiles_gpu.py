@@ -73,3 +73,21 @@ def test_splitting_needs_its_workspace(lib):
     e = a.double().t().cpu() @ b.double().cpu()
     for out in c:        # K 2^-24 sum |a||b| is below 2^-8 sqrt(K) here; one rounding to bf16
         assert ((out.double().cpu() - e).abs() <= 2.0 ** -8 * (e.abs() + K ** 0.5)).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=lambda d: NAME[d])
+@pytest.mark.parametrize("M,N,K", [(16, 1, 4096), (13, 1, 4100), (33, 1, 4099), (16, 2, 4096), (16, 3, 4096), (40, 3, 4099), (7, 5, 4096)], ids=lambda v: str(v))
+def test_split_sums_of_few_columns(M, N, K, dtype):
+    """A split K whose result has fewer columns than the four elements a thread of gemm_finish_kernel makes: the bias
+    of each element is that of its own column.  What lies behind the bias in memory is NaN."""
+    from metalhlo_amd import _lib, kernels
+    code = {torch.bfloat16: 3, torch.float32: 1}[dtype]
+    assert _lib.load().mhip_gemm_workspace(M, N, K, 1, 0, 1, code) > 0           # (the problem is split)
+    rng = np.random.default_rng(M)
+    a, b = to_dev(rng.standard_normal((M, K)), dtype), to_dev(rng.standard_normal((N, K)), dtype)
+    bias = to_dev(np.concatenate([rng.standard_normal(N) * 100, np.full(16, np.nan)]), dtype)[:N]
+    got = as_f64(kernels.matmul(a, b, bias=bias, trans_b=True))
+    A, B, c = as_f64(a), as_f64(b).T, as_f64(bias)
+    e = A @ B + c
+    fp32 = (K + 2) * 2.0 ** -24 * (np.abs(A) @ np.abs(B) + np.abs(c))
+    assert np.all(np.abs(got - e) <= fp32 + ROUNDOFF[dtype] * (np.abs(e) + fp32))
