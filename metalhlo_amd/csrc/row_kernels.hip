@@ -8,6 +8,8 @@
 // of 16, take a workgroup-per-row multi-pass path.
 #include <math.h>
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace mhip {
@@ -214,6 +216,16 @@ template <> struct VecSum<f16_t> {
     }
 };
 
+// Softmax of 16-bit rows forms exp(x - m) as exp2(x u - m u), one fused multiply-add in front of the exp2, with u =
+// log2(e).  What rounding m u leaves is a factor common to the row while it is small (2^-8 in the exponent below
+// |m| = 2^16) and takes the row out of fp32 when it is not.  From 2^16 on (bf16 only) u is 1 and m u exact: numbers
+// lie 256 or more apart there, so the row's maxima give 1 and everything below them 0, as it should be.
+template <typename T>
+__device__ inline float softmax_unit(float m) {
+    constexpr float kLog2e = 1.4426950408889634f;
+    return std::is_same<T, bf16_t>::value && !(fabsf(m) < 65536.f) ? 1.f : kLog2e;
+}
+
 // A row shared by WPR waves of the workgroup (WPR = 2 or 4), R rows per wave group at a time
 // (4 / WPR * R rows per workgroup): each lane holds only NV vectors of each row and of the
 // parameters, so the kernel needs few registers and the CU holds its full complement of waves,
@@ -318,18 +330,17 @@ void row_split_kernel(const T* __restrict__ x, const T* __restrict__ gamma, cons
                 }
             }
             group_reduce(m, true, 0);
-            constexpr float kLog2e = 1.4426950408889634f;
             float s[R];
 #pragma unroll
             for (int r = 0; r < R; r++) {
-                const float ms = m[r] * kLog2e;
+                const float unit = softmax_unit<T>(m[r]), ms = m[r] * unit;
                 s[r] = 0.f;
 #pragma unroll
                 for (int v = 0; v < NV; v++) {
                     float sv = 0.f;
 #pragma unroll
                     for (int e = 0; e < E; e++) {
-                        f[r][v][e] = k16 ? __builtin_amdgcn_exp2f(fmaf(f[r][v][e], kLog2e, -ms)) : expf(f[r][v][e] - m[r]);
+                        f[r][v][e] = k16 ? __builtin_amdgcn_exp2f(fmaf(f[r][v][e], unit, -ms)) : expf(f[r][v][e] - m[r]);
                         sv += f[r][v][e];
                     }
                     s[r] += (live[r] && in[v]) ? sv : 0.f;
@@ -457,7 +468,6 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT) void row_any_kernel(const T* _
                                                                       const T* __restrict__ beta, T* __restrict__ y, int64_t rows,
                                                                       int cols, float eps) {
     constexpr int E = Elem<T>::kPerVec;
-    constexpr float kLog2e = 1.4426950408889634f;
     constexpr bool k16 = sizeof(T) == 2;
     __shared__ float red[2][NT / 64];
     const int64_t row = NT < 256 ? (int64_t)blockIdx.x * (256 / NT) + threadIdx.x / NT : (int64_t)blockIdx.x;
@@ -476,7 +486,7 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT) void row_any_kernel(const T* _
     }
     float ev = ei >= 0 ? Elem<T>::to_f32(xr[ei]) : 0.f;
     const float inv_cols = 1.f / (float)cols;
-    float scale, shift = 0.f;                      // y = f(x) * scale (+ shift)
+    float scale, shift = 0.f, unit = 1.f;          // y = f(x) * scale (+ shift)
     if (OP == kSoftmax) {
         float m = ei >= 0 ? ev : -INFINITY;
 #pragma unroll
@@ -486,15 +496,16 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT) void row_any_kernel(const T* _
                 for (int e = 0; e < E; e++) m = fmaxf(m, Elem<T>::to_f32(raw[v].v[e]));
             }
         m = row_reduce<NT, true>(m, red[0]);
-        shift = k16 ? m * kLog2e : m;
-        float s = ei >= 0 ? (k16 ? __builtin_amdgcn_exp2f(fmaf(ev, kLog2e, -shift)) : expf(ev - m)) : 0.f;
+        unit = softmax_unit<T>(m);
+        shift = k16 ? m * unit : m;
+        float s = ei >= 0 ? (k16 ? __builtin_amdgcn_exp2f(fmaf(ev, unit, -shift)) : expf(ev - m)) : 0.f;
 #pragma unroll
         for (int v = 0; v < NV; v++)
             if (v * NT + t < ph.nvec) {
 #pragma unroll
                 for (int e = 0; e < E; e++) {
                     const float f = Elem<T>::to_f32(raw[v].v[e]);
-                    const float p = k16 ? __builtin_amdgcn_exp2f(fmaf(f, kLog2e, -shift)) : expf(f - m);
+                    const float p = k16 ? __builtin_amdgcn_exp2f(fmaf(f, unit, -shift)) : expf(f - m);
                     if (!k16) raw[v].v[e] = Elem<T>::from_f32(p);       // (kept: exact in fp32)
                     s += p;
                 }
@@ -524,7 +535,7 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT) void row_any_kernel(const T* _
         scale = 1.f / sqrtf(row_reduce<NT, false>(q, red[0]) * inv_cols + eps);
     }
     auto value = [&](float f, float g, float b) {
-        if (OP == kSoftmax) return (k16 ? __builtin_amdgcn_exp2f(fmaf(f, kLog2e, -shift)) : f) * scale;
+        if (OP == kSoftmax) return (k16 ? __builtin_amdgcn_exp2f(fmaf(f, unit, -shift)) : f) * scale;
         return fmaf((f - shift) * scale, g, b);
     };
 #pragma unroll

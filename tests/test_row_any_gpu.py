@@ -45,3 +45,38 @@ def test_argmax_of_any_length(cols, dtype):
         e = np.array([np.flatnonzero(np.isnan(r))[0] if np.isnan(r).any() else int(np.argmax(r)) for r in x])
         assert np.array_equal(idx.cpu().numpy(), e)
         assert np.array_equal(as_f64(val), as_f64(t)[np.arange(6), e], equal_nan=True)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: NAME[d])
+@pytest.mark.parametrize("cols", [3, 64, 513, 768, 1025, 3072, 4096, 8200, 16391, 50257, 140001])
+def test_softmax_at_the_ends_of_the_type(cols, dtype):
+    """Rows of large numbers up to the ends of the type, where a maximum times log2(e) is rounded by more than a weight
+    can stand and in the end leaves fp32: equal elements share the row, an element one representable step below has
+    the weight of its distance.  One column count per row kernel and number of threads.  An exponent of x is off by
+    2^-24 |x| (|x| below 150 where the weight is not zero), the sum of n weights by n 2^-24; one rounding follows."""
+    from metalhlo_amd import kernels
+    low, high = float(torch.finfo(dtype).min), float(torch.finfo(dtype).max)
+    ulp = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    rows = []
+    for m in [low, low * 0.75, low * 0.5, high * 0.5, high * 0.75, high] + [s * 2.0 ** e for e in (13, 14, 15, 16, 17, 24, 31, 40, 100, 126, 127) for s in (-1.0, 1.25) if 2.0 ** e * 1.25 < high]:
+        r = np.full(cols, m)
+        rows.append(r.copy())                                   # equal elements: 1 / n
+        r[1::3] = max(low, m - 2 * ulp * abs(m))
+        rows.append(r.copy())
+        r[0::3] = low
+        rows.append(r.copy())
+        r[cols // 2] = -np.inf
+        rows.append(r)
+    r = np.full(cols, -np.inf)
+    r[cols - 1] = low                                           # one element of weight 1
+    rows.append(r)
+    x = to_dev(np.stack(rows), dtype)
+    x64 = as_f64(x)
+    e = np.exp(x64 - x64.max(-1, keepdims=True))
+    e /= e.sum(-1, keepdims=True)
+    tiny = 2.0 ** -24 if dtype == torch.float16 else 2.0 ** -126    # the smallest normal fp32 number, f16's even spacing
+    for start in (0, 1):                                        # elements in front of the tensor
+        t = torch.cat([x.new_zeros(start), x.reshape(-1)])[start:].view(x.shape)
+        got = as_f64(kernels.softmax(t))
+        bad = ~(np.abs(got - e) <= ((cols + 300) * 2.0 ** -24 + ulp) * e + tiny)
+        assert not bad.any(), (start, x64[bad][:4], got[bad][:4], e[bad][:4])
