@@ -203,7 +203,9 @@ FUNCTION(matmul) {
         if (bd == 2) {
             if (ta && ad != 2) raise(PyExc_ValueError, "trans_a needs a 2-D lhs when rhs is 2-D");
             const int64_t last = a.size(-1);
-            rows = ad == 2 ? a.size(0) : (last ? a.numel() / last : 0);
+            // (as `a.reshape(-1, 0)` says: no number of rows follows from the element count)
+            if (ad != 2 && last == 0) raise(PyExc_RuntimeError, "matmul cannot fold the leading dims of an lhs whose last axis is empty");
+            rows = ad == 2 ? a.size(0) : a.numel() / last;
             M = ta ? last : rows;
             K = ta ? rows : last;
             if (ta) shape.push_back(last);

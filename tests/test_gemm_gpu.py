@@ -640,3 +640,18 @@ def test_gemm_ring_kernel_takes_wide_and_deep_operands(lib):
     # fp32 operands run none of the 16-bit variants
     kernels.matmul(torch.ones(64, 64, device="cuda"), torch.ones(64, 64, device="cuda"))
     assert lib.mhip_gemm_last_variant() == 0
+
+
+@pytest.mark.parametrize("shape", [(2, 3, 0), (0, 3, 0), (0,), (2, 2, 2, 0)], ids=lambda v: str(v))
+def test_gemm_empty_contraction_of_folded_rows(shape):
+    """Leading dims that fold into M cannot be folded when the last axis is empty (the element count says nothing about
+    them): refused, with and without a result to fill; leading dims that are empty themselves give an empty result."""
+    from metalhlo_amd import kernels
+    a, b = torch.empty(shape, dtype=torch.bfloat16, device="cuda"), torch.empty(0, 7, dtype=torch.bfloat16, device="cuda")
+    with pytest.raises(RuntimeError):
+        kernels.matmul(a, b)
+    out = torch.full(shape[:-1] + (7,), 5.0, dtype=torch.bfloat16, device="cuda")
+    with pytest.raises(RuntimeError):
+        kernels.matmul(a, b, out=out)
+    assert (out == 5).all()
+    assert kernels.matmul(torch.empty(0, 3, 8, dtype=torch.bfloat16, device="cuda"), torch.empty(8, 7, dtype=torch.bfloat16, device="cuda")).shape == (0, 3, 7)
