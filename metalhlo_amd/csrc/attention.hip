@@ -21,6 +21,8 @@
 // bits the same to five digits.
 //
 // Everything else (unaligned tensors, larger heads) takes a wave-per-query scalar path.
+#include <type_traits>
+
 #include "attention_common.h"
 
 namespace mhip {
@@ -137,6 +139,10 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(FaArgs a) {
     // of four a run may leave the mask; that block loads element by element.
     const T* mp = HAS_MASK ? static_cast<const T*>(a.mask) + (int64_t)b_i * a.mask_sb + (int64_t)h_i * a.mask_sh + (int64_t)min(qpos, a.Sq - 1) * a.Skv : nullptr;
     const bool whole_runs = a.Skv % 4 == 0;
+    // log2(e) times a mask near bf16's lowest number is -inf.  A row with no other key than such ones so far (m_run is
+    // -inf) shares itself between those of the largest mask, here its value; the first ordinary key drops them.
+    constexpr bool kDeep = HAS_MASK && std::is_same<T, bf16_t>::value;
+    float deep = -INFINITY;
 
     for (int it = 0; it < nkv; it++) {
         const int cur = it % NB, kv0 = it * kBKV;
@@ -226,8 +232,27 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(FaArgs a) {
                 for (int i = 0; i < 32; i++) sv[i] = __builtin_amdgcn_exp2f(fmaf(sv[i], a.c, neg_m));
             }
             const float m_use2 = (m_new == -INFINITY) ? 0.f : m_new;
-            const float alpha = __builtin_amdgcn_exp2f(m_run - m_use2);
+            float alpha = __builtin_amdgcn_exp2f(m_run - m_use2);
             m_run = m_new;
+            if (kDeep && __any(m_new == -INFINITY)) {
+                // (read again, element by element: rare, and the loop above keeps its registers; a NaN score stays one)
+                auto mask_at = [&](int i) {
+                    const int key = kv0 + 32 * (i >> 4) + 8 * ((i & 15) >> 2) + 4 * lhalf + (i & 3);
+                    const float m = key >= a.Skv || (CAUSAL && key > qpos) ? -INFINITY : Elem<T>::to_f32(mp[key]);
+                    return m * kLog2e == -INFINITY ? m : -INFINITY;
+                };
+                float most = deep;
+#pragma unroll
+                for (int i = 0; i < 32; i++) most = fmaxf(most, mask_at(i));
+                most = half_max(most);
+                if (m_new == -INFINITY) {
+                    alpha = most == deep ? 1.f : 0.f;
+                    deep = most;
+#pragma unroll
+                    for (int i = 0; i < 32; i++)
+                        if (most != -INFINITY && mask_at(i) == most) sv[i] += 1.f;      // (exp2(-inf) so far)
+                }
+            }
             float lsum = 0.f;
 #pragma unroll
             for (int i = 0; i < 32; i++) lsum += sv[i];
@@ -442,6 +467,7 @@ static int fa_entry(const char* name, void* stream, const void* q, const void* k
     a.D = (int)D;
     a.B = (int)B; a.H = (int)H; a.Sq = (int)Sq; a.Skv = (int)Skv;
     a.c = fabsf(scale) * kLog2e;
+    a.scale = fabsf(scale);
     a.negate_q = scale < 0.f;
     a.is_causal = is_causal ? 1 : 0;
     a.mask_sb = mask_stride_b; a.mask_sh = mask_stride_h;

@@ -19,6 +19,7 @@ struct FaArgs {
     void* o;
     int B, H, Sq, Skv;
     float c;          // |scale| * log2(e)
+    float scale;      // |scale| (read by the decode kernel)
     int negate_q;     // scale < 0: flip the sign of Q instead
     int is_causal;    // read by the scalar path (the MFMA path is templated on it)
     int64_t mask_sb, mask_sh;
@@ -106,8 +107,18 @@ __device__ inline __amdgpu_buffer_rsrc_t fa_rsrc(const void* p, uint32_t bytes) 
 // function.  What it saves is the rescaling of the output accumulators, which a strict running
 // maximum triggers in nearly every block when 32 rows share a wave.  (-inf + 8 = -inf: the first
 // finite block maximum always moves it; a block of masked scores never does.)
+//
+// NAT: scores and reference as they are, the change to base 2 behind the subtraction.  The decode kernel
+// (bf16) and the fp32 kernels do so where there is a mask: log2(e) times a mask of the type's lowest number is -inf, and
+// a row that hides every key that way would hold no key instead of all of them alike.  (The reference lags by 5.5 < 8 ln 2.)
+template <bool NAT = false>
 __device__ __forceinline__ float moved_reference(float ref, float block_max) {
-    return block_max > ref + 8.f ? block_max : ref;
+    return block_max > ref + (NAT ? 5.5f : 8.f) ? block_max : ref;
+}
+// exp(s - ref) where both are in the kernel's domain
+template <bool NAT = false>
+__device__ __forceinline__ float weight(float s, float ref) {
+    return __builtin_amdgcn_exp2f(NAT ? (s - ref) * kLog2e : s - ref);
 }
 
 // K and V tiles sit in LDS as they lie in memory, [64 keys][D], 16-byte chunks

@@ -11,6 +11,8 @@
 //   O^T += V^T P^T  operand row = d: lane i loads VE = D / 16 neighbouring d of each of its eight keys, and one
 //                   byte permute per register pairs two keys of one d; tile f then holds d = VE i + f.  The
 //                   eight keys of a lane are the ones whose probabilities it just computed.
+#include <type_traits>
+
 #include "attention_common.h"
 
 namespace mhip {
@@ -32,8 +34,13 @@ constexpr int kKeys = 32;        // keys per block
 constexpr int kMaxSq = 16;
 constexpr int kPartKeys = 256;   // a part of a split key range is a multiple of this
 
+// domain of scores and reference (see moved_reference): f16's lowest number is far from fp32's
+template <typename T, bool HAS_MASK>
+constexpr bool kNatural = HAS_MASK && std::is_same<T, bf16_t>::value;
+
 template <typename T, int D, bool HAS_MASK, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* part, int per_part) {
+    constexpr bool NAT = kNatural<T, HAS_MASK>;
     constexpr int NS = D / 32, NF = D / 16, VDw = NF / 2;      // k steps of Q K^T, tiles of O^T, dwords of a lane's V piece
     __shared__ __attribute__((aligned(16))) float sums[WAVES][NF][64][4];
     __shared__ float ml[2][WAVES][kMaxSq];
@@ -96,13 +103,13 @@ __global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* 
 #pragma unroll
             for (int s = 0; s < NS; s++) s4 = Mfma16A<T>::run(blk.k[j][s], qf[s], s4);
 #pragma unroll
-            for (int r = 0; r < 4; r++) sv[4 * j + r] = s4[r] * a.c;
+            for (int r = 0; r < 4; r++) sv[4 * j + r] = s4[r] * (NAT ? a.scale : a.c);
         }
         if (HAS_MASK) {
 #pragma unroll
             for (int t = 0; t < 8; t++) {
                 const int kk = key + 16 * (t >> 2) + 4 * lg + (t & 3);
-                if (li < a.Sq && kk < a.Skv) sv[t] += Elem<T>::to_f32(mp[(int64_t)li * a.Skv + kk]) * kLog2e;
+                if (li < a.Sq && kk < a.Skv) sv[t] += Elem<T>::to_f32(mp[(int64_t)li * a.Skv + kk]) * (NAT ? 1.f : kLog2e);
             }
         }
         if (key + kKeys > k1) {
@@ -115,13 +122,13 @@ __global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* 
         for (int t = 1; t < 8; t++) mloc = fmaxf(mloc, sv[t]);
         mloc = fmaxf(mloc, __shfl_xor(mloc, 16, 64));
         mloc = half_max(mloc);
-        const float m_new = moved_reference(m_run, mloc), m_use = m_new == -INFINITY ? 0.f : m_new;
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+        const float m_new = moved_reference<NAT>(m_run, mloc), m_use = m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = weight<NAT>(m_run, m_use);
         m_run = m_new;
         float lsum = 0.f;
 #pragma unroll
         for (int t = 0; t < 8; t++) {
-            sv[t] = __builtin_amdgcn_exp2f(sv[t] - m_use);
+            sv[t] = weight<NAT>(sv[t], m_use);
             lsum += sv[t];
         }
         l_run = l_run * alpha + lsum;
@@ -170,7 +177,7 @@ __global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* 
         const float m_use = m == -INFINITY ? 0.f : m;
 #pragma unroll
         for (int w = 0; w < WAVES; w++) {
-            const float al = __builtin_amdgcn_exp2f(ml[0][w][q] - m_use);
+            const float al = weight<NAT>(ml[0][w][q], m_use);
             l = fmaf(ml[1][w][q], al, l);
             o = fmaf(sums[w][f][(i >> 2) * 16 + q][i & 3], al, o);
         }
@@ -186,7 +193,7 @@ __global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* 
 }
 
 // The parts of a split key range: one thread per element of O.
-template <typename T, int D>
+template <typename T, int D, bool HAS_MASK>
 __global__ __launch_bounds__(256) void fa_decode_combine_kernel(FaArgs a, const float* part, int parts) {
     const int64_t rows = (int64_t)a.B * a.H * a.Sq, idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (idx >= rows * D) return;
@@ -197,7 +204,7 @@ __global__ __launch_bounds__(256) void fa_decode_combine_kernel(FaArgs a, const 
     for (int p = 0; p < parts; p++) m = fmaxf(m, mls[(p * rows + row) * 2]);
     const float m_use = m == -INFINITY ? 0.f : m;
     for (int p = 0; p < parts; p++) {
-        const float al = __builtin_amdgcn_exp2f(mls[(p * rows + row) * 2] - m_use);
+        const float al = weight<kNatural<T, HAS_MASK>>(mls[(p * rows + row) * 2], m_use);
         l = fmaf(mls[(p * rows + row) * 2 + 1], al, l);
         o = fmaf(part[(p * rows + row) * D + d], al, o);
     }
@@ -222,7 +229,9 @@ int launch(hipStream_t s, const FaArgs& a, float* part, int parts) {
     else hipLaunchKernelGGL((fa_decode_kernel<T, D, false, WAVES>), grid, dim3(64 * WAVES), 0, s, a, parts > 1 ? part : nullptr, per);
     if (parts > 1) {
         const int64_t n = bh * a.Sq * D;
-        hipLaunchKernelGGL((fa_decode_combine_kernel<T, D>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, part, (int)grid.y);
+        const dim3 combine((unsigned)((n + 255) / 256));
+        if (a.mask) hipLaunchKernelGGL((fa_decode_combine_kernel<T, D, true>), combine, dim3(256), 0, s, a, part, (int)grid.y);
+        else hipLaunchKernelGGL((fa_decode_combine_kernel<T, D, false>), combine, dim3(256), 0, s, a, part, (int)grid.y);
     }
     return check_launch("flash_attention_decode");
 }

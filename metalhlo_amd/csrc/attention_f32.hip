@@ -113,7 +113,7 @@ __global__ __launch_bounds__(256, 2) void fa_f32_mfma_kernel(FaArgs a, float sca
         for (int s = 0; s < NS; s++)
             sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(ks[ln * KS + 2 * s + h], qf[s], sacc, 0, 0, 0);
 
-        // ---- scale, mask, block maximum (log2 domain)
+        // ---- scale, mask, block maximum (log2 domain unless there is a mask)
         float t[16];
         float m_blk = -INFINITY;
 #pragma unroll
@@ -123,21 +123,21 @@ __global__ __launch_bounds__(256, 2) void fa_f32_mfma_kernel(FaArgs a, float sca
             bool keep = key < a.Skv && q_live;
             if (CAUSAL) keep = keep && key <= qpos;
             if (HAS_MASK) { if (keep) sv += mp[key]; }
-            t[i] = keep ? sv * kLog2e : -INFINITY;
+            t[i] = keep ? (HAS_MASK ? sv : sv * kLog2e) : -INFINITY;
             m_blk = fmaxf(m_blk, t[i]);
         }
         m_blk = half_max(m_blk);
         // (a reference maximum that moves only when the block exceeds it by 2^8: see moved_reference)
-        const float m_new = moved_reference(m_run, m_blk);
+        const float m_new = moved_reference<HAS_MASK>(m_run, m_blk);
         const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
         // (v_exp_f32 itself, about 1 ulp: the library exp2f wraps it in five more instructions that
         // only serve results below 2^-126, which are zeros here either way)
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+        const float alpha = weight<HAS_MASK>(m_run, m_use);
         m_run = m_new;
         float psum = 0.f;
 #pragma unroll
         for (int i = 0; i < 16; i++) {
-            t[i] = __builtin_amdgcn_exp2f(t[i] - m_use);
+            t[i] = weight<HAS_MASK>(t[i], m_use);
             psum += t[i];
         }
         l_run = l_run * alpha + psum;
@@ -255,18 +255,18 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaAr
             float sv = sacc[i] * scale;
             const bool keep = !edge || (key < a.Skv && (!CAUSAL || key <= qpos));
             if (HAS_MASK) sv += mask_runs ? mrun[HAS_MASK ? i >> 2 : 0][i & 3] : key < a.Skv ? mp[key] : 0.f;
-            t[i] = keep ? sv * kLog2e : -INFINITY;
+            t[i] = keep ? (HAS_MASK ? sv : sv * kLog2e) : -INFINITY;
             m_blk = fmaxf(m_blk, t[i]);
         }
         m_blk = half_max(m_blk);
-        const float m_new = moved_reference(m_run, m_blk);
+        const float m_new = moved_reference<HAS_MASK>(m_run, m_blk);
         const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+        const float alpha = weight<HAS_MASK>(m_run, m_use);
         m_run = m_new;
         float psum = 0.f;
 #pragma unroll
         for (int i = 0; i < 16; i++) {
-            t[i] = __builtin_amdgcn_exp2f(t[i] - m_use);
+            t[i] = weight<HAS_MASK>(t[i], m_use);
             psum += t[i];
         }
         l_run = l_run * alpha + psum;
@@ -303,7 +303,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaAr
             const float m_use = m == -INFINITY ? 0.f : m;
 #pragma unroll
             for (int w = 0; w < 4; w++) {
-                const float al = __builtin_amdgcn_exp2f(ml[0][w][q] - m_use);
+                const float al = weight<HAS_MASK>(ml[0][w][q], m_use);
                 l = fmaf(ml[1][w][q], al, l);
                 sum = fmaf(part[w][q][col], al, sum);
             }
