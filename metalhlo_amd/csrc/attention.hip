@@ -29,6 +29,63 @@ namespace mhip {
 
 template <typename T> struct alignas(4) Pair16 { T v[2]; };
 
+// One query row by one wave, q, k, v, o packed: per block of 64 keys, lanes own keys for the scores, then own head-dim
+// columns for the weighted sum.  The recurrence is the reference's (FlashAttentionKernel.swift:589-598) applied per
+// block of keys; a causally hidden key is never read.  `qs` (256 floats) and `ps` (64): LDS of the wave's own.
+template <typename T>
+__device__ inline void fa_row(const FaArgs& a, int64_t bh, int qpos, int D, float scale, float* qs, float* ps) {
+    const int lane = threadIdx.x & 63;
+    const T* qp = static_cast<const T*>(a.q) + (bh * a.Sq + qpos) * D;
+    const T* kp = static_cast<const T*>(a.k) + bh * a.Skv * D;
+    const T* vp = static_cast<const T*>(a.v) + bh * a.Skv * D;
+    const T* mp = a.mask ? static_cast<const T*>(a.mask) + (bh / a.H) * a.mask_sb +
+                               (bh % a.H) * a.mask_sh + (int64_t)qpos * a.Skv
+                         : nullptr;
+    for (int d = lane; d < D; d += 64) qs[d] = Elem<T>::to_f32(qp[d]);
+    __builtin_amdgcn_wave_barrier();
+    float oacc[4] = {0.f, 0.f, 0.f, 0.f};
+    float m_run = -INFINITY, l_run = 0.f;
+    const int kv_end = a.is_causal ? min(a.Skv, qpos + 1) : a.Skv;
+    for (int kv0 = 0; kv0 < kv_end; kv0 += 64) {
+        const int key = kv0 + lane;
+        float s = -INFINITY;
+        if (key < kv_end) {
+            float acc = 0.f;
+            const T* kr = kp + (int64_t)key * D;
+            for (int d = 0; d < D; d++) acc = fmaf(qs[d], Elem<T>::to_f32(kr[d]), acc);
+            s = acc * scale;
+            if (mp) s += Elem<T>::to_f32(mp[key]);
+        }
+        const float m_new = fmaxf(m_run, wave_max(s));
+        const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+        const float alpha = expf(m_run - m_use);
+        const float p = expf(s - m_use);
+        m_run = m_new;
+        l_run = l_run * alpha + wave_sum(p);
+        ps[lane] = p;
+        __builtin_amdgcn_wave_barrier();
+        const int nk = min(64, kv_end - kv0);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int d = lane + 64 * j;
+            if (d < D) {
+                float acc = oacc[j] * alpha;
+                for (int t = 0; t < nk; t++)
+                    acc = fmaf(ps[t], Elem<T>::to_f32(vp[(int64_t)(kv0 + t) * D + d]), acc);
+                oacc[j] = acc;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    const float inv = l_run > 1e-10f ? 1.f / l_run : 0.f;
+    T* orow = static_cast<T*>(a.o) + (bh * a.Sq + qpos) * D;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int d = lane + 64 * j;
+        if (d < D) orow[d] = Elem<T>::from_f32(oacc[j] * inv);
+    }
+}
+
 // NB: depth of the K and of the V ring in LDS.  Two everywhere: with head size 64 a ring of three or
 // four measured 8 to 13 % slower (B8 H12 S1024: 38.5 / 40.5 against 35.7 us) -- it costs the third
 // resident workgroup per CU, which hides more latency than the deeper prefetch does.
@@ -313,7 +370,20 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(FaArgs a) {
     // ---- normalise and store: lane holds 4 consecutive d per register group -
     const float l_tot = half_sum(l_run);
     const float inv = l_tot > 1e-10f ? 1.f / l_tot : 0.f;
-    if (qpos < a.Sq) {
+    // PART: a product with an infinity or a NaN in V reaches every row whose wave met that key, through a weight of zero
+    // too, and a sum in parts of the weight has no sign for an infinity.  Such rows (a sum that is not finite) are formed
+    // again the scalar way, in the LDS that the tiles no longer need.
+    bool whole = true;
+    if (PART) {
+        float probe = 0.f * l_tot;
+#pragma unroll
+        for (int i = 0; i < ND; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) probe = fmaf(oacc[i][r], 0.f, probe);
+        whole = half_sum(probe) == 0.f;
+        __syncthreads();
+    }
+    if (qpos < a.Sq && whole) {
         T* orow = op + (int64_t)qpos * a.os[2];
 #pragma unroll
         for (int dt = 0; dt < ND; dt++)
@@ -325,75 +395,24 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(FaArgs a) {
                 if (!PART || 32 * dt + 8 * g + 4 * lhalf < head) *reinterpret_cast<u32x2*>(orow + 32 * dt + 8 * g + 4 * lhalf) = w;
             }
     }
+    if (PART) {
+        uint32_t again = (uint32_t)__ballot(!whole && qpos < a.Sq);       // (the lower half holds a bit per row)
+        float* mem = reinterpret_cast<float*>(smem) + wave_s * 320;
+        for (; again; again &= again - 1)
+            fa_row<T>(a, bh, qw + __builtin_ctz(again), head, a.negate_q ? -a.scale : a.scale, mem, mem + 256);
+    }
 }
 
 // ---------------------------------------------------------------------------
 // Scalar path: one wave per query row, any type, D <= 256.
-// Per block of 64 keys: lanes own keys for the scores, then own head-dim
-// columns for the weighted sum.  The recurrence is the reference's
-// (FlashAttentionKernel.swift:589-598) applied per block of keys.
 // ---------------------------------------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(256) void fa_scalar_kernel(FaArgs a, int D, float scale) {
     __shared__ float qs[4][256];
     __shared__ float ps[4][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wave = threadIdx.x >> 6;
     const int64_t row = (int64_t)blockIdx.x * 4 + wave;      // over B*H*Sq
-    const int64_t nrows = (int64_t)a.B * a.H * a.Sq;
-    const bool live = row < nrows;
-    const int64_t bh = live ? row / a.Sq : 0;
-    const int qpos = live ? (int)(row % a.Sq) : 0;
-    const T* qp = static_cast<const T*>(a.q) + (bh * a.Sq + qpos) * D;
-    const T* kp = static_cast<const T*>(a.k) + bh * a.Skv * D;
-    const T* vp = static_cast<const T*>(a.v) + bh * a.Skv * D;
-    const T* mp = a.mask ? static_cast<const T*>(a.mask) + (bh / a.H) * a.mask_sb +
-                               (bh % a.H) * a.mask_sh + (int64_t)qpos * a.Skv
-                         : nullptr;
-    for (int d = lane; d < D; d += 64) qs[wave][d] = live ? Elem<T>::to_f32(qp[d]) : 0.f;
-    __syncthreads();
-    float oacc[4] = {0.f, 0.f, 0.f, 0.f};
-    float m_run = -INFINITY, l_run = 0.f;
-    const int kv_end = live ? (a.is_causal ? min(a.Skv, qpos + 1) : a.Skv) : 0;
-    for (int kv0 = 0; kv0 < kv_end; kv0 += 64) {
-        const int key = kv0 + lane;
-        float s = -INFINITY;
-        if (key < kv_end) {
-            float acc = 0.f;
-            const T* kr = kp + (int64_t)key * D;
-            for (int d = 0; d < D; d++) acc = fmaf(qs[wave][d], Elem<T>::to_f32(kr[d]), acc);
-            s = acc * scale;
-            if (mp) s += Elem<T>::to_f32(mp[key]);
-        }
-        const float m_new = fmaxf(m_run, wave_max(s));
-        const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-        const float alpha = expf(m_run - m_use);
-        const float p = expf(s - m_use);
-        m_run = m_new;
-        l_run = l_run * alpha + wave_sum(p);
-        ps[wave][lane] = p;
-        __builtin_amdgcn_wave_barrier();
-        const int nk = min(64, kv_end - kv0);
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int d = lane + 64 * j;
-            if (d < D) {
-                float acc = oacc[j] * alpha;
-                for (int t = 0; t < nk; t++)
-                    acc = fmaf(ps[wave][t], Elem<T>::to_f32(vp[(int64_t)(kv0 + t) * D + d]), acc);
-                oacc[j] = acc;
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-    }
-    if (live) {
-        const float inv = l_run > 1e-10f ? 1.f / l_run : 0.f;
-        T* orow = static_cast<T*>(a.o) + (bh * a.Sq + qpos) * D;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int d = lane + 64 * j;
-            if (d < D) orow[d] = Elem<T>::from_f32(oacc[j] * inv);
-        }
-    }
+    if (row < (int64_t)a.B * a.H * a.Sq) fa_row<T>(a, row / a.Sq, (int)(row % a.Sq), D, scale, qs[wave], ps[wave]);
 }
 
 template <typename T, int D, int DR = D, bool PART = false>

@@ -19,7 +19,7 @@ struct FaArgs {
     void* o;
     int B, H, Sq, Skv;
     float c;          // |scale| * log2(e)
-    float scale;      // |scale| (read by the decode kernel)
+    float scale;      // |scale|
     int negate_q;     // scale < 0: flip the sign of Q instead
     int is_causal;    // read by the scalar path (the MFMA path is templated on it)
     int64_t mask_sb, mask_sh;

@@ -49,3 +49,32 @@ def test_head_sizes(B, H, Sq, Skv, causal, mask, D, dtype):
     tiny = 2.0 ** -24 if dtype == torch.float16 else 0.0       # f16's smallest numbers are evenly spaced
     assert np.all(diff <= bound + ROUNDOFF[dtype] * (np.abs(e) + bound) + tiny), (diff.max(), np.abs(e).max())
     assert torch.isnan(guard[-64:]).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=lambda d: NAME[d])
+@pytest.mark.parametrize("D", [24, 40, 80, 96, 120])
+@pytest.mark.parametrize("causal,mask", [(True, False), (False, False), (True, True)], ids=lambda v: str(v))
+def test_values_that_are_not_finite(causal, mask, D, dtype):
+    """An infinity or a NaN in V reaches the rows that see its key, as itself, and no other: rows in front of a causally
+    hidden key (same 64-key block included) are those of clean operands, other columns and heads too."""
+    from metalhlo_amd import kernels
+    B, H, S = 2, 3, 200
+    rng = np.random.default_rng(D)
+    q, k, v = (to_dev(rng.standard_normal((B, H, S, D)) * 0.5, dtype) for _ in range(3))
+    md = to_dev(rng.standard_normal((B, 1, S, S)), dtype) if mask else None
+    e, bound = _reference(as_f64(q), as_f64(k), as_f64(v), D ** -0.5, causal, None if md is None else as_f64(md))
+    plus, minus, nan = 131, 150, 190                       # keys
+    w = v.clone()
+    w[0, 1, plus, 3] = float("inf")
+    w[0, 1, minus, D - 1] = float("-inf")
+    w[1, 2, nan] = float("nan")
+    got = as_f64(kernels.flash_attention(q, k, w, is_causal=causal, mask=md))
+    sees = lambda key: np.arange(S) >= key if causal else np.ones(S, bool)  # noqa: E731
+    want = e.copy()
+    want[0, 1, sees(plus), 3] = np.inf
+    want[0, 1, sees(minus), D - 1] = -np.inf
+    want[1, 2, sees(nan)] = np.nan
+    clean = np.isfinite(want)
+    tiny = 2.0 ** -24 if dtype == torch.float16 else 0.0
+    assert np.all(np.abs(got - e)[clean] <= (bound + ROUNDOFF[dtype] * (np.abs(e) + bound) + tiny)[clean])
+    assert np.array_equal(got[~clean], want[~clean], equal_nan=True)
