@@ -14,11 +14,13 @@
 // accumulations are fp32; the output is rounded once.
 //
 // Head sizes other than 64 and 128 lie in LDS rows of 64 or 128 (the pieces behind the row's end are zeros) and
-// skip the matrix steps of whole blocks of 32 d that do not exist.  Their probabilities go through the second
-// product as two 16-bit parts, p = hi + lo: to about 2^-17 they enter it as the fp32 values they are.
+// skip the matrix steps of whole blocks of 32 d that do not exist.  Their probabilities go through the second product
+// with all of their fp32 bits, as three bf16 parts; f16 values as two bf16 parts, which holds them exactly too.
 //
-// On bf16 B4 H12 S1000 causal: D 96 729 -> 31.6 us against the scalar path, D 32 346 -> 20.4, errors against 64
-// bits the same to five digits.
+// On B4 H12 S1000 causal against the scalar path: bf16 D 96 729 -> 35.6 us, D 32 346 -> 20.6; f16 D 96 52.3, D 32 26.6
+// (two products more per part, and V split in registers).  Share of the results that are not the number nearest to
+// the 64-bit one, scalar path / here, D 96: bf16 0.0003 / 0.0002, f16 0.0027 / 0.0016; with two parts of the
+// weights bf16 was at 0.0023.
 //
 // Everything else (unaligned tensors, larger heads) takes a wave-per-query scalar path.
 #include <type_traits>
@@ -86,6 +88,21 @@ __device__ inline void fa_row(const FaArgs& a, int64_t bh, int qpos, int D, floa
     }
 }
 
+// Eight f16 numbers as bf16 pairs hi + lo, exactly: 8 of the 11 significant bits and the other 3.
+__device__ __forceinline__ void split_f16(u32x4& v, u32x4& lo) {
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    auto narrow = [](f16x2 h) {        // (both fit bf16: truncation is exact)
+        return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, (float)h[1]), __builtin_bit_cast(uint32_t, (float)h[0]), 0x07060302u);
+    };
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const uint32_t w = v[e];
+        const f16x2 h = __builtin_bit_cast(f16x2, w & 0xFFF8FFF8u), l = __builtin_bit_cast(f16x2, w) - h;
+        v[e] = narrow(h);
+        lo[e] = narrow(l);
+    }
+}
+
 // NB: depth of the K and of the V ring in LDS.  Two everywhere: with head size 64 a ring of three or
 // four measured 8 to 13 % slower (B8 H12 S1024: 38.5 / 40.5 against 35.7 us) -- it costs the third
 // resident workgroup per CU, which hides more latency than the deeper prefetch does.
@@ -99,6 +116,7 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(FaArgs a) {
     constexpr int kRowsPerInst = 64 / CPR;      // tile rows one wave-wide LDS-DMA load fills
     constexpr int kInst = kBKV / kRowsPerInst / 4;   // such loads per wave per tile
     constexpr int ND = DR / 32, NS = DR / 16;
+    constexpr bool kSplitV = PART && std::is_same<T, f16_t>::value;
     constexpr int kLoadsPerTile = 2 * kInst;    // per wave
     __shared__ __attribute__((aligned(1024))) char smem[2 * NB * kTile];   // K ring, then V ring
 
@@ -321,45 +339,59 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(FaArgs a) {
 #pragma unroll
                     for (int r = 0; r < 16; r++) oacc[i][r] *= alpha;
             }
-            // ---- P^T as B operand: slot j of step u is register 8u + j ------
-            u32x4 pb[4];
+            // ---- O^T += V^T . P^T.  B operand: slot j of step u is register 8u + j; A operand: slot j of step u is
+            // key 16u + 8(j/4) + 4*lhalf + j%4, i.e. two transposing reads 8 keys apart
+            auto v_frag = [&](int u, int dt) {
+                const int row = 16 * u + v_row0;
+                const int d0 = 32 * dt + v_d0;
+                const char* p0 = vt + v_off<D>(row, d0 >> 3) + (d0 & 7) * 2;
+                const char* p1 = vt + v_off<D>(row + 8, d0 >> 3) + (d0 & 7) * 2;
+                const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((fa_lds_s16x4*)p0));
+                const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((fa_lds_s16x4*)p1));
+                return u32x4{lo.x, lo.y, hi.x, hi.y};
+            };
+            if constexpr (PART) {
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                pb[u].x = Mfma32A<T>::pack2(sv[8 * u + 0], sv[8 * u + 1]);
-                pb[u].y = Mfma32A<T>::pack2(sv[8 * u + 2], sv[8 * u + 3]);
-                pb[u].z = Mfma32A<T>::pack2(sv[8 * u + 4], sv[8 * u + 5]);
-                pb[u].w = Mfma32A<T>::pack2(sv[8 * u + 6], sv[8 * u + 7]);
-            }
-            // (PART: what the rounding took, as a second operand)
-            u32x4 pl[PART ? 4 : 1];
-            if (PART) {
+                for (int u = 0; u < 4; u++) {
+                    u32x4 p[3];
+#pragma unroll
+                    for (int part = 0; part < 3; part++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            float &x = sv[8 * u + 2 * e], &y = sv[8 * u + 2 * e + 1];
+                            const uint32_t w = Mfma32A<bf16_t>::pack2(x, y);
+                            p[part][e] = w;
+                            x -= __builtin_bit_cast(float, w << 16);
+                            y -= __builtin_bit_cast(float, w & 0xFFFF0000u);
+                        }
+                    u32x4 vf[ND], vl[ND];
+#pragma unroll
+                    for (int dt = 0; dt < ND; dt++) {
+                        vf[dt] = v_frag(u, dt);
+                        if (kSplitV) split_f16(vf[dt], vl[dt]);
+                    }
+#pragma unroll
+                    for (int part = 2; part >= 0; part--)
+#pragma unroll
+                        for (int dt = 0; dt < ND; dt++) {
+                            if (kSplitV) oacc[dt] = Mfma32A<bf16_t>::run(vl[dt], p[part], oacc[dt]);
+                            oacc[dt] = Mfma32A<bf16_t>::run(vf[dt], p[part], oacc[dt]);
+                        }
+                }
+            } else {
+                u32x4 pb[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    pb[u].x = Mfma32A<T>::pack2(sv[8 * u + 0], sv[8 * u + 1]);
+                    pb[u].y = Mfma32A<T>::pack2(sv[8 * u + 2], sv[8 * u + 3]);
+                    pb[u].z = Mfma32A<T>::pack2(sv[8 * u + 4], sv[8 * u + 5]);
+                    pb[u].w = Mfma32A<T>::pack2(sv[8 * u + 6], sv[8 * u + 7]);
+                }
+                __builtin_amdgcn_s_setprio(2);
 #pragma unroll
                 for (int u = 0; u < 4; u++)
 #pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const uint32_t w = pb[u][e];       // (a value: bit_cast of the vector's element reads element 0)
-                        const Pair16<T> hi = __builtin_bit_cast(Pair16<T>, w);
-                        pl[PART ? u : 0][e] = Mfma32A<T>::pack2(sv[8 * u + 2 * e] - Elem<T>::to_f32(hi.v[0]), sv[8 * u + 2 * e + 1] - Elem<T>::to_f32(hi.v[1]));
-                    }
-            }
-            __builtin_amdgcn_s_setprio(2);
-            // ---- O^T += V^T . P^T: A operand slot j of step u is key
-            // 16u + 8(j/4) + 4*lhalf + j%4, i.e. two transposing reads 8 keys apart
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-#pragma unroll
-                for (int dt = 0; dt < ND; dt++) {
-                    const int row = 16 * u + v_row0;
-                    const int d0 = 32 * dt + v_d0;
-                    const char* p0 = vt + v_off<D>(row, d0 >> 3) + (d0 & 7) * 2;
-                    const char* p1 = vt + v_off<D>(row + 8, d0 >> 3) + (d0 & 7) * 2;
-                    const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((fa_lds_s16x4*)p0));
-                    const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((fa_lds_s16x4*)p1));
-                    u32x4 vf;
-                    vf.x = lo.x; vf.y = lo.y; vf.z = hi.x; vf.w = hi.y;
-                    oacc[dt] = Mfma32A<T>::run(vf, pb[u], oacc[dt]);
-                    if (PART) oacc[dt] = Mfma32A<T>::run(vf, pl[PART ? u : 0], oacc[dt]);
-                }
+                    for (int dt = 0; dt < ND; dt++) oacc[dt] = Mfma32A<T>::run(v_frag(u, dt), pb[u], oacc[dt]);
             }
             __builtin_amdgcn_s_setprio(0);
         }

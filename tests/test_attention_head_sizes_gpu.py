@@ -2,7 +2,7 @@
 (rows padded to 64 or 128 in LDS), the rest on the scalar kernel; block edges, masks, negative scale.
 
 Bound, with P the exact probabilities: a score is off by at most (D + 2) 2^-24 of scale sum |q||k|, a probability
-by twice the largest of those in relative terms, 2^-16 for its two 16-bit parts and Skv 2^-24 for its sums; the
+by twice the largest of those in relative terms, 2^-22 for its exponential and Skv 2^-24 for its sums; the
 result is that times sum P |v|, rounded once to its type."""
 import numpy as np
 import pytest
@@ -24,7 +24,7 @@ def _reference(q, k, v, scale, causal, mask):
     m = s.max(-1, keepdims=True)
     p = np.exp(s - np.where(np.isfinite(m), m, 0))
     p = p / np.maximum(p.sum(-1, keepdims=True), 1e-300)
-    return p @ v, (2 * err + 2.0 ** -16 + (s.shape[-1] + 8) * 2.0 ** -24) * (p @ np.abs(v))
+    return p @ v, (2 * err + 2.0 ** -22 + (s.shape[-1] + 8) * 2.0 ** -24) * (p @ np.abs(v))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=lambda d: NAME[d])
@@ -78,3 +78,40 @@ def test_values_that_are_not_finite(causal, mask, D, dtype):
     tiny = 2.0 ** -24 if dtype == torch.float16 else 0.0
     assert np.all(np.abs(got - e)[clean] <= (bound + ROUNDOFF[dtype] * (np.abs(e) + bound) + tiny)[clean])
     assert np.array_equal(got[~clean], want[~clean], equal_nan=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=lambda d: NAME[d])
+@pytest.mark.parametrize("D", [40, 96])
+def test_probabilities_keep_their_fp32_bits(D, dtype):
+    """Values of +1 and -1 under weights that differ by 2^-15 of themselves: what is left of their sum shows every bit
+    a weight lost on its way into the product.  A score of -t (t below 1) is off by 2^-24, its exponential by 2^-22 in
+    all and the sums of 130 keys by 2^-21 of the sum of weights."""
+    from metalhlo_amd import kernels
+    S, n = 130, 64
+    q, k, v = (np.zeros((1, 2, S, D)) for _ in range(3))
+    q[..., 0] = 0.5 + np.arange(S) / 512
+    q[..., 1] = 2.0 ** -7
+    k[..., 1:1 + n, 0] = k[..., 1 + n:1 + 2 * n, 0] = -1.0
+    k[..., 1 + n:1 + 2 * n, 1] = 2.0 ** -8
+    v[..., 1:1 + n, :], v[..., 1 + n:1 + 2 * n, :] = -1.0, 1.0
+    q, k, v = (to_dev(x, dtype) for x in (q, k, v))
+    got = as_f64(kernels.flash_attention(q, k, v, scale=1.0))
+    e, _ = _reference(as_f64(q), as_f64(k), as_f64(v), 1.0, False, None)
+    assert e.min() > 2.0 ** -17
+    assert np.all(np.abs(got - e) <= 2.0 ** -21 + ROUNDOFF[dtype] * e)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=lambda d: NAME[d])
+def test_small_probabilities_count(dtype):
+    """A key of weight one whose value is zero, and weights of e^-21 on large values, far below f16's smallest number."""
+    from metalhlo_amd import kernels
+    S, D = 100, 72
+    q, k, v = (np.zeros((1, 1, S, D)) for _ in range(3))
+    q[..., :2] = 1.0
+    k[..., 1:, 0], k[..., 1:, 1] = -20.0, -1.0
+    v[..., 1:, :] = 60000.0
+    q, k, v = (to_dev(x, dtype) for x in (q, k, v))
+    got = as_f64(kernels.flash_attention(q, k, v, scale=1.0))
+    e = 99 * np.exp(-21.0) * as_f64(v)[0, 0, 1, 0] / (1 + 99 * np.exp(-21.0))
+    # (an exponent of 21 is off by 2^-19; f16's subnormal numbers do not come into it: e is 4.5e-3)
+    assert np.all(np.abs(got - e) <= (2.0 ** -18 + ROUNDOFF[dtype]) * e)
