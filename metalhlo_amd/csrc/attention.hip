@@ -404,7 +404,9 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(FaArgs a) {
     const float inv = l_tot > 1e-10f ? 1.f / l_tot : 0.f;
     // PART: a product with an infinity or a NaN in V reaches every row whose wave met that key, through a weight of zero
     // too, and a sum in parts of the weight has no sign for an infinity.  Such rows (a sum that is not finite) are formed
-    // again the scalar way, in the LDS that the tiles no longer need.
+    // again the scalar way, in the LDS that the tiles no longer need.  So are rows of scores beyond 2^28 without a
+    // mask: the fused multiply-add of an interior block and the rounded product of a boundary block are then apart by more
+    // than a weight can stand.
     bool whole = true;
     if (PART) {
         float probe = 0.f * l_tot;
@@ -412,7 +414,7 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(FaArgs a) {
         for (int i = 0; i < ND; i++)
 #pragma unroll
             for (int r = 0; r < 16; r++) probe = fmaf(oacc[i][r], 0.f, probe);
-        whole = half_sum(probe) == 0.f;
+        whole = half_sum(probe) == 0.f && (HAS_MASK || m_run == -INFINITY || fabsf(m_run) < 0x1p28f);
         __syncthreads();
     }
     if (qpos < a.Sq && whole) {

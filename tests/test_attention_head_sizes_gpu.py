@@ -115,3 +115,22 @@ def test_small_probabilities_count(dtype):
     e = 99 * np.exp(-21.0) * as_f64(v)[0, 0, 1, 0] / (1 + 99 * np.exp(-21.0))
     # (an exponent of 21 is off by 2^-19; f16's subnormal numbers do not come into it: e is 4.5e-3)
     assert np.all(np.abs(got - e) <= (2.0 ** -18 + ROUNDOFF[dtype]) * e)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=lambda d: NAME[d])
+@pytest.mark.parametrize("D,S,causal,unit", [(24, 70, False, 14), (96, 200, True, 14), (40, 130, True, 12), (72, 300, False, 13)], ids=lambda v: str(v))
+def test_large_scores(D, S, causal, unit, dtype):
+    """Scores of 2^24 to 2^38 that fp32 holds exactly (small integers times a power of two): the largest share the row."""
+    from metalhlo_amd import kernels
+    rng = np.random.default_rng(S)
+    q, k = (to_dev(rng.integers(-3, 4, (1, 2, S, D)) * 2.0 ** unit, dtype) for _ in range(2))
+    k[..., 1::3, :] = k[..., 0:1, :]                        # many equal keys
+    v = to_dev(rng.standard_normal((1, 2, S, D)), dtype)
+    got = as_f64(kernels.flash_attention(q, k, v, scale=1.0, is_causal=causal))
+    s = as_f64(q) @ np.swapaxes(as_f64(k), -1, -2)
+    if causal:
+        s = np.where(np.arange(S) > np.arange(S)[:, None], -np.inf, s)
+    p = (s == s.max(-1, keepdims=True)).astype(float)
+    p /= p.sum(-1, keepdims=True)
+    e, sums = p @ as_f64(v), (S + 8) * 2.0 ** -24 * (p @ np.abs(as_f64(v)))
+    assert np.all(np.abs(got - e) <= sums + ROUNDOFF[dtype] * (np.abs(e) + sums) + 2.0 ** -24)
