@@ -258,17 +258,21 @@ bool wide_strips(int64_t N, int64_t K, int64_t batch, bool tb) {
     return tb ? strips >= 128 && K >= 2048 : strips >= 128 || (strips >= 64 && K >= 2048);
 }
 
-// K split over the grid as well (fp32 sums in a workspace, one more launch) while that leaves every workgroup 1024 k and
-// at most one of them per compute unit, from a K on where the shorter chain pays for the launch.  us, whole / split:
-// [4,4096] x [4096,4096] 13.0 / 9.5, [28,6384] x [6384,688] 17.4 / 8.4, [32,3072] x [3072,768] 10.4 / 8.8 but
-// [4,3072] x [3072,768] 6.4 / 6.7 and [16,2048] x [2048,2048] 6.2 / 7.3.  fp32 [40,3072] x [3072,768] 15.5 / 13.2; blocks of
-// more than 64 rows fill the device earlier ([128,3072] x [3072,768] 16.4 / 20.5) and keep 2048 k.
+// K split over the grid as well (fp32 sums in a workspace, one more launch): parts of about 1024 k, at most one
+// workgroup per compute unit.  From which K on that pays for the launch was swept with weights from memory, M 1 to 64, N 256 to
+// 4096; time in parts over time whole, the range over N:
+//   16-bit [K, N], up to 32 rows   K 2048 0.86 to 1.26   K 2560 0.71 to 1.02   K 3064 0.66 to 0.96
+//   16-bit [N, K], up to 16 rows   K 2560 1.02 to 1.31   K 3064 1.12 to 1.39   K 3584 0.85 to 1.18   (whole lines: it is the shorter
+//   16-bit [N, K], 32 rows         K 2048 1.05           K 2560 0.88 to 0.99   K 3064 0.87 to 0.98    product to begin with)
+//   fp32, up to 32 rows            K 2048 0.82 to 1.31   K 2560 0.70 to 1.08   K 3064 0.66 to 1.02
+//   fp32, 64 rows                  K 2560 0.87 to 1.38   K 3064 0.82 to 1.26   K 3584 0.69 to 1.14
+// Blocks of more than 64 rows (fp32) fill the device earlier ([128,3072] x [3072,768] 16.4 us whole, 20.5) and keep 2048 k.
 int skinny_splits(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b, bool is16) {
     if (batch != 1 || M * N > (1 << 20)) return 1;
     const int64_t width = wide_strips(N, K, 1, trans_b != 0) ? (trans_b ? 32 : 64) : (trans_b ? 16 : 32);
-    const bool fine = K >= 4096 || (K >= 3072 && (M >= 16 || !is16));
-    const int64_t room = 256 / ((N + width - 1) / width), want = M <= 64 && fine ? K / 1024 : K / 2048 + (K % 2048 > 1024);
-    const int64_t n = room < want ? room : want;
+    const int64_t from = is16 ? (trans_b && M <= 16 ? 3584 : 2560) : (M > 32 ? 3072 : 2560);
+    const int64_t want = M > 64 ? K / 2048 + (K % 2048 > 1024) : K >= from ? (K + 512) / 1024 : 1;
+    const int64_t room = 256 / ((N + width - 1) / width), n = room < want ? room : want;
     return n < 2 ? 1 : n > 8 ? 8 : (int)n;
 }
 

@@ -91,3 +91,15 @@ def test_split_sums_of_few_columns(M, N, K, dtype):
     e = A @ B + c
     fp32 = (K + 2) * 2.0 ** -24 * (np.abs(A) @ np.abs(B) + np.abs(c))
     assert np.all(np.abs(got - e) <= fp32 + ROUNDOFF[dtype] * (np.abs(e) + fp32))
+
+
+@pytest.mark.parametrize("M,line,tb,dtype", [(4, 2560, False, torch.bfloat16), (16, 3584, True, torch.bfloat16), (17, 2560, True, torch.bfloat16), (12, 2560, True, torch.float32),
+                                             (40, 3072, False, torch.float32)], ids=str)
+def test_both_sides_of_the_split_lines(M, line, tb, dtype):
+    """From K = line on a few-row product is split; eight k before it is not."""
+    from metalhlo_amd import _lib
+    code = {torch.bfloat16: 3, torch.float32: 1}[dtype]
+    assert _lib.load().mhip_gemm_workspace(M, 264, line, 1, 0, int(tb), code) > 0
+    assert _lib.load().mhip_gemm_workspace(M, 264, line - 8, 1, 0, int(tb), code) == 0
+    for K in (line - 8, line):
+        _check(M, 264, K, dtype, False, tb, residual=True)
