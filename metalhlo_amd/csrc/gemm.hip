@@ -532,6 +532,10 @@ using namespace mhip;
 // 16-bit rows 33 to 64, in two blocks, with weights that were not just used: [37,768] x K 768 7.5 -> 6.7 us, [64,4096] x K 1024
 // 10.0 -> 8.9, but [64,8192] x K 768 9.0 against 11.6; stored [N, K]: [64,2000] x [1000,2000]^T 8.6 -> 6.5, [64,768] x [3072,768]^T
 // 5.9 against 7.3.
+// Both sides of these lines, 16-bit, few-row time over tile time with weights from memory (N 512 to 8192, K 512 to 6144):
+// rows 33 to 64 stored [N, K], K up to 2048: N up to 1536 0.79 to 1.06, N 2048 0.83 to 0.92, N 3072 0.92 to 1.31, and K 3072 1.08
+// to 1.7; stored [K, N], K up to 1536: N up to 4096 0.91 to 1.12, N 6144 1.17 to 1.48, and K 3072 1.06 to 1.7.  Rows 17 to 32:
+// stored [N, K] 0.68 to 1.06 up to N 4096 and K 2048, 0.7 to 1.65 beyond; stored [K, N] 0.8 to 1.4 for 20 rows, 0.9 to 1.5 for 32.
 static bool skinny_rows(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b, bool is16) {
     if (!is16) return M <= 64 || (M <= 192 && (M + 63) / 64 * ((N + 63) / 64) * batch <= 160);
     return M <= 16 || (M <= 32 && N * K <= (32 << 20)) || (M <= 64 && (trans_b ? N * batch <= 1536 && K <= 2048 : N * batch <= 4096 && K <= 1536));

@@ -24,7 +24,7 @@ struct GemmArgs {
     int tiles_m, tiles_n;
     const void* residual = nullptr;   // C's layout and batch stride; added after the activation (may alias c)
     int ldc = 0;                      // row stride of C and the residual in elements; 0 = N (gemm256.hip only: a column slice of a wider C)
-    float* partial = nullptr;         // split K: fp32 sums [split][M][N] go here (batch 1) and finish_split() makes C of them
+    float* partial = nullptr;         // split K: each part's fp32 sums go here (batch 1), [split][M][N] for launch_gemm_finish() or, in gemm_mid.hip, the accumulators of whole tiles
     int splits = 1;
     int stream_c = 0;                 // gemm256.hip: C is far larger than the L2s, store it with the streaming hint
 };
