@@ -122,7 +122,9 @@ int mhip_bias_gelu_erf(void* stream, const void* x, const void* bias, void* y, i
  * op(A) is [M,K] (stored [K,M] when trans_a), op(B) is [K,N] (stored [N,K]
  * when trans_b); strides are in elements between consecutive batch matrices
  * (0 broadcasts an operand).  bias (length N, same dtype) may be NULL.
- * fp32 accumulate, one rounding at the store.  dtype: BF16, F16, F32; also F64 (f64
+ * fp32 accumulate, one rounding at the store.  The order in which a row's products are added, and with it the
+ * last bits, is the same for any number of rows from 193 on while K is below 4096; with fewer rows or a longer K it
+ * may change with M and batch.  dtype: BF16, F16, F32; also F64 (f64
  * accumulate) and I32 / I64 (wrap-around), those three without activation.
  * Replaces the kernel_matmul family and kernel_matmul_bias_act
  * (Compiler/CodeGenerator.swift:3155-4068, 4797-4850); M/K/N/batch are what
@@ -158,12 +160,15 @@ int mhip_gemm_ws(void* stream, const void* a, const void* b, const void* bias, c
 /* O = softmax(scale * Q K^T + mask, causal) V.
  * Q,O [B,H,Sq,D]; K,V [B,H,Skv,D]; mask NULL or additive [B,H,Sq,Skv] with
  * batch/head strides `mask_stride_b`, `mask_stride_h` in elements (0 = broadcast).
- * Causal rule: key position > query position is masked; a row with no
- * unmasked key yields zeros.  fp32 softmax state and accumulation.
+ * Causal rule: key position > query position is masked; a row whose keys are all masked
+ * with -inf yields zeros, one whose keys all have the type's lowest number as mask their mean.
+ * fp32 softmax state and accumulation.  For up to sixteen queries without the causal rule and for F32 the last bits of
+ * a row may change with B * H, which decides over how many parts its keys are dealt.
  * Replaces FlashAttentionTiledKernel (Metal/Kernels/FlashAttentionKernel.swift:462-671)
  * launched from MetalExecutor.executeFlashAttentionDirect
- * (Runtime/MetalExecutor.swift:502-564). dtype: BF16, F16, F32. D in {64, 128}
- * for the MFMA path; other D up to 256 take a scalar path. */
+ * (Runtime/MetalExecutor.swift:502-564). dtype: BF16, F16, F32.  On the
+ * matrix cores: 16-bit D 128 and multiples of 8 below, F32 D 32, 64, 96, 128; other D up to 256 and
+ * unaligned tensors take a scalar path. */
 int mhip_flash_attention(void* stream, const void* q, const void* k, const void* v,
                          const void* mask, void* o, int64_t B, int64_t H, int64_t Sq, int64_t Skv,
                          int64_t D, float scale, int is_causal, int64_t mask_stride_b,

@@ -206,7 +206,7 @@ bool large_tiles(int64_t M, int64_t N, int64_t batch) {
 }
 
 // Parts of K: up to two workgroups per compute unit, each with at least 512 k.  As in gemm_mid.hip a sum is
-// left in one piece from 193 rows on unless K is 4096 or more, so that a batch does not change its sequences' results.
+// left in one piece from 193 rows on unless K is 4096 or more: in that range more rows do not change a row's bits.
 int any_splits(int64_t M, int64_t N, int64_t K, int64_t batch) {
     if (batch != 1 || (M > 192 && K < 4096) || large_tiles(M, N, batch)) return 1;
     const int64_t room = 512 / (((M + 63) / 64) * ((N + 63) / 64)), most = K / 512;

@@ -350,9 +350,11 @@ float form_cost(const Form& f, int64_t M, int64_t N, int64_t K, int64_t batch, i
     return t;
 }
 
-// Smallest estimate.  Two groups of waves and a split K add a sum up in parts.  A batch of sequences must not
-// change a sequence's result, so from 193 rows on such sums are left in the order of the large tiles, unless K
-// is so long (4096) that splitting it is worth a factor.  K goes to a workspace in parts only for a clear gain.
+// Smallest estimate.  Two groups of waves and a split K add a sum up in parts, and how many depends on M: the last
+// bits of a row may then change with the rows beside it.  That is so up to 192 rows and from K 4096 on, where the parts
+// are worth a factor; in between every sum keeps the order of the large tiles, and a sequence its bits in any batch
+// (gemm_skinny.hip, gemm_any.hip and gemm_f32.hip have the same limits).  K goes to a workspace in parts only for a
+// clear gain.
 MidPlan plan_mid(int64_t M, int64_t N, int64_t K, int64_t batch, bool ring_ok, bool may_split) {
     MidPlan best;
     float t_best = 1e30f;

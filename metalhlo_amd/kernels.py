@@ -88,7 +88,8 @@ def matmul(a, b, bias=None, activation: str = "none", trans_a: bool = False,
            trans_b: bool = False, out: Optional[torch.Tensor] = None,
            residual: Optional[torch.Tensor] = None):
     """act(op(a) @ op(b) + bias) (+ residual, which has the result's shape and may be `out`);
-    leading dims of `a` are batch dims when `b` is batched too, otherwise they fold into M."""
+    leading dims of `a` are batch dims when `b` is batched too, otherwise they fold into M.  Up to 192 rows,
+    and from K 4096 on, the last bits of a row may depend on how many rows there are."""
     return (_native or _host()).matmul(a, b, bias, ACTIVATION_CODE[activation], trans_a, trans_b, out, residual)
 
 
@@ -97,7 +98,8 @@ def flash_attention(q, k, v, scale: Optional[float] = None, is_causal: bool = Fa
     """softmax(scale * q k^T + mask, causal) v for [B,H,S,D] tensors.
     Default scale 1/sqrt(D) (FlashAttentionKernel.swift:55).  q, k, v (and `out`, when given)
     may be views with arbitrary batch / head / row strides as long as the last axis is
-    contiguous, e.g. slices of a fused QKV projection; packed tensors take the plain entry."""
+    contiguous, e.g. slices of a fused QKV projection; packed tensors take the plain entry.  The last bits of a
+    row may depend on B * H for fp32 and for up to 16 queries without the causal rule."""
     return (_native or _host()).flash_attention(q, k, v, scale, is_causal, mask, out)
 
 

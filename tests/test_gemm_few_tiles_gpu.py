@@ -103,3 +103,16 @@ def test_both_sides_of_the_split_lines(M, line, tb, dtype):
     assert _lib.load().mhip_gemm_workspace(M, 264, line - 8, 1, 0, int(tb), code) == 0
     for K in (line - 8, line):
         _check(M, 264, K, dtype, False, tb, residual=True)
+
+
+@pytest.mark.parametrize("N,K,dtype", [(768, 768, torch.bfloat16), (2304, 768, torch.float16), (768, 3072, torch.bfloat16), (768, 4088, torch.bfloat16), (770, 771, torch.bfloat16),
+                                       (768, 3072, torch.float32), (2304, 770, torch.float32)], ids=str)
+@pytest.mark.parametrize("tb", [False, True], ids=["nn", "nt"])
+def test_rows_of_a_batch_keep_their_bits(N, K, tb, dtype):
+    """From 193 rows on, and K below 4096, the kernels add a row's products in one order: more rows beside it change nothing."""
+    from metalhlo_amd import kernels
+    rng = np.random.default_rng(K)
+    a, b = to_dev(rng.standard_normal((3000, K)), dtype), to_dev(rng.standard_normal((N, K) if tb else (K, N)), dtype)
+    want = kernels.matmul(a[:193].contiguous(), b, trans_b=tb)
+    for M in (256, 1000, 3000):
+        assert torch.equal(kernels.matmul(a[:M].contiguous(), b, trans_b=tb)[:193], want), M
