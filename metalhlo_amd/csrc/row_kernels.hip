@@ -485,7 +485,8 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT) void row_any_kernel(const T* _
         if (i < ph.nvec) raw[v] = load16_stream(xr + ph.head + i * E);
     }
     float ev = ei >= 0 ? Elem<T>::to_f32(xr[ei]) : 0.f;
-    const float inv_cols = 1.f / (float)cols;
+    // (divided, not multiplied by 1 / cols: a row of one large value then has exactly that mean and no variance)
+    const float n = (float)cols;
     float scale, shift = 0.f, unit = 1.f;          // y = f(x) * scale (+ shift)
     if (OP == kSoftmax) {
         float m = ei >= 0 ? ev : -INFINITY;
@@ -515,7 +516,7 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT) void row_any_kernel(const T* _
         float s = ev;
 #pragma unroll
         for (int v = 0; v < NV; v++) s = VecSum<T>::sum(raw[v], s);
-        const float mean = row_reduce<NT, false>(s, red[0]) * inv_cols;
+        const float mean = row_reduce<NT, false>(s, red[0]) / n;
         float q = ei >= 0 ? (ev - mean) * (ev - mean) : 0.f;
 #pragma unroll
         for (int v = 0; v < NV; v++)
@@ -526,13 +527,13 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT) void row_any_kernel(const T* _
                     q = fmaf(d, d, q);
                 }
             }
-        scale = 1.f / sqrtf(row_reduce<NT, false>(q, red[1]) * inv_cols + eps);
+        scale = 1.f / sqrtf(row_reduce<NT, false>(q, red[1]) / n + eps);
         shift = mean;
     } else {
         float q = ev * ev;
 #pragma unroll
         for (int v = 0; v < NV; v++) q = VecSum<T>::sumsq(raw[v], q);
-        scale = 1.f / sqrtf(row_reduce<NT, false>(q, red[0]) * inv_cols + eps);
+        scale = 1.f / sqrtf(row_reduce<NT, false>(q, red[0]) / n + eps);
     }
     auto value = [&](float f, float g, float b) {
         if (OP == kSoftmax) return (k16 ? __builtin_amdgcn_exp2f(fmaf(f, unit, -shift)) : f) * scale;

@@ -80,3 +80,14 @@ def test_softmax_at_the_ends_of_the_type(cols, dtype):
         got = as_f64(kernels.softmax(t))
         bad = ~(np.abs(got - e) <= ((cols + 300) * 2.0 ** -24 + ulp) * e + tiny)
         assert not bad.any(), (start, x64[bad][:4], got[bad][:4], e[bad][:4])
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: NAME[d])
+@pytest.mark.parametrize("cols", [3, 7, 513, 1025, 3001, 16391, 50257])
+def test_layer_norm_of_equal_elements(cols, dtype):
+    """Rows of one large value: its multiples are exact in fp32, so the mean is the value, the variance zero and the result beta."""
+    from metalhlo_amd import kernels
+    beta = to_dev(np.random.default_rng(cols).standard_normal(cols), dtype)
+    x = torch.tensor([12288.0, -49152.0, 1.5], dtype=dtype, device="cuda").repeat_interleave(cols).view(3, cols)
+    got = kernels.layer_norm(x, torch.full((cols,), 2.0, dtype=dtype, device="cuda"), beta)
+    assert torch.equal(got, beta.expand(3, cols))
