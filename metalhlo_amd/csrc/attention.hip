@@ -17,10 +17,11 @@
 // skip the matrix steps of whole blocks of 32 d that do not exist.  Their probabilities go through the second product
 // with all of their fp32 bits, as three bf16 parts; f16 values as two bf16 parts, which holds them exactly too.
 //
-// On B4 H12 S1000 causal against the scalar path: bf16 D 96 729 -> 35.6 us, D 32 346 -> 20.6; f16 D 96 52.3, D 32 26.6
-// (two products more per part, and V split in registers).  Share of the results that are not the number nearest to
-// the 64-bit one, scalar path / here, D 96: bf16 0.0003 / 0.0002, f16 0.0027 / 0.0016; with two parts of the
-// weights bf16 was at 0.0023.
+// On B4 H12 S1000 causal against the scalar path: bf16 D 96 729 -> 34.3 us, D 32 346 -> 20.2; f16 D 96 51.8, D 32 25.7
+// (two products per part, and V split in registers).  Parts are cut off, not rounded: a conversion to bf16 pairs costs
+// as much as four simple instructions (35.6 and 20.6 us with it), and what is left is exact either way.  Share of the
+// results that are not the number nearest to the 64-bit one, scalar path / here, D 96: bf16 0.0003 / 0.0002, f16 0.0027 /
+// 0.0016; with two parts of the weights bf16 was at 0.0023.
 //
 // Everything else (unaligned tensors, larger heads) takes a wave-per-query scalar path.
 #include <type_traits>
@@ -359,10 +360,10 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(FaArgs a) {
 #pragma unroll
                         for (int e = 0; e < 4; e++) {
                             float &x = sv[8 * u + 2 * e], &y = sv[8 * u + 2 * e + 1];
-                            const uint32_t w = Mfma32A<bf16_t>::pack2(x, y);
-                            p[part][e] = w;
-                            x -= __builtin_bit_cast(float, w << 16);
-                            y -= __builtin_bit_cast(float, w & 0xFFFF0000u);
+                            const uint32_t xb = __builtin_bit_cast(uint32_t, x), yb = __builtin_bit_cast(uint32_t, y);
+                            p[part][e] = __builtin_amdgcn_perm(yb, xb, 0x07060302u);
+                            x -= __builtin_bit_cast(float, xb & 0xFFFF0000u);
+                            y -= __builtin_bit_cast(float, yb & 0xFFFF0000u);
                         }
                     u32x4 vf[ND], vl[ND];
 #pragma unroll
