@@ -121,7 +121,7 @@ class GPT2:
     def capture(self, ids: torch.Tensor) -> "GraphedForward":
         """Records one forward pass for ids of this shape into a HIP graph.  Every launch
         of the pass goes to the stream handed to the kernel library, so the whole
-        pipeline (about 135 launches) replays with one submission instead of one host
+        pipeline (about 100 launches) replays with one submission instead of one host
         call per kernel."""
         static_ids = ids.clone()
         side = torch.cuda.Stream()

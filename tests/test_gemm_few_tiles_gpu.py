@@ -116,3 +116,37 @@ def test_rows_of_a_batch_keep_their_bits(N, K, tb, dtype):
     want = kernels.matmul(a[:193].contiguous(), b, trans_b=tb)
     for M in (256, 1000, 3000):
         assert torch.equal(kernels.matmul(a[:M].contiguous(), b, trans_b=tb)[:193], want), M
+
+
+def test_workspaces_under_capture_and_on_a_side_stream():
+    """Split products and a split decode step whose workspaces are allocated per call: recorded into one graph and replayed
+    with new inputs, with eager calls of the same kernels between the replays, and run on another stream behind a long
+    product there; every result is the eager one bit for bit."""
+    from metalhlo_amd import kernels
+    rng = np.random.default_rng(4)
+    t = lambda *shape: to_dev(rng.standard_normal(shape), torch.bfloat16)  # noqa: E731
+    w, x, dy, k, v = t(4096, 512), t(4, 4096), t(4096, 512), t(2, 4, 2100, 64), t(2, 4, 2100, 64)
+
+    def step(a, q):
+        return (kernels.matmul(a, w), kernels.flash_attention(q, k, v), kernels.matmul(dy, w, trans_a=True, activation="relu"), kernels.matmul(a * 2, dy))
+    a, q = x.clone(), t(2, 4, 1, 64)
+    step(a, q)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step(a, q)
+    for i in range(4):
+        na, nq = t(4, 4096), t(2, 4, 1, 64)
+        a.copy_(na)
+        q.copy_(nq)
+        graph.replay()
+        want = step(na, nq)
+        step(nq.new_ones(4, 4096), nq)
+        assert all(torch.equal(o, e) for o, e in zip(out, want)), i
+    big, side = t(8192, 4096), torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        late = kernels.matmul(big, t(4096, 4096))[:4].contiguous()
+        got = step(late, nq)
+    torch.cuda.current_stream().wait_stream(side)
+    assert all(torch.equal(o, e) for o, e in zip(got, step(late, nq)))
