@@ -1,6 +1,6 @@
 """CPU oracle for the fused transformer kernels (TEST INFRASTRUCTURE ONLY).
 
-This module is a checker. Only tests, the smoke entry and the benchmark's
+Only tests, the smoke entry and the benchmark's
 ``cpu_baseline`` leg may import it; no product code path does.
 
 Every function restates, in NumPy float64 on the *given* (already rounded)

@@ -176,7 +176,7 @@ def test_gather_forms(form, types, sess):
 
 
 def test_spec_gather_reproduces_the_reference_cases():
-    """Pins the checker above: it reproduces the two gather cases of the reference's file."""
+    """Pins the restatement above: it reproduces the two gather cases of the reference's file."""
     seen = 0
     for case in CASES:
         if "gather.mlir" not in case["src"]:
