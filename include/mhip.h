@@ -155,6 +155,27 @@ int mhip_gemm_ws(void* stream, const void* a, const void* b, const void* bias, c
                  int64_t stride_c, int trans_a, int trans_b, int activation, int dtype, void* workspace,
                  int64_t workspace_bytes);
 
+/* A linear layer of up to 192 rows whose parameters are fp32: c = act(x . round(w) + round(bias)) (+ residual), x, residual
+ * and c of `dtype` (BF16 or F16), every parameter rounded to it at use: mhip_convert and mhip_gemm_residual in one launch.
+ * w is [K,N], or [N,K] with trans_b; bias and residual may be NULL.  All pointers are 16-byte aligned.
+ * mhip_linear_w32_ok says whether a problem is served (N and K multiples of 8).  The last bits of a row may change with the
+ * number of rows.
+ * sums (else NULL, with parts = 1): instead of c the fp32 products of `parts` shares of K, [parts][M][N], for
+ * mhip_finish_norm; mhip_linear_w32_parts gives a good number, up to 8.
+ * ahead: up to two weight matrices [K,N] that the next calls on the stream read; workgroups of their own fetch them into the
+ * caches (a hint: no result depends on it; matrices of more than 2^23 elements are passed over). */
+typedef struct { const float* w; int64_t N, K; } mhip_weights;
+int mhip_linear_w32_ok(int64_t M, int64_t N, int64_t K, int dtype);
+int mhip_linear_w32_parts(int64_t M, int64_t N, int64_t K);
+int mhip_linear_w32(void* stream, const void* x, const float* w, const float* bias, const void* residual, void* c, int64_t M,
+                    int64_t N, int64_t K, int trans_b, int activation, int dtype, float* sums, int parts, int n_ahead,
+                    const mhip_weights* ahead);
+/* c = round(sum of sums[parts][M][N] + round(bias)) + residual, or with parts = 0 (sums NULL) the residual itself, and
+ * h = LayerNorm(c; gamma, beta, eps) over its rows.  c may be NULL; bias and residual may be NULL where there are parts.
+ * Parameters fp32, the rest of `dtype` (BF16 or F16); N a multiple of 8 up to 4096; 16-byte aligned pointers. */
+int mhip_finish_norm(void* stream, const float* sums, int parts, const float* bias, const void* residual, void* c,
+                     const float* gamma, const float* beta, float eps, void* h, int64_t M, int64_t N, int dtype);
+
 /* Attention -------------------------------------------------------------- */
 
 /* O = softmax(scale * Q K^T + mask, causal) V.

@@ -1,0 +1,511 @@
+// Linear layers of a few tokens whose parameters are held in fp32:
+//   C = act(x . round(W) + round(bias)),  and behind them  x' = round(sum + round(bias)) + x,  h = LayerNorm(x'),
+// tensors in a 16-bit type, every parameter rounded to that type where it is used.  The results are those of
+// converting the parameters first and launching dot_general, add and LayerNorm one after the other (up to the order of the
+// fp32 sums), without the conversion's pass over all weights (GPT-2-small: 117 us for 124 M parameters).
+//
+// What bounds it: launches (1.6 us each when they depend on one another) and latencies.  A cold matrix answers after about
+// 4 us, address translation included, and a compute unit takes no more than about 30 bytes a nanosecond from memory,
+// 75 from its L2: [4,768] x [768,768] 5.4 us with W from memory, 4.1 from the memory-side cache, 2.7 from the L2s.  Hence
+//   * as in gemm_skinny.hip a workgroup owns a strip of columns, its waves split K, W goes to the operand registers
+//     without a stop in LDS and all of it is in flight before anything else;
+//   * a layer whose result is added to the residual splits K over the grid too ([37,3072] x [3072,768] 19.5 us in 48
+//     workgroups, 7.4 in 192), and the launch that adds the parts up forms the next LayerNorm, whose rows it holds anyway;
+//   * workgroups in front of a launch fetch weights that the next launches will read into the L2 of the XCD that
+//     will want them (fetch_ahead): [37,768] x [768,2304] 7.3 -> 5.0 us, those workgroups included.
+// Workgroups of one XCD take neighbouring strips, so a 128-byte line of W that two strips share is fetched once.
+#include <initializer_list>
+#include <mutex>
+
+#include "gemm_common.h"
+
+namespace mhip {
+namespace {
+
+constexpr int kAhead = 2, kAheadLoads = 16, kWaves = 8;
+
+struct Band { const float* w; int N, K, cols, wgs; uint32_t magic; };      // cols: what the strips of one XCD will cover; wgs: per XCD
+
+struct LinearArgs {
+    const void* x;
+    const float *gamma, *beta;        // finish_norm_kernel only; beta may be NULL
+    float eps;
+    const float* w;
+    const float* bias;                // may be NULL
+    const void* residual;             // may be NULL
+    void* c;
+    float* sums;                      // instead of c: fp32 sums [splits][M][N]
+    int M, N, K, act, splits;
+    int strips, per_xcd, blocks, first;      // first: workgroups in front of the product's
+    Band ahead[kAhead];
+};
+
+template <typename T> struct Tile16;
+template <> struct Tile16<bf16_t> {
+    __device__ static f32x4 run(u32x4 b, u32x4 a, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b), __builtin_bit_cast(bf16x8, a), c, 0, 0, 0);
+    }
+};
+template <> struct Tile16<f16_t> {
+    __device__ static f32x4 run(u32x4 b, u32x4 a, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, b), __builtin_bit_cast(f16x8, a), c, 0, 0, 0);
+    }
+};
+template <typename T>
+__device__ __forceinline__ uint32_t round_pair(float lo, float hi) {
+    typedef T pair __attribute__((ext_vector_type(2)));
+    const pair p = {Elem<T>::from_f32(lo), Elem<T>::from_f32(hi)};
+    return __builtin_bit_cast(uint32_t, p);
+}
+__device__ inline __amdgpu_buffer_rsrc_t lin_rsrc(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+}
+template <typename T>
+__device__ __forceinline__ float rounded(float v) { return Elem<T>::to_f32(Elem<T>::from_f32(v)); }
+// Workgroup `id` of those in front: kAheadLoads 16-byte pieces per thread of the columns that the strips of its XCD cover.
+__device__ __forceinline__ void fetch_ahead(const LinearArgs& g, int id) {
+    const int xcd = id % kXcds;
+    int j = id / kXcds, r = 0;
+    if (j >= g.ahead[0].wgs) { j -= g.ahead[0].wgs; r = 1; }
+    const float* w = r ? g.ahead[1].w : g.ahead[0].w;
+    const int N = r ? g.ahead[1].N : g.ahead[0].N, K = r ? g.ahead[1].K : g.ahead[0].K, cols = r ? g.ahead[1].cols : g.ahead[0].cols;
+    const uint32_t magic = r ? g.ahead[1].magic : g.ahead[0].magic, per_row = (uint32_t)cols / 4;
+    const __amdgpu_buffer_rsrc_t rw = lin_rsrc(w, (uint32_t)((int64_t)N * K * 4));
+    const uint32_t at = (uint32_t)j * (64 * kWaves * kAheadLoads) + threadIdx.x;
+    u32x4 v[kAheadLoads];
+#pragma unroll
+    for (int i = 0; i < kAheadLoads; i++) {
+        const uint32_t p = at + i * 64 * kWaves, row = __umulhi(p, magic), col = xcd * cols + (p - row * per_row) * 4;
+        v[i] = __builtin_amdgcn_raw_buffer_load_b128(rw, (int)row < K && (int)col < N ? (row * (uint32_t)N + col) * 4 : kOob, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < kAheadLoads; i++) asm volatile("" ::"v"(v[i]));
+}
+
+// TB: W stored [N, K].  NF = operands (groups of 16 columns) per strip, MT = groups of 16 rows, U = steps of 32 k that a
+// wave holds at once; LOOP: it has more of them and loads a block ahead.
+template <typename T, bool TB, bool LOOP, int NF, int MT, int U>
+__global__ __launch_bounds__(64 * kWaves, LOOP ? 2 : 4) void linear_w32_kernel(LinearArgs g) {
+    constexpr int KS = 32, NS = 16 * NF;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    if ((int)blockIdx.x < g.first) {
+        fetch_ahead(g, blockIdx.x);
+        return;
+    }
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 15, lg = lane >> 4;
+    const int id = (int)blockIdx.x - g.first, xcd = id % kXcds;
+    int local = id / kXcds;
+    const int m0 = local % g.blocks * (16 * MT);
+    local /= g.blocks;
+    const int split = local % g.splits, strip = xcd * g.per_xcd + local / g.splits, n0 = strip * NS;
+    if (strip >= g.strips) return;
+    const __amdgpu_buffer_rsrc_t rx = lin_rsrc(g.x, (uint32_t)((int64_t)g.M * g.K * 2));
+    const __amdgpu_buffer_rsrc_t rw = lin_rsrc(g.w, (uint32_t)((int64_t)g.N * g.K * 4));
+
+    // ---- this wave's share of the k steps
+    const int all = (g.K + KS - 1) / KS, part_steps = (all + g.splits - 1) / g.splits, p0 = split * part_steps, p1 = min(all, p0 + part_steps);
+    const int per = (part_steps + kWaves - 1) / kWaves, s0 = p0 + wave * per, s1 = min(p1, s0 + per);
+    struct Block {
+        f32x4 wt[TB ? U : 1][TB ? NF : 1][2];                // W stored [N, K]: eight k of a column
+        float wn[TB ? 1 : U][TB ? 1 : 8][NF];                // W stored [K, N]: NF columns of eight k
+        u32x4 a[U][MT];
+    };
+    auto load = [&](Block& b, int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int k = (s + u) * KS + lg * 8;
+            const bool live = s + u < s1 && k < g.K;
+            if (TB) {
+#pragma unroll
+                for (int f = 0; f < NF; f++) {
+                    const int n = n0 + 16 * f + li;
+                    const uint32_t off = live && n < g.N ? (uint32_t)(((int64_t)n * g.K + k) * 4) : kOob;
+#pragma unroll
+                    for (int h = 0; h < 2; h++) b.wt[TB ? u : 0][TB ? f : 0][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, off + 16 * h, 0, 0));
+                }
+            } else {
+                const int n = n0 + NF * li;
+                const uint32_t off = live && n < g.N ? (uint32_t)(((int64_t)k * g.N + n) * 4) : kOob;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const uint32_t o = off + (uint32_t)(j * g.N * 4);
+                    if (NF == 1) b.wn[TB ? 0 : u][TB ? 0 : j][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rw, o, 0, 0));
+                    else {
+                        const u32x2 t = __builtin_amdgcn_raw_buffer_load_b64(rw, o, 0, 0);
+                        b.wn[TB ? 0 : u][TB ? 0 : j][0] = __builtin_bit_cast(float, t.x);
+                        b.wn[TB ? 0 : u][TB ? 0 : j][NF - 1] = __builtin_bit_cast(float, t.y);
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+                const int k = (s + u) * KS + lg * 8, m = m0 + mt * 16 + li;
+                b.a[u][mt] = __builtin_amdgcn_raw_buffer_load_b128(rx, s + u < s1 && k < g.K && m < g.M ? (uint32_t)((m * g.K + k) * 2) : kOob, 0, 0);
+            }
+    };
+    Block cur;
+    load(cur, s0);
+
+    // ---- the epilogue's thread (wave = mt, li, lg) finishes row li of group mt: columns NF 4 lg .. + 4 NF - 1 of the strip (W
+    // stored [K, N]) or four from 4 lg on of each operand (stored [N, K])
+    const int fm = m0 + wave * 16 + li;
+    const bool finisher = wave < MT && fm < g.M;
+    auto column = [&](int q) { return TB ? n0 + 16 * q + 4 * lg : n0 + NF * 4 * lg + 4 * q; };
+    f32x4 bias[NF];
+    u32x2 res[NF];
+#pragma unroll
+    for (int q = 0; q < NF; q++) {
+        bias[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+        res[q] = u32x2{0, 0};
+        if (finisher && column(q) < g.N) {
+            if (g.bias) bias[q] = *reinterpret_cast<const f32x4*>(g.bias + column(q));
+            if (g.residual) res[q] = *reinterpret_cast<const u32x2*>(static_cast<const T*>(g.residual) + (int64_t)fm * g.N + column(q));
+        }
+    }
+
+    f32x4 acc[NF][MT];
+#pragma unroll
+    for (int f = 0; f < NF; f++)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) acc[f][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](const Block& b, int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (s + u >= s1) break;
+#pragma unroll
+            for (int f = 0; f < NF; f++) {
+                u32x4 w;
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    w[j] = TB ? round_pair<T>(b.wt[TB ? u : 0][TB ? f : 0][j / 2][j % 2 * 2], b.wt[TB ? u : 0][TB ? f : 0][j / 2][j % 2 * 2 + 1])
+                              : round_pair<T>(b.wn[TB ? 0 : u][TB ? 0 : 2 * j][f], b.wn[TB ? 0 : u][TB ? 0 : 2 * j + 1][f]);
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++) acc[f][mt] = Tile16<T>::run(w, b.a[u][mt], acc[f][mt]);
+            }
+        }
+    };
+    if (LOOP) {
+        for (int s = s0; s < s1; s += U) {
+            Block nxt;
+            if (s + U < s1) load(nxt, s + U);
+            multiply(cur, s);
+            if (s + U < s1) cur = nxt;
+        }
+    } else multiply(cur, s0);
+
+    // ---- the waves' partial sums, in the accumulators' own layout: lane (li, lg) holds row 16 mt + li and, in its four
+    // registers, operand rows 4 lg .. 4 lg + 3
+    f32x4* part = reinterpret_cast<f32x4*>(smem);
+#pragma unroll
+    for (int f = 0; f < NF; f++)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) part[((wave * NF + f) * MT + mt) * 64 + lane] = acc[f][mt];
+    __syncthreads();
+    if (wave >= MT) return;
+    f32x4 sum[NF];
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+        sum[f] = part[(f * MT + wave) * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < kWaves; w++) sum[f] += part[((w * NF + f) * MT + wave) * 64 + lane];
+    }
+    if (!finisher) return;
+    // place 4 q + e of the thread's columns
+    auto value = [&](int q, int e) { return TB ? sum[q][e] : sum[(4 * q + e) % NF][(4 * q + e) / NF]; };
+    if (g.sums) {
+        float* c = g.sums + ((int64_t)split * g.M + fm) * g.N;
+#pragma unroll
+        for (int q = 0; q < NF; q++)
+            if (column(q) < g.N) *reinterpret_cast<f32x4*>(c + column(q)) = f32x4{value(q, 0), value(q, 1), value(q, 2), value(q, 3)};
+        return;
+    }
+    T* c = static_cast<T*>(g.c) + (int64_t)fm * g.N;
+    dispatch_act(g.act, [&](auto act_tag) {
+        constexpr int ACT = decltype(act_tag)::value;
+#pragma unroll
+        for (int q = 0; q < NF; q++) {
+            Pack4<T> o, r = __builtin_bit_cast(Pack4<T>, res[q]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                o.v[e] = Elem<T>::from_f32(apply_act_c<ACT>(value(q, e) + rounded<T>(bias[q][e])));
+                // (second rounding on purpose: the same result as a separate add over the stored C)
+                if (g.residual) o.v[e] = Elem<T>::from_f32(Elem<T>::to_f32(o.v[e]) + Elem<T>::to_f32(r.v[e]));
+            }
+            if (column(q) < g.N) *reinterpret_cast<u32x2*>(c + column(q)) = __builtin_bit_cast(u32x2, o);
+        }
+    });
+}
+
+// W stored [N, K] where a wave holds its share of the k steps at once (a tied output head: 50304 columns of K 768).  The grid
+// is resident and walks the strips: x stays in registers, the next strip's W is on its way while this one is
+// multiplied and added up, through two sets of partial sums with one barrier per strip.  One strip per workgroup spends as
+// much on x as on W: [37,768] x [50304,768]^T 53 us against 36.7, [128,768] 106 against 58.
+template <typename T, int MT, int U>
+__global__ __launch_bounds__(64 * kWaves, MT < 2 ? 4 : 2) void linear_w32_stream_kernel(LinearArgs g) {
+    constexpr int KS = 32;
+    __shared__ f32x4 part[2][kWaves][MT][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 15, lg = lane >> 4;
+    const int m0 = (int)blockIdx.y * (16 * MT);
+    const __amdgpu_buffer_rsrc_t rx = lin_rsrc(g.x, (uint32_t)((int64_t)g.M * g.K * 2));
+    const __amdgpu_buffer_rsrc_t rw = lin_rsrc(g.w, (uint32_t)((int64_t)g.N * g.K * 4));
+    const int all = (g.K + KS - 1) / KS, per = (all + kWaves - 1) / kWaves, s0 = wave * per, s1 = min(all, s0 + per);
+    u32x4 a[U][MT];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            const int k = (s0 + u) * KS + lg * 8, m = m0 + mt * 16 + li;
+            a[u][mt] = __builtin_amdgcn_raw_buffer_load_b128(rx, s0 + u < s1 && k < g.K && m < g.M ? (uint32_t)((m * g.K + k) * 2) : kOob, 0, 0);
+        }
+    f32x4 w[2][U][2];
+    auto load = [&](f32x4(&v)[U][2], int strip) __attribute__((always_inline)) {
+        const int n = strip * 16 + li;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int k = (s0 + u) * KS + lg * 8;
+            const uint32_t off = s0 + u < s1 && k < g.K && n < g.N ? (uint32_t)((n * g.K + k) * 4) : kOob;
+#pragma unroll
+            for (int h = 0; h < 2; h++) v[u][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, off + 16 * h, 0, 0));
+        }
+    };
+    const int fm = m0 + wave * 16 + li;
+    const bool finisher = wave < MT && fm < g.M;
+    T* c = static_cast<T*>(g.c) + (int64_t)fm * g.N;
+    const T* res = static_cast<const T*>(g.residual) + (int64_t)fm * g.N;
+    auto strip_of = [&](const f32x4(&v)[U][2], int strip, int set) __attribute__((always_inline)) {
+        f32x4 acc[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const u32x4 b = {round_pair<T>(v[u][0][0], v[u][0][1]), round_pair<T>(v[u][0][2], v[u][0][3]),
+                             round_pair<T>(v[u][1][0], v[u][1][1]), round_pair<T>(v[u][1][2], v[u][1][3])};
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) acc[mt] = Tile16<T>::run(b, a[u][mt], acc[mt]);
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) part[set][wave][mt][lane] = acc[mt];
+        // (a barrier that leaves the loads of W in flight; the set is written again behind the next strip's barrier, which
+        // a wave reaches when it has read this one)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (wave >= MT) return;
+        f32x4 sum = part[set][0][wave][lane];
+#pragma unroll
+        for (int i = 1; i < kWaves; i++) sum += part[set][i][wave][lane];
+        const int n = strip * 16 + 4 * lg;
+        if (!finisher || n >= g.N) return;
+        f32x4 bias = {0.f, 0.f, 0.f, 0.f};
+        if (g.bias) bias = *reinterpret_cast<const f32x4*>(g.bias + n);
+        Pack4<T> r = {};
+        if (g.residual) r = *reinterpret_cast<const Pack4<T>*>(res + n);
+        dispatch_act(g.act, [&](auto act_tag) {
+            constexpr int ACT = decltype(act_tag)::value;
+            Pack4<T> o;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                o.v[e] = Elem<T>::from_f32(apply_act_c<ACT>(sum[e] + rounded<T>(bias[e])));
+                if (g.residual) o.v[e] = Elem<T>::from_f32(Elem<T>::to_f32(o.v[e]) + Elem<T>::to_f32(r.v[e]));
+            }
+            *reinterpret_cast<Pack4<T>*>(c + n) = o;
+        });
+    };
+    const int stride = (int)gridDim.x;
+    int strip = blockIdx.x;
+    if (strip >= g.strips) return;
+    load(w[0], strip);
+    for (;;) {
+        if (strip + stride < g.strips) load(w[1], strip + stride);
+        strip_of(w[0], strip, 0);
+        strip += stride;
+        if (strip >= g.strips) break;
+        if (strip + stride < g.strips) load(w[0], strip + stride);
+        strip_of(w[1], strip, 1);
+        strip += stride;
+        if (strip >= g.strips) break;
+    }
+}
+
+// A row per workgroup: x = round(sum of the parts + bias) + residual (or, without parts, the residual itself), stored to c
+// when that is given, and h = LayerNorm(x).  Latency-bound: two memory latencies, two barriers.
+constexpr int kFinishPieces = 4;      // four columns each, 256 threads: N <= 4096
+template <typename T>
+__global__ __launch_bounds__(256) void finish_norm_kernel(LinearArgs g, T* h) {
+    __shared__ float red[2][4];
+    const int64_t row = blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    f32x4 v[kFinishPieces];
+    u32x2 x[kFinishPieces];
+    f32x4 ga[kFinishPieces], be[kFinishPieces];
+    float s = 0.f;
+#pragma unroll
+    for (int p = 0; p < kFinishPieces; p++) {
+        const int n = (p * 256 + (int)threadIdx.x) * 4;
+        v[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+        x[p] = u32x2{0, 0};
+        if (n >= g.N) continue;
+        const int64_t at = row * g.N + n;
+        ga[p] = *reinterpret_cast<const f32x4*>(g.gamma + n);
+        be[p] = g.beta ? *reinterpret_cast<const f32x4*>(g.beta + n) : f32x4{0.f, 0.f, 0.f, 0.f};
+        if (g.residual) x[p] = *reinterpret_cast<const u32x2*>(static_cast<const T*>(g.residual) + at);
+        if (g.splits) {
+            f32x4 b = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (g.bias) b = *reinterpret_cast<const f32x4*>(g.bias + n);
+#pragma unroll 8
+            for (int i = 0; i < g.splits; i++) v[p] += *reinterpret_cast<const f32x4*>(g.sums + (int64_t)i * g.M * g.N + at);
+            Pack4<T> r = __builtin_bit_cast(Pack4<T>, x[p]), o;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                o.v[e] = Elem<T>::from_f32(v[p][e] + rounded<T>(b[e]));
+                if (g.residual) o.v[e] = Elem<T>::from_f32(Elem<T>::to_f32(o.v[e]) + Elem<T>::to_f32(r.v[e]));
+            }
+            x[p] = __builtin_bit_cast(u32x2, o);
+        }
+        if (g.c) *reinterpret_cast<u32x2*>(static_cast<T*>(g.c) + at) = x[p];
+        const Pack4<T> t = __builtin_bit_cast(Pack4<T>, x[p]);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            v[p][e] = Elem<T>::to_f32(t.v[e]);
+            s += v[p][e];
+        }
+    }
+    auto over_row = [&](float t, int set) {
+        t = wave_sum(t);
+        if (lane == 0) red[set][wave] = t;
+        __syncthreads();
+        return (red[set][0] + red[set][1]) + (red[set][2] + red[set][3]);
+    };
+    const float inv = 1.f / (float)g.N, mean = over_row(s, 0) * inv;
+    float q = 0.f;
+#pragma unroll
+    for (int p = 0; p < kFinishPieces; p++)
+        if ((p * 256 + (int)threadIdx.x) * 4 < g.N)
+#pragma unroll
+            for (int e = 0; e < 4; e++) { v[p][e] -= mean; q = fmaf(v[p][e], v[p][e], q); }
+    const float rstd = 1.f / sqrtf(over_row(q, 1) * inv + g.eps);
+#pragma unroll
+    for (int p = 0; p < kFinishPieces; p++) {
+        const int n = (p * 256 + (int)threadIdx.x) * 4;
+        if (n >= g.N) continue;
+        Pack4<T> o;
+#pragma unroll
+        for (int e = 0; e < 4; e++) o.v[e] = Elem<T>::from_f32(fmaf(v[p][e] * rstd, rounded<T>(ga[p][e]), rounded<T>(be[p][e])));
+        *reinterpret_cast<u32x2*>(h + row * g.N + n) = __builtin_bit_cast(u32x2, o);
+    }
+}
+
+template <typename T, bool TB, bool LOOP, int NF, int MT, int U>
+int launch_one(hipStream_t s, LinearArgs g) {
+    auto kern = linear_w32_kernel<T, TB, LOOP, NF, MT, U>;
+    constexpr int kSums = kWaves * NF * MT * 1024;
+    static_assert(kSums <= 64 * 1024, "more LDS than a launch gets unasked");
+    g.blocks = (g.M + 16 * MT - 1) / (16 * MT);
+    g.strips = (g.N + 16 * NF - 1) / (16 * NF);
+    g.per_xcd = (g.strips + kXcds - 1) / kXcds;
+    g.first = 0;
+    for (Band& a : g.ahead) {
+        a.cols = ((a.N + 15) / 16 + kXcds - 1) / kXcds * 16;
+        const int64_t pieces = (int64_t)a.cols / 4 * a.K, per_wg = 64 * kWaves * kAheadLoads;
+        a.wgs = a.w ? (int)((pieces + per_wg - 1) / per_wg) : 0;
+        a.magic = a.w ? (uint32_t)((((uint64_t)1 << 32) + a.cols / 4 - 1) / (a.cols / 4)) : 0;
+        g.first += kXcds * a.wgs;
+    }
+    const int64_t grid = g.first + (int64_t)kXcds * g.per_xcd * g.blocks * g.splits;
+    if (grid > 0x7FFFFFFFLL) return fail(MHIP_ERR_UNSUPPORTED, "linear_w32: grid too large");
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * kWaves), kSums, s, g);
+    return check_launch("linear_w32");
+}
+
+template <typename T, int MT>
+int launch_rows(hipStream_t s, const LinearArgs& g, bool tb) {
+    const bool loop = ((g.K + 31) / 32 + g.splits - 1) / g.splits > 3 * kWaves;
+    if (tb && !loop && !g.sums) {
+        LinearArgs t = g;
+        t.strips = (g.N + 15) / 16;
+        const int blocks = (g.M + 16 * MT - 1) / (16 * MT), room = (MT < 2 ? 2 : 1) * compute_units() / blocks;
+        hipLaunchKernelGGL((linear_w32_stream_kernel<T, MT, 3>), dim3((unsigned)(t.strips < room ? t.strips : room), (unsigned)blocks), dim3(64 * kWaves), 0, s, t);
+        return check_launch("linear_w32_stream");
+    }
+    if (tb) return launch_one<T, true, true, 1, MT, 3>(s, g);
+    return loop ? launch_one<T, false, true, 1, MT, 3>(s, g) : launch_one<T, false, false, 1, MT, 3>(s, g);
+}
+
+template <typename T>
+int launch_type(hipStream_t s, const LinearArgs& g, bool tb) {
+    // blocks of up to 64 rows, of one size
+    const int blocks = (g.M + 63) / 64;
+    switch (((g.M + blocks - 1) / blocks + 15) / 16) {
+        case 1: return launch_rows<T, 1>(s, g, tb);
+        case 2: return launch_rows<T, 2>(s, g, tb);
+        case 3: return launch_rows<T, 3>(s, g, tb);
+        default: return launch_rows<T, 4>(s, g, tb);
+    }
+}
+
+bool aligned16(std::initializer_list<const void*> ps) {
+    uintptr_t all = 0;
+    for (const void* p : ps) all |= reinterpret_cast<uintptr_t>(p);
+    return (all & 15) == 0;
+}
+
+}  // namespace
+}  // namespace mhip
+
+using namespace mhip;
+
+extern "C" int mhip_linear_w32_ok(int64_t M, int64_t N, int64_t K, int dtype) {
+    if (dtype != MHIP_BF16 && dtype != MHIP_F16) return 0;
+    if (M < 1 || M > 192 || N < 1 || K < 1 || N % 8 != 0 || K % 8 != 0 || N > (1 << 24) || K > (1 << 24)) return 0;
+    return (N + 64) * (K + 64) * 4 < 0x7FFFFFFFLL;
+}
+
+// Parts of K: about 768 k, at most two workgroups per compute unit.
+extern "C" int mhip_linear_w32_parts(int64_t M, int64_t N, int64_t K) {
+    const int64_t tiles = (N + 15) / 16 * ((M + 63) / 64), room = tiles > 0 ? 512 / tiles : 1, want = (K + 384) / 768;
+    const int64_t n = room < want ? room : want;
+    return n < 2 ? 1 : n > 8 ? 8 : (int)n;
+}
+
+extern "C" int mhip_linear_w32(void* stream, const void* x, const float* w, const float* bias, const void* residual, void* c, int64_t M,
+                               int64_t N, int64_t K, int trans_b, int activation, int dtype, float* sums, int parts, int n_ahead,
+                               const mhip_weights* ahead) {
+    if (activation < MHIP_ACT_NONE || activation > MHIP_ACT_GELU_ERF)
+        return fail(MHIP_ERR_INVALID_ARGUMENT, "mhip_linear_w32: unknown activation %d", activation);
+    if (!x || !w || (!c && !sums)) return fail(MHIP_ERR_INVALID_ARGUMENT, "mhip_linear_w32: NULL matrix pointer");
+    if (sums ? (parts < 1 || parts > 8 || c || bias || residual || activation != MHIP_ACT_NONE) : parts != 1)
+        return fail(MHIP_ERR_INVALID_ARGUMENT, "mhip_linear_w32: parts of K come as plain sums, eight at most");
+    if (!mhip_linear_w32_ok(M, N, K, dtype))
+        return fail(MHIP_ERR_UNSUPPORTED, "mhip_linear_w32: [%lld,%lld] x K %lld, dtype %d is not served", (long long)M, (long long)N, (long long)K, dtype);
+    if (!aligned16({x, w, bias, residual, c, sums})) return fail(MHIP_ERR_UNSUPPORTED, "mhip_linear_w32: tensors must be 16-byte aligned");
+    if (n_ahead < 0 || n_ahead > kAhead || (n_ahead > 0 && !ahead)) return fail(MHIP_ERR_INVALID_ARGUMENT, "mhip_linear_w32: up to %d matrices ahead", kAhead);
+    LinearArgs g = {};
+    g.x = x; g.w = w; g.bias = bias; g.residual = residual; g.c = c; g.sums = sums;
+    g.M = (int)M; g.N = (int)N; g.K = (int)K; g.act = activation; g.splits = parts;
+    for (int i = 0; i < n_ahead; i++)
+        if (ahead[i].w && ahead[i].N > 0 && ahead[i].K > 0 && ahead[i].N % 8 == 0 && ahead[i].N <= (1 << 16) && ahead[i].K <= (1 << 16) &&
+            ahead[i].N * ahead[i].K <= (1 << 23) && aligned16({ahead[i].w})) {
+            g.ahead[i].w = ahead[i].w; g.ahead[i].N = (int)ahead[i].N; g.ahead[i].K = (int)ahead[i].K;
+        }
+    return dtype == MHIP_BF16 ? launch_type<bf16_t>(as_stream(stream), g, trans_b != 0) : launch_type<f16_t>(as_stream(stream), g, trans_b != 0);
+}
+
+extern "C" int mhip_finish_norm(void* stream, const float* sums, int parts, const float* bias, const void* residual, void* c,
+                                const float* gamma, const float* beta, float eps, void* h, int64_t M, int64_t N, int dtype) {
+    if (M < 0 || N < 1 || parts < 0 || (parts > 0) != (sums != nullptr) || !gamma || !h || (parts == 0 && !residual))
+        return fail(MHIP_ERR_INVALID_ARGUMENT, "mhip_finish_norm: bad argument");
+    if (M == 0) return MHIP_OK;
+    if ((dtype != MHIP_BF16 && dtype != MHIP_F16) || N % 8 != 0 || N > 1024 * kFinishPieces || M > 0x7FFFFFFF || !aligned16({sums, bias, residual, c, gamma, beta, h}))
+        return fail(MHIP_ERR_UNSUPPORTED, "mhip_finish_norm: rows of %lld, dtype %d", (long long)N, dtype);
+    LinearArgs g = {};
+    g.sums = const_cast<float*>(sums); g.splits = parts; g.bias = bias; g.residual = residual; g.c = c; g.gamma = gamma; g.beta = beta;
+    g.eps = eps; g.M = (int)M; g.N = (int)N;
+    if (dtype == MHIP_BF16) hipLaunchKernelGGL((finish_norm_kernel<bf16_t>), dim3((unsigned)M), dim3(256), 0, as_stream(stream), g, static_cast<bf16_t*>(h));
+    else hipLaunchKernelGGL((finish_norm_kernel<f16_t>), dim3((unsigned)M), dim3(256), 0, as_stream(stream), g, static_cast<f16_t*>(h));
+    return check_launch("finish_norm");
+}

@@ -239,6 +239,81 @@ FUNCTION(matmul) {
     });
 }
 
+const float* f32(const at::Tensor* t) { return t ? t->data_ptr<float>() : nullptr; }
+
+// linear(x, weight, bias, residual, activation code, trans_b, parts, (weights ahead)): parameters in fp32;
+// parts > 0: the fp32 sums of so many shares of K instead
+FUNCTION(linear) {
+    return guarded(n, 8, [&] {
+        const at::Tensor &x = dense(arg[0]), &w = dense(arg[1]);
+        const at::Tensor *bias = optional_dense(arg[2]), *res = optional_dense(arg[3]);
+        const bool tb = truth(arg[5]);
+        const int parts = (int)integer(arg[6]);
+        if (x.dim() != 2 || w.dim() != 2) raise(PyExc_ValueError, "linear needs matrices");
+        const int64_t M = x.size(0), K = x.size(1), N = w.size(tb ? 0 : 1);
+        if (w.size(tb ? 1 : 0) != K) raise(PyExc_ValueError, "contracting sizes differ");
+        for (const at::Tensor* p : {&w, bias})
+            if (p && p->scalar_type() != at::kFloat) raise(PyExc_TypeError, "parameters must be fp32");
+        if (bias && bias->numel() != N) raise(PyExc_ValueError, "bias must be [N]");
+        if (res && (res->numel() != M * N || res->scalar_type() != x.scalar_type())) raise(PyExc_ValueError, "residual must have the result's size and dtype");
+        const int dt = dtype_code(x.scalar_type()), act = (int)integer(arg[4]);
+        at::Tensor c = parts > 0 ? empty({parts, M, N}, at::kFloat, x) : empty({M, N}, x.scalar_type(), x);
+        mhip_weights ahead[2] = {};
+        int n_ahead = 0;
+        if (!PyTuple_Check(arg[7]) || PyTuple_GET_SIZE(arg[7]) > 2) raise(PyExc_ValueError, "ahead must be a tuple of up to two matrices");
+        for (; n_ahead < PyTuple_GET_SIZE(arg[7]); n_ahead++) {
+            const at::Tensor* t = &dense(PyTuple_GET_ITEM(arg[7], n_ahead));
+            if (t->dim() != 2 || t->scalar_type() != at::kFloat) raise(PyExc_TypeError, "weights ahead must be fp32 matrices");
+            ahead[n_ahead] = {t->data_ptr<float>(), t->size(1), t->size(0)};
+        }
+        check([&] { return mhip_linear_w32(stream_of(x), x.data_ptr(), f32(&w), f32(bias), ptr(res),
+                                           parts > 0 ? nullptr : c.data_ptr(), M, N, K, tb, act, dt, parts > 0 ? c.data_ptr<float>() : nullptr,
+                                           parts > 0 ? parts : 1, n_ahead, ahead); });
+        return THPVariable_Wrap(std::move(c));
+    });
+}
+
+// finish_norm(sums or None, bias, residual, gamma, beta, eps) -> (c, LayerNorm(c)); without sums c is the residual
+FUNCTION(finish_norm) {
+    return guarded(n, 6, [&]() -> PyObject* {
+        const at::Tensor *sums = optional_dense(arg[0]), *bias = optional_dense(arg[1]), *beta = optional_dense(arg[4]);
+        const at::Tensor &res = dense(arg[2]), &gamma = dense(arg[3]);
+        const int64_t N = last_size(res), M = N ? res.numel() / N : 0;
+        for (const at::Tensor* p : {sums, bias, &gamma, beta})
+            if (p && p->scalar_type() != at::kFloat) raise(PyExc_TypeError, "sums and parameters must be fp32");
+        if (gamma.numel() != N || (beta && beta->numel() != N) || (bias && bias->numel() != N)) raise(PyExc_ValueError, "parameters must have the row length");
+        if (sums && (sums->dim() != 3 || sums->size(1) != M || sums->size(2) != N)) raise(PyExc_ValueError, "sums must be [parts, rows, columns]");
+        const int dt = dtype_code(res.scalar_type());
+        const float eps = (float)number(arg[5]);
+        at::Tensor c = sums ? result_like(res) : res, h = result_like(res);
+        check([&] { return mhip_finish_norm(stream_of(res), f32(sums), sums ? (int)sums->size(0) : 0, f32(bias), res.data_ptr(), sums ? c.data_ptr() : nullptr,
+                                            f32(&gamma), f32(beta), eps, h.data_ptr(), M, N, dt); });
+        PyObject *a = THPVariable_Wrap(std::move(c)), *b = THPVariable_Wrap(std::move(h));
+        PyObject* r = a && b ? PyTuple_Pack(2, a, b) : nullptr;
+        Py_XDECREF(a);
+        Py_XDECREF(b);
+        return r;
+    });
+}
+
+// causal_attention(qkv [B * S, 3 H D], B, H) -> [B * S, H D]: Q, K and V read in place
+FUNCTION(causal_attention) {
+    return guarded(n, 3, [&] {
+        const at::Tensor& x = dense(arg[0]);
+        const int64_t B = integer(arg[1]), H = integer(arg[2]);
+        if (x.dim() != 2 || B < 1 || H < 1 || x.size(0) % B != 0 || x.size(1) % (3 * H) != 0) raise(PyExc_ValueError, "expected a projection [B * S, 3 H D]");
+        const int64_t S = x.size(0) / B, d = x.size(1) / 3, D = d / H;
+        const int dt = dtype_code(x.scalar_type());
+        at::Tensor o = empty({B * S, d}, x.scalar_type(), x);
+        const int64_t in[3] = {S * 3 * d, D, 3 * d}, strides[12] = {in[0], in[1], in[2], in[0], in[1], in[2], in[0], in[1], in[2], S * d, D, d};
+        char* p = static_cast<char*>(x.data_ptr());
+        const int64_t step = d * x.element_size();
+        check([&] { return mhip_flash_attention_strided(stream_of(x), p, p + step, p + 2 * step, nullptr, o.data_ptr(), B, H, S, S, D,
+                                                        (float)(1.0 / std::sqrt((double)D)), 1, 0, 0, dt, strides); });
+        return THPVariable_Wrap(std::move(o));
+    });
+}
+
 // flash_attention(q, k, v, scale or None, is_causal, mask, out)
 FUNCTION(flash_attention) {
     return guarded(n, 7, [&] {
@@ -315,7 +390,7 @@ FUNCTION(bind) {
 }
 
 #define ENTRY(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
-PyMethodDef kMethods[] = {ENTRY(softmax), ENTRY(layer_norm), ENTRY(rms_norm), ENTRY(bias_gelu), ENTRY(matmul),
+PyMethodDef kMethods[] = {ENTRY(softmax), ENTRY(layer_norm), ENTRY(rms_norm), ENTRY(bias_gelu), ENTRY(matmul), ENTRY(linear), ENTRY(finish_norm), ENTRY(causal_attention),
                           ENTRY(flash_attention), ENTRY(argmax), ENTRY(bind), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

@@ -91,6 +91,8 @@ class GPT2:
         cfg = self.cfg
         B, S = ids.shape
         d, H = cfg.d_model, cfg.n_head
+        if self._few_tokens(B * S):
+            return self._forward_few(ids)
         # the graph's `convert` ops: fp32 parameters -> compute type, every step
         p = self.p32 if self.dtype == torch.float32 else self._views(kernels.convert(self.flat32, self.dtype))
         x = kernels.embed_tokens(ids, self.p32["wte"], self.p32["wpe"], self.dtype).reshape(B * S, d)
@@ -116,6 +118,35 @@ class GPT2:
             x = kernels.matmul(u, l["w_proj"], bias=l["b_proj"], residual=x)
         x = kernels.layer_norm(x, p["lnf_g"], p["lnf_b"], eps=1e-5)
         logits = kernels.matmul(x, p["wte_pad"], trans_b=True)   # tied head: x . wte^T (padded columns are 0)
+        return logits.reshape(B, S, self.vocab_pad)[..., :cfg.vocab]
+
+    def _few_tokens(self, tokens: int) -> bool:
+        """Whether every layer of this many tokens reads its parameters as they are held (kernels.linear)."""
+        d, f, dt = self.cfg.d_model, self.cfg.d_ff, self.dtype
+        if dt not in (torch.bfloat16, torch.float16) or d // self.cfg.n_head not in (64, 128) or d % self.cfg.n_head:
+            return False
+        return d <= 4096 and all(kernels.linear_served(tokens, n, k, dt) for n, k in ((3 * d, d), (d, d), (f, d), (d, f), (self.vocab_pad, d)))
+
+    def _forward_few(self, ids: torch.Tensor) -> torch.Tensor:
+        """The same operators for a short prompt: the parameters are rounded to the compute type where they are read
+        (converting all of them first took 117 of 705 us of kernels), and the launch that adds up a residual layer's
+        sums forms the next LayerNorm."""
+        cfg, p = self.cfg, self.p32
+        B, S = ids.shape
+        linear, layers, T = kernels.linear, p["layers"], B * S
+        o_parts, p_parts = (kernels.linear_parts(T, cfg.d_model, k) for k in (cfg.d_model, cfg.d_ff))
+        norms = [(l["ln1_g"], l["ln1_b"], 1e-5) for l in layers] + [(p["lnf_g"], p["lnf_b"], 1e-5)]
+        x = kernels.embed_tokens(ids, p["wte"], p["wpe"], self.dtype).reshape(T, cfg.d_model)
+        x, h = kernels.finish_norm(None, None, x, norms[0])
+        for i, l in enumerate(layers):
+            qkv = linear(h, l["w_qkv"], l["b_qkv"], ahead=(l["w_o"], l["w_fc"]))
+            a = kernels.causal_attention(qkv, B, cfg.n_head)
+            sums = linear(a, l["w_o"], parts=o_parts, ahead=(l["w_proj"],))
+            x, h = kernels.finish_norm(sums, l["b_o"], x, (l["ln2_g"], l["ln2_b"], 1e-5))
+            u = linear(h, l["w_fc"], l["b_fc"], "gelu")
+            sums = linear(u, l["w_proj"], parts=p_parts, ahead=(layers[i + 1]["w_qkv"],) if i + 1 < len(layers) else ())
+            x, h = kernels.finish_norm(sums, l["b_proj"], x, norms[i + 1])
+        logits = linear(h, p["wte_pad"], trans_b=True)
         return logits.reshape(B, S, self.vocab_pad)[..., :cfg.vocab]
 
     def capture(self, ids: torch.Tensor) -> "GraphedForward":

@@ -103,6 +103,32 @@ def flash_attention(q, k, v, scale: Optional[float] = None, is_causal: bool = Fa
     return (_native or _host()).flash_attention(q, k, v, scale, is_causal, mask, out)
 
 
+def linear(x, weight, bias=None, activation: str = "none", trans_b: bool = False, residual=None, parts: int = 0, ahead=()):
+    """act(x @ op(weight) + bias) (+ residual) in x's 16-bit type with parameters held in fp32, each rounded to that type at
+    use: what convert and matmul compute, in one launch; `linear_served` says for which sizes.  `parts` > 0 gives
+    the fp32 sums of so many shares of K ([parts, M, N], for finish_norm; `linear_parts` says how many).  `ahead`: up to two
+    weight matrices [K, N] that the next calls read (a hint, see mhip_linear_w32)."""
+    return (_native or _host()).linear(x, weight, bias, residual, ACTIVATION_CODE[activation], trans_b, parts, ahead)
+
+
+def linear_served(M: int, N: int, K: int, dtype) -> bool:
+    return bool(_lib.load().mhip_linear_w32_ok(M, N, K, DTYPE_CODE[dtype]))
+
+
+def linear_parts(M: int, N: int, K: int) -> int:
+    return _lib.load().mhip_linear_w32_parts(M, N, K)
+
+
+def finish_norm(sums, bias, residual, norm):
+    """(c, LayerNorm(c)) with c = round(sums.sum(0) + bias) + residual, or c = residual where sums is None; fp32 parameters."""
+    return (_native or _host()).finish_norm(sums, bias, residual, *norm)
+
+
+def causal_attention(qkv, batch: int, n_head: int):
+    """flash_attention(is_causal=True) over a fused projection [B * S, 3 H D], read in place -> [B * S, H D]."""
+    return (_native or _host()).causal_attention(qkv, batch, n_head)
+
+
 # ---- glue -------------------------------------------------------------------
 def gather_rows(table, indices):
     _dev(table, indices)
