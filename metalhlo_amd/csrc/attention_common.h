@@ -101,6 +101,19 @@ __device__ inline __amdgpu_buffer_rsrc_t fa_rsrc(const void* p, uint32_t bytes) 
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
 }
 
+// Buffer load of 16 bytes per lane straight into LDS: lane l lands at byte lds + 16 l (lds uniform, a multiple of 16).  As inline
+// assembly because the compiler puts a wait for ALL outstanding loads in front of any LDS read that it cannot tell apart from
+// the builtin's target, which is every read of another tile of the ring: the next block's loads would be waited for in the
+// middle of this one.  The caller counts its loads and waits itself.  (With three waves on a SIMD that hide the wait the builtin
+// is the faster form, by 2 %: it needs no M0 of its own.  M0 is a reserved register that cannot be named as clobbered; nothing
+// else in the caller uses it.)
+__device__ __forceinline__ void fa_load_to_lds(__amdgpu_buffer_rsrc_t rsrc, uint32_t lds, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(rsrc) : "memory");
+}
+__device__ __forceinline__ uint32_t fa_lds_address(const char* p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p;
+}
+
 // The softmax keeps a REFERENCE maximum per row (log2 domain) that moves only when a block's
 // maximum exceeds it by more than 8: probabilities are exp2(s - ref) <= 2^8, accumulated in fp32,
 // and the final division uses the sum taken with the same reference, so the result is the same
