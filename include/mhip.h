@@ -209,6 +209,14 @@ int mhip_flash_attention_strided(void* stream, const void* q, const void* k, con
                                  int64_t mask_stride_b, int64_t mask_stride_h, int dtype,
                                  const int64_t* strides);
 
+/* The same for more types and head sizes: fp32 with D a multiple of 32 up to 128 and strides that are multiples of 4
+ * elements, bf16 / f16 also with any D below 128 that is a multiple of 8. */
+int mhip_flash_attention_views(void* stream, const void* q, const void* k, const void* v,
+                               const void* mask, void* o, int64_t B, int64_t H, int64_t Sq,
+                               int64_t Skv, int64_t D, float scale, int is_causal,
+                               int64_t mask_stride_b, int64_t mask_stride_h, int dtype,
+                               const int64_t* strides);
+
 /* The same (strides may be NULL) with device memory the call may use: a few query rows (a decode step) over a long
  * cache are then split along the keys over the whole device.  mhip_flash_attention_workspace returns the bytes
  * that can be used (0: none); with less, or none, the keys are not split.  16-byte aligned; the content is

@@ -40,6 +40,8 @@ SIGNATURES = {
                                     _f32, _i32, _i64, _i64, _i32]),
     "mhip_flash_attention_strided": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
                                             _f32, _i32, _i64, _i64, _i32, _vp]),
+    "mhip_flash_attention_views": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
+                                          _f32, _i32, _i64, _i64, _i32, _vp]),
     "mhip_flash_attention_workspace": (_i64, [_i64, _i64, _i64, _i64, _i64, _i32, _i32]),
     "mhip_flash_attention_ws": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
                                        _f32, _i32, _i64, _i64, _i32, _vp, _vp, _i64]),

@@ -499,7 +499,7 @@ int launch_fa_decode(hipStream_t s, const FaArgs& a, int64_t D, int dtype, void*
 bool fa_flow_wanted(const FaArgs& a);
 int launch_fa_flow(hipStream_t s, FaArgs a, int64_t D, int dtype);
 // attention_f32.hip: fp32 tensors on the fp32 matrix instruction.
-bool fa_f32_mfma_eligible(const FaArgs& a, int64_t D);
+bool fa_f32_mfma_eligible(const FaArgs& a, int64_t D, bool packed);
 int launch_fa_f32_mfma(hipStream_t s, const FaArgs& a, int64_t D, float scale);
 }  // namespace mhip
 
@@ -509,7 +509,7 @@ using namespace mhip;
 static int fa_entry(const char* name, void* stream, const void* q, const void* k, const void* v, const void* mask, void* o,
                     int64_t B, int64_t H, int64_t Sq, int64_t Skv, int64_t D, float scale, int is_causal,
                     int64_t mask_stride_b, int64_t mask_stride_h, int dtype, const int64_t* strides, void* workspace = nullptr,
-                    int64_t workspace_bytes = 0) {
+                    int64_t workspace_bytes = 0, bool any_views = false) {
     if (B < 0 || H < 0 || Sq < 0 || Skv < 0 || D <= 0)
         return fail(MHIP_ERR_INVALID_ARGUMENT, "%s: bad size", name);
     if (D > 256) return fail(MHIP_ERR_UNSUPPORTED, "%s: head_dim %lld > 256", name, (long long)D);
@@ -566,15 +566,16 @@ static int fa_entry(const char* name, void* stream, const void* q, const void* k
         return D == 128 ? launch_fa<f16_t, 128>(s, a, is_causal, hm)
                         : launch_fa<f16_t, 64>(s, a, is_causal, hm);
     }
-    // (with packed rows of a multiple of 8 elements every piece of 16 bytes is aligned)
-    if (is16 && is_packed && aligned && fits && Skv > 0 && D % 8 == 0 && D < 128)
+    // (with rows of a multiple of 8 elements every piece of 16 bytes is aligned)
+    if (is16 && (is_packed || (any_views && strides_aligned)) && aligned && fits && Skv > 0 && D % 8 == 0 && D < 128)
         return dtype == MHIP_BF16 ? launch_fa_part<bf16_t>(s, a, is_causal, mask != nullptr) : launch_fa_part<f16_t>(s, a, is_causal, mask != nullptr);
+    if (any_views && !is_packed && Skv > 0 && dtype == MHIP_F32 && fa_f32_mfma_eligible(a, D, false)) return launch_fa_f32_mfma(s, a, D, scale);
     if (!is_packed)
         return fail(MHIP_ERR_UNSUPPORTED, "%s: strided layouts need bf16 / f16, head_dim 64 or 128, 16-byte aligned pointers and "
                                           "strides that are multiples of 8 elements", name);
     switch (dtype) {
         case MHIP_F32:
-            if (fa_f32_mfma_eligible(a, D)) return launch_fa_f32_mfma(s, a, D, scale);
+            if (fa_f32_mfma_eligible(a, D, true)) return launch_fa_f32_mfma(s, a, D, scale);
             return launch_fa_scalar<float>(s, a, (int)D, scale);
         case MHIP_BF16: return launch_fa_scalar<bf16_t>(s, a, (int)D, scale);
         case MHIP_F16: return launch_fa_scalar<f16_t>(s, a, (int)D, scale);
@@ -597,6 +598,13 @@ extern "C" int mhip_flash_attention_strided(void* stream, const void* q, const v
                                             const int64_t* strides) {
     return fa_entry("mhip_flash_attention_strided", stream, q, k, v, mask, o, B, H, Sq, Skv, D, scale, is_causal,
                     mask_stride_b, mask_stride_h, dtype, strides);
+}
+
+extern "C" int mhip_flash_attention_views(void* stream, const void* q, const void* k, const void* v, const void* mask, void* o,
+                                          int64_t B, int64_t H, int64_t Sq, int64_t Skv, int64_t D, float scale, int is_causal,
+                                          int64_t mask_stride_b, int64_t mask_stride_h, int dtype, const int64_t* strides) {
+    return fa_entry("mhip_flash_attention_views", stream, q, k, v, mask, o, B, H, Sq, Skv, D, scale, is_causal, mask_stride_b,
+                    mask_stride_h, dtype, strides, nullptr, 0, true);
 }
 
 extern "C" int mhip_flash_attention_ws(void* stream, const void* q, const void* k, const void* v, const void* mask, void* o,

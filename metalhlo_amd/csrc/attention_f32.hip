@@ -10,7 +10,12 @@
 // 32-lane halves, and the probabilities are already laid out as the B operand of the second
 // product O^T += V^T . P^T (k-step i of that product pairs key 8 (i / 4) + 4 (lane / 32) + i % 4
 // of the block with the lane's own register i), so P never moves between lanes.
+//
+// Rows of q, k, v and o lie where the strides say: a transformer block's head split and merge around this kernel (seven
+// copies of 3 us each over [1,128,768], 7 of 5 to 9 us over [4,500,1024]) are then not run.
 #include <math.h>
+
+#include <initializer_list>
 
 #include "attention_common.h"
 
@@ -42,10 +47,12 @@ __global__ __launch_bounds__(256, 2) void fa_f32_mfma_kernel(FaArgs a, float sca
     const int q0 = qb * kFBQ + wave * 32;
     const int qpos = q0 + ln;                       // this lane's query row
     const bool q_live = qpos < a.Sq;
-    const float* qp = static_cast<const float*>(a.q) + (int64_t)bh * a.Sq * D;
-    const float* kp = static_cast<const float*>(a.k) + (int64_t)bh * a.Skv * D;
-    const float* vp = static_cast<const float*>(a.v) + (int64_t)bh * a.Skv * D;
-    float* op = static_cast<float*>(a.o) + (int64_t)bh * a.Sq * D;
+    const int b_i = bh / a.H, h_i = bh % a.H;
+    const float* qp = static_cast<const float*>(a.q) + b_i * a.qs[0] + h_i * a.qs[1];
+    const float* kp = static_cast<const float*>(a.k) + b_i * a.ks[0] + h_i * a.ks[1];
+    const float* vp = static_cast<const float*>(a.v) + b_i * a.vs[0] + h_i * a.vs[1];
+    float* op = static_cast<float*>(a.o) + b_i * a.os[0] + h_i * a.os[1];
+    const int64_t k_rs = a.ks[2], v_rs = a.vs[2];
     const float* mp = HAS_MASK ? static_cast<const float*>(a.mask) + (int64_t)(bh / a.H) * a.mask_sb +
                                      (int64_t)(bh % a.H) * a.mask_sh + (int64_t)qpos * a.Skv
                                : nullptr;
@@ -53,7 +60,7 @@ __global__ __launch_bounds__(256, 2) void fa_f32_mfma_kernel(FaArgs a, float sca
     // Q^T fragments: k-step s holds Q[qpos][2 s + h]
     float qf[NS];
 #pragma unroll
-    for (int s = 0; s < NS; s++) qf[s] = q_live ? qp[(int64_t)qpos * D + 2 * s + h] : 0.f;
+    for (int s = 0; s < NS; s++) qf[s] = q_live ? qp[qpos * a.qs[2] + 2 * s + h] : 0.f;
 
     int nkv = (a.Skv + kFBK - 1) / kFBK;
     if (CAUSAL) {
@@ -77,8 +84,8 @@ __global__ __launch_bounds__(256, 2) void fa_f32_mfma_kernel(FaArgs a, float sca
             const int p = j * 256 + tid, row = p / (D / 4), col = (p % (D / 4)) * 4;
             const int key = blk * kFBK + row;
             if (key < a.Skv) {
-                kr[j] = *reinterpret_cast<const f32x4*>(kp + (int64_t)key * D + col);
-                vr[j] = *reinterpret_cast<const f32x4*>(vp + (int64_t)key * D + col);
+                kr[j] = *reinterpret_cast<const f32x4*>(kp + key * k_rs + col);
+                vr[j] = *reinterpret_cast<const f32x4*>(vp + key * v_rs + col);
             } else {
                 kr[j] = f32x4{0.f, 0.f, 0.f, 0.f};
                 vr[j] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -161,7 +168,7 @@ __global__ __launch_bounds__(256, 2) void fa_f32_mfma_kernel(FaArgs a, float sca
     const float l_tot = half_sum(l_run);
     const float inv = l_tot > 1e-10f ? 1.f / l_tot : 0.f;
     if (q_live) {
-        float* orow = op + (int64_t)qpos * D;
+        float* orow = op + qpos * a.os[2];
 #pragma unroll
         for (int d = 0; d < ND; d++)
 #pragma unroll
@@ -188,10 +195,11 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaAr
     tile_of_workgroup<CAUSAL>(a, blockIdx.x, bh, qb);
     const int q0 = qb * 32, qpos = q0 + ln;
     const bool q_live = qpos < a.Sq;
-    const float* qp = static_cast<const float*>(a.q) + (int64_t)bh * a.Sq * D;
-    const uint32_t bytes = (uint32_t)((int64_t)a.Skv * D * 4);
-    const __amdgpu_buffer_rsrc_t rk = fa_rsrc(static_cast<const float*>(a.k) + (int64_t)bh * a.Skv * D, bytes);
-    const __amdgpu_buffer_rsrc_t rv = fa_rsrc(static_cast<const float*>(a.v) + (int64_t)bh * a.Skv * D, bytes);
+    const int b_i = bh / a.H, h_i = bh % a.H;
+    const float* qp = static_cast<const float*>(a.q) + b_i * a.qs[0] + h_i * a.qs[1];
+    const int k_rs = (int)a.ks[2], v_rs = (int)a.vs[2];
+    const __amdgpu_buffer_rsrc_t rk = fa_rsrc(static_cast<const float*>(a.k) + b_i * a.ks[0] + h_i * a.ks[1], (uint32_t)((((int64_t)a.Skv - 1) * k_rs + D) * 4));
+    const __amdgpu_buffer_rsrc_t rv = fa_rsrc(static_cast<const float*>(a.v) + b_i * a.vs[0] + h_i * a.vs[1], (uint32_t)((((int64_t)a.Skv - 1) * v_rs + D) * 4));
     const float* mp = HAS_MASK ? static_cast<const float*>(a.mask) + (int64_t)(bh / a.H) * a.mask_sb +
                                      (int64_t)(bh % a.H) * a.mask_sh + (int64_t)min(qpos, a.Sq - 1) * a.Skv
                                : nullptr;
@@ -201,7 +209,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaAr
     f32x4 qf[NS];
 #pragma unroll
     for (int j = 0; j < NS; j++)
-        qf[j] = q_live ? *reinterpret_cast<const f32x4*>(qp + (int64_t)qpos * D + 8 * j + 4 * h) : f32x4{0.f, 0.f, 0.f, 0.f};
+        qf[j] = q_live ? *reinterpret_cast<const f32x4*>(qp + qpos * a.qs[2] + 8 * j + 4 * h) : f32x4{0.f, 0.f, 0.f, 0.f};
 
     int nkv = (a.Skv + kFBK - 1) / kFBK;
     if (CAUSAL) nkv = min(nkv, qb + 1);
@@ -210,17 +218,17 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaAr
     f32x4 kr[NS];
     float vr[ND][16];
     auto load_k = [&](int blk) __attribute__((always_inline)) {
-        const uint32_t off = (uint32_t)((blk * kFBK + ln) * (D * 4) + 16 * h);
+        const uint32_t off = (uint32_t)((blk * kFBK + ln) * (k_rs * 4) + 16 * h);
 #pragma unroll
         for (int j = 0; j < NS; j++) kr[j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, off + 32 * j, 0, 0));
     };
     auto load_v = [&](int blk) __attribute__((always_inline)) {
-        const uint32_t off = (uint32_t)((blk * kFBK + 4 * h) * (D * 4) + 4 * ln);
+        const uint32_t off = (uint32_t)((blk * kFBK + 4 * h) * (v_rs * 4) + 4 * ln);
 #pragma unroll
         for (int i = 0; i < 16; i++)
 #pragma unroll
             for (int d = 0; d < ND; d++)
-                vr[d][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, off + (uint32_t)((8 * (i >> 2) + (i & 3)) * (D * 4) + 128 * d), 0, 0));
+                vr[d][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, off + (uint32_t)((8 * (i >> 2) + (i & 3)) * (v_rs * 4) + 128 * d), 0, 0));
     };
 
     f32x16 o[ND];
@@ -286,7 +294,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaAr
     // ---- the waves' states, 32 columns of the output at a time
     l_run = half_sum(l_run);
     if (h == 0) { ml[0][wave][ln] = m_run; ml[1][wave][ln] = l_run; }
-    float* op = static_cast<float*>(a.o) + (int64_t)bh * a.Sq * D;
+    float* op = static_cast<float*>(a.o) + b_i * a.os[0] + h_i * a.os[1];
     const int col = threadIdx.x & 31, row0 = threadIdx.x >> 5;
 #pragma unroll
     for (int d = 0; d < ND; d++) {
@@ -307,7 +315,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaAr
                 l = fmaf(ml[1][w][q], al, l);
                 sum = fmaf(part[w][q][col], al, sum);
             }
-            if (q0 + q < a.Sq) op[(int64_t)(q0 + q) * D + 32 * d + col] = sum * (l > 1e-10f ? 1.f / l : 0.f);
+            if (q0 + q < a.Sq) op[(q0 + q) * a.os[2] + 32 * d + col] = sum * (l > 1e-10f ? 1.f / l : 0.f);
         }
     }
 }
@@ -320,7 +328,7 @@ int launch_f32(hipStream_t s, FaArgs a, float scale, bool causal, bool has_mask)
     // D 128 621 | 738), except where rows are short or keys many: 1024 tiles of D 32 174 | 165, 384 of [4,12,1000,64] 100 | 78
     // (768 of [16,12,512,64] 81 | 95).
     const int64_t tiles = (int64_t)a.B * a.H * ((a.Sq + kFBQ - 1) / kFBQ);
-    const bool split = ((int64_t)a.Skv + kFBQ) * D * 4 < 0x7FFFFFFFLL &&
+    const bool split = ((int64_t)a.Skv + kFBQ) * (a.ks[2] > a.vs[2] ? a.ks[2] : a.vs[2]) * 4 < 0x7FFFFFFFLL &&
                        (tiles < 256 || (D == 32 && tiles <= 1024) || (D == 64 && tiles <= 512 && a.Skv >= 768));
     const int rows = split ? 32 : kFBQ;
     a.nqb = (a.Sq + rows - 1) / rows;
@@ -342,14 +350,18 @@ int launch_f32(hipStream_t s, FaArgs a, float scale, bool causal, bool has_mask)
 
 }  // namespace
 
-// fp32, packed [B,H,S,D], head size a multiple of 32 up to 128, 16-byte aligned tensors.
-// MHIP_FA_F32_MFMA=2 keeps the scalar kernel.
-bool fa_f32_mfma_eligible(const FaArgs& a, int64_t D) {
-    if (tune_int("MHIP_FA_F32_MFMA", 1) == 2) return false;
+// fp32, [B,H,S,D] with strides that are multiples of 4 elements, head size a multiple of 32 up to 128, 16-byte aligned tensors.
+// MHIP_FA_F32_MFMA=2 keeps the scalar kernel for packed tensors, the only ones it reads.
+bool fa_f32_mfma_eligible(const FaArgs& a, int64_t D, bool packed) {
+    if (packed && tune_int("MHIP_FA_F32_MFMA", 1) == 2) return false;
     if (D % 32 != 0 || D > 128 || a.Skv < 1) return false;
     const uintptr_t all = reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) |
                           reinterpret_cast<uintptr_t>(a.v) | reinterpret_cast<uintptr_t>(a.o);
-    return (all & 15) == 0;
+    if ((all & 15) != 0) return false;
+    for (const int64_t* st : {a.qs, a.ks, a.vs, a.os})
+        for (int i = 0; i < 3; i++)
+            if (st[i] % 4 != 0) return false;
+    return true;
 }
 
 int launch_fa_f32_mfma(hipStream_t s, const FaArgs& a, int64_t D, float scale) {

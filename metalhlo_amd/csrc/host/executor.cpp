@@ -465,6 +465,78 @@ static std::vector<int64_t> dot_result_shape(const Op& op, const TensorType& lt,
     return shape;
 }
 
+// Attention in fp32, or in a 16-bit type with a head size other than 64 and 128 (those are rewritten by the fusion pass): a
+// [B,H,S,D] operand that is transpose{0,2,1,3}(reshape [B,S,H,D](slice [:, :, off : off + H D](t))), the slice optional and
+// each step without another reader, is read where t lies, and a result whose only reader is transpose{0,2,1,3} is written in
+// that order.  Those operations stay in the program and launch nothing.  [1,128,768], 12 heads, fp32: seven copies of 3.1 us.
+static void fold_head_views(Executable& exe) {
+    const Function& fn = exe.fn;
+    exe.folded.assign(fn.ops.size(), 0);
+    exe.head_views.clear();
+    if (exe.opt_level < 2) return;
+    const std::vector<TensorType> vt = value_types(fn);
+    std::vector<int> uses(fn.num_values, 0), by(fn.num_values, -1);
+    for (size_t i = 0; i < fn.ops.size(); i++) {
+        by[fn.ops[i].result] = (int)i;
+        for (int v : fn.ops[i].operands) uses[v]++;
+    }
+    for (int r : fn.returns) uses[r]++;
+    const std::vector<int64_t> swap = {0, 2, 1, 3};
+    // the operation behind `v` when it is a `name` that only one operation reads
+    auto only = [&](int v, const char* name) -> int { return by[v] >= 0 && uses[v] == 1 && fn.ops[by[v]].name == name ? by[v] : -1; };
+    for (size_t oi = 0; oi < fn.ops.size(); oi++) {
+        const Op& at = fn.ops[oi];
+        if (at.name != "custom_call" || at.target != "fused_scaled_dot_product_attention" || at.out.shape.size() != 4) continue;
+        if (!parse_config(at.backend_config).get_int_array("views", {}).empty()) continue;
+        const TensorType& qt = vt[at.operands[0]];
+        const TensorType& kt = vt[at.operands[1]];
+        if (qt.shape.size() != 4 || kt.shape.size() != 4 || !(vt[at.operands[2]] == kt) || kt.dtype != qt.dtype || at.out.dtype != qt.dtype) continue;
+        const int64_t B = qt.shape[0], H = qt.shape[1], Sq = qt.shape[2], D = qt.shape[3], Skv = kt.shape[2];
+        if (qt.numel() < 1 || kt.numel() < 1 || D > 128 || D % (qt.dtype == F32 ? 32 : 8) != 0) continue;
+        if (qt.dtype != F32 && qt.dtype != BF16 && qt.dtype != F16) continue;
+        std::array<int64_t, 16> views;
+        std::vector<int> away;
+        for (int t = 0; t < 4; t++) {
+            const int64_t S = t == 0 || t == 3 ? Sq : Skv;
+            const int64_t packed[4] = {0, H * S * D, S * D, D};
+            std::copy(packed, packed + 4, views.begin() + 4 * t);
+        }
+        for (int t = 0; t < 3; t++) {
+            const int64_t S = t == 0 ? Sq : Skv;
+            const int tr = only(at.operands[t], "transpose");
+            const int rs = tr >= 0 && fn.ops[tr].dims == swap ? only(fn.ops[tr].operands[0], "reshape") : -1;
+            if (rs < 0 || vt[fn.ops[rs].operands[0]].shape != std::vector<int64_t>{B, S, H * D}) continue;
+            std::vector<int> steps = {tr, rs};
+            int64_t off = 0, W = H * D;
+            const int sl = only(fn.ops[rs].operands[0], "slice");
+            if (sl >= 0) {
+                const Op& c = fn.ops[sl];
+                const TensorType& wide = vt[c.operands[0]];
+                if (wide.shape.size() == 3 && wide.shape[0] == B && wide.shape[1] == S && c.starts[0] == 0 && c.starts[1] == 0 && c.strides[2] == 1) {
+                    off = c.starts[2];
+                    W = wide.shape[2];
+                    steps.push_back(sl);
+                }
+            }
+            // (16 bytes per piece, and an extent that the kernels' 32-bit byte offsets span)
+            if (off % 8 != 0 || W % 8 != 0 || S * W * 4 >= 0x7FFFFFFF) continue;
+            const int64_t view[4] = {off, S * W, D, W};
+            std::copy(view, view + 4, views.begin() + 4 * t);
+            away.insert(away.end(), steps.begin(), steps.end());
+        }
+        if (uses[at.result] == 1 && Sq * H * D * 4 < 0x7FFFFFFF)
+            for (size_t i = oi + 1; i < fn.ops.size(); i++)
+                if (fn.ops[i].name == "transpose" && fn.ops[i].operands[0] == at.result && fn.ops[i].dims == swap) {
+                    const int64_t view[4] = {0, Sq * H * D, D, H * D};
+                    std::copy(view, view + 4, views.begin() + 12);
+                    away.push_back((int)i);
+                }
+        if (away.empty()) continue;
+        for (int i : away) exe.folded[i] = 1;
+        exe.head_views[(int)oi] = views;
+    }
+}
+
 // The fused kernels derive every extent from their operands and write a result of the operands'
 // element type: a custom_call whose declared result (or an operand) says otherwise would be an
 // out-of-bounds write or a misread buffer, so it is refused here, before anything runs.
@@ -692,6 +764,7 @@ void compile(Executable& exe) {
         std::lock_guard<std::mutex> stream_lock(exe.client->stream_mu);     // another thread may be capturing the stream
         (void)hipStreamSynchronize(exe.client->stream);
     }
+    fold_head_views(exe);
     plan_memory(exe);
 }
 
@@ -768,7 +841,7 @@ static std::vector<DeviceTensor> run_ops(Executable& exe, const std::vector<Devi
         if (n == "constant") {
             out = exe.constants[oi];
             out.type = op.out;
-        } else if (n == "reshape") {
+        } else if (n == "reshape" || exe.folded[oi]) {
             out = in(0);
             out.type = op.out;
         } else {
@@ -1002,13 +1075,22 @@ static std::vector<DeviceTensor> run_ops(Executable& exe, const std::vector<Devi
                         msb = mb == B && B != 1 ? mh * Sq * Skv : 0;
                         mask = in(3).data();
                     }
-                    RUN(mhip_flash_attention(s, in(0).data(), in(1).data(), in(2).data(), mask, out.data(), B, H, Sq, Skv, D,
-                                               scale, cfg.get_bool("is_causal", false), msb, msh, dt));
+                    const auto folded = exe.head_views.find((int)oi);
+                    if (folded != exe.head_views.end()) {
+                        const auto& vw = folded->second;
+                        int64_t strides[12];
+                        for (int t = 0; t < 4; t++) std::copy(vw.begin() + 4 * t + 1, vw.begin() + 4 * t + 4, strides + 3 * t);
+                        auto at = [&](const void* p, int64_t off) { return static_cast<const char*>(p) + off * dtype_bytes(dt); };
+                        RUN(mhip_flash_attention_views(s, at(in(0).data(), vw[0]), at(in(1).data(), vw[4]), at(in(2).data(), vw[8]), mask,
+                                                       out.data(), B, H, Sq, Skv, D, scale, cfg.get_bool("is_causal", false), msb, msh, dt, strides));
+                    } else
+                        RUN(mhip_flash_attention(s, in(0).data(), in(1).data(), in(2).data(), mask, out.data(), B, H, Sq, Skv, D,
+                                                   scale, cfg.get_bool("is_causal", false), msb, msh, dt));
                 }
             }
         }
         val[op.result] = out;
-        if (n != "constant" && n != "reshape") mark((int)oi);
+        if (n != "constant" && n != "reshape" && !exe.folded[oi]) mark((int)oi);
         for (int v : op.operands)
             if (last[v] == (int)oi) val[v] = DeviceTensor();
     }
@@ -1182,7 +1264,7 @@ std::vector<DeviceTensor> execute(Executable& exe, const std::vector<DeviceTenso
     // a replay costs one graph launch plus the copies of the results out of the arena: it pays
     // from roughly twenty launches per execution on, so short programs stay eager by default
     size_t launches = 0;
-    for (auto& op : fn.ops) launches += op.name != "constant" && op.name != "reshape";
+    for (auto& op : fn.ops) launches += op.name != "constant" && op.name != "reshape";     // (folded ones count: the line was drawn so)
     const bool profile_env = env_flag("METALHLO_PROFILE_GPU", false);
     const bool profile = profile_env || exe.profile_next;          // a profiled execution is eager: events between the launches
     exe.profile_next = false;

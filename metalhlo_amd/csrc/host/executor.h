@@ -6,6 +6,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -98,6 +99,8 @@ struct Executable {
     Function fn;
     int opt_level = 2;
     std::vector<DeviceTensor> constants;   // per op index (empty when the op is not a constant)
+    std::vector<char> folded;              // per op index: a step of a view that its only reader takes in place, nothing is launched
+    std::map<int, std::array<int64_t, 16>> head_views;   // attention op index -> {offset, batch, head, row stride} x {q, k, v, o}, elements
     size_t batched_converts = 0;           // leading ops: f32 -> 16-bit converts of arguments, run as one batch
     // statistics (milliseconds), CInterface.swift:63-96
     int64_t exec_count = 0;
