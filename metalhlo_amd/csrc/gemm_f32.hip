@@ -1,7 +1,7 @@
 // fp32 GEMM on the matrix cores of gfx950: v_mfma_f32_32x32x2_f32 (fp32 operands, fp32
 // accumulate -- the products are exact fp32 products, so the 1e-5 bar of fp32 programs holds).
 //
-// Operands whose rows are 16-byte aligned go through the ring further down; this kernel takes the others.
+// Operands that one buffer descriptor spans go through the ring further down; this kernel takes the larger ones.
 //
 // One workgroup = a 64x64 tile of C, four waves (2 x 2), one 32x32 accumulator each (or a
 // 128x128 tile, 2 x 2 accumulators per wave).  K advances in steps of 16 through two LDS stage buffers: while a
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_mfma_kernel(GemmArgs g) {
     store_f32<WB>(g, acc, m0 + wm * 32 * WB, n0 + wn * 32 * WB, batch, lane);
 }
 
-// ---- operands whose rows are 16-byte aligned: a ring of LDS stages filled by the loads themselves ----
+// ---- a ring of LDS stages filled by the loads themselves ----
 //
 // With one stage of 16 k in flight a problem that does not fill the device waits out a load latency per stage
 // (0.55 us; the stage's matrix instructions take 0.21).  [2048,2048] x K 2048 173 -> 143 us (120 TFLOP/s),
@@ -210,9 +210,12 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_mfma_kernel(GemmArgs g) {
 // 128 bytes (lane = row, 16 bytes = four consecutive k), the other one as it lies in memory, [32 k][rows], read
 // one float per lane with the rows k and k + 4 that one issue takes on different halves of the banks.
 // An issue sums k = 8 s + e (lower half of the wave) and 8 s + 4 + e (upper half).
-template <int ROWS, bool KMAJOR>
+// W = bytes per lane and load: 16, or 4 where a row does not start on 16 bytes (four times the loads, sixteen beside sixteen
+// matrix instructions of 64 cycles; the same tile).  us, register-staged | W = 4: [890,712] x K 1536 with A stored [K, M]
+// 78.2 | 46.2, [1001,777] x K 1500 60.4 | 49.2, [2047,2047] x K 2047 192 | 178, [300,333] x K 999 43.0 | 32.8.
+template <int ROWS, bool KMAJOR, int W>
 struct RingLoader {
-    static constexpr int kLoads = ROWS * kRowBytes / 1024 / 4;      // wave-wide loads of 1 KB per stage and wave
+    static constexpr int kLoads = ROWS * kRowBytes / (64 * W) / 4;  // wave-wide loads per stage and wave
     uint32_t off[kLoads];      // byte offset in stage 0, kOob where the row / column does not exist
     int k[kLoads];             // first k of the piece inside the stage
     uint32_t step;
@@ -220,16 +223,17 @@ struct RingLoader {
         step = (uint32_t)(KMAJOR ? 128 : (int64_t)32 * ld * 4);
 #pragma unroll
         for (int i = 0; i < kLoads; i++) {
-            const int p = (i * 4 + wave) * 64 + lane;               // 16-byte slot of the tile
+            // 16-byte slot of the tile, and the element in it
+            const int lin = (i * 4 + wave) * 64 + lane, p = W == 16 ? lin : lin >> 2, e = W == 16 ? 0 : lin & 3;
             if (KMAJOR) {
                 const int r = p >> 3, c = (p & 7) ^ swz(r);
-                k[i] = c * 4;
-                off[i] = row0 + r < rows_total ? (uint32_t)(((int64_t)(row0 + r) * ld + c * 4) * 4) : kOob;
+                k[i] = c * 4 + e;
+                off[i] = row0 + r < rows_total ? (uint32_t)(((int64_t)(row0 + r) * ld + k[i]) * 4) : kOob;
             } else {
                 constexpr int kCpr = ROWS / 4;
-                const int kk = p / kCpr, c = (p % kCpr) ^ (kk >> 2 & 1) << 3;
+                const int kk = p / kCpr, c = (p % kCpr) ^ (kk >> 2 & 1) << 3, col = row0 + c * 4 + e;
                 k[i] = kk;
-                off[i] = row0 + c * 4 < rows_total ? (uint32_t)(((int64_t)kk * ld + row0 + c * 4) * 4) : kOob;
+                off[i] = col < rows_total ? (uint32_t)(((int64_t)kk * ld + col) * 4) : kOob;
             }
         }
     }
@@ -238,7 +242,8 @@ struct RingLoader {
 #pragma unroll
         for (int i = 0; i < kLoads; i++) {
             const bool ok = off[i] != kOob && kt * 32 + k[i] < K;
-            load_to_lds(rsrc, tile + (uint32_t)(i * 4 + wave) * 1024u, ok ? off[i] + at : kOob);
+            if (W == 16) load_to_lds(rsrc, tile + (uint32_t)(i * 4 + wave) * 1024u, ok ? off[i] + at : kOob);
+            else load_dword_to_lds(rsrc, tile + (uint32_t)(i * 4 + wave) * 256u, ok ? off[i] + at : kOob);
         }
     }
 };
@@ -255,7 +260,7 @@ __device__ __forceinline__ f32x4 ring_frag(const char* tile, int row0, int s, in
     return v;
 }
 
-template <bool TA, bool TB, int WB, int S>
+template <bool TA, bool TB, int WB, int S, int W>
 __global__ __launch_bounds__(256) void gemm_f32_ring_kernel(GemmArgs g) {
     constexpr int kTile = 64 * WB, kBytes = kTile * kRowBytes, kStage = 2 * kBytes;
     extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -268,14 +273,14 @@ __global__ __launch_bounds__(256) void gemm_f32_ring_kernel(GemmArgs g) {
     const __amdgpu_buffer_rsrc_t ra = make_rsrc(a, (uint32_t)((int64_t)g.M * g.K * 4)), rb = make_rsrc(b, (uint32_t)((int64_t)g.N * g.K * 4));
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave >> 1, wn = wave & 1;
-    // this workgroup's stages: all of K, or one split's
+    // this workgroup's stages: one part of K, or all parts one after the other
     const int all = (g.K + 31) / 32, per = (all + g.splits - 1) / g.splits;
-    const int kt0 = (int)blockIdx.z * per, kt1 = min(all, kt0 + per), kend = min(g.K, kt1 * 32);
-    RingLoader<kTile, !TA> la;
-    RingLoader<kTile, TB> lb;
+    const int kt0 = (int)blockIdx.z * per, kt1 = g.partial ? min(all, kt0 + per) : all, kend = min(g.K, kt1 * 32);
+    RingLoader<kTile, !TA, W> la;
+    RingLoader<kTile, TB, W> lb;
     la.init(m0, g.M, g.lda, wave, lane);
     lb.init(n0, g.N, g.ldb, wave, lane);
-    constexpr int kLoads = 2 * RingLoader<kTile, !TA>::kLoads;
+    constexpr int kLoads = 2 * RingLoader<kTile, !TA, W>::kLoads;
     // (a stage behind the last one is loaded all the same, out of bounds: the waits count loads)
     const uint32_t ring = lds_address(smem);
     auto load = [&](int kt) {
@@ -284,16 +289,27 @@ __global__ __launch_bounds__(256) void gemm_f32_ring_kernel(GemmArgs g) {
         lb.load(rb, st + kBytes, wave, kt, kend);
     };
 
-    f32x16 acc[WB][WB];
+    // (sum: the parts that are done, added in their order: the bits of the launch that has a workgroup for each)
+    f32x16 acc[WB][WB], sum[WB][WB];
 #pragma unroll
     for (int i = 0; i < WB; i++)
 #pragma unroll
         for (int j = 0; j < WB; j++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
+            for (int e = 0; e < 16; e++) acc[i][j][e] = sum[i][j][e] = 0.f;
+    auto close_part = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < WB; i++)
+#pragma unroll
+            for (int j = 0; j < WB; j++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) { sum[i][j][e] += acc[i][j][e]; acc[i][j][e] = 0.f; }
+    };
 #pragma unroll
     for (int p = 0; p < S - 1; p++) load(kt0 + p);
+    int part_end = kt0 + per;
     for (int kt = kt0; kt < kt1; kt++) {
+        if (kt == part_end) { close_part(); part_end += per; }
         // stage kt has landed when only the S - 2 stages behind it are in flight; past the barrier that holds for
         // every wave's share, and every wave has read stage kt - 1, whose place is reused
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * kLoads) : "memory");
@@ -323,7 +339,8 @@ __global__ __launch_bounds__(256) void gemm_f32_ring_kernel(GemmArgs g) {
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // nothing may land in LDS after the workgroup ends
-    store_f32<WB>(g, acc, m0 + wm * 32 * WB, n0 + wn * 32 * WB, batch, lane);
+    close_part();
+    store_f32<WB>(g, sum, m0 + wm * 32 * WB, n0 + wn * 32 * WB, batch, lane);
 }
 
 template <bool TA, bool TB, int WB>
@@ -337,10 +354,10 @@ int launch_tile(hipStream_t s, GemmArgs g, int64_t batch) {
     return check_launch("gemm_f32_mfma");
 }
 
-template <bool TA, bool TB, int WB, int S>
+template <bool TA, bool TB, int WB, int S, int W>
 int launch_ring(hipStream_t s, GemmArgs g, int64_t batch) {
     constexpr int kTile = 64 * WB, kSmem = S * 2 * kTile * kRowBytes;
-    auto kern = gemm_f32_ring_kernel<TA, TB, WB, S>;
+    auto kern = gemm_f32_ring_kernel<TA, TB, WB, S, W>;
     if (kSmem > 64 * 1024) {
         static std::once_flag once;
         static hipError_t err = hipSuccess;
@@ -351,7 +368,7 @@ int launch_ring(hipStream_t s, GemmArgs g, int64_t batch) {
     g.tiles_n = (g.N + kTile - 1) / kTile;
     const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n;
     if (tiles > 0x7FFFFFFFLL || batch > 65535) return fail(MHIP_ERR_UNSUPPORTED, "gemm: grid too large");
-    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)batch, (unsigned)g.splits), dim3(256), kSmem, s, g);
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)batch, g.partial ? (unsigned)g.splits : 1u), dim3(256), kSmem, s, g);
     return check_launch("gemm_f32_ring");
 }
 
@@ -362,26 +379,27 @@ int64_t large_tiles(int64_t M, int64_t N, int64_t batch) { return ((M + 127) / 1
 // [8192,768] x K 3072 308 | 405; register-staged 1183 at 4096^3 (128), 173 at 2048^3 and 382 (64).  Rings of
 // three and four stages are 2 to 8 % behind two: the workgroups of a unit hide each other's latency.
 template <bool TA, bool TB>
-int launch(hipStream_t s, const GemmArgs& g, int64_t batch, bool ring) {
-    const bool large = large_tiles(g.M, g.N, batch) >= 960 && g.splits == 1;
-    if (ring) return large ? launch_ring<TA, TB, 2, 2>(s, g, batch) : launch_ring<TA, TB, 1, 2>(s, g, batch);
+int launch(hipStream_t s, const GemmArgs& g, int64_t batch, bool ring, bool wide) {
+    const bool large = large_tiles(g.M, g.N, batch) >= 960 && !g.partial;
+    if (ring && wide) return large ? launch_ring<TA, TB, 2, 2, 16>(s, g, batch) : launch_ring<TA, TB, 1, 2, 16>(s, g, batch);
+    if (ring) return large ? launch_ring<TA, TB, 2, 2, 4>(s, g, batch) : launch_ring<TA, TB, 1, 2, 4>(s, g, batch);
     return large ? launch_tile<TA, TB, 2>(s, g, batch) : launch_tile<TA, TB, 1>(s, g, batch);
 }
 
-// Parts of K where a workspace takes them and half of the compute units have no tile: up to two workgroups per compute
-// unit, each with at least 512 k ([512,512] x K 16384 488 -> 89 us; 192 tiles in two parts, [192,4096] x K 1024, take
-// 30.8 us against 26.1 whole).  As with 16-bit operands a sum is left in one piece from 193 rows on unless K is 4096 or more.
-int ring_splits(int64_t M, int64_t N, int64_t K, int64_t batch) {
-    const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
-    if (batch != 1 || tiles > 128 || (M > 192 && K < 4096)) return 1;
-    const int64_t room = 512 / tiles, most = K / 512;
-    const int64_t n = room < most ? room : most;
-    return n < 2 ? 1 : n > 8 ? 8 : (int)n;
+// The parts in which a sum over K is formed: about 256 k each, eight at most, from K alone, so that a row has the same bits
+// whether the parts have workgroups of their own (fp32 sums in a workspace, one more launch) or one that takes them in turn.
+int ring_parts(int64_t K) { return K < 512 ? 1 : K < 2048 ? (int)(K / 256) : 8; }
+
+// Workgroups of their own while tiles of 64x64 leave half of the compute units idle, for short K only if all parts then
+// find an idle one (us, whole | in parts, weights from memory): 48 tiles [256,768] x K 768 19.6 | 13.7 and K 3072 65 | 23.5,
+// 54 tiles [568,384] x K 1016 24.5 | 16.0, 96 tiles [512,768] x K 768 19.6 | 18.9 and K 3072 65 | 31, 121 tiles of K 700 18.2 | 16.5,
+// 144 tiles of K 768 19.8 | 20.3, 256 tiles of K 1024 25.1 | 31.
+bool ring_split(int64_t M, int64_t N, int64_t K, int64_t batch) {
+    const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64), n = ring_parts(K);
+    return batch == 1 && n > 1 && tiles <= 128 && (tiles * n <= 256 || K >= 1024);
 }
 
-bool ring_sizes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb) {
-    return lda % 4 == 0 && ldb % 4 == 0 && M * K < 0x1FFFFFFF && N * K < 0x1FFFFFFF;
-}
+bool ring_sizes(int64_t M, int64_t N, int64_t K) { return M * K < 0x1FFFFFFF && N * K < 0x1FFFFFFF; }
 
 }  // namespace
 
@@ -395,21 +413,20 @@ bool gemm_f32_mfma_wanted(const GemmArgs& g) {
 }
 
 int64_t gemm_f32_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b) {
-    if (!ring_sizes(M, N, K, trans_a ? M : K, trans_b ? K : N)) return 0;
-    const int n = ring_splits(M, N, K, batch);
-    return n == 1 ? 0 : M * N * 4 * n;
+    if (!ring_sizes(M, N, K)) return 0;
+    return ring_split(M, N, K, batch) ? M * N * 4 * ring_parts(K) : 0;
 }
 
 // Without the workspace (g.partial), or with a smaller one, K is not split.
 int launch_gemm_f32_mfma(hipStream_t s, GemmArgs g, int64_t batch, int trans_a, int trans_b, int64_t workspace_bytes) {
-    const bool ring = ring_sizes(g.M, g.N, g.K, g.lda, g.ldb) && g.sa % 4 == 0 && g.sb % 4 == 0 &&
+    const bool ring = ring_sizes(g.M, g.N, g.K);
+    const bool wide = g.lda % 4 == 0 && g.ldb % 4 == 0 && g.sa % 4 == 0 && g.sb % 4 == 0 &&
                       ((reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.b)) & 15) == 0;
-    g.splits = ring && g.partial ? ring_splits(g.M, g.N, g.K, batch) : 1;
-    if ((int64_t)g.M * g.N * 4 * g.splits > workspace_bytes) g.splits = 1;
-    if (g.splits == 1) g.partial = nullptr;
-    const int st = !trans_a ? (!trans_b ? launch<false, false>(s, g, batch, ring) : launch<false, true>(s, g, batch, ring))
-                            : (!trans_b ? launch<true, false>(s, g, batch, ring) : launch<true, true>(s, g, batch, ring));
-    return st != MHIP_OK || g.splits == 1 ? st : launch_gemm_finish(s, g, MHIP_F32);
+    g.splits = ring_parts(g.K);
+    if (!ring || !ring_split(g.M, g.N, g.K, batch) || (int64_t)g.M * g.N * 4 * g.splits > workspace_bytes) g.partial = nullptr;
+    const int st = !trans_a ? (!trans_b ? launch<false, false>(s, g, batch, ring, wide) : launch<false, true>(s, g, batch, ring, wide))
+                            : (!trans_b ? launch<true, false>(s, g, batch, ring, wide) : launch<true, true>(s, g, batch, ring, wide));
+    return st != MHIP_OK || !g.partial ? st : launch_gemm_finish(s, g, MHIP_F32);
 }
 
 }  // namespace mhip

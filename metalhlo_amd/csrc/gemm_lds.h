@@ -25,6 +25,10 @@ __device__ inline __amdgpu_buffer_rsrc_t make_rsrc(const void* p, uint32_t bytes
 __device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t rsrc, uint32_t lds, uint32_t off) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(rsrc) : "memory");
 }
+// The same with 4 bytes per lane (lds a multiple of 4), for rows that start on no 16-byte boundary.
+__device__ __forceinline__ void load_dword_to_lds(__amdgpu_buffer_rsrc_t rsrc, uint32_t lds, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(rsrc) : "memory");
+}
 // LDS address of a shared-memory pointer, as those loads take it.
 __device__ __forceinline__ uint32_t lds_address(const char* p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p;

@@ -848,6 +848,14 @@ static std::vector<DeviceTensor> run_ops(Executable& exe, const std::vector<Devi
             out = al.allocate(op.out);
             const int dt = op.out.dtype;
             const int64_t cnt = op.out.numel();
+            // one product, with the memory that lets its K be split over idle compute units
+            auto gemm = [&](const void* a, const void* b, const void* bias, const void* residual, void* c, int64_t M, int64_t N, int64_t K, bool ta,
+                            bool tb, int act) {
+                const int64_t bytes = mhip_gemm_workspace(M, N, K, 1, ta, tb, dt);
+                DeviceTensor work;
+                if (bytes > 0) work = al.allocate(TensorType{{bytes}, UI8});
+                RUN(mhip_gemm_ws(s, a, b, bias, residual, c, M, N, K, 1, 0, 0, 0, ta, tb, act, dt, work.data(), bytes));
+            };
             if (kUnary.count(n)) {
                 RUN(mhip_unary(s, kUnary.at(n), in(0).data(), out.data(), cnt, dt));
             } else if (kBinary.count(n)) {
@@ -904,8 +912,9 @@ static std::vector<DeviceTensor> run_ops(Executable& exe, const std::vector<Devi
                 }
                 if (p.lhs_copy) a = permuted_copy(al, dry, s, a, p.lhs_perm, op);
                 if (p.rhs_copy) b = permuted_copy(al, dry, s, b, p.rhs_perm, op);
-                RUN(mhip_gemm(s, a.data(), b.data(), nullptr, out.data(), p.M, p.N, p.K, p.B, p.M * p.K, p.K * p.N,
-                                p.M * p.N, p.trans_a, p.trans_b, MHIP_ACT_NONE, dt));
+                if (p.B == 1) gemm(a.data(), b.data(), nullptr, nullptr, out.data(), p.M, p.N, p.K, p.trans_a, p.trans_b, MHIP_ACT_NONE);
+                else RUN(mhip_gemm(s, a.data(), b.data(), nullptr, out.data(), p.M, p.N, p.K, p.B, p.M * p.K, p.K * p.N,
+                                     p.M * p.N, p.trans_a, p.trans_b, MHIP_ACT_NONE, dt));
             } else if (n == "iota") {
                 int64_t outer = 1, inner = 1;
                 for (int64_t d = 0; d < (int64_t)op.out.shape.size(); d++) {
@@ -976,9 +985,9 @@ static std::vector<DeviceTensor> run_ops(Executable& exe, const std::vector<Devi
                     DeviceTensor hidden = al.allocate(TensorType{{rows, F}, dt});
                     // an activation name the handler does not know means no activation (CustomCallHandlers.swift:905)
                     const std::string act_name = cfg.get_string("activation", "gelu");
-                    RUN(mhip_gemm(s, in(0).data(), in(1).data(), nullptr, hidden.data(), rows, F, cols, 1, 0, 0, 0, 0, 0,
-                                  kActivation.count(act_name) ? kActivation.at(act_name) : MHIP_ACT_NONE, dt));
-                    RUN(mhip_gemm(s, hidden.data(), in(2).data(), nullptr, out.data(), rows, d2, F, 1, 0, 0, 0, 0, 0, MHIP_ACT_NONE, dt));
+                    gemm(in(0).data(), in(1).data(), nullptr, nullptr, hidden.data(), rows, F, cols, false, false,
+                         kActivation.count(act_name) ? kActivation.at(act_name) : MHIP_ACT_NONE);
+                    gemm(hidden.data(), in(2).data(), nullptr, nullptr, out.data(), rows, d2, F, false, false, MHIP_ACT_NONE);
                 } else if (op.target == "fused_layer_norm" || op.target == "fused_rms_norm") {
                     const auto axes = cfg.get_int_array("axes", {-1});
                     if (axes.size() != 1 || (axes[0] != -1 && axes[0] != (int64_t)xt.shape.size() - 1))
@@ -1007,8 +1016,8 @@ static std::vector<DeviceTensor> run_ops(Executable& exe, const std::vector<Devi
                     if (bias && (in(2).type.numel() != N || in(2).type.dtype != dt)) throw ExecError(where(op) + "bias must be [N] of the input type");
                     const DeviceTensor* res = has_res ? &in(op.operands.size() - 1) : nullptr;
                     if (res && !(res->type == op.out)) throw ExecError(where(op) + "the residual must have the result's type");
-                    RUN(mhip_gemm_residual(s, in(0).data(), in(1).data(), bias, res ? res->data() : nullptr, out.data(), M, N, K, 1, 0, 0, 0,
-                                           ta, tb, kActivation.at(cfg.get_string("activation", "none")), dt));
+                    gemm(in(0).data(), in(1).data(), bias, res ? res->data() : nullptr, out.data(), M, N, K, ta, tb,
+                         kActivation.at(cfg.get_string("activation", "none")));
                 } else if (!cfg.get_int_array("views", {}).empty()) {   // attention reading / writing views in place
                     const auto dims = cfg.get_int_array("dims", {});
                     const auto vw = cfg.get_int_array("views", {});

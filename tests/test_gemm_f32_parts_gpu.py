@@ -1,0 +1,42 @@
+"""fp32 products whose K is summed in parts: the same bits from workgroups of their own (with a workspace), from one that
+takes the parts in turn (without), from 128-wide tiles and from rows that start on no 16-byte boundary, around the K
+from which there are parts; values against float64 with the bound of tests/test_gemm_few_tiles_gpu.py."""
+import pytest
+import torch
+
+from metalhlo_amd import _lib, kernels
+from tests.test_gemm_few_tiles_gpu import _check
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("layout", [(False, False), (False, True), (True, False), (True, True)], ids=["nn", "nt", "tn", "tt"])
+@pytest.mark.parametrize("M,N,K", [(193, 65, 511), (201, 130, 512), (333, 129, 769), (257, 63, 2049), (1025, 131, 1030), (194, 97, 33)], ids=lambda v: str(v))
+def test_odd_rows(M, N, K, layout):
+    _check(M, N, K, torch.float32, *layout, residual=M % 2 == 0)
+
+
+@pytest.mark.parametrize("N,K", [(2048, 511), (2048, 600), (1000, 1536), (772, 3100), (130, 5000)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 1)])
+def test_parts_have_the_bits_of_the_whole(N, K, ta, tb):
+    lib, f32 = _lib.load(), kernels.DTYPE_CODE[torch.float32]
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    rows = 200
+    x, w = torch.randn(8000, K, generator=g, device="cuda"), torch.randn(N * K + 1, generator=g, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def product(M, odd, parts):
+        a = (x[:M].t() if ta else x[:M]).contiguous()
+        b = w[1:] if odd else w[1:].clone()
+        out = torch.empty(M, N, device="cuda")
+        n = lib.mhip_gemm_workspace(M, N, K, 1, ta, tb, f32) if parts else 0
+        work = torch.empty(n, dtype=torch.uint8, device="cuda") if n else None
+        assert lib.mhip_gemm_ws(stream, a.data_ptr(), b.data_ptr(), None, None, out.data_ptr(), M, N, K, 1, 0, 0, 0, ta, tb, 0, f32,
+                                work.data_ptr() if n else None, n) == 0
+        return out, n
+
+    whole, _ = product(rows, False, False)
+    split, n = product(rows, False, True)
+    assert (n > 0) == (K >= 512) and torch.equal(split, whole)
+    assert torch.equal(product(rows, True, True)[0], whole)
+    assert torch.equal(product(8000, False, True)[0][:rows], whole)
