@@ -81,7 +81,10 @@ template <typename T, int VE, bool VEC> struct RowPiece {
         if (VEC) {
             const uint32_t o = n > 0 ? (uint32_t)(off * (int)sizeof(T)) : kOob;
             if (kDw == 1) w[0] = __builtin_amdgcn_raw_buffer_load_b32(r, o, 0, 0);
-            else {
+            else if (kDw == 3) {
+                const auto t = __builtin_amdgcn_raw_buffer_load_b96(r, o, 0, 0);
+                w[0] = t[0]; w[1 % kDw] = t[1]; w[kDw - 1] = t[2];
+            } else {
                 const u32x2 t = __builtin_amdgcn_raw_buffer_load_b64(r, o, 0, 0);
                 w[0] = t.x; w[kDw - 1] = t.y;
             }
@@ -281,13 +284,26 @@ int launch_shape(hipStream_t s, const GemmArgs& g, int64_t batch) {
     constexpr bool k16 = sizeof(T) == 2;
     const bool wide = wide_strips(g.N, g.K, batch, TB);
     if constexpr (!k16) {
-        // fp32 from 33 rows on: blocks of 32 rows by 16 columns until every compute unit has one, beyond that by 32 columns
-        // unless the strips are wide, whose blocks of 64 rows read B half as often.  us, 32 x 16 / 32 x 32 / 64 rows:
-        // [128,768] x K 768 (192 of the first) 6.7 / 9.1 / 10.0 and K 3072 15.9 / 21.2 / 27.1, [64,2304] x K 768 (288)
-        // 10.0 / 9.2 / 10.1, [128,4096] x K 1024 (1024) 23.0 / 18.9 / 23.1, [64,8192] x K 4096 (wide) - / 59.1 / 52.3.  Up to
-        // 64 rows a split K fills the device as it is: [36,768] x K 8192 24.4 / - / 20.8.
+        // fp32 from 33 rows on: the block of rows by columns that leaves no compute unit a second turn, since a unit takes about 30
+        // bytes a nanosecond of a matrix from memory; beyond that 32 by 32, unless the strips are wide, whose blocks of 64 rows
+        // read B half as often.  Weights from memory, us (workgroups):
+        //                        32 x 16       16 x 48       32 x 32       32 x 48
+        //   [128,768] x K 768      7.0 (192)     8.0 (128)     9.3 (96)     11.2 (64)
+        //   [100,1536] x K 512     7.9 (384)     6.5 (224)     7.4 (192)     8.9 (128)
+        //   [64,3072] x K 1024    12.9 (384)     9.7 (256)    11.0 (192)    13.4 (128)
+        //   [192,768] x K 3072    28.6 (288)    19.0 (192)    22.4 (144)    28.3 (96)
+        //   [100,2048] x K 512     8.0 (512)    10.1 (301)     7.5 (256)     9.7 (172)
+        //   [128,2304] x K 768    13.6 (576)    11.8 (384)    13.9 (288)    11.3 (192)
+        //   [128,3072] x K 1024   17.2 (768)    14.9 (512)    17.4 (384)    13.5 (256)
+        //   [192,2304] x K 768    16.5 (864)    16.3 (576)    14.4 (432)    17.5 (288)
+        // Wide: [64,8192] x K 4096 59.1 in 32 x 32, 52.3 in 64 rows.  Up to 64 rows a split K fills the device as it is:
+        // [36,768] x K 8192 24.4 in 32 x 16, 20.8 in 64 rows.  (Stored [K, N] a strip of 48 columns is three per lane.)
         if (g.M > 32 && (g.M > 64 || g.splits == 1)) {
-            if ((g.N + 15) / 16 * ((g.M + 31) / 32) * batch <= 256) return launch_one<T, TB, VEC, 1, 2, 2>(s, g, batch);
+            auto blocks = [&](int rows, int cols) { return (int64_t)((g.M + rows - 1) / rows) * ((g.N + cols - 1) / cols) * batch; };
+            constexpr bool k48 = VEC && !TB;
+            if (blocks(32, 16) <= 256) return launch_one<T, TB, VEC, 1, 2, 2>(s, g, batch);
+            if constexpr (k48) if (blocks(16, 48) <= 256) return launch_one<T, TB, VEC, 3, 1, 2>(s, g, batch);
+            if constexpr (k48) if (blocks(32, 32) > 256 && blocks(32, 48) <= 256) return launch_one<T, TB, VEC, 3, 2, 2>(s, g, batch);
             if (!wide) return launch_one<T, TB, VEC, 2, 2, 2>(s, g, batch);
         }
     }

@@ -40,3 +40,9 @@ def test_parts_have_the_bits_of_the_whole(N, K, ta, tb):
     assert (n > 0) == (K >= 512) and torch.equal(split, whole)
     assert torch.equal(product(rows, True, True)[0], whole)
     assert torch.equal(product(8000, False, True)[0][:rows], whole)
+
+
+@pytest.mark.parametrize("M,N,K", [(33, 2308, 20), (48, 3068, 132), (100, 1540, 516), (65, 2308, 36), (128, 3076, 772), (192, 772, 1028), (128, 2304, 3072)], ids=lambda v: str(v))
+def test_strips_of_48_columns(M, N, K):
+    """Few-row products whose strips are three columns a lane, the last strip ragged."""
+    _check(M, N, K, torch.float32, False, False, residual=M % 2 == 0)
