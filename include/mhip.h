@@ -170,6 +170,11 @@ int mhip_linear_w32_parts(int64_t M, int64_t N, int64_t K);
 int mhip_linear_w32(void* stream, const void* x, const float* w, const float* bias, const void* residual, void* c, int64_t M,
                     int64_t N, int64_t K, int trans_b, int activation, int dtype, float* sums, int parts, int n_ahead,
                     const mhip_weights* ahead);
+/* The fp32 sums of `parts` shares of K (up to 8), sums[parts][M][N], of a [M,K] . b [K,N] in BF16 or F16, for mhip_finish_norm.
+ * mhip_gemm_sums_parts gives a good number of parts for the sizes, 0 where they are not served (N and K multiples of
+ * 8).  16-byte aligned pointers.  The last bits of a row may change with the number of rows. */
+int mhip_gemm_sums_parts(int64_t M, int64_t N, int64_t K, int dtype);
+int mhip_gemm_sums(void* stream, const void* a, const void* b, float* sums, int64_t M, int64_t N, int64_t K, int dtype, int parts);
 /* c = round(sum of sums[parts][M][N] + round(bias)) + residual, or with parts = 0 (sums NULL) the residual itself, and
  * h = LayerNorm(c; gamma, beta, eps) over its rows.  c may be NULL; bias and residual may be NULL where there are parts.
  * Parameters fp32, the rest of `dtype` (BF16 or F16); N a multiple of 8 up to 4096; 16-byte aligned pointers. */

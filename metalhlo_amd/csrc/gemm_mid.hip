@@ -61,7 +61,7 @@ struct StageLoader {
 // KG groups of four waves: a stage is KG x 64 k, group q multiplies its 64, the groups' sums meet in LDS at the
 // end.  S stages in the ring.
 template <typename T, int BM, int BN, int WGM, bool TA, bool TB, int KG, int S, bool AHEAD>
-__global__ __launch_bounds__(256 * KG) void gemm_mid_kernel(GemmArgs g) {
+__global__ __launch_bounds__(256 * KG) void gemm_mid_kernel(GemmArgs g, int sums_by_row) {
     constexpr int WGN = 4 / WGM, WTM = BM / WGM, WTN = BN / WGN, TM = WTM / 32, TN = WTN / 32;
     constexpr int kATile = BM * kRowBytes, kPart = (BM + BN) * kRowBytes, kStage = KG * kPart;
     extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -169,6 +169,17 @@ __global__ __launch_bounds__(256 * KG) void gemm_mid_kernel(GemmArgs g) {
             __syncthreads();
         }
         if (group > 0) return;
+    }
+    if (g.partial && sums_by_row) {
+        // [part][M][N]: a lane's row, four columns per store (two lanes' stores are 32 consecutive bytes)
+        float* p = g.partial + (int64_t)blockIdx.z * g.M * g.N;
+#pragma unroll
+        for (int x = 0; x < TM * TN * 4; x++) {
+            const f32x16& t = acc[x / 4 / TN][x / 4 % TN];
+            const int m = m0 + wm * WTM + x / 4 / TN * 32 + lrow, n = n0 + wn * WTN + x / 4 % TN * 32 + 8 * (x % 4) + 4 * (lane >> 5);
+            if (m < g.M && n < g.N) *reinterpret_cast<f32x4*>(p + (int64_t)m * g.N + n) = f32x4{t[4 * (x % 4)], t[4 * (x % 4) + 1], t[4 * (x % 4) + 2], t[4 * (x % 4) + 3]};
+        }
+        return;
     }
     if (g.partial) {
         // the block's registers as they are, 1 KB per store: block (i, j) of wave w of tile t, register group q
@@ -306,7 +317,7 @@ __global__ __launch_bounds__(256) void gemm_finish_kernel(GemmArgs g) {
 }
 
 template <typename T, int BM, int BN, int WGM, bool TA, bool TB, int KG, int S, bool AHEAD = false>
-int launch_tile(hipStream_t s, GemmArgs g, int64_t batch) {
+int launch_tile(hipStream_t s, GemmArgs g, int64_t batch, bool by_row) {
     constexpr int kStage = KG * (BM + BN) * kRowBytes, kRing = S * kStage, kSums = KG / 2 * BM * BN * 4, kOut = 4 * (BM / WGM) * ((BN / (4 / WGM)) * 2 + 16);
     constexpr int kUse = kRing > kOut ? kRing : kOut, kSmem = kUse > kSums ? kUse : kSums;
     static_assert(kSmem <= 160 * 1024, "ring larger than LDS");
@@ -319,7 +330,7 @@ int launch_tile(hipStream_t s, GemmArgs g, int64_t batch) {
     g.tiles_n = (g.N + BN - 1) / BN;
     const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n;
     if (tiles > 0x7FFFFFFFLL || batch > 65535) return fail(MHIP_ERR_UNSUPPORTED, "gemm: grid too large");
-    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)batch, (unsigned)g.splits), dim3(256 * KG), kSmem, s, g);
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)batch, (unsigned)g.splits), dim3(256 * KG), kSmem, s, g, by_row ? 1 : 0);
     return check_launch("gemm_mid");
 }
 
@@ -371,25 +382,38 @@ MidPlan plan_mid(int64_t M, int64_t N, int64_t K, int64_t batch, bool ring_ok, b
     return best;
 }
 
+// The same for sums that another launch adds up in any case (mhip_gemm_sums): no order to keep, no launch of its own.
+MidPlan plan_sums(int64_t M, int64_t N, int64_t K, int parts) {
+    MidPlan best;
+    float t_best = 1e30f;
+    for (int f = 0; f < kRing192; f++)
+        for (int s = parts ? parts : 1; s <= (parts ? parts : kMaxSplits); s++) {
+            if (!parts && s > 1 && K / s < 256) break;
+            const float t = form_cost(kForms[f], M, N, K, 1, s) + (s == 1 ? (float)(M * N) * 8e-6f / 5.f : -3.f);
+            if (t < t_best) { t_best = t; best.form = f; best.splits = s; }
+        }
+    return best;
+}
+
 int64_t plan_bytes(const MidPlan& p, int64_t M, int64_t N) {
     const Form& f = kForms[p.form];
     return p.splits == 1 ? 0 : ((M + f.bm - 1) / f.bm) * ((N + f.bn - 1) / f.bn) * f.bm * f.bn * 4 * p.splits;
 }
 
 template <typename T, bool TA, bool TB>
-int launch_form(hipStream_t s, const GemmArgs& g, int64_t batch, int form) {
+int launch_form(hipStream_t s, const GemmArgs& g, int64_t batch, int form, bool by_row = false) {
     // one workgroup per compute unit or fewer: all of LDS for a ring of four that reads ahead; otherwise the ring that two
     // workgroups of a unit share ([2000,2000] x K 2000, 256 of 128x128, 29.7 -> 26.6 us; [1000,3000] x K 1000, 384 of 64x128,
     // 16.4 against 20.2; tiles of 64x64 lose by it, [1000,1000] x K 1000 7.9 against 8.6)
     const Form& f = kForms[form];
     const bool one_each = ((g.M + f.bm - 1) / f.bm) * (int64_t)((g.N + f.bn - 1) / f.bn) * batch * g.splits <= 256;
     switch (form) {
-        case 0: return launch_tile<T, 64, 64, 2, TA, TB, 2, 3>(s, g, batch);
-        case 1: return launch_tile<T, 64, 128, 2, TA, TB, 2, 3>(s, g, batch);
-        case 2: return launch_tile<T, 128, 128, 2, TA, TB, 2, 2>(s, g, batch);
-        case 3: return launch_tile<T, 64, 64, 2, TA, TB, 1, 4>(s, g, batch);
-        case 4: return one_each ? launch_tile<T, 64, 128, 2, TA, TB, 1, 4, true>(s, g, batch) : launch_tile<T, 64, 128, 2, TA, TB, 1, 3>(s, g, batch);
-        default: return one_each ? launch_tile<T, 128, 128, 2, TA, TB, 1, 4, true>(s, g, batch) : launch_tile<T, 128, 128, 2, TA, TB, 1, 2>(s, g, batch);
+        case 0: return launch_tile<T, 64, 64, 2, TA, TB, 2, 3>(s, g, batch, by_row);
+        case 1: return launch_tile<T, 64, 128, 2, TA, TB, 2, 3>(s, g, batch, by_row);
+        case 2: return launch_tile<T, 128, 128, 2, TA, TB, 2, 2>(s, g, batch, by_row);
+        case 3: return launch_tile<T, 64, 64, 2, TA, TB, 1, 4>(s, g, batch, by_row);
+        case 4: return one_each ? launch_tile<T, 64, 128, 2, TA, TB, 1, 4, true>(s, g, batch, by_row) : launch_tile<T, 64, 128, 2, TA, TB, 1, 3>(s, g, batch, by_row);
+        default: return one_each ? launch_tile<T, 128, 128, 2, TA, TB, 1, 4, true>(s, g, batch, by_row) : launch_tile<T, 128, 128, 2, TA, TB, 1, 2>(s, g, batch, by_row);
     }
 }
 
@@ -447,3 +471,23 @@ int launch_gemm_finish(hipStream_t s, const GemmArgs& g, int dtype) {
 }
 
 }  // namespace mhip
+
+using namespace mhip;
+
+extern "C" int mhip_gemm_sums_parts(int64_t M, int64_t N, int64_t K, int dtype) {
+    if ((dtype != MHIP_BF16 && dtype != MHIP_F16) || M < 1 || N < 1 || K < 1 || N % 8 != 0 || K % 8 != 0) return 0;
+    if (M > 0x7FFFFFFF || N > 0x7FFFFFFF || K > 0x7FFFFFFF || M * K * 2 >= 0x7FFFFFFFLL || N * K * 2 >= 0x7FFFFFFFLL) return 0;
+    return plan_sums(M, N, K, 0).splits;
+}
+
+extern "C" int mhip_gemm_sums(void* stream, const void* a, const void* b, float* sums, int64_t M, int64_t N, int64_t K, int dtype, int parts) {
+    if (!a || !b || !sums || parts < 1 || parts > kMaxSplits) return fail(MHIP_ERR_INVALID_ARGUMENT, "mhip_gemm_sums: NULL pointer, or not 1 to 8 parts");
+    if (!mhip_gemm_sums_parts(M, N, K, dtype) || ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(sums)) & 15) != 0)
+        return fail(MHIP_ERR_UNSUPPORTED, "mhip_gemm_sums: [%lld,%lld] x K %lld, dtype %d, or pointers off 16 bytes", (long long)M, (long long)N, (long long)K, dtype);
+    GemmArgs g = {};
+    g.a = a; g.b = b; g.partial = sums;
+    g.M = (int)M; g.N = (int)N; g.K = (int)K; g.lda = (int)K; g.ldb = (int)N;
+    const MidPlan p = plan_sums(M, N, K, parts);
+    g.splits = p.splits;
+    return dtype == MHIP_BF16 ? launch_form<bf16_t, false, false>(as_stream(stream), g, 1, p.form, true) : launch_form<f16_t, false, false>(as_stream(stream), g, 1, p.form, true);
+}

@@ -273,6 +273,21 @@ FUNCTION(linear) {
     });
 }
 
+// matmul_sums(a, b, parts) -> [parts, M, N] fp32
+FUNCTION(matmul_sums) {
+    return guarded(n, 3, [&] {
+        const at::Tensor &a = dense(arg[0]), &b = dense(arg[1]);
+        const int64_t parts = integer(arg[2]);
+        if (a.dim() != 2 || b.dim() != 2 || a.size(1) != b.size(0)) raise(PyExc_ValueError, "matmul_sums needs [M, K] and [K, N]");
+        if (a.scalar_type() != b.scalar_type()) raise(PyExc_TypeError, "operand dtypes differ");
+        if (parts < 1 || parts > 8) raise(PyExc_ValueError, "1 to 8 parts");
+        const int dt = dtype_code(a.scalar_type());
+        at::Tensor c = empty({parts, a.size(0), b.size(1)}, at::kFloat, a);
+        check([&] { return mhip_gemm_sums(stream_of(a), a.data_ptr(), b.data_ptr(), c.data_ptr<float>(), a.size(0), b.size(1), a.size(1), dt, (int)parts); });
+        return THPVariable_Wrap(std::move(c));
+    });
+}
+
 // finish_norm(sums or None, bias, residual, gamma, beta, eps) -> (c, LayerNorm(c)); without sums c is the residual
 FUNCTION(finish_norm) {
     return guarded(n, 6, [&]() -> PyObject* {
@@ -390,7 +405,7 @@ FUNCTION(bind) {
 }
 
 #define ENTRY(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
-PyMethodDef kMethods[] = {ENTRY(softmax), ENTRY(layer_norm), ENTRY(rms_norm), ENTRY(bias_gelu), ENTRY(matmul), ENTRY(linear), ENTRY(finish_norm), ENTRY(causal_attention),
+PyMethodDef kMethods[] = {ENTRY(softmax), ENTRY(layer_norm), ENTRY(rms_norm), ENTRY(bias_gelu), ENTRY(matmul), ENTRY(linear), ENTRY(matmul_sums), ENTRY(finish_norm), ENTRY(causal_attention),
                           ENTRY(flash_attention), ENTRY(argmax), ENTRY(bind), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

@@ -60,7 +60,7 @@ class GPT2:
             off = sum(x.size for x in flat)
             pad = (-a.size) % 8
             flat.append(np.concatenate([a.reshape(-1), np.zeros(pad, np.float32)]))
-            self._slots.append((path, off, a.shape))
+            self._slots.append((path, off, tuple(a.shape)))
 
         # the tied output head multiplies by wte^T: rows padded with zeros to a multiple of 64
         # keep that GEMM on the aligned kernels; "wte" is the view of the real rows
@@ -79,7 +79,7 @@ class GPT2:
     def _views(self, flat: torch.Tensor) -> Dict:
         out: Dict = {"layers": [dict() for _ in range(self.cfg.n_layer)]}
         for path, off, shape in self._slots:
-            v = flat[off:off + int(np.prod(shape))].view(*shape)
+            v = torch.as_strided(flat, shape, (shape[1], 1) if len(shape) == 2 else (1,), off)
             if path[0] == "layers":
                 out["layers"][path[1]][path[2]] = v
             else:
@@ -87,17 +87,31 @@ class GPT2:
         return out
 
     def forward(self, ids: torch.Tensor) -> torch.Tensor:
-        """ids int32 [B,S] on the device -> logits [B,S,vocab] in the compute type."""
+        """ids int32 [B,S] on the device -> logits [B,S,vocab] in the compute type.  With more than 768 tokens in all a
+        sequence has the same bits in any batch; below that fp32 sums are split by the number of tokens."""
         cfg = self.cfg
         B, S = ids.shape
         d, H = cfg.d_model, cfg.n_head
         if self._few_tokens(B * S):
             return self._forward_few(ids)
+        o_parts, p_parts = self._sum_parts(B * S)
         # the graph's `convert` ops: fp32 parameters -> compute type, every step
         p = self.p32 if self.dtype == torch.float32 else self._views(kernels.convert(self.flat32, self.dtype))
         x = kernels.embed_tokens(ids, self.p32["wte"], self.p32["wpe"], self.dtype).reshape(B * S, d)
         # the strided attention entry covers 16-bit types and head sizes 64 / 128
         in_place = self.dtype in (torch.bfloat16, torch.float16) and d // H in (64, 128)
+        if o_parts:
+            # K of the layers in front of a residual over the whole device; the launch that adds the parts up forms the next LayerNorm
+            layers = self.p32["layers"]
+            norms = [(l["ln1_g"], l["ln1_b"], 1e-5) for l in layers] + [(self.p32["lnf_g"], self.p32["lnf_b"], 1e-5)]
+            x, h = kernels.finish_norm(None, None, x, norms[0])
+            for l, l32, norm in zip(p["layers"], layers, norms[1:]):
+                a = kernels.causal_attention(kernels.matmul(h, l["w_qkv"], bias=l["b_qkv"]), B, H)
+                x, h = kernels.finish_norm(kernels.matmul_sums(a, l["w_o"], o_parts), l32["b_o"], x, (l32["ln2_g"], l32["ln2_b"], 1e-5))
+                u = kernels.matmul(h, l["w_fc"], bias=l["b_fc"], activation="gelu")
+                x, h = kernels.finish_norm(kernels.matmul_sums(u, l["w_proj"], p_parts), l32["b_proj"], x, norm)
+            logits = kernels.matmul(h, p["wte_pad"], trans_b=True)
+            return logits.reshape(B, S, self.vocab_pad)[..., :cfg.vocab]
         for l in p["layers"]:
             h = kernels.layer_norm(x, l["ln1_g"], l["ln1_b"], eps=1e-5)
             qkv = kernels.matmul(h, l["w_qkv"], bias=l["b_qkv"])
@@ -125,7 +139,26 @@ class GPT2:
         d, f, dt = self.cfg.d_model, self.cfg.d_ff, self.dtype
         if dt not in (torch.bfloat16, torch.float16) or d // self.cfg.n_head not in (64, 128) or d % self.cfg.n_head:
             return False
+        # (each 64 rows read a matrix again: three times from memory cost more than converting it, 150 tokens 784 us against 669,
+        # 128 tokens 692 against 669, 96 tokens 627 against 647, replayed; a matrix of up to 4 MB stays in an L2)
+        if tokens > 128 and 4 * d * f > 4 << 20:
+            return False
         return d <= 4096 and all(kernels.linear_served(tokens, n, k, dt) for n, k in ((3 * d, d), (d, d), (f, d), (d, f), (self.vocab_pad, d)))
+
+    # 64x64 tiles of the layers in front of a residual from which on they fill the device whole
+    # (us whole and in parts, replayed: 193 tokens 813 and 679, 300 842 and 721, 576 952 and 875, 768 (144 tiles) 1109 and 1050;
+    # 1024 (192 tiles) 1233 and 1218, which leaves a sequence of full length its bits in any batch)
+    _full_tiles = 144
+
+    def _sum_parts(self, tokens: int):
+        """Shares of K for the two layers in front of a residual, (0, 0) where their tiles fill the device without."""
+        d, f = self.cfg.d_model, self.cfg.d_ff
+        if d // self.cfg.n_head not in (64, 128) or d % self.cfg.n_head or d > 4096 or -(-tokens // 64) * -(-d // 64) > self._full_tiles:
+            return 0, 0
+        if self.dtype not in (torch.bfloat16, torch.float16):
+            return 0, 0
+        parts = tuple(kernels.matmul_sums_parts(tokens, d, k, self.dtype) for k in (d, f))
+        return parts if all(parts) else (0, 0)
 
     def _forward_few(self, ids: torch.Tensor) -> torch.Tensor:
         """The same operators for a short prompt: the parameters are rounded to the compute type where they are read

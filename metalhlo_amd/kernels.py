@@ -119,6 +119,16 @@ def linear_parts(M: int, N: int, K: int) -> int:
     return _lib.load().mhip_linear_w32_parts(M, N, K)
 
 
+def matmul_sums(a, b, parts: int):
+    """The fp32 sums of so many shares of K of a [M, K] @ b [K, N] in a 16-bit type: [parts, M, N], for finish_norm."""
+    return (_native or _host()).matmul_sums(a, b, parts)
+
+
+def matmul_sums_parts(M: int, N: int, K: int, dtype) -> int:
+    """A good number of parts for these sizes, 0 where matmul_sums does not serve them."""
+    return _lib.load().mhip_gemm_sums_parts(M, N, K, DTYPE_CODE[dtype])
+
+
 def finish_norm(sums, bias, residual, norm):
     """(c, LayerNorm(c)) with c = round(sums.sum(0) + bias) + residual, or c = residual where sums is None; fp32 parameters."""
     return (_native or _host()).finish_norm(sums, bias, residual, *norm)
