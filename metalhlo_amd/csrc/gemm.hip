@@ -303,7 +303,7 @@ int launch_gemm_any(hipStream_t s, GemmArgs g, int64_t batch, int trans_a, int t
 int64_t gemm_any_workspace(int64_t M, int64_t N, int64_t K, int64_t batch);
 int launch_gemm_skinny(hipStream_t s, GemmArgs g, int64_t batch, int trans_b, int dtype, int64_t workspace_bytes);
 // gemm_mid.hip: 64- and 128-row tiles through a ring of LDS stages, K split where that leaves units idle.
-int64_t gemm_mid_workspace(int64_t M, int64_t N, int64_t K, int64_t batch);
+int64_t gemm_mid_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b);
 int launch_gemm_mid(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_a, int trans_b, int dtype, int64_t workspace_bytes);
 // gemm_f32.hip: fp32 operands on the fp32 matrix instruction, 128x128 tiles.
 bool gemm_f32_mfma_wanted(const GemmArgs& g);
@@ -441,11 +441,11 @@ static int pick_tile(hipStream_t s, const GemmArgs& g, int64_t batch, int64_t wo
     const int64_t narrow_cost = ((narrow + cus - 1) / cus) * (stages * 18 + 500);
     // (wide tiles on the columns that make whole rounds + one round of a narrow band, where the default takes that form)
     int n_split = 0;
-    const bool split_ok = gemm_split_shape(g, batch, &n_split) && narrow > 2 * cus;
+    const bool split_ok = g.K % 32 == 0 && gemm_split_shape(g, batch, &n_split) && narrow > 2 * cus;
     const int64_t split_cost = split_ok ? (tiles_m * (n_split / 256) / cus) * (stages * 32 + 700) + (stages * 18 + 500) : ((int64_t)1 << 62);
     const bool wider_ok = gemm256_eligible(g, batch, TA, TB, dt, 384) && gemm384_activation_ok(g.act);
     const int64_t wider_cost = ((tiles_m * ((g.N + 383) / 384) * batch + cus - 1) / cus) * (stages * 53 + 1050);
-    if (force == 0 && g.K >= 512 && gemm256_eligible(g, batch, TA, TB, dt, 192)) {
+    if (force == 0 && g.K >= 512 && g.K % 32 == 0 && gemm256_eligible(g, batch, TA, TB, dt, 192)) {
         // The 128x192 tile where 256-row tiles leave compute units idle: its stage moves 20 KB
         // from the L2s against the narrow tile's 24 and costs 14 slots, the ends 500 -- fitted to
         // [8192,3072] x [3072,768] (256 tiles of it against 192 narrow ones: 46.4 us against 53.5
@@ -646,5 +646,5 @@ extern "C" int64_t mhip_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t 
     if (!is16) return gemm_f32_workspace(M, N, K, batch, trans_a, trans_b);
     if (!vec) return short_product(M, N, K) ? 0 : gemm_any_workspace(M, N, K, batch);
     if (M > 192 && (double)M * N * batch >= 192.0 * 256 * 256) return 0;
-    return gemm_mid_workspace(M, N, K, batch);
+    return gemm_mid_workspace(M, N, K, batch, trans_a, trans_b);
 }

@@ -330,7 +330,8 @@ int family256(hipStream_t s, const GemmArgs& g, int64_t batch, int ta, int tb, i
 // tiles (256 x `bw`) to occupy the device.
 bool gemm256_eligible(const GemmArgs& g, int64_t batch, int trans_a, int trans_b, int dtype, int bw, bool any_tile_count) {
     if (dtype != MHIP_BF16 && dtype != MHIP_F16) return false;
-    if (g.K % 32 != 0 || g.K < 32) return false;
+    // (the 128x192 kernel multiplies the rest of K behind its loop where k is the slow axis of both operands)
+    if ((g.K % 32 != 0 && !(bw == 192 && trans_a && !trans_b)) || g.K < 32) return false;
     if ((reinterpret_cast<uintptr_t>(g.c) & 15) != 0 || (batch > 1 && g.sc % 8 != 0)) return false;
     if (g.residual && (reinterpret_cast<uintptr_t>(g.residual) & 15) != 0) return false;
     if (g.bias && (reinterpret_cast<uintptr_t>(g.bias) & 7) != 0) return false;

@@ -375,6 +375,7 @@ MidPlan plan_mid(int64_t M, int64_t N, int64_t K, int64_t batch, bool ring_ok, b
         for (int s = 1; s <= (may_split && batch == 1 && !in_order ? kMaxSplits : 1); s++) {
             if (s > 1 && K / s < 256) break;
             float t = form_cost(kForms[f], M, N, K, batch, s);
+            if (f == kRing192 && K % 32 != 0) t += 1.5f;             // (the rest of K: one load latency more)
             if (s > 1) t *= 1.08f;
             if (t < t_best) { t_best = t; best.form = f; best.splits = s; }
         }
@@ -448,8 +449,8 @@ int launch_plan(hipStream_t s, GemmArgs g, int64_t batch, int ta, int tb, int dt
 }  // namespace
 
 // Bytes of workspace the choice for this problem can use (0 = none); a function of the sizes alone.
-int64_t gemm_mid_workspace(int64_t M, int64_t N, int64_t K, int64_t batch) {
-    return plan_bytes(plan_mid(M, N, K, batch, K % 32 == 0, true), M, N);
+int64_t gemm_mid_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b) {
+    return plan_bytes(plan_mid(M, N, K, batch, K >= 32 && (K % 32 == 0 || (trans_a && !trans_b)), true), M, N);
 }
 
 // 16-bit operands with 16-byte-aligned rows (the caller has checked).  `workspace` (g.partial) may be absent or

@@ -3,6 +3,7 @@
 // registers, the 128x192 tile for problems with few columns, and the 256x128 tile in 256 registers a wave
 // for two workgroups per compute unit.  Operand layouts and the epilogue of the narrow tile are those of
 // gemm256.hip (gemm_ring.h).
+#include "gemm_lds.h"
 #include "gemm_ring.h"
 
 namespace mhip {
@@ -477,8 +478,48 @@ __device__ __forceinline__ void store_partial192(f32x16 (&acc)[6], float* p, int
     });
 }
 
-// SPLIT: the grid's second axis is the part of K (g.splits of them, whole stages) instead of the batch, and
-// the tile's sums go to g.partial.
+// The last K % 32 k of the 128x192 tile where both operands have k as the slow axis (x^T dy over any number of tokens), which
+// the loop's whole stages leave: one stage of its own in the layout of gemm_mid.hip (what lies past K reads zero),
+// multiplied behind the loop in the order of k.  It waits out one load latency.  us on gemm_mid.hip's tiles | here:
+// [2944,2880] x K 1522 41.9 | 36.7, [768,3072] x K 8200 86.7 | 59.7, [6000,1504] x K 1007 32.7 | 31.5.  (Operands with k
+// contiguous lose by it, [1768,1768] x K 1768 with B stored [N, K] 22.0 | 29.4, [1000,3000] x K 1000 15.5 | 17.1.)
+template <int ROWS>
+__device__ __forceinline__ void load_tail(__amdgpu_buffer_rsrc_t rsrc, uint32_t tile, int col0, int cols_total, int ld, int k0, int K, int wave, int lane) {
+#pragma unroll
+    for (int i = 0; i < ROWS * 64 / 4096; i++) {
+        const int p = (i * 4 + wave) * 64 + lane, k = p / (ROWS / 8);       // 16-byte slot of the tile, its row
+        const int col = col0 + (p % (ROWS / 8) ^ mn_swz<ROWS>(k)) * 8;
+        load_to_lds(rsrc, tile + (uint32_t)(i * 4 + wave) * 1024u, col < cols_total && k0 + k < K ? (uint32_t)(((int64_t)(k0 + k) * ld + col) * 2) : kOob);
+    }
+}
+
+template <typename T>
+__device__ __forceinline__ void add_tail192(f32x16 (&acc)[6], char* smem, uint32_t lds0, const GemmArgs& g, __amdgpu_buffer_rsrc_t rsa,
+                                            __amdgpu_buffer_rsrc_t rsb, int m0, int n0, int k0, int K) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave >> 1, wn = wave & 1;
+    constexpr uint32_t kB = 128 * 64;
+    load_tail<128>(rsa, lds0, m0, g.M, g.lda, k0, K, wave, lane);
+    load_tail<256>(rsb, lds0 + kB, n0, min(g.N, n0 + 192), g.ldb, k0, K, wave, lane);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+        u32x4 af[2], bf[3];
+#pragma unroll
+        for (int i = 0; i < 2; i++) af[i] = frag_mn<128>(smem, wm * 64 + 32 * i, s, lane);
+#pragma unroll
+        for (int j = 0; j < 3; j++) bf[j] = frag_mn<256>(smem + kB, wn * 96 + 32 * j, s, lane);
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 3; j++) acc[3 * i + j] = Mfma32<T>::run(bf[j], af[i], acc[3 * i + j]);
+    }
+    __syncthreads();                                        // the epilogue writes where other waves read
+}
+
+// SPLIT: the grid's second axis is the part of K (g.splits of them, whole stages, the last one with the rest of K)
+// instead of the batch, and the tile's sums go to g.partial.
 template <typename T, bool TA, bool TB, bool SPLIT>
 __global__ __launch_bounds__(256) void gemm192_kernel(GemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -489,7 +530,7 @@ __global__ __launch_bounds__(256) void gemm192_kernel(GemmArgs g) {
     tile_of(blockIdx.x, gridDim.x, g.tiles_m, g.tiles_n, tm, tn);
     const int m0 = tm * 128, n0 = tn * 192;
     const int64_t batch = SPLIT ? 0 : blockIdx.y;
-    const int stages = g.K / 32, per = SPLIT ? (stages + g.splits - 1) / g.splits : stages;
+    const int stages = g.K / 32, rest = g.K % 32, per = SPLIT ? (stages + (rest != 0) + g.splits - 1) / g.splits : stages;
     const int first = SPLIT ? (int)blockIdx.y * per : 0, kt = min(per, stages - first);
     // (elements of a k-contiguous / a k-slow operand in front of this part)
     const int64_t skip_a = (int64_t)first * 32 * (TA ? g.lda : 1), skip_b = (int64_t)first * 32 * (TB ? 1 : g.ldb);
@@ -520,6 +561,8 @@ __global__ __launch_bounds__(256) void gemm192_kernel(GemmArgs g) {
     f32x16 acc[6];
     main_loop192<T, TA, TB>(acc, ra, rb, goff, rsa, rsb, LA::pass_stride(g.lda), LB::pass_stride(g.ldb),
                             LA::stage_stride(g.lda), LB::stage_stride(g.ldb), m0b, (uint32_t)kt);
+    if constexpr (TA && !TB)
+        if (rest && (!SPLIT || first + per > stages)) add_tail192<T>(acc, smem, lds0, g, rsa, rsb, m0, n0, kt * 32, kt * 32 + rest);
     if constexpr (SPLIT) store_partial192(acc, g.partial, ((int)blockIdx.y * g.tiles_m + tm) * g.tiles_n + tn);
     else store_tile192<T>(acc, smem, g, c, res, m0, n0);
 }
