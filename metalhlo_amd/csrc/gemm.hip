@@ -545,6 +545,13 @@ static bool skinny_rows(int64_t M, int64_t N, int64_t K, int64_t batch, int tran
 // gemm_any.hip's 64-row tiles for up to 16 rows of a weight matrix that keeps few workgroups busy ([4,767] x
 // [767,769] 7.3 us against 10.1; [4,4097] x [4097,4097] 48 against 19, [16,1001] x K 8191 30 against 21).
 static bool skinny_unaligned(int64_t M, int64_t N, int64_t K) { return M <= 16 && N * K <= (1 << 20); }
+// fp32 rows off 16 bytes: from 33 rows on the ring of gemm_f32.hip in parts is ahead of element-wise loads once K is long
+// ([48,2304] x [2304,4111]^T 81 us against 29, [48,2303] x K 1024 21.5 against 18.0, [100,767] x K 3073 52 against 24;
+// [32,767] x K 3073 22.3 against 23.2, [48,1001] x K 777 12.2 against 17.6).  Bytes of workspace it takes there, 0 elsewhere.
+static int64_t f32_rows_in_parts(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b) {
+    if (trans_a || M <= 32 || K < 1024 || (K % 4 == 0 && (trans_b || N % 4 == 0))) return 0;
+    return gemm_f32_workspace(M, N, K, batch, trans_a, trans_b);
+}
 // The plain kernel is ahead of a matrix tile that is mostly edges: [65,33] x [33,77] 3.4 us against 4.7, [300,77] x
 // [77,333] 4.7 against 5.3; behind from there on: [128,130] x [130,129] 6.2 against 5.8, [1000,67] x [67,1001] 14.9 against 5.7.
 static bool short_product(int64_t M, int64_t N, int64_t K) { return K < 96 && M * N <= (1 << 17); }
@@ -587,7 +594,8 @@ static int gemm_entry(void* stream, const void* a, const void* b, const void* bi
     // name or by the tuning table.
     if ((is16 || dtype == MHIP_F32) && gemm_skinny_eligible(g, trans_a, is16 ? 2 : 4) && (is16 && !vec_ok ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, batch, trans_b, is16)) &&
         tune_int("MHIP_GEMM_TILE", 0) == 0 && tune_int("MHIP_GEMM_F32_MFMA", 1) == 1 &&
-        (!is16 || few_row_choice(tuned_gemm_variant(g, batch, trans_a, trans_b, dtype)) || !vec_ok))
+        (is16 ? few_row_choice(tuned_gemm_variant(g, batch, trans_a, trans_b, dtype)) || !vec_ok
+              : !(g.partial && f32_rows_in_parts(M, N, K, batch, trans_a, trans_b) > 0 && workspace_bytes >= f32_rows_in_parts(M, N, K, batch, trans_a, trans_b))))
         return chose(vec_ok ? 128 : 0, launch_gemm_skinny(s, g, batch, trans_b, dtype, workspace_bytes));
     if (vec_ok) {
         if (dtype == MHIP_BF16) return pick_layout<bf16_t>(s, g, batch, trans_a, trans_b, workspace_bytes);
@@ -641,6 +649,7 @@ extern "C" int64_t mhip_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t 
     const bool is16 = dtype == MHIP_BF16 || dtype == MHIP_F16;
     if (!is16 && dtype != MHIP_F32) return 0;
     const bool vec = is16 && (trans_a ? M : K) % 8 == 0 && (trans_b ? K : N) % 8 == 0;
+    if (!is16 && f32_rows_in_parts(M, N, K, batch, trans_a, trans_b) > 0) return f32_rows_in_parts(M, N, K, batch, trans_a, trans_b);
     if (!trans_a && M <= (is16 ? 64 : 192) && (is16 && !vec ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, batch, trans_b, is16))) return gemm_skinny_workspace(M, N, K, batch, trans_b, is16);
     // (a large problem goes to the ring kernels, whose tiles fill the device)
     if (!is16) return gemm_f32_workspace(M, N, K, batch, trans_a, trans_b);

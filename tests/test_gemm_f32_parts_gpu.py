@@ -46,3 +46,8 @@ def test_parts_have_the_bits_of_the_whole(N, K, ta, tb):
 def test_strips_of_48_columns(M, N, K):
     """Few-row products whose strips are three columns a lane, the last strip ragged."""
     _check(M, N, K, torch.float32, False, False, residual=M % 2 == 0)
+
+
+@pytest.mark.parametrize("M,N,K,tb", [(33, 2304, 1025, True), (48, 2303, 1024, False), (100, 767, 3073, True), (192, 101, 1030, False), (32, 767, 1025, True)], ids=lambda v: str(v))
+def test_few_rows_off_16_bytes(M, N, K, tb):
+    _check(M, N, K, torch.float32, False, tb, residual=M % 2 == 0)
