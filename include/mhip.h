@@ -170,6 +170,11 @@ int mhip_linear_w32_parts(int64_t M, int64_t N, int64_t K);
 int mhip_linear_w32(void* stream, const void* x, const float* w, const float* bias, const void* residual, void* c, int64_t M,
                     int64_t N, int64_t K, int trans_b, int activation, int dtype, float* sums, int parts, int n_ahead,
                     const mhip_weights* ahead);
+/* c [M,N] = x [M,K] . round(w)^T with w [N,K] in fp32, rounded to x's type (BF16 or F16) at use: the output head of a network
+ * whose embedding table is tied to it.  mhip_tied_head_ok: up to 768 rows, K a multiple of 32 up to 768, N a multiple of 8.
+ * 16-byte aligned pointers. */
+int mhip_tied_head_ok(int64_t M, int64_t N, int64_t K, int dtype);
+int mhip_tied_head(void* stream, const void* x, const float* w, void* c, int64_t M, int64_t N, int64_t K, int dtype);
 /* The fp32 sums of `parts` shares of K (up to 8), sums[parts][M][N], of a [M,K] . b [K,N] in BF16 or F16, for mhip_finish_norm.
  * mhip_gemm_sums_parts gives a good number of parts for the sizes, 0 where they are not served (N and K multiples of
  * 8).  16-byte aligned pointers.  The last bits of a row may change with the number of rows. */

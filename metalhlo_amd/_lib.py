@@ -35,6 +35,8 @@ SIGNATURES = {
     "mhip_linear_w32_ok": (_i32, [_i64, _i64, _i64, _i32]),
     "mhip_linear_w32_parts": (_i32, [_i64, _i64, _i64]),
     "mhip_linear_w32": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _i32, _i32, _vp, _i32, _i32, _vp]),
+    "mhip_tied_head_ok": (_i32, [_i64, _i64, _i64, _i32]),
+    "mhip_tied_head": (_i32, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32]),
     "mhip_gemm_sums_parts": (_i32, [_i64, _i64, _i64, _i32]),
     "mhip_gemm_sums": (_i32, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _i32]),
     "mhip_finish_norm": (_i32, [_vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _f32, _vp, _i64, _i64, _i32]),

@@ -433,8 +433,9 @@ static int pick_tile(hipStream_t s, const GemmArgs& g, int64_t batch, int64_t wo
     if (force == 2567) {
         if (gemm256_eligible(g, batch, TA, TB, dt, 384) && gemm384_activation_ok(g.act)) return chose(2567, launch_gemm256(s, g, batch, TA, TB, dt, 384, 4));
     }
-    // (up to 192 rows: half of a 256-row tile would be padding)
-    if (force == 128 || (force == 0 && g.M <= 192)) return chose(128, launch_gemm_mid(s, g, batch, TA, TB, dt, workspace_bytes));
+    // (up to 192 rows: much of a 256-row tile would be padding; with more than 128 it is ahead all the same where its columns fill
+    // the device, [150,768] x [50304,768]^T 40.9 us in 128-row tiles, 27.4)
+    if (force == 128 || (force == 0 && g.M <= 192 && (g.M <= 128 || g.K < 512 || !gemm256_eligible(g, batch, TA, TB, dt)))) return chose(128, launch_gemm_mid(s, g, batch, TA, TB, dt, workspace_bytes));
     constexpr int cus = 256;                           // compute units of the device this is written for
     const int64_t narrow = tiles_m * ((g.N + 127) / 128) * batch, stages = g.K / 32;
     const int64_t wide_cost = ((big + cus - 1) / cus) * (stages * 32 + 700);

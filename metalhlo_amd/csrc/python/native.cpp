@@ -273,6 +273,19 @@ FUNCTION(linear) {
     });
 }
 
+// tied_head(x, weight fp32 [N, K])
+FUNCTION(tied_head) {
+    return guarded(n, 2, [&] {
+        const at::Tensor &x = dense(arg[0]), &w = dense(arg[1]);
+        if (x.dim() != 2 || w.dim() != 2 || x.size(1) != w.size(1)) raise(PyExc_ValueError, "tied_head needs [M, K] and [N, K]");
+        if (w.scalar_type() != at::kFloat) raise(PyExc_TypeError, "parameters must be fp32");
+        const int dt = dtype_code(x.scalar_type());
+        at::Tensor c = empty({x.size(0), w.size(0)}, x.scalar_type(), x);
+        check([&] { return mhip_tied_head(stream_of(x), x.data_ptr(), w.data_ptr<float>(), c.data_ptr(), x.size(0), w.size(0), x.size(1), dt); });
+        return THPVariable_Wrap(std::move(c));
+    });
+}
+
 // matmul_sums(a, b, parts) -> [parts, M, N] fp32
 FUNCTION(matmul_sums) {
     return guarded(n, 3, [&] {
@@ -405,7 +418,7 @@ FUNCTION(bind) {
 }
 
 #define ENTRY(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
-PyMethodDef kMethods[] = {ENTRY(softmax), ENTRY(layer_norm), ENTRY(rms_norm), ENTRY(bias_gelu), ENTRY(matmul), ENTRY(linear), ENTRY(matmul_sums), ENTRY(finish_norm), ENTRY(causal_attention),
+PyMethodDef kMethods[] = {ENTRY(softmax), ENTRY(layer_norm), ENTRY(rms_norm), ENTRY(bias_gelu), ENTRY(matmul), ENTRY(linear), ENTRY(matmul_sums), ENTRY(tied_head), ENTRY(finish_norm), ENTRY(causal_attention),
                           ENTRY(flash_attention), ENTRY(argmax), ENTRY(bind), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

@@ -70,16 +70,20 @@ class GPT2:
         self._slots.append((("wte",), self._slots[-1][1], wte.shape))
         for name in ("wpe", "lnf_g", "lnf_b"):
             put((name,), params[name])
+        self._layers_at = sum(x.size for x in flat)
         for i, l in enumerate(params["layers"]):
             for k, v in l.items():
                 put(("layers", i, k), v)
         self.flat32 = torch.from_numpy(np.concatenate(flat)).to(device)
         self.p32 = self._views(self.flat32)
 
-    def _views(self, flat: torch.Tensor) -> Dict:
+    def _views(self, flat: torch.Tensor, start: int = 0) -> Dict:
+        """The parameters from element `start` of the buffer on, which `flat` holds."""
         out: Dict = {"layers": [dict() for _ in range(self.cfg.n_layer)]}
         for path, off, shape in self._slots:
-            v = torch.as_strided(flat, shape, (shape[1], 1) if len(shape) == 2 else (1,), off)
+            if off < start:
+                continue
+            v = torch.as_strided(flat, shape, (shape[1], 1) if len(shape) == 2 else (1,), off - start)
             if path[0] == "layers":
                 out["layers"][path[1]][path[2]] = v
             else:
@@ -96,7 +100,10 @@ class GPT2:
             return self._forward_few(ids)
         o_parts, p_parts = self._sum_parts(B * S)
         # the graph's `convert` ops: fp32 parameters -> compute type, every step
-        p = self.p32 if self.dtype == torch.float32 else self._views(kernels.convert(self.flat32, self.dtype))
+        # (a short prompt's output head reads its fp32 rows where they are)
+        fp32_head = o_parts and kernels.tied_head_served(B * S, self.vocab_pad, d, self.dtype)
+        start = self._layers_at if fp32_head else 0
+        p = self.p32 if self.dtype == torch.float32 else self._views(kernels.convert(self.flat32[start:], self.dtype), start)
         x = kernels.embed_tokens(ids, self.p32["wte"], self.p32["wpe"], self.dtype).reshape(B * S, d)
         # the strided attention entry covers 16-bit types and head sizes 64 / 128
         in_place = self.dtype in (torch.bfloat16, torch.float16) and d // H in (64, 128)
@@ -110,7 +117,7 @@ class GPT2:
                 x, h = kernels.finish_norm(kernels.matmul_sums(a, l["w_o"], o_parts), l32["b_o"], x, (l32["ln2_g"], l32["ln2_b"], 1e-5))
                 u = kernels.matmul(h, l["w_fc"], bias=l["b_fc"], activation="gelu")
                 x, h = kernels.finish_norm(kernels.matmul_sums(u, l["w_proj"], p_parts), l32["b_proj"], x, norm)
-            logits = kernels.matmul(h, p["wte_pad"], trans_b=True)
+            logits = kernels.tied_head(h, self.p32["wte_pad"]) if fp32_head else kernels.matmul(h, p["wte_pad"], trans_b=True)
             return logits.reshape(B, S, self.vocab_pad)[..., :cfg.vocab]
         for l in p["layers"]:
             h = kernels.layer_norm(x, l["ln1_g"], l["ln1_b"], eps=1e-5)
@@ -139,15 +146,15 @@ class GPT2:
         d, f, dt = self.cfg.d_model, self.cfg.d_ff, self.dtype
         if dt not in (torch.bfloat16, torch.float16) or d // self.cfg.n_head not in (64, 128) or d % self.cfg.n_head:
             return False
-        # (each 64 rows read a matrix again: three times from memory cost more than converting it, 150 tokens 784 us against 669,
-        # 128 tokens 692 against 669, 96 tokens 627 against 647, replayed; a matrix of up to 4 MB stays in an L2)
-        if tokens > 128 and 4 * d * f > 4 << 20:
+        # (each 64 rows read a matrix again, which from memory costs as much as converting it: us as they are held and converted,
+        # replayed, 65 tokens 585 and 591, 96 tokens 615 and 612, 128 tokens 679 and 635; a matrix of up to 4 MB stays in an L2)
+        if tokens > 96 and 4 * d * f > 4 << 20:
             return False
         return d <= 4096 and all(kernels.linear_served(tokens, n, k, dt) for n, k in ((3 * d, d), (d, d), (f, d), (d, f), (self.vocab_pad, d)))
 
     # 64x64 tiles of the layers in front of a residual from which on they fill the device whole
-    # (us whole and in parts, replayed: 193 tokens 813 and 679, 300 842 and 721, 576 952 and 875, 768 (144 tiles) 1109 and 1050;
-    # 1024 (192 tiles) 1233 and 1218, which leaves a sequence of full length its bits in any batch)
+    # (us whole and in parts, replayed: 193 tokens 810 and 642, 300 841 and 692, 576 949 and 844, 768 (144 tiles) 1098 and 1008;
+    # 1024 (192 tiles) 1206 and 1202, which leaves a sequence of full length its bits in any batch)
     _full_tiles = 144
 
     def _sum_parts(self, tokens: int):
@@ -179,7 +186,11 @@ class GPT2:
             u = linear(h, l["w_fc"], l["b_fc"], "gelu")
             sums = linear(u, l["w_proj"], parts=p_parts, ahead=(layers[i + 1]["w_qkv"],) if i + 1 < len(layers) else ())
             x, h = kernels.finish_norm(sums, l["b_proj"], x, norms[i + 1])
-        logits = linear(h, p["wte_pad"], trans_b=True)
+        # (us, strips that walk the device against x that stays: 64 tokens 36.9 and 38.5, 65 48.5 and 39.2, 128 53.5 and 45.1)
+        if T > 64 and kernels.tied_head_served(T, self.vocab_pad, cfg.d_model, self.dtype):
+            logits = kernels.tied_head(h, p["wte_pad"])
+        else:
+            logits = linear(h, p["wte_pad"], trans_b=True)
         return logits.reshape(B, S, self.vocab_pad)[..., :cfg.vocab]
 
     def capture(self, ids: torch.Tensor) -> "GraphedForward":

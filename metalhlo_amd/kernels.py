@@ -119,6 +119,15 @@ def linear_parts(M: int, N: int, K: int) -> int:
     return _lib.load().mhip_linear_w32_parts(M, N, K)
 
 
+def tied_head(x, weight):
+    """x [M, K] @ weight [N, K].T in x's 16-bit type, the fp32 weight rounded to it at use; `tied_head_served` says for which sizes."""
+    return (_native or _host()).tied_head(x, weight)
+
+
+def tied_head_served(M: int, N: int, K: int, dtype) -> bool:
+    return bool(_lib.load().mhip_tied_head_ok(M, N, K, DTYPE_CODE[dtype]))
+
+
 def matmul_sums(a, b, parts: int):
     """The fp32 sums of so many shares of K of a [M, K] @ b [K, N] in a 16-bit type: [parts, M, N], for finish_norm."""
     return (_native or _host()).matmul_sums(a, b, parts)

@@ -35,7 +35,7 @@ def test_refusals():
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("B,S,few,parts", [(1, 128, True, True), (3, 43, False, True), (2, 150, False, True), (1, 768, False, True), (1, 769, False, False)])
+@pytest.mark.parametrize("B,S,few,parts", [(1, 96, True, True), (1, 97, False, True), (2, 150, False, True), (1, 768, False, True), (1, 769, False, False)])
 def test_gpt2_forms_agree(dtype, B, S, few, parts):
     """The form a token count takes against the one for many tokens: the same roundings, fp32 sums in another order.  Where
     those differ a value rounds the other way and carries on, at most a few units by the second layer."""
