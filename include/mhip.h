@@ -145,7 +145,8 @@ int mhip_gemm_residual(void* stream, const void* a, const void* b, const void* b
                        int trans_a, int trans_b, int activation, int dtype);
 
 /* The same (residual may be NULL) with device memory the call may use for partial sums: a problem with few
- * tiles and a long K is then split along K over the whole device.  mhip_gemm_workspace returns the bytes the
+ * tiles and a long K is then split along K over the whole device; and for copies of large 16-bit operands whose rows
+ * start off 16-byte boundaries (up to 512 MB).  mhip_gemm_workspace returns the bytes the
  * choice for a problem can use (0: none); with less, or none, the result is computed without splitting.  The
  * workspace is 16-byte aligned, its content is overwritten and meaningless afterwards, and it may be reused as
  * soon as work enqueued behind this call on the same stream may run. */

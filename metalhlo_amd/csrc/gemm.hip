@@ -301,6 +301,9 @@ int64_t gemm_skinny_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, in
 // gemm_any.hip: any alignment and size.
 int launch_gemm_any(hipStream_t s, GemmArgs g, int64_t batch, int trans_a, int trans_b, int dtype, int64_t workspace_bytes);
 int64_t gemm_any_workspace(int64_t M, int64_t N, int64_t K, int64_t batch);
+// gemm_any.hip also makes copies with aligned rows.
+GemmPack gemm_pack_plan(const GemmArgs& g, int trans_a, int trans_b, bool a_off, bool b_off);
+int launch_gemm_pack(hipStream_t s, const GemmArgs& g, const GemmPack& p, int trans_a, int trans_b, char* to);
 int launch_gemm_skinny(hipStream_t s, GemmArgs g, int64_t batch, int trans_b, int dtype, int64_t workspace_bytes);
 // gemm_mid.hip: 64- and 128-row tiles through a ring of LDS stages, K split where that leaves units idle.
 int64_t gemm_mid_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b);
@@ -557,6 +560,27 @@ static int64_t f32_rows_in_parts(int64_t M, int64_t N, int64_t K, int64_t batch,
 // [77,333] 4.7 against 5.3; behind from there on: [128,130] x [130,129] 6.2 against 5.8, [1000,67] x [67,1001] 14.9 against 5.7.
 static bool short_product(int64_t M, int64_t N, int64_t K) { return K < 96 && M * N <= (1 << 17); }
 
+// The aligned problem that copies of the operands give, in mhip_gemm's workspace: the copies, then what the aligned
+// problem itself can use.
+static GemmArgs packed_args(const GemmArgs& g, const GemmPack& p) {
+    GemmArgs q = g;
+    q.K = p.K; q.lda = p.lda; q.ldb = p.ldb;
+    return q;
+}
+static int64_t aligned_workspace(int64_t M, int64_t N, int64_t K, int trans_a, int trans_b) {
+    if (M > 192 && (double)M * N >= 192.0 * 256 * 256) return 0;         // (a large problem goes to the ring kernels, whose tiles fill the device)
+    return gemm_mid_workspace(M, N, K, 1, trans_a, trans_b);
+}
+// Where copies pay: gemm_any.hip's tiles wait out a load latency per stage, 11.7 ns a k, and touch two lines per load.  us, as they
+// are | copied (the copies included), over the four layouts: [1001,1001] x K 4001 47 to 50 | 30 to 32, [301,2001] x K 3001 36 to 38 |
+// 27 to 28, [513,3000] x K 16001 (x^T dy) 221 | 118, [4096,4097] x K 4096 235 | 155, [7613,2305] x K 833 71 | 58, [2047,2047] x K 2047
+// 43.6 | 35.7, [769,769] x K 2001 (169 tiles of 64x64) 26 to 28 | 22 to 23; but [513,3001] x K 2001 (423 tiles) 28 | 28 to 29,
+// [1500,1501] x K 1500 26 to 28 | 31 to 34, [3001,1001] x K 1501 29 | 29, [65,4097] x K 4096 25 | 32.  No more than 512 MB of them.
+static bool pack_pays(int64_t M, int64_t N, int64_t K) {
+    if (M <= 192 || (M + N) * K * 2 > (512ll << 20)) return false;
+    return K >= 3000 || (double)M * N * K >= 8e9 || (K >= 2000 && ((M + 63) / 64) * ((N + 63) / 64) <= 256);
+}
+
 static bool few_row_choice(int tuned) { return tuned == 0 || tuned == 128; }
 
 static int gemm_entry(void* stream, const void* a, const void* b, const void* bias, const void* residual, void* c,
@@ -608,6 +632,22 @@ static int gemm_entry(void* stream, const void* a, const void* b, const void* bi
             return launch_simple<float>(s, g, batch, trans_a, trans_b);
         case MHIP_BF16:
         case MHIP_F16:
+            // (the kernel that reads such rows as they are, unless the workspace takes copies and those pay)
+            if (g.partial && batch == 1 && pack_pays(M, N, K)) {
+                const bool a_off = g.lda % 8 != 0 || (reinterpret_cast<uintptr_t>(a) & 15) != 0, b_off = g.ldb % 8 != 0 || (reinterpret_cast<uintptr_t>(b) & 15) != 0;
+                const GemmPack p = gemm_pack_plan(g, trans_a, trans_b, a_off, b_off);
+                GemmArgs q = packed_args(g, p);
+                const int64_t left = workspace_bytes - p.a_bytes - p.b_bytes;
+                if (left >= 0 && (int64_t)(trans_a ? q.K : M) * q.lda * 2 < 0x7FFFFFFFLL && (int64_t)(trans_b ? N : q.K) * q.ldb * 2 < 0x7FFFFFFFLL) {
+                    char* to = static_cast<char*>(workspace);
+                    const int st = launch_gemm_pack(s, g, p, trans_a, trans_b, to);
+                    if (st != MHIP_OK) return st;
+                    if (p.a) q.a = to;
+                    if (p.b) q.b = to + p.a_bytes;
+                    q.partial = left > 0 ? reinterpret_cast<float*>(to + p.a_bytes + p.b_bytes) : nullptr;
+                    return dtype == MHIP_BF16 ? pick_layout<bf16_t>(s, q, 1, trans_a, trans_b, left) : pick_layout<f16_t>(s, q, 1, trans_a, trans_b, left);
+                }
+            }
             if (!short_product(M, N, K)) return launch_gemm_any(s, g, batch, trans_a, trans_b, dtype, workspace_bytes);
             return dtype == MHIP_BF16 ? launch_simple<bf16_t>(s, g, batch, trans_a, trans_b) : launch_simple<f16_t>(s, g, batch, trans_a, trans_b);
         case MHIP_I32: return launch_exact<int32_t>(s, g, batch, trans_a, trans_b);
@@ -654,7 +694,13 @@ extern "C" int64_t mhip_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t 
     if (!trans_a && M <= (is16 ? 64 : 192) && (is16 && !vec ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, batch, trans_b, is16))) return gemm_skinny_workspace(M, N, K, batch, trans_b, is16);
     // (a large problem goes to the ring kernels, whose tiles fill the device)
     if (!is16) return gemm_f32_workspace(M, N, K, batch, trans_a, trans_b);
+    if (!vec && pack_pays(M, N, K)) {
+        // (whether a pointer is off 16 bytes is not known here: room for both copies)
+        GemmArgs g = {};
+        g.M = (int)M; g.N = (int)N; g.K = (int)K; g.lda = (int)(trans_a ? M : K); g.ldb = (int)(trans_b ? K : N);
+        const GemmPack p = gemm_pack_plan(g, trans_a, trans_b, g.lda % 8 != 0, g.ldb % 8 != 0);
+        return p.a_bytes + p.b_bytes + aligned_workspace(M, N, p.K, trans_a, trans_b);
+    }
     if (!vec) return short_product(M, N, K) ? 0 : gemm_any_workspace(M, N, K, batch);
-    if (M > 192 && (double)M * N * batch >= 192.0 * 256 * 256) return 0;
-    return gemm_mid_workspace(M, N, K, batch, trans_a, trans_b);
+    return aligned_workspace(M, N, K, trans_a, trans_b);
 }

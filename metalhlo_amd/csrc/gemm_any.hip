@@ -10,6 +10,9 @@
 // 64x64 tiles (five workgroups per compute unit) until 128x128 ones fill the device; a long K is split over the
 // grid where a workspace takes the parts.  bf16 [2047,2047] x K 2047 1077 -> 54 us, x^T dy of 769 x 3071 over 8192 tokens
 // 2707 -> 129, [4096,4097] x K 4096 8662 -> 231 (595 TFLOP/s; the loads of unaligned rows touch two lines each).
+//
+// Large ones are copied to rows on 16-byte boundaries instead (gemm_pack_kernel, about 4.5 TB/s of reads and writes) and take the
+// kernels for aligned operands; gemm.hip says from where on.
 #include "gemm_lds.h"
 
 namespace mhip {
@@ -228,7 +231,76 @@ int launch_tile(hipStream_t s, GemmArgs g, int64_t batch, int ta, int tb) {
     return check_launch("gemm_any");
 }
 
+// ---- copies with rows on 16-byte boundaries ----
+struct PackArgs {
+    const uint16_t* src[2];
+    uint16_t* dst[2];
+    int rows[2], cols[2];              // what exists
+    int dst_rows[2], dst_cols[2];      // zeros behind it; columns a multiple of eight
+    unsigned blocks0;                  // workgroups of the first matrix
+};
+constexpr int kPackPieces = 4;         // 16 bytes each, per thread
+
+__global__ __launch_bounds__(256) void gemm_pack_kernel(PackArgs p) {
+    const int o = blockIdx.x >= p.blocks0 ? 1 : 0;
+    const int rows = p.rows[o], cols = p.cols[o], cpr = p.dst_cols[o] / 8;
+    const int64_t all = (int64_t)p.dst_rows[o] * cpr, first = (int64_t)(blockIdx.x - (o ? p.blocks0 : 0)) * (256 * kPackPieces) + threadIdx.x;
+    u32x4 v[kPackPieces];
+#pragma unroll
+    for (int i = 0; i < kPackPieces; i++) {
+        const int64_t at = first + i * 256;
+        v[i] = u32x4{0u, 0u, 0u, 0u};
+        if (at >= all) continue;
+        const int64_t row = at / cpr;
+        const int c = (int)(at - row * cpr) * 8, n = row < rows ? min(8, cols - c) : 0;
+        if (n <= 0) continue;
+        const uint16_t* s = p.src[o] + row * cols + c;
+        if (n == 8) v[i] = load_piece(s);
+        else if (cols >= 8) v[i] = keep_last(load_piece(s - (8 - n)), n);      // (the piece that ends where the row does)
+        else v[i] = load_part(s, n);
+    }
+#pragma unroll
+    for (int i = 0; i < kPackPieces; i++)
+        if (first + i * 256 < all) *reinterpret_cast<u32x4*>(p.dst[o] + (first + i * 256) * 8) = v[i];
+}
+
 }  // namespace
+
+// How an unaligned problem becomes an aligned one: a copy of each operand whose rows need it; k is padded with zeros to
+// whole stages where both are copied, and where k is the row of one, both are.
+GemmPack gemm_pack_plan(const GemmArgs& g, int trans_a, int trans_b, bool a_off, bool b_off) {
+    GemmPack p;
+    p.a = a_off || g.K % 8 != 0;
+    p.b = b_off || g.K % 8 != 0;
+    const int64_t k = p.a && p.b ? (g.K + 31) / 32 * 32 : g.K;
+    p.K = (int)k;
+    const int64_t m = (g.M + 7) / 8 * 8, n = (g.N + 7) / 8 * 8;
+    p.lda = !p.a ? g.lda : (int)(trans_a ? m : k);
+    p.ldb = !p.b ? g.ldb : (int)(trans_b ? k : n);
+    p.a_bytes = p.a ? (trans_a ? k * m : (int64_t)g.M * k) * 2 : 0;
+    p.b_bytes = p.b ? (trans_b ? (int64_t)g.N * k : k * n) * 2 : 0;
+    p.a_bytes = (p.a_bytes + 255) / 256 * 256;
+    p.b_bytes = (p.b_bytes + 255) / 256 * 256;
+    return p;
+}
+
+int launch_gemm_pack(hipStream_t s, const GemmArgs& g, const GemmPack& p, int trans_a, int trans_b, char* to) {
+    PackArgs w = {};
+    int n = 0;
+    int64_t blocks[2] = {0, 0};
+    auto add = [&](const void* src, char* dst, int rows, int cols, int dst_rows, int dst_cols) {
+        w.src[n] = static_cast<const uint16_t*>(src); w.dst[n] = reinterpret_cast<uint16_t*>(dst);
+        w.rows[n] = rows; w.cols[n] = cols; w.dst_rows[n] = dst_rows; w.dst_cols[n] = dst_cols;
+        blocks[n] = ((int64_t)dst_rows * (dst_cols / 8) + 256 * kPackPieces - 1) / (256 * kPackPieces);
+        n++;
+    };
+    if (p.a) add(g.a, to, trans_a ? g.K : g.M, trans_a ? g.M : g.K, trans_a ? p.K : g.M, p.lda);
+    if (p.b) add(g.b, to + p.a_bytes, trans_b ? g.N : g.K, trans_b ? g.K : g.N, trans_b ? g.N : p.K, p.ldb);
+    w.blocks0 = (unsigned)blocks[0];
+    if (blocks[0] + blocks[1] > 0x7FFFFFFFLL) return fail(MHIP_ERR_UNSUPPORTED, "gemm: grid too large");
+    hipLaunchKernelGGL(gemm_pack_kernel, dim3((unsigned)(blocks[0] + blocks[1])), dim3(256), 0, s, w);
+    return check_launch("gemm_pack");
+}
 
 int64_t gemm_any_workspace(int64_t M, int64_t N, int64_t K, int64_t batch) {
     const int n = any_splits(M, N, K, batch);

@@ -29,6 +29,13 @@ struct GemmArgs {
     int stream_c = 0;                 // gemm256.hip: C is far larger than the L2s, store it with the streaming hint
 };
 
+// Copies of operands whose rows are off 16 bytes (gemm_any.hip): which are made, and the aligned problem they give.
+struct GemmPack {
+    bool a = false, b = false;
+    int K = 0, lda = 0, ldb = 0;
+    int64_t a_bytes = 0, b_bytes = 0;      // of the copies, each a multiple of 256
+};
+
 template <typename T> struct Mfma32;
 template <> struct Mfma32<bf16_t> {
     __device__ static f32x16 run(u32x4 a, u32x4 b, f32x16 c) {

@@ -1,0 +1,62 @@
+"""16-bit products whose operands are copied to rows on 16-byte boundaries, against the kernel that reads them as they are (the
+same bits below K 4096) and float64: one or both operands off, k padded to whole stages, rows and columns ragged."""
+import pytest
+import torch
+
+from metalhlo_amd import _lib, kernels
+
+pytestmark = pytest.mark.gpu
+
+EPS = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+
+
+def _inside_nan(shape, dtype, g, scale=1.0):
+    """A dense matrix with NaN in front of it and behind it: what lies outside must not be multiplied."""
+    n = shape[0] * shape[1]
+    buf = torch.full((n + 96,), float("nan"), dtype=dtype, device="cuda")
+    x = buf[16:16 + n].view(*shape)
+    x.copy_(torch.randn(*shape, generator=g, device="cuda") * scale)
+    return x
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(201, 203, 3001), (769, 515, 2001), (264, 257, 3008), (257, 264, 3016), (2049, 2051, 2041), (193, 9, 4999), (300, 1, 3002)])
+def test_copies(dtype, ta, tb, M, N, K):
+    lib, code = _lib.load(), kernels.DTYPE_CODE[dtype]
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a, b = _inside_nan((K, M) if ta else (M, K), dtype, g), _inside_nan((N, K) if tb else (K, N), dtype, g, K ** -0.5)
+    bias, res = torch.randn(N, generator=g, device="cuda").to(dtype), torch.randn(M, N, generator=g, device="cuda").to(dtype)
+
+    def product(bytes_):
+        out = torch.full((M * N + 64,), 7.0, dtype=dtype, device="cuda")
+        work = torch.full((max(bytes_, 1),), 255, dtype=torch.uint8, device="cuda")
+        assert lib.mhip_gemm_ws(torch.cuda.current_stream().cuda_stream, a.data_ptr(), b.data_ptr(), bias.data_ptr(), res.data_ptr(), out.data_ptr(), M, N, K, 1, 0, 0, 0,
+                                ta, tb, 1, code, work.data_ptr() if bytes_ else None, bytes_) == 0
+        assert (out[M * N:] == 7.0).all()
+        return out[:M * N].view(M, N)
+
+    need = lib.mhip_gemm_workspace(M, N, K, 1, ta, tb, code)
+    if (ta and M % 8 != 0) or (not ta and K % 8 != 0) or (tb and K % 8 != 0) or (not tb and N % 8 != 0):
+        assert need >= 2 * min(M, N) * K
+    got = product(need)
+    exp = torch.relu((a.double().T if ta else a.double()).contiguous() @ (b.double().T if tb else b.double()).contiguous() + bias.double())
+    assert ((got.double() - exp - res.double()).abs() <= 2 * EPS[dtype] * (exp.abs() + res.double().abs()).clamp(min=1.0)).all()
+    if K < 4096:
+        assert torch.equal(got, product(0))
+    assert torch.isfinite(product(need // 2)).all()              # less than the copies take: as they are
+
+
+def test_copies_from_a_graph():
+    g = torch.Generator(device="cuda").manual_seed(1)
+    a, b = torch.randn(301, 3001, generator=g, device="cuda").bfloat16(), torch.randn(3001, 501, generator=g, device="cuda").bfloat16()
+    kernels.matmul(a, b)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = kernels.matmul(a, b)
+    for i in range(3):
+        a.normal_(generator=g)
+        want = kernels.matmul(a, b)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
