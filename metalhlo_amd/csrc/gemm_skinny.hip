@@ -102,6 +102,12 @@ template <typename T, int VE, bool VEC> struct RowPiece {
     }
 };
 
+// Whether neighbouring strips go to one XCD: rows of a strip that are half a line or less, whose other half the same L2 then holds for the
+// neighbour.  us, without | with: [1,6720] x K 832 bf16 5.9 | 5.0, [8,1024] x K 4096 bf16 9.3 | 8.8, [16,6720] x K 832 fp32
+// 10.4 | 9.0; strips of 128 or 192 bytes lose by it, [4,4096] x K 4096 bf16 11.0 | 11.3, [128,3072] x K 768 fp32 11.5 | 12.0.
+template <typename T, bool TB, int NF>
+constexpr bool strip_order() { return !TB && 16 * NF * (int)sizeof(T) < 128; }
+
 // NF = operands (groups of 16 columns) per strip, MT = groups of 16 rows, U = k steps loaded as one block.
 template <typename T, bool TB, bool VEC, int NF, int MT, int U, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(GemmArgs g) {
@@ -111,7 +117,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(GemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) float part[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     const int li = lane & 15, lg = lane >> 4;
-    const int n0 = blockIdx.x * NS;
+    const int strip = strip_order<T, TB, NF>() ? (int)(blockIdx.x % kXcds * (gridDim.x / kXcds) + blockIdx.x / kXcds) : (int)blockIdx.x, n0 = strip * NS;
+    if (strip_order<T, TB, NF>() && n0 >= g.N) return;
     int batch_i = blockIdx.y, m0 = 0;
     if (g.tiles_m > 1) { m0 = batch_i % g.tiles_m * (16 * MT); batch_i /= g.tiles_m; }
     const int64_t batch = batch_i;
@@ -247,8 +254,9 @@ int launch_one(hipStream_t s, GemmArgs g, int64_t batch) {
     const int waves = want < 1 ? 1 : want > WAVES ? WAVES : want;
     const int64_t strips = (g.N + 16 * NF - 1) / (16 * NF);
     g.tiles_m = (g.M + 16 * MT - 1) / (16 * MT);
-    if (strips > 0x7FFFFFFFLL || batch * g.tiles_m > 65535) return fail(MHIP_ERR_UNSUPPORTED, "gemm: grid too large");
-    hipLaunchKernelGGL(kern, dim3((unsigned)strips, (unsigned)(batch * g.tiles_m), (unsigned)g.splits), dim3(64 * waves), waves * NF * MT * 1024, s, g);
+    const int64_t grid = strip_order<T, TB, NF>() ? (strips + kXcds - 1) / kXcds * kXcds : strips;
+    if (grid > 0x7FFFFFFFLL || batch * g.tiles_m > 65535) return fail(MHIP_ERR_UNSUPPORTED, "gemm: grid too large");
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid, (unsigned)(batch * g.tiles_m), (unsigned)g.splits), dim3(64 * waves), waves * NF * MT * 1024, s, g);
     return check_launch("gemm_skinny");
 }
 
