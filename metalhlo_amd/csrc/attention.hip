@@ -500,7 +500,7 @@ bool fa_flow_wanted(const FaArgs& a);
 int launch_fa_flow(hipStream_t s, FaArgs a, int64_t D, int dtype);
 // attention_f32.hip: fp32 tensors on the fp32 matrix instruction.
 bool fa_f32_mfma_eligible(const FaArgs& a, int64_t D, bool packed);
-int launch_fa_f32_mfma(hipStream_t s, const FaArgs& a, int64_t D, float scale);
+int launch_fa_f32_mfma(hipStream_t s, const FaArgs& a, int64_t D, float scale, bool packed);
 }  // namespace mhip
 
 using namespace mhip;
@@ -569,13 +569,13 @@ static int fa_entry(const char* name, void* stream, const void* q, const void* k
     // (with rows of a multiple of 8 elements every piece of 16 bytes is aligned)
     if (is16 && (is_packed || (any_views && strides_aligned)) && aligned && fits && Skv > 0 && D % 8 == 0 && D < 128)
         return dtype == MHIP_BF16 ? launch_fa_part<bf16_t>(s, a, is_causal, mask != nullptr) : launch_fa_part<f16_t>(s, a, is_causal, mask != nullptr);
-    if (any_views && !is_packed && Skv > 0 && dtype == MHIP_F32 && fa_f32_mfma_eligible(a, D, false)) return launch_fa_f32_mfma(s, a, D, scale);
+    if (any_views && !is_packed && Skv > 0 && dtype == MHIP_F32 && fa_f32_mfma_eligible(a, D, false)) return launch_fa_f32_mfma(s, a, D, scale, false);
     if (!is_packed)
         return fail(MHIP_ERR_UNSUPPORTED, "%s: strided layouts need bf16 / f16, head_dim 64 or 128, 16-byte aligned pointers and "
                                           "strides that are multiples of 8 elements", name);
     switch (dtype) {
         case MHIP_F32:
-            if (fa_f32_mfma_eligible(a, D, true)) return launch_fa_f32_mfma(s, a, D, scale);
+            if (fa_f32_mfma_eligible(a, D, true)) return launch_fa_f32_mfma(s, a, D, scale, true);
             return launch_fa_scalar<float>(s, a, (int)D, scale);
         case MHIP_BF16: return launch_fa_scalar<bf16_t>(s, a, (int)D, scale);
         case MHIP_F16: return launch_fa_scalar<f16_t>(s, a, (int)D, scale);

@@ -26,10 +26,18 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 constexpr int kFBQ = 128;     // query rows per workgroup
 constexpr int kFBK = 32;      // keys per block
 
+// Element offset of head bh: `packed` elements a head, or where the strides say.
+template <bool VIEWS>
+__device__ __forceinline__ int64_t head_at(const FaArgs& a, const int64_t (&strides)[3], int bh, int64_t packed) {
+    return VIEWS ? bh / a.H * strides[0] + bh % a.H * strides[1] : bh * packed;
+}
+
 // key (within a block) of accumulator register i in the 32-lane half h
 __device__ __forceinline__ int f32_key(int i, int h) { return 8 * (i >> 2) + 4 * h + (i & 3); }
 
-template <int D, bool CAUSAL, bool HAS_MASK>
+// VIEWS: rows lie where the strides say; without it they are packed and every row offset is a constant (strides from memory
+// cost the packed tensors 1 to 4 %, [2,8,512,128] 27.7 against 28.8 us).
+template <int D, bool CAUSAL, bool HAS_MASK, bool VIEWS>
 __global__ __launch_bounds__(256, 2) void fa_f32_mfma_kernel(FaArgs a, float scale) {
     // K rows padded to D + 2 floats (lane = key reads fall on distinct banks), V rows to D + 8
     // (the two halves of a wave read rows four apart)
@@ -47,12 +55,11 @@ __global__ __launch_bounds__(256, 2) void fa_f32_mfma_kernel(FaArgs a, float sca
     const int q0 = qb * kFBQ + wave * 32;
     const int qpos = q0 + ln;                       // this lane's query row
     const bool q_live = qpos < a.Sq;
-    const int b_i = bh / a.H, h_i = bh % a.H;
-    const float* qp = static_cast<const float*>(a.q) + b_i * a.qs[0] + h_i * a.qs[1];
-    const float* kp = static_cast<const float*>(a.k) + b_i * a.ks[0] + h_i * a.ks[1];
-    const float* vp = static_cast<const float*>(a.v) + b_i * a.vs[0] + h_i * a.vs[1];
-    float* op = static_cast<float*>(a.o) + b_i * a.os[0] + h_i * a.os[1];
-    const int64_t k_rs = a.ks[2], v_rs = a.vs[2];
+    const float* qp = static_cast<const float*>(a.q) + head_at<VIEWS>(a, a.qs, bh, a.Sq * (int64_t)D);
+    const float* kp = static_cast<const float*>(a.k) + head_at<VIEWS>(a, a.ks, bh, a.Skv * (int64_t)D);
+    const float* vp = static_cast<const float*>(a.v) + head_at<VIEWS>(a, a.vs, bh, a.Skv * (int64_t)D);
+    float* op = static_cast<float*>(a.o) + head_at<VIEWS>(a, a.os, bh, a.Sq * (int64_t)D);
+    const int64_t q_rs = VIEWS ? a.qs[2] : D, k_rs = VIEWS ? a.ks[2] : D, v_rs = VIEWS ? a.vs[2] : D, o_rs = VIEWS ? a.os[2] : D;
     const float* mp = HAS_MASK ? static_cast<const float*>(a.mask) + (int64_t)(bh / a.H) * a.mask_sb +
                                      (int64_t)(bh % a.H) * a.mask_sh + (int64_t)qpos * a.Skv
                                : nullptr;
@@ -60,7 +67,7 @@ __global__ __launch_bounds__(256, 2) void fa_f32_mfma_kernel(FaArgs a, float sca
     // Q^T fragments: k-step s holds Q[qpos][2 s + h]
     float qf[NS];
 #pragma unroll
-    for (int s = 0; s < NS; s++) qf[s] = q_live ? qp[qpos * a.qs[2] + 2 * s + h] : 0.f;
+    for (int s = 0; s < NS; s++) qf[s] = q_live ? qp[qpos * q_rs + 2 * s + h] : 0.f;
 
     int nkv = (a.Skv + kFBK - 1) / kFBK;
     if (CAUSAL) {
@@ -168,7 +175,7 @@ __global__ __launch_bounds__(256, 2) void fa_f32_mfma_kernel(FaArgs a, float sca
     const float l_tot = half_sum(l_run);
     const float inv = l_tot > 1e-10f ? 1.f / l_tot : 0.f;
     if (q_live) {
-        float* orow = op + qpos * a.os[2];
+        float* orow = op + qpos * o_rs;
 #pragma unroll
         for (int d = 0; d < ND; d++)
 #pragma unroll
@@ -184,7 +191,7 @@ __global__ __launch_bounds__(256, 2) void fa_f32_mfma_kernel(FaArgs a, float sca
 // with a quarter of the chain; K and V go from memory straight to the operand registers (a lane's 16 bytes of
 // its key's row serve four issues: k = 8 j + 4 h + e on both operands), so there is no barrier in the loop, and
 // each set of registers is loaded again as soon as its product has read it, half a block ahead of its use.
-template <int D, bool CAUSAL, bool HAS_MASK>
+template <int D, bool CAUSAL, bool HAS_MASK, bool VIEWS>
 __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaArgs a, float scale) {
     constexpr int NS = D / 8, ND = D / 32;
     __shared__ float part[4][32][33];
@@ -195,11 +202,11 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaAr
     tile_of_workgroup<CAUSAL>(a, blockIdx.x, bh, qb);
     const int q0 = qb * 32, qpos = q0 + ln;
     const bool q_live = qpos < a.Sq;
-    const int b_i = bh / a.H, h_i = bh % a.H;
-    const float* qp = static_cast<const float*>(a.q) + b_i * a.qs[0] + h_i * a.qs[1];
-    const int k_rs = (int)a.ks[2], v_rs = (int)a.vs[2];
-    const __amdgpu_buffer_rsrc_t rk = fa_rsrc(static_cast<const float*>(a.k) + b_i * a.ks[0] + h_i * a.ks[1], (uint32_t)((((int64_t)a.Skv - 1) * k_rs + D) * 4));
-    const __amdgpu_buffer_rsrc_t rv = fa_rsrc(static_cast<const float*>(a.v) + b_i * a.vs[0] + h_i * a.vs[1], (uint32_t)((((int64_t)a.Skv - 1) * v_rs + D) * 4));
+    const float* qp = static_cast<const float*>(a.q) + head_at<VIEWS>(a, a.qs, bh, a.Sq * (int64_t)D);
+    const int64_t q_rs = VIEWS ? a.qs[2] : D, o_rs = VIEWS ? a.os[2] : D;
+    const int k_rs = VIEWS ? (int)a.ks[2] : D, v_rs = VIEWS ? (int)a.vs[2] : D;
+    const __amdgpu_buffer_rsrc_t rk = fa_rsrc(static_cast<const float*>(a.k) + head_at<VIEWS>(a, a.ks, bh, a.Skv * (int64_t)D), (uint32_t)((((int64_t)a.Skv - 1) * k_rs + D) * 4));
+    const __amdgpu_buffer_rsrc_t rv = fa_rsrc(static_cast<const float*>(a.v) + head_at<VIEWS>(a, a.vs, bh, a.Skv * (int64_t)D), (uint32_t)((((int64_t)a.Skv - 1) * v_rs + D) * 4));
     const float* mp = HAS_MASK ? static_cast<const float*>(a.mask) + (int64_t)(bh / a.H) * a.mask_sb +
                                      (int64_t)(bh % a.H) * a.mask_sh + (int64_t)min(qpos, a.Sq - 1) * a.Skv
                                : nullptr;
@@ -209,7 +216,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaAr
     f32x4 qf[NS];
 #pragma unroll
     for (int j = 0; j < NS; j++)
-        qf[j] = q_live ? *reinterpret_cast<const f32x4*>(qp + qpos * a.qs[2] + 8 * j + 4 * h) : f32x4{0.f, 0.f, 0.f, 0.f};
+        qf[j] = q_live ? *reinterpret_cast<const f32x4*>(qp + qpos * q_rs + 8 * j + 4 * h) : f32x4{0.f, 0.f, 0.f, 0.f};
 
     int nkv = (a.Skv + kFBK - 1) / kFBK;
     if (CAUSAL) nkv = min(nkv, qb + 1);
@@ -222,13 +229,15 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaAr
 #pragma unroll
         for (int j = 0; j < NS; j++) kr[j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, off + 32 * j, 0, 0));
     };
+    // (VIEWS: a key's row is a scalar offset, a column block an immediate one: nothing to compute per load)
     auto load_v = [&](int blk) __attribute__((always_inline)) {
         const uint32_t off = (uint32_t)((blk * kFBK + 4 * h) * (v_rs * 4) + 4 * ln);
 #pragma unroll
         for (int i = 0; i < 16; i++)
 #pragma unroll
             for (int d = 0; d < ND; d++)
-                vr[d][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, off + (uint32_t)((8 * (i >> 2) + (i & 3)) * (v_rs * 4) + 128 * d), 0, 0));
+                vr[d][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, off + (uint32_t)((VIEWS ? 0 : (8 * (i >> 2) + (i & 3)) * (D * 4)) + 128 * d),
+                                                                                              VIEWS ? (8 * (i >> 2) + (i & 3)) * (v_rs * 4) : 0, 0));
     };
 
     f32x16 o[ND];
@@ -294,7 +303,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaAr
     // ---- the waves' states, 32 columns of the output at a time
     l_run = half_sum(l_run);
     if (h == 0) { ml[0][wave][ln] = m_run; ml[1][wave][ln] = l_run; }
-    float* op = static_cast<float*>(a.o) + b_i * a.os[0] + h_i * a.os[1];
+    float* op = static_cast<float*>(a.o) + head_at<VIEWS>(a, a.os, bh, a.Sq * (int64_t)D);
     const int col = threadIdx.x & 31, row0 = threadIdx.x >> 5;
 #pragma unroll
     for (int d = 0; d < ND; d++) {
@@ -315,12 +324,12 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaAr
                 l = fmaf(ml[1][w][q], al, l);
                 sum = fmaf(part[w][q][col], al, sum);
             }
-            if (q0 + q < a.Sq) op[(q0 + q) * a.os[2] + 32 * d + col] = sum * (l > 1e-10f ? 1.f / l : 0.f);
+            if (q0 + q < a.Sq) op[(q0 + q) * o_rs + 32 * d + col] = sum * (l > 1e-10f ? 1.f / l : 0.f);
         }
     }
 }
 
-template <int D>
+template <int D, bool V>
 int launch_f32(hipStream_t s, FaArgs a, float scale, bool causal, bool has_mask) {
     // Keys over the waves while tiles of 128 rows leave compute units idle or nearly so (us, 128 rows | split, causal):
     // 12 tiles [1,12,128,64] 16.2 | 7.6; 64 [2,8,512,64] 48 | 16, D 128 83 | 29; 128 [1,8,2048,64] 175 | 50, D 128 302 | 114.
@@ -337,8 +346,8 @@ int launch_f32(hipStream_t s, FaArgs a, float scale, bool causal, bool has_mask)
     if (grid > 0x7FFFFFFFLL) return fail(MHIP_ERR_UNSUPPORTED, "flash_attention: grid too large");
 #define MHIP_FA32(C, M)                                                                                                     \
     do {                                                                                                                    \
-        if (split) hipLaunchKernelGGL((fa_f32_split_kernel<D, C, M>), dim3((unsigned)grid), dim3(256), 0, s, a, scale);     \
-        else hipLaunchKernelGGL((fa_f32_mfma_kernel<D, C, M>), dim3((unsigned)grid), dim3(256), 0, s, a, scale);            \
+        if (split) hipLaunchKernelGGL((fa_f32_split_kernel<D, C, M, V>), dim3((unsigned)grid), dim3(256), 0, s, a, scale);  \
+        else hipLaunchKernelGGL((fa_f32_mfma_kernel<D, C, M, V>), dim3((unsigned)grid), dim3(256), 0, s, a, scale);         \
     } while (0)
     if (causal && has_mask) MHIP_FA32(true, true);
     else if (causal) MHIP_FA32(true, false);
@@ -364,13 +373,13 @@ bool fa_f32_mfma_eligible(const FaArgs& a, int64_t D, bool packed) {
     return true;
 }
 
-int launch_fa_f32_mfma(hipStream_t s, const FaArgs& a, int64_t D, float scale) {
+int launch_fa_f32_mfma(hipStream_t s, const FaArgs& a, int64_t D, float scale, bool packed) {
     const bool causal = a.is_causal != 0, has_mask = a.mask != nullptr;
     switch (D) {
-        case 32: return launch_f32<32>(s, a, scale, causal, has_mask);
-        case 64: return launch_f32<64>(s, a, scale, causal, has_mask);
-        case 96: return launch_f32<96>(s, a, scale, causal, has_mask);
-        default: return launch_f32<128>(s, a, scale, causal, has_mask);
+        case 32: return packed ? launch_f32<32, false>(s, a, scale, causal, has_mask) : launch_f32<32, true>(s, a, scale, causal, has_mask);
+        case 64: return packed ? launch_f32<64, false>(s, a, scale, causal, has_mask) : launch_f32<64, true>(s, a, scale, causal, has_mask);
+        case 96: return packed ? launch_f32<96, false>(s, a, scale, causal, has_mask) : launch_f32<96, true>(s, a, scale, causal, has_mask);
+        default: return packed ? launch_f32<128, false>(s, a, scale, causal, has_mask) : launch_f32<128, true>(s, a, scale, causal, has_mask);
     }
 }
 
