@@ -60,8 +60,9 @@ struct StageLoader {
 
 // KG groups of four waves: a stage is KG x 64 k, group q multiplies its 64, the groups' sums meet in LDS at the
 // end.  S stages in the ring.
-template <typename T, int BM, int BN, int WGM, bool TA, bool TB, int KG, int S, bool AHEAD>
-__global__ __launch_bounds__(256 * KG) void gemm_mid_kernel(GemmArgs g, int sums_by_row) {
+// SUMS: each part's sums by row for mhip_gemm_sums, a kernel of its own (as an argument it cost the others 0.1 us a launch).
+template <typename T, int BM, int BN, int WGM, bool TA, bool TB, int KG, int S, bool AHEAD, bool SUMS>
+__global__ __launch_bounds__(256 * KG) void gemm_mid_kernel(GemmArgs g) {
     constexpr int WGN = 4 / WGM, WTM = BM / WGM, WTN = BN / WGN, TM = WTM / 32, TN = WTN / 32;
     constexpr int kATile = BM * kRowBytes, kPart = (BM + BN) * kRowBytes, kStage = KG * kPart;
     extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -170,7 +171,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_mid_kernel(GemmArgs g, int sums
         }
         if (group > 0) return;
     }
-    if (g.partial && sums_by_row) {
+    if constexpr (SUMS) {
         // [part][M][N]: a lane's row, four columns per store (two lanes' stores are 32 consecutive bytes)
         float* p = g.partial + (int64_t)blockIdx.z * g.M * g.N;
 #pragma unroll
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_mid_kernel(GemmArgs g, int sums
         }
         return;
     }
-    if (g.partial) {
+    if (!SUMS && g.partial) {
         // the block's registers as they are, 1 KB per store: block (i, j) of wave w of tile t, register group q
         f32x4* dst = reinterpret_cast<f32x4*>(g.partial) + ((((int64_t)blockIdx.z * g.tiles_m * g.tiles_n + tm * g.tiles_n + tn) * 4 + wave) * TM * TN) * 256 + lane;
 #pragma unroll
@@ -191,7 +192,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_mid_kernel(GemmArgs g, int sums
         }
         return;
     }
-    store_tile<T, TM, TN>(g, acc, smem + wave * (WTM * (WTN * 2 + 16)), m0 + wm * WTM, n0 + wn * WTN, batch, lane);
+    if constexpr (!SUMS) store_tile<T, TM, TN>(g, acc, smem + wave * (WTM * (WTN * 2 + 16)), m0 + wm * WTM, n0 + wn * WTN, batch, lane);
 }
 
 // C from the splits' sums in the accumulators' own layout (tiles of BM x BN, WGM x 4 / WGM waves): a wave of
@@ -316,12 +317,12 @@ __global__ __launch_bounds__(256) void gemm_finish_kernel(GemmArgs g) {
     });
 }
 
-template <typename T, int BM, int BN, int WGM, bool TA, bool TB, int KG, int S, bool AHEAD = false>
-int launch_tile(hipStream_t s, GemmArgs g, int64_t batch, bool by_row) {
+template <typename T, int BM, int BN, int WGM, bool TA, bool TB, bool SUMS, int KG, int S, bool AHEAD = false>
+int launch_tile(hipStream_t s, GemmArgs g, int64_t batch) {
     constexpr int kStage = KG * (BM + BN) * kRowBytes, kRing = S * kStage, kSums = KG / 2 * BM * BN * 4, kOut = 4 * (BM / WGM) * ((BN / (4 / WGM)) * 2 + 16);
     constexpr int kUse = kRing > kOut ? kRing : kOut, kSmem = kUse > kSums ? kUse : kSums;
     static_assert(kSmem <= 160 * 1024, "ring larger than LDS");
-    auto kern = gemm_mid_kernel<T, BM, BN, WGM, TA, TB, KG, S, AHEAD>;
+    auto kern = gemm_mid_kernel<T, BM, BN, WGM, TA, TB, KG, S, AHEAD, SUMS>;
     static std::once_flag once;
     static hipError_t err = hipSuccess;
     std::call_once(once, [&] { err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kSmem); });
@@ -330,7 +331,7 @@ int launch_tile(hipStream_t s, GemmArgs g, int64_t batch, bool by_row) {
     g.tiles_n = (g.N + BN - 1) / BN;
     const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n;
     if (tiles > 0x7FFFFFFFLL || batch > 65535) return fail(MHIP_ERR_UNSUPPORTED, "gemm: grid too large");
-    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)batch, (unsigned)g.splits), dim3(256 * KG), kSmem, s, g, by_row ? 1 : 0);
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)batch, (unsigned)g.splits), dim3(256 * KG), kSmem, s, g);
     return check_launch("gemm_mid");
 }
 
@@ -401,20 +402,20 @@ int64_t plan_bytes(const MidPlan& p, int64_t M, int64_t N) {
     return p.splits == 1 ? 0 : ((M + f.bm - 1) / f.bm) * ((N + f.bn - 1) / f.bn) * f.bm * f.bn * 4 * p.splits;
 }
 
-template <typename T, bool TA, bool TB>
-int launch_form(hipStream_t s, const GemmArgs& g, int64_t batch, int form, bool by_row = false) {
+template <typename T, bool TA, bool TB, bool SUMS = false>
+int launch_form(hipStream_t s, const GemmArgs& g, int64_t batch, int form) {
     // one workgroup per compute unit or fewer: all of LDS for a ring of four that reads ahead; otherwise the ring that two
     // workgroups of a unit share ([2000,2000] x K 2000, 256 of 128x128, 29.7 -> 26.6 us; [1000,3000] x K 1000, 384 of 64x128,
     // 16.4 against 20.2; tiles of 64x64 lose by it, [1000,1000] x K 1000 7.9 against 8.6)
     const Form& f = kForms[form];
     const bool one_each = ((g.M + f.bm - 1) / f.bm) * (int64_t)((g.N + f.bn - 1) / f.bn) * batch * g.splits <= 256;
     switch (form) {
-        case 0: return launch_tile<T, 64, 64, 2, TA, TB, 2, 3>(s, g, batch, by_row);
-        case 1: return launch_tile<T, 64, 128, 2, TA, TB, 2, 3>(s, g, batch, by_row);
-        case 2: return launch_tile<T, 128, 128, 2, TA, TB, 2, 2>(s, g, batch, by_row);
-        case 3: return launch_tile<T, 64, 64, 2, TA, TB, 1, 4>(s, g, batch, by_row);
-        case 4: return one_each ? launch_tile<T, 64, 128, 2, TA, TB, 1, 4, true>(s, g, batch, by_row) : launch_tile<T, 64, 128, 2, TA, TB, 1, 3>(s, g, batch, by_row);
-        default: return one_each ? launch_tile<T, 128, 128, 2, TA, TB, 1, 4, true>(s, g, batch, by_row) : launch_tile<T, 128, 128, 2, TA, TB, 1, 2>(s, g, batch, by_row);
+        case 0: return launch_tile<T, 64, 64, 2, TA, TB, SUMS, 2, 3>(s, g, batch);
+        case 1: return launch_tile<T, 64, 128, 2, TA, TB, SUMS, 2, 3>(s, g, batch);
+        case 2: return launch_tile<T, 128, 128, 2, TA, TB, SUMS, 2, 2>(s, g, batch);
+        case 3: return launch_tile<T, 64, 64, 2, TA, TB, SUMS, 1, 4>(s, g, batch);
+        case 4: return one_each ? launch_tile<T, 64, 128, 2, TA, TB, SUMS, 1, 4, true>(s, g, batch) : launch_tile<T, 64, 128, 2, TA, TB, SUMS, 1, 3>(s, g, batch);
+        default: return one_each ? launch_tile<T, 128, 128, 2, TA, TB, SUMS, 1, 4, true>(s, g, batch) : launch_tile<T, 128, 128, 2, TA, TB, SUMS, 1, 2>(s, g, batch);
     }
 }
 
@@ -490,5 +491,5 @@ extern "C" int mhip_gemm_sums(void* stream, const void* a, const void* b, float*
     g.M = (int)M; g.N = (int)N; g.K = (int)K; g.lda = (int)K; g.ldb = (int)N;
     const MidPlan p = plan_sums(M, N, K, parts);
     g.splits = p.splits;
-    return dtype == MHIP_BF16 ? launch_form<bf16_t, false, false>(as_stream(stream), g, 1, p.form, true) : launch_form<f16_t, false, false>(as_stream(stream), g, 1, p.form, true);
+    return dtype == MHIP_BF16 ? launch_form<bf16_t, false, false, true>(as_stream(stream), g, 1, p.form) : launch_form<f16_t, false, false, true>(as_stream(stream), g, 1, p.form);
 }
