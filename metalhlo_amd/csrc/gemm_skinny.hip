@@ -104,9 +104,10 @@ template <typename T, int VE, bool VEC> struct RowPiece {
 
 // Whether neighbouring strips go to one XCD: rows of a strip that are half a line or less, whose other half the same L2 then holds for the
 // neighbour.  us, without | with: [1,6720] x K 832 bf16 5.9 | 5.0, [8,1024] x K 4096 bf16 9.3 | 8.8, [16,6720] x K 832 fp32
-// 10.4 | 9.0; strips of 128 or 192 bytes lose by it, [4,4096] x K 4096 bf16 11.0 | 11.3, [128,3072] x K 768 fp32 11.5 | 12.0.
-template <typename T, bool TB, int NF>
-constexpr bool strip_order() { return !TB && 16 * NF * (int)sizeof(T) < 128; }
+// 10.4 | 9.0; strips of 128 or 192 bytes lose by it, [4,4096] x K 4096 bf16 11.0 | 11.3, [128,3072] x K 768 fp32 11.5 | 12.0, and
+// so do blocks of 32 fp32 rows, [100,512] x K 2048 11.8 | 12.2, [190,256] x K 2048 12.0 | 12.6.
+template <typename T, bool TB, int NF, int MT>
+constexpr bool strip_order() { return !TB && 16 * NF * (int)sizeof(T) < 128 && (sizeof(T) == 2 || MT == 1); }
 
 // NF = operands (groups of 16 columns) per strip, MT = groups of 16 rows, U = k steps loaded as one block.
 template <typename T, bool TB, bool VEC, int NF, int MT, int U, int WAVES>
@@ -117,8 +118,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(GemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) float part[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     const int li = lane & 15, lg = lane >> 4;
-    const int strip = strip_order<T, TB, NF>() ? (int)(blockIdx.x % kXcds * (gridDim.x / kXcds) + blockIdx.x / kXcds) : (int)blockIdx.x, n0 = strip * NS;
-    if (strip_order<T, TB, NF>() && n0 >= g.N) return;
+    const int strip = strip_order<T, TB, NF, MT>() ? (int)(blockIdx.x % kXcds * (gridDim.x / kXcds) + blockIdx.x / kXcds) : (int)blockIdx.x, n0 = strip * NS;
+    if (strip_order<T, TB, NF, MT>() && n0 >= g.N) return;
     int batch_i = blockIdx.y, m0 = 0;
     if (g.tiles_m > 1) { m0 = batch_i % g.tiles_m * (16 * MT); batch_i /= g.tiles_m; }
     const int64_t batch = batch_i;
@@ -254,7 +255,7 @@ int launch_one(hipStream_t s, GemmArgs g, int64_t batch) {
     const int waves = want < 1 ? 1 : want > WAVES ? WAVES : want;
     const int64_t strips = (g.N + 16 * NF - 1) / (16 * NF);
     g.tiles_m = (g.M + 16 * MT - 1) / (16 * MT);
-    const int64_t grid = strip_order<T, TB, NF>() ? (strips + kXcds - 1) / kXcds * kXcds : strips;
+    const int64_t grid = strip_order<T, TB, NF, MT>() ? (strips + kXcds - 1) / kXcds * kXcds : strips;
     if (grid > 0x7FFFFFFFLL || batch * g.tiles_m > 65535) return fail(MHIP_ERR_UNSUPPORTED, "gemm: grid too large");
     hipLaunchKernelGGL(kern, dim3((unsigned)grid, (unsigned)(batch * g.tiles_m), (unsigned)g.splits), dim3(64 * waves), waves * NF * MT * 1024, s, g);
     return check_launch("gemm_skinny");
@@ -278,8 +279,31 @@ bool wide_strips(int64_t N, int64_t K, int64_t batch, bool tb) {
 //   fp32, up to 32 rows            K 2048 0.82 to 1.31   K 2560 0.70 to 1.08   K 3064 0.66 to 1.02
 //   fp32, 64 rows                  K 2560 0.87 to 1.38   K 3064 0.82 to 1.26   K 3584 0.69 to 1.14
 // Blocks of more than 64 rows (fp32) fill the device earlier ([128,3072] x [3072,768] 16.4 us whole, 20.5) and keep 2048 k.
+//
+// fp32 of 33 to 64 rows from K 3000 on, of more from K 3500 on: the block, 16 x 48 or 32 x 32, whose number times the parts comes
+// closest to one workgroup per compute unit, if that leaves few of them idle.  us, before | 16 x 48 / parts (workgroups) | 32 x 32 / parts:
+//   [48,768] x K 3072  15.2 | 11.9 / 4 (192) | 13.1 / 4 (192)      [128,1024] x K 4096 24.3 | 24.6 / 1 (176) | 19.8 / 2 (256)
+//   [64,1024] x K 4096 17.0 | -              | 14.8 / 4 (256)      [70,1024] x K 4096  23.4 | 21.8 / 2 (220) | 19.7 / 2 (192)
+// Shorter: [40,2048] x K 2048 12.3 | 14.4, [60,3000] x K 2500 22.4 | 24.1, [150,512] x K 2048 11.9 | 12.6, [128,768] x K 3072 16.6 | 15.1
+// for one more launch; below 216 workgroups: [160,640] x K 2560 15.0 whole | - | 15.9 / 2 (200).
+struct RowsPlan { int rows = 0, cols = 0, splits = 1; };
+RowsPlan rows_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool tb) {
+    RowsPlan best;
+    if (batch != 1 || M <= 32 || K < (M <= 64 ? 3000 : 3500)) return best;
+    int64_t most = 215;
+    auto consider = [&](int rows, int cols) {
+        const int64_t blocks = (M + rows - 1) / rows * ((N + cols - 1) / cols), room = 256 / blocks, parts = room < K / 512 ? room : K / 512;
+        const int64_t s = parts > 8 ? 8 : parts;
+        if (s >= 2 && blocks * s > most) { most = blocks * s; best.rows = rows; best.cols = cols; best.splits = (int)s; }
+    };
+    if (!tb && K % 4 == 0 && N % 4 == 0) consider(16, 48);
+    consider(32, 32);
+    return best;
+}
+
 int skinny_splits(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b, bool is16) {
     if (batch != 1 || M * N > (1 << 20)) return 1;
+    if (!is16 && rows_plan(M, N, K, batch, trans_b != 0).splits > 1) return rows_plan(M, N, K, batch, trans_b != 0).splits;
     const int64_t width = wide_strips(N, K, 1, trans_b != 0) ? (trans_b ? 32 : 64) : (trans_b ? 16 : 32);
     const int64_t from = is16 ? (trans_b && M <= 16 ? 3584 : 2560) : (M > 32 ? 3072 : 2560);
     const int64_t want = M > 64 ? K / 2048 + (K % 2048 > 1024) : K >= from ? (K + 512) / 1024 : 1;
@@ -306,12 +330,18 @@ int launch_shape(hipStream_t s, const GemmArgs& g, int64_t batch) {
         //   [192,2304] x K 768    16.5 (864)    16.3 (576)    14.4 (432)    17.5 (288)
         // Wide: [64,8192] x K 4096 59.1 in 32 x 32, 52.3 in 64 rows.  Up to 64 rows a split K fills the device as it is:
         // [36,768] x K 8192 24.4 in 32 x 16, 20.8 in 64 rows.  (Stored [K, N] a strip of 48 columns is three per lane.)
+        const RowsPlan plan = rows_plan(g.M, g.N, g.K, batch, TB);
+        if (g.splits > 1 && plan.splits == g.splits) {
+            if constexpr (VEC && !TB) if (plan.cols == 48) return launch_one<T, TB, VEC, 3, 1, 2>(s, g, batch);
+            return launch_one<T, TB, VEC, 2, 2, 2>(s, g, batch);
+        }
         if (g.M > 32 && (g.M > 64 || g.splits == 1)) {
             auto blocks = [&](int rows, int cols) { return (int64_t)((g.M + rows - 1) / rows) * ((g.N + cols - 1) / cols) * batch; };
             constexpr bool k48 = VEC && !TB;
             if (blocks(32, 16) <= 256) return launch_one<T, TB, VEC, 1, 2, 2>(s, g, batch);
-            if constexpr (k48) if (blocks(16, 48) <= 256) return launch_one<T, TB, VEC, 3, 1, 2>(s, g, batch);
-            if constexpr (k48) if (blocks(32, 32) > 256 && blocks(32, 48) <= 256) return launch_one<T, TB, VEC, 3, 2, 2>(s, g, batch);
+            // (48 columns where rows start on lines: [60,3000] x K 2500 22.5 in 32 x 32, 24.1)
+            if constexpr (k48) if (g.N % 32 == 0 && blocks(16, 48) <= 256) return launch_one<T, TB, VEC, 3, 1, 2>(s, g, batch);
+            if constexpr (k48) if (g.N % 32 == 0 && blocks(32, 32) > 256 && blocks(32, 48) <= 256) return launch_one<T, TB, VEC, 3, 2, 2>(s, g, batch);
             if (!wide) return launch_one<T, TB, VEC, 2, 2, 2>(s, g, batch);
         }
     }

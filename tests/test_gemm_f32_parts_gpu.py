@@ -42,7 +42,7 @@ def test_parts_have_the_bits_of_the_whole(N, K, ta, tb):
     assert torch.equal(product(8000, False, True)[0][:rows], whole)
 
 
-@pytest.mark.parametrize("M,N,K", [(33, 2308, 20), (48, 3068, 132), (100, 1540, 516), (65, 2308, 36), (128, 3076, 772), (192, 772, 1028), (128, 2304, 3072)], ids=lambda v: str(v))
+@pytest.mark.parametrize("M,N,K", [(33, 2336, 20), (48, 3104, 132), (100, 1568, 516), (65, 2336, 36), (128, 3104, 772), (192, 800, 1028), (128, 2304, 3072), (48, 3068, 132)], ids=lambda v: str(v))
 def test_strips_of_48_columns(M, N, K):
     """Few-row products whose strips are three columns a lane, the last strip ragged."""
     _check(M, N, K, torch.float32, False, False, residual=M % 2 == 0)
@@ -51,3 +51,9 @@ def test_strips_of_48_columns(M, N, K):
 @pytest.mark.parametrize("M,N,K,tb", [(33, 2304, 1025, True), (48, 2303, 1024, False), (100, 767, 3073, True), (192, 101, 1030, False), (32, 767, 1025, True)], ids=lambda v: str(v))
 def test_few_rows_off_16_bytes(M, N, K, tb):
     _check(M, N, K, torch.float32, False, tb, residual=M % 2 == 0)
+
+
+@pytest.mark.parametrize("M,N,K,tb", [(33, 768, 2048, False), (48, 772, 3076, False), (128, 768, 3072, False), (100, 512, 2052, False), (64, 1024, 4096, True),
+                                      (128, 511, 2047, True), (128, 1024, 4096, False)], ids=lambda v: str(v))
+def test_few_rows_with_blocks_and_parts_chosen_together(M, N, K, tb):
+    _check(M, N, K, torch.float32, False, tb, residual=M % 8 == 0)
