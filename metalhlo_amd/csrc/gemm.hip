@@ -695,7 +695,7 @@ extern "C" int64_t mhip_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t 
     // (a large problem goes to the ring kernels, whose tiles fill the device)
     if (!is16) return gemm_f32_workspace(M, N, K, batch, trans_a, trans_b);
     if (!vec && pack_pays(M, N, K)) {
-        // (whether a pointer is off 16 bytes is not known here: room for both copies)
+        // (from the sizes; where a pointer is off 16 bytes besides, a copy more may not fit, and the rows are read as they are)
         GemmArgs g = {};
         g.M = (int)M; g.N = (int)N; g.K = (int)K; g.lda = (int)(trans_a ? M : K); g.ldb = (int)(trans_b ? K : N);
         const GemmPack p = gemm_pack_plan(g, trans_a, trans_b, g.lda % 8 != 0, g.ldb % 8 != 0);
