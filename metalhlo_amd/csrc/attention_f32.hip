@@ -229,15 +229,14 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_f32_split_kernel(FaAr
 #pragma unroll
         for (int j = 0; j < NS; j++) kr[j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, off + 32 * j, 0, 0));
     };
-    // (VIEWS: a key's row is a scalar offset, a column block an immediate one: nothing to compute per load)
+    // (a key's row is part of the vector offset: a scalar offset is outside the bounds check, and keys past the end must read zero)
     auto load_v = [&](int blk) __attribute__((always_inline)) {
         const uint32_t off = (uint32_t)((blk * kFBK + 4 * h) * (v_rs * 4) + 4 * ln);
 #pragma unroll
         for (int i = 0; i < 16; i++)
 #pragma unroll
             for (int d = 0; d < ND; d++)
-                vr[d][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, off + (uint32_t)((VIEWS ? 0 : (8 * (i >> 2) + (i & 3)) * (D * 4)) + 128 * d),
-                                                                                              VIEWS ? (8 * (i >> 2) + (i & 3)) * (v_rs * 4) : 0, 0));
+                vr[d][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, off + (uint32_t)((8 * (i >> 2) + (i & 3)) * (v_rs * 4) + 128 * d), 0, 0));
     };
 
     f32x16 o[ND];

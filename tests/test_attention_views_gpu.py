@@ -37,6 +37,28 @@ def test_views_give_the_bits_of_packed_tensors(dtype, D, B, H, S):
         assert torch.equal(out.permute(0, 2, 1, 3), want)
 
 
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 32), (torch.float32, 64), (torch.float32, 128), (torch.bfloat16, 32), (torch.float16, 72)])
+@pytest.mark.parametrize("B,H", [(2, 3), (24, 12)])
+@pytest.mark.parametrize("S", [1, 5, 27, 28, 33, 40])
+def test_nothing_behind_the_last_key_counts(dtype, D, B, H, S):
+    """Rows of NaN behind the last key of every sequence, the other sequences' rows among them: a view reads what it spans."""
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(S + D)
+    rows, W = S + 96, 3 * H * D
+    x = torch.full((B, rows, 3, H, D), float("nan"), dtype=dtype, device="cuda")
+    x[:, :S] = torch.randn(B, S, 3, H, D, generator=g, device="cuda").to(dtype)
+    q, k, v = x[:, :S].permute(2, 0, 3, 1, 4).unbind(0)
+    st = (C.c_int64 * 12)(*([rows * W, D, W] * 3 + [S * H * D, D, H * D]))
+    for causal in (False, True):
+        want = kernels.flash_attention(q.contiguous(), k.contiguous(), v.contiguous(), is_causal=causal)
+        out = torch.full((B, S, H, D), float("nan"), dtype=dtype, device="cuda")
+        assert lib.mhip_flash_attention_views(torch.cuda.current_stream().cuda_stream, q.data_ptr(), k.data_ptr(), v.data_ptr(), None, out.data_ptr(),
+                                              B, H, S, S, D, D ** -0.5, int(causal), 0, 0, CODE[dtype], C.addressof(st)) == 0
+        got = out.permute(0, 2, 1, 3)
+        assert torch.isfinite(got).all()
+        assert torch.equal(got, want)
+
+
 def test_refused_views():
     lib = _lib.load()
     x = torch.zeros(4096, dtype=torch.float32, device="cuda")
