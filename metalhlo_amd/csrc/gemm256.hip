@@ -78,8 +78,8 @@ __global__ __launch_bounds__(256) void gemm256_kernel(GemmArgs g) {
     T* c = static_cast<T*>(g.c) + batch * g.sc;
     const T* res = g.residual ? static_cast<const T*>(g.residual) + batch * g.sc : nullptr;
     // (extents to the last element: the matrices may be column slices of wider ones)
-    const uint32_t a_bytes = (uint32_t)(((int64_t)((TA ? g.K : g.M) - 1) * g.lda + (TA ? g.M : g.K)) * 2);
-    const uint32_t b_bytes = (uint32_t)(((int64_t)((TB ? g.N : g.K) - 1) * g.ldb + (TB ? g.K : g.N)) * 2);
+    const uint32_t a_bytes = (uint32_t)operand_bytes(TA ? g.K : g.M, TA ? g.M : g.K, g.lda);
+    const uint32_t b_bytes = (uint32_t)operand_bytes(TB ? g.N : g.K, TB ? g.K : g.N, g.ldb);
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
@@ -337,8 +337,8 @@ bool gemm256_eligible(const GemmArgs& g, int64_t batch, int trans_a, int trans_b
     if (g.bias && (reinterpret_cast<uintptr_t>(g.bias) & 7) != 0) return false;
     // (the extents the kernel puts into its buffer descriptors: the last stored row ends the operand;
     // a column slice keeps the row stride of the whole matrix)
-    const int64_t a_bytes = ((int64_t)((trans_a ? g.K : g.M) - 1) * g.lda + (trans_a ? g.M : g.K)) * 2;
-    const int64_t b_bytes = ((int64_t)((trans_b ? g.N : g.K) - 1) * g.ldb + (trans_b ? g.K : g.N)) * 2;
+    const int64_t a_bytes = operand_bytes(trans_a ? g.K : g.M, trans_a ? g.M : g.K, g.lda);
+    const int64_t b_bytes = operand_bytes(trans_b ? g.N : g.K, trans_b ? g.K : g.N, g.ldb);
     if (a_bytes >= 0x70000000LL || b_bytes >= 0x70000000LL) return false;
     const int tile_rows = bw == 192 ? 128 : 256;
     const int64_t tiles = (int64_t)((g.M + tile_rows - 1) / tile_rows) * ((g.N + bw - 1) / bw) * batch;

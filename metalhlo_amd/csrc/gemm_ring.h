@@ -27,6 +27,10 @@ __device__ inline void static_for(F&& f) {
     static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
+// Bytes that a descriptor spans of an operand of `rows` stored rows of `cols` elements: up to the end of the last 16-byte piece that
+// holds an element.  (Rows are whole pieces: of an operand whose columns are not, a copy is multiplied, with zeros behind them.)
+__host__ __device__ inline int64_t operand_bytes(int64_t rows, int64_t cols, int64_t ld) { return ((rows - 1) * ld + (cols + 7) / 8 * 8) * 2; }
+
 // ---- operand with k contiguous in memory --------------------------------------
 // One load instruction of wave w in pass p fills rows 64p + 16w .. +15 (64 bytes
 // each): lane -> row (lane >> 2), position (lane & 3).

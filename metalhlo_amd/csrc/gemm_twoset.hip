@@ -184,8 +184,8 @@ __global__ __launch_bounds__(256) void gemm384_kernel(GemmArgs g) {
     const char* b = reinterpret_cast<const char*>(static_cast<const T*>(g.b) + batch * g.sb);
     T* c = static_cast<T*>(g.c) + batch * g.sc;
     const T* res = g.residual ? static_cast<const T*>(g.residual) + batch * g.sc : nullptr;
-    const uint32_t a_bytes = (uint32_t)(((int64_t)((TA ? g.K : g.M) - 1) * g.lda + (TA ? g.M : g.K)) * 2);
-    const uint32_t b_bytes = (uint32_t)(((int64_t)((TB ? g.N : g.K) - 1) * g.ldb + (TB ? g.K : g.N)) * 2);
+    const uint32_t a_bytes = (uint32_t)operand_bytes(TA ? g.K : g.M, TA ? g.M : g.K, g.lda);
+    const uint32_t b_bytes = (uint32_t)operand_bytes(TB ? g.N : g.K, TB ? g.K : g.N, g.ldb);
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
@@ -281,8 +281,8 @@ __global__ __launch_bounds__(256, 2) void gemm_pair_kernel(GemmArgs g) {
     const char* b = reinterpret_cast<const char*>(static_cast<const T*>(g.b) + batch * g.sb);
     T* c = static_cast<T*>(g.c) + batch * g.sc;
     const T* res = g.residual ? static_cast<const T*>(g.residual) + batch * g.sc : nullptr;
-    const uint32_t a_bytes = (uint32_t)(((int64_t)((TA ? g.K : g.M) - 1) * g.lda + (TA ? g.M : g.K)) * 2);
-    const uint32_t b_bytes = (uint32_t)(((int64_t)((TB ? g.N : g.K) - 1) * g.ldb + (TB ? g.K : g.N)) * 2);
+    const uint32_t a_bytes = (uint32_t)operand_bytes(TA ? g.K : g.M, TA ? g.M : g.K, g.lda);
+    const uint32_t b_bytes = (uint32_t)operand_bytes(TB ? g.N : g.K, TB ? g.K : g.N, g.ldb);
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
@@ -538,8 +538,8 @@ __global__ __launch_bounds__(256) void gemm192_kernel(GemmArgs g) {
     const char* b = reinterpret_cast<const char*>(static_cast<const T*>(g.b) + batch * g.sb + skip_b);
     T* c = static_cast<T*>(g.c) + batch * g.sc;
     const T* res = g.residual ? static_cast<const T*>(g.residual) + batch * g.sc : nullptr;
-    const uint32_t a_bytes = (uint32_t)(((int64_t)((TA ? g.K : g.M) - 1) * g.lda + (TA ? g.M : g.K) - skip_a) * 2);
-    const uint32_t b_bytes = (uint32_t)(((int64_t)((TB ? g.N : g.K) - 1) * g.ldb + (TB ? g.K : g.N) - skip_b) * 2);
+    const uint32_t a_bytes = (uint32_t)(operand_bytes(TA ? g.K : g.M, TA ? g.M : g.K, g.lda) - skip_a * 2);
+    const uint32_t b_bytes = (uint32_t)(operand_bytes(TB ? g.N : g.K, TB ? g.K : g.N, g.ldb) - skip_b * 2);
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
@@ -747,8 +747,8 @@ __global__ __launch_bounds__(256) void gemm288_kernel(GemmArgs g) {
     const char* b = reinterpret_cast<const char*>(static_cast<const T*>(g.b) + batch * g.sb);
     T* c = static_cast<T*>(g.c) + batch * g.sc;
     const T* res = g.residual ? static_cast<const T*>(g.residual) + batch * g.sc : nullptr;
-    const uint32_t a_bytes = (uint32_t)(((int64_t)((TA ? g.K : g.M) - 1) * g.lda + (TA ? g.M : g.K)) * 2);
-    const uint32_t b_bytes = (uint32_t)(((int64_t)((TB ? g.N : g.K) - 1) * g.ldb + (TB ? g.K : g.N)) * 2);
+    const uint32_t a_bytes = (uint32_t)operand_bytes(TA ? g.K : g.M, TA ? g.M : g.K, g.lda);
+    const uint32_t b_bytes = (uint32_t)operand_bytes(TB ? g.N : g.K, TB ? g.K : g.N, g.ldb);
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;

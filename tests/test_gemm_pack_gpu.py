@@ -60,3 +60,24 @@ def test_copies_from_a_graph():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tile", [2560, 2561, 2564, 2566, 2567, 2568, 2569, 2570])
+@pytest.mark.parametrize("ta", [0, 1])
+def test_the_last_row_of_k_ends_in_an_odd_column(monkeypatch, dtype, tile, ta):
+    """The descriptors of the ring kernels reach the last element of a copied row whose length is odd: only the last k is not zero."""
+    lib, code = _lib.load(), kernels.DTYPE_CODE[dtype]
+    M, N, K = 3841 if ta else 3848, 6273, 3008               # 192 tiles of 256x384; K is whole stages, so nothing is padded behind it
+    g = torch.Generator(device="cuda").manual_seed(tile)
+    a, b = torch.zeros((K, M) if ta else (M, K), dtype=dtype, device="cuda"), torch.zeros(K, N, dtype=dtype, device="cuda")
+    u, v = torch.randn(M, generator=g, device="cuda").to(dtype), torch.randn(N, generator=g, device="cuda").to(dtype)
+    a[K - 1 if ta else slice(None), slice(None) if ta else K - 1] = u
+    b[K - 1] = v
+    need = lib.mhip_gemm_workspace(M, N, K, 1, ta, 0, code)
+    work, out = torch.full((need,), 255, dtype=torch.uint8, device="cuda"), torch.empty(M, N, dtype=dtype, device="cuda")
+    monkeypatch.setenv("MHIP_GEMM_TILE", str(tile))
+    assert lib.mhip_gemm_ws(torch.cuda.current_stream().cuda_stream, a.data_ptr(), b.data_ptr(), None, None, out.data_ptr(), M, N, K, 1, 0, 0, 0, ta, 0, 0, code,
+                            work.data_ptr(), need) == 0
+    assert lib.mhip_gemm_last_variant() == tile
+    assert torch.equal(out, (u.float()[:, None] * v.float()[None, :]).to(dtype))
