@@ -496,7 +496,7 @@ bool fa_decode_eligible(const FaArgs& a);
 int64_t fa_decode_workspace(int64_t bh, int64_t Sq, int64_t Skv, int64_t D);
 int launch_fa_decode(hipStream_t s, const FaArgs& a, int64_t D, int dtype, void* workspace, int64_t workspace_bytes);
 // attention_flow.hip: head sizes 64 and 128 without a mask, few tiles.
-bool fa_flow_wanted(const FaArgs& a);
+bool fa_flow_wanted(const FaArgs& a, int64_t D);
 int launch_fa_flow(hipStream_t s, FaArgs a, int64_t D, int dtype);
 // attention_f32.hip: fp32 tensors on the fp32 matrix instruction.
 bool fa_f32_mfma_eligible(const FaArgs& a, int64_t D, bool packed);
@@ -559,7 +559,7 @@ static int fa_entry(const char* name, void* stream, const void* q, const void* k
         if (variant == 0 && fa_decode_eligible(a) && B * H <= 0x7FFFFFFF) return launch_fa_decode(s, a, D, dtype, workspace, workspace_bytes);
         if (is_packed && fa_pipe_eligible(a, D, dtype, hm, variant))
             return launch_fa_pipe(s, a, dtype, is_causal != 0, variant == 2 ? 0 : variant == 3 ? 1 : -1);
-        if (!hm && fa_flow_wanted(a)) return launch_fa_flow(s, a, D, dtype);
+        if (!hm && fa_flow_wanted(a, D)) return launch_fa_flow(s, a, D, dtype);
         if (dtype == MHIP_BF16)
             return D == 128 ? launch_fa<bf16_t, 128>(s, a, is_causal, hm)
                             : launch_fa<bf16_t, 64>(s, a, is_causal, hm);

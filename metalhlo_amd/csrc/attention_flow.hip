@@ -15,8 +15,12 @@ namespace mhip {
 namespace {
 
 // A ring of NB tiles for K and for V; K's tiles are a block ahead of V's.
+//
+// Nothing may be spilled: a reload waits for every load in flight, the tiles just asked for among them.  With head size 128 and no
+// causal rule the compiler does not fit a wave into the 256 registers of two workgroups a unit (9 spilled, [1,12,1024] 34.3 us);
+// one workgroup a unit has 512 (25.3; fa_fwd_kernel 26.4).
 template <typename T, int D, bool CAUSAL>
-__global__ __launch_bounds__(256, 2) void fa_flow_kernel(FaArgs a) {
+__global__ __launch_bounds__(256, D == 128 && !CAUSAL ? 1 : 2) void fa_flow_kernel(FaArgs a) {
     constexpr int NB = 2;
     constexpr int CPR = D / 8;                  // 16-byte chunks per row
     constexpr int kTile = kBKV * D * 2;         // bytes of one K (or V) tile
@@ -41,8 +45,12 @@ __global__ __launch_bounds__(256, 2) void fa_flow_kernel(FaArgs a) {
     T* op = static_cast<T*>(a.o) + b_i * a.os[0] + h_i * a.os[1];
     const int q_rs = (int)a.qs[2], k_rs = (int)a.ks[2], v_rs = (int)a.vs[2];      // row pitches in elements
     const __amdgpu_buffer_rsrc_t rq = fa_rsrc(qp, (uint32_t)((((int64_t)a.Sq - 1) * q_rs + D) * 2));
-    const __amdgpu_buffer_rsrc_t rk = fa_rsrc(kp, (uint32_t)((((int64_t)a.Skv - 1) * k_rs + D) * 2));
-    const __amdgpu_buffer_rsrc_t rv = fa_rsrc(vp, (uint32_t)((((int64_t)a.Skv - 1) * v_rs + D) * 2));
+    int nkv = (a.Skv + kBKV - 1) / kBKV;
+    if (CAUSAL) nkv = min(nkv, (min(qblk0 + kBQ, a.Sq) - 1) / kBKV + 1);
+    // (the last block's loads ask for blocks behind it: nothing is fetched past the keys this workgroup sees)
+    const int keys = CAUSAL ? min(a.Skv, nkv * kBKV) : a.Skv;
+    const __amdgpu_buffer_rsrc_t rk = fa_rsrc(kp, (uint32_t)((((int64_t)keys - 1) * k_rs + D) * 2));
+    const __amdgpu_buffer_rsrc_t rv = fa_rsrc(vp, (uint32_t)((((int64_t)keys - 1) * v_rs + D) * 2));
 
     // ---- Q^T operand: lane = query column, 8 consecutive d per k-step
     u32x4 qf[NS];
@@ -55,8 +63,6 @@ __global__ __launch_bounds__(256, 2) void fa_flow_kernel(FaArgs a) {
         }
     }
 
-    int nkv = (a.Skv + kBKV - 1) / kBKV;
-    if (CAUSAL) nkv = min(nkv, (min(qblk0 + kBQ, a.Sq) - 1) / kBKV + 1);
     // blocks that this wave multiplies: the rest of the workgroup's it only helps to load
     const int mine = CAUSAL ? min(nkv, (qw + 31) / kBKV + 1) : nkv;
 
@@ -82,7 +88,7 @@ __global__ __launch_bounds__(256, 2) void fa_flow_kernel(FaArgs a) {
     // loads land in program order: K of the next block but one and V of the next have landed when only the pairs issued behind
     // them are in flight
     auto tiles_ready = [&]() __attribute__((always_inline)) {
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 2) * 2 * kInst) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NB - 2) * 2 * kInst) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
@@ -244,7 +250,11 @@ __global__ __launch_bounds__(256, 2) void fa_flow_kernel(FaArgs a) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // nothing may land in LDS after the workgroup ends
 
     // ---- normalise and store: lane holds 4 consecutive d per register group
-    const float l_tot = half_sum(l_run);
+    // (half_sum with the lane's half counted anew: kept from the start it was the one register too many of head size 128, causal)
+    const unsigned lsum = __builtin_bit_cast(unsigned, l_run);
+    const auto lr = __builtin_amdgcn_permlane32_swap(lsum, lsum, false, false);
+    const int el = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    const float l_tot = l_run + __builtin_bit_cast(float, (el & 32) ? lr[0] : lr[1]);
     const float inv = l_tot > 1e-10f ? 1.f / l_tot : 0.f;
     if (qpos < a.Sq) {
         T* orow = op + (int64_t)qpos * a.os[2];
@@ -269,15 +279,24 @@ int launch_form(hipStream_t s, const FaArgs& a, unsigned grid) {
 
 }  // namespace
 
-// 16-bit q, k, v, o of head size 64 or 128 with 16-byte aligned rows and no mask, while two workgroups a compute unit hold all
-// tiles.  Beyond that the third workgroup of D 64 that fa_fwd_kernel keeps on a unit is worth more.  us, fa_fwd_kernel | this one:
-//   D 64   causal [1,12,1024] (96 tiles) 17.9 | 15.4, [3,12,1000] (288) 19.3 | 16.3, [8,8,1000] (512) 19.2 | 17.1, [1,8,4096] (256)
-//          57.3 | 46.6, not causal [1,32,2048] (512) 47.3 | 44.7; [9,8,1000] (576) 20.8 | 19.8, [10,8,1000] (640) 21.6 | 22.4,
-//          [16,12,512] (768) 17.1 | 19.2, [8,12,1024] (768) 23.9 | 25.0
-//   D 128  causal [1,8,512] (32) 15.8 | 14.8, [2,8,1000] (128) 25.7 | 23.7, [2,4,4096] (256) 84.1 | 77.6, [4,16,1000] (512) 34.9 | 34.2
-bool fa_flow_wanted(const FaArgs& a) {
-    const int64_t tiles = (int64_t)a.B * a.H * ((a.Sq + kBQ - 1) / kBQ);
-    return tiles <= 2 * (int64_t)compute_units();
+// 16-bit q, k, v, o of head size 64 or 128 with 16-byte aligned rows and no mask, while the workgroups that a compute unit keeps
+// hold all tiles: two, or one with head size 128 and no causal rule (see the kernel).  Beyond that the third workgroup of D 64 that
+// fa_fwd_kernel keeps on a unit is worth more, and so it is, for more than one workgroup a unit, where the longest tile has
+// few blocks of keys: what is fetched ahead is then most of what there is.  us, fa_fwd_kernel | this one:
+//   D 64   causal  [1,12,1024] (96 tiles) 18.1 | 15.5, [4,8,1000] (256) 18.4 | 16.1, [3,12,1000] (288) 18.8 | 16.5, [8,8,1000] (512) 19.7 | 17.8,
+//                  [1,8,4096] (256) 57.4 | 47.3, [9,8,1000] (576) 20.7 | 20.1, [10,8,1000] (640) 21.3 | 22.5; by blocks of keys [8,32,16] (256, 1 block)
+//                  4.5 | 4.6, [1,12,100] (12, 2) 6.0 | 5.8, [16,32,128] (512, 2) 10.0 | 10.3, [8,32,256] (512, 4) 10.7 | 10.9, [4,32,500] (512, 8) 13.3 | 12.6
+//          else    [1,12,1024] 17.4 | 14.8, [8,8,1000] 26.6 | 25.0, [9,8,1000] 32.9 | 34.1, 300 queries over 3000 keys (48) 42.2 | 34.3; [1,12,64] (12, 1)
+//                  4.3 | 4.1, [8,32,64] (256, 1) 4.7 | 4.5, [16,32,64] over 37 keys (512, 1) 5.2 | 5.4, [8,32,192] (512, 3) 10.0 | 9.7
+//   D 128  causal  [1,8,512] (32) 15.8 | 15.0, [2,8,1000] (128) 25.8 | 24.4, [2,4,4096] (256) 85.2 | 80.4, [6,8,1000] (384) 27.9 | 26.6, [8,8,1000] (512)
+//                  33.9 | 33.9; [8,32,128] (256, 2) 10.7 | 10.9, [2,32,192] (128, 3) 9.3 | 8.9, [12,32,128] (384, 2) 13.9 | 14.6
+//          else    [1,8,512] 15.7 | 15.2, [2,8,1000] 26.6 | 25.6, [2,4,4096] 88.2 | 84.3, 100 queries over 2000 keys (256) 65.6 | 56.9, [6,8,1000] (384)
+//                  37.8 | 49.4; [8,32,128] (256, 2) 10.9 | 11.2
+bool fa_flow_wanted(const FaArgs& a, int64_t D) {
+    const int64_t tiles = (int64_t)a.B * a.H * ((a.Sq + kBQ - 1) / kBQ), cus = compute_units();
+    const int blocks = ((a.is_causal && a.Sq < a.Skv ? a.Sq : a.Skv) + kBKV - 1) / kBKV;
+    if (tiles <= cus) return blocks >= (D == 128 ? 3 : a.is_causal ? 2 : 1);
+    return tiles <= 2 * cus && (a.is_causal ? blocks >= 5 : D == 64 && blocks >= 3);
 }
 
 int launch_fa_flow(hipStream_t s, FaArgs a, int64_t D, int dtype) {

@@ -6,7 +6,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 SIZES = [(1, 1, 1), (31, 31, 1), (32, 33, 1), (64, 64, 1), (65, 200, 1), (127, 127, 1), (128, 128, 0), (129, 129, 1), (200, 63, 1),
-         (40, 320, 0), (257, 257, 1), (130, 449, 0)]
+         (40, 320, 0), (257, 257, 1), (130, 449, 0), (190, 500, 1), (129, 192, 0), (321, 321, 1)]
 
 
 def _views(B, H, S, D, x):

@@ -1,0 +1,43 @@
+"""What the compiler made of the kernels that count the loads they have in flight: a register that does not fit goes to memory, and
+its reload waits for every load before it, tiles asked for ahead of their use among them.  Read from the metadata of the built library."""
+import os
+import struct
+
+import pytest
+
+msgpack = pytest.importorskip("msgpack")
+LIB = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "metalhlo_amd", "lib", "libmetalhlo_hip.so")
+
+
+def _code_objects(data):
+    at = data.find(b"__CLANG_OFFLOAD_BUNDLE__")
+    while at >= 0:
+        count, p = struct.unpack_from("<Q", data, at + 24)[0], at + 32
+        for _ in range(count):
+            off, size, n = struct.unpack_from("<QQQ", data, p)
+            if b"gfx950" in data[p + 24:p + 24 + n] and size:
+                yield data[at + off:at + off + size]
+            p += 24 + n
+        at = data.find(b"__CLANG_OFFLOAD_BUNDLE__", at + 24)
+
+
+def _kernels():
+    for elf in _code_objects(open(LIB, "rb").read()):
+        table, = struct.unpack_from("<Q", elf, 0x28)
+        size, count = struct.unpack_from("<HH", elf, 0x3A)
+        for i in range(count):
+            kind, = struct.unpack_from("<I", elf, table + i * size + 4)
+            if kind == 7:                                      # a note: sizes of name and content, type, name, content
+                at, = struct.unpack_from("<Q", elf, table + i * size + 24)
+                name, content, _ = struct.unpack_from("<III", elf, at)
+                yield from msgpack.unpackb(elf[at + 12 + (name + 3) // 4 * 4:][:content], strict_map_key=False)["amdhsa.kernels"]
+
+
+@pytest.mark.parametrize("name", ["fa_flow_kernel", "gemm_f32_ring_kernel", "gemm_mid_kernel", "gemm192_kernel", "linear_w32_kernel",
+                                  "linear_w32_stream_kernel", "tied_head_kernel"])
+def test_nothing_is_spilled(name):
+    if not os.path.exists(LIB):
+        pytest.skip("no built library")
+    found = [k for k in _kernels() if name in k[".name"]]
+    assert found
+    assert [k[".name"] for k in found if k[".private_segment_fixed_size"] or k[".vgpr_spill_count"]] == []
