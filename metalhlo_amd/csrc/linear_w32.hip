@@ -462,7 +462,8 @@ using namespace mhip;
 extern "C" int mhip_linear_w32_ok(int64_t M, int64_t N, int64_t K, int dtype) {
     if (dtype != MHIP_BF16 && dtype != MHIP_F16) return 0;
     if (M < 1 || M > 192 || N < 1 || K < 1 || N % 8 != 0 || K % 8 != 0 || N > (1 << 24) || K > (1 << 24)) return 0;
-    return (N + 64) * (K + 64) * 4 < 0x7FFFFFFFLL;
+    // (x and w each inside one descriptor, whose last byte lies below kOob)
+    return (N + 64) * (K + 64) * 4 < 0x7FFFFFFFLL && M * K * 2 < 0x7FFFFFFFLL;
 }
 
 // Parts of K: about 768 k, at most two workgroups per compute unit.
