@@ -306,8 +306,8 @@ GemmPack gemm_pack_plan(const GemmArgs& g, int trans_a, int trans_b, bool a_off,
 int launch_gemm_pack(hipStream_t s, const GemmArgs& g, const GemmPack& p, int trans_a, int trans_b, char* to);
 int launch_gemm_skinny(hipStream_t s, GemmArgs g, int64_t batch, int trans_b, int dtype, int64_t workspace_bytes);
 // gemm_mid.hip: 64- and 128-row tiles through a ring of LDS stages, K split where that leaves units idle.
-int64_t gemm_mid_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b);
-int launch_gemm_mid(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_a, int trans_b, int dtype, int64_t workspace_bytes);
+int64_t gemm_mid_workspace(int64_t M, int64_t N, int64_t K, int64_t sum_k, int64_t batch, int trans_a, int trans_b);
+int launch_gemm_mid(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_a, int trans_b, int dtype, int64_t workspace_bytes, int64_t sum_k);
 // gemm_f32.hip: fp32 operands on the fp32 matrix instruction, 128x128 tiles.
 bool gemm_f32_mfma_wanted(const GemmArgs& g);
 int launch_gemm_f32_mfma(hipStream_t s, GemmArgs g, int64_t batch, int trans_a, int trans_b, int64_t workspace_bytes);
@@ -397,7 +397,7 @@ static thread_local int g_last_variant = 0;
 static inline int chose(int variant, int status) { g_last_variant = variant; return status; }
 
 template <typename T, bool TA, bool TB>
-static int pick_tile(hipStream_t s, const GemmArgs& g, int64_t batch, int64_t workspace_bytes) {
+static int pick_tile(hipStream_t s, const GemmArgs& g, int64_t batch, int64_t workspace_bytes, int64_t sum_k) {
     const int64_t tiles_m = (g.M + 255) / 256;
     const int64_t big = tiles_m * ((g.N + 255) / 256) * batch;
     constexpr int dt = std::is_same<T, bf16_t>::value ? MHIP_BF16 : MHIP_F16;
@@ -438,7 +438,7 @@ static int pick_tile(hipStream_t s, const GemmArgs& g, int64_t batch, int64_t wo
     }
     // (up to 192 rows: much of a 256-row tile would be padding; with more than 128 it is ahead all the same where its columns fill
     // the device, [150,768] x [50304,768]^T 40.9 us in 128-row tiles, 27.4)
-    if (force == 128 || (force == 0 && g.M <= 192 && (g.M <= 128 || g.K < 512 || !gemm256_eligible(g, batch, TA, TB, dt)))) return chose(128, launch_gemm_mid(s, g, batch, TA, TB, dt, workspace_bytes));
+    if (force == 128 || (force == 0 && g.M <= 192 && (g.M <= 128 || g.K < 512 || !gemm256_eligible(g, batch, TA, TB, dt)))) return chose(128, launch_gemm_mid(s, g, batch, TA, TB, dt, workspace_bytes, sum_k));
     constexpr int cus = 256;                           // compute units of the device this is written for
     const int64_t narrow = tiles_m * ((g.N + 127) / 128) * batch, stages = g.K / 32;
     const int64_t wide_cost = ((big + cus - 1) / cus) * (stages * 32 + 700);
@@ -493,16 +493,16 @@ static int pick_tile(hipStream_t s, const GemmArgs& g, int64_t batch, int64_t wo
     }
     // (fewer than 192 tiles of any ring kernel, a ragged K, or so few rows that 256-row tiles are mostly padding)
     const bool large = big >= 192 && (g.K >= 1024 || g.N % 8 != 0);
-    if (!large && force != 256) return chose(128, launch_gemm_mid(s, g, batch, TA, TB, dt, workspace_bytes));
+    if (!large && force != 256) return chose(128, launch_gemm_mid(s, g, batch, TA, TB, dt, workspace_bytes, sum_k));
     return chose(256, launch_mfma<T, 256, 256, 2, 4, TA, TB>(s, g, batch));
 }
 
 template <typename T>
-static int pick_layout(hipStream_t s, const GemmArgs& g, int64_t batch, int ta, int tb, int64_t workspace_bytes) {
-    if (!ta && !tb) return pick_tile<T, false, false>(s, g, batch, workspace_bytes);
-    if (!ta && tb) return pick_tile<T, false, true>(s, g, batch, workspace_bytes);
-    if (ta && !tb) return pick_tile<T, true, false>(s, g, batch, workspace_bytes);
-    return pick_tile<T, true, true>(s, g, batch, workspace_bytes);
+static int pick_layout(hipStream_t s, const GemmArgs& g, int64_t batch, int ta, int tb, int64_t workspace_bytes, int64_t sum_k) {
+    if (!ta && !tb) return pick_tile<T, false, false>(s, g, batch, workspace_bytes, sum_k);
+    if (!ta && tb) return pick_tile<T, false, true>(s, g, batch, workspace_bytes, sum_k);
+    if (ta && !tb) return pick_tile<T, true, false>(s, g, batch, workspace_bytes, sum_k);
+    return pick_tile<T, true, true>(s, g, batch, workspace_bytes, sum_k);
 }
 
 template <typename T>
@@ -567,9 +567,9 @@ static GemmArgs packed_args(const GemmArgs& g, const GemmPack& p) {
     q.K = p.K; q.lda = p.lda; q.ldb = p.ldb;
     return q;
 }
-static int64_t aligned_workspace(int64_t M, int64_t N, int64_t K, int trans_a, int trans_b) {
+static int64_t aligned_workspace(int64_t M, int64_t N, int64_t K, int64_t sum_k, int trans_a, int trans_b) {
     if (M > 192 && (double)M * N >= 192.0 * 256 * 256) return 0;         // (a large problem goes to the ring kernels, whose tiles fill the device)
-    return gemm_mid_workspace(M, N, K, 1, trans_a, trans_b);
+    return gemm_mid_workspace(M, N, K, sum_k, 1, trans_a, trans_b);
 }
 // Where copies pay: gemm_any.hip's tiles wait out a load latency per stage, 11.7 ns a k, and touch two lines per load.  us, as they
 // are | copied (the copies included), over the four layouts: [1001,1001] x K 4001 47 to 50 | 30 to 32, [301,2001] x K 3001 36 to 38 |
@@ -623,8 +623,8 @@ static int gemm_entry(void* stream, const void* a, const void* b, const void* bi
               : !(g.partial && f32_rows_in_parts(M, N, K, batch, trans_a, trans_b) > 0 && workspace_bytes >= f32_rows_in_parts(M, N, K, batch, trans_a, trans_b))))
         return chose(vec_ok ? 128 : 0, launch_gemm_skinny(s, g, batch, trans_b, dtype, workspace_bytes));
     if (vec_ok) {
-        if (dtype == MHIP_BF16) return pick_layout<bf16_t>(s, g, batch, trans_a, trans_b, workspace_bytes);
-        return pick_layout<f16_t>(s, g, batch, trans_a, trans_b, workspace_bytes);
+        if (dtype == MHIP_BF16) return pick_layout<bf16_t>(s, g, batch, trans_a, trans_b, workspace_bytes, K);
+        return pick_layout<f16_t>(s, g, batch, trans_a, trans_b, workspace_bytes, K);
     }
     switch (dtype) {
         case MHIP_F32:
@@ -645,7 +645,7 @@ static int gemm_entry(void* stream, const void* a, const void* b, const void* bi
                     if (p.a) q.a = to;
                     if (p.b) q.b = to + p.a_bytes;
                     q.partial = left > 0 ? reinterpret_cast<float*>(to + p.a_bytes + p.b_bytes) : nullptr;
-                    return dtype == MHIP_BF16 ? pick_layout<bf16_t>(s, q, 1, trans_a, trans_b, left) : pick_layout<f16_t>(s, q, 1, trans_a, trans_b, left);
+                    return dtype == MHIP_BF16 ? pick_layout<bf16_t>(s, q, 1, trans_a, trans_b, left, K) : pick_layout<f16_t>(s, q, 1, trans_a, trans_b, left, K);
                 }
             }
             if (!short_product(M, N, K)) return launch_gemm_any(s, g, batch, trans_a, trans_b, dtype, workspace_bytes);
@@ -699,8 +699,8 @@ extern "C" int64_t mhip_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t 
         GemmArgs g = {};
         g.M = (int)M; g.N = (int)N; g.K = (int)K; g.lda = (int)(trans_a ? M : K); g.ldb = (int)(trans_b ? K : N);
         const GemmPack p = gemm_pack_plan(g, trans_a, trans_b, g.lda % 8 != 0, g.ldb % 8 != 0);
-        return p.a_bytes + p.b_bytes + aligned_workspace(M, N, p.K, trans_a, trans_b);
+        return p.a_bytes + p.b_bytes + aligned_workspace(M, N, p.K, K, trans_a, trans_b);
     }
     if (!vec) return short_product(M, N, K) ? 0 : gemm_any_workspace(M, N, K, batch);
-    return aligned_workspace(M, N, K, trans_a, trans_b);
+    return aligned_workspace(M, N, K, K, trans_a, trans_b);
 }

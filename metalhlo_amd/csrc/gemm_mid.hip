@@ -367,10 +367,11 @@ float form_cost(const Form& f, int64_t M, int64_t N, int64_t K, int64_t batch, i
 // are worth a factor; in between every sum keeps the order of the large tiles, and a sequence its bits in any batch
 // (gemm_skinny.hip, gemm_any.hip and gemm_f32.hip have the same limits).  K goes to a workspace in parts only for a
 // clear gain.
-MidPlan plan_mid(int64_t M, int64_t N, int64_t K, int64_t batch, bool ring_ok, bool may_split) {
+// `sum_k`: K without the zeros behind it that copied operands have (gemm_any.hip).
+MidPlan plan_mid(int64_t M, int64_t N, int64_t K, int64_t sum_k, int64_t batch, bool ring_ok, bool may_split) {
     MidPlan best;
     float t_best = 1e30f;
-    const bool in_order = M > 192 && K < 4096;
+    const bool in_order = M > 192 && sum_k < 4096;
     for (int f = 0; f <= (ring_ok ? kRing192 : kRing192 - 1); f++) {
         if (in_order && !kForms[f].in_order) continue;
         for (int s = 1; s <= (may_split && batch == 1 && !in_order ? kMaxSplits : 1); s++) {
@@ -450,16 +451,16 @@ int launch_plan(hipStream_t s, GemmArgs g, int64_t batch, int ta, int tb, int dt
 }  // namespace
 
 // Bytes of workspace the choice for this problem can use (0 = none); a function of the sizes alone.
-int64_t gemm_mid_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b) {
-    return plan_bytes(plan_mid(M, N, K, batch, K >= 32 && (K % 32 == 0 || (trans_a && !trans_b)), true), M, N);
+int64_t gemm_mid_workspace(int64_t M, int64_t N, int64_t K, int64_t sum_k, int64_t batch, int trans_a, int trans_b) {
+    return plan_bytes(plan_mid(M, N, K, sum_k, batch, K >= 32 && (K % 32 == 0 || (trans_a && !trans_b)), true), M, N);
 }
 
 // 16-bit operands with 16-byte-aligned rows (the caller has checked).  `workspace` (g.partial) may be absent or
 // smaller than asked for: then K is not split.
-int launch_gemm_mid(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_a, int trans_b, int dtype, int64_t workspace_bytes) {
+int launch_gemm_mid(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_a, int trans_b, int dtype, int64_t workspace_bytes, int64_t sum_k) {
     const bool ring = gemm256_eligible(g, batch, trans_a, trans_b, dtype, 192, true);
-    MidPlan p = plan_mid(g.M, g.N, g.K, batch, ring, g.partial != nullptr);
-    if (plan_bytes(p, g.M, g.N) > workspace_bytes) p = plan_mid(g.M, g.N, g.K, batch, ring, false);
+    MidPlan p = plan_mid(g.M, g.N, g.K, sum_k, batch, ring, g.partial != nullptr);
+    if (plan_bytes(p, g.M, g.N) > workspace_bytes) p = plan_mid(g.M, g.N, g.K, sum_k, batch, ring, false);
     return dtype == MHIP_BF16 ? launch_plan<bf16_t>(s, g, batch, trans_a, trans_b, dtype, p) : launch_plan<f16_t>(s, g, batch, trans_a, trans_b, dtype, p);
 }
 

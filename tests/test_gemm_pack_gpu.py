@@ -81,3 +81,24 @@ def test_the_last_row_of_k_ends_in_an_odd_column(monkeypatch, dtype, tile, ta):
                             work.data_ptr(), need) == 0
     assert lib.mhip_gemm_last_variant() == tile
     assert torch.equal(out, (u.float()[:, None] * v.float()[None, :]).to(dtype))
+
+
+@pytest.mark.parametrize("K", [4065, 4090, 4095])
+@pytest.mark.parametrize("N,M", [(300, (200, 1001, 2001)), (1001, (264, 1001))])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_padding_k_to_4096_leaves_the_order_of_a_sum(ta, tb, N, M, K):
+    """From 193 rows on a row has the same bits for any number of rows while the caller's K is below 4096, also where the copies
+    have 4096 columns."""
+    lib, code = _lib.load(), kernels.DTYPE_CODE[torch.bfloat16]
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a, b = torch.randn(max(M), K, generator=g, device="cuda").bfloat16(), torch.randn(K, N, generator=g, device="cuda").bfloat16()
+    rhs, rows = b.T.contiguous() if tb else b, {}
+    for m in M:
+        lhs, need = a[:m].T.contiguous() if ta else a[:m], lib.mhip_gemm_workspace(m, N, K, 1, ta, tb, code)
+        assert need >= 2 * (m + N) * K                            # both are copied
+        for bytes_ in (need, 0):
+            out, work = torch.empty(m, N, dtype=torch.bfloat16, device="cuda"), torch.empty(need, dtype=torch.uint8, device="cuda")
+            assert lib.mhip_gemm_ws(torch.cuda.current_stream().cuda_stream, lhs.data_ptr(), rhs.data_ptr(), None, None, out.data_ptr(), m, N, K, 1, 0, 0, 0, ta, tb, 0,
+                                    code, work.data_ptr() if bytes_ else None, bytes_) == 0
+            rows[m, bytes_ > 0] = out[:min(M)]
+    assert all(torch.equal(v, rows[M[0], False]) for v in rows.values())
