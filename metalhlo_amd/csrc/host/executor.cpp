@@ -851,9 +851,13 @@ static std::vector<DeviceTensor> run_ops(Executable& exe, const std::vector<Devi
             // one product, with the memory that lets its K be split over idle compute units
             auto gemm = [&](const void* a, const void* b, const void* bias, const void* residual, void* c, int64_t M, int64_t N, int64_t K, bool ta,
                             bool tb, int act) {
-                const int64_t bytes = mhip_gemm_workspace(M, N, K, 1, ta, tb, dt);
+                int64_t bytes = exe.no_workspace ? 0 : mhip_gemm_workspace(M, N, K, 1, ta, tb, dt);
                 DeviceTensor work;
-                if (bytes > 0) work = al.allocate(TensorType{{bytes}, UI8});
+                try {
+                    if (bytes > 0) work = al.allocate(TensorType{{bytes}, UI8});
+                } catch (const BufferError&) {          // (a block of its own, METALHLO_ARENA=0: the product has a form without)
+                    bytes = 0;
+                }
                 RUN(mhip_gemm_ws(s, a, b, bias, residual, c, M, N, K, 1, 0, 0, 0, ta, tb, act, dt, work.data(), bytes));
             };
             if (kUnary.count(n)) {
@@ -1115,38 +1119,39 @@ static bool env_flag(const char* name, bool dflt) {
 }
 
 static void plan_memory(Executable& exe) {
-    exe.plan = ArenaPlan();
+    ArenaPlan plan;
     try {
         Allocator al;
         al.mode = Allocator::RECORD;
-        al.plan = &exe.plan;
+        al.plan = &plan;
         std::vector<DeviceTensor> ins;
         for (auto& t : exe.fn.arg_types) { DeviceTensor d; d.type = t; ins.push_back(d); }
         {
             const std::vector<DeviceTensor> rets = run_ops(exe, ins, al, true);
-            for (auto& r : rets) if (r.mem && r.mem->recorder) exe.plan.slots[r.mem->slot].escapes = true;
+            for (auto& r : rets) if (r.mem && r.mem->recorder) plan.slots[r.mem->slot].escapes = true;
         }
-        for (auto& sl : exe.plan.slots) {
+        for (auto& sl : plan.slots) {
             if (sl.escapes) sl.end = 0x7FFFFFFF;
-            else exe.plan.sum_bytes += sl.bytes;
+            else plan.sum_bytes += sl.bytes;
         }
         // Both placements are made; the one by recency is kept unless it needs over a quarter more
         // bytes than the packed one (METALHLO_ARENA_PLACEMENT=packed keeps the packed one regardless).
         // GPT-2-small forward, B8 S1024: 361 MB against 319 MB, and 0.02-0.03 ms of 3.5 ms faster.
         const char* how = getenv("METALHLO_ARENA_PLACEMENT");
-        const size_t packed = place_slots(exe.plan, false, 0);
-        exe.plan.core_bytes = packed;
+        const size_t packed = place_slots(plan, false, 0);
+        plan.core_bytes = packed;
         if (!how || strcmp(how, "packed")) {
-            const std::vector<ArenaPlan::Slot> keep = exe.plan.slots;
-            const size_t recent = place_slots_recent(exe.plan, false, 0);
-            if (recent <= packed + packed / 4) exe.plan.core_bytes = recent;
-            else exe.plan.slots = keep;
+            const std::vector<ArenaPlan::Slot> keep = plan.slots;
+            const size_t recent = place_slots_recent(plan, false, 0);
+            if (recent <= packed + packed / 4) plan.core_bytes = recent;
+            else plan.slots = keep;
         }
-        exe.plan.full_bytes = place_slots(exe.plan, true, exe.plan.core_bytes);
-        exe.plan.valid = true;
+        plan.full_bytes = place_slots(plan, true, plan.core_bytes);
+        plan.valid = true;
     } catch (const std::exception&) {
-        exe.plan = ArenaPlan();     // the execution reports the problem; it allocates per value
+        plan = ArenaPlan();     // the execution reports the problem; it allocates per value
     }
+    exe.plan = std::move(plan);
 }
 
 static void ensure_arena(Executable& exe, size_t bytes) {
@@ -1290,7 +1295,19 @@ std::vector<DeviceTensor> execute(Executable& exe, const std::vector<DeviceTenso
     // client (or a PJRT transfer) can then never launch into, or wait for, a stream that is being
     // captured, where its work would be recorded into the graph instead of run.
     std::unique_lock<std::mutex> stream_lock(c.stream_mu);
-    if (use_arena) ensure_arena(exe, want_graph && !direct_results(exe) ? exe.plan.full_bytes : exe.plan.core_bytes);
+    if (use_arena) {
+        auto bytes = [&] { return want_graph && !direct_results(exe) ? exe.plan.full_bytes : exe.plan.core_bytes; };
+        try {
+            ensure_arena(exe, bytes());
+        } catch (const BufferError&) {
+            // workspaces only make products faster: a plan without them, once, before the execution fails for want of memory
+            if (exe.no_workspace) throw;
+            exe.no_workspace = true;
+            plan_memory(exe);
+            if (!exe.plan.valid) throw;
+            ensure_arena(exe, bytes());
+        }
+    }
     // the first execution runs eagerly (kernels set their attributes, tuning tables load); from the
     // second on the op list is one graph per set of input addresses
     if (want_graph && !exe.graph_failed && exe.eager_runs > 0) {

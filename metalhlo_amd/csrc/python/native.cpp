@@ -76,6 +76,16 @@ void* stream_of(const at::Tensor&) { return c10::hip::getCurrentHIPStream().stre
 at::Tensor empty(at::IntArrayRef shape, at::ScalarType dtype, const at::Tensor& like) {
     return at::detail::empty_cuda(shape, dtype, like.device(), std::nullopt);
 }
+// Memory that only makes a call faster, from the current stream's pool or a capturing graph's own: none where the device has no more, the
+// call then takes its form without it.
+at::Tensor workspace(int64_t bytes, const at::Tensor& like) {
+    if (bytes <= 0) return {};
+    try {
+        return empty({bytes}, at::kByte, like);
+    } catch (const c10::OutOfMemoryError&) {
+        return {};
+    }
+}
 at::Tensor result_like(const at::Tensor& t) { return empty(t.sizes(), t.scalar_type(), t); }
 
 bool truth(PyObject* o) {
@@ -229,12 +239,9 @@ FUNCTION(matmul) {
         if (res && (res->numel() != c.numel() || res->scalar_type() != c.scalar_type()))
             raise(PyExc_ValueError, "residual must have the result's size and dtype");
         const int dt = dtype_code(a.scalar_type()), act = (int)integer(arg[3]);
-        // (partial sums of a split K: memory of the current stream's, or a capturing graph's own)
-        const int64_t bytes = mhip_gemm_workspace(M, N, K, batch, ta, tb, dt);
-        at::Tensor work;
-        if (bytes) work = empty({bytes}, at::kByte, a);
+        const at::Tensor work = workspace(mhip_gemm_workspace(M, N, K, batch, ta, tb, dt), a);
         check([&] { return mhip_gemm_ws(stream_of(a), a.data_ptr(), b.data_ptr(), ptr(bias), ptr(res), c.data_ptr(), M, N, K, batch, sa, sb, M * N, ta, tb,
-                           act, dt, bytes ? work.data_ptr() : nullptr, bytes); });
+                           act, dt, work.defined() ? work.data_ptr() : nullptr, work.defined() ? work.numel() : 0); });
         return THPVariable_Wrap(std::move(c));
     });
 }
@@ -378,11 +385,10 @@ FUNCTION(flash_attention) {
         views[3] = &o;
         for (int t = 0; !packed && t < 4; t++)
             for (int d = 0; d < 3; d++) strides[3 * t + d] = views[t]->stride(d);
-        const int64_t bytes = mhip_flash_attention_workspace(B, H, Sq, Skv, D, causal, dt);
-        at::Tensor work;
-        if (bytes) work = empty({bytes}, at::kByte, q);
+        const at::Tensor work = workspace(mhip_flash_attention_workspace(B, H, Sq, Skv, D, causal, dt), q);
         check([&] { return mhip_flash_attention_ws(stream_of(q), q.data_ptr(), k.data_ptr(), v.data_ptr(), ptr(mask), o.data_ptr(), B, H, Sq, Skv, D,
-                                                   (float)scale, causal, msb, msh, dt, packed ? nullptr : strides, bytes ? work.data_ptr() : nullptr, bytes); });
+                                                   (float)scale, causal, msb, msh, dt, packed ? nullptr : strides, work.defined() ? work.data_ptr() : nullptr,
+                                                   work.defined() ? work.numel() : 0); });
         return THPVariable_Wrap(std::move(o));
     });
 }
