@@ -92,7 +92,8 @@ class GPT2:
 
     def forward(self, ids: torch.Tensor) -> torch.Tensor:
         """ids int32 [B,S] on the device -> logits [B,S,vocab] in the compute type.  With more than 768 tokens in all a
-        sequence has the same bits in any batch; below that fp32 sums are split by the number of tokens."""
+        sequence has the same bits in any batch (d_model and d_ff below 4096, where products keep the order of a sum); up to that
+        fp32 sums are split by the number of tokens."""
         cfg = self.cfg
         B, S = ids.shape
         d, H = cfg.d_model, cfg.n_head
@@ -156,11 +157,13 @@ class GPT2:
     # (us whole and in parts, replayed: 193 tokens 810 and 642, 300 841 and 692, 576 949 and 844, 768 (144 tiles) 1098 and 1008;
     # 1024 (192 tiles) 1206 and 1202, which leaves a sequence of full length its bits in any batch)
     _full_tiles = 144
+    # (narrower layers have so few tiles for more tokens, but a sequence keeps its bits from here on whatever the width)
+    _most_tokens = 768
 
     def _sum_parts(self, tokens: int):
         """Shares of K for the two layers in front of a residual, (0, 0) where their tiles fill the device without."""
         d, f = self.cfg.d_model, self.cfg.d_ff
-        if d // self.cfg.n_head not in (64, 128) or d % self.cfg.n_head or d > 4096 or -(-tokens // 64) * -(-d // 64) > self._full_tiles:
+        if d // self.cfg.n_head not in (64, 128) or d % self.cfg.n_head or d > 4096 or tokens > self._most_tokens or -(-tokens // 64) * -(-d // 64) > self._full_tiles:
             return 0, 0
         if self.dtype not in (torch.bfloat16, torch.float16):
             return 0, 0

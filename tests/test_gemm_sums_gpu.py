@@ -53,6 +53,17 @@ def test_gpt2_forms_agree(dtype, B, S, few, parts):
         assert torch.equal(got, whole)
 
 
+@pytest.mark.parametrize("d_model,d_ff", [(256, 1024), (512, 2048), (768, 3072), (1024, 2048)])
+def test_a_sequence_has_the_same_bits_in_any_batch_of_more_than_768_tokens(d_model, d_ff):
+    from metalhlo_amd.gpt2 import GPT2, GPT2Config, init_params
+    cfg = GPT2Config(n_layer=2, d_model=d_model, n_head=d_model // 64, d_ff=d_ff, vocab=1000)
+    model = GPT2(cfg, init_params(cfg, seed=5))
+    ids = torch.randint(0, cfg.vocab, (8, 257), generator=torch.Generator().manual_seed(2), dtype=torch.int32).cuda()
+    whole = model.forward(ids)
+    for batch in (3, 5):                                         # 771 and 1285 tokens
+        assert torch.equal(model.forward(ids[:batch]), whole[:batch])
+
+
 def test_gpt2_in_parts_from_a_graph():
     """Replays with eager work between them give the eager bits."""
     from metalhlo_amd.gpt2 import GPT2, GPT2Config, init_params
