@@ -381,14 +381,15 @@ __global__ __launch_bounds__(256) void finish_norm_kernel(LinearArgs g, T* h) {
         __syncthreads();
         return (red[set][0] + red[set][1]) + (red[set][2] + red[set][3]);
     };
-    const float inv = 1.f / (float)g.N, mean = over_row(s, 0) * inv;
+    // (quotients: a row of equal elements has that mean and no variance)
+    const float mean = over_row(s, 0) / (float)g.N;
     float q = 0.f;
 #pragma unroll
     for (int p = 0; p < kFinishPieces; p++)
         if ((p * 256 + (int)threadIdx.x) * 4 < g.N)
 #pragma unroll
             for (int e = 0; e < 4; e++) { v[p][e] -= mean; q = fmaf(v[p][e], v[p][e], q); }
-    const float rstd = 1.f / sqrtf(over_row(q, 1) * inv + g.eps);
+    const float rstd = 1.f / sqrtf(over_row(q, 1) / (float)g.N + g.eps);
 #pragma unroll
     for (int p = 0; p < kFinishPieces; p++) {
         const int n = (p * 256 + (int)threadIdx.x) * 4;

@@ -65,6 +65,18 @@ def test_parts_and_finish_norm(dtype, M, N, K, parts):
     _close(h, n * g.to(dtype).double() + be.to(dtype).double(), 1.0, 1)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N", [24, 40, 200, 768, 1000, 3080, 4096])
+def test_rows_of_equal_elements_have_no_variance(dtype, N):
+    """The sum of N equal elements of up to 11 bits is exact, so is its quotient by N: nothing is left in front of beta."""
+    from metalhlo_amd import kernels
+    v = torch.cat([torch.arange(1, 200, device="cuda") / 16, torch.linspace(300, 2000, 57, device="cuda")]).to(dtype)
+    x, g, b = v[:, None].repeat(1, N), _draw(1, N, shift=1.0), _draw(2, N)
+    for beta in (b, torch.zeros(N, device="cuda")):
+        _, h = kernels.finish_norm(None, None, x, (g, beta, 1e-12))
+        assert torch.equal(h, beta.to(dtype).expand_as(h))
+
+
 def test_refusals():
     from metalhlo_amd import _lib, kernels
     bf = torch.bfloat16
