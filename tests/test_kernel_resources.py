@@ -41,3 +41,14 @@ def test_nothing_is_spilled(name):
     found = [k for k in _kernels() if name in k[".name"]]
     assert found
     assert [k[".name"] for k in found if k[".private_segment_fixed_size"] or k[".vgpr_spill_count"]] == []
+
+
+def test_whole_stages_do_not_pay_for_the_rest_of_k():
+    """x^T dy on the 128x192 tile over a multiple of 32 tokens has no more registers than the product of operands as they are stored."""
+    if not os.path.exists(LIB):
+        pytest.skip("no built library")
+    count = {k[".name"]: k[".vgpr_count"] for k in _kernels() if "gemm192_kernel" in k[".name"]}
+    for split in "01":
+        # (type, A and B transposed, K in parts, a rest of K)
+        tn, nn = ([n for n in count if "Lb%cELb0ELb%cELb0E" % (ta, split) in n] for ta in "10")
+        assert len(tn) == len(nn) == 2 and max(count[n] for n in tn) <= max(count[n] for n in nn)
