@@ -106,6 +106,7 @@ struct Executable {
     int64_t exec_count = 0;
     double total_ms = 0, last_ms = 0;
     std::mutex mu;
+    bool whole_sums = false;               // 16-bit products keep K in one piece (plan_memory says when)
     bool no_workspace = false;             // the device had no room for an arena with the products' workspaces: planned without them
     // arena and captured graphs (one execution at a time per executable while they are in use)
     ArenaPlan plan;
