@@ -34,6 +34,26 @@ __device__ __forceinline__ uint32_t lds_address(const char* p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p;
 }
 
+// c + 16 x 32 . 32 x 16 on operands of a 16-bit type, eight k a lane; b's side comes out in the four registers.
+template <typename T> struct Tile16;
+template <> struct Tile16<bf16_t> {
+    __device__ static f32x4 run(u32x4 b, u32x4 a, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b), __builtin_bit_cast(bf16x8, a), c, 0, 0, 0);
+    }
+};
+template <> struct Tile16<f16_t> {
+    __device__ static f32x4 run(u32x4 b, u32x4 a, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, b), __builtin_bit_cast(f16x8, a), c, 0, 0, 0);
+    }
+};
+// Two fp32 values rounded to T, the first one in the low half.
+template <typename T>
+__device__ __forceinline__ uint32_t round_pair(float lo, float hi) {
+    typedef T pair __attribute__((ext_vector_type(2)));
+    const pair p = {Elem<T>::from_f32(lo), Elem<T>::from_f32(hi)};
+    return __builtin_bit_cast(uint32_t, p);
+}
+
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 

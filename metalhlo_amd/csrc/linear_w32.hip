@@ -15,9 +15,8 @@
 //     will want them (fetch_ahead): [37,768] x [768,2304] 7.3 -> 5.0 us, those workgroups included.
 // Workgroups of one XCD take neighbouring strips, so a 128-byte line of W that two strips share is fetched once.
 #include <initializer_list>
-#include <mutex>
 
-#include "gemm_common.h"
+#include "gemm_lds.h"
 
 namespace mhip {
 namespace {
@@ -40,26 +39,6 @@ struct LinearArgs {
     Band ahead[kAhead];
 };
 
-template <typename T> struct Tile16;
-template <> struct Tile16<bf16_t> {
-    __device__ static f32x4 run(u32x4 b, u32x4 a, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b), __builtin_bit_cast(bf16x8, a), c, 0, 0, 0);
-    }
-};
-template <> struct Tile16<f16_t> {
-    __device__ static f32x4 run(u32x4 b, u32x4 a, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, b), __builtin_bit_cast(f16x8, a), c, 0, 0, 0);
-    }
-};
-template <typename T>
-__device__ __forceinline__ uint32_t round_pair(float lo, float hi) {
-    typedef T pair __attribute__((ext_vector_type(2)));
-    const pair p = {Elem<T>::from_f32(lo), Elem<T>::from_f32(hi)};
-    return __builtin_bit_cast(uint32_t, p);
-}
-__device__ inline __amdgpu_buffer_rsrc_t lin_rsrc(const void* p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
-}
 template <typename T>
 __device__ __forceinline__ float rounded(float v) { return Elem<T>::to_f32(Elem<T>::from_f32(v)); }
 // Workgroup `id` of those in front: kAheadLoads 16-byte pieces per thread of the columns that the strips of its XCD cover.
@@ -70,7 +49,7 @@ __device__ __forceinline__ void fetch_ahead(const LinearArgs& g, int id) {
     const float* w = r ? g.ahead[1].w : g.ahead[0].w;
     const int N = r ? g.ahead[1].N : g.ahead[0].N, K = r ? g.ahead[1].K : g.ahead[0].K, cols = r ? g.ahead[1].cols : g.ahead[0].cols;
     const uint32_t magic = r ? g.ahead[1].magic : g.ahead[0].magic, per_row = (uint32_t)cols / 4;
-    const __amdgpu_buffer_rsrc_t rw = lin_rsrc(w, (uint32_t)((int64_t)N * K * 4));
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(w, (uint32_t)((int64_t)N * K * 4));
     const uint32_t at = (uint32_t)j * (64 * kWaves * kAheadLoads) + threadIdx.x;
     u32x4 v[kAheadLoads];
 #pragma unroll
@@ -82,11 +61,11 @@ __device__ __forceinline__ void fetch_ahead(const LinearArgs& g, int id) {
     for (int i = 0; i < kAheadLoads; i++) asm volatile("" ::"v"(v[i]));
 }
 
-// TB: W stored [N, K].  NF = operands (groups of 16 columns) per strip, MT = groups of 16 rows, U = steps of 32 k that a
-// wave holds at once; LOOP: it has more of them and loads a block ahead.
-template <typename T, bool TB, bool LOOP, int NF, int MT, int U>
+// A strip of 16 columns.  TB: W stored [N, K].  MT = groups of 16 rows, U = steps of 32 k that a wave holds at once; LOOP: it has
+// more of them and loads a block ahead.
+template <typename T, bool TB, bool LOOP, int MT, int U>
 __global__ __launch_bounds__(64 * kWaves, LOOP ? 2 : 4) void linear_w32_kernel(LinearArgs g) {
-    constexpr int KS = 32, NS = 16 * NF;
+    constexpr int KS = 32;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     if ((int)blockIdx.x < g.first) {
         fetch_ahead(g, blockIdx.x);
@@ -98,17 +77,17 @@ __global__ __launch_bounds__(64 * kWaves, LOOP ? 2 : 4) void linear_w32_kernel(L
     int local = id / kXcds;
     const int m0 = local % g.blocks * (16 * MT);
     local /= g.blocks;
-    const int split = local % g.splits, strip = xcd * g.per_xcd + local / g.splits, n0 = strip * NS;
+    const int split = local % g.splits, strip = xcd * g.per_xcd + local / g.splits, n0 = strip * 16;
     if (strip >= g.strips) return;
-    const __amdgpu_buffer_rsrc_t rx = lin_rsrc(g.x, (uint32_t)((int64_t)g.M * g.K * 2));
-    const __amdgpu_buffer_rsrc_t rw = lin_rsrc(g.w, (uint32_t)((int64_t)g.N * g.K * 4));
+    const __amdgpu_buffer_rsrc_t rx = make_rsrc(g.x, (uint32_t)((int64_t)g.M * g.K * 2));
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(g.w, (uint32_t)((int64_t)g.N * g.K * 4));
 
     // ---- this wave's share of the k steps
     const int all = (g.K + KS - 1) / KS, part_steps = (all + g.splits - 1) / g.splits, p0 = split * part_steps, p1 = min(all, p0 + part_steps);
     const int per = (part_steps + kWaves - 1) / kWaves, s0 = p0 + wave * per, s1 = min(p1, s0 + per);
     struct Block {
-        f32x4 wt[TB ? U : 1][TB ? NF : 1][2];                // W stored [N, K]: eight k of a column
-        float wn[TB ? 1 : U][TB ? 1 : 8][NF];                // W stored [K, N]: NF columns of eight k
+        f32x4 wt[TB ? U : 1][2];                             // W stored [N, K]: eight k of a column
+        float wn[TB ? 1 : U][TB ? 1 : 8];                    // W stored [K, N]: the same, one by one
         u32x4 a[U][MT];
     };
     auto load = [&](Block& b, int s) __attribute__((always_inline)) {
@@ -116,27 +95,16 @@ __global__ __launch_bounds__(64 * kWaves, LOOP ? 2 : 4) void linear_w32_kernel(L
         for (int u = 0; u < U; u++) {
             const int k = (s + u) * KS + lg * 8;
             const bool live = s + u < s1 && k < g.K;
+            const int n = n0 + li;
             if (TB) {
+                const uint32_t off = live && n < g.N ? (uint32_t)(((int64_t)n * g.K + k) * 4) : kOob;
 #pragma unroll
-                for (int f = 0; f < NF; f++) {
-                    const int n = n0 + 16 * f + li;
-                    const uint32_t off = live && n < g.N ? (uint32_t)(((int64_t)n * g.K + k) * 4) : kOob;
-#pragma unroll
-                    for (int h = 0; h < 2; h++) b.wt[TB ? u : 0][TB ? f : 0][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, off + 16 * h, 0, 0));
-                }
+                for (int h = 0; h < 2; h++) b.wt[TB ? u : 0][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, off + 16 * h, 0, 0));
             } else {
-                const int n = n0 + NF * li;
                 const uint32_t off = live && n < g.N ? (uint32_t)(((int64_t)k * g.N + n) * 4) : kOob;
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const uint32_t o = off + (uint32_t)(j * g.N * 4);
-                    if (NF == 1) b.wn[TB ? 0 : u][TB ? 0 : j][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rw, o, 0, 0));
-                    else {
-                        const u32x2 t = __builtin_amdgcn_raw_buffer_load_b64(rw, o, 0, 0);
-                        b.wn[TB ? 0 : u][TB ? 0 : j][0] = __builtin_bit_cast(float, t.x);
-                        b.wn[TB ? 0 : u][TB ? 0 : j][NF - 1] = __builtin_bit_cast(float, t.y);
-                    }
-                }
+                for (int j = 0; j < 8; j++)
+                    b.wn[TB ? 0 : u][TB ? 0 : j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rw, off + (uint32_t)(j * g.N * 4), 0, 0));
             }
         }
 #pragma unroll
@@ -150,42 +118,30 @@ __global__ __launch_bounds__(64 * kWaves, LOOP ? 2 : 4) void linear_w32_kernel(L
     Block cur;
     load(cur, s0);
 
-    // ---- the epilogue's thread (wave = mt, li, lg) finishes row li of group mt: columns NF 4 lg .. + 4 NF - 1 of the strip (W
-    // stored [K, N]) or four from 4 lg on of each operand (stored [N, K])
-    const int fm = m0 + wave * 16 + li;
+    // ---- the epilogue's thread (wave = mt, li, lg) finishes row li of group mt: columns 4 lg .. 4 lg + 3 of the strip
+    const int fm = m0 + wave * 16 + li, column = n0 + 4 * lg;
     const bool finisher = wave < MT && fm < g.M;
-    auto column = [&](int q) { return TB ? n0 + 16 * q + 4 * lg : n0 + NF * 4 * lg + 4 * q; };
-    f32x4 bias[NF];
-    u32x2 res[NF];
-#pragma unroll
-    for (int q = 0; q < NF; q++) {
-        bias[q] = f32x4{0.f, 0.f, 0.f, 0.f};
-        res[q] = u32x2{0, 0};
-        if (finisher && column(q) < g.N) {
-            if (g.bias) bias[q] = *reinterpret_cast<const f32x4*>(g.bias + column(q));
-            if (g.residual) res[q] = *reinterpret_cast<const u32x2*>(static_cast<const T*>(g.residual) + (int64_t)fm * g.N + column(q));
-        }
+    f32x4 bias = {0.f, 0.f, 0.f, 0.f};
+    u32x2 res = {0, 0};
+    if (finisher && column < g.N) {
+        if (g.bias) bias = *reinterpret_cast<const f32x4*>(g.bias + column);
+        if (g.residual) res = *reinterpret_cast<const u32x2*>(static_cast<const T*>(g.residual) + (int64_t)fm * g.N + column);
     }
 
-    f32x4 acc[NF][MT];
+    f32x4 acc[MT];
 #pragma unroll
-    for (int f = 0; f < NF; f++)
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) acc[f][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int mt = 0; mt < MT; mt++) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto multiply = [&](const Block& b, int s) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
             if (s + u >= s1) break;
+            u32x4 w;
 #pragma unroll
-            for (int f = 0; f < NF; f++) {
-                u32x4 w;
+            for (int j = 0; j < 4; j++)
+                w[j] = TB ? round_pair<T>(b.wt[TB ? u : 0][j / 2][j % 2 * 2], b.wt[TB ? u : 0][j / 2][j % 2 * 2 + 1])
+                          : round_pair<T>(b.wn[TB ? 0 : u][TB ? 0 : 2 * j], b.wn[TB ? 0 : u][TB ? 0 : 2 * j + 1]);
 #pragma unroll
-                for (int j = 0; j < 4; j++)
-                    w[j] = TB ? round_pair<T>(b.wt[TB ? u : 0][TB ? f : 0][j / 2][j % 2 * 2], b.wt[TB ? u : 0][TB ? f : 0][j / 2][j % 2 * 2 + 1])
-                              : round_pair<T>(b.wn[TB ? 0 : u][TB ? 0 : 2 * j][f], b.wn[TB ? 0 : u][TB ? 0 : 2 * j + 1][f]);
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++) acc[f][mt] = Tile16<T>::run(w, b.a[u][mt], acc[f][mt]);
-            }
+            for (int mt = 0; mt < MT; mt++) acc[mt] = Tile16<T>::run(w, b.a[u][mt], acc[mt]);
         }
     };
     if (LOOP) {
@@ -198,45 +154,31 @@ __global__ __launch_bounds__(64 * kWaves, LOOP ? 2 : 4) void linear_w32_kernel(L
     } else multiply(cur, s0);
 
     // ---- the waves' partial sums, in the accumulators' own layout: lane (li, lg) holds row 16 mt + li and, in its four
-    // registers, operand rows 4 lg .. 4 lg + 3
+    // registers, columns 4 lg .. 4 lg + 3
     f32x4* part = reinterpret_cast<f32x4*>(smem);
 #pragma unroll
-    for (int f = 0; f < NF; f++)
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) part[((wave * NF + f) * MT + mt) * 64 + lane] = acc[f][mt];
+    for (int mt = 0; mt < MT; mt++) part[(wave * MT + mt) * 64 + lane] = acc[mt];
     __syncthreads();
     if (wave >= MT) return;
-    f32x4 sum[NF];
+    f32x4 sum = part[wave * 64 + lane];
 #pragma unroll
-    for (int f = 0; f < NF; f++) {
-        sum[f] = part[(f * MT + wave) * 64 + lane];
-#pragma unroll
-        for (int w = 1; w < kWaves; w++) sum[f] += part[((w * NF + f) * MT + wave) * 64 + lane];
-    }
-    if (!finisher) return;
-    // place 4 q + e of the thread's columns
-    auto value = [&](int q, int e) { return TB ? sum[q][e] : sum[(4 * q + e) % NF][(4 * q + e) / NF]; };
+    for (int w = 1; w < kWaves; w++) sum += part[(w * MT + wave) * 64 + lane];
+    if (!finisher || column >= g.N) return;
     if (g.sums) {
-        float* c = g.sums + ((int64_t)split * g.M + fm) * g.N;
-#pragma unroll
-        for (int q = 0; q < NF; q++)
-            if (column(q) < g.N) *reinterpret_cast<f32x4*>(c + column(q)) = f32x4{value(q, 0), value(q, 1), value(q, 2), value(q, 3)};
+        *reinterpret_cast<f32x4*>(g.sums + ((int64_t)split * g.M + fm) * g.N + column) = sum;
         return;
     }
-    T* c = static_cast<T*>(g.c) + (int64_t)fm * g.N;
+    T* c = static_cast<T*>(g.c) + (int64_t)fm * g.N + column;
     dispatch_act(g.act, [&](auto act_tag) {
         constexpr int ACT = decltype(act_tag)::value;
+        Pack4<T> o, r = __builtin_bit_cast(Pack4<T>, res);
 #pragma unroll
-        for (int q = 0; q < NF; q++) {
-            Pack4<T> o, r = __builtin_bit_cast(Pack4<T>, res[q]);
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                o.v[e] = Elem<T>::from_f32(apply_act_c<ACT>(value(q, e) + rounded<T>(bias[q][e])));
-                // (second rounding on purpose: the same result as a separate add over the stored C)
-                if (g.residual) o.v[e] = Elem<T>::from_f32(Elem<T>::to_f32(o.v[e]) + Elem<T>::to_f32(r.v[e]));
-            }
-            if (column(q) < g.N) *reinterpret_cast<u32x2*>(c + column(q)) = __builtin_bit_cast(u32x2, o);
+        for (int e = 0; e < 4; e++) {
+            o.v[e] = Elem<T>::from_f32(apply_act_c<ACT>(sum[e] + rounded<T>(bias[e])));
+            // (second rounding on purpose: the same result as a separate add over the stored C)
+            if (g.residual) o.v[e] = Elem<T>::from_f32(Elem<T>::to_f32(o.v[e]) + Elem<T>::to_f32(r.v[e]));
         }
+        *reinterpret_cast<u32x2*>(c) = __builtin_bit_cast(u32x2, o);
     });
 }
 
@@ -251,8 +193,8 @@ __global__ __launch_bounds__(64 * kWaves, MT < 2 ? 4 : 2) void linear_w32_stream
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int li = lane & 15, lg = lane >> 4;
     const int m0 = (int)blockIdx.y * (16 * MT);
-    const __amdgpu_buffer_rsrc_t rx = lin_rsrc(g.x, (uint32_t)((int64_t)g.M * g.K * 2));
-    const __amdgpu_buffer_rsrc_t rw = lin_rsrc(g.w, (uint32_t)((int64_t)g.N * g.K * 4));
+    const __amdgpu_buffer_rsrc_t rx = make_rsrc(g.x, (uint32_t)((int64_t)g.M * g.K * 2));
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(g.w, (uint32_t)((int64_t)g.N * g.K * 4));
     const int all = (g.K + KS - 1) / KS, per = (all + kWaves - 1) / kWaves, s0 = wave * per, s1 = min(all, s0 + per);
     u32x4 a[U][MT];
 #pragma unroll
@@ -401,13 +343,13 @@ __global__ __launch_bounds__(256) void finish_norm_kernel(LinearArgs g, T* h) {
     }
 }
 
-template <typename T, bool TB, bool LOOP, int NF, int MT, int U>
+template <typename T, bool TB, bool LOOP, int MT, int U>
 int launch_one(hipStream_t s, LinearArgs g) {
-    auto kern = linear_w32_kernel<T, TB, LOOP, NF, MT, U>;
-    constexpr int kSums = kWaves * NF * MT * 1024;
+    auto kern = linear_w32_kernel<T, TB, LOOP, MT, U>;
+    constexpr int kSums = kWaves * MT * 1024;
     static_assert(kSums <= 64 * 1024, "more LDS than a launch gets unasked");
     g.blocks = (g.M + 16 * MT - 1) / (16 * MT);
-    g.strips = (g.N + 16 * NF - 1) / (16 * NF);
+    g.strips = (g.N + 15) / 16;
     g.per_xcd = (g.strips + kXcds - 1) / kXcds;
     g.first = 0;
     for (Band& a : g.ahead) {
@@ -433,8 +375,8 @@ int launch_rows(hipStream_t s, const LinearArgs& g, bool tb) {
         hipLaunchKernelGGL((linear_w32_stream_kernel<T, MT, 3>), dim3((unsigned)(t.strips < room ? t.strips : room), (unsigned)blocks), dim3(64 * kWaves), 0, s, t);
         return check_launch("linear_w32_stream");
     }
-    if (tb) return launch_one<T, true, true, 1, MT, 3>(s, g);
-    return loop ? launch_one<T, false, true, 1, MT, 3>(s, g) : launch_one<T, false, false, 1, MT, 3>(s, g);
+    if (tb) return launch_one<T, true, true, MT, 3>(s, g);
+    return loop ? launch_one<T, false, true, MT, 3>(s, g) : launch_one<T, false, false, MT, 3>(s, g);
 }
 
 template <typename T>

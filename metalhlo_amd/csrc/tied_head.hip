@@ -31,24 +31,6 @@ struct HeadArgs {
     int strips, per;      // sixteen columns each; strips per workgroup
 };
 
-template <typename T> struct HeadMfma;
-template <> struct HeadMfma<bf16_t> {
-    __device__ static f32x4 run(u32x4 b, u32x4 a, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b), __builtin_bit_cast(bf16x8, a), c, 0, 0, 0);
-    }
-};
-template <> struct HeadMfma<f16_t> {
-    __device__ static f32x4 run(u32x4 b, u32x4 a, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, b), __builtin_bit_cast(f16x8, a), c, 0, 0, 0);
-    }
-};
-template <typename T>
-__device__ __forceinline__ uint32_t head_pair(float lo, float hi) {
-    typedef T pair __attribute__((ext_vector_type(2)));
-    const pair p = {Elem<T>::from_f32(lo), Elem<T>::from_f32(hi)};
-    return __builtin_bit_cast(uint32_t, p);
-}
-
 template <typename T>
 __global__ __launch_bounds__(64 * kHeadWaves) void tied_head_kernel(HeadArgs g) {
     extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -116,9 +98,9 @@ __global__ __launch_bounds__(64 * kHeadWaves) void tied_head_kernel(HeadArgs g) 
                 if (s + 1 < kHeadSteps) read(s + 1);
                 __builtin_amdgcn_sched_barrier(0);           // (left alone the compiler moves the reads down to their use)
                 const f32x4 lo = raw[s & 1][0], hi = raw[s & 1][1];
-                const u32x4 b = {head_pair<T>(lo[0], lo[1]), head_pair<T>(lo[2], lo[3]), head_pair<T>(hi[0], hi[1]), head_pair<T>(hi[2], hi[3])};
-                acc[0] = HeadMfma<T>::run(b, a[0][s], acc[0]);
-                acc[1] = HeadMfma<T>::run(b, a[1][s], acc[1]);
+                const u32x4 b = {round_pair<T>(lo[0], lo[1]), round_pair<T>(lo[2], lo[3]), round_pair<T>(hi[0], hi[1]), round_pair<T>(hi[2], hi[3])};
+                acc[0] = Tile16<T>::run(b, a[0][s], acc[0]);
+                acc[1] = Tile16<T>::run(b, a[1][s], acc[1]);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -126,7 +108,7 @@ __global__ __launch_bounds__(64 * kHeadWaves) void tied_head_kernel(HeadArgs g) 
         const int n = strip * kHeadCols + 4 * lg;
 #pragma unroll
         for (int b = 0; b < 2; b++) {
-            const u32x2 v = {head_pair<T>(acc[b][0], acc[b][1]), head_pair<T>(acc[b][2], acc[b][3])};
+            const u32x2 v = {round_pair<T>(acc[b][0], acc[b][1]), round_pair<T>(acc[b][2], acc[b][3])};
             __builtin_amdgcn_raw_buffer_store_b64(v, rc, row[b] >= 0 && n < g.N ? (uint32_t)(((int64_t)row[b] * g.N + n) * 2) : kOob, 0, 0);
         }
         slot = slot == 2 ? 0 : slot + 1;
