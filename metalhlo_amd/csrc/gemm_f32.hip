@@ -381,11 +381,14 @@ int64_t large_tiles(int64_t M, int64_t N, int64_t batch) { return ((M + 127) / 1
 // per compute unit) below that.  Measured with the ring (us, 64 | 128): 4096^3 1060 | 1038, 2048^3 143 | 157,
 // [8192,768] x K 3072 308 | 405; register-staged 1183 at 4096^3 (128), 173 at 2048^3 and 382 (64).  Rings of
 // three and four stages are 2 to 8 % behind two: the workgroups of a unit hide each other's latency.
+// Four-byte loads keep the 64x64 tiles: 128x128 ones take 272 to 308 registers, one workgroup a unit (us, 64 | 128 | register-staged
+// 128): [4095,4095] x K 1023 366 | 467 | 425, [16383,1027] x K 771 stored [N, K] 309 | 449 | 333, [8191,2047] x K 2047 707 | 844 | 687,
+// [6001,3001] x K 3001 1133 | 1442 | 1203, [4093,4097] x K 4099 with A stored [K, M] 1403 | 1766 | 1599.
 template <bool TA, bool TB>
 int launch(hipStream_t s, const GemmArgs& g, int64_t batch, bool ring, bool wide) {
     const bool large = large_tiles(g.M, g.N, batch) >= 960 && !g.partial;
     if (ring && wide) return large ? launch_ring<TA, TB, 2, 2, 16>(s, g, batch) : launch_ring<TA, TB, 1, 2, 16>(s, g, batch);
-    if (ring) return large ? launch_ring<TA, TB, 2, 2, 4>(s, g, batch) : launch_ring<TA, TB, 1, 2, 4>(s, g, batch);
+    if (ring) return launch_ring<TA, TB, 1, 2, 4>(s, g, batch);
     return large ? launch_tile<TA, TB, 2>(s, g, batch) : launch_tile<TA, TB, 1>(s, g, batch);
 }
 

@@ -57,3 +57,11 @@ def test_few_rows_off_16_bytes(M, N, K, tb):
                                       (128, 511, 2047, True), (128, 1024, 4096, False)], ids=lambda v: str(v))
 def test_few_rows_with_blocks_and_parts_chosen_together(M, N, K, tb):
     _check(M, N, K, torch.float32, False, tb, residual=M % 8 == 0)
+
+
+@pytest.mark.parametrize("M,N,K", [(3970, 3972, 36), (3969, 3972, 516)], ids=lambda v: str(v))
+def test_large_products_off_16_bytes_have_the_bits_of_aligned_ones(M, N, K):
+    """Tiles of 64x64 with four-byte loads where an aligned product has 128x128."""
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a, w = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N * K + 1, generator=g, device="cuda")
+    assert torch.equal(kernels.matmul(a, w[1:].view(K, N)), kernels.matmul(a, w[1:].clone().view(K, N)))

@@ -52,3 +52,12 @@ def test_whole_stages_do_not_pay_for_the_rest_of_k():
         # (type, A and B transposed, K in parts, a rest of K)
         tn, nn = ([n for n in count if "Lb%cELb0ELb%cELb0E" % (ta, split) in n] for ta in "10")
         assert len(tn) == len(nn) == 2 and max(count[n] for n in tn) <= max(count[n] for n in nn)
+
+
+def test_fp32_rings_leave_a_unit_several_workgroups():
+    """A workgroup of the fp32 ring waits at a barrier per stage: another one of the unit has to fill that time."""
+    if not os.path.exists(LIB):
+        pytest.skip("no built library")
+    found = [k for k in _kernels() if "gemm_f32_ring_kernel" in k[".name"]]
+    assert found
+    assert [(k[".name"], k[".vgpr_count"]) for k in found if k[".vgpr_count"] > 256] == []
