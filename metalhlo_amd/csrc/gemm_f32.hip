@@ -309,39 +309,48 @@ __global__ __launch_bounds__(256) void gemm_f32_ring_kernel(GemmArgs g) {
     for (int p = 0; p < S - 1; p++) load(kt0 + p);
     // A loop for the stages of each part: with the end of a part tested in one loop over all stages a stage took 0.07 us more,
     // [512,768] x K 768 stored [N, K] 20.9 -> 19.4 us, [476,1232] x K 264 13.9 -> 13.3, [1000,1000] x K 500 16.6 -> 15.5.
+    // Small tiles add a part up in the next one's first stage, where the barrier and the LDS reads give its last products time.
+    // us, behind its last stage | in the next one's first: [2048,768] x K 3072 112.3 | 110.8, [3782,1120] x K 2048 175.0 | 172.7, x^T dy [768,3072]
+    // over 8192 404 | 398; without parts 111.3, 173.7 and 405; few stages a part: [512,768] x K 768 19.8 | 19.4, stored [N, K] 19.5 | 19.6.
+    // (The other forms have no registers for a stage of its own: 228 -> 264 with 128x128 tiles, one workgroup a unit instead of two.)
+    constexpr bool kLate = WB == 1 && W == 16;
+    auto stage = [&](int kt, auto first) __attribute__((always_inline)) {
+        // stage kt has landed when only the S - 2 stages behind it are in flight; past the barrier that holds for
+        // every wave's share, and every wave has read stage kt - 1, whose place is reused
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * kLoads) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        load(kt + S - 1);
+        const char* at = smem + ((kt - kt0) % S) * kStage;
+        f32x4 af[2][WB], bf[2][WB];
+        auto read = [&](int s, f32x4(&fa)[WB], f32x4(&fb)[WB]) {
+#pragma unroll
+            for (int i = 0; i < WB; i++) {
+                fa[i] = ring_frag<kTile, !TA>(at, (wm * WB + i) * 32, s, lane);
+                fb[i] = ring_frag<kTile, TB>(at + kBytes, (wn * WB + i) * 32, s, lane);
+            }
+        };
+        read(0, af[0], bf[0]);
+        if (first) close_part();
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            if (s < 3) read(s + 1, af[(s + 1) & 1], bf[(s + 1) & 1]);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int i = 0; i < WB; i++)
+#pragma unroll
+                    for (int j = 0; j < WB; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(bf[s & 1][j][e], af[s & 1][i][e], acc[i][j], 0, 0, 0);
+        }
+    };
     for (int k0 = kt0; k0 < kt1; k0 += per) {
         const int k1 = min(kt1, k0 + per);
-        for (int kt = k0; kt < k1; kt++) {
-            // stage kt has landed when only the S - 2 stages behind it are in flight; past the barrier that holds for
-            // every wave's share, and every wave has read stage kt - 1, whose place is reused
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * kLoads) : "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            load(kt + S - 1);
-            const char* at = smem + ((kt - kt0) % S) * kStage;
-            f32x4 af[2][WB], bf[2][WB];
-            auto read = [&](int s, f32x4(&fa)[WB], f32x4(&fb)[WB]) {
-#pragma unroll
-                for (int i = 0; i < WB; i++) {
-                    fa[i] = ring_frag<kTile, !TA>(at, (wm * WB + i) * 32, s, lane);
-                    fb[i] = ring_frag<kTile, TB>(at + kBytes, (wn * WB + i) * 32, s, lane);
-                }
-            };
-            read(0, af[0], bf[0]);
-#pragma unroll
-            for (int s = 0; s < 4; s++) {
-                if (s < 3) read(s + 1, af[(s + 1) & 1], bf[(s + 1) & 1]);
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-#pragma unroll
-                    for (int i = 0; i < WB; i++)
-#pragma unroll
-                        for (int j = 0; j < WB; j++)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(bf[s & 1][j][e], af[s & 1][i][e], acc[i][j], 0, 0, 0);
-            }
-        }
-        close_part();
+        if (kLate) stage(k0, std::true_type{});
+        for (int kt = k0 + kLate; kt < k1; kt++) stage(kt, std::false_type{});
+        if (!kLate) close_part();
     }
+    if (kLate) close_part();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // nothing may land in LDS after the workgroup ends
     store_f32<WB>(g, sum, m0 + wm * 32 * WB, n0 + wn * 32 * WB, batch, lane);
 }
