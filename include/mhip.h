@@ -123,8 +123,8 @@ int mhip_bias_gelu_erf(void* stream, const void* x, const void* bias, void* y, i
  * when trans_b); strides are in elements between consecutive batch matrices
  * (0 broadcasts an operand).  bias (length N, same dtype) may be NULL.
  * fp32 accumulate, one rounding at the store.  The order in which a row's products are added, and with it the
- * last bits, is the same for any number of rows from 193 on while K is below 4096 (for F32: any K); with fewer rows
- * or a longer K it may change with M and batch.  dtype: BF16, F16, F32; also F64 (f64
+ * last bits, is the same for any number of rows from 193 on while K is below 4096 (for F32: any K, with at least 12
+ * columns and while op(A) and op(B) are below 2 GB each); otherwise it may change with M and batch.  dtype: BF16, F16, F32; also F64 (f64
  * accumulate) and I32 / I64 (wrap-around), those three without activation.
  * Replaces the kernel_matmul family and kernel_matmul_bias_act
  * (Compiler/CodeGenerator.swift:3155-4068, 4797-4850); M/K/N/batch are what

@@ -65,3 +65,15 @@ def test_large_products_off_16_bytes_have_the_bits_of_aligned_ones(M, N, K):
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     a, w = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N * K + 1, generator=g, device="cuda")
     assert torch.equal(kernels.matmul(a, w[1:].view(K, N)), kernels.matmul(a, w[1:].clone().view(K, N)))
+
+
+@pytest.mark.parametrize("ta", [False, True])
+def test_twelve_columns_keep_a_rows_bits(ta):
+    """The narrowest C whose rows have the same bits from 193 rows on."""
+    g = torch.Generator(device="cuda").manual_seed(12)
+    a, b = torch.randn(4000, 1030, generator=g, device="cuda"), torch.randn(1030, 12, generator=g, device="cuda")
+
+    def rows(n):
+        x = (a[:n].t() if ta else a[:n]).contiguous()
+        return kernels.matmul(x, b, trans_a=ta)[:193]
+    assert torch.equal(rows(193), rows(4000))
