@@ -30,6 +30,7 @@ SIGNATURES = {
     "mhip_gemm_residual": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                                   _i32, _i32, _i32, _i32]),
     "mhip_gemm_workspace": (_i64, [_i64, _i64, _i64, _i64, _i32, _i32, _i32]),
+    "mhip_gemm_workspace_launches": (_i32, [_i64, _i64, _i64, _i64, _i32, _i32, _i32]),
     "mhip_gemm_ws": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                             _i32, _i32, _i32, _i32, _vp, _i64]),
     "mhip_linear_w32_ok": (_i32, [_i64, _i64, _i64, _i32]),

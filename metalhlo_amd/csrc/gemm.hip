@@ -304,6 +304,10 @@ int64_t gemm_any_workspace(int64_t M, int64_t N, int64_t K, int64_t batch);
 // gemm_any.hip also makes copies with aligned rows.
 GemmPack gemm_pack_plan(const GemmArgs& g, int trans_a, int trans_b, bool a_off, bool b_off);
 int launch_gemm_pack(hipStream_t s, const GemmArgs& g, const GemmPack& p, int trans_a, int trans_b, char* to);
+// gemm_strip.hip: few rows, K in parts that one launch adds up.
+bool gemm_parts_wanted(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b);
+int64_t gemm_parts_workspace(int64_t M, int64_t N, int64_t K);
+int launch_gemm_parts(hipStream_t s, const GemmArgs& g, int trans_b, int dtype);
 int launch_gemm_skinny(hipStream_t s, GemmArgs g, int64_t batch, int trans_b, int dtype, int64_t workspace_bytes);
 // gemm_mid.hip: 64- and 128-row tiles through a ring of LDS stages, K split where that leaves units idle.
 int64_t gemm_mid_workspace(int64_t M, int64_t N, int64_t K, int64_t sum_k, int64_t batch, int trans_a, int trans_b);
@@ -615,6 +619,9 @@ static int gemm_entry(void* stream, const void* a, const void* b, const void* bi
                         stride_b % 8 == 0 && (int64_t)M * K * 2 < 0x7FFFFFFFLL &&
                         (int64_t)N * K * 2 < 0x7FFFFFFFLL;
     g.partial = static_cast<float*>(workspace);
+    if (vec_ok && g.partial && gemm_parts_wanted(M, N, K, batch, trans_a, trans_b) && workspace_bytes >= gemm_parts_workspace(M, N, K) &&
+        tune_int("MHIP_GEMM_TILE", 0) == 0 && few_row_choice(tuned_gemm_variant(g, batch, trans_a, trans_b, dtype)))
+        return chose(128, launch_gemm_parts(s, g, trans_b, dtype));
     // Few rows: the kernel that reads B once with all of its loads in flight, unless a tile kernel is asked for by
     // name or by the tuning table.
     if ((is16 || dtype == MHIP_F32) && gemm_skinny_eligible(g, trans_a, is16 ? 2 : 4) && (is16 && !vec_ok ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, batch, trans_b, is16)) &&
@@ -691,6 +698,7 @@ extern "C" int64_t mhip_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t 
     if (!is16 && dtype != MHIP_F32) return 0;
     const bool vec = is16 && (trans_a ? M : K) % 8 == 0 && (trans_b ? K : N) % 8 == 0;
     if (!is16 && f32_rows_in_parts(M, N, K, batch, trans_a, trans_b) > 0) return f32_rows_in_parts(M, N, K, batch, trans_a, trans_b);
+    if (vec && gemm_parts_wanted(M, N, K, batch, trans_a, trans_b)) return gemm_parts_workspace(M, N, K);
     if (!trans_a && M <= (is16 ? 64 : 192) && (is16 && !vec ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, batch, trans_b, is16))) return gemm_skinny_workspace(M, N, K, batch, trans_b, is16);
     // (a large problem goes to the ring kernels, whose tiles fill the device)
     if (!is16) return gemm_f32_workspace(M, N, K, batch, trans_a, trans_b);
@@ -703,4 +711,10 @@ extern "C" int64_t mhip_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t 
     }
     if (!vec) return short_product(M, N, K) ? 0 : gemm_any_workspace(M, N, K, batch);
     return aligned_workspace(M, N, K, K, trans_a, trans_b);
+}
+
+extern "C" int mhip_gemm_workspace_launches(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b, int dtype) {
+    if (mhip_gemm_workspace(M, N, K, batch, trans_a, trans_b, dtype) == 0) return 0;
+    const bool vec = (dtype == MHIP_BF16 || dtype == MHIP_F16) && (trans_a ? M : K) % 8 == 0 && (trans_b ? K : N) % 8 == 0;
+    return vec && gemm_parts_wanted(M, N, K, batch, trans_a, trans_b) ? 0 : 1;
 }

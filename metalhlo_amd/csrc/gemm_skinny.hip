@@ -21,6 +21,8 @@
 namespace mhip {
 
 int launch_gemm_finish(hipStream_t s, const GemmArgs& g, int dtype);     // gemm_mid.hip
+bool gemm_strip_wanted(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b);          // gemm_strip.hip
+int launch_gemm_strip(hipStream_t s, const GemmArgs& g, int64_t batch, int dtype);
 
 namespace {
 
@@ -302,7 +304,7 @@ RowsPlan rows_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool tb) {
 }
 
 int skinny_splits(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b, bool is16) {
-    if (batch != 1 || M * N > (1 << 20)) return 1;
+    if (batch != 1 || M * N > (1 << 20) || (is16 && gemm_strip_wanted(M, N, K, batch, trans_b))) return 1;
     if (!is16 && rows_plan(M, N, K, batch, trans_b != 0).splits > 1) return rows_plan(M, N, K, batch, trans_b != 0).splits;
     const int64_t width = wide_strips(N, K, 1, trans_b != 0) ? (trans_b ? 32 : 64) : (trans_b ? 16 : 32);
     const int64_t from = is16 ? (trans_b && M <= 16 ? 3584 : 2560) : (M > 32 ? 3072 : 2560);
@@ -369,6 +371,7 @@ int dtype_launch(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_b, i
     const int per16 = dtype == MHIP_F32 ? 4 : 8;
     const bool vec = g.lda % per16 == 0 && g.ldb % per16 == 0 && g.sa % per16 == 0 && g.sb % per16 == 0 &&
                      ((reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.b)) & 15) == 0;
+    if (vec && dtype != MHIP_F32 && gemm_strip_wanted(g.M, g.N, g.K, batch, trans_b)) return launch_gemm_strip(s, g, batch, dtype);
 #define MHIP_SKINNY(T)                                                                                              \
     (vec ? (trans_b ? launch_shape<T, true, true>(s, g, batch) : launch_shape<T, false, true>(s, g, batch))         \
          : (trans_b ? launch_shape<T, true, false>(s, g, batch) : launch_shape<T, false, false>(s, g, batch)))

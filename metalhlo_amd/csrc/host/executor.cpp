@@ -862,9 +862,9 @@ static std::vector<DeviceTensor> run_ops(Executable& exe, const std::vector<Devi
                 int64_t bytes = exe.no_workspace ? 0 : mhip_gemm_workspace(M, N, K, 1, ta, tb, dt);
                 // (16-bit rows on 16 bytes: the workspace is for parts of K alone)
                 const bool parts_only = (dt == BF16 || dt == F16) && (ta ? M : K) % 8 == 0 && (tb ? K : N) % 8 == 0;
-                const bool small = parts_only && K < 8192;
+                const bool more = bytes > 0 && mhip_gemm_workspace_launches(M, N, K, 1, ta, tb, dt) > 0, small = more && parts_only && K < 8192;
                 if (small && exe.whole_sums) bytes = 0;
-                if (bytes > 0) {
+                if (bytes > 0 && more) {
                     count.finishes++;
                     count.small += small;
                 }

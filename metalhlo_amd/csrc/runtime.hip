@@ -4,7 +4,11 @@
 #include <stdlib.h>
 #include <string.h>
 
-#include "common.h"
+#include <atomic>
+#include <chrono>
+#include <random>
+
+#include "arrive.h"
 
 namespace mhip {
 
@@ -30,6 +34,17 @@ int tune_int(const char* name, int fallback) {
     char* end = nullptr;
     const long r = strtol(v, &end, 10);
     return (end && *end == 0 && r > 0 && r < (1 << 20)) ? (int)r : fallback;
+}
+
+uint64_t launch_tag() {
+    static std::atomic<uint64_t> next{[] {
+        std::random_device r;
+        return ((uint64_t)r() << 32) ^ r() ^ (uint64_t)std::chrono::steady_clock::now().time_since_epoch().count();
+    }()};
+    // (a bijection of a counter whose upper 56 bits all differ: steps of 256 reach every one of them)
+    const uint64_t n = next.fetch_add(256, std::memory_order_relaxed) & ~(uint64_t)255;
+    const uint64_t t = (n * 0x9E3779B97F4A7C15ull) & ~(uint64_t)255;
+    return t ? t : launch_tag();
 }
 
 int compute_units() {
