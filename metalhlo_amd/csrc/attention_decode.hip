@@ -4,7 +4,8 @@
 // A query tile of 128 rows would be almost all padding, and its one workgroup per head walks the keys through
 // LDS stages with little in flight.  Here every wave of a workgroup takes blocks of 32 keys of its own, loads
 // them straight into matrix operands (no LDS, no barrier in the loop) one block ahead, and keeps its own
-// softmax state; the waves meet at the end in LDS, and the parts of a split key range in a workspace.
+// softmax state; the waves meet at the end in LDS, and the parts of a split key range in a workspace, where the last
+// workgroup of a head to arrive puts them together (arrive.h).
 //
 //   S^T = K Q^T     v_mfma_f32_16x16x32: operand row = key, so a lane loads 16 bytes of one key's row; a lane
 //                   of the result holds four keys of one query.
@@ -13,6 +14,7 @@
 //                   eight keys of a lane are the ones whose probabilities it just computed.
 #include <type_traits>
 
+#include "arrive.h"
 #include "attention_common.h"
 
 namespace mhip {
@@ -32,18 +34,22 @@ template <> struct Mfma16A<f16_t> {
 
 constexpr int kKeys = 32;        // keys per block
 constexpr int kMaxSq = 16;
-constexpr int kPartKeys = 256;   // a part of a split key range is a multiple of this
+// A part of a split key range is a multiple of this.  us, multiples of 128 | 256 keys: one query of 32 heads over 512 keys, head size 128,
+// 6.7 | 8.1, of 24 over 1024, 64, 6.4 | 6.7, of 8 over 2048, 128, 8.7 | 8.5; eight queries of 8 heads over 4096, 64, 15.9 | 10.5; 12 heads
+// over 300 keys 6.4 | 5.4 (whole).
+constexpr int part_keys(int64_t Skv) { return Skv >= 512 && Skv <= 1024 ? 128 : 256; }
 
 // domain of scores and reference (see moved_reference): f16's lowest number is far from fp32's
 template <typename T, bool HAS_MASK>
 constexpr bool kNatural = HAS_MASK && std::is_same<T, bf16_t>::value;
 
 template <typename T, int D, bool HAS_MASK, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* part, int per_part) {
+__global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* part, int per_part, uint64_t* words, uint64_t tag) {
     constexpr bool NAT = kNatural<T, HAS_MASK>;
     constexpr int NS = D / 32, NF = D / 16, VDw = NF / 2;      // k steps of Q K^T, tiles of O^T, dwords of a lane's V piece
     __shared__ __attribute__((aligned(16))) float sums[WAVES][NF][64][4];
     __shared__ float ml[2][WAVES][kMaxSq];
+    __shared__ int last;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int li = lane & 15, lg = lane >> 4;
     const int bh = blockIdx.x, b_i = bh / a.H, h_i = bh % a.H;
@@ -56,6 +62,8 @@ __global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* 
     const __amdgpu_buffer_rsrc_t rv = fa_rsrc(vp, (uint32_t)((((int64_t)a.Skv - 1) * v_rs + D) * 2));
     const T* mp = HAS_MASK ? static_cast<const T*>(a.mask) + (int64_t)b_i * a.mask_sb + (int64_t)h_i * a.mask_sh : nullptr;
 
+    uint64_t seen = 0;
+    if (part && threadIdx.x == 0) seen = arrive_look(words + bh);
     u32x4 qf[NS];
 #pragma unroll
     for (int s = 0; s < NS; s++) {
@@ -161,6 +169,7 @@ __global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* 
         }
     }
 
+    if (part && threadIdx.x == 0) arrive_claim(words + bh, seen, tag);
     // ---- the waves' states
     l_run += __shfl_xor(l_run, 16, 64);
     l_run = half_sum(l_run);
@@ -184,37 +193,54 @@ __global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* 
         if (part) {
             // [part][bh][Sq][D] sums, then [part][bh][Sq][2] reference maximum and sum
             const int64_t at = ((int64_t)blockIdx.y * gridDim.x + bh) * a.Sq + q;
-            part[at * D + d] = o;
-            if (d < 2) part[(int64_t)gridDim.y * gridDim.x * a.Sq * D + at * 2 + d] = d ? l : m;
+            store_part(part + at * D + d, o);
+            if (d < 2) store_part(part + (int64_t)gridDim.y * gridDim.x * a.Sq * D + at * 2 + d, d ? l : m);
         } else {
             op[(int64_t)q * a.os[2] + d] = Elem<T>::from_f32(o * (l > 1e-10f ? 1.f / l : 0.f));
         }
     }
-}
+    const int parts = gridDim.y;
+    if (!part || !arrive_last(words + bh, parts, &last)) return;
 
-// The parts of a split key range: one thread per element of O.
-template <typename T, int D, bool HAS_MASK>
-__global__ __launch_bounds__(256) void fa_decode_combine_kernel(FaArgs a, const float* part, int parts) {
-    const int64_t rows = (int64_t)a.B * a.H * a.Sq, idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= rows * D) return;
-    const int64_t row = idx / D;
-    const int d = (int)(idx % D);
-    const float* mls = part + (int64_t)parts * rows * D;
-    float m = -INFINITY, l = 0.f, o = 0.f;
-    for (int p = 0; p < parts; p++) m = fmaxf(m, mls[(p * rows + row) * 2]);
-    const float m_use = m == -INFINITY ? 0.f : m;
-    for (int p = 0; p < parts; p++) {
-        const float al = weight<kNatural<T, HAS_MASK>>(mls[(p * rows + row) * 2], m_use);
-        l = fmaf(mls[(p * rows + row) * 2 + 1], al, l);
-        o = fmaf(part[(p * rows + row) * D + d], al, o);
+    // ---- the last part of the head to arrive: an element of O a thread, eight parts' loads in flight
+    const int64_t rows = (int64_t)gridDim.x * a.Sq;
+    for (int idx = threadIdx.x; idx < a.Sq * D; idx += 64 * WAVES) {
+        const int q = idx / D, d = idx % D;
+        const int64_t row = (int64_t)bh * a.Sq + q;
+        const float* mls = part + parts * rows * D + row * 2;
+        const float* os = part + row * D + d;
+        float m = -INFINITY, l = 0.f, o = 0.f;
+        for (int p0 = 0; p0 < parts; p0 += 8) {
+            float pm[8], pl[8], po[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const int p = min(p0 + u, parts - 1);
+                pm[u] = load_part(mls + p * rows * 2);
+                pl[u] = load_part(mls + p * rows * 2 + 1);
+                po[u] = load_part(os + p * rows * D);
+            }
+            float m_new = m;
+#pragma unroll
+            for (int u = 0; u < 8; u++) m_new = fmaxf(m_new, pm[u]);
+            const float m_use = m_new == -INFINITY ? 0.f : m_new, old = weight<NAT>(m, m_use);
+            l *= old;
+            o *= old;
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                if (p0 + u >= parts) break;
+                const float al = weight<NAT>(pm[u], m_use);
+                l = fmaf(pl[u], al, l);
+                o = fmaf(po[u], al, o);
+            }
+            m = m_new;
+        }
+        op[(int64_t)q * a.os[2] + d] = Elem<T>::from_f32(o * (l > 1e-10f ? 1.f / l : 0.f));
     }
-    const int64_t bh = row / a.Sq;
-    static_cast<T*>(a.o)[bh / a.H * a.os[0] + bh % a.H * a.os[1] + row % a.Sq * a.os[2] + d] = Elem<T>::from_f32(o * (l > 1e-10f ? 1.f / l : 0.f));
 }
 
-// Parts of the key range: enough workgroups for two per compute unit, each with at least 256 keys.
+// Parts of the key range: enough workgroups for two per compute unit, each with at least part_keys().
 int decode_parts(int64_t bh, int64_t Skv) {
-    const int64_t want = (512 + bh - 1) / bh, most = Skv / kPartKeys;
+    const int64_t want = (512 + bh - 1) / bh, most = Skv / part_keys(Skv);
     const int64_t n = want < most ? want : most;
     return n < 2 ? 1 : n > 64 ? 64 : (int)n;
 }
@@ -222,17 +248,14 @@ int decode_parts(int64_t bh, int64_t Skv) {
 template <typename T, int D>
 int launch(hipStream_t s, const FaArgs& a, float* part, int parts) {
     const int64_t bh = (int64_t)a.B * a.H;
-    const int per = parts == 1 ? a.Skv : (int)(((a.Skv + parts - 1) / parts + kPartKeys - 1) / kPartKeys * kPartKeys);
+    const int per = parts == 1 ? a.Skv : (int)(((a.Skv + parts - 1) / parts + part_keys(a.Skv) - 1) / part_keys(a.Skv) * part_keys(a.Skv));
     const dim3 grid((unsigned)bh, (unsigned)((a.Skv + per - 1) / per));
     constexpr int WAVES = 4;
-    if (a.mask) hipLaunchKernelGGL((fa_decode_kernel<T, D, true, WAVES>), grid, dim3(64 * WAVES), 0, s, a, parts > 1 ? part : nullptr, per);
-    else hipLaunchKernelGGL((fa_decode_kernel<T, D, false, WAVES>), grid, dim3(64 * WAVES), 0, s, a, parts > 1 ? part : nullptr, per);
-    if (parts > 1) {
-        const int64_t n = bh * a.Sq * D;
-        const dim3 combine((unsigned)((n + 255) / 256));
-        if (a.mask) hipLaunchKernelGGL((fa_decode_combine_kernel<T, D, true>), combine, dim3(256), 0, s, a, part, (int)grid.y);
-        else hipLaunchKernelGGL((fa_decode_combine_kernel<T, D, false>), combine, dim3(256), 0, s, a, part, (int)grid.y);
-    }
+    uint64_t* words = reinterpret_cast<uint64_t*>(part + (int64_t)parts * bh * a.Sq * (D + 2));
+    const uint64_t tag = parts > 1 ? launch_tag() : 0;
+    if (parts == 1) part = nullptr;
+    if (a.mask) hipLaunchKernelGGL((fa_decode_kernel<T, D, true, WAVES>), grid, dim3(64 * WAVES), 0, s, a, part, per, words, tag);
+    else hipLaunchKernelGGL((fa_decode_kernel<T, D, false, WAVES>), grid, dim3(64 * WAVES), 0, s, a, part, per, words, tag);
     return check_launch("flash_attention_decode");
 }
 
@@ -244,7 +267,7 @@ bool fa_decode_eligible(const FaArgs& a) { return a.Sq <= kMaxSq && !a.is_causal
 int64_t fa_decode_workspace(int64_t bh, int64_t Sq, int64_t Skv, int64_t D) {
     if (Sq < 1 || Sq > kMaxSq || (D != 64 && D != 128)) return 0;
     const int parts = decode_parts(bh, Skv);
-    return parts == 1 ? 0 : parts * bh * Sq * (D + 2) * 4;
+    return parts == 1 ? 0 : parts * bh * Sq * (D + 2) * 4 + bh * 8;
 }
 
 int launch_fa_decode(hipStream_t s, const FaArgs& a, int64_t D, int dtype, void* workspace, int64_t workspace_bytes) {
