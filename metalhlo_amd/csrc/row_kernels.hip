@@ -429,8 +429,11 @@ void row_split_kernel(const T* __restrict__ x, const T* __restrict__ gamma, cons
 // write.  A row that starts at an odd address begins with up to 16 / sizeof(T) - 1 single elements, then whole
 // aligned vectors, then the rest; thread t < 16 owns head element t, thread 16 + t tail element t.  The
 // parameters are read at the row's phase, unaligned (cached, and global loads need no alignment here).
-// What bounds a launch with few rows is what one compute unit moves: [128,50257] bf16 107 us with the
-// scalar three-pass kernel below -> 8.5 us.
+// What bounds a launch with few rows is what one compute unit moves, and for softmax its exponentials (16 cycles a wave each, 1.3 us
+// of a row of 50257, which is why they are computed once): [128,50257] bf16 107 us with the scalar three-pass kernel below, 8.9
+// here with the exponentials computed for the sum and again for the result, 8.4 with them kept.  SHARE workgroups of one XCD then take a row together: each reads all of it, its own
+// share first, which is the one it writes; what the others have read by then comes from the L2.  The partial sums of shares are added in
+// an order that is the same for all of them, so that a row is scaled by one number.
 // ---------------------------------------------------------------------------
 typedef u32x4 u32x4_any __attribute__((aligned(2)));
 
@@ -463,16 +466,33 @@ __device__ inline float row_reduce(float v, float* slots) {
     return r;
 }
 
-template <typename T, int OP, int NT, int NV>
+template <typename T, int OP, int NT, int NV, int SHARE>
 __global__ __launch_bounds__(NT < 256 ? 256 : NT) void row_any_kernel(const T* __restrict__ x, const T* __restrict__ gamma,
                                                                       const T* __restrict__ beta, T* __restrict__ y, int64_t rows,
                                                                       int cols, float eps) {
     constexpr int E = Elem<T>::kPerVec;
     constexpr bool k16 = sizeof(T) == 2;
     __shared__ float red[2][NT / 64];
-    const int64_t row = NT < 256 ? (int64_t)blockIdx.x * (256 / NT) + threadIdx.x / NT : (int64_t)blockIdx.x;
+    static_assert(SHARE == 1 || (NT >= 256 && NV % SHARE == 0 && (SHARE & (SHARE - 1)) == 0), "whole vectors a share");
+    constexpr int kXcd = 8, NS = NV / SHARE;
+    const int64_t row = NT < 256 ? (int64_t)blockIdx.x * (256 / NT) + threadIdx.x / NT
+                        : SHARE > 1 ? (int64_t)(blockIdx.x / (kXcd * SHARE) * kXcd + blockIdx.x % kXcd) : (int64_t)blockIdx.x;
+    const int share = SHARE > 1 ? (int)(blockIdx.x / kXcd % SHARE) : 0;
     const int t = threadIdx.x % NT;
-    if (row >= rows) return;                       // (whole waves: NT >= 64, and only the form without barriers)
+    if (row >= rows) return;                       // (whole waves: NT >= 64, and only the form without barriers, or whole workgroups)
+    // the vector that this workgroup holds as its v-th: those of share (v / NS) ^ share, its own come first
+    auto at = [&](int v) { return ((v / NS ^ share) * NS + v % NS) * NT + t; };
+    // softmax in 16 bits: the exponentials that this workgroup writes, where registers hold them
+    constexpr bool kKeep = OP == kSoftmax && k16 && NS * E <= 64;
+    float kept[kKeep ? NS : 1][kKeep ? E : 1];
+    // (a + b of two shares, then of two pairs: the same for every order that an exclusive or gives)
+    auto add_shares = [&](float(&s)[SHARE]) {
+#pragma unroll
+        for (int w = 1; w < SHARE; w *= 2)
+#pragma unroll
+            for (int i = 0; i < SHARE; i += 2 * w) s[i] += s[i + w];
+        return s[0];
+    };
     const T* xr = x + row * cols;
     T* yr = y + row * cols;
     const RowPhase<T> ph(xr, cols);
@@ -480,7 +500,7 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT) void row_any_kernel(const T* _
     Vec16<T> raw[NV];
 #pragma unroll
     for (int v = 0; v < NV; v++) {
-        const int i = v * NT + t;
+        const int i = at(v);
         raw[v] = __builtin_bit_cast(Vec16<T>, u32x4{0, 0, 0, 0});
         if (i < ph.nvec) raw[v] = load16_stream(xr + ph.head + i * E);
     }
@@ -492,67 +512,69 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT) void row_any_kernel(const T* _
         float m = ei >= 0 ? ev : -INFINITY;
 #pragma unroll
         for (int v = 0; v < NV; v++)
-            if (v * NT + t < ph.nvec) {
+            if (at(v) < ph.nvec) {
 #pragma unroll
                 for (int e = 0; e < E; e++) m = fmaxf(m, Elem<T>::to_f32(raw[v].v[e]));
             }
         m = row_reduce<NT, true>(m, red[0]);
         unit = softmax_unit<T>(m);
         shift = k16 ? m * unit : m;
-        float s = ei >= 0 ? (k16 ? __builtin_amdgcn_exp2f(fmaf(ev, unit, -shift)) : expf(ev - m)) : 0.f;
+        float s[SHARE] = {};
+        const float se = ei >= 0 ? (k16 ? __builtin_amdgcn_exp2f(fmaf(ev, unit, -shift)) : expf(ev - m)) : 0.f;
 #pragma unroll
         for (int v = 0; v < NV; v++)
-            if (v * NT + t < ph.nvec) {
+            if (at(v) < ph.nvec) {
 #pragma unroll
                 for (int e = 0; e < E; e++) {
                     const float f = Elem<T>::to_f32(raw[v].v[e]);
                     const float p = k16 ? __builtin_amdgcn_exp2f(fmaf(f, unit, -shift)) : expf(f - m);
                     if (!k16) raw[v].v[e] = Elem<T>::from_f32(p);       // (kept: exact in fp32)
-                    s += p;
+                    if (kKeep && v < NS) kept[kKeep ? v : 0][kKeep ? e : 0] = p;
+                    s[v / NS] += p;
                 }
             }
-        scale = 1.f / row_reduce<NT, false>(s, red[1]);
+        scale = 1.f / row_reduce<NT, false>(add_shares(s) + se, red[1]);
     } else if (OP == kLayerNorm) {
-        float s = ev;
+        float s[SHARE] = {}, q[SHARE] = {};
 #pragma unroll
-        for (int v = 0; v < NV; v++) s = VecSum<T>::sum(raw[v], s);
-        const float mean = row_reduce<NT, false>(s, red[0]) / n;
-        float q = ei >= 0 ? (ev - mean) * (ev - mean) : 0.f;
+        for (int v = 0; v < NV; v++) s[v / NS] = VecSum<T>::sum(raw[v], s[v / NS]);
+        const float mean = row_reduce<NT, false>(add_shares(s) + ev, red[0]) / n;
+        const float qe = ei >= 0 ? (ev - mean) * (ev - mean) : 0.f;
 #pragma unroll
         for (int v = 0; v < NV; v++)
-            if (v * NT + t < ph.nvec) {
+            if (at(v) < ph.nvec) {
 #pragma unroll
                 for (int e = 0; e < E; e++) {
                     const float d = Elem<T>::to_f32(raw[v].v[e]) - mean;
-                    q = fmaf(d, d, q);
+                    q[v / NS] = fmaf(d, d, q[v / NS]);
                 }
             }
-        scale = 1.f / sqrtf(row_reduce<NT, false>(q, red[1]) / n + eps);
+        scale = 1.f / sqrtf(row_reduce<NT, false>(add_shares(q) + qe, red[1]) / n + eps);
         shift = mean;
     } else {
-        float q = ev * ev;
+        float q[SHARE] = {};
 #pragma unroll
-        for (int v = 0; v < NV; v++) q = VecSum<T>::sumsq(raw[v], q);
-        scale = 1.f / sqrtf(row_reduce<NT, false>(q, red[0]) / n + eps);
+        for (int v = 0; v < NV; v++) q[v / NS] = VecSum<T>::sumsq(raw[v], q[v / NS]);
+        scale = 1.f / sqrtf(row_reduce<NT, false>(add_shares(q) + ev * ev, red[0]) / n + eps);
     }
     auto value = [&](float f, float g, float b) {
         if (OP == kSoftmax) return (k16 ? __builtin_amdgcn_exp2f(fmaf(f, unit, -shift)) : f) * scale;
         return fmaf((f - shift) * scale, g, b);
     };
 #pragma unroll
-    for (int v = 0; v < NV; v++) {
-        const int i = v * NT + t;
+    for (int v = 0; v < NS; v++) {
+        const int i = at(v);
         if (i >= ph.nvec) continue;
         Vec16<T> gv, bv, o;
         if (OP != kSoftmax && gamma) gv = __builtin_bit_cast(Vec16<T>, *reinterpret_cast<const u32x4_any*>(gamma + ph.head + i * E));
         if (OP == kLayerNorm && beta) bv = __builtin_bit_cast(Vec16<T>, *reinterpret_cast<const u32x4_any*>(beta + ph.head + i * E));
 #pragma unroll
         for (int e = 0; e < E; e++)
-            o.v[e] = Elem<T>::from_f32(value(Elem<T>::to_f32(raw[v].v[e]), OP != kSoftmax && gamma ? Elem<T>::to_f32(gv.v[e]) : 1.f,
+            o.v[e] = Elem<T>::from_f32(kKeep ? kept[kKeep ? v : 0][kKeep ? e : 0] * scale : value(Elem<T>::to_f32(raw[v].v[e]), OP != kSoftmax && gamma ? Elem<T>::to_f32(gv.v[e]) : 1.f,
                                              OP == kLayerNorm && beta ? Elem<T>::to_f32(bv.v[e]) : 0.f));
         store16_stream(yr + ph.head + i * E, o);
     }
-    if (ei >= 0) {
+    if (ei >= 0 && share == 0) {
         if (OP == kSoftmax && !k16) ev = expf(ev - shift);
         yr[ei] = Elem<T>::from_f32(value(ev, OP != kSoftmax && gamma ? Elem<T>::to_f32(gamma[ei]) : 1.f,
                                          OP == kLayerNorm && beta ? Elem<T>::to_f32(beta[ei]) : 0.f));
@@ -880,18 +902,36 @@ static int launch_row(hipStream_t s, const void* x, const void* g, const void* b
         // threads per row by its length: a wave up to 128 vectors, 256 threads up to 1024, 1024 beyond
         const int64_t nvec = cols / E;
 #define MHIP_ROW_ANY(NT, NV)                                                                                            \
-    hipLaunchKernelGGL((row_any_kernel<T, OP, NT, NV>), dim3((unsigned)((rows + rows_per_group(NT) - 1) / rows_per_group(NT))), \
+    hipLaunchKernelGGL((row_any_kernel<T, OP, NT, NV, 1>), dim3((unsigned)((rows + rows_per_group(NT) - 1) / rows_per_group(NT))), \
                        dim3(NT < 256 ? 256 : NT), 0, s, xp, gp, bp, yp, rows, (int)cols, eps)
+#define MHIP_ROW_SHARED(NT, NV, SHARE)                                                                                  \
+    hipLaunchKernelGGL((row_any_kernel<T, OP, NT, NV, SHARE>), dim3((unsigned)((rows + 7) / 8 * 8 * SHARE)), dim3(NT), 0, s, xp, gp, bp, yp, rows, (int)cols, eps)
+        // Workgroups per row where rows leave units idle (not in place: one would read what another has written).  us, one | two | four a
+        // row, 50257 columns: softmax bf16 128 rows 8.4 | 8.5 | 12.7, 64 rows 7.6 | 7.3 | 7.1, 8 rows 6.3 | 6.1 | 5.7; LayerNorm bf16 128 rows
+        // 12.6 | 10.4 | 10.9, 64 rows 12.2 | 9.6 | 7.8, fp32 128 rows 16.4 | 14.1 | 18.7, 33 rows 14.7 | 11.0 | 9.1; RMSNorm bf16 128 rows 8.6 | 7.7 |
+        // 10.4, fp32 11.8 | 12.5 | 16.5, 33 rows 10.6 | 9.1 | 7.6.  Rows of 9001 to 16001 columns gain 0 to 1 us.
+        const char *x0 = reinterpret_cast<const char*>(xp), *y0 = reinterpret_cast<const char*>(yp);
+        const int64_t bytes = rows * cols * (int64_t)sizeof(T);
+        const bool apart = x0 + bytes <= y0 || y0 + bytes <= x0;
+        const int share = !apart ? 1 : rows <= 64 ? 4 : rows <= 128 && (OP == kLayerNorm || (OP == kRmsNorm && sizeof(T) == 2)) ? 2 : 1;
         if (nvec <= 64) MHIP_ROW_ANY(64, 1);
         else if (nvec <= 128) MHIP_ROW_ANY(64, 2);
         else if (nvec <= 256) MHIP_ROW_ANY(256, 1);
         else if (nvec <= 512) MHIP_ROW_ANY(256, 2);
         else if (nvec <= 1024) MHIP_ROW_ANY(256, 4);
+        else if (nvec <= 2048 && share >= 2) MHIP_ROW_SHARED(1024, 2, 2);
+        else if (nvec <= 4096 && share >= 4) MHIP_ROW_SHARED(1024, 4, 4);
+        else if (nvec <= 4096 && share >= 2) MHIP_ROW_SHARED(1024, 4, 2);
+        else if (nvec <= 8192 && share >= 4) MHIP_ROW_SHARED(1024, 8, 4);
+        else if (nvec <= 8192 && share >= 2) MHIP_ROW_SHARED(1024, 8, 2);
+        else if (nvec > 8192 && share >= 4) MHIP_ROW_SHARED(1024, 16, 4);
+        else if (nvec > 8192 && share >= 2) MHIP_ROW_SHARED(1024, 16, 2);
         else if (nvec <= 2048) MHIP_ROW_ANY(1024, 2);
         else if (nvec <= 4096) MHIP_ROW_ANY(1024, 4);
         else if (nvec <= 8192) MHIP_ROW_ANY(1024, 8);
         else MHIP_ROW_ANY(1024, 16);
 #undef MHIP_ROW_ANY
+#undef MHIP_ROW_SHARED
     } else {
         hipLaunchKernelGGL((row_block_kernel<T, OP>), dim3((unsigned)rows), dim3(256), 0, s, xp,
                            gp, bp, yp, cols, eps);
