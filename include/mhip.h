@@ -189,6 +189,15 @@ int mhip_gemm_sums(void* stream, const void* a, const void* b, float* sums, int6
 int mhip_finish_norm(void* stream, const float* sums, int parts, const float* bias, const void* residual, void* c,
                      const float* gamma, const float* beta, float eps, void* h, int64_t M, int64_t N, int dtype);
 
+/* c = act(n(x) . round(w) + round(bias)) (+ residual) as mhip_linear_w32 computes it, w stored [K, N]; n(x) is x, or with `gamma` (beta may be
+ * NULL) LayerNorm(x) rounded to x's type (K up to 768: mhip_linear_w32_norm_ok).  Without gamma a long K is split over the device where
+ * the workspace (mhip_linear_w32_workspace bytes, 0: of no use; overwritten) allows, and the last workgroup adds the parts up. */
+int mhip_linear_w32_norm_ok(int64_t M, int64_t N, int64_t K, int dtype);
+int64_t mhip_linear_w32_workspace(int64_t M, int64_t N, int64_t K);
+int mhip_linear_w32_layer(void* stream, const void* x, const float* gamma, const float* beta, float eps, const float* w, const float* bias,
+                          const void* residual, void* c, int64_t M, int64_t N, int64_t K, int activation, int dtype, void* workspace,
+                          int64_t workspace_bytes, int n_ahead, const mhip_weights* ahead);
+
 /* Attention -------------------------------------------------------------- */
 
 /* O = softmax(scale * Q K^T + mask, causal) V.

@@ -16,6 +16,7 @@
 // Workgroups of one XCD take neighbouring strips, so a 128-byte line of W that two strips share is fetched once.
 #include <initializer_list>
 
+#include "arrive.h"
 #include "gemm_lds.h"
 
 namespace mhip {
@@ -27,13 +28,14 @@ struct Band { const float* w; int N, K, cols, wgs; uint32_t magic; };      // co
 
 struct LinearArgs {
     const void* x;
-    const float *gamma, *beta;        // finish_norm_kernel only; beta may be NULL
+    const float *gamma, *beta;        // finish_norm_kernel, and a product that normalises the rows of x; beta may be NULL
     float eps;
     const float* w;
     const float* bias;                // may be NULL
     const void* residual;             // may be NULL
     void* c;
     float* sums;                      // instead of c: fp32 sums [splits][M][N]
+    uint64_t *words, tag;             // with sums: the last part to arrive adds them up to c (arrive.h)
     int M, N, K, act, splits;
     int strips, per_xcd, blocks, first;      // first: workgroups in front of the product's
     Band ahead[kAhead];
@@ -62,10 +64,14 @@ __device__ __forceinline__ void fetch_ahead(const LinearArgs& g, int id) {
 }
 
 // A strip of 16 columns.  TB: W stored [N, K].  MT = groups of 16 rows, U = steps of 32 k that a wave holds at once; LOOP: it has
-// more of them and loads a block ahead.
-template <typename T, bool TB, bool LOOP, int MT, int U>
+// more of them and loads a block ahead.  FORM kArrive: the last part of K to arrive adds the parts up.  kNorm: the rows of x are normalised first, LayerNorm(x) rounded to T, which a workgroup with
+// all of K holds anyway: two barriers here instead of a launch (finish_norm_kernel 3.8 us; GPT-2-small's two norms a layer cost 0.7 each).
+enum Form { kPlain = 0, kNorm = 1, kArrive = 2 };
+template <typename T, bool TB, bool LOOP, int FORM, int MT, int U>
 __global__ __launch_bounds__(64 * kWaves, LOOP ? 2 : 4) void linear_w32_kernel(LinearArgs g) {
     constexpr int KS = 32;
+    constexpr bool NORM = FORM == kNorm, ARRIVE = FORM == kArrive;
+    static_assert(!NORM || (!TB && !LOOP), "all of K in the workgroup");
     extern __shared__ __attribute__((aligned(16))) char smem[];
     if ((int)blockIdx.x < g.first) {
         fetch_ahead(g, blockIdx.x);
@@ -85,6 +91,15 @@ __global__ __launch_bounds__(64 * kWaves, LOOP ? 2 : 4) void linear_w32_kernel(L
     // ---- this wave's share of the k steps
     const int all = (g.K + KS - 1) / KS, part_steps = (all + g.splits - 1) / g.splits, p0 = split * part_steps, p1 = min(all, p0 + part_steps);
     const int per = (part_steps + kWaves - 1) / kWaves, s0 = p0 + wave * per, s1 = min(p1, s0 + per);
+    uint64_t* const word = ARRIVE ? g.words + strip * g.blocks + m0 / (16 * MT) : nullptr;
+    uint64_t seen = 0;
+    if (ARRIVE && threadIdx.x == 0) seen = arrive_look(word);
+    f32x4 ga = {0.f, 0.f, 0.f, 0.f}, be = ga;
+    const int gn = threadIdx.x * 4;
+    if (NORM && gn < g.K) {
+        ga = *reinterpret_cast<const f32x4*>(g.gamma + gn);
+        if (g.beta) be = *reinterpret_cast<const f32x4*>(g.beta + gn);
+    }
     struct Block {
         f32x4 wt[TB ? U : 1][2];                             // W stored [N, K]: eight k of a column
         float wn[TB ? 1 : U][TB ? 1 : 8];                    // W stored [K, N]: the same, one by one
@@ -128,6 +143,83 @@ __global__ __launch_bounds__(64 * kWaves, LOOP ? 2 : 4) void linear_w32_kernel(L
         if (g.residual) res = *reinterpret_cast<const u32x2*>(static_cast<const T*>(g.residual) + (int64_t)fm * g.N + column);
     }
 
+    if constexpr (NORM) {
+        constexpr int kMostK = kWaves * U * KS;
+        float* const stat = reinterpret_cast<float*>(smem);              // [2][wave][row]
+        float* const gb = stat + 2 * kWaves * MT * 16;                   // gamma, beta
+        if (gn < g.K) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) { gb[gn + e] = rounded<T>(ga[e]); gb[kMostK + gn + e] = rounded<T>(be[e]); }
+        }
+        typedef T vec8 __attribute__((ext_vector_type(8)));
+        auto over_row = [&](float(&v)[MT], int set) __attribute__((always_inline)) {
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+                v[mt] += __shfl_xor(v[mt], 16, 64);
+                v[mt] += __shfl_xor(v[mt], 32, 64);
+                if (lg == 0) stat[(set * kWaves + wave) * MT * 16 + mt * 16 + li] = v[mt];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+                v[mt] = 0.f;
+#pragma unroll
+                for (int w = 0; w < kWaves; w++) v[mt] += stat[(set * kWaves + w) * MT * 16 + mt * 16 + li];
+                v[mt] = v[mt] / (float)g.K;                              // (a quotient: a row of equal elements has that mean and no variance)
+            }
+            // (from here on the operand as 16-bit values only: kept as the fp32 values of this pass they would be spilled)
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) asm("" : "+v"(cur.a[u][mt][e]));
+        };
+        float mean[MT], var[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            mean[mt] = 0.f;
+#pragma unroll
+            for (int u = 0; u < U; u++) {                                // (what is not there reads zero)
+                const vec8 v = __builtin_bit_cast(vec8, cur.a[u][mt]);
+#pragma unroll
+                for (int e = 0; e < 8; e++) mean[mt] += (float)v[e];
+            }
+        }
+        over_row(mean, 0);
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            var[mt] = 0.f;
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const vec8 v = __builtin_bit_cast(vec8, cur.a[u][mt]);
+                if (s0 + u < s1 && (s0 + u) * KS + lg * 8 < g.K)
+#pragma unroll
+                    for (int e = 0; e < 8; e++) { const float t = (float)v[e] - mean[mt]; var[mt] = fmaf(t, t, var[mt]); }
+            }
+        }
+        over_row(var, 1);
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) var[mt] = 1.f / sqrtf(var[mt] + g.eps);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int k = (s0 + u) * KS + lg * 8;
+            if (s0 + u >= s1 || k >= g.K) continue;
+            const f32x4 *gs = reinterpret_cast<const f32x4*>(gb + k), *bs = reinterpret_cast<const f32x4*>(gb + kMostK + k);
+            const f32x4 g2[2] = {gs[0], gs[1]}, b2[2] = {bs[0], bs[1]};
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+                const vec8 v = __builtin_bit_cast(vec8, cur.a[u][mt]);
+                float o[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) o[e] = fmaf(((float)v[e] - mean[mt]) * var[mt], g2[e / 4][e % 4], b2[e / 4][e % 4]);
+#pragma unroll
+                for (int e = 0; e < 4; e++) cur.a[u][mt][e] = round_pair<T>(o[2 * e], o[2 * e + 1]);
+            }
+        }
+        __syncthreads();                                                 // the sums below go where this has been read
+    }
+
     f32x4 acc[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -152,6 +244,7 @@ __global__ __launch_bounds__(64 * kWaves, LOOP ? 2 : 4) void linear_w32_kernel(L
             if (s + U < s1) cur = nxt;
         }
     } else multiply(cur, s0);
+    if (ARRIVE && threadIdx.x == 0) arrive_claim(word, seen, g.tag);
 
     // ---- the waves' partial sums, in the accumulators' own layout: lane (li, lg) holds row 16 mt + li and, in its four
     // registers, columns 4 lg .. 4 lg + 3
@@ -159,12 +252,25 @@ __global__ __launch_bounds__(64 * kWaves, LOOP ? 2 : 4) void linear_w32_kernel(L
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) part[(wave * MT + mt) * 64 + lane] = acc[mt];
     __syncthreads();
-    if (wave >= MT) return;
-    f32x4 sum = part[wave * 64 + lane];
+    if (!ARRIVE && wave >= MT) return;
+    f32x4 sum = part[(ARRIVE ? min(wave, MT - 1) : wave) * 64 + lane];
 #pragma unroll
-    for (int w = 1; w < kWaves; w++) sum += part[(w * MT + wave) * 64 + lane];
-    if (!finisher || column >= g.N) return;
-    if (g.sums) {
+    for (int w = 1; w < kWaves; w++) sum += part[(w * MT + (ARRIVE ? min(wave, MT - 1) : wave)) * 64 + lane];
+    const bool mine = finisher && column < g.N;
+    if constexpr (ARRIVE) {
+        __shared__ int last;
+        const __amdgpu_buffer_rsrc_t rp = parts_rsrc(g.sums);
+        if (mine) store_part(rp, (uint32_t)(((split * g.M + fm) * g.N + column) * 4), sum);
+        if (!arrive_last(word, g.splits, &last) || !mine) return;
+        f32x4 v[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = load_part(rp, i < g.splits ? (uint32_t)(((i * g.M + fm) * g.N + column) * 4) : kOob);
+        sum = v[0];
+#pragma unroll
+        for (int i = 1; i < 8; i++) sum += v[i];
+    }
+    if (!mine) return;
+    if (!ARRIVE && g.sums) {
         *reinterpret_cast<f32x4*>(g.sums + ((int64_t)split * g.M + fm) * g.N + column) = sum;
         return;
     }
@@ -343,11 +449,11 @@ __global__ __launch_bounds__(256) void finish_norm_kernel(LinearArgs g, T* h) {
     }
 }
 
-template <typename T, bool TB, bool LOOP, int MT, int U>
+template <typename T, bool TB, bool LOOP, int FORM, int MT, int U>
 int launch_one(hipStream_t s, LinearArgs g) {
-    auto kern = linear_w32_kernel<T, TB, LOOP, MT, U>;
-    constexpr int kSums = kWaves * MT * 1024;
-    static_assert(kSums <= 64 * 1024, "more LDS than a launch gets unasked");
+    auto kern = linear_w32_kernel<T, TB, LOOP, FORM, MT, U>;
+    constexpr int kShares = kWaves * MT * 1024, kStats = FORM == kNorm ? 2 * kWaves * MT * 64 + 2 * kWaves * U * 32 * 4 : 0, kSums = kShares > kStats ? kShares : kStats;
+    static_assert(kSums < 64 * 1024, "more LDS than a launch gets unasked");
     g.blocks = (g.M + 16 * MT - 1) / (16 * MT);
     g.strips = (g.N + 15) / 16;
     g.per_xcd = (g.strips + kXcds - 1) / kXcds;
@@ -375,8 +481,12 @@ int launch_rows(hipStream_t s, const LinearArgs& g, bool tb) {
         hipLaunchKernelGGL((linear_w32_stream_kernel<T, MT, 3>), dim3((unsigned)(t.strips < room ? t.strips : room), (unsigned)blocks), dim3(64 * kWaves), 0, s, t);
         return check_launch("linear_w32_stream");
     }
-    if (tb) return launch_one<T, true, true, MT, 3>(s, g);
-    return loop ? launch_one<T, false, true, MT, 3>(s, g) : launch_one<T, false, false, MT, 3>(s, g);
+    if (tb) return launch_one<T, true, true, kPlain, MT, 3>(s, g);
+    if constexpr (MT <= 2) {
+        if (g.gamma) return launch_one<T, false, false, kNorm, MT, 3>(s, g);
+        if (g.words) return loop ? launch_one<T, false, true, kArrive, MT, 3>(s, g) : launch_one<T, false, false, kArrive, MT, 3>(s, g);
+    }
+    return loop ? launch_one<T, false, true, kPlain, MT, 3>(s, g) : launch_one<T, false, false, kPlain, MT, 3>(s, g);
 }
 
 template <typename T>
@@ -416,27 +526,63 @@ extern "C" int mhip_linear_w32_parts(int64_t M, int64_t N, int64_t K) {
     return n < 2 ? 1 : n > 8 ? 8 : (int)n;
 }
 
-extern "C" int mhip_linear_w32(void* stream, const void* x, const float* w, const float* bias, const void* residual, void* c, int64_t M,
-                               int64_t N, int64_t K, int trans_b, int activation, int dtype, float* sums, int parts, int n_ahead,
-                               const mhip_weights* ahead) {
+namespace mhip {
+namespace {
+int linear_entry(void* stream, const void* x, const float* w, const float* bias, const void* residual, void* c, int64_t M, int64_t N, int64_t K, int trans_b,
+                 int activation, int dtype, const float* gamma, const float* beta, float eps, float* sums, uint64_t* words, int parts, int n_ahead,
+                 const mhip_weights* ahead) {
     if (activation < MHIP_ACT_NONE || activation > MHIP_ACT_GELU_ERF)
         return fail(MHIP_ERR_INVALID_ARGUMENT, "mhip_linear_w32: unknown activation %d", activation);
     if (!x || !w || (!c && !sums)) return fail(MHIP_ERR_INVALID_ARGUMENT, "mhip_linear_w32: NULL matrix pointer");
-    if (sums ? (parts < 1 || parts > 8 || c || bias || residual || activation != MHIP_ACT_NONE) : parts != 1)
+    if (sums && !words ? (parts < 1 || parts > 8 || c || bias || residual || activation != MHIP_ACT_NONE) : !words && parts != 1)
         return fail(MHIP_ERR_INVALID_ARGUMENT, "mhip_linear_w32: parts of K come as plain sums, eight at most");
     if (!mhip_linear_w32_ok(M, N, K, dtype))
         return fail(MHIP_ERR_UNSUPPORTED, "mhip_linear_w32: [%lld,%lld] x K %lld, dtype %d is not served", (long long)M, (long long)N, (long long)K, dtype);
-    if (!aligned16({x, w, bias, residual, c, sums})) return fail(MHIP_ERR_UNSUPPORTED, "mhip_linear_w32: tensors must be 16-byte aligned");
+    if (!aligned16({x, w, bias, residual, c, sums, gamma, beta})) return fail(MHIP_ERR_UNSUPPORTED, "mhip_linear_w32: tensors must be 16-byte aligned");
     if (n_ahead < 0 || n_ahead > kAhead || (n_ahead > 0 && !ahead)) return fail(MHIP_ERR_INVALID_ARGUMENT, "mhip_linear_w32: up to %d matrices ahead", kAhead);
     LinearArgs g = {};
     g.x = x; g.w = w; g.bias = bias; g.residual = residual; g.c = c; g.sums = sums;
     g.M = (int)M; g.N = (int)N; g.K = (int)K; g.act = activation; g.splits = parts;
+    g.gamma = gamma; g.beta = beta; g.eps = eps; g.words = words; g.tag = words ? launch_tag() : 0;
     for (int i = 0; i < n_ahead; i++)
         if (ahead[i].w && ahead[i].N > 0 && ahead[i].K > 0 && ahead[i].N % 8 == 0 && ahead[i].N <= (1 << 16) && ahead[i].K <= (1 << 16) &&
             ahead[i].N * ahead[i].K <= (1 << 23) && aligned16({ahead[i].w})) {
             g.ahead[i].w = ahead[i].w; g.ahead[i].N = (int)ahead[i].N; g.ahead[i].K = (int)ahead[i].K;
         }
     return dtype == MHIP_BF16 ? launch_type<bf16_t>(as_stream(stream), g, trans_b != 0) : launch_type<f16_t>(as_stream(stream), g, trans_b != 0);
+}
+
+int64_t part_bytes(int64_t M, int64_t N, int parts) { return (parts * M * N * 4 + 255) / 256 * 256; }
+}  // namespace
+}  // namespace mhip
+
+extern "C" int mhip_linear_w32(void* stream, const void* x, const float* w, const float* bias, const void* residual, void* c, int64_t M,
+                               int64_t N, int64_t K, int trans_b, int activation, int dtype, float* sums, int parts, int n_ahead,
+                               const mhip_weights* ahead) {
+    return linear_entry(stream, x, w, bias, residual, c, M, N, K, trans_b, activation, dtype, nullptr, nullptr, 0.f, sums, nullptr, parts, n_ahead, ahead);
+}
+
+// Up to 32 rows: every workgroup normalises all of them, 10 operations an element, 0.7 us for 16 rows and 2.3 for 48.
+extern "C" int mhip_linear_w32_norm_ok(int64_t M, int64_t N, int64_t K, int dtype) { return mhip_linear_w32_ok(M, N, K, dtype) && M <= 32 && K <= kWaves * 3 * 32; }
+
+extern "C" int64_t mhip_linear_w32_workspace(int64_t M, int64_t N, int64_t K) {
+    const int parts = mhip_linear_w32_parts(M, N, K);
+    return parts == 1 || M < 1 || M > 32 ? 0 : part_bytes(M, N, parts) + (N + 15) / 16 * ((M + 63) / 64) * 8;
+}
+
+extern "C" int mhip_linear_w32_layer(void* stream, const void* x, const float* gamma, const float* beta, float eps, const float* w, const float* bias,
+                                     const void* residual, void* c, int64_t M, int64_t N, int64_t K, int activation, int dtype, void* workspace,
+                                     int64_t workspace_bytes, int n_ahead, const mhip_weights* ahead) {
+    if (!c) return fail(MHIP_ERR_INVALID_ARGUMENT, "mhip_linear_w32_layer: NULL result");
+    if (gamma && !mhip_linear_w32_norm_ok(M, N, K, dtype))
+        return fail(MHIP_ERR_UNSUPPORTED, "mhip_linear_w32_layer: rows of %lld are not normalised", (long long)K);
+    // (normalised rows need all of K in a workgroup)
+    const int64_t need = mhip_linear_w32_workspace(M, N, K);
+    const bool split = !gamma && need > 0 && workspace && workspace_bytes >= need;
+    const int parts = split ? mhip_linear_w32_parts(M, N, K) : 1;
+    char* ws = static_cast<char*>(workspace);
+    return linear_entry(stream, x, w, bias, residual, c, M, N, K, 0, activation, dtype, gamma, beta, eps, split ? reinterpret_cast<float*>(ws) : nullptr,
+                        split ? reinterpret_cast<uint64_t*>(ws + part_bytes(M, N, parts)) : nullptr, parts, n_ahead, ahead);
 }
 
 extern "C" int mhip_finish_norm(void* stream, const float* sums, int parts, const float* bias, const void* residual, void* c,

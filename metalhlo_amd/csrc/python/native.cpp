@@ -308,6 +308,43 @@ FUNCTION(matmul_sums) {
     });
 }
 
+// linear_layer(x, norm or None = (gamma, beta, eps), weight, bias, residual, activation code, (weights ahead))
+FUNCTION(linear_layer) {
+    return guarded(n, 7, [&] {
+        const at::Tensor &x = dense(arg[0]), &w = dense(arg[2]);
+        const at::Tensor *bias = optional_dense(arg[3]), *res = optional_dense(arg[4]), *gamma = nullptr, *beta = nullptr;
+        float eps = 0.f;
+        if (arg[1] != Py_None) {
+            if (!PyTuple_Check(arg[1]) || PyTuple_GET_SIZE(arg[1]) != 3) raise(PyExc_ValueError, "norm must be (gamma, beta, eps)");
+            gamma = &dense(PyTuple_GET_ITEM(arg[1], 0));
+            beta = optional_dense(PyTuple_GET_ITEM(arg[1], 1));
+            eps = (float)number(PyTuple_GET_ITEM(arg[1], 2));
+        }
+        if (x.dim() != 2 || w.dim() != 2 || w.size(0) != x.size(1)) raise(PyExc_ValueError, "linear_layer needs matrices [M, K] and [K, N]");
+        const int64_t M = x.size(0), K = x.size(1), N = w.size(1);
+        for (const at::Tensor* p : {&w, bias, gamma, beta})
+            if (p && p->scalar_type() != at::kFloat) raise(PyExc_TypeError, "parameters must be fp32");
+        if (bias && bias->numel() != N) raise(PyExc_ValueError, "bias must be [N]");
+        if ((gamma && gamma->numel() != K) || (beta && beta->numel() != K)) raise(PyExc_ValueError, "gamma and beta must be [K]");
+        if (res && (res->numel() != M * N || res->scalar_type() != x.scalar_type())) raise(PyExc_ValueError, "residual must have the result's size and dtype");
+        const int dt = dtype_code(x.scalar_type()), act = (int)integer(arg[5]);
+        at::Tensor c = empty({M, N}, x.scalar_type(), x), work;
+        const int64_t bytes = gamma ? 0 : mhip_linear_w32_workspace(M, N, K);
+        if (bytes > 0) work = empty({bytes}, at::kByte, x);
+        mhip_weights ahead[2] = {};
+        int n_ahead = 0;
+        if (!PyTuple_Check(arg[6]) || PyTuple_GET_SIZE(arg[6]) > 2) raise(PyExc_ValueError, "ahead must be a tuple of up to two matrices");
+        for (; n_ahead < PyTuple_GET_SIZE(arg[6]); n_ahead++) {
+            const at::Tensor* t = &dense(PyTuple_GET_ITEM(arg[6], n_ahead));
+            if (t->dim() != 2 || t->scalar_type() != at::kFloat) raise(PyExc_TypeError, "weights ahead must be fp32 matrices");
+            ahead[n_ahead] = {t->data_ptr<float>(), t->size(1), t->size(0)};
+        }
+        check([&] { return mhip_linear_w32_layer(stream_of(x), x.data_ptr(), f32(gamma), f32(beta), eps, f32(&w), f32(bias), ptr(res), c.data_ptr(), M, N, K, act, dt,
+                                                 bytes > 0 ? work.data_ptr() : nullptr, bytes, n_ahead, ahead); });
+        return THPVariable_Wrap(std::move(c));
+    });
+}
+
 // finish_norm(sums or None, bias, residual, gamma, beta, eps) -> (c, LayerNorm(c)); without sums c is the residual
 FUNCTION(finish_norm) {
     return guarded(n, 6, [&]() -> PyObject* {
@@ -424,7 +461,7 @@ FUNCTION(bind) {
 }
 
 #define ENTRY(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
-PyMethodDef kMethods[] = {ENTRY(softmax), ENTRY(layer_norm), ENTRY(rms_norm), ENTRY(bias_gelu), ENTRY(matmul), ENTRY(linear), ENTRY(matmul_sums), ENTRY(tied_head), ENTRY(finish_norm), ENTRY(causal_attention),
+PyMethodDef kMethods[] = {ENTRY(softmax), ENTRY(layer_norm), ENTRY(rms_norm), ENTRY(bias_gelu), ENTRY(matmul), ENTRY(linear), ENTRY(linear_layer), ENTRY(matmul_sums), ENTRY(tied_head), ENTRY(finish_norm), ENTRY(causal_attention),
                           ENTRY(flash_attention), ENTRY(argmax), ENTRY(bind), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

@@ -180,6 +180,15 @@ class GPT2:
         o_parts, p_parts = (kernels.linear_parts(T, cfg.d_model, k) for k in (cfg.d_model, cfg.d_ff))
         norms = [(l["ln1_g"], l["ln1_b"], 1e-5) for l in layers] + [(p["lnf_g"], p["lnf_b"], 1e-5)]
         x = kernels.embed_tokens(ids, p["wte"], p["wpe"], self.dtype).reshape(T, cfg.d_model)
+        if kernels.linear_norm_served(T, cfg.d_model, cfg.d_model, self.dtype):
+            layer = kernels.linear_layer
+            for i, l in enumerate(layers):
+                qkv = layer(x, l["w_qkv"], l["b_qkv"], norm=norms[i], ahead=(l["w_o"], l["w_fc"]))
+                a = kernels.causal_attention(qkv, B, cfg.n_head)
+                x = layer(a, l["w_o"], l["b_o"], residual=x, ahead=(l["w_proj"],))
+                u = layer(x, l["w_fc"], l["b_fc"], "gelu", norm=(l["ln2_g"], l["ln2_b"], 1e-5))
+                x = layer(u, l["w_proj"], l["b_proj"], residual=x, ahead=(layers[i + 1]["w_qkv"],) if i + 1 < len(layers) else ())
+            return self._head(kernels.finish_norm(None, None, x, norms[-1])[1], B, S)
         x, h = kernels.finish_norm(None, None, x, norms[0])
         for i, l in enumerate(layers):
             qkv = linear(h, l["w_qkv"], l["b_qkv"], ahead=(l["w_o"], l["w_fc"]))
@@ -189,11 +198,16 @@ class GPT2:
             u = linear(h, l["w_fc"], l["b_fc"], "gelu")
             sums = linear(u, l["w_proj"], parts=p_parts, ahead=(layers[i + 1]["w_qkv"],) if i + 1 < len(layers) else ())
             x, h = kernels.finish_norm(sums, l["b_proj"], x, norms[i + 1])
+        return self._head(h, B, S)
+
+    def _head(self, h: torch.Tensor, B: int, S: int) -> torch.Tensor:
+        """Logits of a short prompt from the fp32 table."""
+        cfg, p, T = self.cfg, self.p32, B * S
         # (us, strips that walk the device against x that stays: 64 tokens 36.9 and 38.5, 65 48.5 and 39.2, 128 53.5 and 45.1)
         if T > 64 and kernels.tied_head_served(T, self.vocab_pad, cfg.d_model, self.dtype):
             logits = kernels.tied_head(h, p["wte_pad"])
         else:
-            logits = linear(h, p["wte_pad"], trans_b=True)
+            logits = kernels.linear(h, p["wte_pad"], trans_b=True)
         return logits.reshape(B, S, self.vocab_pad)[..., :cfg.vocab]
 
     def capture(self, ids: torch.Tensor) -> "GraphedForward":

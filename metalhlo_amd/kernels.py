@@ -119,6 +119,16 @@ def linear_parts(M: int, N: int, K: int) -> int:
     return _lib.load().mhip_linear_w32_parts(M, N, K)
 
 
+def linear_layer(x, weight, bias=None, activation: str = "none", residual=None, norm=None, ahead=()):
+    """`linear` with weight [K, N], of LayerNorm(x) where `norm` is (gamma, beta, eps) in fp32; a long K without it is split over the device and
+    added up in the same launch.  `linear_norm_served` says which rows are normalised."""
+    return (_native or _host()).linear_layer(x, norm, weight, bias, residual, ACTIVATION_CODE[activation], ahead)
+
+
+def linear_norm_served(M: int, N: int, K: int, dtype) -> bool:
+    return bool(_lib.load().mhip_linear_w32_norm_ok(M, N, K, DTYPE_CODE[dtype]))
+
+
 def tied_head(x, weight):
     """x [M, K] @ weight [N, K].T in x's 16-bit type, the fp32 weight rounded to it at use; `tied_head_served` says for which sizes."""
     return (_native or _host()).tied_head(x, weight)
