@@ -14,7 +14,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 ROOT = os.path.dirname(HERE)
 
-HIP_SOURCES = ["runtime.hip", "row_kernels.hip", "gemm.hip", "gemm_skinny.hip", "gemm_strip.hip", "linear_w32.hip", "tied_head.hip", "gemm_mid.hip", "gemm_any.hip", "gemm_f32.hip", "gemm256.hip", "gemm_twoset.hip", "tuning.hip", "attention.hip", "attention_flow.hip", "attention_pipe.hip", "attention_decode.hip", "attention_f32.hip", "glue_kernels.hip", "elementwise.hip", "fused_misc.hip"]
+HIP_SOURCES = ["runtime.hip", "row_kernels.hip", "gemm.hip", "gemm_skinny.hip", "gemm_strip.hip", "linear_w32.hip", "tied_head.hip", "gemm_mid.hip", "gemm_any.hip", "gemm_f32.hip", "gemm256.hip", "gemm_twoset.hip", "tuning.hip", "attention.hip", "attention_flow.hip", "attention_short.hip", "attention_pipe.hip", "attention_decode.hip", "attention_f32.hip", "glue_kernels.hip", "elementwise.hip", "fused_misc.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=fast",

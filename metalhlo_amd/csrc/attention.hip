@@ -498,6 +498,9 @@ int launch_fa_decode(hipStream_t s, const FaArgs& a, int64_t D, int dtype, void*
 // attention_flow.hip: head sizes 64 and 128 without a mask, few tiles.
 bool fa_flow_wanted(const FaArgs& a, int64_t D);
 int launch_fa_flow(hipStream_t s, FaArgs a, int64_t D, int dtype);
+// attention_short.hip: few keys.
+bool fa_short_wanted(const FaArgs& a);
+int launch_fa_short(hipStream_t s, const FaArgs& a, int64_t D, int dtype);
 // attention_f32.hip: fp32 tensors on the fp32 matrix instruction.
 bool fa_f32_mfma_eligible(const FaArgs& a, int64_t D, bool packed);
 int launch_fa_f32_mfma(hipStream_t s, const FaArgs& a, int64_t D, float scale, bool packed);
@@ -557,6 +560,7 @@ static int fa_entry(const char* name, void* stream, const void* q, const void* k
         // 0 = no tuned choice; 1 = 128-row kernel; 2 / 3 = 256-row pipelined kernel, causal tiles unpaired / paired
         const int variant = is_packed ? tuned_attention_variant(dtype, B * H, Sq, Skv, D, is_causal != 0) : 0;
         if (variant == 0 && fa_decode_eligible(a) && B * H <= 0x7FFFFFFF) return launch_fa_decode(s, a, D, dtype, workspace, workspace_bytes);
+        if (variant == 0 && !hm && fa_short_wanted(a)) return launch_fa_short(s, a, D, dtype);
         if (is_packed && fa_pipe_eligible(a, D, dtype, hm, variant))
             return launch_fa_pipe(s, a, dtype, is_causal != 0, variant == 2 ? 0 : variant == 3 ? 1 : -1);
         if (!hm && fa_flow_wanted(a, D)) return launch_fa_flow(s, a, D, dtype);
