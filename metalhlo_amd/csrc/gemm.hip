@@ -183,7 +183,9 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(GemmArgs g) {
         __syncthreads();
     }
 
-    store_tile<T, TM, TN>(g, acc, smem + wave * (WTM * (WTN * 2 + 16)), m0 + wm * WTM, n0 + wn * WTN, batch, lane);
+    TileBias<T, TN> bias;
+    bias.load(g, n0 + wn * WTN, lane);
+    store_tile<T, TM, TN>(g, acc, bias, smem + wave * (WTM * (WTN * 2 + 16)), m0 + wm * WTM, n0 + wn * WTN, batch, lane);
 }
 
 // ---------------------------------------------------------------------------

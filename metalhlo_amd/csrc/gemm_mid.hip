@@ -95,6 +95,8 @@ __global__ __launch_bounds__(256 * KG) void gemm_mid_kernel(GemmArgs g) {
         lb.load(rb, st + kATile, wave, (kt * KG + group) * kBK, kend);
     };
 
+    TileBias<T, TN> bias;
+    if (!SUMS) bias.load(g, n0 + wn * WTN, lane);
     f32x16 acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; i++)
@@ -192,7 +194,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_mid_kernel(GemmArgs g) {
         }
         return;
     }
-    if constexpr (!SUMS) store_tile<T, TM, TN>(g, acc, smem + wave * (WTM * (WTN * 2 + 16)), m0 + wm * WTM, n0 + wn * WTN, batch, lane);
+    if constexpr (!SUMS) store_tile<T, TM, TN>(g, acc, bias, smem + wave * (WTM * (WTN * 2 + 16)), m0 + wm * WTM, n0 + wn * WTN, batch, lane);
 }
 
 // C from the splits' sums in the accumulators' own layout (tiles of BM x BN, WGM x 4 / WGM waves): a wave of
