@@ -121,6 +121,19 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, const f32x16 (&acc
     // 32x32 accumulator tile is held transposed: a lane owns row m = lrow and,
     // in register group q = r/4, the four consecutive columns 8q + 4*lhalf + r%4.
     const bool vec_store = (g.N % 8 == 0) && (((reinterpret_cast<uintptr_t>(c) | reinterpret_cast<uintptr_t>(res)) & 15) == 0);
+    // The residual's chunks in the order of the stores below, up to kAtOnce of them on their way while the tile is activated and staged (one
+    // behind the other, each between two stores that may alias it, they took a latency each: [1000,3000] x K 1000 22.7 -> 16.6 us).
+    constexpr int kCpr = WTN / 8;                    // 16-byte chunks per row
+    constexpr int kRowsPerPass = 64 / kCpr, kPasses = WTM / kRowsPerPass, kAtOnce = kPasses < 8 ? kPasses : 8;
+    static_assert(kPasses % kAtOnce == 0, "whole groups of chunks");
+    const int cc = lane % kCpr, rr = lane / kCpr;
+    u32x4 rv[kAtOnce];
+    auto load_residual = [&](int p0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < kAtOnce; p++)
+            rv[p] = *reinterpret_cast<const u32x4*>(res + (int64_t)min(row0 + (p0 + p) * kRowsPerPass + rr, g.M - 1) * g.N + min(col0 + cc * 8, g.N - 8));
+    };
+    if (res && vec_store) load_residual(0);
     // Stage the wave's sub-tile in LDS as rounded 16-bit rows (padded by 16 bytes
     // against bank conflicts); the rows then go out with lanes running along n, so
     // every store instruction writes whole contiguous row segments.
@@ -155,18 +168,19 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, const f32x16 (&acc
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     if (vec_store) {
-        constexpr int kCpr = WTN / 8;                // 16-byte chunks per row
-        constexpr int kRowsPerPass = 64 / kCpr;
-        const int cc = lane % kCpr, rr = lane / kCpr;
 #pragma unroll
-        for (int p = 0; p < WTM / kRowsPerPass; p++) {
-            const int ml = p * kRowsPerPass + rr;
-            const int m = row0 + ml;
-            const int n = col0 + cc * 8;
-            if (m < g.M && n < g.N) {
-                u32x4 w = *reinterpret_cast<const u32x4*>(stage + ml * kRowPad + cc * 16);
-                if (res) w = add_chunk<T>(w, *reinterpret_cast<const u32x4*>(res + (int64_t)m * g.N + n));
-                *reinterpret_cast<u32x4*>(c + (int64_t)m * g.N + n) = w;
+        for (int p0 = 0; p0 < kPasses; p0 += kAtOnce) {
+            if (p0 > 0 && res) load_residual(p0);
+#pragma unroll
+            for (int p = 0; p < kAtOnce; p++) {
+                const int ml = (p0 + p) * kRowsPerPass + rr;
+                const int m = row0 + ml;
+                const int n = col0 + cc * 8;
+                if (m < g.M && n < g.N) {
+                    u32x4 w = *reinterpret_cast<const u32x4*>(stage + ml * kRowPad + cc * 16);
+                    if (res) w = add_chunk<T>(w, rv[p]);
+                    *reinterpret_cast<u32x4*>(c + (int64_t)m * g.N + n) = w;
+                }
             }
         }
     } else {
