@@ -185,7 +185,8 @@ __global__ __launch_bounds__(WGM* WGN * 64) void gemm_mfma_kernel(GemmArgs g) {
 
     TileBias<T, TN> bias;
     bias.load(g, n0 + wn * WTN, lane);
-    store_tile<T, TM, TN>(g, acc, bias, smem + wave * (WTM * (WTN * 2 + 16)), m0 + wm * WTM, n0 + wn * WTN, batch, lane);
+    TileResidual<T, TM, TN> residual;
+    store_tile<T, TM, TN>(g, acc, bias, residual, false, smem + wave * (WTM * (WTN * 2 + 16)), m0 + wm * WTM, n0 + wn * WTN, batch, lane);
 }
 
 // ---------------------------------------------------------------------------

@@ -203,7 +203,8 @@ __global__ __launch_bounds__(256, 2) void gemm_any_kernel(GemmArgs g) {
     }
     TileBias<T, TM> bias;
     bias.load(g, n0 + wn * WT, lane);
-    store_tile<T, TM, TM>(g, acc, bias, smem + wave * (WT * (WT * 2 + 16)), m0 + wm * WT, n0 + wn * WT, batch, lane);
+    TileResidual<T, TM, TM> residual;
+    store_tile<T, TM, TM>(g, acc, bias, residual, false, smem + wave * (WT * (WT * 2 + 16)), m0 + wm * WT, n0 + wn * WT, batch, lane);
 }
 
 bool large_tiles(int64_t M, int64_t N, int64_t batch) {

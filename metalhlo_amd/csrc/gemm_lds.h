@@ -109,10 +109,30 @@ struct TileBias {
     }
 };
 
+// Chunks of 16 bytes of the residual of a wave's tile, in the order of store_tile's stores, kAtOnce of them on their way together (one behind the
+// other, each between two stores that may alias it, they took a latency each: [1000,3000] x K 1000 22.8 us, 18.6 asked for while
+// the tile is activated, 18.4 in front of the loop over K).
+template <typename T, int TM, int TN>
+struct TileResidual {
+    static constexpr int kCpr = 4 * TN, kRowsPerPass = 64 / kCpr, kPasses = 32 * TM / kRowsPerPass, kAtOnce = kPasses < 8 ? kPasses : 8;
+    static_assert(kPasses % kAtOnce == 0, "whole groups of chunks");
+    u32x4 v[kAtOnce];
+    // whether C's rows, and the residual's, are stored in 16-byte chunks
+    __device__ static bool chunks(const GemmArgs& g, const T* c, const T* res) {
+        return (g.N % 8 == 0) && (((reinterpret_cast<uintptr_t>(c) | reinterpret_cast<uintptr_t>(res)) & 15) == 0);
+    }
+    __device__ __forceinline__ void load(const GemmArgs& g, const T* res, int row0, int col0, int lane, int p0) {
+        const int cc = lane % kCpr, rr = lane / kCpr;
+#pragma unroll
+        for (int p = 0; p < kAtOnce; p++)
+            v[p] = *reinterpret_cast<const u32x4*>(res + (int64_t)min(row0 + (p0 + p) * kRowsPerPass + rr, g.M - 1) * g.N + min(col0 + cc * 8, g.N - 8));
+    }
+};
+
 // The wave's (32 TM) x (32 TN) sub-tile at (row0, col0) of C: bias, activation, rounding, residual, store.
 // `stage` is this wave's LDS area of 32 TM rows of 64 TN + 16 bytes.
 template <typename T, int TM, int TN>
-__device__ __forceinline__ void store_tile(const GemmArgs& g, const f32x16 (&acc)[TM][TN], const TileBias<T, TN>& bias, char* stage, int row0, int col0, int64_t batch, int lane) {
+__device__ __forceinline__ void store_tile(const GemmArgs& g, const f32x16 (&acc)[TM][TN], const TileBias<T, TN>& bias, TileResidual<T, TM, TN>& rv, bool have_residual, char* stage, int row0, int col0, int64_t batch, int lane) {
     constexpr int WTM = 32 * TM, WTN = 32 * TN;
     const int lrow = lane & 31, lhalf = lane >> 5;
     T* c = static_cast<T*>(g.c) + batch * g.sc;
@@ -120,20 +140,11 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, const f32x16 (&acc
     // Epilogue.  The MFMAs were issued as (B-fragment, A-fragment), so each
     // 32x32 accumulator tile is held transposed: a lane owns row m = lrow and,
     // in register group q = r/4, the four consecutive columns 8q + 4*lhalf + r%4.
-    const bool vec_store = (g.N % 8 == 0) && (((reinterpret_cast<uintptr_t>(c) | reinterpret_cast<uintptr_t>(res)) & 15) == 0);
-    // The residual's chunks in the order of the stores below, up to kAtOnce of them on their way while the tile is activated and staged (one
-    // behind the other, each between two stores that may alias it, they took a latency each: [1000,3000] x K 1000 22.7 -> 16.6 us).
-    constexpr int kCpr = WTN / 8;                    // 16-byte chunks per row
-    constexpr int kRowsPerPass = 64 / kCpr, kPasses = WTM / kRowsPerPass, kAtOnce = kPasses < 8 ? kPasses : 8;
-    static_assert(kPasses % kAtOnce == 0, "whole groups of chunks");
+    const bool vec_store = TileResidual<T, TM, TN>::chunks(g, c, res);
+    using Res = TileResidual<T, TM, TN>;
+    constexpr int kCpr = Res::kCpr, kRowsPerPass = Res::kRowsPerPass, kPasses = Res::kPasses, kAtOnce = Res::kAtOnce;
     const int cc = lane % kCpr, rr = lane / kCpr;
-    u32x4 rv[kAtOnce];
-    auto load_residual = [&](int p0) __attribute__((always_inline)) {
-#pragma unroll
-        for (int p = 0; p < kAtOnce; p++)
-            rv[p] = *reinterpret_cast<const u32x4*>(res + (int64_t)min(row0 + (p0 + p) * kRowsPerPass + rr, g.M - 1) * g.N + min(col0 + cc * 8, g.N - 8));
-    };
-    if (res && vec_store) load_residual(0);
+    if (!have_residual && res && vec_store) rv.load(g, res, row0, col0, lane, 0);
     // Stage the wave's sub-tile in LDS as rounded 16-bit rows (padded by 16 bytes
     // against bank conflicts); the rows then go out with lanes running along n, so
     // every store instruction writes whole contiguous row segments.
@@ -170,7 +181,7 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, const f32x16 (&acc
     if (vec_store) {
 #pragma unroll
         for (int p0 = 0; p0 < kPasses; p0 += kAtOnce) {
-            if (p0 > 0 && res) load_residual(p0);
+            if (p0 > 0 && res) rv.load(g, res, row0, col0, lane, p0);
 #pragma unroll
             for (int p = 0; p < kAtOnce; p++) {
                 const int ml = (p0 + p) * kRowsPerPass + rr;
@@ -178,7 +189,7 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, const f32x16 (&acc
                 const int n = col0 + cc * 8;
                 if (m < g.M && n < g.N) {
                     u32x4 w = *reinterpret_cast<const u32x4*>(stage + ml * kRowPad + cc * 16);
-                    if (res) w = add_chunk<T>(w, rv[p]);
+                    if (res) w = add_chunk<T>(w, rv.v[p]);
                     *reinterpret_cast<u32x4*>(c + (int64_t)m * g.N + n) = w;
                 }
             }

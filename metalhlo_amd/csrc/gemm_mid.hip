@@ -97,6 +97,10 @@ __global__ __launch_bounds__(256 * KG) void gemm_mid_kernel(GemmArgs g) {
 
     TileBias<T, TN> bias;
     if (!SUMS) bias.load(g, n0 + wn * WTN, lane);
+    TileResidual<T, TM, TN> residual;
+    const T* res = static_cast<const T*>(g.residual) + batch * g.sc;
+    const bool early = !SUMS && g.residual && !g.partial && residual.kPasses == residual.kAtOnce && residual.chunks(g, static_cast<const T*>(g.c) + batch * g.sc, res);
+    if (early) residual.load(g, res, m0 + wm * WTM, n0 + wn * WTN, lane, 0);
     f32x16 acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; i++)
@@ -194,7 +198,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_mid_kernel(GemmArgs g) {
         }
         return;
     }
-    if constexpr (!SUMS) store_tile<T, TM, TN>(g, acc, bias, smem + wave * (WTM * (WTN * 2 + 16)), m0 + wm * WTM, n0 + wn * WTN, batch, lane);
+    if constexpr (!SUMS) store_tile<T, TM, TN>(g, acc, bias, residual, early, smem + wave * (WTM * (WTN * 2 + 16)), m0 + wm * WTM, n0 + wn * WTN, batch, lane);
 }
 
 // C from the splits' sums in the accumulators' own layout (tiles of BM x BN, WGM x 4 / WGM waves): a wave of
