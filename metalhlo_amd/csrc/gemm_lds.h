@@ -55,6 +55,7 @@ __device__ __forceinline__ uint32_t round_pair(float lo, float hi) {
 }
 
 typedef u32x2 u32x2_any __attribute__((aligned(2)));
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
@@ -117,15 +118,11 @@ struct TileResidual {
     static constexpr int kCpr = 4 * TN, kRowsPerPass = 64 / kCpr, kPasses = 32 * TM / kRowsPerPass, kAtOnce = kPasses < 8 ? kPasses : 8;
     static_assert(kPasses % kAtOnce == 0, "whole groups of chunks");
     u32x4 v[kAtOnce];
-    // whether C's rows, and the residual's, are stored in 16-byte chunks
-    __device__ static bool chunks(const GemmArgs& g, const T* c, const T* res) {
-        return (g.N % 8 == 0) && (((reinterpret_cast<uintptr_t>(c) | reinterpret_cast<uintptr_t>(res)) & 15) == 0);
-    }
     __device__ __forceinline__ void load(const GemmArgs& g, const T* res, int row0, int col0, int lane, int p0) {
         const int cc = lane % kCpr, rr = lane / kCpr;
 #pragma unroll
         for (int p = 0; p < kAtOnce; p++)
-            v[p] = *reinterpret_cast<const u32x4*>(res + (int64_t)min(row0 + (p0 + p) * kRowsPerPass + rr, g.M - 1) * g.N + min(col0 + cc * 8, g.N - 8));
+            v[p] = *reinterpret_cast<const u32x4_any*>(res + (int64_t)min(row0 + (p0 + p) * kRowsPerPass + rr, g.M - 1) * g.N + min(col0 + cc * 8, g.N - 8));
     }
 };
 
@@ -140,11 +137,10 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, const f32x16 (&acc
     // Epilogue.  The MFMAs were issued as (B-fragment, A-fragment), so each
     // 32x32 accumulator tile is held transposed: a lane owns row m = lrow and,
     // in register group q = r/4, the four consecutive columns 8q + 4*lhalf + r%4.
-    const bool vec_store = TileResidual<T, TM, TN>::chunks(g, c, res);
     using Res = TileResidual<T, TM, TN>;
     constexpr int kCpr = Res::kCpr, kRowsPerPass = Res::kRowsPerPass, kPasses = Res::kPasses, kAtOnce = Res::kAtOnce;
     const int cc = lane % kCpr, rr = lane / kCpr;
-    if (!have_residual && res && vec_store) rv.load(g, res, row0, col0, lane, 0);
+    if (!have_residual && res && g.N >= 8) rv.load(g, res, row0, col0, lane, 0);
     // Stage the wave's sub-tile in LDS as rounded 16-bit rows (padded by 16 bytes
     // against bank conflicts); the rows then go out with lanes running along n, so
     // every store instruction writes whole contiguous row segments.
@@ -178,41 +174,27 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, const f32x16 (&acc
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (vec_store) {
+    // (rows of any alignment in chunks of 16 bytes, which global memory takes; what is left of a row, up to seven elements, one by one:
+    // element by element [5000,1001] x K 1000 with a residual 55.5 us, 30.4 so, [1500,1500] x K 1500 stored [N, K] 25.8, 24.7)
 #pragma unroll
-        for (int p0 = 0; p0 < kPasses; p0 += kAtOnce) {
-            if (p0 > 0 && res) rv.load(g, res, row0, col0, lane, p0);
+    for (int p0 = 0; p0 < kPasses; p0 += kAtOnce) {
+        if (p0 > 0 && res && g.N >= 8) rv.load(g, res, row0, col0, lane, p0);
 #pragma unroll
-            for (int p = 0; p < kAtOnce; p++) {
-                const int ml = (p0 + p) * kRowsPerPass + rr;
-                const int m = row0 + ml;
-                const int n = col0 + cc * 8;
-                if (m < g.M && n < g.N) {
-                    u32x4 w = *reinterpret_cast<const u32x4*>(stage + ml * kRowPad + cc * 16);
-                    if (res) w = add_chunk<T>(w, rv.v[p]);
-                    *reinterpret_cast<u32x4*>(c + (int64_t)m * g.N + n) = w;
-                }
-            }
-        }
-    } else {
-        // rows of C are not 16-byte aligned (odd N): one element per lane, 64
-        // consecutive columns per store instruction
-        const uint16_t* st16 = reinterpret_cast<const uint16_t*>(stage);
-        uint16_t* c16 = reinterpret_cast<uint16_t*>(c);
-constexpr int kLanes = WTN < 64 ? WTN : 64, kRowsAtOnce = 64 / kLanes;
-#pragma unroll 4
-        for (int mb = 0; mb < WTM; mb += kRowsAtOnce) {
-            const int ml = mb + lane / kLanes, m = row0 + ml;
-            if (m >= g.M) break;
+        for (int p = 0; p < kAtOnce; p++) {
+            const int ml = (p0 + p) * kRowsPerPass + rr;
+            const int m = row0 + ml, n = col0 + cc * 8;
+            if (m >= g.M || n >= g.N) continue;
+            u32x4 w = *reinterpret_cast<const u32x4*>(stage + ml * kRowPad + cc * 16);
+            T* to = c + (int64_t)m * g.N + n;
+            if (n + 8 <= g.N) {
+                if (res) w = add_chunk<T>(w, rv.v[p]);
+                *reinterpret_cast<u32x4_any*>(to) = w;
+            } else {
+                const Vec16<T> t = __builtin_bit_cast(Vec16<T>, w);
+                const T* from = res + (int64_t)m * g.N + n;
 #pragma unroll
-            for (int cb = 0; cb < WTN / kLanes; cb++) {
-                const int nl = cb * kLanes + lane % kLanes;
-                const int n = col0 + nl;
-                if (n < g.N) {
-                    T val = __builtin_bit_cast(T, st16[ml * (kRowPad / 2) + nl]);
-                    if (res) val = Elem<T>::from_f32(Elem<T>::to_f32(val) + Elem<T>::to_f32(res[(int64_t)m * g.N + n]));
-                    c16[(int64_t)m * g.N + n] = __builtin_bit_cast(uint16_t, val);
-                }
+                for (int e = 0; e < 7; e++)
+                    if (n + e < g.N) to[e] = res ? Elem<T>::from_f32(Elem<T>::to_f32(t.v[e]) + Elem<T>::to_f32(from[e])) : t.v[e];
             }
         }
     }

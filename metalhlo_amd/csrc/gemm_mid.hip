@@ -99,7 +99,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_mid_kernel(GemmArgs g) {
     if (!SUMS) bias.load(g, n0 + wn * WTN, lane);
     TileResidual<T, TM, TN> residual;
     const T* res = static_cast<const T*>(g.residual) + batch * g.sc;
-    const bool early = !SUMS && g.residual && !g.partial && residual.kPasses == residual.kAtOnce && residual.chunks(g, static_cast<const T*>(g.c) + batch * g.sc, res);
+    const bool early = !SUMS && g.residual && !g.partial && residual.kPasses == residual.kAtOnce && g.N >= 8;
     if (early) residual.load(g, res, m0 + wm * WTM, n0 + wn * WTN, lane, 0);
     f32x16 acc[TM][TN];
 #pragma unroll
