@@ -695,6 +695,12 @@ extern "C" int mhip_gemm_ws(void* stream, const void* a, const void* b, const vo
                       activation, dtype, workspace_bytes > 0 ? workspace : nullptr, workspace ? workspace_bytes : 0);
 }
 
+// Whether the sizes go to the few-row kernel, from which on nothing but alignment decides.
+static bool few_rows(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b, bool is16, bool vec) {
+    if (!is16 && f32_rows_in_parts(M, N, K, batch, trans_a, trans_b) > 0) return false;
+    return !trans_a && M <= (is16 ? 64 : 192) && (is16 && !vec ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, batch, trans_b, is16));
+}
+
 extern "C" int64_t mhip_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b, int dtype) {
     if (M <= 0 || N <= 0 || K <= 0 || batch != 1 || M > 0x7FFFFFFF || N > 0x7FFFFFFF || K > 0x7FFFFFFF) return 0;
     const bool is16 = dtype == MHIP_BF16 || dtype == MHIP_F16;
@@ -702,7 +708,7 @@ extern "C" int64_t mhip_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t 
     const bool vec = is16 && (trans_a ? M : K) % 8 == 0 && (trans_b ? K : N) % 8 == 0;
     if (!is16 && f32_rows_in_parts(M, N, K, batch, trans_a, trans_b) > 0) return f32_rows_in_parts(M, N, K, batch, trans_a, trans_b);
     if (vec && gemm_parts_wanted(M, N, K, batch, trans_a, trans_b)) return gemm_parts_workspace(M, N, K);
-    if (!trans_a && M <= (is16 ? 64 : 192) && (is16 && !vec ? skinny_unaligned(M, N, K) : skinny_rows(M, N, K, batch, trans_b, is16))) return gemm_skinny_workspace(M, N, K, batch, trans_b, is16);
+    if (few_rows(M, N, K, batch, trans_a, trans_b, is16, vec)) return gemm_skinny_workspace(M, N, K, batch, trans_b, is16);
     // (a large problem goes to the ring kernels, whose tiles fill the device)
     if (!is16) return gemm_f32_workspace(M, N, K, batch, trans_a, trans_b);
     if (!vec && pack_pays(M, N, K)) {
@@ -718,6 +724,7 @@ extern "C" int64_t mhip_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t 
 
 extern "C" int mhip_gemm_workspace_launches(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b, int dtype) {
     if (mhip_gemm_workspace(M, N, K, batch, trans_a, trans_b, dtype) == 0) return 0;
-    const bool vec = (dtype == MHIP_BF16 || dtype == MHIP_F16) && (trans_a ? M : K) % 8 == 0 && (trans_b ? K : N) % 8 == 0;
-    return vec && gemm_parts_wanted(M, N, K, batch, trans_a, trans_b) ? 0 : 1;
+    const bool is16 = dtype == MHIP_BF16 || dtype == MHIP_F16, vec = is16 && (trans_a ? M : K) % 8 == 0 && (trans_b ? K : N) % 8 == 0;
+    if (vec && gemm_parts_wanted(M, N, K, batch, trans_a, trans_b)) return 0;
+    return few_rows(M, N, K, batch, trans_a, trans_b, is16, vec) ? 0 : 1;
 }

@@ -26,6 +26,8 @@ struct GemmArgs {
     int ldc = 0;                      // row stride of C and the residual in elements; 0 = N (gemm256.hip only: a column slice of a wider C)
     float* partial = nullptr;         // split K: each part's fp32 sums go here (batch 1), [split][M][N] for launch_gemm_finish() or, in gemm_mid.hip, the accumulators of whole tiles
     int splits = 1;
+    uint64_t* words = nullptr;        // gemm_skinny.hip, split K: counts of arrivals behind the parts (arrive.h), and this launch's tag
+    uint64_t tag = 0;
     int stream_c = 0;                 // gemm256.hip: C is far larger than the L2s, store it with the streaming hint
 };
 

@@ -16,11 +16,10 @@
 // vector loads (odd K or N) load element by element (VEC = false), still with every load in flight.
 #include <mutex>
 
-#include "gemm_common.h"
+#include "arrive.h"
 
 namespace mhip {
 
-int launch_gemm_finish(hipStream_t s, const GemmArgs& g, int dtype);     // gemm_mid.hip
 bool gemm_strip_wanted(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b);          // gemm_strip.hip
 int launch_gemm_strip(hipStream_t s, const GemmArgs& g, int64_t batch, int dtype);
 
@@ -111,8 +110,9 @@ template <typename T, int VE, bool VEC> struct RowPiece {
 template <typename T, bool TB, int NF, int MT>
 constexpr bool strip_order() { return !TB && 16 * NF * (int)sizeof(T) < 128 && (sizeof(T) == 2 || MT == 1); }
 
-// NF = operands (groups of 16 columns) per strip, MT = groups of 16 rows, U = k steps loaded as one block.
-template <typename T, bool TB, bool VEC, int NF, int MT, int U, int WAVES>
+// NF = operands (groups of 16 columns) per strip, MT = groups of 16 rows, U = k steps loaded as one block.  PARTS: K is split over the grid too,
+// a kernel of its own: compiled into the others the arrivals cost up to 8 %, [128,768] x K 768 fp32 6.9 -> 7.5 us.
+template <typename T, bool TB, bool VEC, int NF, int MT, int U, int WAVES, bool PARTS>
 __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(GemmArgs g) {
     constexpr int KPL = Mfma16<T>::kKpl, KS = 4 * KPL;      // k per step
     constexpr int VE = NF, NS = 16 * NF;                     // (stored [K, N]: NF consecutive columns per lane)
@@ -130,6 +130,9 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(GemmArgs g) {
     const __amdgpu_buffer_rsrc_t ra = skinny_rsrc(a, (uint32_t)((int64_t)g.M * g.lda * sizeof(T)));
     const __amdgpu_buffer_rsrc_t rb = skinny_rsrc(b, (uint32_t)((int64_t)(TB ? g.N : g.K) * g.ldb * sizeof(T)));
 
+    uint64_t* const word = PARTS ? g.words + (int64_t)blockIdx.y * gridDim.x + blockIdx.x : nullptr;
+    uint64_t seen = 0;
+    if (PARTS && threadIdx.x == 0) seen = arrive_look(word);
     // this workgroup's k steps (all of them, or one split's), and this wave's share of them
     const int all_steps = (g.K + KS - 1) / KS, per_split = (all_steps + (int)gridDim.z - 1) / (int)gridDim.z;
     const int first = (int)blockIdx.z * per_split, steps = min(all_steps - first, per_split), per = (steps + waves - 1) / waves;
@@ -204,6 +207,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(GemmArgs g) {
         }
     }
 
+    if (PARTS && threadIdx.x == 0) arrive_claim(word, seen, g.tag);
     // ---- the waves' partial sums, in the accumulators' own layout: lane (li, lg) holds row 16 mt + li and,
     // in its four registers, operand rows 4 lg .. 4 lg + 3
 #pragma unroll
@@ -215,24 +219,41 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(GemmArgs g) {
     const T* bias = static_cast<const T*>(g.bias);
     const T* res = g.residual ? static_cast<const T*>(g.residual) + batch * g.sc : nullptr;
     T* c = static_cast<T*>(g.c) + batch * g.sc;
+    const int total = min(g.M - m0, 16 * MT) * NS;
+    auto sum_of = [&](int m, int nl) {
+        const int f = TB ? nl / 16 : nl % VE, i = TB ? nl % 16 : nl / VE;
+        const float* p = part + ((f * MT + m / 16) * 64 + (i >> 2) * 16 + (m & 15)) * 4 + (i & 3);
+        float v = 0.f;
+        for (int w = 0; w < waves; w++) v += p[w * (NF * MT * 256)];
+        return v;
+    };
+    if constexpr (PARTS) {
+        __shared__ int last;
+        // one split's sums; the last split to arrive goes on with all of them
+        for (int idx = threadIdx.x; idx < total; idx += blockDim.x) {
+            const int m = idx / NS, nl = idx % NS;
+            if (n0 + nl < g.N) store_part(g.partial + ((int64_t)blockIdx.z * g.M + m0 + m) * g.N + n0 + nl, sum_of(m, nl));
+        }
+        if (!arrive_last(word, (int)gridDim.z, &last)) return;
+    }
     auto finish = [&](auto act_tag) {
         constexpr int ACT = decltype(act_tag)::value;
-        const int total = min(g.M - m0, 16 * MT) * NS;
         for (int idx = threadIdx.x; idx < total; idx += blockDim.x) {
             const int m = idx / NS, nl = idx % NS, n = n0 + nl;
             if (n >= g.N) continue;
-            const int f = TB ? nl / 16 : nl % VE, i = TB ? nl % 16 : nl / VE;
-            const float* p = part + ((f * MT + m / 16) * 64 + (i >> 2) * 16 + (m & 15)) * 4 + (i & 3);
+            const int64_t at = (int64_t)(m0 + m) * g.N + n;
             float v = 0.f;
-            for (int w = 0; w < waves; w++) v += p[w * (NF * MT * 256)];
-            if (g.partial) {
-                g.partial[((int64_t)blockIdx.z * g.M + m0 + m) * g.N + n] = v;
-                continue;
-            }
+            if (PARTS) {
+                const int64_t mn = (int64_t)g.M * g.N;
+                float t[8];                                  // (eight splits at most, their loads in flight together)
+#pragma unroll
+                for (int s = 0; s < 8; s++) t[s] = load_part(g.partial + min(s, (int)gridDim.z - 1) * mn + at);
+#pragma unroll
+                for (int s = 0; s < 8; s++) if (s < (int)gridDim.z) v += t[s];
+            } else v = sum_of(m, nl);
             if (bias) v += Elem<T>::to_f32(bias[n]);
             v = sizeof(T) == 4 ? apply_act(v, ACT) : apply_act_c<ACT>(v);
             T o = Elem<T>::from_f32(v);
-            const int64_t at = (int64_t)(m0 + m) * g.N + n;
             // (second rounding on purpose: the same result as a separate add over the stored C)
             if (res) o = Elem<T>::from_f32(Elem<T>::to_f32(o) + Elem<T>::to_f32(res[at]));
             c[at] = o;
@@ -241,10 +262,10 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(GemmArgs g) {
     dispatch_act(g.act, finish);
 }
 
-template <typename T, bool TB, bool VEC, int NF, int MT, int U, int WAVES = 8>
-int launch_one(hipStream_t s, GemmArgs g, int64_t batch) {
-    constexpr int KS = 4 * Mfma16<T>::kKpl;
-    auto kern = gemm_skinny_kernel<T, TB, VEC, NF, MT, U, WAVES>;
+template <typename T, bool TB, bool VEC, int NF, int MT, int U, bool PARTS>
+int launch_kernel(hipStream_t s, GemmArgs g, int64_t batch) {
+    constexpr int KS = 4 * Mfma16<T>::kKpl, WAVES = 8;
+    auto kern = gemm_skinny_kernel<T, TB, VEC, NF, MT, U, WAVES, PARTS>;
     constexpr int kLds = WAVES * NF * MT * 1024;
     if (kLds > 64 * 1024) {
         static std::once_flag once;
@@ -263,6 +284,11 @@ int launch_one(hipStream_t s, GemmArgs g, int64_t batch) {
     return check_launch("gemm_skinny");
 }
 
+template <typename T, bool TB, bool VEC, int NF, int MT, int U>
+int launch_one(hipStream_t s, const GemmArgs& g, int64_t batch) {
+    return g.splits > 1 ? launch_kernel<T, TB, VEC, NF, MT, U, true>(s, g, batch) : launch_kernel<T, TB, VEC, NF, MT, U, false>(s, g, batch);
+}
+
 // Strip width: narrow strips put a small weight matrix on as many compute units as it has columns for, wide
 // ones read whole 128-byte lines per row.  Stored [K, N], us narrow / wide: [4,4096] x [4096,4096] 14.4 / 13.0,
 // [4,3072] x [3072,768] 5.8 / 9.4.  Stored [N, K] every strip reads whole lines and the wide one only saves reads
@@ -272,7 +298,8 @@ bool wide_strips(int64_t N, int64_t K, int64_t batch, bool tb) {
     return tb ? strips >= 128 && K >= 2048 : strips >= 128 || (strips >= 64 && K >= 2048);
 }
 
-// K split over the grid as well (fp32 sums in a workspace, one more launch): parts of about 1024 k, at most one
+// K split over the grid as well (fp32 sums in a workspace, added up by the last split of a block to arrive: 2 to 3 us less than by a launch
+// of its own, with which the lines below were drawn; fp32 [4,1024] x K 4096 12.3 -> 9.7, [64,768] x K 3072 12.5 -> 10.5): parts of about 1024 k, at most one
 // workgroup per compute unit.  From which K on that pays for the launch was swept with weights from memory, M 1 to 64, N 256 to
 // 4096; time in parts over time whole, the range over N:
 //   16-bit [K, N], up to 32 rows   K 2048 0.86 to 1.26   K 2560 0.71 to 1.02   K 3064 0.66 to 0.96
@@ -391,17 +418,23 @@ bool gemm_skinny_eligible(const GemmArgs& g, int trans_a, int elem_bytes) {
            ((int64_t)g.N + 64) * g.K * elem_bytes < 0x7FFFFFFFLL && ((int64_t)g.K + 64) * g.N * elem_bytes < 0x7FFFFFFFLL;
 }
 
+// The splits' sums, and a word for each block of at least 16 columns and 16 rows (strips in multiples of eight).
+static int64_t parts_bytes(int64_t M, int64_t N, int n) { return (M * N * 4 * n + 255) / 256 * 256; }
+static int64_t words_bytes(int64_t M, int64_t N) { return ((N + 15) / 16 + kXcds) * ((M + 15) / 16) * 8; }
 int64_t gemm_skinny_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b, bool is16) {
     const int n = skinny_splits(M, N, K, batch, trans_b, is16);
-    return n == 1 ? 0 : M * N * 4 * n;
+    return n == 1 ? 0 : parts_bytes(M, N, n) + words_bytes(M, N);
 }
 
 int launch_gemm_skinny(hipStream_t s, GemmArgs g, int64_t batch, int trans_b, int dtype, int64_t workspace_bytes) {
     g.splits = g.partial ? skinny_splits(g.M, g.N, g.K, batch, trans_b, dtype != MHIP_F32) : 1;
-    if ((int64_t)g.M * g.N * 4 * g.splits > workspace_bytes) g.splits = 1;
+    if (g.splits > 1 && parts_bytes(g.M, g.N, g.splits) + words_bytes(g.M, g.N) > workspace_bytes) g.splits = 1;
     if (g.splits == 1) g.partial = nullptr;
-    const int st = dtype_launch(s, g, batch, trans_b, dtype);
-    return st != MHIP_OK || g.splits == 1 ? st : launch_gemm_finish(s, g, dtype);
+    else {
+        g.words = reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(g.partial) + parts_bytes(g.M, g.N, g.splits));
+        g.tag = launch_tag();
+    }
+    return dtype_launch(s, g, batch, trans_b, dtype);
 }
 
 }  // namespace mhip
