@@ -95,12 +95,13 @@ __global__ __launch_bounds__(256 * KG) void gemm_mid_kernel(GemmArgs g) {
         lb.load(rb, st + kATile, wave, (kt * KG + group) * kBK, kend);
     };
 
+    // (two groups of waves, few stages each: behind the loop)
+    constexpr bool kAhead = KG == 1 && !SUMS;
     TileBias<T, TN> bias;
-    if (!SUMS) bias.load(g, n0 + wn * WTN, lane);
+    if (kAhead) bias.load(g, n0 + wn * WTN, lane);
     TileResidual<T, TM, TN> residual;
-    const T* res = static_cast<const T*>(g.residual) + batch * g.sc;
-    const bool early = !SUMS && g.residual && !g.partial && residual.kPasses == residual.kAtOnce && g.N >= 8;
-    if (early) residual.load(g, res, m0 + wm * WTM, n0 + wn * WTN, lane, 0);
+    const bool early = kAhead && g.residual && !g.partial && residual.kPasses == residual.kAtOnce && g.N >= 8;
+    if (early) residual.load(g, static_cast<const T*>(g.residual) + batch * g.sc, m0 + wm * WTM, n0 + wn * WTN, lane, 0);
     f32x16 acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; i++)
@@ -198,6 +199,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_mid_kernel(GemmArgs g) {
         }
         return;
     }
+    if (!SUMS && !kAhead) bias.load(g, n0 + wn * WTN, lane);
     if constexpr (!SUMS) store_tile<T, TM, TN>(g, acc, bias, residual, early, smem + wave * (WTM * (WTN * 2 + 16)), m0 + wm * WTM, n0 + wn * WTN, batch, lane);
 }
 
@@ -439,12 +441,14 @@ template <typename T>
 int launch_plan(hipStream_t s, GemmArgs g, int64_t batch, int ta, int tb, int dtype, const MidPlan& p) {
     g.splits = p.splits;
     if (p.splits == 1) g.partial = nullptr;
+    GemmArgs k = g;                       // (a split stores sums: bias and residual are the finish kernel's)
+    if (p.splits > 1) k.bias = k.residual = nullptr;
     int st;
-    if (p.form == kRing192) st = launch_gemm192(s, g, batch, ta, tb, dtype);
-    else if (!ta && !tb) st = launch_form<T, false, false>(s, g, batch, p.form);
-    else if (!ta) st = launch_form<T, false, true>(s, g, batch, p.form);
-    else if (!tb) st = launch_form<T, true, false>(s, g, batch, p.form);
-    else st = launch_form<T, true, true>(s, g, batch, p.form);
+    if (p.form == kRing192) st = launch_gemm192(s, k, batch, ta, tb, dtype);
+    else if (!ta && !tb) st = launch_form<T, false, false>(s, k, batch, p.form);
+    else if (!ta) st = launch_form<T, false, true>(s, k, batch, p.form);
+    else if (!tb) st = launch_form<T, true, false>(s, k, batch, p.form);
+    else st = launch_form<T, true, true>(s, k, batch, p.form);
     if (st != MHIP_OK || p.splits == 1) return st;
     switch (p.form) {
         case 0: case 3: return launch_finish<T, 64, 64>(s, g);
