@@ -18,7 +18,6 @@ namespace mhip {
 uint64_t launch_tag();
 
 constexpr int kAgentScope = 16;            // sc1 of a buffer access
-constexpr int kMostParts = 255;
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t parts_rsrc(const void* p) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, 0x7FFFFFFF, 0x00020000);
@@ -43,7 +42,7 @@ __device__ __forceinline__ void arrive_claim(uint64_t* word, uint64_t seen, uint
         __hip_atomic_compare_exchange_strong(word, &seen, tag, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// By the whole workgroup, when its word is claimed and its parts are stored: whether all `parts` workgroups have come by now.  `flag`: a word of LDS.
+// By the whole workgroup, when its word is claimed and its part is stored: whether all `parts` workgroups (255 at most) have come by now.  `flag`: a word of LDS.
 __device__ __forceinline__ bool arrive_last(uint64_t* word, int parts, int* flag) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();

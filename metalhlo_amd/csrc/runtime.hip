@@ -38,8 +38,13 @@ int tune_int(const char* name, int fallback) {
 
 uint64_t launch_tag() {
     static std::atomic<uint64_t> next{[] {
-        std::random_device r;
-        return ((uint64_t)r() << 32) ^ r() ^ (uint64_t)std::chrono::steady_clock::now().time_since_epoch().count();
+        uint64_t seed = (uint64_t)std::chrono::steady_clock::now().time_since_epoch().count();
+        try {
+            std::random_device r;
+            seed ^= ((uint64_t)r() << 32) ^ r();
+        } catch (...) {                    // (no source of random numbers: the clock alone, nothing passes a C entry)
+        }
+        return seed;
     }()};
     // (a bijection of a counter whose upper 56 bits all differ: steps of 256 reach every one of them)
     const uint64_t n = next.fetch_add(256, std::memory_order_relaxed) & ~(uint64_t)255;
