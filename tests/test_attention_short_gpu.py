@@ -1,4 +1,4 @@
-"""GPU parity of attention over few keys (attention_short.hip): queries and keys around its groups of 16 rows, 64 rows and 32 keys, more queries than keys and fewer, views, a negative scale.  Bars as for the other attention kernels (tests/test_attention_gpu.py)."""
+"""GPU parity of attention over few keys (attention_short.hip): queries and keys around its groups of 32 rows and 32 keys, more queries than keys and fewer, views, a negative scale.  Bars as for the other attention kernels (tests/test_attention_gpu.py)."""
 import numpy as np
 import pytest
 import torch
@@ -40,3 +40,17 @@ def test_projection_in_place():
     q, k, v = (as_f64(t) for t in qkv.view(B, S, 3, H, D).permute(2, 0, 3, 1, 4).unbind(0))
     got = kernels.causal_attention(qkv, B, H).view(B, S, H, D).permute(0, 2, 1, 3)
     assert_close(got, oracle.attention(q, k, v, is_causal=True), TOL[torch.bfloat16], "short, in place")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=lambda d: NAME[d])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("S", [1, 17, 32, 33, 37, 64])
+def test_a_row_keeps_its_bits_when_its_sequence_goes_on(S, D, dtype):
+    """What stands behind a row is hidden from it: the kernels for longer sequences form the same products and sums in the same order."""
+    from metalhlo_amd import kernels
+    q, k, v = (to_dev(np.random.default_rng(i + S).standard_normal((2, 3, 300, D)) * 2, dtype) for i in range(3))
+    scale = -0.2 if S == 33 else None
+    short = kernels.flash_attention(*(t[:, :, :S].contiguous() for t in (q, k, v)), is_causal=True, scale=scale)
+    for n in (65, 129, 300):
+        longer = kernels.flash_attention(*(t[:, :, :n].contiguous() for t in (q, k, v)), is_causal=True, scale=scale)
+        assert torch.equal(short, longer[:, :, :S]), n
