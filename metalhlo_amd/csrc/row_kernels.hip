@@ -432,8 +432,8 @@ void row_split_kernel(const T* __restrict__ x, const T* __restrict__ gamma, cons
 // What bounds a launch with few rows is what one compute unit moves, and for softmax its exponentials (16 cycles a wave each, 1.3 us
 // of a row of 50257, which is why they are computed once): [128,50257] bf16 107 us with the scalar three-pass kernel below, 8.9
 // here with the exponentials computed for the sum and again for the result, 8.4 with them kept.  SHARE workgroups of one XCD then take a row together: each reads all of it, its own
-// share first, which is the one it writes; what the others have read by then comes from the L2.  The partial sums of shares are added in
-// an order that is the same for all of them, so that a row is scaled by one number.
+// share first, which is the one it writes; what the others have read by then comes from the L2.  All of them add up in
+// one order, as a workgroup that has the row to itself does: a row has the same bits in every form, whatever rows are beside it.
 // ---------------------------------------------------------------------------
 typedef u32x4 u32x4_any __attribute__((aligned(2)));
 
@@ -485,12 +485,15 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT) void row_any_kernel(const T* _
     // softmax in 16 bits: the exponentials that this workgroup writes, where registers hold them
     constexpr bool kKeep = OP == kSoftmax && k16 && NS * E <= 64;
     float kept[kKeep ? NS : 1][kKeep ? E : 1];
-    // (a + b of two shares, then of two pairs: the same for every order that an exclusive or gives)
-    auto add_shares = [&](float(&s)[SHARE]) {
+    // Sums over the row in quarters of a thread's vectors, whatever SHARE is: a share is one or two of them, and (a + b) + (c + d) is the
+    // same for every order that the exclusive or above gives.
+    constexpr int kSums = NT < 1024 ? 1 : NV < 4 ? NV : 4;
+    auto part = [](int v) { return v / (NV / kSums); };
+    auto add_up = [](float(&s)[kSums]) {
 #pragma unroll
-        for (int w = 1; w < SHARE; w *= 2)
+        for (int w = 1; w < kSums; w *= 2)
 #pragma unroll
-            for (int i = 0; i < SHARE; i += 2 * w) s[i] += s[i + w];
+            for (int i = 0; i < kSums; i += 2 * w) s[i] += s[i + w];
         return s[0];
     };
     const T* xr = x + row * cols;
@@ -519,7 +522,7 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT) void row_any_kernel(const T* _
         m = row_reduce<NT, true>(m, red[0]);
         unit = softmax_unit<T>(m);
         shift = k16 ? m * unit : m;
-        float s[SHARE] = {};
+        float s[kSums] = {};
         const float se = ei >= 0 ? (k16 ? __builtin_amdgcn_exp2f(fmaf(ev, unit, -shift)) : expf(ev - m)) : 0.f;
 #pragma unroll
         for (int v = 0; v < NV; v++)
@@ -530,15 +533,15 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT) void row_any_kernel(const T* _
                     const float p = k16 ? __builtin_amdgcn_exp2f(fmaf(f, unit, -shift)) : expf(f - m);
                     if (!k16) raw[v].v[e] = Elem<T>::from_f32(p);       // (kept: exact in fp32)
                     if (kKeep && v < NS) kept[kKeep ? v : 0][kKeep ? e : 0] = p;
-                    s[v / NS] += p;
+                    s[part(v)] += p;
                 }
             }
-        scale = 1.f / row_reduce<NT, false>(add_shares(s) + se, red[1]);
+        scale = 1.f / row_reduce<NT, false>(add_up(s) + se, red[1]);
     } else if (OP == kLayerNorm) {
-        float s[SHARE] = {}, q[SHARE] = {};
+        float s[kSums] = {}, q[kSums] = {};
 #pragma unroll
-        for (int v = 0; v < NV; v++) s[v / NS] = VecSum<T>::sum(raw[v], s[v / NS]);
-        const float mean = row_reduce<NT, false>(add_shares(s) + ev, red[0]) / n;
+        for (int v = 0; v < NV; v++) s[part(v)] = VecSum<T>::sum(raw[v], s[part(v)]);
+        const float mean = row_reduce<NT, false>(add_up(s) + ev, red[0]) / n;
         const float qe = ei >= 0 ? (ev - mean) * (ev - mean) : 0.f;
 #pragma unroll
         for (int v = 0; v < NV; v++)
@@ -546,16 +549,17 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT) void row_any_kernel(const T* _
 #pragma unroll
                 for (int e = 0; e < E; e++) {
                     const float d = Elem<T>::to_f32(raw[v].v[e]) - mean;
-                    q[v / NS] = fmaf(d, d, q[v / NS]);
+                    q[part(v)] = fmaf(d, d, q[part(v)]);
                 }
             }
-        scale = 1.f / sqrtf(row_reduce<NT, false>(add_shares(q) + qe, red[1]) / n + eps);
+        scale = 1.f / sqrtf(row_reduce<NT, false>(add_up(q) + qe, red[1]) / n + eps);
         shift = mean;
     } else {
-        float q[SHARE] = {};
+        float q[kSums] = {};
 #pragma unroll
-        for (int v = 0; v < NV; v++) q[v / NS] = VecSum<T>::sumsq(raw[v], q[v / NS]);
-        scale = 1.f / sqrtf(row_reduce<NT, false>(add_shares(q) + ev * ev, red[0]) / n + eps);
+        for (int v = 0; v < NV; v++) q[part(v)] = VecSum<T>::sumsq(raw[v], q[part(v)]);
+        const float qe = ev * ev;
+        scale = 1.f / sqrtf(row_reduce<NT, false>(add_up(q) + qe, red[0]) / n + eps);
     }
     auto value = [&](float f, float g, float b) {
         if (OP == kSoftmax) return (k16 ? __builtin_amdgcn_exp2f(fmaf(f, unit, -shift)) : f) * scale;
@@ -569,9 +573,17 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT) void row_any_kernel(const T* _
         if (OP != kSoftmax && gamma) gv = __builtin_bit_cast(Vec16<T>, *reinterpret_cast<const u32x4_any*>(gamma + ph.head + i * E));
         if (OP == kLayerNorm && beta) bv = __builtin_bit_cast(Vec16<T>, *reinterpret_cast<const u32x4_any*>(beta + ph.head + i * E));
 #pragma unroll
-        for (int e = 0; e < E; e++)
+        for (int e = 0; e < E; e++) {
             o.v[e] = Elem<T>::from_f32(kKeep ? kept[kKeep ? v : 0][kKeep ? e : 0] * scale : value(Elem<T>::to_f32(raw[v].v[e]), OP != kSoftmax && gamma ? Elem<T>::to_f32(gv.v[e]) : 1.f,
                                              OP == kLayerNorm && beta ? Elem<T>::to_f32(bv.v[e]) : 0.f));
+            // (f16: the multiply-add that rounds once, to f16, in every form.  A lone vector is otherwise converted in pairs behind
+            // fp32 multiply-adds, and rounded twice.)
+            if constexpr (std::is_same<T, f16_t>::value && OP != kSoftmax && SHARE > 1 && NS == 1) {
+                uint32_t bits = __builtin_bit_cast(uint16_t, o.v[e]);
+                asm("" : "+v"(bits));
+                o.v[e] = __builtin_bit_cast(T, (uint16_t)bits);
+            }
+        }
         store16_stream(yr + ph.head + i * E, o);
     }
     if (ei >= 0 && share == 0) {
