@@ -1,5 +1,6 @@
-"""What the compiler made of the kernels that count the loads they have in flight: a register that does not fit goes to memory, and
-its reload waits for every load before it, tiles asked for ahead of their use among them.  Read from the metadata of the built library."""
+"""What the compiler made of the kernels that count the loads they have in flight, or keep a row in registers: a register that does not fit
+goes to memory, and its reload waits for every load before it, tiles asked for ahead of their use among them.  Read from the metadata of
+the built library."""
 import os
 import struct
 
@@ -34,7 +35,7 @@ def _kernels():
 
 
 @pytest.mark.parametrize("name", ["fa_flow_kernel", "gemm_f32_ring_kernel", "gemm_mid_kernel", "gemm192_kernel", "linear_w32_kernel",
-                                  "linear_w32_stream_kernel", "tied_head_kernel"])
+                                  "linear_w32_stream_kernel", "tied_head_kernel", "row_any_kernelIDF16bLi0E", "row_any_kernelIDF16_Li0E"])
 def test_nothing_is_spilled(name):
     if not os.path.exists(LIB):
         pytest.skip("no built library")
