@@ -930,7 +930,10 @@ static int launch_row(hipStream_t s, const void* x, const void* g, const void* b
         const char *x0 = reinterpret_cast<const char*>(xp), *y0 = reinterpret_cast<const char*>(yp);
         const int64_t bytes = rows * cols * (int64_t)sizeof(T);
         const bool apart = x0 + bytes <= y0 || y0 + bytes <= x0;
-        const int share = !apart ? 1 : rows <= 64 ? 4 : rows <= 128 && (OP == kLayerNorm || (OP == kRmsNorm && sizeof(T) == 2)) ? 2 : 1;
+        constexpr bool kTwo = OP == kLayerNorm || (OP == kRmsNorm && sizeof(T) == 2);
+        const int share = !apart ? 1 : rows <= 64 ? 4 : kTwo && rows <= 128 ? 2 : 1;
+        // (two vectors a thread: two workgroups where four are wanted too)
+#define MHIP_ROW_TWO(NT, NV) do { if constexpr (kTwo) MHIP_ROW_SHARED(NT, NV, 2); } while (0)
         if (nvec <= 64) MHIP_ROW_ANY(64, 1);
         else if (nvec <= 128) MHIP_ROW_ANY(64, 2);
         else if (nvec <= 256) MHIP_ROW_ANY(256, 1);
@@ -938,16 +941,17 @@ static int launch_row(hipStream_t s, const void* x, const void* g, const void* b
         else if (nvec <= 1024) MHIP_ROW_ANY(256, 4);
         else if (nvec <= 2048 && share >= 2) MHIP_ROW_SHARED(1024, 2, 2);
         else if (nvec <= 4096 && share >= 4) MHIP_ROW_SHARED(1024, 4, 4);
-        else if (nvec <= 4096 && share >= 2) MHIP_ROW_SHARED(1024, 4, 2);
+        else if (nvec <= 4096 && share >= 2) MHIP_ROW_TWO(1024, 4);
         else if (nvec <= 8192 && share >= 4) MHIP_ROW_SHARED(1024, 8, 4);
-        else if (nvec <= 8192 && share >= 2) MHIP_ROW_SHARED(1024, 8, 2);
+        else if (nvec <= 8192 && share >= 2) MHIP_ROW_TWO(1024, 8);
         else if (nvec > 8192 && share >= 4) MHIP_ROW_SHARED(1024, 16, 4);
-        else if (nvec > 8192 && share >= 2) MHIP_ROW_SHARED(1024, 16, 2);
+        else if (nvec > 8192 && share >= 2) MHIP_ROW_TWO(1024, 16);
         else if (nvec <= 2048) MHIP_ROW_ANY(1024, 2);
         else if (nvec <= 4096) MHIP_ROW_ANY(1024, 4);
         else if (nvec <= 8192) MHIP_ROW_ANY(1024, 8);
         else MHIP_ROW_ANY(1024, 16);
 #undef MHIP_ROW_ANY
+#undef MHIP_ROW_TWO
 #undef MHIP_ROW_SHARED
     } else {
         hipLaunchKernelGGL((row_block_kernel<T, OP>), dim3((unsigned)rows), dim3(256), 0, s, xp,

@@ -2,6 +2,7 @@
 goes to memory, and its reload waits for every load before it, tiles asked for ahead of their use among them.  Read from the metadata of
 the built library."""
 import os
+import re
 import struct
 
 import pytest
@@ -62,3 +63,13 @@ def test_fp32_rings_leave_a_unit_several_workgroups():
     found = [k for k in _kernels() if "gemm_f32_ring_kernel" in k[".name"]]
     assert found
     assert [(k[".name"], k[".vgpr_count"]) for k in found if k[".vgpr_count"] > 256] == []
+
+
+def test_shared_rows_have_the_forms_that_a_launch_chooses():
+    """Two workgroups a row with more than two vectors a thread: LayerNorm, and RMSNorm of 16-bit types."""
+    if not os.path.exists(LIB):
+        pytest.skip("no built library")
+    two = {m.groups() for k in _kernels() for m in [re.search(r"row_any_kernelI(f|DF16b|DF16_)Li(\d)ELi1024ELi(\d+)ELi2E", k[".name"])] if m}
+    want = {(t, op, "2") for t in ("f", "DF16b", "DF16_") for op in "012"}
+    want |= {(t, op, nv) for t in ("f", "DF16b", "DF16_") for op in "12" for nv in ("4", "8", "16") if t != "f" or op == "1"}
+    assert two == want
