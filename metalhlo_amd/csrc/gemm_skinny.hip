@@ -228,13 +228,13 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(GemmArgs g) {
         return v;
     };
     if constexpr (PARTS) {
-        __shared__ int last;
         // one split's sums; the last split to arrive goes on with all of them
         for (int idx = threadIdx.x; idx < total; idx += blockDim.x) {
             const int m = idx / NS, nl = idx % NS;
             if (n0 + nl < g.N) store_part(g.partial + ((int64_t)blockIdx.z * g.M + m0 + m) * g.N + n0 + nl, sum_of(m, nl));
         }
-        if (!arrive_last(word, (int)gridDim.z, &last)) return;
+        // (the flag where the sums were, which nobody reads behind the arrival's barrier: a word beside 64 KB is more than a launch gets unasked)
+        if (!arrive_last(word, (int)gridDim.z, reinterpret_cast<int*>(part))) return;
     }
     auto finish = [&](auto act_tag) {
         constexpr int ACT = decltype(act_tag)::value;

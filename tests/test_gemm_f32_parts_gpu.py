@@ -77,3 +77,9 @@ def test_twelve_columns_keep_a_rows_bits(ta):
         x = (a[:n].t() if ta else a[:n]).contiguous()
         return kernels.matmul(x, b, trans_a=ta)[:193]
     assert torch.equal(rows(193), rows(4000))
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 4096, 4096), (33, 4100, 4096), (52, 8192, 3264)], ids=lambda v: str(v))
+def test_few_rows_whose_sums_take_all_of_64_kb(M, N, K):
+    """Strips of 32 columns by 64 rows in parts of K: the waves' sums fill what a launch gets without asking for more."""
+    _check(M, N, K, torch.float32, False, False, residual=M % 2 == 0)

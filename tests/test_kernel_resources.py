@@ -73,3 +73,14 @@ def test_shared_rows_have_the_forms_that_a_launch_chooses():
     want = {(t, op, "2") for t in ("f", "DF16b", "DF16_") for op in "012"}
     want |= {(t, op, nv) for t in ("f", "DF16b", "DF16_") for op in "12" for nv in ("4", "8", "16") if t != "f" or op == "1"}
     assert two == want
+
+
+def test_few_row_sums_fit_what_a_launch_gets():
+    """gemm_skinny_kernel asks for more LDS than 64 KB where its waves' sums alone are more: 1 KB a wave, group of columns and group of rows."""
+    if not os.path.exists(LIB):
+        pytest.skip("no built library")
+    found = [(k, re.search(r"gemm_skinny_kernelI\w+?Lb\dELb\dELi(\d)ELi(\d)ELi\dELi8E", k[".name"])) for k in _kernels() if "gemm_skinny_kernel" in k[".name"]]
+    assert found and all(m for _, m in found)
+    sums = [(k, int(m.group(1)) * int(m.group(2)) * 8 * 1024) for k, m in found]
+    assert any(n == 64 * 1024 for _, n in sums)
+    assert [k[".name"] for k, n in sums if n <= 64 * 1024 < n + k[".group_segment_fixed_size"]] == []
