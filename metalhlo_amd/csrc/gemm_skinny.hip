@@ -330,8 +330,10 @@ RowsPlan rows_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool tb) {
     return best;
 }
 
-int skinny_splits(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b, bool is16) {
-    if (batch != 1 || M * N > (1 << 20) || (is16 && gemm_strip_wanted(M, N, K, batch, trans_b))) return 1;
+// (The strip kernel, which holds all of K, takes 16-bit operands on 16 bytes only: `vec`.  Others of its sizes are split: [8,256] x K 4096 two
+// bytes off 48.9 us whole, 17.5.)
+int skinny_splits(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b, bool is16, bool vec) {
+    if (batch != 1 || M * N > (1 << 20) || (is16 && vec && gemm_strip_wanted(M, N, K, batch, trans_b))) return 1;
     if (!is16 && rows_plan(M, N, K, batch, trans_b != 0).splits > 1) return rows_plan(M, N, K, batch, trans_b != 0).splits;
     const int64_t width = wide_strips(N, K, 1, trans_b != 0) ? (trans_b ? 32 : 64) : (trans_b ? 16 : 32);
     const int64_t from = is16 ? (trans_b && M <= 16 ? 3584 : 2560) : (M > 32 ? 3072 : 2560);
@@ -394,10 +396,14 @@ int launch_shape(hipStream_t s, const GemmArgs& g, int64_t batch) {
     }
 }
 
-int dtype_launch(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_b, int dtype) {
+bool on_16_bytes(const GemmArgs& g, int dtype) {
     const int per16 = dtype == MHIP_F32 ? 4 : 8;
-    const bool vec = g.lda % per16 == 0 && g.ldb % per16 == 0 && g.sa % per16 == 0 && g.sb % per16 == 0 &&
-                     ((reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.b)) & 15) == 0;
+    return g.lda % per16 == 0 && g.ldb % per16 == 0 && g.sa % per16 == 0 && g.sb % per16 == 0 &&
+           ((reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.b)) & 15) == 0;
+}
+
+int dtype_launch(hipStream_t s, const GemmArgs& g, int64_t batch, int trans_b, int dtype) {
+    const bool vec = on_16_bytes(g, dtype);
     if (vec && dtype != MHIP_F32 && gemm_strip_wanted(g.M, g.N, g.K, batch, trans_b)) return launch_gemm_strip(s, g, batch, dtype);
 #define MHIP_SKINNY(T)                                                                                              \
     (vec ? (trans_b ? launch_shape<T, true, true>(s, g, batch) : launch_shape<T, false, true>(s, g, batch))         \
@@ -422,12 +428,13 @@ bool gemm_skinny_eligible(const GemmArgs& g, int trans_a, int elem_bytes) {
 static int64_t parts_bytes(int64_t M, int64_t N, int n) { return (M * N * 4 * n + 255) / 256 * 256; }
 static int64_t words_bytes(int64_t M, int64_t N) { return ((N + 15) / 16 + kXcds) * ((M + 15) / 16) * 8; }
 int64_t gemm_skinny_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_b, bool is16) {
-    const int n = skinny_splits(M, N, K, batch, trans_b, is16);
+    // (from the sizes: the pointers may lie anywhere)
+    const int n = skinny_splits(M, N, K, batch, trans_b, is16, false);
     return n == 1 ? 0 : parts_bytes(M, N, n) + words_bytes(M, N);
 }
 
 int launch_gemm_skinny(hipStream_t s, GemmArgs g, int64_t batch, int trans_b, int dtype, int64_t workspace_bytes) {
-    g.splits = g.partial ? skinny_splits(g.M, g.N, g.K, batch, trans_b, dtype != MHIP_F32) : 1;
+    g.splits = g.partial ? skinny_splits(g.M, g.N, g.K, batch, trans_b, dtype != MHIP_F32, on_16_bytes(g, dtype)) : 1;
     if (g.splits > 1 && parts_bytes(g.M, g.N, g.splits) + words_bytes(g.M, g.N) > workspace_bytes) g.splits = 1;
     if (g.splits == 1) g.partial = nullptr;
     else {

@@ -150,3 +150,19 @@ def test_workspaces_under_capture_and_on_a_side_stream():
         got = step(late, nq)
     torch.cuda.current_stream().wait_stream(side)
     assert all(torch.equal(o, e) for o, e in zip(got, step(late, nq)))
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 256, 4096), (1, 64, 3584)], ids=lambda v: str(v))
+def test_few_rows_off_16_bytes_are_split(lib, M, N, K):
+    """Sizes whose strips hold all of K on 16 bytes: other addresses are served in parts, which lie in the workspace afterwards."""
+    need = lib.mhip_gemm_workspace(M, N, K, 1, 0, 1, 3)
+    assert need > 0
+    a, b = torch.randn(M, K, device="cuda").bfloat16(), torch.randn(N * K + 1, device="cuda").bfloat16()
+    for off in (0, 1):
+        w = b[off:off + N * K].view(N, K)
+        out, ws = torch.empty(M, N, dtype=torch.bfloat16, device="cuda"), torch.full((need,), 170, dtype=torch.uint8, device="cuda")
+        assert lib.mhip_gemm_ws(torch.cuda.current_stream().cuda_stream, a.data_ptr(), w.data_ptr(), None, None, out.data_ptr(), M, N, K, 1, 0, 0, 0, 0, 1, 0, 3,
+                                ws.data_ptr(), need) == 0
+        e, fp32 = a.double() @ w.double().t(), K * 2.0 ** -24 * (a.double().abs() @ w.double().abs().t())
+        assert ((out.double() - e).abs() <= fp32 + ROUNDOFF[torch.bfloat16] * (e.abs() + fp32)).all()
+        assert bool((ws[:2 * M * N * 4] != 170).any()) == bool(off)
