@@ -34,9 +34,9 @@ template <> struct Mfma16A<f16_t> {
 
 constexpr int kKeys = 32;        // keys per block
 constexpr int kMaxSq = 16;
-// A part of a split key range is a multiple of this.  us, multiples of 128 | 256 keys: one query of 32 heads over 512 keys, head size 128,
-// 6.7 | 8.1, of 24 over 1024, 64, 6.4 | 6.7, of 8 over 2048, 128, 8.7 | 8.5; eight queries of 8 heads over 4096, 64, 15.9 | 10.5; 12 heads
-// over 300 keys 6.4 | 5.4 (whole).
+// A part of a split key range is a multiple of this.  us, multiples of 128 | 256 keys, one query (eight): 32 heads over 512 keys, head size 128,
+// 6.7 | 8.0 (7.2 | 8.6), 12 over 640, 64, 5.2 | 7.5 (5.6 | 7.7), 24 over 1024, 64, 6.2 | 6.7 (6.3 | 6.9), 8 over 1536, 64, 6.7 | 6.9 (6.8 | 6.9), 8 over
+// 2048, 128, 8.7 | 8.5 (9.1 | 9.4), 8 over 4096, 64, 11.7 | 9.0 (12.5 | 9.0); 12 over 300 6.0 | 4.7 (whole).
 constexpr int part_keys(int64_t Skv) { return Skv >= 512 && Skv <= 1024 ? 128 : 256; }
 
 // domain of scores and reference (see moved_reference): f16's lowest number is far from fp32's
@@ -178,9 +178,34 @@ __global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* 
     for (int f = 0; f < NF; f++) *reinterpret_cast<f32x4*>(sums[wave][f][lane]) = oacc[f];
     __syncthreads();
     T* op = static_cast<T*>(a.o) + b_i * a.os[0] + h_i * a.os[1];
-    for (int idx = threadIdx.x; idx < a.Sq * D; idx += 64 * WAVES) {
-        const int q = idx / D, d = idx % D, f = d % NF, i = d / NF;
-        float m = -INFINITY, l = 0.f, o = 0.f;
+    if (!part) {
+        for (int idx = threadIdx.x; idx < a.Sq * D; idx += 64 * WAVES) {
+            const int q = idx / D, d = idx % D, f = d % NF, i = d / NF;
+            float m = -INFINITY, l = 0.f, o = 0.f;
+#pragma unroll
+            for (int w = 0; w < WAVES; w++) m = fmaxf(m, ml[0][w][q]);
+            const float m_use = m == -INFINITY ? 0.f : m;
+#pragma unroll
+            for (int w = 0; w < WAVES; w++) {
+                const float al = weight<NAT>(ml[0][w][q], m_use);
+                l = fmaf(ml[1][w][q], al, l);
+                o = fmaf(sums[w][f][(i >> 2) * 16 + q][i & 3], al, o);
+            }
+            op[(int64_t)q * a.os[2] + d] = Elem<T>::from_f32(o * (l > 1e-10f ? 1.f / l : 0.f));
+        }
+        return;
+    }
+
+    // ---- this part of the keys: [part][bh][Sq] x 4 NF groups of four sums, as the accumulators hold them (group 4 f + g: d = NF (4 g + e) + f), then
+    // [part][bh][Sq] pairs of reference maximum and sum
+    constexpr int kGroups = 4 * NF;
+    const int parts = gridDim.y;
+    const __amdgpu_buffer_rsrc_t rp = parts_rsrc(part), rl = parts_rsrc(part + (int64_t)parts * gridDim.x * a.Sq * D);
+    auto row_of = [&](int p, int q) __attribute__((always_inline)) { return (p * (int)gridDim.x + bh) * a.Sq + q; };
+    for (int idx = threadIdx.x; idx < a.Sq * kGroups; idx += 64 * WAVES) {
+        const int q = idx / kGroups, group = idx % kGroups;
+        float m = -INFINITY, l = 0.f;
+        f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < WAVES; w++) m = fmaxf(m, ml[0][w][q]);
         const float m_use = m == -INFINITY ? 0.f : m;
@@ -188,53 +213,124 @@ __global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* 
         for (int w = 0; w < WAVES; w++) {
             const float al = weight<NAT>(ml[0][w][q], m_use);
             l = fmaf(ml[1][w][q], al, l);
-            o = fmaf(sums[w][f][(i >> 2) * 16 + q][i & 3], al, o);
+            const f32x4 v = *reinterpret_cast<const f32x4*>(sums[w][group >> 2][(group & 3) * 16 + q]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[e] = fmaf(v[e], al, o[e]);
         }
-        if (part) {
-            // [part][bh][Sq][D] sums, then [part][bh][Sq][2] reference maximum and sum
-            const int64_t at = ((int64_t)blockIdx.y * gridDim.x + bh) * a.Sq + q;
-            store_part(part + at * D + d, o);
-            if (d < 2) store_part(part + (int64_t)gridDim.y * gridDim.x * a.Sq * D + at * 2 + d, d ? l : m);
-        } else {
-            op[(int64_t)q * a.os[2] + d] = Elem<T>::from_f32(o * (l > 1e-10f ? 1.f / l : 0.f));
-        }
+        store_part(rp, (uint32_t)((row_of(blockIdx.y, q) * kGroups + group) * 16), o);
+        if (group == 0)
+            __builtin_amdgcn_raw_buffer_store_b64(u32x2{__builtin_bit_cast(uint32_t, m), __builtin_bit_cast(uint32_t, l)}, rl, (uint32_t)(row_of(blockIdx.y, q) * 8), 0, kAgentScope);
     }
-    const int parts = gridDim.y;
-    if (!part || !arrive_last(words + bh, parts, &last)) return;
+    if (!arrive_last(words + bh, parts, &last)) return;
 
-    // ---- the last part of the head to arrive: an element of O a thread, eight parts' loads in flight
-    const int64_t rows = (int64_t)gridDim.x * a.Sq;
-    for (int idx = threadIdx.x; idx < a.Sq * D; idx += 64 * WAVES) {
-        const int q = idx / D, d = idx % D;
-        const int64_t row = (int64_t)bh * a.Sq + q;
-        const float* mls = part + parts * rows * D + row * 2;
-        const float* os = part + row * D + d;
-        float m = -INFINITY, l = 0.f, o = 0.f;
-        for (int p0 = 0; p0 < parts; p0 += 8) {
-            float pm[8], pl[8], po[8];
+    // ---- the last part of the head to arrive, four sums a thread.  (One element of O a thread, with the weights formed for each of them, 16 queries of
+    // 8 heads over 16384 keys of head size 128 took 67.4 us, 32 so, and with a launch of
+    // its own behind it 48.2.)
+    auto put = [&](int q, int group, int e, float v) __attribute__((always_inline)) {
+        op[(int64_t)q * a.os[2] + NF * (4 * (group & 3) + e) + (group >> 2)] = Elem<T>::from_f32(v);
+    };
+    // Up to sixteen parts: every thread asks for its row's references and sums too, and all is there after one latency.
+    auto few = [&](auto most_tag) __attribute__((always_inline)) {
+        constexpr int kMost = decltype(most_tag)::value;
+        for (int idx = threadIdx.x; idx < a.Sq * kGroups; idx += 64 * WAVES) {
+            const int q = idx / kGroups, group = idx % kGroups;
+            u32x2 state[kMost];
+            f32x4 v[kMost], o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const int p = min(p0 + u, parts - 1);
-                pm[u] = load_part(mls + p * rows * 2);
-                pl[u] = load_part(mls + p * rows * 2 + 1);
-                po[u] = load_part(os + p * rows * D);
+            for (int p = 0; p < kMost; p++) {
+                state[p] = __builtin_amdgcn_raw_buffer_load_b64(rl, p < parts ? (uint32_t)(row_of(p, q) * 8) : kOobA, 0, kAgentScope);
+                v[p] = load_part(rp, p < parts ? (uint32_t)((row_of(p, q) * kGroups + group) * 16) : kOobA);
             }
-            float m_new = m;
+            float pm[kMost], m = -INFINITY, l = 0.f;
 #pragma unroll
-            for (int u = 0; u < 8; u++) m_new = fmaxf(m_new, pm[u]);
-            const float m_use = m_new == -INFINITY ? 0.f : m_new, old = weight<NAT>(m, m_use);
-            l *= old;
-            o *= old;
-#pragma unroll
-            for (int u = 0; u < 8; u++) {
-                if (p0 + u >= parts) break;
-                const float al = weight<NAT>(pm[u], m_use);
-                l = fmaf(pl[u], al, l);
-                o = fmaf(po[u], al, o);
+            for (int p = 0; p < kMost; p++) {
+                const uint32_t bits = state[p].x;
+                pm[p] = p < parts ? __builtin_bit_cast(float, bits) : -INFINITY;
+                m = fmaxf(m, pm[p]);
             }
-            m = m_new;
+            const float m_use = m == -INFINITY ? 0.f : m;
+#pragma unroll
+            for (int p = 0; p < kMost; p++) {
+                const uint32_t bits = state[p].y;
+                const float al = weight<NAT>(pm[p], m_use);
+                l = fmaf(__builtin_bit_cast(float, bits), al, l);
+#pragma unroll
+                for (int e = 0; e < 4; e++) o[e] = fmaf(v[p][e], al, o[e]);
+            }
+            const float inv = l > 1e-10f ? 1.f / l : 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) put(q, group, e, o[e] * inv);
         }
-        op[(int64_t)q * a.os[2] + d] = Elem<T>::from_f32(o * (l > 1e-10f ? 1.f / l : 0.f));
+    };
+    if (parts <= 4) return few(std::integral_constant<int, 4>{});
+    if (parts <= 8) return few(std::integral_constant<int, 8>{});
+    if (parts <= 16) return few(std::integral_constant<int, 16>{});
+    // More: a row's weights are formed once, a lane a part (64 at most), while the first loads are on their way, and the parts are dealt over
+    // threads where there are few queries.
+    constexpr int kSlots = 64 * WAVES / kGroups;
+    float* const weights = &sums[0][0][0][0];                // [kMaxSq][64]
+    float* const inverse = weights + kMaxSq * 64;            // [kMaxSq]
+    float* const shares = inverse + 64;                      // [sharers][Sq][D]
+    static_assert((kMaxSq * 64 + 64 + kMaxSq * D) * 4 <= (int)sizeof(sums) && kSlots <= kMaxSq, "in place of the waves' sums");
+    int together = 1;                                        // queries at a time, a power of two
+    while (together < a.Sq && together < kSlots) together *= 2;
+    const int sharers = min(kSlots / together, 4), group = threadIdx.x % kGroups, slot = threadIdx.x / kGroups, first = slot / together;
+    constexpr int kLoads = 16;
+    f32x4 v[kLoads];
+    // sixteen loads of 16 bytes in flight: parts first, first + step, ... of a row
+    auto ask = [&](int q, int group, int first, int step) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < kLoads; u++) {
+            const int p = first + u * step;
+            v[u] = load_part(rp, p < parts && q < a.Sq ? (uint32_t)((row_of(p, q) * kGroups + group) * 16) : kOobA);
+        }
+    };
+    u32x2 state[kMaxSq / WAVES];
+#pragma unroll
+    for (int j = 0; j < kMaxSq / WAVES; j++) {
+        const int q = wave + j * WAVES;
+        state[j] = __builtin_amdgcn_raw_buffer_load_b64(rl, lane < parts && q < a.Sq ? (uint32_t)(row_of(lane, q) * 8) : kOobA, 0, kAgentScope);
+    }
+    int q = first < sharers ? slot % together : a.Sq;
+    ask(q, group, first, sharers);
+#pragma unroll
+    for (int j = 0; j < kMaxSq / WAVES; j++) {
+        const int qw = wave + j * WAVES;
+        if (qw >= a.Sq) break;
+        const uint32_t m_bits = state[j].x, l_bits = state[j].y;
+        const float pm = lane < parts ? __builtin_bit_cast(float, m_bits) : -INFINITY, m = wave_max(pm);
+        const float al = lane < parts ? weight<NAT>(pm, m == -INFINITY ? 0.f : m) : 0.f;
+        const float l = wave_sum(__builtin_bit_cast(float, l_bits) * al);
+        weights[qw * 64 + lane] = al;
+        if (lane == 0) inverse[qw] = l > 1e-10f ? 1.f / l : 0.f;
+    }
+    __syncthreads();
+    for (; q < a.Sq; q += together) {
+        f32x4 o = {0.f, 0.f, 0.f, 0.f};
+        for (int p0 = first;;) {
+#pragma unroll
+            for (int u = 0; u < kLoads; u++) {
+                const float al = weights[q * 64 + min(p0 + u * sharers, 63)];
+#pragma unroll
+                for (int e = 0; e < 4; e++) o[e] = fmaf(v[u][e], al, o[e]);
+            }
+            p0 += kLoads * sharers;
+            if (p0 >= parts) break;
+            ask(q, group, p0, sharers);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            if (sharers == 1) put(q, group, e, o[e] * inverse[q]);
+            else shares[(first * a.Sq + q) * D + NF * (4 * (group & 3) + e) + (group >> 2)] = o[e];
+        }
+        if (q + together < a.Sq) ask(q + together, group, first, sharers);
+    }
+    if (sharers == 1) return;
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < a.Sq * D; idx += 64 * WAVES) {
+        float o = shares[idx] + shares[a.Sq * D + idx];       // (two threads share four sums, or four)
+        if (sharers == 4) o += shares[2 * a.Sq * D + idx] + shares[3 * a.Sq * D + idx];
+        op[(int64_t)(idx / D) * a.os[2] + idx % D] = Elem<T>::from_f32(o * inverse[idx / D]);
     }
 }
 

@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=lambda d: NAME[d])
-@pytest.mark.parametrize("B,H,Sq,Skv,D", [(1, 3, 1, 512, 64), (2, 2, 16, 640, 128), (1, 2, 3, 1024, 64), (1, 2, 2, 1025, 64), (1, 1, 5, 2304, 128), (1, 1, 1, 16384, 64)],
+@pytest.mark.parametrize("B,H,Sq,Skv,D", [(1, 3, 1, 512, 64), (2, 2, 16, 640, 128), (1, 2, 3, 1024, 64), (1, 2, 2, 1025, 64), (1, 1, 5, 2304, 128), (1, 1, 1, 16384, 64),
+                                         (1, 2, 16, 8192, 128), (1, 1, 13, 16384, 64), (1, 5, 7, 4000, 128), (1, 3, 9, 1100, 64)],
                          ids=lambda v: str(v))
 def test_parts_and_workspace_of_any_content(lib, B, H, Sq, Skv, D, dtype):
     from metalhlo_amd import kernels
