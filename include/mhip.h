@@ -151,7 +151,8 @@ int mhip_gemm_residual(void* stream, const void* a, const void* b, const void* b
  * workspace is 16-byte aligned, its content is overwritten and meaningless afterwards, and it may be reused as
  * soon as work enqueued behind this call on the same stream may run. */
 int64_t mhip_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b, int dtype);
-/* Launches that the use of that workspace adds to the product's own: 0 also where its last workgroup adds the parts up. */
+/* Launches that the use of that workspace can add to the product's own, the tuning table's entry considered: 0 also where its last workgroup
+ * adds the parts up. */
 int mhip_gemm_workspace_launches(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b, int dtype);
 int mhip_gemm_ws(void* stream, const void* a, const void* b, const void* bias, const void* residual, void* c,
                  int64_t M, int64_t N, int64_t K, int64_t batch, int64_t stride_a, int64_t stride_b,

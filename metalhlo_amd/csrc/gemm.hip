@@ -725,6 +725,10 @@ extern "C" int64_t mhip_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t 
 extern "C" int mhip_gemm_workspace_launches(int64_t M, int64_t N, int64_t K, int64_t batch, int trans_a, int trans_b, int dtype) {
     if (mhip_gemm_workspace(M, N, K, batch, trans_a, trans_b, dtype) == 0) return 0;
     const bool is16 = dtype == MHIP_BF16 || dtype == MHIP_F16, vec = is16 && (trans_a ? M : K) % 8 == 0 && (trans_b ? K : N) % 8 == 0;
+    GemmArgs g;
+    g.M = (int)M; g.N = (int)N; g.K = (int)K;
+    // (a table entry sends the product to a tile, whose parts a launch of its own adds up)
+    if (vec && !few_row_choice(tuned_gemm_variant(g, batch, trans_a, trans_b, dtype))) return 1;
     if (vec && gemm_parts_wanted(M, N, K, batch, trans_a, trans_b)) return 0;
     return few_rows(M, N, K, batch, trans_a, trans_b, is16, vec) ? 0 : 1;
 }

@@ -40,6 +40,19 @@ def test_tuning_table_round_trip(lib, tmp_path):
     assert lib.mhip_tuning_device()            # "nodevice/0" here, "<arch>/<compute units>" on a GPU
 
 
+def test_an_entry_counts_in_the_launches_of_a_product(lib):
+    """Few rows have their parts of K added up in their own launch, unless the table sends them to a tile."""
+    lib.mhip_tuning_clear()
+    few, parts = (4, 4096, 2560, 1, 0, 0, 3), (4, 4096, 4096, 1, 0, 0, 3)
+    for size in (few, parts):
+        assert lib.mhip_gemm_workspace(*size) > 0 and lib.mhip_gemm_workspace_launches(*size) == 0
+        for variant, launches in ((128, 0), (2569, 1), (256, 1)):
+            assert lib.mhip_tuning_set_gemm(*size, variant, 1.0) == 0
+            assert lib.mhip_gemm_workspace_launches(*size) == launches, variant
+    lib.mhip_tuning_clear()
+    assert lib.mhip_gemm_workspace_launches(*few) == 0
+
+
 def _as64(t):
     return t.float().cpu().numpy().astype(np.float64)
 
