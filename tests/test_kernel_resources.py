@@ -36,7 +36,8 @@ def _kernels():
 
 
 @pytest.mark.parametrize("name", ["fa_flow_kernel", "gemm_f32_ring_kernel", "gemm_mid_kernel", "gemm192_kernel", "linear_w32_kernel",
-                                  "linear_w32_stream_kernel", "tied_head_kernel", "row_any_kernelIDF16bLi0E", "row_any_kernelIDF16_Li0E"])
+                                  "linear_w32_stream_kernel", "tied_head_kernel", "gemm_strip_kernel", "gemm_parts_kernel", "fa_short_kernel", "fa_decode_kernel",
+                                  "row_any_kernelIDF16bLi0E", "row_any_kernelIDF16_Li0E"])
 def test_nothing_is_spilled(name):
     if not os.path.exists(LIB):
         pytest.skip("no built library")
