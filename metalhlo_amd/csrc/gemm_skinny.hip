@@ -314,7 +314,7 @@ bool wide_strips(int64_t N, int64_t K, int64_t batch, bool tb) {
 //   [48,768] x K 3072  15.2 | 11.9 / 4 (192) | 13.1 / 4 (192)      [128,1024] x K 4096 24.3 | 24.6 / 1 (176) | 19.8 / 2 (256)
 //   [64,1024] x K 4096 17.0 | -              | 14.8 / 4 (256)      [70,1024] x K 4096  23.4 | 21.8 / 2 (220) | 19.7 / 2 (192)
 // Shorter: [40,2048] x K 2048 12.3 | 14.4, [60,3000] x K 2500 22.4 | 24.1, [150,512] x K 2048 11.9 | 12.6, [128,768] x K 3072 16.6 | 15.1
-// for one more launch; below 216 workgroups: [160,640] x K 2560 15.0 whole | - | 15.9 / 2 (200).
+// (all of these with a launch of its own for the parts, when the lines were drawn); below 216 workgroups: [160,640] x K 2560 15.0 whole | - | 15.9 / 2 (200).
 struct RowsPlan { int rows = 0, cols = 0, splits = 1; };
 RowsPlan rows_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool tb) {
     RowsPlan best;
