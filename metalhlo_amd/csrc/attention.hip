@@ -531,7 +531,7 @@ static int fa_entry(const char* name, void* stream, const void* q, const void* k
     a.negate_q = scale < 0.f;
     a.is_causal = is_causal ? 1 : 0;
     a.mask_sb = mask_stride_b; a.mask_sh = mask_stride_h;
-    a.nqb = 0; a.xcd_map = 0; a.pair_tiles = 0; a.cu_group = 1;
+    a.nqb = 0; a.pair_tiles = 0; a.cu_group = 1;
     const int64_t packed[12] = {H * Sq * D, Sq * D, D, H * Skv * D, Skv * D, D, H * Skv * D, Skv * D, D, H * Sq * D, Sq * D, D};
     bool is_packed = true;
     int64_t max_row = D, max_span = 0;

@@ -74,15 +74,11 @@ __global__ __launch_bounds__(256, 1) void fa_pipe_kernel(FaArgs a) {
     const int slots = paired ? (a.nqb + 1) / 2 : a.nqb;
     int bh, slot;
     {
-        const int id = blockIdx.x;
-        if (a.xcd_map) {
-            const int xcd = id & 7, local = id >> 3;
-            bh = (local / slots) * 8 + xcd;
-            slot = local % slots;
-        } else {
-            bh = id / slots;
-            slot = id % slots;
-        }
+        // an XCD (ids go round-robin over the eight) takes every eighth head; the up to seven that are left over are dealt out by tiles
+        const int id = blockIdx.x, xcd = id & 7, local = id >> 3, heads = (a.B * a.H) >> 3;
+        const int rest = id - 8 * heads * slots;
+        bh = rest < 0 ? (local / slots) * 8 + xcd : 8 * heads + rest / slots;
+        slot = rest < 0 ? local % slots : rest % slots;
     }
     const int npass = (paired && slot != a.nqb - 1 - slot) ? 2 : 1;
 #pragma nounroll
@@ -319,7 +315,6 @@ int launch_pipe(hipStream_t s, FaArgs a, int pair) {
                     hipGetErrorString(attr_err));
     a.nqb = (a.Sq + kPBQ - 1) / kPBQ;
     const int64_t bh = (int64_t)a.B * a.H;
-    a.xcd_map = (bh % 8 == 0) ? 1 : 0;
     // pairing halves the number of workgroups: only when they still fill the chip
     const int pair_env = pair >= 0 ? pair : tune_int("MHIP_FA_PAIR", -1);
     a.pair_tiles = CAUSAL && (pair_env >= 0 ? pair_env != 0 : bh * ((a.nqb + 1) / 2) >= 256);
