@@ -271,7 +271,7 @@ __global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* 
     float* const weights = &sums[0][0][0][0];                // [kMaxSq][64]
     float* const inverse = weights + kMaxSq * 64;            // [kMaxSq]
     float* const shares = inverse + 64;                      // [sharers][Sq][D]
-    static_assert((kMaxSq * 64 + 64 + kMaxSq * D) * 4 <= (int)sizeof(sums) && kSlots <= kMaxSq, "in place of the waves' sums");
+    static_assert((kMaxSq * 64 + 64 + (kSlots > kMaxSq ? kSlots : kMaxSq) * D) * 4 <= (int)sizeof(sums), "in place of the waves' sums");
     int together = 1;                                        // queries at a time, a power of two
     while (together < a.Sq && together < kSlots) together *= 2;
     const int sharers = min(kSlots / together, 4), group = threadIdx.x % kGroups, slot = threadIdx.x / kGroups, first = slot / together;
@@ -334,25 +334,42 @@ __global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* 
     }
 }
 
-// Parts of the key range: enough workgroups for two per compute unit, each with at least part_keys().
-int decode_parts(int64_t bh, int64_t Skv) {
-    const int64_t want = (512 + bh - 1) / bh, most = Skv / part_keys(Skv);
-    const int64_t n = want < most ? want : most;
-    return n < 2 ? 1 : n > 64 ? 64 : (int)n;
+// How a launch's keys are dealt: parts of the range, keys a part, waves of a workgroup.
+struct DecodePlan { int parts, per, waves; };
+
+DecodePlan decode_plan(int64_t bh, int64_t Skv) {
+    auto dealt = [&](int64_t want, int waves) {
+        const int64_t unit = part_keys(Skv), most = Skv / unit, n = want < most ? want : most;
+        const int parts = n < 2 ? 1 : n > 64 ? 64 : (int)n;
+        return DecodePlan{parts, parts == 1 ? (int)Skv : (int)(((Skv + parts - 1) / parts + unit - 1) / unit * unit), waves};
+    };
+    // Workgroups of eight waves, one a compute unit, where whole parts of all heads fill three quarters of the units and eight waves have
+    // a block of keys: half as many parts to write and to put together as with two workgroups of four waves a unit, which is what
+    // the others take.  us, four | eight waves, one query: 8 heads over 16384 keys of head size 128 23.0 | 17.7 (eight queries 26.3 | 19.2), 32 over 4096
+    // 15.8 | 14.7, 192 over 700 16.3 | 13.2, 256 over 4096 93.9 | 93.2, of 64 48.8 | 46.1, 12 over 5632 of 64 11.3 | 9.1, 12 over 300 5.1 | 4.8; of more heads a
+    // second turn ([32,12,1000] of 64, four queries, 21.2 | 22.6, 512 over 4096 177 | 179); parts of 128 keys 24 over 1024 of 64 6.1 | 6.4.
+    if (bh <= 256 && 256 / bh * bh >= 192) {
+        const DecodePlan p = dealt(256 / bh, 8);
+        if (p.per > 4 * kKeys) return p;
+    }
+    return dealt((512 + bh - 1) / bh, 4);
+}
+
+template <typename T, int D, int WAVES>
+int launch_waves(hipStream_t s, const FaArgs& a, float* part, const DecodePlan& plan) {
+    const int64_t bh = (int64_t)a.B * a.H;
+    const dim3 grid((unsigned)bh, (unsigned)((a.Skv + plan.per - 1) / plan.per));
+    uint64_t* words = reinterpret_cast<uint64_t*>(part + (int64_t)plan.parts * bh * a.Sq * (D + 2));
+    const uint64_t tag = plan.parts > 1 ? launch_tag() : 0;
+    if (plan.parts == 1) part = nullptr;
+    if (a.mask) hipLaunchKernelGGL((fa_decode_kernel<T, D, true, WAVES>), grid, dim3(64 * WAVES), 0, s, a, part, plan.per, words, tag);
+    else hipLaunchKernelGGL((fa_decode_kernel<T, D, false, WAVES>), grid, dim3(64 * WAVES), 0, s, a, part, plan.per, words, tag);
+    return check_launch("flash_attention_decode");
 }
 
 template <typename T, int D>
-int launch(hipStream_t s, const FaArgs& a, float* part, int parts) {
-    const int64_t bh = (int64_t)a.B * a.H;
-    const int per = parts == 1 ? a.Skv : (int)(((a.Skv + parts - 1) / parts + part_keys(a.Skv) - 1) / part_keys(a.Skv) * part_keys(a.Skv));
-    const dim3 grid((unsigned)bh, (unsigned)((a.Skv + per - 1) / per));
-    constexpr int WAVES = 4;
-    uint64_t* words = reinterpret_cast<uint64_t*>(part + (int64_t)parts * bh * a.Sq * (D + 2));
-    const uint64_t tag = parts > 1 ? launch_tag() : 0;
-    if (parts == 1) part = nullptr;
-    if (a.mask) hipLaunchKernelGGL((fa_decode_kernel<T, D, true, WAVES>), grid, dim3(64 * WAVES), 0, s, a, part, per, words, tag);
-    else hipLaunchKernelGGL((fa_decode_kernel<T, D, false, WAVES>), grid, dim3(64 * WAVES), 0, s, a, part, per, words, tag);
-    return check_launch("flash_attention_decode");
+int launch(hipStream_t s, const FaArgs& a, float* part, const DecodePlan& plan) {
+    return plan.waves == 8 ? launch_waves<T, D, 8>(s, a, part, plan) : launch_waves<T, D, 4>(s, a, part, plan);
 }
 
 }  // namespace
@@ -362,16 +379,17 @@ bool fa_decode_eligible(const FaArgs& a) { return a.Sq <= kMaxSq && !a.is_causal
 
 int64_t fa_decode_workspace(int64_t bh, int64_t Sq, int64_t Skv, int64_t D) {
     if (Sq < 1 || Sq > kMaxSq || (D != 64 && D != 128)) return 0;
-    const int parts = decode_parts(bh, Skv);
+    const int parts = decode_plan(bh, Skv).parts;
     return parts == 1 ? 0 : parts * bh * Sq * (D + 2) * 4 + bh * 8;
 }
 
 int launch_fa_decode(hipStream_t s, const FaArgs& a, int64_t D, int dtype, void* workspace, int64_t workspace_bytes) {
     const int64_t bh = (int64_t)a.B * a.H, need = fa_decode_workspace(bh, a.Sq, a.Skv, D);
-    const int parts = need > 0 && workspace && need <= workspace_bytes ? decode_parts(bh, a.Skv) : 1;
+    DecodePlan plan = decode_plan(bh, a.Skv);
+    if (!workspace || need > workspace_bytes) { plan.parts = 1; plan.per = a.Skv; }
     float* part = static_cast<float*>(workspace);
-    if (dtype == MHIP_BF16) return D == 128 ? launch<bf16_t, 128>(s, a, part, parts) : launch<bf16_t, 64>(s, a, part, parts);
-    return D == 128 ? launch<f16_t, 128>(s, a, part, parts) : launch<f16_t, 64>(s, a, part, parts);
+    if (dtype == MHIP_BF16) return D == 128 ? launch<bf16_t, 128>(s, a, part, plan) : launch<bf16_t, 64>(s, a, part, plan);
+    return D == 128 ? launch<f16_t, 128>(s, a, part, plan) : launch<f16_t, 64>(s, a, part, plan);
 }
 
 }  // namespace mhip
