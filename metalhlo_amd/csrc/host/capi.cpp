@@ -269,7 +269,9 @@ static MHLOStatusCode make_buffer(MHLOClientRef client, const void* data, size_t
         if (init && t.bytes()) {
             // explicit host -> device copy on the client's stream (the reference relies on unified memory)
             std::lock_guard<std::mutex> stream_lock(c->stream_mu);      // not into another thread's graph capture
-            if (hipMemcpyAsync(d.data(), data, t.bytes(), hipMemcpyHostToDevice, c->stream) != hipSuccess ||
+            const void* from = data;
+            if (char* pinned = c->staging_for(t.bytes())) from = memcpy(pinned, data, t.bytes());
+            if (hipMemcpyAsync(d.data(), from, t.bytes(), hipMemcpyHostToDevice, c->stream) != hipSuccess ||
                 hipStreamSynchronize(c->stream) != hipSuccess) {
                 (void)hipGetLastError();
                 throw BufferError("host to device copy failed");
@@ -324,11 +326,13 @@ MHLOStatusCode mhlo_buffer_to_host(MHLOBufferRef buffer, void* out_data, size_t 
     clear_error();
     if (need == 0) return MHLO_OK;
     std::lock_guard<std::mutex> stream_lock(h->client->stream_mu);      // not into another thread's graph capture
-    if (hipMemcpyAsync(out_data, h->t.data(), need, hipMemcpyDeviceToHost, h->client->stream) != hipSuccess ||
+    char* const pinned = h->client->staging_for(need);
+    if (hipMemcpyAsync(pinned ? pinned : out_data, h->t.data(), need, hipMemcpyDeviceToHost, h->client->stream) != hipSuccess ||
         hipStreamSynchronize(h->client->stream) != hipSuccess) {
         (void)hipGetLastError();
         return set_error(MHLO_ERROR_TRANSFER_FAILED, "device to host copy failed");
     }
+    if (pinned) memcpy(out_data, pinned, need);
     return MHLO_OK;
 }
 

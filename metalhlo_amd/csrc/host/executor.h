@@ -89,7 +89,25 @@ struct Client {
     // capturing state; this client captures nothing further (every execution is eager).
     hipStream_t capture_stream = nullptr;
     bool capture_broken = false;
-    ~Client() { if (capture_stream && !capture_broken) (void)hipStreamDestroy(capture_stream); }
+    // Transfers of up to kStagingBytes go through pinned memory of the client's, allocated at the first of them: the runtime takes longer over host
+    // memory that it does not know than a copy in front of or behind the transfer does.  For the holder of stream_mu, who waits for the
+    // transfer before it is let go.  NULL: `bytes` are too many, or there is no such memory.
+    static constexpr size_t kStagingBytes = 512 << 10;
+    char* staging = nullptr;
+    bool no_staging = false;
+    char* staging_for(size_t bytes) {
+        if (bytes > kStagingBytes || no_staging) return nullptr;
+        if (!staging && hipHostMalloc(reinterpret_cast<void**>(&staging), kStagingBytes, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            staging = nullptr;
+            no_staging = true;
+        }
+        return staging;
+    }
+    ~Client() {
+        if (capture_stream && !capture_broken) (void)hipStreamDestroy(capture_stream);
+        if (staging) (void)hipHostFree(staging);
+    }
     DevicePool pool;
     DeviceTensor allocate(const TensorType& t);
 };
