@@ -156,16 +156,27 @@ __global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* 
             oacc[f] = Mfma16A<T>::run(vf, pb, oacc[f]);
         }
     };
-    int key = k0 + wave * kKeys;
-    if (key < k1) {
+    // Blocks of this wave, in a ring from one that a hash of head and part chooses (head size 128): workgroups that all walk from the start of their
+    // keys are a power of two apart where caches are as long as one, and meet in the same banks of the memory.  (A start that
+    // grows with the head can be worse, 64 heads over 8192 keys 50.6 -> 65 us.)  us, from the first block | so, one query: 256 heads over 4096 keys
+    // 93.2 | 89.6, over 2048 49.1 | 47.6, 96 over 4096 40.1 | 37.8, 64 over 8192 50.6 | 49.0, 192 over 3000 53.5 | 51.8, 256 over 4000 89.6 | 89.2, 512 over 4096
+    // 177 | 175; head size 64, whose rows are a line each, lost by it: 128 over 8192 48.4 | 49.4.
+    constexpr int kStride = WAVES * kKeys;
+    const int base = k0 + wave * kKeys;
+    if (base < k1) {
+        int left = (k1 - base + kStride - 1) / kStride, key = base;
+        if (D == 128 && left >= 4) key += (int)(((uint32_t)(bh * 64 + (int)blockIdx.y) * 2246822519u >> 24) * (uint32_t)left >> 8) * kStride;
         Block cur;
         load(cur, key);
-        for (; key < k1; key += WAVES * kKeys) {
+        for (;;) {
             Block nxt;
-            const bool more = key + WAVES * kKeys < k1;
-            if (more) load(nxt, key + WAVES * kKeys);
+            const int next = key + kStride < k1 ? key + kStride : base;
+            const bool more = --left > 0;
+            if (more) load(nxt, next);
             attend(cur, key);
-            if (more) cur = nxt;
+            if (!more) break;
+            cur = nxt;
+            key = next;
         }
     }
 
@@ -337,7 +348,7 @@ __global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* 
 // How a launch's keys are dealt: parts of the range, keys a part, waves of a workgroup.
 struct DecodePlan { int parts, per, waves; };
 
-DecodePlan decode_plan(int64_t bh, int64_t Skv) {
+DecodePlan decode_plan(int64_t bh, int64_t Sq, int64_t Skv) {
     auto dealt = [&](int64_t want, int waves) {
         const int64_t unit = part_keys(Skv), most = Skv / unit, n = want < most ? want : most;
         const int parts = n < 2 ? 1 : n > 64 ? 64 : (int)n;
@@ -350,7 +361,7 @@ DecodePlan decode_plan(int64_t bh, int64_t Skv) {
     // second turn ([32,12,1000] of 64, four queries, 21.2 | 22.6, 512 over 4096 177 | 179); parts of 128 keys 24 over 1024 of 64 6.1 | 6.4.
     if (bh <= 256 && 256 / bh * bh >= 192) {
         const DecodePlan p = dealt(256 / bh, 8);
-        if (p.per > 4 * kKeys) return p;
+        if (p.per > (Sq > 8 ? 8 : 4) * kKeys) return p;      // (16 queries of 16 heads over 2048 10.9 | 11.0)
     }
     return dealt((512 + bh - 1) / bh, 4);
 }
@@ -379,13 +390,13 @@ bool fa_decode_eligible(const FaArgs& a) { return a.Sq <= kMaxSq && !a.is_causal
 
 int64_t fa_decode_workspace(int64_t bh, int64_t Sq, int64_t Skv, int64_t D) {
     if (Sq < 1 || Sq > kMaxSq || (D != 64 && D != 128)) return 0;
-    const int parts = decode_plan(bh, Skv).parts;
+    const int parts = decode_plan(bh, Sq, Skv).parts;
     return parts == 1 ? 0 : parts * bh * Sq * (D + 2) * 4 + bh * 8;
 }
 
 int launch_fa_decode(hipStream_t s, const FaArgs& a, int64_t D, int dtype, void* workspace, int64_t workspace_bytes) {
     const int64_t bh = (int64_t)a.B * a.H, need = fa_decode_workspace(bh, a.Sq, a.Skv, D);
-    DecodePlan plan = decode_plan(bh, a.Skv);
+    DecodePlan plan = decode_plan(bh, a.Sq, a.Skv);
     if (!workspace || need > workspace_bytes) { plan.parts = 1; plan.per = a.Skv; }
     float* part = static_cast<float*>(workspace);
     if (dtype == MHIP_BF16) return D == 128 ? launch<bf16_t, 128>(s, a, part, plan) : launch<bf16_t, 64>(s, a, part, plan);
