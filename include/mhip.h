@@ -198,6 +198,12 @@ int64_t mhip_linear_w32_workspace(int64_t M, int64_t N, int64_t K);
 int mhip_linear_w32_layer(void* stream, const void* x, const float* gamma, const float* beta, float eps, const float* w, const float* bias,
                           const void* residual, void* c, int64_t M, int64_t N, int64_t K, int activation, int dtype, void* workspace,
                           int64_t workspace_bytes, int n_ahead, const mhip_weights* ahead);
+/* The fp32 sums sums[parts][B S][N] of causal_attention(qkv) . round(w) for mhip_finish_norm: qkv [B S, 3 H D] in BF16 or F16 with heads of 64 (scale
+ * 1 / 8), w [H D, N] in fp32, a part being the heads that mhip_attend_project_parts deals to one (0: not served; up to 64 rows in all).
+ * 16-byte aligned pointers; `ahead` as in mhip_linear_w32. */
+int mhip_attend_project_parts(int64_t B, int64_t S, int64_t H, int64_t D, int64_t N, int dtype);
+int mhip_attend_project(void* stream, const void* qkv, const float* w, float* sums, int64_t B, int64_t S, int64_t H, int64_t D, int64_t N, int dtype,
+                        int n_ahead, const mhip_weights* ahead);
 
 /* Attention -------------------------------------------------------------- */
 

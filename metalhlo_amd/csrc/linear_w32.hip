@@ -15,8 +15,11 @@
 //     will want them (fetch_ahead): [37,768] x [768,2304] 7.3 -> 5.0 us, those workgroups included.
 // Workgroups of one XCD take neighbouring strips, so a 128-byte line of W that two strips share is fetched once.
 #include <initializer_list>
+#include <mutex>
+#include <type_traits>
 
 #include "arrive.h"
+#include "attention_short.h"
 #include "gemm_lds.h"
 
 namespace mhip {
@@ -38,8 +41,15 @@ struct LinearArgs {
     uint64_t *words, tag;             // with sums: the last part to arrive adds them up to c (arrive.h)
     int M, N, K, act, splits;
     int strips, per_xcd, blocks, first;      // first: workgroups in front of the product's
+    int part_steps, per;              // k steps of a part and of a wave
+    uint32_t by_blocks, by_splits;    // divided(n, .): n / blocks, n / splits
     Band ahead[kAhead];
 };
+
+// A launch here is a few hundred instructions a wave, 2 to 3 ns each where nothing overlaps them, and a division is 25 of them: the ones that a
+// workgroup needs to find its place are formed by a multiplication (exact for numbers below 2^32 / n; GPT-2-small over 37 tokens 446 -> 436 us).
+inline uint32_t divisor(int n) { return n == 1 ? 0 : (uint32_t)((((uint64_t)1 << 32) + n - 1) / n); }
+__device__ __forceinline__ int divided(int n, uint32_t by) { return by ? (int)__umulhi((uint32_t)n, by) : n; }
 
 template <typename T>
 __device__ __forceinline__ float rounded(float v) { return Elem<T>::to_f32(Elem<T>::from_f32(v)); }
@@ -79,18 +89,15 @@ __global__ __launch_bounds__(64 * kWaves, LOOP ? 2 : 4) void linear_w32_kernel(L
     }
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int li = lane & 15, lg = lane >> 4;
-    const int id = (int)blockIdx.x - g.first, xcd = id % kXcds;
-    int local = id / kXcds;
-    const int m0 = local % g.blocks * (16 * MT);
-    local /= g.blocks;
-    const int split = local % g.splits, strip = xcd * g.per_xcd + local / g.splits, n0 = strip * 16;
+    const uint32_t id = blockIdx.x - (uint32_t)g.first;
+    const int xcd = id % kXcds, local = id / kXcds, column = divided(local, g.by_blocks), m0 = (local - column * g.blocks) * (16 * MT);
+    const int place = divided(column, g.by_splits), split = column - place * g.splits, strip = xcd * g.per_xcd + place, n0 = strip * 16;
     if (strip >= g.strips) return;
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(g.x, (uint32_t)((int64_t)g.M * g.K * 2));
     const __amdgpu_buffer_rsrc_t rw = make_rsrc(g.w, (uint32_t)((int64_t)g.N * g.K * 4));
 
     // ---- this wave's share of the k steps
-    const int all = (g.K + KS - 1) / KS, part_steps = (all + g.splits - 1) / g.splits, p0 = split * part_steps, p1 = min(all, p0 + part_steps);
-    const int per = (part_steps + kWaves - 1) / kWaves, s0 = p0 + wave * per, s1 = min(p1, s0 + per);
+    const int all = (g.K + KS - 1) / KS, p0 = split * g.part_steps, p1 = min(all, p0 + g.part_steps), s0 = p0 + wave * g.per, s1 = min(p1, s0 + g.per);
     uint64_t* const word = ARRIVE ? g.words + strip * g.blocks + m0 / (16 * MT) : nullptr;
     uint64_t seen = 0;
     if (ARRIVE && threadIdx.x == 0) seen = arrive_look(word);
@@ -134,13 +141,13 @@ __global__ __launch_bounds__(64 * kWaves, LOOP ? 2 : 4) void linear_w32_kernel(L
     load(cur, s0);
 
     // ---- the epilogue's thread (wave = mt, li, lg) finishes row li of group mt: columns 4 lg .. 4 lg + 3 of the strip
-    const int fm = m0 + wave * 16 + li, column = n0 + 4 * lg;
+    const int fm = m0 + wave * 16 + li, col = n0 + 4 * lg;
     const bool finisher = wave < MT && fm < g.M;
     f32x4 bias = {0.f, 0.f, 0.f, 0.f};
     u32x2 res = {0, 0};
-    if (finisher && column < g.N) {
-        if (g.bias) bias = *reinterpret_cast<const f32x4*>(g.bias + column);
-        if (g.residual) res = *reinterpret_cast<const u32x2*>(static_cast<const T*>(g.residual) + (int64_t)fm * g.N + column);
+    if (finisher && col < g.N) {
+        if (g.bias) bias = *reinterpret_cast<const f32x4*>(g.bias + col);
+        if (g.residual) res = *reinterpret_cast<const u32x2*>(static_cast<const T*>(g.residual) + (int64_t)fm * g.N + col);
     }
 
     if constexpr (NORM) {
@@ -256,25 +263,25 @@ __global__ __launch_bounds__(64 * kWaves, LOOP ? 2 : 4) void linear_w32_kernel(L
     f32x4 sum = part[(ARRIVE ? min(wave, MT - 1) : wave) * 64 + lane];
 #pragma unroll
     for (int w = 1; w < kWaves; w++) sum += part[(w * MT + (ARRIVE ? min(wave, MT - 1) : wave)) * 64 + lane];
-    const bool mine = finisher && column < g.N;
+    const bool mine = finisher && col < g.N;
     if constexpr (ARRIVE) {
         __shared__ int last;
         const __amdgpu_buffer_rsrc_t rp = parts_rsrc(g.sums);
-        if (mine) store_part(rp, (uint32_t)(((split * g.M + fm) * g.N + column) * 4), sum);
+        if (mine) store_part(rp, (uint32_t)(((split * g.M + fm) * g.N + col) * 4), sum);
         if (!arrive_last(word, g.splits, &last) || !mine) return;
         f32x4 v[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) v[i] = load_part(rp, i < g.splits ? (uint32_t)(((i * g.M + fm) * g.N + column) * 4) : kOob);
+        for (int i = 0; i < 8; i++) v[i] = load_part(rp, i < g.splits ? (uint32_t)(((i * g.M + fm) * g.N + col) * 4) : kOob);
         sum = v[0];
 #pragma unroll
         for (int i = 1; i < 8; i++) sum += v[i];
     }
     if (!mine) return;
     if (!ARRIVE && g.sums) {
-        *reinterpret_cast<f32x4*>(g.sums + ((int64_t)split * g.M + fm) * g.N + column) = sum;
+        *reinterpret_cast<f32x4*>(g.sums + ((int64_t)split * g.M + fm) * g.N + col) = sum;
         return;
     }
-    T* c = static_cast<T*>(g.c) + (int64_t)fm * g.N + column;
+    T* c = static_cast<T*>(g.c) + (int64_t)fm * g.N + col;
     dispatch_act(g.act, [&](auto act_tag) {
         constexpr int ACT = decltype(act_tag)::value;
         Pack4<T> o, r = __builtin_bit_cast(Pack4<T>, res);
@@ -380,20 +387,91 @@ __global__ __launch_bounds__(64 * kWaves, MT < 2 ? 4 : 2) void linear_w32_stream
     }
 }
 
+// Causal attention of a short prompt and the projection behind it: fp32 sums [part][M][N] of attention(x) . round(W), a part being `group` heads of size 64
+// (their 64 group rows of W), for the launch that adds parts up.  Two launches that depend on one another cost 1.6 us between them and a trip of
+// the attention's result past the L2s; what it takes to have it in every workgroup, 14 KB of x a head, comes from an L2 while W, which
+// is fetched first, is on its way.  (GPT-2-small, against two launches: 37 tokens 453.5 -> 446.4 us, 2 x 20 452.7 -> 442.9.  A workgroup's waves take the heads of a part
+// in one turn: with two, 4 x 12 tokens went from 462 to 465.)
+// A workgroup owns 32 columns and a part: each wave takes 32 queries of a head, leaves the result in LDS, rounded as the attention kernel
+// rounds it, and then takes 32 k of W.
+constexpr int kProjectCols = 32, kProjectHead = 64;
+template <typename T, int MT>
+__global__ __launch_bounds__(64 * kWaves) void attend_project_kernel(FaArgs a, LinearArgs g, int group) {
+    constexpr int NF = kProjectCols / 16, kValues = 64 * kProjectHead * 2;      // bytes of values a wave holds at once
+    extern __shared__ __attribute__((aligned(1024))) char smem[];
+    if ((int)blockIdx.x < g.first) {
+        fetch_ahead(g, blockIdx.x);
+        return;
+    }
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 15, lg = lane >> 4;
+    // the columns of an XCD's strips are those that fetch_ahead gives its L2
+    const uint32_t id = blockIdx.x - (uint32_t)g.first;
+    const int xcd = id % kXcds, place = divided(id / kXcds, g.by_splits), part = id / kXcds - place * g.splits;
+    const int n0 = xcd * g.per_xcd * 16 + place * kProjectCols, n1 = min(g.N, (xcd + 1) * g.per_xcd * 16);
+    if (n0 >= n1) return;
+    const int depth = group * kProjectHead, pitch = depth * 2 + 16;
+    char* const rows = smem + kWaves * kValues;              // the attention's result, [M][depth]
+    const bool active = wave * 32 < depth;
+
+    float wn[NF][8];
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(g.w, (uint32_t)((int64_t)g.N * g.K * 4));
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+        const int n = n0 + 16 * f + li, k = part * depth + wave * 32 + lg * 8;
+        const uint32_t off = active && n < n1 ? (uint32_t)(((int64_t)k * g.N + n) * 4) : kOob;
+#pragma unroll
+        for (int j = 0; j < 8; j++) wn[f][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rw, off + (uint32_t)(j * g.N * 4), 0, 0));
+    }
+
+    // (a wave's 32 queries: half of sequence b, head h of the group; by_blocks divides by the sequences)
+    const int halves = a.Sq > 32 ? 2 : 1, pair = wave >> (halves - 1), h = divided(pair, g.by_blocks), b = pair - h * a.B, half = wave & (halves - 1);
+    if (h < group) {
+        auto store = [&](int query, int d, u32x2 v) __attribute__((always_inline)) {
+            *reinterpret_cast<u32x2*>(rows + (b * a.Sq + query) * pitch + (h * kProjectHead + d) * 2) = v;
+        };
+        if (half) short_rows<T, kProjectHead, 2>(a, b * a.H + part * group + h, smem + wave * kValues, store);
+        else short_rows<T, kProjectHead, 1>(a, b * a.H + part * group + h, smem + wave * kValues, store);
+    }
+    __syncthreads();
+
+    // (rows past the last hold whatever LDS held: each is a row of the product of its own, and not stored)
+    f32x4* const sums = reinterpret_cast<f32x4*>(smem);      // [wave][MT][NF], where the values were
+    if (active) {
+        u32x4 w[NF];
+#pragma unroll
+        for (int f = 0; f < NF; f++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) w[f][j] = round_pair<T>(wn[f][2 * j], wn[f][2 * j + 1]);
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            const u32x4 x = *reinterpret_cast<const u32x4*>(rows + (mt * 16 + li) * pitch + (wave * 32 + lg * 8) * 2);
+#pragma unroll
+            for (int f = 0; f < NF; f++) sums[((wave * MT + mt) * NF + f) * 64 + lane] = Tile16<T>::run(w[f], x, f32x4{0.f, 0.f, 0.f, 0.f});
+        }
+    }
+    __syncthreads();
+    if (wave >= MT * NF) return;
+    const int mt = wave / NF, f = wave % NF, m = mt * 16 + li, n = n0 + 16 * f + 4 * lg;
+    f32x4 sum = sums[(mt * NF + f) * 64 + lane];
+    for (int i = 1; i < depth / 32; i++) sum += sums[((i * MT + mt) * NF + f) * 64 + lane];
+    if (m < g.M && n < n1) *reinterpret_cast<f32x4*>(g.sums + ((int64_t)part * g.M + m) * g.N + n) = sum;
+}
+
 // A row per workgroup: x = round(sum of the parts + bias) + residual (or, without parts, the residual itself), stored to c
 // when that is given, and h = LayerNorm(x).  Latency-bound: two memory latencies, two barriers.
 constexpr int kFinishPieces = 4;      // four columns each, 256 threads: N <= 4096
-template <typename T>
+template <typename T, int PIECES>
 __global__ __launch_bounds__(256) void finish_norm_kernel(LinearArgs g, T* h) {
     __shared__ float red[2][4];
     const int64_t row = blockIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    f32x4 v[kFinishPieces];
-    u32x2 x[kFinishPieces];
-    f32x4 ga[kFinishPieces], be[kFinishPieces];
+    f32x4 v[PIECES];
+    u32x2 x[PIECES];
+    f32x4 ga[PIECES], be[PIECES];
     float s = 0.f;
 #pragma unroll
-    for (int p = 0; p < kFinishPieces; p++) {
+    for (int p = 0; p < PIECES; p++) {
         const int n = (p * 256 + (int)threadIdx.x) * 4;
         v[p] = f32x4{0.f, 0.f, 0.f, 0.f};
         x[p] = u32x2{0, 0};
@@ -433,19 +511,31 @@ __global__ __launch_bounds__(256) void finish_norm_kernel(LinearArgs g, T* h) {
     const float mean = over_row(s, 0) / (float)g.N;
     float q = 0.f;
 #pragma unroll
-    for (int p = 0; p < kFinishPieces; p++)
+    for (int p = 0; p < PIECES; p++)
         if ((p * 256 + (int)threadIdx.x) * 4 < g.N)
 #pragma unroll
             for (int e = 0; e < 4; e++) { v[p][e] -= mean; q = fmaf(v[p][e], v[p][e], q); }
     const float rstd = 1.f / sqrtf(over_row(q, 1) / (float)g.N + g.eps);
 #pragma unroll
-    for (int p = 0; p < kFinishPieces; p++) {
+    for (int p = 0; p < PIECES; p++) {
         const int n = (p * 256 + (int)threadIdx.x) * 4;
         if (n >= g.N) continue;
         Pack4<T> o;
 #pragma unroll
         for (int e = 0; e < 4; e++) o.v[e] = Elem<T>::from_f32(fmaf(v[p][e] * rstd, rounded<T>(ga[p][e]), rounded<T>(be[p][e])));
         *reinterpret_cast<u32x2*>(h + row * g.N + n) = __builtin_bit_cast(u32x2, o);
+    }
+}
+
+// The workgroups that fetch g.ahead, in front of a launch's own.
+void plan_ahead(LinearArgs& g) {
+    g.first = 0;
+    for (Band& a : g.ahead) {
+        a.cols = ((a.N + 15) / 16 + kXcds - 1) / kXcds * 16;
+        const int64_t pieces = (int64_t)a.cols / 4 * a.K, per_wg = 64 * kWaves * kAheadLoads;
+        a.wgs = a.w ? (int)((pieces + per_wg - 1) / per_wg) : 0;
+        a.magic = a.w ? (uint32_t)((((uint64_t)1 << 32) + a.cols / 4 - 1) / (a.cols / 4)) : 0;
+        g.first += kXcds * a.wgs;
     }
 }
 
@@ -457,14 +547,11 @@ int launch_one(hipStream_t s, LinearArgs g) {
     g.blocks = (g.M + 16 * MT - 1) / (16 * MT);
     g.strips = (g.N + 15) / 16;
     g.per_xcd = (g.strips + kXcds - 1) / kXcds;
-    g.first = 0;
-    for (Band& a : g.ahead) {
-        a.cols = ((a.N + 15) / 16 + kXcds - 1) / kXcds * 16;
-        const int64_t pieces = (int64_t)a.cols / 4 * a.K, per_wg = 64 * kWaves * kAheadLoads;
-        a.wgs = a.w ? (int)((pieces + per_wg - 1) / per_wg) : 0;
-        a.magic = a.w ? (uint32_t)((((uint64_t)1 << 32) + a.cols / 4 - 1) / (a.cols / 4)) : 0;
-        g.first += kXcds * a.wgs;
-    }
+    plan_ahead(g);
+    g.part_steps = ((g.K + 31) / 32 + g.splits - 1) / g.splits;
+    g.per = (g.part_steps + kWaves - 1) / kWaves;
+    g.by_blocks = divisor(g.blocks);
+    g.by_splits = divisor(g.splits);
     const int64_t grid = g.first + (int64_t)kXcds * g.per_xcd * g.blocks * g.splits;
     if (grid > 0x7FFFFFFFLL) return fail(MHIP_ERR_UNSUPPORTED, "linear_w32: grid too large");
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * kWaves), kSums, s, g);
@@ -528,6 +615,56 @@ extern "C" int mhip_linear_w32_parts(int64_t M, int64_t N, int64_t K) {
 
 namespace mhip {
 namespace {
+// The matrices that can be fetched ahead; the others are left to the calls that read them.
+void take_ahead(LinearArgs& g, int n_ahead, const mhip_weights* ahead) {
+    for (int i = 0; i < n_ahead; i++)
+        if (ahead[i].w && ahead[i].N > 0 && ahead[i].K > 0 && ahead[i].N % 8 == 0 && ahead[i].N <= (1 << 16) && ahead[i].K <= (1 << 16) &&
+            ahead[i].N * ahead[i].K <= (1 << 23) && aligned16({ahead[i].w})) {
+            g.ahead[i].w = ahead[i].w; g.ahead[i].N = (int)ahead[i].N; g.ahead[i].K = (int)ahead[i].K;
+        }
+}
+
+// Heads a part of attend_project_kernel, 0 where it does not serve: a divisor of the heads of which up to four parts come, or eight where they are many;
+// 64 rows, and a wave for every 32 of a head's.
+int project_group(int64_t B, int64_t S, int64_t H) {
+    if (B < 1 || S < 1 || H < 1 || H > 32 || S > 64 || B * S > 64) return 0;
+    int group = 0;
+    for (int n = 1; n <= 4 && !group; n++)
+        if (H % n == 0 && H / n <= 4) group = n;
+    if (!group && H % 4 == 0) group = 4;
+    return group && group * B * ((S + 31) / 32) <= kWaves ? group : 0;
+}
+
+template <typename T, int MT>
+int launch_project(hipStream_t s, const FaArgs& a, LinearArgs g, int group) {
+    auto kern = attend_project_kernel<T, MT>;
+    constexpr int kMost = kWaves * 64 * kProjectHead * 2 + 64 * (4 * kProjectHead * 2 + 16);
+    static_assert(kWaves * MT * kProjectCols / 16 * 1024 <= kWaves * 64 * kProjectHead * 2, "the sums lie where the values were");
+    static std::once_flag once;
+    static hipError_t err = hipSuccess;
+    std::call_once(once, [&] { err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kMost); });
+    if (err != hipSuccess) return fail(MHIP_ERR_LAUNCH, "attend_project: cannot reserve %d bytes of LDS: %s", kMost, hipGetErrorString(err));
+    const int lds = kWaves * 64 * kProjectHead * 2 + MT * 16 * (group * kProjectHead * 2 + 16);
+    g.per_xcd = ((g.N + 15) / 16 + kXcds - 1) / kXcds;
+    plan_ahead(g);
+    g.by_splits = divisor(g.splits);
+    g.by_blocks = divisor(a.B);
+    const int64_t grid = g.first + (int64_t)kXcds * ((g.per_xcd + 1) / 2) * g.splits;
+    if (grid > 0x7FFFFFFFLL) return fail(MHIP_ERR_UNSUPPORTED, "attend_project: grid too large");
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * kWaves), lds, s, a, g, group);
+    return check_launch("attend_project");
+}
+
+template <typename T>
+int project_type(hipStream_t s, const FaArgs& a, const LinearArgs& g, int group) {
+    switch ((g.M + 15) / 16) {
+        case 1: return launch_project<T, 1>(s, a, g, group);
+        case 2: return launch_project<T, 2>(s, a, g, group);
+        case 3: return launch_project<T, 3>(s, a, g, group);
+        default: return launch_project<T, 4>(s, a, g, group);
+    }
+}
+
 int linear_entry(void* stream, const void* x, const float* w, const float* bias, const void* residual, void* c, int64_t M, int64_t N, int64_t K, int trans_b,
                  int activation, int dtype, const float* gamma, const float* beta, float eps, float* sums, uint64_t* words, int parts, int n_ahead,
                  const mhip_weights* ahead) {
@@ -544,11 +681,7 @@ int linear_entry(void* stream, const void* x, const float* w, const float* bias,
     g.x = x; g.w = w; g.bias = bias; g.residual = residual; g.c = c; g.sums = sums;
     g.M = (int)M; g.N = (int)N; g.K = (int)K; g.act = activation; g.splits = parts;
     g.gamma = gamma; g.beta = beta; g.eps = eps; g.words = words; g.tag = words ? launch_tag() : 0;
-    for (int i = 0; i < n_ahead; i++)
-        if (ahead[i].w && ahead[i].N > 0 && ahead[i].K > 0 && ahead[i].N % 8 == 0 && ahead[i].N <= (1 << 16) && ahead[i].K <= (1 << 16) &&
-            ahead[i].N * ahead[i].K <= (1 << 23) && aligned16({ahead[i].w})) {
-            g.ahead[i].w = ahead[i].w; g.ahead[i].N = (int)ahead[i].N; g.ahead[i].K = (int)ahead[i].K;
-        }
+    take_ahead(g, n_ahead, ahead);
     return dtype == MHIP_BF16 ? launch_type<bf16_t>(as_stream(stream), g, trans_b != 0) : launch_type<f16_t>(as_stream(stream), g, trans_b != 0);
 }
 
@@ -595,7 +728,44 @@ extern "C" int mhip_finish_norm(void* stream, const float* sums, int parts, cons
     LinearArgs g = {};
     g.sums = const_cast<float*>(sums); g.splits = parts; g.bias = bias; g.residual = residual; g.c = c; g.gamma = gamma; g.beta = beta;
     g.eps = eps; g.M = (int)M; g.N = (int)N;
-    if (dtype == MHIP_BF16) hipLaunchKernelGGL((finish_norm_kernel<bf16_t>), dim3((unsigned)M), dim3(256), 0, as_stream(stream), g, static_cast<bf16_t*>(h));
-    else hipLaunchKernelGGL((finish_norm_kernel<f16_t>), dim3((unsigned)M), dim3(256), 0, as_stream(stream), g, static_cast<f16_t*>(h));
+    auto launch = [&](auto* to, auto pieces) {
+        hipLaunchKernelGGL((finish_norm_kernel<std::remove_pointer_t<decltype(to)>, decltype(pieces)::value>), dim3((unsigned)M), dim3(256), 0, as_stream(stream), g, to);
+    };
+    auto type = [&](auto* to) {
+        if (N <= 1024) launch(to, std::integral_constant<int, 1>{});
+        else launch(to, std::integral_constant<int, kFinishPieces>{});
+    };
+    if (dtype == MHIP_BF16) type(static_cast<bf16_t*>(h));
+    else type(static_cast<f16_t*>(h));
     return check_launch("finish_norm");
+}
+
+extern "C" int mhip_attend_project_parts(int64_t B, int64_t S, int64_t H, int64_t D, int64_t N, int dtype) {
+    const int group = D == kProjectHead && (dtype == MHIP_BF16 || dtype == MHIP_F16) && N >= 1 && N % 8 == 0 ? project_group(B, S, H) : 0;
+    return group && (N + 64) * H * D * 4 < 0x7FFFFFFFLL ? (int)H / group : 0;
+}
+
+extern "C" int mhip_attend_project(void* stream, const void* qkv, const float* w, float* sums, int64_t B, int64_t S, int64_t H, int64_t D, int64_t N, int dtype,
+                                   int n_ahead, const mhip_weights* ahead) {
+    if (!qkv || !w || !sums) return fail(MHIP_ERR_INVALID_ARGUMENT, "mhip_attend_project: NULL pointer");
+    if (n_ahead < 0 || n_ahead > kAhead || (n_ahead > 0 && !ahead)) return fail(MHIP_ERR_INVALID_ARGUMENT, "mhip_attend_project: up to %d matrices ahead", kAhead);
+    const int parts = mhip_attend_project_parts(B, S, H, D, N, dtype);
+    if (!parts || !aligned16({qkv, w, sums}))
+        return fail(MHIP_ERR_UNSUPPORTED, "mhip_attend_project: [%lld,%lld], %lld heads of %lld, %lld columns, dtype %d, or pointers off 16 bytes", (long long)B,
+                    (long long)S, (long long)H, (long long)D, (long long)N, dtype);
+    const int64_t d = H * D;
+    FaArgs a = {};
+    a.q = qkv;
+    a.k = static_cast<const char*>(qkv) + d * 2;
+    a.v = static_cast<const char*>(qkv) + 2 * d * 2;
+    a.B = (int)B; a.H = (int)H; a.Sq = a.Skv = (int)S; a.D = (int)D;
+    a.scale = (float)(1.0 / sqrt((double)D));
+    a.c = a.scale * kLog2e;
+    a.is_causal = 1;
+    for (int64_t* st : {a.qs, a.ks, a.vs}) { st[0] = S * 3 * d; st[1] = D; st[2] = 3 * d; }
+    LinearArgs g = {};
+    g.w = w; g.sums = sums;
+    g.M = (int)(B * S); g.N = (int)N; g.K = (int)d; g.splits = parts;
+    take_ahead(g, n_ahead, ahead);
+    return dtype == MHIP_BF16 ? project_type<bf16_t>(as_stream(stream), a, g, (int)H / parts) : project_type<f16_t>(as_stream(stream), a, g, (int)H / parts);
 }

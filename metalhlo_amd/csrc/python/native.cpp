@@ -248,6 +248,18 @@ FUNCTION(matmul) {
 
 const float* f32(const at::Tensor* t) { return t ? t->data_ptr<float>() : nullptr; }
 
+// A tuple of up to two matrices that the next calls read.
+int weights_ahead(PyObject* o, mhip_weights (&ahead)[2]) {
+    int n = 0;
+    if (!PyTuple_Check(o) || PyTuple_GET_SIZE(o) > 2) raise(PyExc_ValueError, "ahead must be a tuple of up to two matrices");
+    for (; n < PyTuple_GET_SIZE(o); n++) {
+        const at::Tensor* t = &dense(PyTuple_GET_ITEM(o, n));
+        if (t->dim() != 2 || t->scalar_type() != at::kFloat) raise(PyExc_TypeError, "weights ahead must be fp32 matrices");
+        ahead[n] = {t->data_ptr<float>(), t->size(1), t->size(0)};
+    }
+    return n;
+}
+
 // linear(x, weight, bias, residual, activation code, trans_b, parts, (weights ahead)): parameters in fp32;
 // parts > 0: the fp32 sums of so many shares of K instead
 FUNCTION(linear) {
@@ -266,13 +278,7 @@ FUNCTION(linear) {
         const int dt = dtype_code(x.scalar_type()), act = (int)integer(arg[4]);
         at::Tensor c = parts > 0 ? empty({parts, M, N}, at::kFloat, x) : empty({M, N}, x.scalar_type(), x);
         mhip_weights ahead[2] = {};
-        int n_ahead = 0;
-        if (!PyTuple_Check(arg[7]) || PyTuple_GET_SIZE(arg[7]) > 2) raise(PyExc_ValueError, "ahead must be a tuple of up to two matrices");
-        for (; n_ahead < PyTuple_GET_SIZE(arg[7]); n_ahead++) {
-            const at::Tensor* t = &dense(PyTuple_GET_ITEM(arg[7], n_ahead));
-            if (t->dim() != 2 || t->scalar_type() != at::kFloat) raise(PyExc_TypeError, "weights ahead must be fp32 matrices");
-            ahead[n_ahead] = {t->data_ptr<float>(), t->size(1), t->size(0)};
-        }
+        const int n_ahead = weights_ahead(arg[7], ahead);
         check([&] { return mhip_linear_w32(stream_of(x), x.data_ptr(), f32(&w), f32(bias), ptr(res),
                                            parts > 0 ? nullptr : c.data_ptr(), M, N, K, tb, act, dt, parts > 0 ? c.data_ptr<float>() : nullptr,
                                            parts > 0 ? parts : 1, n_ahead, ahead); });
@@ -332,13 +338,7 @@ FUNCTION(linear_layer) {
         const int64_t bytes = gamma ? 0 : mhip_linear_w32_workspace(M, N, K);
         if (bytes > 0) work = empty({bytes}, at::kByte, x);
         mhip_weights ahead[2] = {};
-        int n_ahead = 0;
-        if (!PyTuple_Check(arg[6]) || PyTuple_GET_SIZE(arg[6]) > 2) raise(PyExc_ValueError, "ahead must be a tuple of up to two matrices");
-        for (; n_ahead < PyTuple_GET_SIZE(arg[6]); n_ahead++) {
-            const at::Tensor* t = &dense(PyTuple_GET_ITEM(arg[6], n_ahead));
-            if (t->dim() != 2 || t->scalar_type() != at::kFloat) raise(PyExc_TypeError, "weights ahead must be fp32 matrices");
-            ahead[n_ahead] = {t->data_ptr<float>(), t->size(1), t->size(0)};
-        }
+        const int n_ahead = weights_ahead(arg[6], ahead);
         check([&] { return mhip_linear_w32_layer(stream_of(x), x.data_ptr(), f32(gamma), f32(beta), eps, f32(&w), f32(bias), ptr(res), c.data_ptr(), M, N, K, act, dt,
                                                  bytes > 0 ? work.data_ptr() : nullptr, bytes, n_ahead, ahead); });
         return THPVariable_Wrap(std::move(c));
@@ -383,6 +383,24 @@ FUNCTION(causal_attention) {
         check([&] { return mhip_flash_attention_strided(stream_of(x), p, p + step, p + 2 * step, nullptr, o.data_ptr(), B, H, S, S, D,
                                                         (float)(1.0 / std::sqrt((double)D)), 1, 0, 0, dt, strides); });
         return THPVariable_Wrap(std::move(o));
+    });
+}
+
+// attend_project(qkv [B * S, 3 H D], weight fp32 [H D, N], B, H, (weights ahead)) -> fp32 [parts, B * S, N]
+FUNCTION(attend_project) {
+    return guarded(n, 5, [&] {
+        const at::Tensor &x = dense(arg[0]), &w = dense(arg[1]);
+        const int64_t B = integer(arg[2]), H = integer(arg[3]);
+        if (x.dim() != 2 || B < 1 || H < 1 || x.size(0) % B != 0 || x.size(1) % (3 * H) != 0) raise(PyExc_ValueError, "expected a projection [B * S, 3 H D]");
+        const int64_t S = x.size(0) / B, D = x.size(1) / 3 / H;
+        if (w.dim() != 2 || w.size(0) != H * D) raise(PyExc_ValueError, "expected a weight [H D, N]");
+        if (w.scalar_type() != at::kFloat) raise(PyExc_TypeError, "parameters must be fp32");
+        const int dt = dtype_code(x.scalar_type());
+        mhip_weights ahead[2] = {};
+        const int n_ahead = weights_ahead(arg[4], ahead), parts = mhip_attend_project_parts(B, S, H, D, w.size(1), dt);
+        at::Tensor c = empty({parts > 0 ? parts : 1, x.size(0), w.size(1)}, at::kFloat, x);
+        check([&] { return mhip_attend_project(stream_of(x), x.data_ptr(), w.data_ptr<float>(), c.data_ptr<float>(), B, S, H, D, w.size(1), dt, n_ahead, ahead); });
+        return THPVariable_Wrap(std::move(c));
     });
 }
 
@@ -461,7 +479,7 @@ FUNCTION(bind) {
 }
 
 #define ENTRY(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
-PyMethodDef kMethods[] = {ENTRY(softmax), ENTRY(layer_norm), ENTRY(rms_norm), ENTRY(bias_gelu), ENTRY(matmul), ENTRY(linear), ENTRY(linear_layer), ENTRY(matmul_sums), ENTRY(tied_head), ENTRY(finish_norm), ENTRY(causal_attention),
+PyMethodDef kMethods[] = {ENTRY(softmax), ENTRY(layer_norm), ENTRY(rms_norm), ENTRY(bias_gelu), ENTRY(matmul), ENTRY(linear), ENTRY(linear_layer), ENTRY(matmul_sums), ENTRY(tied_head), ENTRY(finish_norm), ENTRY(causal_attention), ENTRY(attend_project),
                           ENTRY(flash_attention), ENTRY(argmax), ENTRY(bind), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

@@ -190,10 +190,13 @@ class GPT2:
                 x = layer(u, l["w_proj"], l["b_proj"], residual=x, ahead=(layers[i + 1]["w_qkv"],) if i + 1 < len(layers) else ())
             return self._head(kernels.finish_norm(None, None, x, norms[-1])[1], B, S)
         x, h = kernels.finish_norm(None, None, x, norms[0])
+        merged = kernels.attend_project_served(B, S, cfg.n_head, cfg.d_model // cfg.n_head, cfg.d_model, self.dtype)
         for i, l in enumerate(layers):
             qkv = linear(h, l["w_qkv"], l["b_qkv"], ahead=(l["w_o"], l["w_fc"]))
-            a = kernels.causal_attention(qkv, B, cfg.n_head)
-            sums = linear(a, l["w_o"], parts=o_parts, ahead=(l["w_proj"],))
+            if merged:
+                sums = kernels.attend_project(qkv, l["w_o"], B, cfg.n_head, ahead=(l["w_proj"],))
+            else:
+                sums = linear(kernels.causal_attention(qkv, B, cfg.n_head), l["w_o"], parts=o_parts, ahead=(l["w_proj"],))
             x, h = kernels.finish_norm(sums, l["b_o"], x, (l["ln2_g"], l["ln2_b"], 1e-5))
             u = linear(h, l["w_fc"], l["b_fc"], "gelu")
             sums = linear(u, l["w_proj"], parts=p_parts, ahead=(layers[i + 1]["w_qkv"],) if i + 1 < len(layers) else ())

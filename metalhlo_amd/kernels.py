@@ -158,6 +158,16 @@ def causal_attention(qkv, batch: int, n_head: int):
     return (_native or _host()).causal_attention(qkv, batch, n_head)
 
 
+def attend_project(qkv, weight, batch: int, n_head: int, ahead=()):
+    """matmul of causal_attention(qkv) and the fp32 weight [H D, N], rounded at use, in one launch: fp32 sums [parts, B * S, N] for finish_norm.
+    `attend_project_served` says for which sizes; `ahead` as in `linear`."""
+    return (_native or _host()).attend_project(qkv, weight, batch, n_head, ahead)
+
+
+def attend_project_served(batch: int, length: int, n_head: int, head_size: int, N: int, dtype) -> bool:
+    return bool(_lib.load().mhip_attend_project_parts(batch, length, n_head, head_size, N, DTYPE_CODE[dtype]))
+
+
 # ---- glue -------------------------------------------------------------------
 def gather_rows(table, indices):
     _dev(table, indices)

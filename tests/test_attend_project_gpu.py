@@ -1,0 +1,46 @@
+"""GPU parity of attention and its projection in one launch (attend_project of linear_w32.hip): one and two groups of 32 queries, rows around its groups of 16, heads in one
+part and in several, columns around its strips of 32 and the eighths that an XCD takes.
+
+The attention in front is causal_attention's, bit for bit (one code), so the sums differ from its result times the rounded weights in 64 bits by fp32 additions of K products
+alone: at most K 2^-23 of the sum of their magnitudes, a product of 16-bit numbers being exact."""
+import numpy as np
+import pytest
+import torch
+
+from tests.util import NAME, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=lambda d: NAME[d])
+@pytest.mark.parametrize("B,S,H,N", [(1, 1, 4, 8), (1, 31, 12, 768), (1, 32, 4, 264), (1, 33, 12, 40), (1, 64, 8, 1032), (2, 16, 4, 72), (2, 20, 12, 768), (2, 32, 8, 256), (4, 1, 1, 32), (3, 5, 2, 1000)], ids=str)
+def test_sums(B, S, H, N, dtype):
+    from metalhlo_amd import kernels
+    assert kernels.attend_project_served(B, S, H, 64, N, dtype)
+    rng = np.random.default_rng(B * 1000 + S + N)
+    qkv = to_dev(rng.standard_normal((B * S, 3 * H * 64)), dtype)
+    w = to_dev(rng.standard_normal((H * 64, N)), torch.float32)
+    sums = kernels.attend_project(qkv, w, B, H, ahead=(to_dev(rng.standard_normal((64, 128)), torch.float32),))
+    assert sums.dtype == torch.float32 and sums.shape[1:] == (B * S, N)
+    x, r = kernels.causal_attention(qkv, B, H).double(), w.to(dtype).double()
+    error = (sums.double().sum(0) - x @ r).abs()
+    assert bool((error <= H * 64 * 2.0 ** -23 * (x.abs() @ r.abs())).all()), float(error.max())
+
+
+def test_a_part_that_sees_nothing_behind_its_rows():
+    """Infinities and NaN behind the last row, of qkv and of W, reach no sum."""
+    from metalhlo_amd import kernels
+    rng = np.random.default_rng(5)
+    room = torch.full((64, 3 * 256), float("nan"), dtype=torch.bfloat16, device="cuda")
+    room[:37] = to_dev(rng.standard_normal((37, 768)), torch.bfloat16)
+    w = to_dev(rng.standard_normal((256, 72)), torch.float32)
+    wide = torch.full((320, 72), float("inf"), device="cuda")
+    wide[:256] = w
+    assert torch.equal(kernels.attend_project(room[:37], wide[:256], 1, 4), kernels.attend_project(room[:37].clone(), w, 1, 4))
+
+
+@pytest.mark.parametrize("B,S,H,D,N,dtype", [(1, 65, 4, 64, 64, torch.bfloat16), (3, 22, 4, 64, 64, torch.bfloat16), (1, 8, 4, 128, 64, torch.bfloat16), (1, 8, 4, 64, 60, torch.bfloat16),
+                                             (1, 8, 4, 64, 64, torch.float32), (0, 8, 4, 64, 64, torch.bfloat16), (1, 8, 4, 64, 0, torch.bfloat16)], ids=str)
+def test_what_is_not_served(B, S, H, D, N, dtype):
+    from metalhlo_amd import kernels
+    assert not kernels.attend_project_served(B, S, H, D, N, dtype)
