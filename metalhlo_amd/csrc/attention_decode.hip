@@ -50,6 +50,9 @@ __global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* 
     __shared__ __attribute__((aligned(16))) float sums[WAVES][NF][64][4];
     __shared__ float ml[2][WAVES][kMaxSq];
     __shared__ int last;
+    // (the arguments in one go: 1 x 8 heads over 4096 keys 9.40 -> 9.18 us, 8 x 32 over 512 12.94 -> 12.76)
+    asm volatile("" ::"s"(a.q), "s"(a.k), "s"(a.v), "s"(a.o), "s"(a.H), "s"(a.Sq), "s"(a.Skv), "s"(a.c), "s"(a.negate_q), "s"(a.qs[0]), "s"(a.qs[1]), "s"(a.ks[0]), "s"(a.ks[1]),
+                 "s"(a.vs[0]), "s"(a.vs[1]), "s"((int)a.qs[2]), "s"((int)a.ks[2]), "s"((int)a.vs[2]), "s"(part), "s"(per_part), "s"(words), "s"(tag));
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int li = lane & 15, lg = lane >> 4;
     const int bh = blockIdx.x, b_i = bh / a.H, h_i = bh % a.H;

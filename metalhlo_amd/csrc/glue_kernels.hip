@@ -69,11 +69,13 @@ __global__ __launch_bounds__(256) void embed_kernel(const int32_t* __restrict__ 
                                                     int64_t vocab, int vec4) {
     // over B*S; with a grid that is a multiple of 8, XCD x (workgroup ids x, x + 8, ...) takes the
     // x-th eighth of the tokens: the rows a following row kernel or GEMM handles on that XCD
+    // (the arguments in one go)
+    asm volatile("" ::"s"(ids), "s"(wte), "s"(wpe), "s"(out), "s"(S), "s"(d), "s"(vocab), "s"(vec4));
     const int64_t tok = gridDim.x % 8 == 0 ? (int64_t)(blockIdx.x % 8u) * (gridDim.x / 8u) + blockIdx.x / 8u : blockIdx.x;
     int64_t id = ids[tok];
     id = id < 0 ? 0 : (id > vocab - 1 ? vocab - 1 : id);
     const P* te = wte + id * d;
-    const P* pe = wpe + (tok % S) * d;
+    const P* pe = wpe + (int64_t)((uint32_t)tok % (uint32_t)S) * d;      // (a grid holds fewer than 2^31 tokens; 64 bits: 100 instructions more)
     O* o = out + tok * d;
     if (vec4) {       // rows of all three tensors start on 16-byte (params) / 8-byte (result) boundaries
         struct alignas(4 * sizeof(P)) P4 { P v[4]; };

@@ -34,6 +34,8 @@ struct HeadArgs {
 template <typename T>
 __global__ __launch_bounds__(64 * kHeadWaves) void tied_head_kernel(HeadArgs g) {
     extern __shared__ __attribute__((aligned(1024))) char smem[];
+    // (the arguments in one go)
+    asm volatile("" ::"s"(g.x), "s"(g.w), "s"(g.c), "s"(g.M), "s"(g.N), "s"(g.K), "s"(g.rows), "s"(g.strips), "s"(g.per));
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, lg = lane >> 4;
     const int first = (int)blockIdx.x * g.per, last = min(g.strips, first + g.per);
     if (first >= last) return;
