@@ -44,6 +44,8 @@ SIGNATURES = {
     "mhip_linear_w32_norm_ok": (_i32, [_i64, _i64, _i64, _i32]),
     "mhip_linear_w32_workspace": (_i64, [_i64, _i64, _i64]),
     "mhip_linear_w32_layer": (_i32, [_vp, _vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _i32, _vp, _i64, _i32, _vp]),
+    "mhip_attend_project_layer_ok": (_i32, [_i64, _i64, _i64, _i64, _i64, _i32]),
+    "mhip_attend_project_layer": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i32, _i32, _vp]),
     "mhip_attend_project_parts": (_i32, [_i64, _i64, _i64, _i64, _i64, _i32]),
     "mhip_attend_project": (_i32, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i32, _i32, _vp]),
     "mhip_flash_attention": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,

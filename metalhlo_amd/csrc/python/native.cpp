@@ -386,6 +386,29 @@ FUNCTION(causal_attention) {
     });
 }
 
+// attend_project_layer(qkv [B * S, 3 H D], weight fp32 [H D, N], bias, residual, B, H, (weights ahead)) -> [B * S, N]
+FUNCTION(attend_project_layer) {
+    return guarded(n, 7, [&] {
+        const at::Tensor &x = dense(arg[0]), &w = dense(arg[1]);
+        const at::Tensor *bias = optional_dense(arg[2]), *res = optional_dense(arg[3]);
+        const int64_t B = integer(arg[4]), H = integer(arg[5]);
+        if (x.dim() != 2 || B < 1 || H < 1 || x.size(0) % B != 0 || x.size(1) % (3 * H) != 0) raise(PyExc_ValueError, "expected a projection [B * S, 3 H D]");
+        const int64_t S = x.size(0) / B, D = x.size(1) / 3 / H;
+        if (w.dim() != 2 || w.size(0) != H * D) raise(PyExc_ValueError, "expected a weight [H D, N]");
+        const int64_t M = x.size(0), N = w.size(1);
+        for (const at::Tensor* p : {&w, bias})
+            if (p && p->scalar_type() != at::kFloat) raise(PyExc_TypeError, "parameters must be fp32");
+        if (bias && bias->numel() != N) raise(PyExc_ValueError, "bias must be [N]");
+        if (res && (res->numel() != M * N || res->scalar_type() != x.scalar_type())) raise(PyExc_ValueError, "residual must have the result's size and dtype");
+        const int dt = dtype_code(x.scalar_type());
+        mhip_weights ahead[2] = {};
+        const int n_ahead = weights_ahead(arg[6], ahead);
+        at::Tensor c = empty({M, N}, x.scalar_type(), x);
+        check([&] { return mhip_attend_project_layer(stream_of(x), x.data_ptr(), f32(&w), f32(bias), ptr(res), c.data_ptr(), B, S, H, D, N, dt, n_ahead, ahead); });
+        return THPVariable_Wrap(std::move(c));
+    });
+}
+
 // attend_project(qkv [B * S, 3 H D], weight fp32 [H D, N], B, H, (weights ahead)) -> fp32 [parts, B * S, N]
 FUNCTION(attend_project) {
     return guarded(n, 5, [&] {
@@ -479,7 +502,7 @@ FUNCTION(bind) {
 }
 
 #define ENTRY(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
-PyMethodDef kMethods[] = {ENTRY(softmax), ENTRY(layer_norm), ENTRY(rms_norm), ENTRY(bias_gelu), ENTRY(matmul), ENTRY(linear), ENTRY(linear_layer), ENTRY(matmul_sums), ENTRY(tied_head), ENTRY(finish_norm), ENTRY(causal_attention), ENTRY(attend_project),
+PyMethodDef kMethods[] = {ENTRY(softmax), ENTRY(layer_norm), ENTRY(rms_norm), ENTRY(bias_gelu), ENTRY(matmul), ENTRY(linear), ENTRY(linear_layer), ENTRY(matmul_sums), ENTRY(tied_head), ENTRY(finish_norm), ENTRY(causal_attention), ENTRY(attend_project), ENTRY(attend_project_layer),
                           ENTRY(flash_attention), ENTRY(argmax), ENTRY(bind), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

@@ -182,10 +182,13 @@ class GPT2:
         x = kernels.embed_tokens(ids, p["wte"], p["wpe"], self.dtype).reshape(T, cfg.d_model)
         if kernels.linear_norm_served(T, cfg.d_model, cfg.d_model, self.dtype):
             layer = kernels.linear_layer
+            merged = kernels.attend_project_layer_served(B, S, cfg.n_head, cfg.d_model // cfg.n_head, cfg.d_model, self.dtype)
             for i, l in enumerate(layers):
                 qkv = layer(x, l["w_qkv"], l["b_qkv"], norm=norms[i], ahead=(l["w_o"], l["w_fc"]))
-                a = kernels.causal_attention(qkv, B, cfg.n_head)
-                x = layer(a, l["w_o"], l["b_o"], residual=x, ahead=(l["w_proj"],))
+                if merged:
+                    x = kernels.attend_project_layer(qkv, l["w_o"], l["b_o"], x, B, cfg.n_head, ahead=(l["w_proj"],))
+                else:
+                    x = layer(kernels.causal_attention(qkv, B, cfg.n_head), l["w_o"], l["b_o"], residual=x, ahead=(l["w_proj"],))
                 u = layer(x, l["w_fc"], l["b_fc"], "gelu", norm=(l["ln2_g"], l["ln2_b"], 1e-5))
                 x = layer(u, l["w_proj"], l["b_proj"], residual=x, ahead=(layers[i + 1]["w_qkv"],) if i + 1 < len(layers) else ())
             return self._head(kernels.finish_norm(None, None, x, norms[-1])[1], B, S)

@@ -168,6 +168,15 @@ def attend_project_served(batch: int, length: int, n_head: int, head_size: int, 
     return bool(_lib.load().mhip_attend_project_parts(batch, length, n_head, head_size, N, DTYPE_CODE[dtype]))
 
 
+def attend_project_layer(qkv, weight, bias, residual, batch: int, n_head: int, ahead=()):
+    """linear_layer(causal_attention(qkv), weight, bias, residual=residual) in one launch; `attend_project_layer_served` says for which sizes."""
+    return (_native or _host()).attend_project_layer(qkv, weight, bias, residual, batch, n_head, ahead)
+
+
+def attend_project_layer_served(batch: int, length: int, n_head: int, head_size: int, N: int, dtype) -> bool:
+    return bool(_lib.load().mhip_attend_project_layer_ok(batch, length, n_head, head_size, N, DTYPE_CODE[dtype]))
+
+
 # ---- glue -------------------------------------------------------------------
 def gather_rows(table, indices):
     _dev(table, indices)
