@@ -204,7 +204,7 @@ int mhip_linear_w32_layer(void* stream, const void* x, const float* gamma, const
 int mhip_attend_project_parts(int64_t B, int64_t S, int64_t H, int64_t D, int64_t N, int dtype);
 int mhip_attend_project(void* stream, const void* qkv, const float* w, float* sums, int64_t B, int64_t S, int64_t H, int64_t D, int64_t N, int dtype,
                         int n_ahead, const mhip_weights* ahead);
-/* In one launch up to 32 rows, whose heads times sequences are 16 at most (mhip_attend_project_layer_ok): c = causal_attention(qkv) . round(w) + round(bias)
+/* In one launch up to 32 rows, whose heads times sequences are 16 at most, 32 for up to 16 rows (mhip_attend_project_layer_ok): c = causal_attention(qkv) . round(w) + round(bias)
  * (+ residual) as mhip_linear_w32_layer rounds it, bias [N] in fp32 and residual [B S, N], either may be NULL. */
 int mhip_attend_project_layer_ok(int64_t B, int64_t S, int64_t H, int64_t D, int64_t N, int dtype);
 int mhip_attend_project_layer(void* stream, const void* qkv, const float* w, const float* bias, const void* residual, void* c, int64_t B, int64_t S, int64_t H,

@@ -466,7 +466,7 @@ __global__ __launch_bounds__(64 * kWaves) void attend_project_kernel(FaArgs a, L
     if (m < g.M && n < n1) *reinterpret_cast<f32x4*>(g.sums + ((int64_t)part * g.M + m) * g.N + n) = sum;
 }
 
-// The same for up to 32 rows with all heads in a workgroup, a wave for a head of a sequence: 16 columns of c = round(attention(x) . round(W) + round(bias)) +
+// The same for up to 32 rows with all heads in a workgroup, a wave for one head of a sequence or two: 16 columns of c = round(attention(x) . round(W) + round(bias)) +
 // residual, and no launch that adds parts up.  The wave of head h then takes its 64 rows of W.
 // (GPT-2-small, against two launches: 4 tokens 331 -> 298 us, 8 tokens 335 -> 307, 16 tokens 348 -> 323, 32 tokens 405 -> 400.)
 constexpr int kLayerWaves = 16, kLayerRows = 32;
@@ -506,11 +506,13 @@ __global__ __launch_bounds__(64 * kLayerWaves) void attend_project_layer_kernel(
     if (mine && g.residual) res = *reinterpret_cast<const u32x2*>(static_cast<const T*>(g.residual) + (int64_t)fm * g.N + col);
 
     // (by_blocks divides by the sequences)
-    const int h = divided(wave, g.by_blocks), b = wave - h * a.B;
-    if (h < a.H)
+    for (int pair = wave; pair < a.B * a.H; pair += waves) {
+        const int h = divided(pair, g.by_blocks), b = pair - h * a.B;
         short_rows<T, kProjectHead, 1>(a, b * a.H + h, smem + wave * kValues, [&](int query, int d, u32x2 v) __attribute__((always_inline)) {
             *reinterpret_cast<u32x2*>(rows + (b * a.Sq + query) * pitch + (h * kProjectHead + d) * 2) = v;
         });
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the next turn's values come to the same place)
+    }
     __syncthreads();
 
     // (rows past the last hold whatever LDS held: each is a row of the product of its own, and not stored)
@@ -752,7 +754,8 @@ int launch_project_layer(hipStream_t s, const FaArgs& a, LinearArgs g) {
     static hipError_t err = hipSuccess;
     std::call_once(once, [&] { err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kMost); });
     if (err != hipSuccess) return fail(MHIP_ERR_LAUNCH, "attend_project_layer: cannot reserve %d bytes of LDS: %s", kMost, hipGetErrorString(err));
-    const int pairs = a.B * a.H, waves = pairs < kWaves ? kWaves : pairs;      // (a workgroup in front is kWaves of them)
+    const int pairs = a.B * a.H, turns = (pairs + kLayerWaves - 1) / kLayerWaves, deal = (pairs + turns - 1) / turns;
+    const int least = a.H < kWaves ? kWaves : a.H, waves = deal < least ? least : deal;      // (a wave for each head's rows of W; a workgroup in front is kWaves of them)
     g.strips = (g.N + 15) / 16;
     g.per_xcd = (g.strips + kXcds - 1) / kXcds;
     plan_ahead(g);
@@ -870,9 +873,10 @@ void project_args(FaArgs& a, LinearArgs& g, const void* qkv, const float* w, int
 }  // namespace
 }  // namespace mhip
 
+// Two turns of the waves up to 16 rows only (GPT-2-small, in one launch and in two: 2 x 4 tokens 333.6 and 346.0 us, 2 x 8 340 and 348, 2 x 12 395 and 392, 2 x 16 413 and 404).
 extern "C" int mhip_attend_project_layer_ok(int64_t B, int64_t S, int64_t H, int64_t D, int64_t N, int dtype) {
     if (D != kProjectHead || (dtype != MHIP_BF16 && dtype != MHIP_F16) || N < 1 || N % 8 != 0 || N > (1 << 24)) return 0;
-    if (B < 1 || H < 1 || S < 1 || B > kLayerWaves || H > kLayerWaves || S > kLayerRows || B * H > kLayerWaves || B * S > kLayerRows) return 0;
+    if (B < 1 || H < 1 || S < 1 || B > kLayerRows || H > kLayerWaves || S > kLayerRows || B * H > (B * S <= 16 ? 2 : 1) * kLayerWaves || B * S > kLayerRows) return 0;
     return (N + 64) * H * D * 4 < 0x7FFFFFFFLL;
 }
 
