@@ -159,16 +159,17 @@ __global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* 
             oacc[f] = Mfma16A<T>::run(vf, pb, oacc[f]);
         }
     };
-    // Blocks of this wave, in a ring from one that a hash of head and part chooses (head size 128): workgroups that all walk from the start of their
-    // keys are a power of two apart where caches are as long as one, and meet in the same banks of the memory.  (A start that
-    // grows with the head can be worse, 64 heads over 8192 keys 50.6 -> 65 us.)  us, from the first block | so, one query: 256 heads over 4096 keys
-    // 93.2 | 89.6, over 2048 49.1 | 47.6, 96 over 4096 40.1 | 37.8, 64 over 8192 50.6 | 49.0, 192 over 3000 53.5 | 51.8, 256 over 4000 89.6 | 89.2, 512 over 4096
-    // 177 | 175; head size 64, whose rows are a line each, lost by it: 128 over 8192 48.4 | 49.4.
+    // Blocks of this wave, in a ring; of eight waves with head size 128 wave w starts w eighths of the way round.  Workgroups that walk side by side from the start of their
+    // keys are a power of two apart where caches are as long as one, and meet in the same banks of the memory; so a workgroup itself is in eight places at a time.  us, from the first
+    // block | so, one query: 256 heads over 4096 keys 93.9 | 90.8, over 2048 47.7 | 47.3, 96 over 4096 38.9 | 37.6, 64 over 8192 50.0 | 48.9, 192 over 3000
+    // 52.9 | 51.8, 256 over 4000 91.2 | 88.7, 48 over 4096 22.7 | 21.7.  The place depends on nothing but the wave, so that a head's bits do not say where in the launch it is (a start that a hash
+    // of the head chooses: 89.8, 47.3, 37.5, 49.4, 51.6, 88.6, 21.5).  Four waves of two workgroups a unit lose by it, 512 heads over 4096 177 | 180; eight waves with a run of blocks each
+    // instead 96.4 for 256 heads; head size 64, whose rows are a line each, by a ring from a hash, 128 over 8192 48.4 | 49.4.
     constexpr int kStride = WAVES * kKeys;
     const int base = k0 + wave * kKeys;
     if (base < k1) {
         int left = (k1 - base + kStride - 1) / kStride, key = base;
-        if (D == 128 && left >= 4) key += (int)(((uint32_t)(bh * 64 + (int)blockIdx.y) * 2246822519u >> 24) * (uint32_t)left >> 8) * kStride;
+        if (WAVES == 8 && D == 128 && left >= 4) key += left * wave / WAVES * kStride;
         Block cur;
         load(cur, key);
         for (;;) {
