@@ -218,8 +218,8 @@ int mhip_attend_project_layer(void* stream, const void* qkv, const float* w, con
  * Causal rule: key position > query position is masked; a row whose keys are all masked
  * with -inf yields zeros, one whose keys all have the type's lowest number as mask their mean.
  * fp32 softmax state and accumulation.  For up to sixteen queries without the causal rule and for F32 the last bits of
- * a row may change with B * H, which decides over how many parts its keys are dealt; where in the launch
- * the head is they do not say.
+ * a row may change with B * H, which decides over how many parts its keys are dealt, and over more
+ * than sixteen parts with Sq; where in the launch the head is they do not say.
  * Replaces FlashAttentionTiledKernel (Metal/Kernels/FlashAttentionKernel.swift:462-671)
  * launched from MetalExecutor.executeFlashAttentionDirect
  * (Runtime/MetalExecutor.swift:502-564). dtype: BF16, F16, F32.  On the

@@ -352,20 +352,21 @@ __global__ __launch_bounds__(64 * WAVES) void fa_decode_kernel(FaArgs a, float* 
 // How a launch's keys are dealt: parts of the range, keys a part, waves of a workgroup.
 struct DecodePlan { int parts, per, waves; };
 
-DecodePlan decode_plan(int64_t bh, int64_t Sq, int64_t Skv) {
+DecodePlan decode_plan(int64_t bh, int64_t Skv) {
     auto dealt = [&](int64_t want, int waves) {
         const int64_t unit = part_keys(Skv), most = Skv / unit, n = want < most ? want : most;
         const int parts = n < 2 ? 1 : n > 64 ? 64 : (int)n;
         return DecodePlan{parts, parts == 1 ? (int)Skv : (int)(((Skv + parts - 1) / parts + unit - 1) / unit * unit), waves};
     };
-    // Workgroups of eight waves, one a compute unit, where whole parts of all heads fill three quarters of the units and eight waves have
-    // a block of keys: half as many parts to write and to put together as with two workgroups of four waves a unit, which is what
-    // the others take.  us, four | eight waves, one query: 8 heads over 16384 keys of head size 128 23.0 | 17.7 (eight queries 26.3 | 19.2), 32 over 4096
-    // 15.8 | 14.7, 192 over 700 16.3 | 13.2, 256 over 4096 93.9 | 93.2, of 64 48.8 | 46.1, 12 over 5632 of 64 11.3 | 9.1, 12 over 300 5.1 | 4.8; of more heads a
-    // second turn ([32,12,1000] of 64, four queries, 21.2 | 22.6, 512 over 4096 177 | 179); parts of 128 keys 24 over 1024 of 64 6.1 | 6.4.
+    // Workgroups of eight waves, one a compute unit, where 256 units divided among the heads leave fewer than a quarter of them over and more than four waves of a workgroup get
+    // a block of keys (a part being 256 keys at least, or 128, and parts 64 at most, few heads over few keys do not fill the units either way): half as many parts to write and
+    // to put together as with two workgroups of four waves a unit, which is what the others take.  us, four | eight waves, one query: 8 heads over 16384 keys of head size 128
+    // 23.0 | 17.7 (eight queries 26.3 | 19.2), 32 over 4096 15.8 | 14.7, 192 over 700 16.3 | 13.2, 64 over 200 6.0 | 5.1, 256 over 4096 93.9 | 93.2, of 64 48.8 | 46.1, 12 over 5632
+    // of 64 11.3 | 9.1, 12 over 300 5.1 | 4.8; sixteen queries, 256 over 250 of 128 10.5 | 11.2, 16 over 2048 11.5 | 11.6, nine of 128 over 512 11.7 | 10.9 (their number is left out of the rule, so that
+    // a row's bits do not follow from it); of more heads a second turn ([32,12,1000] of 64, four queries, 21.2 | 22.6, 512 over 4096 177 | 179); parts of 128 keys 24 over 1024 of 64 6.1 | 6.4.
     if (bh <= 256 && 256 / bh * bh >= 192) {
         const DecodePlan p = dealt(256 / bh, 8);
-        if (p.per > (Sq > 8 ? 8 : 4) * kKeys) return p;      // (16 queries of 16 heads over 2048 10.9 | 11.0)
+        if (p.per > 4 * kKeys) return p;
     }
     return dealt((512 + bh - 1) / bh, 4);
 }
@@ -394,13 +395,13 @@ bool fa_decode_eligible(const FaArgs& a) { return a.Sq <= kMaxSq && !a.is_causal
 
 int64_t fa_decode_workspace(int64_t bh, int64_t Sq, int64_t Skv, int64_t D) {
     if (Sq < 1 || Sq > kMaxSq || (D != 64 && D != 128)) return 0;
-    const int parts = decode_plan(bh, Sq, Skv).parts;
+    const int parts = decode_plan(bh, Skv).parts;
     return parts == 1 ? 0 : parts * bh * Sq * (D + 2) * 4 + bh * 8;
 }
 
 int launch_fa_decode(hipStream_t s, const FaArgs& a, int64_t D, int dtype, void* workspace, int64_t workspace_bytes) {
     const int64_t bh = (int64_t)a.B * a.H, need = fa_decode_workspace(bh, a.Sq, a.Skv, D);
-    DecodePlan plan = decode_plan(bh, a.Sq, a.Skv);
+    DecodePlan plan = decode_plan(bh, a.Skv);
     if (!workspace || need > workspace_bytes) { plan.parts = 1; plan.per = a.Skv; }
     float* part = static_cast<float*>(workspace);
     if (dtype == MHIP_BF16) return D == 128 ? launch<bf16_t, 128>(s, a, part, plan) : launch<bf16_t, 64>(s, a, part, plan);

@@ -99,7 +99,7 @@ def flash_attention(q, k, v, scale: Optional[float] = None, is_causal: bool = Fa
     Default scale 1/sqrt(D) (FlashAttentionKernel.swift:55).  q, k, v (and `out`, when given)
     may be views with arbitrary batch / head / row strides as long as the last axis is
     contiguous, e.g. slices of a fused QKV projection; packed tensors take the plain entry.  The last bits of a
-    row may depend on B * H for fp32 and for up to 16 queries without the causal rule."""
+    row may depend on B * H for fp32 and for up to 16 queries without the causal rule, as mhip.h says."""
     return (_native or _host()).flash_attention(q, k, v, scale, is_causal, mask, out)
 
 
