@@ -220,8 +220,16 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(FaArgs a) {
     constexpr bool kDeep = HAS_MASK && std::is_same<T, bf16_t>::value;
     float deep = -INFINITY;
 
-    auto block = [&](int it, int cur) __attribute__((always_inline)) {
-        const int kv0 = it * kBKV;
+    // Two blocks a turn where there is no mask, their places in the rings then constants of the LDS addresses: 14 of 165 vector instructions of a block less.  us, one | two, head
+    // size 64: causal [4,16,4096] 165.4 | 163.0, [8,12,1024] 22.4 | 22.1, [16,12,512] 16.0 | 15.6, full [4,16,4096] 308.2 | 300.3, [8,12,1024] 34.5 | 34.0; of 128 within 0.5 %.  (Blocks as a
+    // function that the loop calls cost the masked forms up to 10 %, [2,16,4096] of 64 291 | 320, and the forms without a mask 8 to 31 spilled scalars.)
+    static_assert(NB == 2, "two blocks a turn");
+    constexpr int kTurn = HAS_MASK || PART ? 1 : NB;
+    for (int turn = 0; turn < nkv; turn += kTurn)
+#pragma unroll
+    for (int u = 0; u < kTurn; u++) {
+        const int it = turn + u, cur = kTurn == NB ? u : it % NB, kv0 = it * kBKV;
+        if (u && it >= nkv) break;
         load_tile(kv0 + (NB - 1) * kBKV, (cur + NB - 1) % NB);
 
         const bool wave_active = !CAUSAL || kv0 <= qw + 31;
@@ -397,16 +405,6 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(FaArgs a) {
             __builtin_amdgcn_s_setprio(0);
         }
         if (it + 1 < nkv) tiles_ready();
-    };
-    // (Two blocks a turn, whose place in the rings is then a constant of the LDS addresses: 14 of 165 vector instructions of a block less.  us: causal
-    // [4,16,4096] of head size 64 181.2 -> 178.9, [8,12,1024] 25.1 -> 24.8, [16,32,256] 20.2 -> 19.7, of 128 within 0.5 %.)
-    static_assert(NB == 2, "two blocks a turn");
-    for (int it = 0; it < nkv; it++) {
-        if constexpr (HAS_MASK || PART) block(it, it & 1);
-        else {
-            block(it, 0);
-            if (++it < nkv) block(it, 1);
-        }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // nothing may land in LDS after the workgroup ends
 
