@@ -46,24 +46,36 @@ struct FaArgs {
 // transformer layer in front ([B*S, 3*H*D], whose row tiles a GEMM writes XCD by XCD in eighths
 // of the rows) and the output projection behind, a batch's heads then read what its own XCD's
 // L2 may still hold and leave their output where the next GEMM looks for it.
-// Up to seven heads are left over where eight does not divide their number.  Their tiles are dealt over the XCDs one by one, so that
-// every XCD has the same work whichever tiles they are, and come first: some of them are the longest.  An XCD then reads K and V of
-// its own heads and of those few.  us, every head on every XCD | so: causal [3,12,1000] of head size 64 16.55 | 16.28, [7,12,1024] 22.9 | 22.2,
-// else [3,12,1000] 23.1 | 21.9, fp32 [3,4,2048] causal 72.2 | 71.2; the pipelined kernel, which orders its tiles likewise, [3,12,4096] of 128 242 | 232.
-template <bool CAUSAL>
-__device__ inline void tile_of_workgroup(const FaArgs& a, int id, int& bh, int& qb) {
-    const int xcd = id & 7, local = id >> 3;
-    const int heads = (a.B * a.H) >> 3, left = (a.B * a.H) & 7;      // of every XCD; left over
-    const int shared = (left * a.nqb - xcd + 7) / 8;                 // tiles of the latter that this XCD takes
+// Up to seven heads are left over where eight does not divide their number.  Their tiles are dealt over the XCDs one of every eight, from the front and from the back in turn, so that
+// every XCD has the same work; an XCD then reads K and V of its own heads and of those few.  us, every head on every XCD | so: causal [3,4,2048] of fp32 and head size 64 72.7 | 72.0,
+// [12,1500] 44.3 | 44.0, [28,1500] of 128 246 | 245, else bf16 [3,12,1000] of 64 23.1 | 21.9; the pipelined kernel, which orders its tiles likewise, [3,12,4096] of 128 242 | 232.  (Theirs in front
+// of the others in a causal list, which is then not sorted: [12,1500] 52.6, [28,1500] of 128 272, bf16 [20,4096] of 32 72.8 | 73.4 and 78.4.)
+// SORTED false: theirs in front all the same, for a kernel that has up to two tiles a unit, where the shorter way to the tile counts for more (fa_flow_kernel,
+// causal [3,12,1000] of 64 16.5 sorted and 16.3, [12,300] 7.35 and 7.2, [12,2048] 26.2 and 26.1).
+template <bool CAUSAL, bool SORTED = true>
+__host__ __device__ inline void tile_of_workgroup(const FaArgs& a, int id, int& bh, int& qb) {
+    const int all = a.B * a.H, xcd = id & 7, local = id >> 3;
+    const int heads = all >> 3, left = all & 7;                      // of every XCD; left over
+    const int whole = SORTED ? left * a.nqb >> 3 : 0;
+    auto turn = [&](int s) { return (s & 1) && s < whole ? 7 - xcd : xcd; };
+    auto taken = [&](int n) { return (n >> 3) + (turn(n >> 3) < (n & 7) ? 1 : 0); };      // of the first n tiles left over
+    const int shared = SORTED ? taken(left * a.nqb) : (left * a.nqb - xcd + 7) / 8;
     int e = local;
     if (CAUSAL) {
-        const int total = shared + heads * a.nqb;
         const int round = local / a.cu_group, c = local % a.cu_group;
-        const int in_round = min(a.cu_group, total - round * a.cu_group);
+        const int in_round = min(a.cu_group, shared + heads * a.nqb - round * a.cu_group);
         e = round * a.cu_group + ((round & 1) ? in_round - 1 - c : c);   // place in the longest-first list
     }
-    if (e < shared) {
-        const int j = 8 * e + xcd;
+    if (CAUSAL && SORTED) {
+        // level n, the tiles of one length, has its own heads' first and then its share of the others; before(n) places lie in front of it, and e is in level 8 e / all or the next one
+        auto before = [&](int n) { return heads * n + taken(left * n); };
+        int n = heads ? 8 * e / all : (8 * e + turn(e)) / left;
+        if (heads && before(n + 1) <= e) n++;
+        const int f = e - before(n), s = e - heads * (n + 1);
+        bh = f < heads ? xcd * heads + f : 8 * heads + 8 * s + turn(s) - left * n;
+        qb = a.nqb - 1 - n;
+    } else if (e < shared) {
+        const int j = 8 * e + (SORTED ? turn(e) : xcd);
         bh = 8 * heads + (CAUSAL ? j % left : j / a.nqb);
         qb = CAUSAL ? a.nqb - 1 - j / left : j % a.nqb;
     } else {

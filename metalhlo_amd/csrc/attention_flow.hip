@@ -31,7 +31,7 @@ __global__ __launch_bounds__(256, D == 128 && !CAUSAL ? 1 : 2) void fa_flow_kern
     __shared__ __attribute__((aligned(1024))) char smem[2 * NB * kTile];
 
     int bh, qb;
-    tile_of_workgroup<CAUSAL>(a, blockIdx.x, bh, qb);
+    tile_of_workgroup<CAUSAL, false>(a, blockIdx.x, bh, qb);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lrow = lane & 31, lhalf = lane >> 5;
     const int qblk0 = qb * kBQ;
