@@ -221,10 +221,11 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(FaArgs a) {
     float deep = -INFINITY;
 
     // Two blocks a turn where there is no mask, their places in the rings then constants of the LDS addresses: 14 of 165 vector instructions of a block less.  us, one | two, head
-    // size 64: causal [4,16,4096] 165.4 | 163.0, [8,12,1024] 22.4 | 22.1, [16,12,512] 16.0 | 15.6, full [4,16,4096] 308.2 | 300.3, [8,12,1024] 34.5 | 34.0; of 128 within 0.5 %.  (Blocks as a
-    // function that the loop calls cost the masked forms up to 10 %, [2,16,4096] of 64 291 | 320, and the forms without a mask 8 to 31 spilled scalars.)
+    // size 64: causal [4,16,4096] 165.4 | 163.0, [8,12,1024] 22.4 | 22.1, [16,12,512] 16.0 | 15.6, full [4,16,4096] 308.2 | 300.3, [8,12,1024] 34.5 | 34.0; of 128 within 0.5 %; in parts, [12,2048]
+    // causal and full, of 96 56.6 | 54.2 and 57.3 | 55.3, f16 93.7 | 90.9 and 93.7 | 92.7, of 32 35.4 | 34.0 and 33.5 | 33.9.  (Blocks as a function that the loop calls cost the masked forms up to 10 %,
+    // [2,16,4096] of 64 291 | 320, and the forms without a mask 8 to 31 spilled scalars.)
     static_assert(NB == 2, "two blocks a turn");
-    constexpr int kTurn = HAS_MASK || PART ? 1 : NB;
+    constexpr int kTurn = HAS_MASK ? 1 : NB;
     for (int turn = 0; turn < nkv; turn += kTurn)
 #pragma unroll
     for (int u = 0; u < kTurn; u++) {
