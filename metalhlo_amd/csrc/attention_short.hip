@@ -37,7 +37,7 @@ int launch_type(hipStream_t s, const FaArgs& a, int64_t D) {
 }  // namespace
 
 // us, fa_fwd_kernel | here, in a graph, up to 16 states in turn, D 64: [1,12,16] 4.1 | 2.7, [1,12,64] 4.5 | 3.5, [8,32,64] 5.9 | 4.5, [64,32,64] 17.7 | 14.6;
-// D 128: [1,32,40] 5.7 | 4.3, [8,32,64] 8.1 | 6.2, [32,32,64] 18.8 | 16.2; GPT-2 over 37 tokens, behind a projection and with cold caches, 467 | 451.
+// D 128: [1,32,40] 5.7 | 4.3, [8,32,64] 8.1 | 6.2, [32,32,64] 18.8 | 16.2.  (GPT-2 launches this where attend_project does not serve: more than 64 tokens in all, or more heads times sequences than its waves.)
 // Past 64 keys or without the causal rule 16 rows a wave were tried: they read the keys again for every 16 rows ([8,32,100] 6.9 | 7.8, every
 // key for every query D 128 [16,32,64] 10.4 | 11.5).
 bool fa_short_wanted(const FaArgs& a) { return a.is_causal && a.Sq <= kRows * kMostWaves && a.Skv <= 64; }

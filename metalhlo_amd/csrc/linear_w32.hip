@@ -812,7 +812,9 @@ extern "C" int mhip_linear_w32(void* stream, const void* x, const float* w, cons
     return linear_entry(stream, x, w, bias, residual, c, M, N, K, trans_b, activation, dtype, nullptr, nullptr, 0.f, sums, nullptr, parts, n_ahead, ahead);
 }
 
-// Up to 32 rows: every workgroup normalises all of them, 10 operations an element, 0.7 us for 16 rows and 2.3 for 48.
+// Up to 32 rows: every workgroup normalises all of them, 10 operations an element, 0.7 us for 16 rows and 2.3 for 48.  GPT-2-small, us, so | normalised by finish_norm_kernel behind
+// attend_project: 16 tokens 322 | 355, 17 363 | 358, 24 380 | 363, 32 399 | 368, 2 x 8 336 | 352, 2 x 12 392 | 365, 2 x 16 403 | 370; 3 x 5 342 | 400, 3 x 8 390 | 400, 4 x 8 402 | 404.
+// The line is the one from before attend_project; from 17 rows on the other form is the faster one for one or two sequences.
 extern "C" int mhip_linear_w32_norm_ok(int64_t M, int64_t N, int64_t K, int dtype) { return mhip_linear_w32_ok(M, N, K, dtype) && M <= 32 && K <= kWaves * 3 * 32; }
 
 extern "C" int64_t mhip_linear_w32_workspace(int64_t M, int64_t N, int64_t K) {
@@ -881,7 +883,8 @@ void project_args(FaArgs& a, LinearArgs& g, const void* qkv, const float* w, int
 }  // namespace
 }  // namespace mhip
 
-// Two turns of the waves up to 16 rows only (GPT-2-small, in one launch and in two: 2 x 4 tokens 333.6 and 346.0 us, 2 x 8 340 and 348, 2 x 12 395 and 392, 2 x 16 413 and 404).
+// Two turns of the waves up to 16 rows only (GPT-2-small, in one launch and in two: 2 x 4 tokens 324 and 334 us, 2 x 8 336 and 344, 2 x 12 395 and 392, 2 x 16 413 and 404; past 16
+// rows the form with finish_norm is faster than both, see mhip_linear_w32_norm_ok).
 extern "C" int mhip_attend_project_layer_ok(int64_t B, int64_t S, int64_t H, int64_t D, int64_t N, int dtype) {
     if (D != kProjectHead || (dtype != MHIP_BF16 && dtype != MHIP_F16) || N < 1 || N % 8 != 0 || N > (1 << 24)) return 0;
     if (B < 1 || H < 1 || S < 1 || B > kLayerRows || H > kLayerWaves || S > kLayerRows || B * H > (B * S <= 16 ? 2 : 1) * kLayerWaves || B * S > kLayerRows) return 0;

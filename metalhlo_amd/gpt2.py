@@ -148,7 +148,8 @@ class GPT2:
         if dt not in (torch.bfloat16, torch.float16) or d // self.cfg.n_head not in (64, 128) or d % self.cfg.n_head:
             return False
         # (each 64 rows read a matrix again, which from memory costs as much as converting it: us as they are held and converted,
-        # replayed, 97 tokens 615 and 614, 112 tokens 626 and 624, 128 tokens 643 and 634; a matrix of up to 4 MB stays in an L2)
+        # replayed, 65 tokens 559 and 571, 80 567 and 585, 96 581 and 595, 97, which are blocks of 64 rows instead of 48, 616 and 595,
+        # 128 643 and 615; a matrix of up to 4 MB stays in an L2)
         if tokens > 96 and 4 * d * f > 4 << 20:
             return False
         return d <= 4096 and all(kernels.linear_served(tokens, n, k, dt) for n, k in ((3 * d, d), (d, d), (f, d), (d, f), (self.vocab_pad, d)))
